@@ -120,76 +120,138 @@ DEV const T* operand(const LinArgs& a, int feature) {
 }
 
 // ---- prompts -------------------------------------------------------------------------------------
-// grid.x: row tiles of 128 (experts: entries of the tile table), grid.y: feature tiles of 128.
-// rows: a gather table (slot -> row) or nullptr; out rows are row0 + local row.
+// What a workgroup keeps in LDS.  bf16: two stages of two k tiles (8 weight tiles and 8 row groups each), 64 KiB; deeper rings with a barrier
+// per k tile were no faster (two workgroups on a compute unit hide each other's waits).  32 bits: a ring of three stages of one k tile, 72 KiB.
+__host__ DEV constexpr int lin_stages(int size) { return size == 2 ? 2 : 3; }
+__host__ DEV constexpr int lin_step(int size) { return size == 2 ? 2 : 1; }
+__host__ DEV constexpr int lin_stage(int size) { return lin_step(size) * 8 * 1024 * (1 + size / 2); }
+// 128 features from f0 on x n_rows <= 128 rows, k tiles [k0, k1): 4 waves of 64 x 64.  gather: a table (slot -> row) or nullptr; out rows are
+// row0 + local row.
 template <typename T>
 DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
   typedef typename Frag<T>::type frag;
   constexpr int AB = 64 * (int)sizeof(frag);  // bytes of an A fragment
-  constexpr int STAGE = 16 * 1024 + 16 * AB;  // 8 row tiles x 2 k tiles of each operand
+  constexpr int KS = lin_step(sizeof(T)), STAGE = lin_stage(sizeof(T)), R = lin_stages(sizeof(T)), H = sizeof(T) / 2, WB = 8 * KS * 1024;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave & 1, wn = wave >> 1, n = k1 - k0;
   const int rt0 = f0 >> 4;
-  // this wave's share of the staging: weight tiles rt0 + 2 * wave + {0, 1}, row groups 2 * wave + {0, 1}, both k tiles of a step
-  const char* src_w[2];
-  const T* src_a[2];
+  // this wave's share of the staging: two weight tiles and two row groups, the k tiles of a stage
+  const char *src_w[2], *src_a[2][H];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)  // (tiles past the end: any valid one, never stored)
+    src_w[i] = reinterpret_cast<const char*>(a.w) + ((size_t)min(rt0 + 2 * wave + i, a.rt - 1) * a.kt + k0) * 1024 + lane * 16;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int t = 2 * wave + i;
-    const int rt = min(rt0 + t, a.rt - 1);  // (tiles past the end: any valid one, never stored)
-    src_w[i] = reinterpret_cast<const char*>(a.w) + (size_t)rt * a.kt * 1024 + lane * 16;
-    int r = min(t * 16 + (sizeof(T) == 2 ? block_row(lane) : lane & 15), n_rows - 1);
-    r = gather ? gather[row0 + r] : row0 + r;
-    src_a[i] = operand<T>(a, f0) + (size_t)r * a.lda + (sizeof(T) == 2 ? block_group(lane) : lane >> 4) * 8;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {  // (a block of 16 x 32 floats is two loads of 8 rows)
+      int r = min(t * 16 + (H == 1 ? block_row(lane) : h * 8 + (lane >> 3)), n_rows - 1);
+      r = gather ? gather[row0 + r] : row0 + r;
+      src_a[i][h] = reinterpret_cast<const char*>(operand<T>(a, f0) + (size_t)r * a.lda + (size_t)k0 * 32) + (H == 1 ? block_group(lane) : (lane & 7) ^ (lane >> 3)) * 16;
+    }
   }
   auto stage = [&](int kt, char* buf) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const int slot = (2 * wave + i) * 2 + kk;
-        __builtin_amdgcn_global_load_lds((gptr)(src_w[i] + (size_t)(kt + kk) * 1024), (lptr)(buf + slot * 1024), 16, 0, 0);
-        const char* s = reinterpret_cast<const char*>(src_a[i] + (size_t)(kt + kk) * 32);
+      for (int kk = 0; kk < KS; ++kk)
+        __builtin_amdgcn_global_load_lds((gptr)(src_w[i] + (size_t)(kt + kk) * 1024), (lptr)(buf + ((2 * wave + i) * KS + kk) * 1024), 16, 0, 0);
 #pragma unroll
-        for (int h = 0; h < (int)sizeof(T) / 2; ++h)
-          __builtin_amdgcn_global_load_lds((gptr)(s + h * 16), (lptr)(buf + 16 * 1024 + slot * AB + h * 1024), 16, 0, 0);
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        const int slot = (2 * wave + i) * KS + kk;
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+          __builtin_amdgcn_global_load_lds((gptr)(src_a[i][h] + (size_t)(kt + kk) * 32 * sizeof(T)), (lptr)(buf + WB + slot * AB + h * 1024), 16, 0, 0);
       }
-  };
-  auto read_a = [&](const char* buf, int slot) {
-    frag f;
-    if constexpr (sizeof(T) == 2) {
-      f = *reinterpret_cast<const frag*>(buf + 16 * 1024 + slot * AB + block_place(lane) * 16);
-    } else {
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(buf + 16 * 1024 + slot * AB + lane * 16);
-      const f32x4 hi = *reinterpret_cast<const f32x4*>(buf + 16 * 1024 + slot * AB + 1024 + lane * 16);
-      f = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    }
-    return f;
   };
   f32x4 acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  stage(k0, lds + ((k0 >> 1) & 1) * STAGE);
-  for (int kt = k0; kt < k1; kt += 2) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads into LDS; the barrier makes it everybody's
-    __syncthreads();
-    char* cur = lds + ((kt >> 1) & 1) * STAGE;
-    if (kt + 2 < k1) stage(kt + 2, lds + (((kt >> 1) & 1) ^ 1) * STAGE);
+  if constexpr (sizeof(T) == 2) {
+    stage(0, lds);
+    for (int kt = 0; kt < n; kt += KS) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads into LDS; the barrier makes it everybody's
+      __syncthreads();
+      char* cur = lds + ((kt / KS) & 1) * STAGE;
+      if (kt + KS < n) stage(kt + KS, lds + (((kt / KS) & 1) ^ 1) * STAGE);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8 w[4];
-      frag x[4];
+      for (int kk = 0; kk < KS; ++kk) {
+        bf16x8 w[4], x[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const bf16x8*>(cur + ((wm * 4 + i) * 2 + kk) * 1024 + lane * 16);
+        for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const bf16x8*>(cur + ((wm * 4 + i) * KS + kk) * 1024 + lane * 16);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = read_a(cur, (wn * 4 + j) * 2 + kk);
+        for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const bf16x8*>(cur + WB + ((wn * 4 + j) * KS + kk) * AB + block_place(lane) * 16);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mma(w[i], x[j], acc[i][j]);
+          for (int j = 0; j < 4; ++j) acc[i][j] = mma(w[i], x[j], acc[i][j]);
+      }
     }
+  } else {
+    // While a k tile is multiplied the next one's operands are read into the other set of registers and the loads of R - 1 more are on
+    // their way.  What bounds it: per wave and k tile 48 matrix instructions (768 cycles) and the 208 vector instructions (832 cycles)
+    // that take 32 activations apart; they are issued in turns, a row group's matrix work beside the splitting of the next.
+    // 301 x 2048 x 16896: 303 us with v_mfma_f32_16x16x4_f32, 101 us so; 301 x 16896 x 2048 in 4 parts: 304 -> 114 us.
+    struct Operands {
+      bf16x8 w[4];
+      f32x8 x[4];
+    };
+    // eight lanes to the 128 bytes of a row, its pieces of 16 bytes exchanged by the row's place as in block_place
+    const int at = (lane & 15) * 128 + (((lane >> 4) * 2) ^ (lane & 7)) * 16;
+    auto read = [&](const char* buf, Operands& o) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const char* s = buf + WB + (wn * 4 + j) * AB;
+        o.x[j] = __builtin_shufflevector(*reinterpret_cast<const f32x4*>(s + at), *reinterpret_cast<const f32x4*>(s + (at ^ 16)), 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.w[i] = *reinterpret_cast<const bf16x8*>(buf + (wm * 4 + i) * 1024 + lane * 16);
+    };
+    int cur = 0;
+    auto step = [&](int kt, const Operands& now, Operands& next) {
+      // tile kt + 1 is here when at most the loads of R - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
+      // tile kt in registers, so that its buffer takes tile kt + R (past the end: the last one again, never read)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 + 2 * H) * (R - 2)) : "memory");
+      lds_barrier();
+      stage(min(kt + R, n - 1), lds + cur * STAGE);
+      cur = cur + 1 == R ? 0 : cur + 1;
+      read(lds + cur * STAGE, next);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const Split x = split3(now.x[j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[i], x.b2, acc[i][j]);  // (one piece after the other: no instruction waits for the last)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[i], x.b1, acc[i][j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[i], x.b0, acc[i][j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j == 0) __builtin_amdgcn_sched_group_barrier(0x002, 52, 0);
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (j == 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          if (j < 3) __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        }
+      }
+    };
+    Operands p, q;
+#pragma unroll
+    for (int i = 0; i < R; ++i) stage(min(i, n - 1), lds + i * STAGE);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 + 2 * H) * (R - 1)) : "memory");
+    lds_barrier();
+    read(lds, p);
+    for (int kt = 0; kt < n; kt += 2) {  // (n is even)
+      step(kt, p, q);
+      step(kt + 1, q, p);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -208,7 +270,7 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
   }
 }
 template <typename T>
-__global__ __launch_bounds__(256) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
+__global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 128, per = part_tiles(a), k0 = blockIdx.y * per;
   a.out_f += blockIdx.y * a.part_stride;
@@ -413,7 +475,7 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
 }
 
 // ---- launches ------------------------------------------------------------------------------------
-static int lin_lds(bool f32) { return 2 * (16 * 1024 + 16 * 64 * (f32 ? 32 : 16)); }
+static int lin_lds(bool f32) { return lin_stages(f32 ? 4 : 2) * lin_stage(f32 ? 4 : 2); }
 static int check_lin(const LinArgs& a, const char* what) {
   if (!a.w || !a.a_t || a.rows < 1 || a.kt < 2 || (a.kt & 1) || a.rt < 1 || a.lda < a.kt * 32) DSK_FAIL(DSK_ERR_INVALID, "%s: rows %d kt %d rt %d lda %d", what, a.rows, a.kt, a.rt, a.lda);
   if (a.parts > 1 && (a.n_wide || a.epi != LIN_STORE || part_tiles(a) * (a.parts - 1) >= a.kt)) DSK_FAIL(DSK_ERR_INVALID, "%s: %d parts of %d", what, a.parts, a.kt);
@@ -427,21 +489,22 @@ static int allow_lds(K k, int bytes) {
 }
 // Microseconds a prompt product takes on 256 compute units, by measurement: two workgroups of 128 x 128 on one work 1.3 us on a step of 64
 // columns (one alone 1.05), one of 256 x 256 takes 1.84 us and starts and ends slower; a part more writes and reads its sums.
-static double lin_cost(int rows, int rt, int kt, int parts, bool big) {
+// In 32 bits a step of 64 columns takes 1.75 us alone and 3.2 us of two.
+static double lin_cost(int rows, int rt, int kt, int parts, bool big, bool f32) {
   const double k = part_tiles(kt, parts) / 2, sums = (parts - 1) * 3.2e-5 * rows * rt;
-  if (big) return cdiv(cdiv(rows, 256) * cdiv(rt, 16) * parts, 256) * (15 + 1.84 * k) + sums;
+  if (big) return f32 ? 1e9 : cdiv(cdiv(rows, 256) * cdiv(rt, 16) * parts, 256) * (15 + 1.84 * k) + sums;
   const int n = cdiv(rows, 128) * cdiv(rt, 8) * parts;
-  return (n <= 256 ? 1.05 * k : cdiv(n, 512) * 1.3 * k) + 5 + sums;
+  return (n <= 256 ? (f32 ? 1.75 : 1.05) * k : cdiv(n, 512) * (f32 ? 3.2 : 1.3) * k) + 5 + sums;
 }
 static bool lin_big(const LinArgs& a, int parts, bool f32) {
   if (f32 || (a.a_seg & 255)) return false;
-  return a.tile ? a.tile == 256 : lin_cost(a.rows, a.rt, a.kt, parts, true) < lin_cost(a.rows, a.rt, a.kt, parts, false);
+  return a.tile ? a.tile == 256 : lin_cost(a.rows, a.rt, a.kt, parts, true, f32) < lin_cost(a.rows, a.rt, a.kt, parts, false, f32);
 }
 int lin_parts(int rows, int rt, int kt, bool f32, int most) {
   int best = 1;
   double least = 0;
   for (int n = 1; n <= most && (n == 1 || kt / n >= 16); ++n) {
-    const double c = std::min(lin_cost(rows, rt, kt, n, false), f32 ? 1e9 : lin_cost(rows, rt, kt, n, true));
+    const double c = std::min(lin_cost(rows, rt, kt, n, false, f32), lin_cost(rows, rt, kt, n, true, f32));
     if (n == 1 || c < least) {
       least = c;
       best = n;
@@ -462,16 +525,11 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32) {
     hipLaunchKernelGGL(lin_big_kernel, dim3(tiles, std::max(a.parts, 1)), dim3(512), RING * 32 * 1024, st, a, row_tiles, tiles);
     return DSK_OK;
   }
-  const int row_tiles = cdiv(a.rows, 128), tiles = row_tiles * cdiv(a.rt, 8);
+  const int row_tiles = cdiv(a.rows, 128), tiles = row_tiles * cdiv(a.rt, 8), lds = lin_lds(f32);
   const dim3 grid(tiles, std::max(a.parts, 1));
-  const int lds = lin_lds(f32);
-  if (f32) {
-    DSK_TRY(allow_lds(lin_kernel<float>, lds));
-    hipLaunchKernelGGL(lin_kernel<float>, grid, dim3(256), lds, st, a, row_tiles, tiles);
-  } else {
-    DSK_TRY(allow_lds(lin_kernel<bf16>, lds));
-    hipLaunchKernelGGL(lin_kernel<bf16>, grid, dim3(256), lds, st, a, row_tiles, tiles);
-  }
+  auto k = f32 ? lin_kernel<float> : lin_kernel<bf16>;
+  DSK_TRY(allow_lds(k, lds));
+  hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, row_tiles, tiles);
   return DSK_OK;
 }
 int launch_experts(hipStream_t st, const MoeArgs& m, bool down, bool f32) {

@@ -4,7 +4,8 @@
 // lives as FRAGMENTS of 16 rows x 32 columns: 64 lanes x 8 consecutive k, lane = (k / 8) * 16 + row, 1 KiB contiguous - the
 // operand order of v_mfma_f32_16x16x32_bf16.  A wave reads a fragment with one 16-byte load per lane from consecutive
 // addresses, in HBM and in LDS alike.  A 32-bit run multiplies the same fragments with eight v_mfma_f32_16x16x4_f32: step j
-// takes element j of every lane, so lane groups stand for the k values {8 g + j}.
+// takes element j of every lane, so lane groups stand for the k values {8 g + j}.  Its prompt products take each activation apart
+// into three bf16 numbers instead (Split).
 #pragma once
 #include "dsk_internal.h"
 
@@ -38,6 +39,38 @@ DEV f32x4 mma(const f32x8& w, const f32x8& a, f32x4 c) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], a[j], c, 0, 0, 0);
   return c;
+}
+
+// A 32-bit activation as the exact sum of three bf16 numbers: its top 8 significant bits, the next 8, the last 8 (cut off, not rounded, so
+// that each rest is exact; b2 alone can fall under the smallest bf16, below 2^-110).  A product with a bf16 weight is then three bf16
+// products, each exact in 32 bits and summed in 32 bits: the precision of v_mfma_f32_16x16x4_f32 at a fifth of its cycles (three
+// 16x16x32 of 16 cycles for eight of 32).
+struct Split {
+  bf16x8 b0, b1, b2;
+};
+DEV Split split3(const f32x8& x) {
+  typedef unsigned u32x8 __attribute__((ext_vector_type(8)));
+  typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
+  u32x8 p0, p1, p2;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float v = x[i];  // (a bit cast of an element of a vector reads element 0)
+    const unsigned bits = __builtin_bit_cast(unsigned, v);
+    // (of an infinity: inf - inf, NaN, for which fmaxf takes a number that is small beside it; no other rest is below -2^121)
+    const float r = fmaxf(v - __builtin_bit_cast(float, bits & 0xffff0000u), -0x1p121f);
+    const unsigned rest = __builtin_bit_cast(unsigned, r);
+    p0[i] = bits;
+    p1[i] = rest;
+    p2[i] = __builtin_bit_cast(unsigned, r - __builtin_bit_cast(float, rest & 0xffff0000u));
+  }
+  u32x4v o0, o1, o2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // the high halves of two words
+    o0[i] = __builtin_amdgcn_perm(p0[2 * i + 1], p0[2 * i], 0x07060302);
+    o1[i] = __builtin_amdgcn_perm(p1[2 * i + 1], p1[2 * i], 0x07060302);
+    o2[i] = __builtin_amdgcn_perm(p2[2 * i + 1], p2[2 * i], 0x07060302);
+  }
+  return {__builtin_bit_cast(bf16x8, o0), __builtin_bit_cast(bf16x8, o1), __builtin_bit_cast(bf16x8, o2)};
 }
 
 // A block of 16 rows x 32 columns on its way from row-major memory to operands: loaded row by row, four lanes to a row, lane l's 8 columns
