@@ -5,7 +5,9 @@
 //   lin_big_kernel  the same with 256 x 256 and a ring of four stages, where there are enough of such tiles (bf16)
 //   few_kernel      up to 16 rows (decoding): 4 waves share 16 features and split k; weights stream from HBM straight into the
 //                   MFMA operand registers, 1 KiB contiguous per wave and load
-// Both take plain products and the experts' (rows gathered per expert); a launch of few_kernel can hold several products.
+//   expert_kernel   the experts' products of prompts, rows gathered per expert: 256 features x 128 (64, 32) rows, weights straight
+//                   into registers (32 bits: lin_kernel's tiles)
+// few_kernel takes plain products and the experts', several of them in one launch.
 #include "layered_kernels.h"
 #include "seq_device.h"
 
@@ -269,6 +271,95 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
     }
   }
 }
+
+// bf16, 256 features x up to 16 NJ rows: 4 waves of 64 features each, all of them on every row.  A weight tile is one wave's own, so weights go
+// straight into its registers a step (two k tiles) ahead - 1 KiB of consecutive bytes a load -, and LDS holds the rows alone: 8 + NJ operand
+// reads out of it feed 4 NJ matrix instructions where lin_body needs 16 for 16.  What bounds it is what a compute unit takes out of L2 (about
+// 48 GB/s) and, with the last tiles of experts seldom full, work on rows that are not there: hence NJ = 8, 4 and 2.  64 experts of 1408 over
+// 2048 rows, top 6, width 2048: gate / up 337 -> 254 us, down 201 -> 164 us (lin_body with a grid of row tiles x feature tiles before).
+// For plain products, whose row tiles are full, it is within 3 % of lin_kernel either way, and lin_big_kernel has more work per byte.
+template <int NJ>
+__host__ DEV constexpr int wide_stage() { return 2 * NJ * 1024; }
+template <int NJ>
+DEV void wide_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
+  constexpr int STAGE = wide_stage<NJ>(), AL = NJ / 2;  // AL: this wave's loads of rows in a step
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = k1 - k0;
+  const int rt0 = (f0 >> 4) + 4 * wave;
+  const char *src_w[4], *src_a[AL];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) src_w[i] = reinterpret_cast<const char*>(a.w) + ((size_t)min(rt0 + i, a.rt - 1) * a.kt + k0) * 1024;  // (past the end: never stored)
+#pragma unroll
+  for (int i = 0; i < AL; ++i) {
+    const int id = wave * AL + i;  // row group id / 2, k tile id % 2
+    int r = min((id >> 1) * 16 + block_row(lane), n_rows - 1);
+    r = gather ? gather[row0 + r] : row0 + r;
+    src_a[i] = reinterpret_cast<const char*>(operand<bf16>(a, f0) + (size_t)r * a.lda + (size_t)(k0 + (id & 1)) * 32 + block_group(lane) * 8);
+  }
+  struct Weights {
+    bf16x8 w[2][4];
+  };
+  auto load = [&](int kt, char* buf, Weights& o) {
+#pragma unroll
+    for (int i = 0; i < AL; ++i)
+      __builtin_amdgcn_global_load_lds((gptr)(src_a[i] + (size_t)kt * 64), (lptr)(buf + (wave * AL + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.w[kk][i] = *reinterpret_cast<const bf16x8*>(src_w[i] + (size_t)(kt + kk) * 1024 + lane * 16);
+  };
+  f32x4 acc[4][NJ];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int kt, const char* cur, char* other, const Weights& now, Weights& next) {
+    // what was requested a step ago is here, the barrier makes it everybody's (the builtin: the compiler counts the weights' loads itself)
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    lds_barrier();
+    load(min(kt + 2, n - 2), other, next);  // (past the end: the last step's again, not used)
+    bf16x8 x[2][NJ];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) x[kk][j] = *reinterpret_cast<const bf16x8*>(cur + (2 * j + kk) * 1024 + block_place(lane) * 16);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[kk][i], x[kk][j], acc[i][j]);
+    // requests first, then an operand is read four groups of matrix instructions ahead of its own
+    __builtin_amdgcn_sched_group_barrier(0x020, 8 + AL, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * NJ; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+      if (i < 2 * NJ - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+  };
+  Weights p, q;
+  load(0, lds, p);
+  for (int kt = 0; kt < n; kt += 4) {  // (n is even)
+    step(kt, lds, lds + STAGE, p, q);
+    if (kt + 2 < n) step(kt + 2, lds + STAGE, lds, q, p);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int r = j * 16 + (lane & 15);
+    if (r >= n_rows) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rt = rt0 + i;
+      if (rt >= a.rt) continue;
+      if (a.epi == LIN_GLU) {
+        if (!(i & 1)) store_glu<bf16>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[i][j], acc[i | 1][j]);
+      } else {
+        store_plain<bf16>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+      }
+    }
+  }
+}
 template <typename T>
 __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -380,14 +471,41 @@ DEV void set_expert(LinArgs& a, const MoeArgs& m, const ExpertMat& e, int expert
   a.rt = sh ? e.shared_rt : e.rt;
   a.p0 = sh ? m.shared_limit : m.limit;
 }
+// grid.x: an upper bound of the tiles.  The routed experts' come first, in groups of four row tiles (mostly one expert's, they are sorted) and in a
+// group feature tile by feature tile, and an XCD takes a contiguous range: the workgroups that read one weight tile meet in one L2, and
+// the rows of a group stay in it.  The shared expert's tiles, the longest, start first.
 template <typename T>
-__global__ __launch_bounds__(256) void expert_kernel(LinArgs a, const MoeArgs m, const int down) {
+__global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs m, const int down, const int shared_tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  if ((int)blockIdx.x >= *m.n_tiles) return;
-  const int expert = m.tiles[4 * blockIdx.x], s0 = m.tiles[4 * blockIdx.x + 1], n = m.tiles[4 * blockIdx.x + 2];
-  set_expert(a, m, down ? m.down : m.up, expert);
-  if ((int)blockIdx.y * 8 >= a.rt) return;
-  lin_body<T>(a, down ? nullptr : m.slot_row, s0, n, blockIdx.y * 128, 0, a.kt, lds);
+  constexpr int FT = sizeof(T) == 2 ? 16 : 8;
+  const ExpertMat& e = down ? m.down : m.up;
+  const int row_tiles = *m.n_tiles - shared_tiles, ft = (e.rt + FT - 1) / FT, sft = (e.shared_rt + FT - 1) / FT;
+  int b = blockIdx.x, tile, f;
+  const int first = (shared_tiles * sft + 7) & ~7;
+  if (b < first) {
+    if (b >= shared_tiles * sft) return;
+    b = xcd_range(b, shared_tiles * sft);
+    f = b / shared_tiles;
+    tile = row_tiles + b % shared_tiles;
+  } else {
+    b -= first;
+    if (b >= row_tiles * ft) return;
+    b = xcd_range(b, row_tiles * ft);
+    const int group = b / (4 * ft), n = min(4, row_tiles - 4 * group);
+    b -= group * 4 * ft;
+    f = b / n;
+    tile = 4 * group + b % n;
+  }
+  set_expert(a, m, e, m.tiles[4 * tile]);
+  const int* gather = down ? nullptr : m.slot_row;
+  const int row0 = m.tiles[4 * tile + 1], rows = m.tiles[4 * tile + 2];
+  if constexpr (sizeof(T) == 2) {
+    if (rows > 64) wide_body<8>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    else if (rows > 32) wide_body<4>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    else wide_body<2>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+  } else {
+    lin_body<T>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
+  }
 }
 
 // ---- up to 16 rows -------------------------------------------------------------------------------
@@ -535,14 +653,14 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32) {
 int launch_experts(hipStream_t st, const MoeArgs& m, bool down, bool f32) {
   const LinArgs a = expert_lin(m, down);
   const ExpertMat& e = down ? m.down : m.up;
-  const dim3 grid(m.max_tiles, cdiv(m.shared ? (e.rt > e.shared_rt ? e.rt : e.shared_rt) : e.rt, 8));
-  const int lds = lin_lds(f32);
+  const int shared_tiles = m.shared ? cdiv(m.rows, MOE_TILE) : 0, ft = f32 ? 8 : 16;
+  const dim3 grid((m.max_tiles - shared_tiles) * cdiv(e.rt, ft) + ((shared_tiles * cdiv(e.shared_rt, ft) + 7) & ~7));
   if (f32) {
+    const int lds = lin_lds(f32);
     DSK_TRY(allow_lds(expert_kernel<float>, lds));
-    hipLaunchKernelGGL(expert_kernel<float>, grid, dim3(256), lds, st, a, m, (int)down);
+    hipLaunchKernelGGL(expert_kernel<float>, grid, dim3(256), lds, st, a, m, (int)down, shared_tiles);
   } else {
-    DSK_TRY(allow_lds(expert_kernel<bf16>, lds));
-    hipLaunchKernelGGL(expert_kernel<bf16>, grid, dim3(256), lds, st, a, m, (int)down);
+    hipLaunchKernelGGL(expert_kernel<bf16>, grid, dim3(256), 2 * wide_stage<8>(), st, a, m, (int)down, shared_tiles);
   }
   return DSK_OK;
 }

@@ -14,6 +14,38 @@ def ctx():
     c.close()
 
 
+def no_mixers(W):
+    for k in W:
+        if k.endswith("left.out") or k.endswith("right.out"):
+            W[k][:] = 0
+
+
+# one expert takes every row (and the shared one too), so a prompt's length is its number of rows: both sides of the 32-, 64- and 128-row
+# forms; ff: feature tiles short of, at and behind a workgroup's 256 features (gate and up: 2 ff of them)
+@pytest.mark.parametrize("ff,shared", [(40, 0), (128, 24), (136, 272)])
+@pytest.mark.parametrize("dtype,tol", [("bfloat16", 0.02), ("float32", U.F32)])
+def test_expert_products_at_the_edges_of_row_tiles(ctx, tmp_path, ff, shared, dtype, tol):
+    # bf16: inputs, hidden values and outputs are each rounded to 2^-9, relative to values of about the result's size: 3 roundings of
+    # independent terms, far below 0.02 of the rows' scale
+    K = U.Case(ctx, tmp_path, U.config([U.parallel(mlp=U.moe(1, 1, ff, 0.8, shared, 1.2))], width=264), edit=no_mixers, dtype=dtype)
+    t = K.tokens(257)
+    want = []
+    K.ref.run(U.O.Sequence(K.ref), t, want)
+    K.lm.set_trace(True)
+    for n in (17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 161, 193, 257):
+        s = K.lm.seq_open()
+        K.lm.step([(s, t[:n], [n - 1])])
+        assert U.err(K.lm.trace_rows(0, n), want[0][:n]) < tol, n
+        K.lm.seq_close(s)
+
+
+# several experts, rows spread unevenly: groups of four row tiles with and without neighbours of the same expert, a last group that is short
+@pytest.mark.parametrize("experts,top", [(3, 1), (6, 2), (40, 7)])
+def test_expert_products_over_many_experts(ctx, tmp_path, experts, top):
+    K = U.Case(ctx, tmp_path, U.config([U.parallel(mlp=U.moe(experts, top, 72, 0.8, 40, 1.2))]), edit=no_mixers)
+    K.check_trace(700, cuts=([129],))
+
+
 # 32-bit activations are multiplied in three bf16 pieces.  Two pieces alone would be up to 2^-16 off; 32-bit sums, through the model's four
 # products and a softmax, stay under a quarter of that (v_mfma_f32_16x16x4_f32 gave up to 2.2e-6 here, this gives up to 2.1e-6).
 @pytest.mark.parametrize("width", [64, 328, 1000])
