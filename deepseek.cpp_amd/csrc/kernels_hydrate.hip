@@ -392,162 +392,257 @@ DEV void hyd16_item_end(Hyd16Acc& acc) {
 }
 DEV float hyd16_value(const Hyd16Acc& acc, int r) { return (acc.S[r][0] + acc.S[r][1]) + (acc.S[r][2] + acc.S[r][3]); }
 
-// The workgroup: up to 8 waves = 8 consecutive STRIPS times the SAME 16 tokens (blockIdx.y = the token chunk).  The tokens' operands
-// of HYD16_SB blocks at a time are staged once per workgroup in LDS (double-buffered, one barrier per stage) and every wave reads its
-// matrix operands from there: a wave's vector-memory traffic is its own tiles only.  (First form, measured: the waves of a workgroup
-// on different token chunks of one strip, each loading its 4.4 KB of operands per block from L2 - SQ counters: 51 % of the wave time
-// parked on s_waitcnt, VALU 32 %: 46 KB per CU and block through a memory path that carries ~27 GB/s per CU; wo 108 us at P = 64.)
-#define HYD16_SB 4          // blocks per stage
+// The workgroup: up to 8 waves = 8 consecutive STRIPS (GLU: 4 strips, one wave on the w1 strip and its neighbour on the w3 strip) times the
+// SAME 16 MT tokens.  The tokens' operands of HYD16_SB blocks at a time are staged once per workgroup in LDS (double-buffered, one
+// barrier per stage) and every wave reads its matrix operands from there: a wave's vector-memory traffic is its own tiles only.
+// What bounds it is vector instructions (about 80 % of the issue slots of two waves a SIMD): a tile's expansion (~90, once per pass) and the
+// float stage (~100 per 16 tokens and tile), so a pass takes MT = 2 groups of tokens wherever more than 16 are left: ~145 a tile and
+// 16 tokens.  512 tokens of DeepSeek-V3, against MT = 1 with the min operand masked per group (~215) and a GLU pair in one wave: experts'
+// w1 / w3 1502 -> 896 us, w2 813 -> 590, wo 429 -> 343, dense w1 / w3 1327 -> 710.
+// The min term: one v_mfma_i32_16x16x32_i8 per group.  Its 8 bytes a lane are two digit words of the token's: word 4 g + kg' is in the half that
+// g & 1 names and the weight side has zeros in the other half.
+#define HYD16_SB 2          // blocks per stage
 #define HYD16_TOK_B 272     // LDS bytes of a token's codes of one block (256 + 16: the 16 tokens of an operand read spread over the banks)
-#define HYD16_STAGE_B (HYD16_SB * (16 * HYD16_TOK_B + 16 * 64 + 16 * 4))   // codes | sub-block sums as digit words (hyd16_split) | scales, per block
-template <int R> struct Hyd16Stage { u32x4 c[R]; u32x4 bs; u32x4 d; };
-// Plain matrices: blockIdx.x = strip group, blockIdx.y = the chunk of 16 tokens.  Expert stacks (A.n_experts > 0: the task's rows come
-// through its list, src/infer.cpp:853-878): blockIdx.x = task x strip groups, the workgroup walks the task's rows 16 at a time (a
-// launch may be restricted to tasks with a row count in [cnt_min, cnt_max]: the few-row tasks stay with hyd_gemm_kernel's quads).
-template <bool GLU, int NW>
-__global__ __launch_bounds__(64 * NW) void hyd_gemm16_kernel(const HydGemmArgs A) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // 2 x HYD16_STAGE_B
+template <int MT>
+constexpr int hyd16_stage_b() { return HYD16_SB * MT * (16 * HYD16_TOK_B + 16 * 64 + 16 * 4); }  // codes | digit words (hyd16_split), [kg'][g] | scales, per block
+typedef long i64x1;
+struct Hyd16W {  // a tile's weight side
+  i32x4 B[4];   // the scaled group operands
+  u32x2_t m[4]; // the min operands
+};
+DEV void hyd16_weights(const HydTile& T, int kgp, Hyd16W& o) {
+  const u32 w[4] = {T.w.x, T.w.y, T.w.z, T.w.w};
+  u32 lo[4], hi[4];  // (hyd16_expand)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(w[i], w[i], false, false);
+    lo[i] = sw[0];
+    hi[i] = sw[1];
+  }
+  const int fs = kgp >> 1;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int sh = 2 * (2 * (g & 1) + fs);
+    const u32 scm = T.sc[g] >> (8 * kgp);  // the sub-block's scale | min nibbles
+    const u32 sc = scm & 0xFu, pair = sc | (sc << 16), mn = ((scm >> 4) & 0xFu) * 0x00080801u;
+    const u32* src = (g >> 1) ? hi : lo;
+    o.B[g].x = (int)pkmul16((src[0] >> sh) & 0x03030303u, pair);
+    o.B[g].y = (int)pkmul16((src[1] >> sh) & 0x03030303u, pair);
+    o.B[g].z = (int)pkmul16((src[2] >> sh) & 0x03030303u, pair);
+    o.B[g].w = (int)pkmul16((src[3] >> sh) & 0x03030303u, pair);
+    o.m[g] = (g & 1) ? u32x2_t{0u, mn} : u32x2_t{mn, 0u};
+  }
+}
+DEV float hyd16_item1(float dd, float D, float dmn, float M) {  // an item of one block: its two chains are a product each
+#pragma clang fp contract(off)
+  return dd * D - dmn * M;
+}
+// One pass: 16 MT of the task's rows, from `base` on, through all blocks of this wave's strip (matrix W).  Every wave of the workgroup calls it.
+// SEG4 (rows of more than 8 blocks, tile_device.h tile_seg): an item is 4 blocks, its chains ad and am end with it; otherwise every block is an item.
+template <bool GLU, bool SEG4, int NW, int MT>
+DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, const rsrc_t& RB, const rsrc_t& RD, const int* list, int base, int cnt, bool live,
+                    int strip, uint8_t* lds) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  constexpr int nwaves = NW, nthreads = 64 * NW;
-  constexpr int R = HYD16_SB * 256 / nthreads;  // 16-byte pieces of a stage's codes per thread
+  constexpr int nthreads = 64 * NW, TT = 16 * MT, STAGE = hyd16_stage_b<MT>();
+  constexpr int R = HYD16_SB * TT * 16 / nthreads;              // 16-byte pieces of a stage's codes per thread
+  constexpr int BP = HYD16_SB * TT * 2, RB_N = (BP + nthreads - 1) / nthreads;  // pieces of 8 sums
+  constexpr int D_LDS = HYD16_SB * TT * (HYD16_TOK_B + 64);
+  static_assert(R >= 1 && HYD16_SB == 2 && TT <= nthreads, "staging");
+  const int n = A.n, nb = n >> 8;
+  const int kgp = lane >> 4, tl = lane & 15;   // operand side: token tl of a group, K-group kg'
+  const int q = lane >> 4, rown = lane & 15;   // result side: tokens 4 q .. 4 q + 3, row rown of the strip
+  auto arow_of = [&](int e) { return (list ? list[e] : e) / A.a_div; };  // (e < cnt)
+  // ---- staging: thread -> its pieces of a stage (a row past the count reads zeros) ----
+  int c_off[R], b_off[RB_N];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int idx = tid + k * nthreads, e = base + (idx >> 4) % TT;
+    c_off[k] = e < cnt ? arow_of(e) * n + (idx & 15) * 16 : HYD_OOB;
+  }
+#pragma unroll
+  for (int k = 0; k < RB_N; ++k) {
+    const int idx = tid + k * nthreads, e = base + (idx >> 1) % TT;
+    b_off[k] = idx < BP && e < cnt ? arow_of(e) * (n >> 4) * 2 + (idx & 1) * 16 : HYD_OOB;
+  }
+  const int d_off = (tid < TT && base + tid < cnt) ? arow_of(base + tid) * nb * 4 : HYD_OOB;
+  struct Stage { u32x4 c[R], bs[RB_N]; u32 d0, d1; };
+  auto request = [&](Stage& G, int b0) {  // (blocks past the row's end: some other row's values, never multiplied)
+#pragma unroll
+    for (int k = 0; k < R; ++k) G.c[k] = __builtin_amdgcn_raw_buffer_load_b128(RA, c_off[k], (b0 + (tid + k * nthreads) / (TT * 16)) * 256, 0);
+#pragma unroll
+    for (int k = 0; k < RB_N; ++k)
+      if (tid + k * nthreads < BP) G.bs[k] = __builtin_amdgcn_raw_buffer_load_b128(RB, b_off[k], (b0 + (tid + k * nthreads) / (TT * 2)) * 32, 0);
+    if (tid < TT) {
+      G.d0 = __builtin_amdgcn_raw_buffer_load_b32(RD, d_off, b0 * 4, 0);
+      G.d1 = __builtin_amdgcn_raw_buffer_load_b32(RD, d_off, b0 * 4 + 4, 0);
+    }
+  };
+  auto write = [&](const Stage& G, uint8_t* buf) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int idx = tid + k * nthreads;
+      *reinterpret_cast<u32x4*>(buf + (idx >> 4) * HYD16_TOK_B + (idx & 15) * 16) = G.c[k];
+    }
+#pragma unroll
+    for (int k = 0; k < RB_N; ++k) {  // the sums become the min term's operand words ONCE per workgroup, not per wave and block
+      const int idx = tid + k * nthreads;
+      if (idx < BP) {
+        const u32 w[4] = {G.bs[k].x, G.bs[k].y, G.bs[k].z, G.bs[k].w};  // 8 sums: groups 2 p, 2 p + 1 of piece p
+        uint8_t* at = buf + HYD16_SB * TT * HYD16_TOK_B + (idx >> 1) * 64 + (idx & 1) * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // sub-block kg' = i of both groups
+          const int sh = 16 * (i & 1);
+          const u32x2_t v = {hyd16_split((int)(short)((w[i >> 1] >> sh) & 0xFFFFu)), hyd16_split((int)(short)((w[2 + (i >> 1)] >> sh) & 0xFFFFu))};
+          *reinterpret_cast<u32x2_t*>(at + 16 * i) = v;
+        }
+      }
+    }
+    if (tid < TT) {
+      float* dl = reinterpret_cast<float*>(buf + D_LDS);
+      dl[tid] = u2f(G.d0);
+      dl[TT + tid] = u2f(G.d1);
+    }
+  };
+  // The loop has no branch around a load, and a tile's loads go into the registers that its predecessor was just expanded out of: what is on its way
+  // at the end of a stage stays on its way.  (Loads under conditions cost a wait for all of them and ~40 moves per stage.)  Past the
+  // row's end the last block is loaded again, and a wave without a strip multiplies strip 0: neither is used.
+  HydTile T[HYD16_SB];
+#pragma unroll
+  for (int u = 0; u < HYD16_SB; ++u) hyd_tile_load(T[u], W, lane, min(u, nb - 1) * TILE_B);
+  Stage G;
+  request(G, 0);
+  write(G, lds);
+  __syncthreads();
+  float S[MT][4][4], ad[SEG4 ? MT : 1][4][4], am[SEG4 ? MT : 1][4][4];  // [token group][token of the lane's four][sub-block group]
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        S[t][r][g] = 0.f;
+        if (SEG4) ad[t][r][g] = am[t][r][g] = 0.f;
+      }
+  auto item_end = [&]() {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          S[t][r][g] += ad[t][r][g] - am[t][r][g];
+          ad[t][r][g] = am[t][r][g] = 0.f;
+        }
+  };
+  auto block = [&](int u, int b, const uint8_t* cur) {
+    Hyd16W E;
+    hyd16_weights(T[u], kgp, E);
+    const float d = h2f(T[u].dm & 0xffff), dmin = h2f(T[u].dm >> 16);
+    hyd_tile_load(T[u], W, lane, min(b + HYD16_SB, nb - 1) * TILE_B);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const uint8_t* cb = cur + (u * TT + t * 16 + tl) * HYD16_TOK_B + 16 * kgp;
+      i32x4 a[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) a[g] = *reinterpret_cast<const i32x4*>(cb + 64 * g);
+      const u32x4 dig = *reinterpret_cast<const u32x4*>(cur + HYD16_SB * TT * HYD16_TOK_B + (u * TT + t * 16 + tl) * 64 + 16 * kgp);
+      const f32x4 dx = *reinterpret_cast<const f32x4*>(cur + D_LDS + (u * TT + t * 16 + 4 * q) * 4);
+      const i32x4 z = {0, 0, 0, 0};
+      const i64x1 dig01 = __builtin_bit_cast(i64x1, (u32x2_t{dig.x, dig.y})), dig23 = __builtin_bit_cast(i64x1, (u32x2_t{dig.z, dig.w}));
+      i32x4 D[4], M[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        D[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], E.B[g], z, 0, 0, 0);
+        M[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8((g >> 1) ? dig23 : dig01, __builtin_bit_cast(i64x1, E.m[g]), z, 0, 0, 0);
+      }
+      const float dxr[4] = {dx.x, dx.y, dx.z, dx.w};
+      float dd[4], dmn[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) { dd[r] = dxr[r] * d; dmn[r] = dxr[r] * dmin; }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int Dr[4] = {D[g].x, D[g].y, D[g].z, D[g].w}, Mr[4] = {M[g].x, M[g].y, M[g].z, M[g].w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (SEG4) {
+            ad[t][r][g] = fmaf(dd[r], (float)Dr[r], ad[t][r][g]);
+            am[t][r][g] = fmaf(dmn[r], (float)Mr[r], am[t][r][g]);
+          } else {
+            S[t][r][g] += hyd16_item1(dd[r], (float)Dr[r], dmn[r], (float)Mr[r]);
+          }
+        }
+      }
+    }
+  };
+  int b0 = 0;
+  for (; b0 + HYD16_SB <= nb; b0 += HYD16_SB) {
+    uint8_t* cur = lds + ((b0 / HYD16_SB) & 1) * STAGE;
+    uint8_t* nxt = lds + (((b0 / HYD16_SB) & 1) ^ 1) * STAGE;
+    request(G, min(b0 + HYD16_SB, nb - 1));
+    block(0, b0, cur);
+    block(1, b0 + 1, cur);
+    if (SEG4 && (b0 & 2)) item_end();
+    write(G, nxt);
+    lds_barrier();  // (also in front of the next pass's first stage: every wave is done with both buffers)
+  }
+  if (b0 < nb) block(0, b0, lds + ((b0 / HYD16_SB) & 1) * STAGE);
+  if (nb & 1) __syncthreads();
+  if (SEG4 && (nb & 3)) item_end();
+  const int row = strip * 16 + rown;
+  float* meet = reinterpret_cast<float*>(lds) + (size_t)(wave >> 1) * MT * 4 * 64 + lane;  // GLU: the w3 waves' values
+  if (GLU) {
+    if (wave & 1) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) meet[(t * 4 + r) * 64] = (S[t][r][0] + S[t][r][1]) + (S[t][r][2] + S[t][r][3]);
+    }
+    __syncthreads();
+  }
+  if (live && row < A.rows && !(GLU && (wave & 1))) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int eD = base + t * 16 + 4 * q + r;
+        if (eD < cnt) {
+          const int vD = list ? list[eD] : eD;
+          float* o = A.out + (size_t)vD * A.out_stride + row;
+          const float v = (S[t][r][0] + S[t][r][1]) + (S[t][r][2] + S[t][r][3]);  // tile_strip_value
+          if (GLU) *o = act_fn(v, A.act) * meet[(t * 4 + r) * 64];                 // src/infer.cpp:859-872
+          else if (A.epilogue == EPI_ADD) *o += v;                                 // src/infer.cpp:832-834, 928-930
+          else *o = v;
+        }
+      }
+  }
+  if (GLU) __syncthreads();  // (the next pass stages where the values met)
+}
+// Plain matrices: blockIdx.x = strip group, blockIdx.y = the chunk of 16 MT tokens.  Expert stacks (A.n_experts > 0: the task's rows come
+// through its list, src/infer.cpp:853-878): blockIdx.x = task x strip groups, the workgroup walks the task's rows 16 MT at a time (a
+// launch may be restricted to tasks with a row count in [cnt_min, cnt_max]: the few-row tasks stay with hyd_gemm_kernel's quads).
+template <bool GLU, bool SEG4, int NW, int MT>
+__global__ __launch_bounds__(64 * NW, 2) void hyd_gemm16_kernel(const HydGemmArgs A) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // 2 x hyd16_stage_b
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  constexpr int SG = GLU ? NW / 2 : NW;  // strips per workgroup
   const int strips = (A.rows + 15) >> 4;
-  const int groups = (strips + nwaves - 1) / nwaves;
+  const int groups = (strips + SG - 1) / SG;
   const int task = A.n_experts > 0 ? (int)blockIdx.x / groups : 0;
   const int group = (int)blockIdx.x - task * groups;
   const int cnt = A.count ? __builtin_amdgcn_readfirstlane(A.count[task]) : A.m;
   if (cnt <= 0 || cnt < A.cnt_min || (A.cnt_max > 0 && cnt > A.cnt_max)) return;
   const int* list = A.list ? A.list + (size_t)task * A.list_stride : nullptr;
-  const int strip = group * nwaves + wave;
+  const int strip = group * SG + (GLU ? wave >> 1 : wave);
   const bool live = strip < strips;  // (a wave without a strip still stages and keeps the barriers)
   const int n = A.n, nb = n >> 8;
   const size_t woff = (size_t)task * A.e_bytes + (size_t)(live ? strip : 0) * nb * TILE_B;
-  const rsrc_t W1 = make_rsrc(A.W + woff);
-  const rsrc_t W3 = make_rsrc(GLU ? A.W3 + woff : A.W + woff);
-  const bool seg4 = nb > 8;  // tile_seg
+  const rsrc_t W = make_rsrc((GLU && (wave & 1) ? A.W3 : A.W) + woff);
   const rsrc_t RA = make_rsrc_n(A.a_qs, (u32)((size_t)A.a_rows * n));
   const rsrc_t RB = make_rsrc_n(A.a_bsums, (u32)((size_t)A.a_rows * (n >> 4) * 2));
   const rsrc_t RD = make_rsrc_n(A.a_d, (u32)((size_t)A.a_rows * nb * 4));
-  const int kgp = lane >> 4, tl = lane & 15;   // operand side: token tl of the chunk, K-group kg'
-  const int q = lane >> 4, rown = lane & 15;   // result side: tokens 4 q .. 4 q + 3, row rown of the strip
-  auto c_sb = [&](int k) { return (tid + k * nthreads) >> 8; };
-  auto c_lds = [&](int k) { const int idx = tid + k * nthreads; return ((idx >> 8) * 16 + ((idx >> 4) & 15)) * HYD16_TOK_B + (idx & 15) * 16; };
-  const int b_sb = tid >> 5, b_t = (tid >> 1) & 15, b_piece = tid & 1;
-  const int b_lds = HYD16_SB * 16 * HYD16_TOK_B + (b_sb * 16 + b_t) * 64 + b_piece * 32;   // (8 sums -> 8 digit words)
-  const int d_lds = HYD16_SB * (16 * HYD16_TOK_B + 16 * 64);
-  auto arow_of = [&](int e) { return (list ? list[e] : e) / A.a_div; };  // (e < cnt)
-  for (int base = (int)blockIdx.y * 16; base < cnt; base += (int)gridDim.y * 16) {
-    // ---- staging: thread -> its pieces of a stage (wave-uniform loop bounds; a row past the count reads zeros) ----
-    // codes: HYD16_SB x 16 tokens x 16 pieces of 16 bytes; sums: HYD16_SB x 16 x 2 pieces; scales: 16 tokens x (HYD16_SB floats = 16 bytes)
-    int c_off[R];
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      const int idx = tid + k * nthreads;
-      const int t = (idx >> 4) & 15, piece = idx & 15;
-      const int e = base + t;
-      c_off[k] = e < cnt ? arow_of(e) * n + piece * 16 : HYD_OOB;
-    }
-    const int b_off = (base + b_t < cnt) ? arow_of(base + b_t) * (n >> 4) * 2 + b_piece * 16 : HYD_OOB;
-    const int d_off = (tid < 16 && base + tid < cnt) ? arow_of(base + tid) * nb * 4 : HYD_OOB;
-    auto stage_request = [&](Hyd16Stage<R>& G, int b0) {
-#pragma unroll
-      for (int k = 0; k < R; ++k) G.c[k] = __builtin_amdgcn_raw_buffer_load_b128(RA, c_off[k], (b0 + c_sb(k)) * 256, 0);
-      if (tid < HYD16_SB * 32) G.bs = __builtin_amdgcn_raw_buffer_load_b128(RB, b_off, (b0 + b_sb) * 32, 0);
-      if (tid < 16) {  // the token's scales of blocks b0 .. b0 + 3 (past the row's end: never multiplied)
-        G.d.x = __builtin_amdgcn_raw_buffer_load_b32(RD, d_off, (b0 + 0) * 4, 0);
-        G.d.y = b0 + 1 < nb ? __builtin_amdgcn_raw_buffer_load_b32(RD, d_off, (b0 + 1) * 4, 0) : 0u;
-        G.d.z = b0 + 2 < nb ? __builtin_amdgcn_raw_buffer_load_b32(RD, d_off, (b0 + 2) * 4, 0) : 0u;
-        G.d.w = b0 + 3 < nb ? __builtin_amdgcn_raw_buffer_load_b32(RD, d_off, (b0 + 3) * 4, 0) : 0u;
-      }
-    };
-    auto stage_write = [&](const Hyd16Stage<R>& G, uint8_t* buf) {
-#pragma unroll
-      for (int k = 0; k < R; ++k) *reinterpret_cast<u32x4*>(buf + c_lds(k)) = G.c[k];
-      if (tid < HYD16_SB * 32) {  // the sums go to LDS as the min term's operand words: split ONCE per workgroup, not per wave and block
-        const u32 w[4] = {G.bs.x, G.bs.y, G.bs.z, G.bs.w};
-        u32x4 lo, hi;
-        lo.x = hyd16_split((int)(short)(w[0] & 0xFFFFu)); lo.y = hyd16_split((int)(short)(w[0] >> 16));
-        lo.z = hyd16_split((int)(short)(w[1] & 0xFFFFu)); lo.w = hyd16_split((int)(short)(w[1] >> 16));
-        hi.x = hyd16_split((int)(short)(w[2] & 0xFFFFu)); hi.y = hyd16_split((int)(short)(w[2] >> 16));
-        hi.z = hyd16_split((int)(short)(w[3] & 0xFFFFu)); hi.w = hyd16_split((int)(short)(w[3] >> 16));
-        *reinterpret_cast<u32x4*>(buf + b_lds) = lo;
-        *reinterpret_cast<u32x4*>(buf + b_lds + 16) = hi;
-      }
-      if (tid < 16) {
-        float* dl = reinterpret_cast<float*>(buf + d_lds);
-        dl[0 * 16 + tid] = u2f(G.d.x); dl[1 * 16 + tid] = u2f(G.d.y); dl[2 * 16 + tid] = u2f(G.d.z); dl[3 * 16 + tid] = u2f(G.d.w);
-      }
-    };
-    HydTile T1, T3, N1, N3;
-    if (live) {  // (a further pass over the same strip: L2 hits)
-      hyd_tile_load(T1, W1, lane, 0);
-      if (GLU) hyd_tile_load(T3, W3, lane, 0);
-      if (nb > 1) {
-        hyd_tile_load(N1, W1, lane, TILE_B);
-        if (GLU) hyd_tile_load(N3, W3, lane, TILE_B);
-      }
-    }
-    Hyd16Stage<R> G;
-    stage_request(G, 0);
-    stage_write(G, lds);
-    __syncthreads();
-    Hyd16Acc acc1, acc3;
-    hyd16_acc_zero(acc1);
-    if (GLU) hyd16_acc_zero(acc3);
-    for (int b0 = 0; b0 < nb; b0 += HYD16_SB) {
-      uint8_t* cur = lds + ((b0 / HYD16_SB) & 1) * HYD16_STAGE_B;
-      uint8_t* nxt = lds + (((b0 / HYD16_SB) & 1) ^ 1) * HYD16_STAGE_B;
-      const bool more = b0 + HYD16_SB < nb;
-      if (more) stage_request(G, b0 + HYD16_SB);
-      if (live) {
-#pragma unroll
-        for (int u = 0; u < HYD16_SB; ++u) {
-          const int b = b0 + u;
-          if (b < nb) {
-            HydTile M1, M3;
-            if (b + 2 < nb) {
-              hyd_tile_load(M1, W1, lane, (b + 2) * TILE_B);
-              if (GLU) hyd_tile_load(M3, W3, lane, (b + 2) * TILE_B);
-            }
-            Hyd16Act X;
-            const uint8_t* cb = cur + (u * 16 + tl) * HYD16_TOK_B + 16 * kgp;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) X.a[g] = *reinterpret_cast<const i32x4*>(cb + 64 * g);
-            const i32x4 am4 = *reinterpret_cast<const i32x4*>(cur + HYD16_SB * 16 * HYD16_TOK_B + (u * 16 + tl) * 64 + 16 * kgp);
-            const f32x4 dq = *reinterpret_cast<const f32x4*>(cur + d_lds + (u * 16 + 4 * q) * 4);
-            X.dx[0] = dq.x; X.dx[1] = dq.y; X.dx[2] = dq.z; X.dx[3] = dq.w;
-            const bool item_end = !seg4 || (b & 3) == 3 || b == nb - 1;
-            i32x4 B[4], Bm;
-            hyd16_expand(T1, kgp, B, Bm);
-            hyd16_block_d(T1, B, Bm, X, am4, kgp, acc1);
-            if (item_end) hyd16_item_end(acc1);
-            if (GLU) {
-              hyd16_expand(T3, kgp, B, Bm);
-              hyd16_block_d(T3, B, Bm, X, am4, kgp, acc3);
-              if (item_end) hyd16_item_end(acc3);
-            }
-            T1 = N1; N1 = M1;
-            if (GLU) { T3 = N3; N3 = M3; }
-          }
-        }
-      }
-      if (more) stage_write(G, nxt);
-      __syncthreads();  // (also in front of the next chunk's first stage: every wave is done with both buffers)
-    }
-    if (live) {
-      const int row = strip * 16 + rown;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int eD = base + 4 * q + r;
-        if (eD < cnt && row < A.rows) {
-          const int vD = list ? list[eD] : eD;
-          float* o = A.out + (size_t)vD * A.out_stride + row;
-          const float v = hyd16_value(acc1, r);
-          if (GLU) *o = act_fn(v, A.act) * hyd16_value(acc3, r);   // src/infer.cpp:859-872
-          else if (A.epilogue == EPI_ADD) *o += v;                  // src/infer.cpp:832-834, 928-930
-          else *o = v;
-        }
-      }
-    }
+  for (int base = (int)blockIdx.y * 16 * MT; base < cnt; base += (int)gridDim.y * 16 * MT) {
+    if (MT > 1 && cnt - base > 16) hyd16_pass<GLU, SEG4, NW, MT>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
+    else hyd16_pass<GLU, SEG4, NW, 1>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
   }
 }
 
@@ -652,6 +747,11 @@ __global__ __launch_bounds__(512) void hyd_gemm16k_kernel(const HydGemmArgs A) {
   }
 }
 
+template <bool GLU, int NW, int MT>
+static void hyd_gemm16_launch(hipStream_t st, dim3 grid, const HydGemmArgs& A) {
+  if (A.n > 8 * 256) hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, true, NW, MT>), grid, dim3(64 * NW), 2 * hyd16_stage_b<MT>(), st, A);
+  else hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, false, NW, MT>), grid, dim3(64 * NW), 2 * hyd16_stage_b<MT>(), st, A);
+}
 template <bool GLU, int NQ>
 static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
   const long long units = (long long)(A.n_experts > 0 ? A.n_experts : 1) * ((A.rows + 15) >> 4);
@@ -661,9 +761,9 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
     HydGemmArgs B = A;
     B.cnt_min = HYD16_EXPERT_MIN;
     const int strips = (A.rows + 15) >> 4;
-    constexpr int NW = GLU ? 4 : 8;
-    const int groups = (strips + NW - 1) / NW;
-    hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, NW>), dim3((unsigned)(A.n_experts * groups), 1u), dim3(64 * NW), 2 * HYD16_STAGE_B, st, B);
+    constexpr int SG = GLU ? 4 : 8;
+    const int groups = (strips + SG - 1) / SG;
+    hyd_gemm16_launch<GLU, 8, 2>(st, dim3((unsigned)(A.n_experts * groups), 1u), B);
     HydGemmArgs C = A;
     C.cnt_max = HYD16_EXPERT_MIN - 1;
     if (C.a_dig) hipLaunchKernelGGL((hyd_gemm_kernel<GLU, NQ, false, true>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, st, C);
@@ -680,14 +780,20 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
       hipLaunchKernelGGL((hyd_gemm16k_kernel<GLU>), dim3((unsigned)units, (unsigned)chunks), dim3(64 * ips_), lds_k, st, A);
       return;
     }
-    // strips per workgroup: as many as still give most CUs a workgroup (the staging is paid once per workgroup, and every choice
-    // puts the same number of waves on the chip); at least 2 (the staging indices assume >= 128 threads)
-    int nw = GLU ? 4 : 8;
-    while (nw > 2 && ((units + nw - 1) / nw) * chunks < 192) nw >>= 1;
-    const dim3 grid((unsigned)((units + nw - 1) / nw), (unsigned)chunks);
-    if (nw == 8) hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, 8>), grid, dim3(512), 2 * HYD16_STAGE_B, st, A);
-    else if (nw == 4) hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, 4>), grid, dim3(256), 2 * HYD16_STAGE_B, st, A);
-    else hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, 2>), grid, dim3(128), 2 * HYD16_STAGE_B, st, A);
+    // 32 tokens a pass where that leaves most CUs a workgroup, else 16; then as many strips per workgroup as still do (the staging is paid once
+    // per workgroup, and every choice puts the same number of waves on the chip); at least 2 waves (the staging indices assume >= 128 threads)
+    const int per = GLU ? 2 : 1, chunks2 = (A.m + 31) / 32;
+    auto groups = [&](int nw) { return (unsigned)((units * per + nw - 1) / nw); };
+    if (A.m > 16 && (long long)groups(8) * chunks2 >= 192) {
+      hyd_gemm16_launch<GLU, 8, 2>(st, dim3(groups(8), (unsigned)chunks2), A);
+      return;
+    }
+    int nw = 8;
+    while (nw > 2 && (long long)groups(nw) * chunks < 192) nw >>= 1;
+    const dim3 grid(groups(nw), (unsigned)chunks);
+    if (nw == 8) hyd_gemm16_launch<GLU, 8, 1>(st, grid, A);
+    else if (nw == 4) hyd_gemm16_launch<GLU, 4, 1>(st, grid, A);
+    else hyd_gemm16_launch<GLU, 2, 1>(st, grid, A);
     return;
   }
   // plain matrices with more rows of activations than one wave takes per pass: the waves of a workgroup share a strip

@@ -1,0 +1,29 @@
+"""The batched prompt path's products at row lengths of an odd number of blocks and at both sides of its groups of 16 and 32 tokens: the per-token
+loop's bits (option q2k_tiles = 2), like tests/test_hydrate_gpu.py."""
+import numpy as np
+import pytest
+
+from tests.test_hydrate_gpu import _assert_identical, compare_hydrate
+from tools import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import dsk
+    c = dsk.Ctx(0)
+    yield c
+    c.close()
+
+
+# blocks per row: model width 3 or 11, dense hidden vectors 11 or 13 (items of 4 blocks, a last one of 3 or 1), experts' 3, wo 1; experts
+# 4 of 6: most tasks have more than 16 rows, their last pass from 1 to 32
+@pytest.mark.parametrize("dim,hidden", [(768, 2816), (2816, 3328)])
+@pytest.mark.parametrize("P", [12, 31, 32, 33, 49, 65])
+def test_odd_rows_of_blocks(ctx, dim, hidden, P):
+    c = synth.preset("tiny_v3", "q2_k", False, dim=dim, hidden_dim=hidden, moe_intermediate_size=768, n_routed_experts=6, n_group=2, topk_group=3,
+                     vocab_size=512, max_seq_len=96)
+    T = synth.synth_model(c, seed=83)
+    tokens = np.random.default_rng(P).integers(0, c.vocab_size, P)
+    _assert_identical(compare_hydrate(ctx, c, T, tokens=tokens, pos0=1), P, 1)
