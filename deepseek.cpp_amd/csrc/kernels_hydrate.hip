@@ -1019,6 +1019,202 @@ __global__ __launch_bounds__(1024, 8) void hyd_attn_kernel(const AttnMhaArgs a, 
   if (tid < vd) out[(size_t)p * out_stride + (size_t)h * vd + tid] = o;
   }
 }
+// The same attention for 16 tokens of a head at a time, on the matrix pipe: v_mfma_f32_16x16x1_4b_f32 is 4 x 16 x 16 independent f32 FMAs
+// (round to nearest, subnormals kept), so a chain of them IS the chain of fmaf() of attn_mha_body, and what is left is to keep its trees:
+//   scores   lane sl of a position's 16 sums dimensions 64 j + 4 sl + i in the order (j, i), then the lanes meet pairwise.  Block b of the
+//            instruction takes the lanes 4 b + s, one accumulator per s: a lane of the result holds all 16 partial sums of its pairs.
+//   softmax  the maximum; sums of 64 positions by wave_sum_dpp, added in order; a division each
+//   values   thread group g of 4096 / v_dim sums positions g, g + 32, ... in order and the groups are added in order: block b takes group
+//            4 G + b, G in turn.  Positions behind a token's context are left out by selection, not by a weight of zero: they may hold anything.
+// Same bits as hyd_attn_kernel, which reads a head's keys and values once per token and is bound by the round trips of 16-wave workgroups:
+// 512 tokens of DeepSeek-V3's 128 heads 1180 -> 327 us.  4 waves: key tiles in turn, then 4 tokens' softmax each, then 32 value columns each.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+enum { HYD_AT = 16, HYD_AT_MAX_KV = 1024, HYD_AT_V = 128, HYD_AT_NJ = 3 };  // tokens; contexts of one position per softmax thread; v_dim; head_dim <= 64 NJ
+__host__ DEV int hyd_at_row(int max_kv) { return (max_kv + 63) / 64 * 64 + 4; }  // floats of a token's weights in LDS: 16 tokens x 4 positions meet 64 banks
+__global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs a, const StepParams* __restrict__ sps, const float* __restrict__ q, int q_stride,
+                                                               float* __restrict__ out, int out_stride, int n_tok, int max_kv) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ __attribute__((aligned(16))) float q_s[HYD_AT][64 * HYD_AT_NJ + 4];
+  float* att = reinterpret_cast<float*>(smem);
+  const int TP = hyd_at_row(max_kv);
+  // a head's tokens on one XCD, the longest contexts first (hyd_attn_kernel)
+  const int tiles = (n_tok + HYD_AT - 1) / HYD_AT;
+  int h, tile;
+  if (a.n_heads % 8 == 0) {
+    const int xcd = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
+    h = j / tiles * 8 + xcd;
+    tile = j % tiles;
+  } else {
+    h = (int)blockIdx.x / tiles;
+    tile = (int)blockIdx.x % tiles;
+  }
+  const int p0 = (tiles - 1 - tile) * HYD_AT;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, b = lane >> 4;  // operand side: row (token, key or value column) n, block b; result side: column n, tokens 4 b ..
+  const int hd = a.head_dim, nope = a.nope, rope = a.rope, H = a.n_heads;
+  auto token = [&](int r) { return min(p0 + r, n_tok - 1); };  // (rows past the end repeat the last token and are not stored)
+  for (int i = tid; i < HYD_AT * 64 * HYD_AT_NJ; i += 256) {
+    const int r = i / (64 * HYD_AT_NJ), d = i - r * (64 * HYD_AT_NJ);
+    q_s[r][d] = d < hd ? q[(size_t)token(r) * q_stride + (size_t)h * hd + d] : 0.f;
+  }
+  __syncthreads();
+  // rope_kv_from_lds, the query part: 16 threads a token
+  float re[4], im[4];
+  const int rr = tid >> 4, half = rope >> 1;  // (rope <= 128)
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = (tid & 15) + 16 * k;
+    if (i < half) {
+      const float* cs = sps[token(rr)].rope_cs;
+      ad::rope_rot(q_s[rr][nope + 2 * i], q_s[rr][nope + 2 * i + 1], cs[2 * i], cs[2 * i + 1], re[k], im[k]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = (tid & 15) + 16 * k;
+    if (i < half) {
+      q_s[rr][a.is_v3 ? nope + 2 * i : nope + i] = re[k];
+      q_s[rr][a.is_v3 ? nope + 2 * i + 1 : nope + i + half] = im[k];
+    }
+  }
+  __syncthreads();
+  float qv[HYD_AT_NJ][16];
+#pragma unroll
+  for (int j = 0; j < HYD_AT_NJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&q_s[n][64 * j + 16 * b + 4 * i]);
+      qv[j][4 * i] = v.x; qv[j][4 * i + 1] = v.y; qv[j][4 * i + 2] = v.z; qv[j][4 * i + 3] = v.w;
+    }
+  int len[4];  // contexts of this lane's tokens on the result side
+#pragma unroll
+  for (int r = 0; r < 4; ++r) len[r] = sps[token(4 * b + r)].kv_len;
+  const int most = sps[token(HYD_AT - 1)].kv_len, least = sps[p0].kv_len;  // (ascending)
+  const float inv = sqrtf((float)hd);
+  typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+  struct Keys { f16x8 k[HYD_AT_NJ][2]; };
+  auto keys = [&](int t0, Keys& o) {
+    const uint16_t* row = a.key_cache + ((size_t)min(t0 + n, most - 1) * H + h) * hd + 16 * b;
+#pragma unroll
+    for (int j = 0; j < HYD_AT_NJ; ++j)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) o.k[j][u] = 64 * j + 16 * b < hd ? *reinterpret_cast<const f16x8*>(row + 64 * j + 8 * u) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  };
+  Keys K;
+  keys(wave * 16, K);
+  for (int t0 = wave * 16; t0 < most; t0 += 64) {
+    Keys N;
+    keys(t0 + 64, N);
+    f32x16 acc[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[s][i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < HYD_AT_NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[j][4 * s + i], (float)K.k[j][s >> 1][4 * (s & 1) + i], acc[s], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float quad[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) quad[u] = (acc[0][4 * u + r] + acc[1][4 * u + r]) + (acc[2][4 * u + r] + acc[3][4 * u + r]);  // row16_sum
+      const float p = (quad[0] + quad[1]) + (quad[2] + quad[3]);
+      att[(4 * b + r) * TP + t0 + n] = p / inv;
+    }
+    K = N;
+  }
+  __syncthreads();
+  // softmax, src/infer.cpp:472-487
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = wave * 4 + u, L = sps[token(r)].kv_len;
+    float* w = att + r * TP;
+    float mx = -INFINITY;
+    for (int t = lane; t < L; t += 64) mx = fmaxf(mx, w[t]);
+    mx = ad::wave_max_dpp(mx);
+    float sum = 0.f;
+    for (int t0 = 0; t0 < L; t0 += 64) {
+      const float e = t0 + lane < L ? expf(w[t0 + lane] - mx) : 0.f;
+      if (t0 + lane < L) w[t0 + lane] = e;
+      sum += ad::wave_sum_dpp(e);
+    }
+    for (int t = lane; t < L; t += 64) w[t] = w[t] / sum;
+  }
+  __syncthreads();
+  // values: columns 32 wave + 2 n + {0, 1}; the groups 4 G + b, two values of G at a time
+  const uint16_t* vc = a.value_cache + (size_t)h * HYD_AT_V + 32 * wave + 2 * n;
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  float o[4][2];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r][0] = o[r][1] = 0.f;
+  const int whole = least / 32, steps = (most + 31) / 32;  // steps that every token has all positions of; all steps
+#pragma unroll 1
+  for (int G = 0; G < 8; G += 2) {
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[u][c][i] = 0.f;
+    const int t0 = 4 * G + b;  // (and t0 + 4)
+    auto load = [&](int step, int u) { return *reinterpret_cast<const f16x2*>(vc + (size_t)min(32 * step + t0 + 4 * u, most - 1) * H * HYD_AT_V); };
+    f16x2 v[4][2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) v[k][u] = load(k, u);
+    int step = 0;
+    for (; step + 4 <= whole; step += 4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        f16x2 now[2] = {v[k][0], v[k][1]};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) v[k][u] = load(step + k + 4, u);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const float w = att[n * TP + 32 * (step + k) + t0 + 4 * u];
+          acc[u][0] = __builtin_amdgcn_mfma_f32_16x16x1f32(w, (float)now[u].x, acc[u][0], 0, 0, 0);
+          acc[u][1] = __builtin_amdgcn_mfma_f32_16x16x1f32(w, (float)now[u].y, acc[u][1], 0, 0, 0);
+        }
+      }
+    }
+    for (; step < steps; ++step) {
+      const f16x2 now[2] = {load(step, 0), load(step, 1)};
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float w = att[n * TP + min(32 * step + t0 + 4 * u, TP - 1)];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const f32x16 next = __builtin_amdgcn_mfma_f32_16x16x1f32(w, (float)now[u][c], acc[u][c], 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[u][c][4 * k + r] = 32 * step + 4 * (G + u) + k < len[r] ? next[4 * k + r] : acc[u][c][4 * k + r];
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) o[r][c] += acc[u][c][4 * k + r];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (p0 + 4 * b + r < n_tok) {
+      float* to = out + (size_t)(p0 + 4 * b + r) * out_stride + (size_t)h * HYD_AT_V + 32 * wave + 2 * n;
+      to[0] = o[r][0];
+      to[1] = o[r][1];
+    }
+}
 int launch_hyd_kv_write(hipStream_t st, const AttnMhaArgs& a, const StepParams* sps, int P, const float* kv_b, int kvb_stride, const float* kv_a, int kva_stride) {
   hipLaunchKernelGGL(hyd_kv_write_kernel, dim3(a.n_heads, P), dim3(256), 0, st, a, sps, kv_b, kvb_stride, kv_a, kva_stride);
   return DSK_OK;
@@ -1029,6 +1225,16 @@ int launch_hyd_attn(hipStream_t st, const AttnMhaArgs& a, const StepParams* sps,
   if (lds > 96 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_attn: kv_len %d does not fit LDS", max_kv);
   if (a.head_dim > 256 || a.v_dim > 256) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_attn: head_dim %d / v_head_dim %d", a.head_dim, a.v_dim);
   if (n_split > MHA_SPLIT_MAX) n_split = MHA_SPLIT_MAX;  // (launch_head_attn's clamp)
+  // 16 tokens at a time while a context is one softmax and one position a thread (the chunk's contexts are max_kv - P + 1 ... max_kv)
+  const int limit = std::min((int)HYD_AT_MAX_KV, n_split > 1 ? split_min - 1 : max_kv);
+  const int n_tile = std::max(0, std::min(P, P - (max_kv - limit)));
+  if (n_tile >= 8 && a.v_dim == HYD_AT_V && a.head_dim % 16 == 0 && a.head_dim <= 64 * HYD_AT_NJ && a.rope <= 128) {
+    const int kv = max_kv - (P - n_tile), bytes = HYD_AT * hyd_at_row(kv) * 4;
+    if (bytes > 48 * 1024) hipFuncSetAttribute((const void*)hyd_attn_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    hipLaunchKernelGGL(hyd_attn_tile_kernel, dim3(a.n_heads * ((n_tile + HYD_AT - 1) / HYD_AT)), dim3(256), bytes, st, a, sps, q, q_stride, out, out_stride, n_tile, kv);
+    if (n_tile == P) return DSK_OK;
+    sps += n_tile; q += (size_t)n_tile * q_stride; out += (size_t)n_tile * out_stride; P -= n_tile;
+  }
   const bool split = n_split > 1 && max_kv >= split_min;
   auto k = split ? hyd_attn_kernel<true> : hyd_attn_kernel<false>;
   if (lds > 32 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -27,3 +27,12 @@ def test_odd_rows_of_blocks(ctx, dim, hidden, P):
     T = synth.synth_model(c, seed=83)
     tokens = np.random.default_rng(P).integers(0, c.vocab_size, P)
     _assert_identical(compare_hydrate(ctx, c, T, tokens=tokens, pos0=1), P, 1)
+
+
+# attention of 16 tokens at a time (from 8 tokens on, DeepSeek-V3's head sizes): full and ragged tiles of tokens, contexts that end at both sides of
+# 32 (a step of the values), 64 (a sum of the softmax) and of a tile of keys, a chunk that begins inside a context
+@pytest.mark.parametrize("P,pos0", [(7, 0), (8, 0), (9, 24), (17, 14), (31, 33), (40, 90)])
+def test_attention_of_token_tiles(ctx, P, pos0):
+    c = synth.preset("v3", "q2_k", False, n_layers=1, first_k_dense_replace=1, max_seq_len=192, vocab_size=1024)
+    tokens = np.random.default_rng(P).integers(0, c.vocab_size, P)
+    _assert_identical(compare_hydrate(ctx, c, None, seed=23, tokens=tokens, pos0=pos0), P, pos0)
