@@ -1519,6 +1519,76 @@ __global__ __launch_bounds__(1024) void hyd_router_rows_kernel(const float* __re
     }
   }
 }
+// The same rows for 16 tokens x 16 NC rows a wave on the matrix pipe, as in hyd_attn_tile_kernel: lane 16 R + 4 b + s of router_body's wave is block b of
+// accumulator s in turn R, its chain runs over (k, i) as there, and the results meet in wave_sum_dpp's order.  Wave w = column slice w; the
+// slices meet in LDS, in slice order.  512 tokens x 256 rows of 7168: 275 us with a row's weights in registers and the tokens one by one -> 49 us; 77 tokens 46 -> 28 us.
+template <int SL, int NC>
+__global__ __launch_bounds__(64 * SL, 2) void hyd_router_tile_kernel(const float* __restrict__ W, const float* __restrict__ Y, int dim, int E, int P, float* __restrict__ partial) {
+  __shared__ float part_s[SL][16][16 * NC + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, b = lane >> 4;
+  const int p0 = (int)blockIdx.x * 16, r0 = (int)blockIdx.y * 16 * NC;
+  const int chunk = ((dim / 4 + SL - 1) / SL + 63) / 64 * 64 * 4;  // floats per column slice (router_body)
+  const int k0 = wave * chunk, k1 = min(dim, k0 + chunk);
+  const float* y = Y + (size_t)min(p0 + n, P - 1) * dim + 16 * b;  // (rows past the ends: any valid ones, not stored)
+  const float* w[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) w[c] = W + (size_t)min(r0 + 16 * c + n, E - 1) * dim + 16 * b;
+  float lo[NC][4], hi[NC][4];  // [row tile][token of the lane's four]: turns 0 + 1, turn 2
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) lo[c][r] = hi[c][r] = 0.f;
+#pragma unroll 1
+  for (int R = 0; R < 4; ++R) {
+    f32x16 acc[NC][4];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[c][s][i] = 0.f;
+#pragma unroll 1
+    for (int k = k0; k < k1; k += 256) {
+      f32x4 a[4], v[NC][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        a[s] = *reinterpret_cast<const f32x4*>(y + k + 64 * R + 4 * s);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c][s] = *reinterpret_cast<const f32x4*>(w[c] + k + 64 * R + 4 * s);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc[c][s] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[s][i], v[c][s][i], acc[c][s], 0, 0, 0);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float quad[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) quad[u] = (acc[c][0][4 * u + r] + acc[c][1][4 * u + r]) + (acc[c][2][4 * u + r] + acc[c][3][4 * u + r]);
+        const float v = (quad[0] + quad[1]) + (quad[2] + quad[3]);
+        if (R == 0) lo[c][r] = v;
+        else if (R == 1) lo[c][r] += v;
+        else if (R == 2) hi[c][r] = v;
+        else part_s[wave][4 * b + r][16 * c + n] = lo[c][r] + (hi[c][r] + v);
+      }
+  }
+  __syncthreads();
+  for (int i = tid; i < 256 * NC; i += 64 * SL) {
+    const int t = i / (16 * NC), row = i % (16 * NC);
+    if (p0 + t < P && r0 + row < E) {
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < SL; ++k) v += part_s[k][t][row];  // slice order, like router_body
+      partial[(size_t)(p0 + t) * E + r0 + row] = v;
+    }
+  }
+}
 __global__ __launch_bounds__(1024) void hyd_gate_kernel(const RouterArgs a, int K) {
   __shared__ __attribute__((aligned(16))) float s[512];
   __shared__ __attribute__((aligned(16))) int surv[256];
@@ -1551,7 +1621,13 @@ int launch_hyd_router(hipStream_t st, const RouterArgs& a, int P, float* Y) {
   const size_t lds = (size_t)P * 16 * 4;
   if (Y && a.norm_w && a.dim % 256 == 0 && chunk <= 2048 && lds <= 60 * 1024 && a.n_routed <= 1024) {
     hipLaunchKernelGGL(hyd_router_norm_kernel, dim3(P), dim3(1024), 0, st, a, Y);
-    if (RW == 2) hipLaunchKernelGGL(hyd_router_rows_kernel<2>, dim3((a.n_routed + 1) / 2), dim3(1024), lds, st, a.w, Y, a.dim, a.n_routed, P, a.partial);
+    // 32 rows a wave where that gives every CU a workgroup, 16 below; a few tokens alone: rows in registers
+    const int wide = (P + 15) / 16 * ((a.n_routed + 31) / 32) >= 256 ? 2 : 1;
+    const dim3 tiles((P + 15) / 16, (a.n_routed + 16 * wide - 1) / (16 * wide));
+    if (P >= 16) {
+      auto k = RW == 2 ? (wide == 2 ? hyd_router_tile_kernel<8, 2> : hyd_router_tile_kernel<8, 1>) : (wide == 2 ? hyd_router_tile_kernel<4, 2> : hyd_router_tile_kernel<4, 1>);
+      hipLaunchKernelGGL(k, tiles, dim3(64 * SL), 0, st, a.w, Y, a.dim, a.n_routed, P, a.partial);
+    } else if (RW == 2) hipLaunchKernelGGL(hyd_router_rows_kernel<2>, dim3((a.n_routed + 1) / 2), dim3(1024), lds, st, a.w, Y, a.dim, a.n_routed, P, a.partial);
     else hipLaunchKernelGGL(hyd_router_rows_kernel<4>, dim3((a.n_routed + 3) / 4), dim3(1024), lds, st, a.w, Y, a.dim, a.n_routed, P, a.partial);
     hipLaunchKernelGGL(hyd_gate_kernel, dim3(P), dim3(1024), 0, st, a, a.n_active);
     return DSK_OK;
