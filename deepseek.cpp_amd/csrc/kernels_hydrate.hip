@@ -1399,6 +1399,141 @@ __global__ __launch_bounds__(1024) void hyd_mla_attn_kernel(const AttnMlaArgs a,
     }
   }
 }
+// The same for 16 heads of a token at a time on the matrix pipe (hyd_attn_tile_kernel says how the chains and trees stay the per-token kernel's; the latent
+// rows are shared by all heads, so heads are the rows of the products and end at one context length).  77 tokens of DeepSeek-V3 (contexts to
+// 77): 184 -> 36 us a block.  4 waves: key tiles in turn, 4 heads' softmax each, 128 latent columns each.
+enum { HYD_ML_L = 512, HYD_ML_R = 64 };
+__global__ __launch_bounds__(256, 2) void hyd_mla_attn_tile_kernel(const AttnMlaArgs a, const StepParams* __restrict__ sps, const float* __restrict__ q_c, int qc_stride,
+                                                                   const float* __restrict__ q_rope, int qr_stride, float* __restrict__ latent, int lat_stride, int max_kv) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr int NJ = (HYD_ML_L + HYD_ML_R) / 64;
+  __shared__ __attribute__((aligned(16))) float q_s[16][64 * NJ + 4];
+  float* att = reinterpret_cast<float*>(smem);
+  const int TP = hyd_at_row(max_kv);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, b = lane >> 4, h0 = (int)blockIdx.x * 16, p = blockIdx.y;
+  const StepParams* sp = sps + p;
+  const int rope = a.rope, L = sp->kv_len;
+  typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+  struct Keys { f16x8 k[NJ][2]; };
+  auto keys = [&](int t0, Keys& o) {
+    const size_t t = min(t0 + n, L - 1);
+    const uint16_t* c = a.nope_cache + t * HYD_ML_L + 16 * b;
+    const uint16_t* r = a.rope_cache + t * rope + 16 * b;
+#pragma unroll
+    for (int j = 0; j < NJ - 1; ++j)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) o.k[j][u] = *reinterpret_cast<const f16x8*>(c + 64 * j + 8 * u);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) o.k[NJ - 1][u] = 16 * b < rope ? *reinterpret_cast<const f16x8*>(r + 8 * u) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  };
+  Keys K;
+  keys(wave * 16, K);
+  for (int i = tid; i < 16 * (HYD_ML_L / 4); i += 256) {
+    const int r = i / (HYD_ML_L / 4), d = (i % (HYD_ML_L / 4)) * 4;
+    *reinterpret_cast<f32x4*>(&q_s[r][d]) = *reinterpret_cast<const f32x4*>(q_c + (size_t)p * qc_stride + (size_t)(h0 + r) * HYD_ML_L + d);
+  }
+  for (int i = tid; i < 16 * (HYD_ML_R / 2); i += 256) {  // rope part rotated (src/infer.cpp:1075-1084)
+    const int r = i / (HYD_ML_R / 2), k = i % (HYD_ML_R / 2);
+    float re = 0.f, im = 0.f;
+    if (k < rope / 2) {
+      const float* qr = q_rope + (size_t)p * qr_stride + (size_t)(h0 + r) * rope;
+      ad::rope_rot(qr[2 * k], qr[2 * k + 1], sp->rope_cs[2 * k], sp->rope_cs[2 * k + 1], re, im);
+    }
+    const bool pairs = a.is_v3 || k >= rope / 2;  // (past the rotated part: zeros)
+    q_s[r][HYD_ML_L + (pairs ? 2 * k : k)] = re;
+    q_s[r][HYD_ML_L + (pairs ? 2 * k + 1 : k + rope / 2)] = im;
+  }
+  __syncthreads();
+  const float inv = sqrtf((float)a.head_dim);
+  for (int t0 = wave * 16; t0 < L; t0 += 64) {
+    if (t0 != wave * 16) keys(t0, K);
+    f32x16 acc[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[s][i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      f32x4 qv[4];
+      if (j % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // else the reads of all nine steps are put first and do not fit the registers
+#pragma unroll
+      for (int s = 0; s < 4; ++s) qv[s] = *reinterpret_cast<const f32x4*>(&q_s[n][64 * j + 16 * b + 4 * s]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[s][i], (float)K.k[j][s >> 1][4 * (s & 1) + i], acc[s], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float quad[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) quad[u] = (acc[0][4 * u + r] + acc[1][4 * u + r]) + (acc[2][4 * u + r] + acc[3][4 * u + r]);
+      const float v = (quad[0] + quad[1]) + (quad[2] + quad[3]);
+      att[(4 * b + r) * TP + t0 + n] = v / inv;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    float* w = att + (wave * 4 + u) * TP;
+    float mx = -INFINITY;
+    for (int t = lane; t < L; t += 64) mx = fmaxf(mx, w[t]);
+    mx = ad::wave_max_dpp(mx);
+    float sum = 0.f;
+    for (int t0 = 0; t0 < L; t0 += 64) {
+      const float e = t0 + lane < L ? expf(w[t0 + lane] - mx) : 0.f;
+      w[t0 + lane] = e;
+      sum += ad::wave_sum_dpp(e);
+    }
+    for (int t = lane; t < L; t += 64) w[t] = w[t] / sum;
+  }
+  __syncthreads();
+  // latent values: thread group g of the per-token kernel's 8 sums positions g, g + 8, ...: block b takes group 4 G + b; 64 columns at a time
+  // (of 128, 8 a lane, the accumulators go to scratch memory)
+  typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half) {
+    const int c0 = 128 * wave + 64 * half + 4 * n;
+    const uint16_t* vc = a.nope_cache + c0;
+    float o[4][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[r][c] = 0.f;
+#pragma unroll 1
+    for (int G = 0; G < 2; ++G) {
+      f32x16 acc[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[c][i] = 0.f;
+      auto load = [&](int t) { return *reinterpret_cast<const f16x4*>(vc + (size_t)min(t, L - 1) * HYD_ML_L); };
+      f16x4 v[2] = {load(4 * G + b), load(4 * G + b + 8)};
+      for (int first = 4 * G; first < L; first += 16) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int t = first + 8 * u + b;
+          const f16x4 now = v[u];
+          v[u] = load(t + 16);
+          const bool in = t < L;
+          const float w = in ? att[n * TP + t] : 0.f;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(w, in ? (float)now[c] : 0.f, acc[c], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) o[r][c] += acc[c][4 * k + r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<f32x4*>(latent + (size_t)p * lat_stride + (size_t)(h0 + 4 * b + r) * HYD_ML_L + c0) = f32x4{o[r][0], o[r][1], o[r][2], o[r][3]};
+  }
+}
 // the long-context tokens of a chunk: per (head, token) the merge of mla_flash_kernel's chunk partials (mla_head_kernel, `merged`)
 __global__ __launch_bounds__(1024) void hyd_mla_merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_o, int H, int lora, int n_chunks,
                                                              const StepParams* __restrict__ sps, float* __restrict__ latent, int lat_stride) {
@@ -1435,6 +1570,13 @@ int launch_hyd_mla_attn(hipStream_t st, const AttnMlaArgs& a, const StepParams* 
   if (a.lora > 512 || a.lora % 64 || a.rope > 64 || a.rope % 4) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_mla_attn: kv_lora_rank %d / rope %d", a.lora, a.rope);
   const size_t lds = (size_t)max_kv * 4;
   if (lds > 96 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_mla_attn: kv_len %d does not fit LDS", max_kv);
+  // 16 heads of a token at a time; below 8 tokens a workgroup per head fills more of the card (8 workgroups a token against 128)
+  if (P >= 8 && a.lora == HYD_ML_L && a.rope % 16 == 0 && a.n_heads % 16 == 0 && max_kv <= HYD_AT_MAX_KV) {
+    const int bytes = 16 * hyd_at_row(max_kv) * 4;
+    hipFuncSetAttribute((const void*)hyd_mla_attn_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    hipLaunchKernelGGL(hyd_mla_attn_tile_kernel, dim3(a.n_heads / 16, P), dim3(256), bytes, st, a, sps, q_c, qc_stride, q_rope, qr_stride, latent, lat_stride, max_kv);
+    return DSK_OK;
+  }
   auto k = hyd_mla_attn_kernel;
   if (lds > 32 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL(k, dim3(a.n_heads, P), dim3(1024), lds, st, a, sps, q_c, qc_stride, q_rope, qr_stride, latent, lat_stride);

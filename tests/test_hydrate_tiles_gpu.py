@@ -36,3 +36,12 @@ def test_attention_of_token_tiles(ctx, P, pos0):
     c = synth.preset("v3", "q2_k", False, n_layers=1, first_k_dense_replace=1, max_seq_len=192, vocab_size=1024)
     tokens = np.random.default_rng(P).integers(0, c.vocab_size, P)
     _assert_identical(compare_hydrate(ctx, c, None, seed=23, tokens=tokens, pos0=pos0), P, pos0)
+
+
+# latent attention of 16 heads at a time (from 8 tokens on): contexts at both sides of 16 (a tile of keys, a step of the values), 64 (a sum of the
+# softmax) and 128, up to the last one before the long-context kernels take over
+@pytest.mark.parametrize("P,pos0", [(7, 0), (8, 0), (20, 1), (14, 55), (12, 123), (30, 294)])
+def test_latent_attention_of_head_tiles(ctx, P, pos0):
+    c = synth.preset("v3", "q2_k", True, n_layers=1, first_k_dense_replace=1, max_seq_len=384, vocab_size=1024)
+    tokens = np.random.default_rng(P).integers(0, c.vocab_size, P)
+    _assert_identical(compare_hydrate(ctx, c, None, seed=29, tokens=tokens, pos0=pos0), P, pos0)
