@@ -395,20 +395,23 @@ DEV float hyd16_value(const Hyd16Acc& acc, int r) { return (acc.S[r][0] + acc.S[
 // The workgroup: up to 8 waves = 8 consecutive STRIPS (GLU: 4 strips, one wave on the w1 strip and its neighbour on the w3 strip) times the
 // SAME 16 MT tokens.  The tokens' operands of HYD16_SB blocks at a time are staged once per workgroup in LDS (double-buffered, one
 // barrier per stage) and every wave reads its matrix operands from there: a wave's vector-memory traffic is its own tiles only.
-// What bounds it is vector instructions (about 80 % of the issue slots of two waves a SIMD): a tile's expansion (~90, once per pass) and the
-// float stage (~100 per 16 tokens and tile), so a pass takes MT = 2 groups of tokens wherever more than 16 are left: ~145 a tile and
-// 16 tokens.  512 tokens of DeepSeek-V3, against MT = 1 with the min operand masked per group (~215) and a GLU pair in one wave: experts'
-// w1 / w3 1502 -> 896 us, w2 813 -> 590, wo 429 -> 343, dense w1 / w3 1327 -> 710.
-// The min term: one v_mfma_i32_16x16x32_i8 per group.  Its 8 bytes a lane are two digit words of the token's: word 4 g + kg' is in the half that
-// g & 1 names and the weight side has zeros in the other half.
+// What bounds it is vector instructions (about 80 % of the issue slots of two waves a SIMD): a tile's expansion (~75, once per pass) and the
+// float stage (~85 per 16 tokens and tile), so a pass takes MT = 2 groups of tokens wherever more than 16 are left.  512 tokens of
+// DeepSeek-V3, with MT = 1, the min operand masked per group and a GLU pair in one wave (~215 instructions per tile and 16 tokens) -> MT = 2 and a
+// min term of integer products (~145) -> now (~120): experts' w1 / w3 1502 -> 896 -> 728 us, w2 813 -> 590 -> 537, wo 429 -> 343 -> 286, dense
+// w1 / w3 1327 -> 710 -> 595.
+// The min term of all four groups: one v_mfma_f32_16x16x4_4b_f16, block g the four sub-blocks of group g.  Sums (<= 2048) and mins (<= 15) are
+// integers that f16 holds and every product's sum (< 2^17) one that f32 holds: the integer products' value, already as float.
 #define HYD16_SB 2          // blocks per stage
 #define HYD16_TOK_B 272     // LDS bytes of a token's codes of one block (256 + 16: the 16 tokens of an operand read spread over the banks)
 template <int MT>
-constexpr int hyd16_stage_b() { return HYD16_SB * MT * (16 * HYD16_TOK_B + 16 * 64 + 16 * 4); }  // codes | digit words (hyd16_split), [kg'][g] | scales, per block
-typedef long i64x1;
+constexpr int hyd16_stage_b() { return HYD16_SB * MT * (16 * HYD16_TOK_B + 16 * 32 + 16 * 4); }  // codes | sums as f16 | scales, per block
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 struct Hyd16W {  // a tile's weight side
   i32x4 B[4];   // the scaled group operands
-  u32x2_t m[4]; // the min operands
+  f16x4_t m;    // the min operand: the mins of group kg'
 };
 DEV void hyd16_weights(const HydTile& T, int kgp, Hyd16W& o) {
   const u32 w[4] = {T.w.x, T.w.y, T.w.z, T.w.w};
@@ -424,14 +427,19 @@ DEV void hyd16_weights(const HydTile& T, int kgp, Hyd16W& o) {
   for (int g = 0; g < 4; ++g) {
     const int sh = 2 * (2 * (g & 1) + fs);
     const u32 scm = T.sc[g] >> (8 * kgp);  // the sub-block's scale | min nibbles
-    const u32 sc = scm & 0xFu, pair = sc | (sc << 16), mn = ((scm >> 4) & 0xFu) * 0x00080801u;
+    const u32 sc = scm & 0xFu, pair = sc | (sc << 16);
     const u32* src = (g >> 1) ? hi : lo;
     o.B[g].x = (int)pkmul16((src[0] >> sh) & 0x03030303u, pair);
     o.B[g].y = (int)pkmul16((src[1] >> sh) & 0x03030303u, pair);
     o.B[g].z = (int)pkmul16((src[2] >> sh) & 0x03030303u, pair);
     o.B[g].w = (int)pkmul16((src[3] >> sh) & 0x03030303u, pair);
-    o.m[g] = (g & 1) ? u32x2_t{0u, mn} : u32x2_t{mn, 0u};
   }
+  const u32 s01 = (kgp & 1) ? T.sc[1] : T.sc[0], s23 = (kgp & 1) ? T.sc[3] : T.sc[2];
+  const u32 mn = (((kgp & 2) ? s23 : s01) >> 4) & 0x0F0F0F0Fu;  // four mins; 0x64nn is 1024 + nn in f16
+  const f16x2_t k1024 = {(_Float16)1024.f, (_Float16)1024.f};
+  const u32 w01 = __builtin_amdgcn_perm(0x64646464u, mn, 0x04010400u), w23 = __builtin_amdgcn_perm(0x64646464u, mn, 0x04030402u);
+  const f16x2_t m01 = __builtin_bit_cast(f16x2_t, w01) - k1024, m23 = __builtin_bit_cast(f16x2_t, w23) - k1024;
+  o.m = f16x4_t{m01.x, m01.y, m23.x, m23.y};
 }
 DEV float hyd16_item1(float dd, float D, float dmn, float M) {  // an item of one block: its two chains are a product each
 #pragma clang fp contract(off)
@@ -446,7 +454,7 @@ DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, con
   constexpr int nthreads = 64 * NW, TT = 16 * MT, STAGE = hyd16_stage_b<MT>();
   constexpr int R = HYD16_SB * TT * 16 / nthreads;              // 16-byte pieces of a stage's codes per thread
   constexpr int BP = HYD16_SB * TT * 2, RB_N = (BP + nthreads - 1) / nthreads;  // pieces of 8 sums
-  constexpr int D_LDS = HYD16_SB * TT * (HYD16_TOK_B + 64);
+  constexpr int D_LDS = HYD16_SB * TT * (HYD16_TOK_B + 32);
   static_assert(R >= 1 && HYD16_SB == 2 && TT <= nthreads, "staging");
   const int n = A.n, nb = n >> 8;
   const int kgp = lane >> 4, tl = lane & 15;   // operand side: token tl of a group, K-group kg'
@@ -484,17 +492,17 @@ DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, con
       *reinterpret_cast<u32x4*>(buf + (idx >> 4) * HYD16_TOK_B + (idx & 15) * 16) = G.c[k];
     }
 #pragma unroll
-    for (int k = 0; k < RB_N; ++k) {  // the sums become the min term's operand words ONCE per workgroup, not per wave and block
+    for (int k = 0; k < RB_N; ++k) {  // the sums become f16 (exactly: at most 16 x 128) ONCE per workgroup, not per wave and block
       const int idx = tid + k * nthreads;
       if (idx < BP) {
-        const u32 w[4] = {G.bs[k].x, G.bs[k].y, G.bs[k].z, G.bs[k].w};  // 8 sums: groups 2 p, 2 p + 1 of piece p
-        uint8_t* at = buf + HYD16_SB * TT * HYD16_TOK_B + (idx >> 1) * 64 + (idx & 1) * 8;
+        const u32 w[4] = {G.bs[k].x, G.bs[k].y, G.bs[k].z, G.bs[k].w};
+        u32 f[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {  // sub-block kg' = i of both groups
-          const int sh = 16 * (i & 1);
-          const u32x2_t v = {hyd16_split((int)(short)((w[i >> 1] >> sh) & 0xFFFFu)), hyd16_split((int)(short)((w[2 + (i >> 1)] >> sh) & 0xFFFFu))};
-          *reinterpret_cast<u32x2_t*>(at + 16 * i) = v;
+        for (int i = 0; i < 4; ++i) {
+          const f16x2_t v = {(_Float16)(short)(w[i] & 0xFFFFu), (_Float16)(short)(w[i] >> 16)};
+          f[i] = __builtin_bit_cast(u32, v);
         }
+        *reinterpret_cast<u32x4*>(buf + HYD16_SB * TT * HYD16_TOK_B + idx * 16) = u32x4{f[0], f[1], f[2], f[3]};
       }
     }
     if (tid < TT) {
@@ -521,18 +529,22 @@ DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, con
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         S[t][r][g] = 0.f;
-        if (SEG4) ad[t][r][g] = am[t][r][g] = 0.f;
       }
+  auto item_begin = [&]() {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) ad[t][r][g] = am[t][r][g] = 0.f;
+  };
   auto item_end = [&]() {
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          S[t][r][g] += ad[t][r][g] - am[t][r][g];
-          ad[t][r][g] = am[t][r][g] = 0.f;
-        }
+        for (int g = 0; g < 4; ++g) S[t][r][g] += ad[t][r][g] - am[t][r][g];
   };
   auto block = [&](int u, int b, const uint8_t* cur) {
     Hyd16W E;
@@ -545,46 +557,64 @@ DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, con
       i32x4 a[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) a[g] = *reinterpret_cast<const i32x4*>(cb + 64 * g);
-      const u32x4 dig = *reinterpret_cast<const u32x4*>(cur + HYD16_SB * TT * HYD16_TOK_B + (u * TT + t * 16 + tl) * 64 + 16 * kgp);
+      const f16x4_t sums = *reinterpret_cast<const f16x4_t*>(cur + HYD16_SB * TT * HYD16_TOK_B + (u * TT + t * 16 + tl) * 32 + 8 * kgp);
       const f32x4 dx = *reinterpret_cast<const f32x4*>(cur + D_LDS + (u * TT + t * 16 + 4 * q) * 4);
       const i32x4 z = {0, 0, 0, 0};
-      const i64x1 dig01 = __builtin_bit_cast(i64x1, (u32x2_t{dig.x, dig.y})), dig23 = __builtin_bit_cast(i64x1, (u32x2_t{dig.z, dig.w}));
-      i32x4 D[4], M[4];
+      f32x16 M;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        D[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], E.B[g], z, 0, 0, 0);
-        M[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8((g >> 1) ? dig23 : dig01, __builtin_bit_cast(i64x1, E.m[g]), z, 0, 0, 0);
-      }
+      for (int i = 0; i < 16; ++i) M[i] = 0.f;
+      i32x4 D[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) D[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], E.B[g], z, 0, 0, 0);
+      M = __builtin_amdgcn_mfma_f32_16x16x4f16(sums, E.m, M, 0, 0, 0);
       const float dxr[4] = {dx.x, dx.y, dx.z, dx.w};
       float dd[4], dmn[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) { dd[r] = dxr[r] * d; dmn[r] = dxr[r] * dmin; }
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int Dr[4] = {D[g].x, D[g].y, D[g].z, D[g].w}, Mr[4] = {M[g].x, M[g].y, M[g].z, M[g].w};
+        const int Dr[4] = {D[g].x, D[g].y, D[g].z, D[g].w};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           if (SEG4) {
             ad[t][r][g] = fmaf(dd[r], (float)Dr[r], ad[t][r][g]);
-            am[t][r][g] = fmaf(dmn[r], (float)Mr[r], am[t][r][g]);
+            am[t][r][g] = fmaf(dmn[r], M[4 * g + r], am[t][r][g]);
           } else {
-            S[t][r][g] += hyd16_item1(dd[r], (float)Dr[r], dmn[r], (float)Mr[r]);
+            S[t][r][g] += hyd16_item1(dd[r], (float)Dr[r], dmn[r], M[4 * g + r]);
           }
         }
       }
     }
   };
-  int b0 = 0;
-  for (; b0 + HYD16_SB <= nb; b0 += HYD16_SB) {
+  auto pin = [&]() {  // the chains up to here are computed here: the compiler moved a whole item's to its end, with all the products in scratch memory
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) asm volatile("" : "+v"(ad[t][r][g]), "+v"(am[t][r][g]));
+  };
+  auto stage = [&](int b0) {
     uint8_t* cur = lds + ((b0 / HYD16_SB) & 1) * STAGE;
     uint8_t* nxt = lds + (((b0 / HYD16_SB) & 1) ^ 1) * STAGE;
     request(G, min(b0 + HYD16_SB, nb - 1));
     block(0, b0, cur);
     block(1, b0 + 1, cur);
-    if (SEG4 && (b0 & 2)) item_end();
+    if (SEG4) pin();
     write(G, nxt);
     lds_barrier();  // (also in front of the next pass's first stage: every wave is done with both buffers)
+  };
+  int b0 = 0;
+  if (SEG4) {
+    for (; b0 + 4 <= nb; b0 += 4) {  // an item at a time: its chains begin with a constant zero, not with a register to be cleared
+      item_begin();
+      stage(b0);
+      stage(b0 + 2);
+      item_end();
+    }
+    item_begin();
   }
+  for (; b0 + HYD16_SB <= nb; b0 += HYD16_SB) stage(b0);
   if (b0 < nb) block(0, b0, lds + ((b0 / HYD16_SB) & 1) * STAGE);
   if (nb & 1) __syncthreads();
   if (SEG4 && (nb & 3)) item_end();
@@ -1028,7 +1058,6 @@ __global__ __launch_bounds__(1024, 8) void hyd_attn_kernel(const AttnMhaArgs a, 
 //            4 G + b, G in turn.  Positions behind a token's context are left out by selection, not by a weight of zero: they may hold anything.
 // Same bits as hyd_attn_kernel, which reads a head's keys and values once per token and is bound by the round trips of 16-wave workgroups:
 // 512 tokens of DeepSeek-V3's 128 heads 1180 -> 327 us.  4 waves: key tiles in turn, then 4 tokens' softmax each, then 32 value columns each.
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 enum { HYD_AT = 16, HYD_AT_MAX_KV = 1024, HYD_AT_V = 128, HYD_AT_NJ = 3 };  // tokens; contexts of one position per softmax thread; v_dim; head_dim <= 64 NJ
 __host__ DEV int hyd_at_row(int max_kv) { return (max_kv + 63) / 64 * 64 + 4; }  // floats of a token's weights in LDS: 16 tokens x 4 positions meet 64 banks
 __global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs a, const StepParams* __restrict__ sps, const float* __restrict__ q, int q_stride,
