@@ -29,7 +29,10 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 #define HYD16_MIN_TOKENS 12  // plain matrices: from this many tokens on, 16 tokens per wave (hyd_gemm16_kernel)
 #endif
 #ifndef HYD16_EXPERT_MIN
-#define HYD16_EXPERT_MIN 6   // expert stacks: tasks with at least this many rows take the 16-token form (0: never)
+// Expert stacks: tasks with at least this many rows take the 16-token form (0: never).  A quad's pass over a tile costs as many vector instructions
+// (~125) for 4 rows as that form's for 16, so a fifth row is the line: 77 tokens of DeepSeek-V3, w1 / w3 of a block in both launches 378 us with
+// the line at 6, 345 at 5, 424 at 1 (few waves in flight: 8 a CU against 12).
+#define HYD16_EXPERT_MIN 5
 #endif
 #define HYD_OOB 0x40000000  // a buffer offset beyond any activation array (all far below 1 GiB): the load returns zeros and touches no memory
 
@@ -586,13 +589,16 @@ DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, con
       }
     }
   };
-  auto pin = [&]() {  // the chains up to here are computed here: the compiler moved a whole item's to its end, with all the products in scratch memory
+  auto pin = [&]() {  // the chains up to here are computed here: the compiler moved a whole item's to its end, with the products in scratch memory
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) asm volatile("" : "+v"(ad[t][r][g]), "+v"(am[t][r][g]));
+        for (int g = 0; g < 4; ++g) {
+          if (SEG4) asm volatile("" : "+v"(ad[t][r][g]), "+v"(am[t][r][g]));
+          else asm volatile("" : "+v"(S[t][r][g]));
+        }
   };
   auto stage = [&](int b0) {
     uint8_t* cur = lds + ((b0 / HYD16_SB) & 1) * STAGE;
@@ -600,7 +606,7 @@ DEV void hyd16_pass(const HydGemmArgs& A, const rsrc_t& W, const rsrc_t& RA, con
     request(G, min(b0 + HYD16_SB, nb - 1));
     block(0, b0, cur);
     block(1, b0 + 1, cur);
-    if (SEG4) pin();
+    pin();
     write(G, nxt);
     lds_barrier();  // (also in front of the next pass's first stage: every wave is done with both buffers)
   };
