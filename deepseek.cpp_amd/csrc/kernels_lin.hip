@@ -574,10 +574,13 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
     set_expert(a, f.m, f.down ? f.m.down : f.m.up, expert);
     const int nr = f.down ? 1 : 2;
     if (tile * nr >= a.rt) return;
-    const int row = min(c, f.m.rows - 1);
-    const int slot = f.m.active_slot[i * 16 + row];
-    const int pos = row * (f.m.top + f.m.shared) + max(slot, 0);
-    const int out = c < f.m.rows && slot >= 0 ? pos : -1;
+    // a lane whose row did not choose the expert reads the first row that did: a load of the operand then touches as many lines as the expert has
+    // rows, not 16
+    const int slot = c < f.m.rows ? f.m.active_slot[i * 16 + c] : -1;
+    const int own = min(c, f.m.rows - 1) * (f.m.top + f.m.shared) + max(slot, 0);
+    const int one = max(__ffsll(__ballot(slot >= 0)) - 1, 0);
+    const int row = slot >= 0 ? c : one, pos = slot >= 0 ? own : __shfl(own, one);
+    const int out = slot >= 0 ? own : -1;
     if (f.down) few_body<T, 1>(a, tile, 0, a.kt, pos, out, lds);
     else few_body<T, 2>(a, tile * 2, 0, a.kt, row, out, lds);
     return;
