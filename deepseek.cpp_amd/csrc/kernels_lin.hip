@@ -509,51 +509,71 @@ __global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs
 }
 
 // ---- up to 16 rows -------------------------------------------------------------------------------
-// One workgroup = 16 features (32 with a gate / up pair): wave w takes k tiles w, w + 4, ...; partial sums meet in LDS.
-// row_of: A row of this lane's column; keep: out row or -1.
-template <typename T, int NR>
+// One workgroup = NR feature tiles of 16 (GLU: NR / 2 gate / up pairs): wave w takes k tiles w, w + 4, ...; partial sums meet in LDS.
+// a_row: A row of this lane's column; out_row: out row or -1.
+template <typename T, int NR, bool GLU>
 DEV void few_body(const LinArgs& a, int rt0, int k_first, int k_end, int a_row, int out_row, float* lds) {
   typedef typename Frag<T>::type frag;
   constexpr int U = NR == 1 && sizeof(T) == 2 ? 8 : 4;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const bf16x8* w0 = reinterpret_cast<const bf16x8*>(a.w) + (size_t)rt0 * a.kt * 64 + lane;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bf16x8* w0 = reinterpret_cast<const bf16x8*>(a.w) + lane;
+  size_t tile[NR];  // (a group's tiles past the last are its last, and not stored)
+#pragma unroll
+  for (int i = 0; i < NR; ++i) tile[i] = (size_t)min(rt0 + i, a.rt - 1) * a.kt;
   const T* x0 = operand<T>(a, rt0 * 16) + (size_t)a_row * a.lda + (lane >> 4) * 8;
   f32x4 acc[NR];
 #pragma unroll
   for (int i = 0; i < NR; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = k_first + wave; k0 < k_end; k0 += 4 * U) {
-    bf16x8 w[U][NR];
-    frag x[U];
+  bf16x8 w[U][NR];
+  frag x[U];
+  auto load = [&](int u, int k) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = min(k0 + 4 * u, k_end - 1);
+    for (int i = 0; i < NR; ++i) w[u][i] = w0[(tile[i] + k) * 64];
+    x[u] = *reinterpret_cast<const frag*>(x0 + (size_t)k * 32);
+  };
+  int k0 = k_first + wave;
+  for (; k0 + 4 * (U - 1) < k_end; k0 += 4 * U) {  // no condition inside: a load is moved behind it, and then waited for alone
 #pragma unroll
-      for (int i = 0; i < NR; ++i) w[u][i] = w0[((size_t)i * a.kt + k) * 64];
-      x[u] = *reinterpret_cast<const frag*>(x0 + (size_t)k * 32);
-    }
+    for (int u = 0; u < U; ++u) load(u, k0 + 4 * u);
+    __builtin_amdgcn_sched_barrier(0);  // (all on their way first)
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (k0 + 4 * u < k_end)
 #pragma unroll
-        for (int i = 0; i < NR; ++i) acc[i] = mma(w[u][i], x[u], acc[i]);
+      for (int i = 0; i < NR; ++i) acc[i] = mma(w[u][i], x[u], acc[i]);
+  }
+  if (k0 < k_end) {  // the last, short one: zeros behind the end
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u) load(u, min(k0 + 4 * u, k_end - 1));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u) {
+      const bool in = k0 + 4 * u < k_end;
+      const frag xu = in ? x[u] : frag{};
+#pragma unroll
+      for (int i = 0; i < NR; ++i) acc[i] = mma(in ? w[u][i] : bf16x8{}, xu, acc[i]);
+    }
   }
 #pragma unroll
   for (int i = 0; i < NR; ++i) *reinterpret_cast<f32x4*>(lds + ((wave * NR + i) * 64 + lane) * 4) = acc[i];
   __syncthreads();
-  if (wave != 0) return;
+  constexpr int PER = GLU ? 2 : 1;  // wave v adds up the v-th tile or pair
+  if (wave >= NR / PER || rt0 + wave * PER >= a.rt) return;
+  f32x4 sum[PER];
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
+  for (int i = 0; i < PER; ++i) {
+    sum[i] = *reinterpret_cast<const f32x4*>(lds + ((wave * PER + i) * 64 + lane) * 4);
 #pragma unroll
-    for (int v = 1; v < 4; ++v) acc[i] += *reinterpret_cast<const f32x4*>(lds + ((v * NR + i) * 64 + lane) * 4);
+    for (int v = 1; v < 4; ++v) sum[i] += *reinterpret_cast<const f32x4*>(lds + ((v * NR + wave * PER + i) * 64 + lane) * 4);
   }
   if (out_row < 0) return;
-  if constexpr (NR == 2) store_glu<T>(a, out_row, (rt0 >> 1) * 16 + (lane >> 4) * 4, acc[0], acc[1]);
-  else store_plain<T>(a, out_row, rt0 * 16 + (lane >> 4) * 4, acc[0]);
+  if constexpr (GLU) store_glu<T>(a, out_row, ((rt0 >> 1) + wave) * 16 + (lane >> 4) * 4, sum[0], sum[1]);
+  else store_plain<T>(a, out_row, (rt0 + wave) * 16 + (lane >> 4) * 4, sum[0]);
 }
 
 struct FewArgs {
   LinArgs t[4];
   int wg_end[4];   // workgroups of products 0 .. i
+  int groups[4];   // ... of one part of product i
   int n;
   int expert_wgs;  // in front of them: expert blocks
   int tiles_per_expert;
@@ -561,9 +581,12 @@ struct FewArgs {
   LinArgs e;
   MoeArgs m;
 };
-template <typename T>
+// A load of the operand is `rows` segments of 64 bytes in as many lines, at 16 rows twice the lines of a weight tile's load: where enough
+// workgroups are left (launch_few) one takes NT tiles (of gate and up: two pairs) per load of the operand.
+template <typename T, int NT>
 __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * 2 * 64 * 4];
+  constexpr int GT = NT > 1 ? 4 : 2;  // tiles of a gate / up group
+  __shared__ __attribute__((aligned(16))) float lds[4 * (NT > GT ? NT : GT) * 64 * 4];
   const int c = threadIdx.x & 15;
   int b = blockIdx.x;
   if (b < f.expert_wgs) {
@@ -572,7 +595,7 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
     const int expert = f.m.active[i];
     LinArgs a = f.e;
     set_expert(a, f.m, f.down ? f.m.down : f.m.up, expert);
-    const int nr = f.down ? 1 : 2;
+    const int nr = f.down ? NT : GT;
     if (tile * nr >= a.rt) return;
     // a lane whose row did not choose the expert reads the first row that did: a load of the operand then touches as many lines as the expert has
     // rows, not 16
@@ -581,8 +604,8 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
     const int one = max(__ffsll(__ballot(slot >= 0)) - 1, 0);
     const int row = slot >= 0 ? c : one, pos = slot >= 0 ? own : __shfl(own, one);
     const int out = slot >= 0 ? own : -1;
-    if (f.down) few_body<T, 1>(a, tile, 0, a.kt, pos, out, lds);
-    else few_body<T, 2>(a, tile * 2, 0, a.kt, row, out, lds);
+    if (f.down) few_body<T, NT, false>(a, tile * NT, 0, a.kt, pos, out, lds);
+    else few_body<T, GT, true>(a, tile * GT, 0, a.kt, row, out, lds);
     return;
   }
   b -= f.expert_wgs;
@@ -590,9 +613,9 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
   while (i + 1 < f.n && b >= f.wg_end[i]) ++i;
   LinArgs a = f.t[i];
   if (i > 0) b -= f.wg_end[i - 1];
-  const int row = min(c, a.rows - 1), part = b / a.rt, per = part_tiles(a);
+  const int row = min(c, a.rows - 1), part = b / f.groups[i], per = part_tiles(a);
   a.out_f += part * a.part_stride;
-  few_body<T, 1>(a, b % a.rt, part * per, min(a.kt, part * per + per), a.row_seq ? a.seqs[a.row_seq[row]].row0 : row, c < a.rows ? c : -1, lds);
+  few_body<T, NT, false>(a, b % f.groups[i] * NT, part * per, min(a.kt, part * per + per), a.row_seq ? a.seqs[a.row_seq[row]].row0 : row, c < a.rows ? c : -1, lds);
 }
 
 // ---- launches ------------------------------------------------------------------------------------
@@ -667,7 +690,19 @@ int launch_experts(hipStream_t st, const MoeArgs& m, bool down, bool f32) {
   }
   return DSK_OK;
 }
-static int launch_few(hipStream_t st, FewArgs& f, const LinArgs* a, int n, bool f32) {
+// Four tiles per workgroup from 9 rows and 1536 tiles on, in bf16: a step of 16 sequences, us with one tile -> four, 8080 tiles 450 -> 320, 2328
+// tiles 136 -> 106, 1572 94 -> 71, the experts' down 8832 88 -> 66; below, the card is left empty: 1056 tiles 16.4 -> 21, 582 13 -> 15.5.  Up to
+// 8 rows the operand is the smaller part (6400 tiles of 8 rows 84 -> 82), and in 32 bits 5 rows of 896 tiles were slower (105 -> 133).
+constexpr int FEW_TILES = 4;
+static int launch_few(hipStream_t st, FewArgs& f, const LinArgs* a, int n, int experts, int expert_tiles, int rows, bool f32) {
+  int tiles = experts * expert_tiles;
+  bool whole = true;  // (a workgroup's tiles read one operand)
+  for (int i = 0; i < n; ++i) {
+    rows = std::max(rows, a[i].rows);
+    tiles += a[i].rt * std::max(a[i].parts, 1);
+    whole = whole && a[i].a_seg % (16 * FEW_TILES) == 0;
+  }
+  const int nt = !f32 && rows > 8 && tiles >= 1536 && whole ? FEW_TILES : 1;
   if (n > 4) DSK_FAIL(DSK_ERR_INVALID, "lin_few: %d products", n);
   f.n = n;
   int wgs = 0;
@@ -675,16 +710,18 @@ static int launch_few(hipStream_t st, FewArgs& f, const LinArgs* a, int n, bool 
     DSK_TRY(check_lin(a[i], "lin_few"));
     if (a[i].rows > 16) DSK_FAIL(DSK_ERR_INVALID, "lin_few: %d rows", a[i].rows);
     f.t[i] = a[i];
-    f.wg_end[i] = wgs += a[i].rt * std::max(a[i].parts, 1);
+    f.groups[i] = cdiv(a[i].rt, nt);
+    f.wg_end[i] = wgs += f.groups[i] * std::max(a[i].parts, 1);
   }
-  const dim3 grid(f.expert_wgs + wgs);
-  if (f32) hipLaunchKernelGGL(few_kernel<float>, grid, dim3(256), 0, st, f);
-  else hipLaunchKernelGGL(few_kernel<bf16>, grid, dim3(256), 0, st, f);
+  f.tiles_per_expert = cdiv(expert_tiles, f.down ? nt : nt > 1 ? 4 : 2);
+  f.expert_wgs = experts * f.tiles_per_expert;
+  auto k = f32 ? few_kernel<float, 1> : nt > 1 ? few_kernel<bf16, FEW_TILES> : few_kernel<bf16, 1>;
+  hipLaunchKernelGGL(k, dim3(f.expert_wgs + wgs), dim3(256), 0, st, f);
   return DSK_OK;
 }
 int launch_lin_few(hipStream_t st, const LinArgs* a, int n, bool f32) {
   FewArgs f{};
-  return launch_few(st, f, a, n, f32);
+  return launch_few(st, f, a, n, 0, 0, 0, f32);
 }
 int launch_experts_few(hipStream_t st, const MoeArgs& m, bool down, const LinArgs* also, int n_also, bool f32) {
   if (m.rows > 16) DSK_FAIL(DSK_ERR_INVALID, "experts_few: %d rows", m.rows);
@@ -694,7 +731,5 @@ int launch_experts_few(hipStream_t st, const MoeArgs& m, bool down, const LinArg
   f.e = expert_lin(m, down);
   const ExpertMat& e = down ? m.down : m.up;
   const int rt = m.shared ? (e.rt > e.shared_rt ? e.rt : e.shared_rt) : e.rt;
-  f.tiles_per_expert = down ? rt : rt / 2;
-  f.expert_wgs = m.max_active * f.tiles_per_expert;
-  return launch_few(st, f, also, n_also, f32);
+  return launch_few(st, f, also, n_also, m.max_active, rt, m.rows, f32);
 }

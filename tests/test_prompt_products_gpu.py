@@ -1,4 +1,5 @@
 """Products of prompts at the edges of their tiles (kernels_lin.hip), against the plain statement of the design (oracle/layered.py)."""
+import numpy as np
 import pytest
 
 from tests import layered_util as U
@@ -53,3 +54,27 @@ def test_32_bit_products_keep_32_bits(ctx, tmp_path, width):
     K = U.Case(ctx, tmp_path, U.sandwich([U.no_ff(U.latent())], width=width), dtype="float32")
     t = K.tokens(140)
     assert U.err(K.got(t), K.want(t)) < 2.0 ** -18
+
+
+# decoding steps: from 9 rows and 1536 tiles on a workgroup takes four feature tiles.  Vocabulary, experts' hidden sizes and width leave a last group
+# of 1, 2 or 3 tiles (pairs: of one); experts without a row, with one and with several.  A row's sums are added in the same order
+# either way: the bits of steps of 8 rows.
+@pytest.mark.parametrize("width,ff,vocab", [(400, 264, 24600), (432, 200, 24620), (264, 296, 24590)])
+def test_steps_of_many_tiles_per_workgroup(ctx, tmp_path, width, ff, vocab):
+    K = U.Case(ctx, tmp_path, U.config([U.parallel(mlp=U.moe(100, 7, ff, 0.8, 40, 1.2))], width=width, vocab=vocab), dtype="bfloat16")
+    toks = [K.tokens(3, seed=n) for n in range(16)]
+
+    def decode(sizes):
+        seqs, out = [K.lm.seq_open() for _ in toks], []
+        K.lm.step([(s, t[:2], []) for s, t in zip(seqs, toks)])
+        for n in sizes:
+            part = slice(len(out), len(out) + n)
+            out.extend(K.lm.step([(s, t[2:], [0]) for s, t in zip(seqs[part], toks[part])]))
+        for s in seqs:
+            K.lm.seq_close(s)
+        return np.array(out)
+
+    few = decode([8, 8])
+    assert np.array_equal(decode([16]), few)
+    assert np.array_equal(decode([9, 7]), few)
+    assert U.err(few[:1], K.want(toks[0])[-1:]) < K.tol
