@@ -23,6 +23,7 @@
 #include "dsk_internal.h"
 #include "tile_device.h"
 #include <algorithm>
+#include <type_traits>
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 #ifndef HYD16_MIN_TOKENS
@@ -1061,9 +1062,11 @@ __global__ __launch_bounds__(1024, 8) void hyd_attn_kernel(const AttnMhaArgs a, 
 //            instruction takes the lanes 4 b + s, one accumulator per s: a lane of the result holds all 16 partial sums of its pairs.
 //   softmax  the maximum; sums of 64 positions by wave_sum_dpp, added in order; a division each
 //   values   thread group g of 4096 / v_dim sums positions g, g + 32, ... in order and the groups are added in order: block b takes group
-//            4 G + b, G in turn.  Positions behind a token's context are left out by selection, not by a weight of zero: they may hold anything.
+//            4 G + b, G in turn.  Positions behind a token's context have a weight of zero, or, where a later token's value is no number, are
+//            left out by selection.
 // Same bits as hyd_attn_kernel, which reads a head's keys and values once per token and is bound by the round trips of 16-wave workgroups:
-// 512 tokens of DeepSeek-V3's 128 heads 1180 -> 327 us.  4 waves: key tiles in turn, then 4 tokens' softmax each, then 32 value columns each.
+// 512 tokens of DeepSeek-V3's 128 heads 1180 -> 261 us (327 with all partial steps by selection and loads under conditions; the matrix instructions
+// alone are ~75).  4 waves: key tiles in turn, then 4 tokens' softmax each, then 32 value columns each.
 enum { HYD_AT = 16, HYD_AT_MAX_KV = 1024, HYD_AT_V = 128, HYD_AT_NJ = 3 };  // tokens; contexts of one position per softmax thread; v_dim; head_dim <= 64 NJ
 __host__ DEV int hyd_at_row(int max_kv) { return (max_kv + 63) / 64 * 64 + 4; }  // floats of a token's weights in LDS: 16 tokens x 4 positions meet 64 banks
 __global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs a, const StepParams* __restrict__ sps, const float* __restrict__ q, int q_stride,
@@ -1128,19 +1131,21 @@ __global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs
   const int most = sps[token(HYD_AT - 1)].kv_len, least = sps[p0].kv_len;  // (ascending)
   const float inv = sqrtf((float)hd);
   typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+  // Keys and values through buffer loads: what lies past the context or the head reads as zero without a branch (a load under a condition is
+  // waited for where the paths meet).
+  const rsrc_t RK = make_rsrc_n(a.key_cache, (u32)((size_t)most * H * hd * 2)), RV = make_rsrc_n(a.value_cache, (u32)((size_t)most * H * HYD_AT_V * 2));
   struct Keys { f16x8 k[HYD_AT_NJ][2]; };
+  int key_off[HYD_AT_NJ];
+#pragma unroll
+  for (int j = 0; j < HYD_AT_NJ; ++j) key_off[j] = 64 * j + 16 * b < hd ? ((n * H + h) * hd + 64 * j + 16 * b) * 2 : HYD_OOB;
   auto keys = [&](int t0, Keys& o) {
-    const uint16_t* row = a.key_cache + ((size_t)min(t0 + n, most - 1) * H + h) * hd + 16 * b;
+    const int row = min(t0, most - 1) * H * hd * 2;
 #pragma unroll
     for (int j = 0; j < HYD_AT_NJ; ++j)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) o.k[j][u] = 64 * j + 16 * b < hd ? *reinterpret_cast<const f16x8*>(row + 64 * j + 8 * u) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      for (int u = 0; u < 2; ++u) o.k[j][u] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(RK, key_off[j] + 16 * u, row, 0));
   };
-  Keys K;
-  keys(wave * 16, K);
-  for (int t0 = wave * 16; t0 < most; t0 += 64) {
-    Keys N;
-    keys(t0 + 64, N);
+  auto scores = [&](int t0, const Keys& K) {
     f32x16 acc[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s)
@@ -1160,33 +1165,75 @@ __global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs
       const float p = (quad[0] + quad[1]) + (quad[2] + quad[3]);
       att[(4 * b + r) * TP + t0 + n] = p / inv;
     }
-    K = N;
+  };
+  {
+    Keys K, N;
+    int t0 = wave * 16;
+    keys(t0, K);
+    keys(t0 + 64, N);
+    for (; t0 + 64 < most; t0 += 128) {
+      scores(t0, K);
+      keys(t0 + 128, K);
+      __builtin_amdgcn_sched_barrier(0);
+      scores(t0 + 64, N);
+      keys(t0 + 192, N);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (t0 < most) scores(t0, K);
   }
   __syncthreads();
   // softmax, src/infer.cpp:472-487
+  {  // four tokens a wave, side by side
+    float* w = att + wave * 4 * TP;
+    int L[4];
+    float mx[4], sum[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = wave * 4 + u, L = sps[token(r)].kv_len;
-    float* w = att + r * TP;
-    float mx = -INFINITY;
-    for (int t = lane; t < L; t += 64) mx = fmaxf(mx, w[t]);
-    mx = ad::wave_max_dpp(mx);
-    float sum = 0.f;
-    for (int t0 = 0; t0 < L; t0 += 64) {
-      const float e = t0 + lane < L ? expf(w[t0 + lane] - mx) : 0.f;
-      if (t0 + lane < L) w[t0 + lane] = e;
-      sum += ad::wave_sum_dpp(e);
+    for (int u = 0; u < 4; ++u) {
+      L[u] = sps[token(wave * 4 + u)].kv_len;
+      mx[u] = -INFINITY;
+      sum[u] = 0.f;
     }
-    for (int t = lane; t < L; t += 64) w[t] = w[t] / sum;
+    for (int t = lane; t < L[3]; t += 64)  // (ascending)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) mx[u] = t < L[u] ? fmaxf(mx[u], w[u * TP + t]) : mx[u];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) mx[u] = ad::wave_max_dpp(mx[u]);
+    for (int t0 = 0; t0 < L[3]; t0 += 64) {
+      const int t = t0 + lane;
+      float e[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        e[u] = expf(w[u * TP + t] - mx[u]);
+        e[u] = t < L[u] ? e[u] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        w[u * TP + t] = e[u];
+        sum[u] += ad::wave_sum_dpp(e[u]);
+      }
+    }
+    for (int t = lane; t < L[3]; t += 64)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u * TP + t] = w[u * TP + t] / sum[u];
   }
   __syncthreads();
   // values: columns 32 wave + 2 n + {0, 1}; the groups 4 G + b, two values of G at a time
-  const uint16_t* vc = a.value_cache + (size_t)h * HYD_AT_V + 32 * wave + 2 * n;
   typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
   float o[4][2];
 #pragma unroll
   for (int r = 0; r < 4; ++r) o[r][0] = o[r][1] = 0.f;
   const int whole = least / 32, steps = (most + 31) / 32;  // steps that every token has all positions of; all steps
+  // Behind them a token without a position has weight 0 for it: nothing is added, unless the value (of a later token) is no number.  Then, and
+  // only then, sums are chosen one by one.
+  const int len_n = sps[token(n)].kv_len;
+  bool odd = false;
+  for (int t = 32 * whole + (lane >> 4) * 2; t < most; t += 8)  // (this wave's 32 columns)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const u32 two = __builtin_amdgcn_raw_buffer_load_b32(RV, ((min(t + u, most - 1) * H + h) * HYD_AT_V + 32 * wave + 2 * n) * 2, 0, 0);
+      odd = odd || (two & 0x7C00u) == 0x7C00u || (two & 0x7C000000u) == 0x7C000000u;
+    }
+  odd = __any(odd);
 #pragma unroll 1
   for (int G = 0; G < 8; G += 2) {
     f32x16 acc[2][2];
@@ -1197,42 +1244,51 @@ __global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[u][c][i] = 0.f;
     const int t0 = 4 * G + b;  // (and t0 + 4)
-    auto load = [&](int step, int u) { return *reinterpret_cast<const f16x2*>(vc + (size_t)min(32 * step + t0 + 4 * u, most - 1) * H * HYD_AT_V); };
+    const int off = ((t0 * H + h) * HYD_AT_V + 32 * wave + 2 * n) * 2;
+    auto load = [&](int step, int u) {
+      return __builtin_bit_cast(f16x2, __builtin_amdgcn_raw_buffer_load_b32(RV, off + u * 4 * H * HYD_AT_V * 2, min(step, steps - 1) * 32 * H * HYD_AT_V * 2, 0));
+    };
     f16x2 v[4][2];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
       for (int u = 0; u < 2; ++u) v[k][u] = load(k, u);
-    int step = 0;
-    for (; step + 4 <= whole; step += 4) {
+    auto next4 = [&](int step0, auto form) {  // four steps.  0: every token has all of their positions; 1: weights of 0; 2: sums chosen
+      constexpr int FORM = decltype(form)::value;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        f16x2 now[2] = {v[k][0], v[k][1]};
+        const int step = step0 + k;
+        __builtin_amdgcn_sched_barrier(0);  // (else the conversions of all four come first, and wait for the last load)
+        const float now[2][2] = {{(float)v[k][0].x, (float)v[k][0].y}, {(float)v[k][1].x, (float)v[k][1].y}};
 #pragma unroll
-        for (int u = 0; u < 2; ++u) v[k][u] = load(step + k + 4, u);
+        for (int u = 0; u < 2; ++u) v[k][u] = load(step + 4, u);
+        const float* wt = att + n * TP + 32 * min(step, steps - 1) + t0;  // (a row has whole 64s of positions)
+        float w[2] = {wt[0], wt[4]};
+        if (FORM == 1)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const float w = att[n * TP + 32 * (step + k) + t0 + 4 * u];
-          acc[u][0] = __builtin_amdgcn_mfma_f32_16x16x1f32(w, (float)now[u].x, acc[u][0], 0, 0, 0);
-          acc[u][1] = __builtin_amdgcn_mfma_f32_16x16x1f32(w, (float)now[u].y, acc[u][1], 0, 0, 0);
-        }
+          for (int u = 0; u < 2; ++u) w[u] = 32 * step + t0 + 4 * u < len_n ? w[u] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const f32x16 sum = __builtin_amdgcn_mfma_f32_16x16x1f32(w[u], now[u][c], acc[u][c], 0, 0, 0);
+            if (FORM < 2) {
+              acc[u][c] = sum;
+              continue;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[u][c][4 * i + r] = 32 * step + 4 * (G + u) + i < len[r] ? sum[4 * i + r] : acc[u][c][4 * i + r];
+          }
       }
-    }
-    for (; step < steps; ++step) {
-      const f16x2 now[2] = {load(step, 0), load(step, 1)};
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const float w = att[n * TP + min(32 * step + t0 + 4 * u, TP - 1)];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const f32x16 next = __builtin_amdgcn_mfma_f32_16x16x1f32(w, (float)now[u][c], acc[u][c], 0, 0, 0);
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[u][c][4 * k + r] = 32 * step + 4 * (G + u) + k < len[r] ? next[4 * k + r] : acc[u][c][4 * k + r];
-        }
-      }
-    }
+    };
+    int step = 0;
+    for (; step + 4 <= whole; step += 4) next4(step, std::integral_constant<int, 0>{});
+    if (!odd)
+      for (; step < steps; step += 4) next4(step, std::integral_constant<int, 1>{});
+    else
+      for (; step < steps; step += 4) next4(step, std::integral_constant<int, 2>{});
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll

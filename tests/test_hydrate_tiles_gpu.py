@@ -3,7 +3,7 @@ loop's bits (option q2k_tiles = 2), like tests/test_hydrate_gpu.py."""
 import numpy as np
 import pytest
 
-from tests.test_hydrate_gpu import _assert_identical, compare_hydrate
+from tests.test_hydrate_gpu import _assert_identical, _caches, _loop, compare_hydrate
 from tools import synth
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +45,37 @@ def test_latent_attention_of_head_tiles(ctx, P, pos0):
     c = synth.preset("v3", "q2_k", True, n_layers=1, first_k_dense_replace=1, max_seq_len=384, vocab_size=1024)
     tokens = np.random.default_rng(P).integers(0, c.vocab_size, P)
     _assert_identical(compare_hydrate(ctx, c, None, seed=29, tokens=tokens, pos0=pos0), P, pos0)
+
+
+# a key and value that overflow the cache's f16 (infinite) inside a tile of tokens: the tokens before it know nothing of them
+def test_attention_before_an_infinite_value(ctx):
+    import dsk
+    c = synth.preset("tiny_v3", "q2_k", False, n_layers=1, first_k_dense_replace=1, v_head_dim=128, qk_nope_head_dim=128, qk_rope_head_dim=64, max_seq_len=96)
+    T = synth.synth_model(c, seed=5)
+    tokens = [int(t) for t in np.random.default_rng(3).integers(0, c.vocab_size, 30)]
+    norm = T["model.layers.0.attn.kv_a_norm.weight"]
+
+    def run(batched):
+        m = dsk.Model(ctx, c, T, options={"q2k_tiles": 2})
+        try:
+            assert m.hydrate_why_not() == ""
+            m.set_trace(True)
+            if batched:
+                m.hydrate(tokens, 0, dsk.MODE_OUTPUT_LOGITS)
+                x = [m.hydrate_trace_x(0, i) for i in range(len(tokens))]
+            else:
+                x = [a[0] for a in _loop(m, tokens, 0, trace=True)[1]]
+            return x, [np.asarray(r).view(np.float16).astype(np.float32) for r in _caches(m, c, len(tokens))[0]]
+        finally:
+            m.close()
+
+    largest = np.max([np.abs(r).max(axis=1) for r in run(False)[1]], axis=0)
+    first = 1 + int(np.argmax(largest[1:]))
+    norm.data = (norm.data * np.float32(1.05 * 65504 / largest[first])).astype(np.float32)
+    (want, rows), (got, same) = run(False), run(True)
+    bad = ~np.isfinite(rows[0]).all(axis=1) | ~np.isfinite(rows[1]).all(axis=1)
+    assert bad.any() and not bad[0]
+    first = int(np.argmax(bad))
+    for i in range(first):
+        assert np.isfinite(want[i]).all() and np.array_equal(want[i], got[i]), i
+        assert np.array_equal(rows[0][i], same[0][i]) and np.array_equal(rows[1][i], same[1][i]), i
