@@ -3,7 +3,7 @@
 //   lin_kernel      prompts: 128 features x 128 rows per workgroup, 4 waves of 64 x 64, both operands through LDS in fragment
 //                   order (global_load_lds, 16 bytes per lane: LDS reads are lane-linear, no bank conflicts), two buffers
 //   lin_big_kernel  the same with 256 x 256 and a ring of four stages, where there are enough of such tiles (bf16)
-//   few_kernel      up to 16 rows (decoding): 4 waves share 16 features and split k; weights stream from HBM straight into the
+//   few_kernel      up to 16 rows (decoding): 4 waves share 16 or 64 features and split k; weights stream from HBM straight into the
 //                   MFMA operand registers, 1 KiB contiguous per wave and load
 //   expert_kernel   the experts' products of prompts, rows gathered per expert: 256 features x 128 (64, 32) rows, weights straight
 //                   into registers (32 bits: lin_kernel's tiles)
