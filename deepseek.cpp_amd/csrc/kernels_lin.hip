@@ -3,6 +3,7 @@
 //   lin_kernel      prompts: 128 features x 128 rows per workgroup, 4 waves of 64 x 64, both operands through LDS in fragment
 //                   order (global_load_lds, 16 bytes per lane: LDS reads are lane-linear, no bank conflicts), two buffers
 //   lin_big_kernel  the same with 256 x 256 and a ring of four stages, where there are enough of such tiles (bf16)
+//   lin_direct_kernel  32-bit activations times a few k tiles, operands straight from memory
 //   few_kernel      up to 16 rows (decoding): 4 waves share 16 or 64 features and split k; weights stream from HBM straight into the
 //                   MFMA operand registers, 1 KiB contiguous per wave and load
 //   expert_kernel   the experts' products of prompts, rows gathered per expert: 256 features x 128 (64, 32) rows, weights straight
@@ -127,6 +128,55 @@ DEV const T* operand(const LinArgs& a, int feature) {
 __host__ DEV constexpr int lin_stages(int size) { return size == 2 ? 2 : 3; }
 __host__ DEV constexpr int lin_step(int size) { return size == 2 ? 2 : 1; }
 __host__ DEV constexpr int lin_stage(int size) { return lin_step(size) * 8 * 1024 * (1 + size / 2); }
+// 32 features (tiles rt, rt + 1) x 32 rows (from `first` on) of a wave by itself on v_mfma_f32_16x16x4_f32, operands straight from memory: one chain of
+// the instruction per sum.  f0: a feature whose operand it is.
+DEV void direct_tile(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int rt, int first, int k0, int k1) {
+  const int lane = threadIdx.x & 63;
+  const bf16x8* w[2];
+  const float* x[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    w[i] = reinterpret_cast<const bf16x8*>(a.w) + (size_t)min(rt + i, a.rt - 1) * a.kt * 64 + lane;
+    int r = min(first + i * 16 + (lane & 15), n_rows - 1);
+    r = gather ? gather[row0 + r] : row0 + r;
+    x[i] = operand<float>(a, f0) + (size_t)r * a.lda + (lane >> 4) * 8;
+  }
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int kt = k0; kt < k1; kt += 2) {  // (k1 - k0 is even)
+    bf16x8 wk[2][2];
+    f32x8 xk[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        wk[u][i] = w[i][(size_t)(kt + u) * 64];
+        xk[u][i] = *reinterpret_cast<const f32x8*>(x[i] + (size_t)(kt + u) * 32);
+      }
+    __builtin_amdgcn_sched_barrier(0);  // (all on their way first)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = mma(wk[u][i], xk[u][j], acc[i][j]);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = first + j * 16 + (lane & 15);
+    if (r >= n_rows || rt >= a.rt) continue;
+    if (a.epi == LIN_GLU) {
+      store_glu<float>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[0][j], acc[1][j]);
+    } else {
+      store_plain<float>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[0][j]);
+      if (rt + 1 < a.rt) store_plain<float>(a, row0 + r, rt * 16 + 16 + (lane >> 4) * 4, acc[1][j]);
+    }
+  }
+}
 // 128 features from f0 on x n_rows <= 128 rows, k tiles [k0, k1): 4 waves of 64 x 64.  gather: a table (slot -> row) or nullptr; out rows are
 // row0 + local row.
 template <typename T>
@@ -366,6 +416,15 @@ __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_ti
   const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 128, per = part_tiles(a), k0 = blockIdx.y * per;
   a.out_f += blockIdx.y * a.part_stride;
   lin_body<T>(a, nullptr, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
+}
+
+// LinArgs.direct: products of a few k tiles (the decay of time mixing: two), 64 features x 64 rows per workgroup.  Three pieces have nothing to save
+// there, latency and the output bound it: 2048 features of 1996 rows 12.4 us, of 301 rows 8.0 (in three pieces by lin_kernel's tiles 21.6 and 9.6, by
+// its tiles with this instruction 24.8 and 11.6; waves of 64 x 64 with the whole k in one straight line 24.5 and 21.7).  And a sum is one chain, as in
+// few_body: in bfloat16 runs another rounding of the decay turns roundings behind it.
+__global__ __launch_bounds__(256) void lin_direct_kernel(const LinArgs a, const int row_tiles, const int tiles) {
+  const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 64, f0 = b / row_tiles * 64, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  direct_tile(a, nullptr, row0, min(64, a.rows - row0), f0, (f0 >> 4) + (wave & 1) * 2, (wave >> 1) * 32, 0, a.kt);
 }
 
 // 256 features x 256 rows per workgroup: 8 waves of 128 x 64; twice the matrix work per byte staged.  A ring of RING stages of one k tile
@@ -667,6 +726,12 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32) {
     const int row_tiles = cdiv(a.rows, 256), tiles = row_tiles * cdiv(a.rt, 16);
     DSK_TRY(allow_lds(lin_big_kernel, RING * 32 * 1024));
     hipLaunchKernelGGL(lin_big_kernel, dim3(tiles, std::max(a.parts, 1)), dim3(512), RING * 32 * 1024, st, a, row_tiles, tiles);
+    return DSK_OK;
+  }
+  if (a.direct) {
+    if (!f32 || a.parts > 1) DSK_FAIL(DSK_ERR_INVALID, "lin: direct products are 32-bit ones in one part");
+    const int row_tiles = cdiv(a.rows, 64), tiles = row_tiles * cdiv(a.rt, 4);
+    hipLaunchKernelGGL(lin_direct_kernel, dim3(tiles), dim3(256), 0, st, a, row_tiles, tiles);
     return DSK_OK;
   }
   const int row_tiles = cdiv(a.rows, 128), tiles = row_tiles * cdiv(a.rt, 8), lds = lin_lds(f32);

@@ -919,8 +919,9 @@ WkvArgs wkv_args(LayeredModel* m, const PassDesc& p, const LayerSpec& l, const L
 }
 int wkv(LayeredModel* m, const WkvArgs& a, const LayerW& w, bool few) {
   hipStream_t st = m->ctx->stream;
-  // the decay's second product multiplies 32-bit activations, in bfloat16 runs too
-  const LinArgs low = lin_f(w.w_low2, m->narrow + w.w_low, m->ldf, a.p.rows, m->low, m->low_ld);
+  // the decay's second product multiplies 32-bit activations, in bfloat16 runs too: whole, not in bfloat16 pieces
+  LinArgs low = lin_f(w.w_low2, m->narrow + w.w_low, m->ldf, a.p.rows, m->low, m->low_ld);
+  low.direct = 1;
   DSK_TRY(few ? launch_lin_few(st, &low, 1, true) : launch_lin(st, low, true));
   if (in_chunks(m, a.p)) DSK_TRY(launch_wkv_chunks(st, a, m->scan, m->f32));
   else DSK_TRY(launch_wkv_scan(st, a, m->f32));

@@ -78,3 +78,42 @@ def test_steps_of_many_tiles_per_workgroup(ctx, tmp_path, width, ff, vocab):
     assert np.array_equal(decode([16]), few)
     assert np.array_equal(decode([9, 7]), few)
     assert U.err(few[:1], K.want(toks[0])[-1:]) < K.tol
+
+
+# The decay of time mixing multiplies 32-bit activations in bfloat16 runs too, by the 32-bit matrix instruction: a pass of 20 single tokens (a
+# prompt's kernels) and steps of 10 (a step's) give the same bits where every sum runs over one k tile.  Its terms nearly cancel in pairs, so that
+# sums added up otherwise show behind the rounding to bfloat16.
+def test_decay_of_prompts_and_steps_in_bfloat16(ctx, tmp_path):
+    def edit(W):
+        W["l0.mix.w1"][1::2] = W["l0.mix.w1"][::2] * (1 + 2.0 ** -6)
+        W["l0.mix.w2"] *= 256
+        W["l0.mix.w2"][:, 1::2] = -W["l0.mix.w2"][:, ::2]
+    K = U.Case(ctx, tmp_path, U.sandwich([U.no_ff(U.wkv(2, 16))], width=32), edit=edit, dtype="bfloat16", options="fused_decode=0", rank_a=32)
+    toks = [K.tokens(16, seed=n) for n in range(20)]
+    K.lm.set_trace(True)
+
+    def rows(size):
+        seqs, out = [K.lm.seq_open() for _ in toks], []
+        for i in range(16):
+            for a in range(0, 20, size):
+                K.lm.step([(s, t[i:i + 1], []) for s, t in zip(seqs[a:a + size], toks[a:a + size])])
+                out.append(K.lm.trace_rows(0, size))
+        for s in seqs:
+            K.lm.seq_close(s)
+        return np.concatenate(out)
+
+    assert np.array_equal(rows(20), rows(10))
+
+
+# its kernel: 64 features x 64 rows a workgroup, 32 x 32 a wave.  Feature tiles that end inside a wave's pair, a k of two and of four tiles
+@pytest.mark.parametrize("heads,dim,rank", [(3, 20, 12), (5, 20, 70), (2, 52, 33), (1, 16, 100)])
+def test_decay_at_the_edges_of_its_tiles(ctx, tmp_path, heads, dim, rank):
+    K = U.Case(ctx, tmp_path, U.sandwich([U.no_ff(U.wkv(heads, dim))]), rank_a=rank)
+    t, want = K.tokens(131), []
+    K.ref.run(U.O.Sequence(K.ref), t, want)
+    K.lm.set_trace(True)
+    for n in (17, 31, 32, 33, 63, 64, 65, 97, 128, 131):
+        s = K.lm.seq_open()
+        K.lm.step([(s, t[:n], [n - 1])])
+        assert U.err(K.lm.trace_rows(0, n), want[0][:n]) < U.F32, n
+        K.lm.seq_close(s)
