@@ -245,9 +245,9 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
     }
   } else {
     // While a k tile is multiplied the next one's operands are read into the other set of registers and the loads of R - 1 more are on
-    // their way.  What bounds it: per wave and k tile 48 matrix instructions (768 cycles) and the 208 vector instructions (832 cycles)
+    // their way.  What bounds it: per wave and k tile 48 matrix instructions (768 cycles) and the 176 vector instructions (704 cycles)
     // that take 32 activations apart; they are issued in turns, a row group's matrix work beside the splitting of the next.
-    // 301 x 2048 x 16896: 303 us with v_mfma_f32_16x16x4_f32, 101 us so; 301 x 16896 x 2048 in 4 parts: 304 -> 114 us.
+    // 301 x 2048 x 16896: 303 us with v_mfma_f32_16x16x4_f32, 97 us so; 301 x 16896 x 2048 in 4 parts: 304 -> 108 us.
     struct Operands {
       bf16x8 w[4];
       f32x8 x[4];
@@ -284,12 +284,12 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        if (j == 0) __builtin_amdgcn_sched_group_barrier(0x002, 52, 0);
+        if (j == 0) __builtin_amdgcn_sched_group_barrier(0x002, 48, 0);
 #pragma unroll
         for (int i = 0; i < 12; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           if (j == 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          if (j < 3) __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+          if (j < 3) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
         }
       }
     };
@@ -304,6 +304,20 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
       step(kt + 1, q, p);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // Three pieces stand for the activation while everything is finite: an infinity's rest is no number, and neither is a zero rest times an
+    // infinite weight.  A wave with a sum that is not finite adds its tiles up again.
+    float bad = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad = fmaf(acc[i][j][e], 0.f, bad);
+    if (__any(bad != bad)) {
+#pragma unroll 1
+      for (int i = 0; i < 4; ++i) direct_tile(a, gather, row0, n_rows, f0, rt0 + wm * 4 + (i & 1) * 2, wn * 64 + (i >> 1) * 32, k0, k1);
+      return;
+    }
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {

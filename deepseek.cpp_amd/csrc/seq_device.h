@@ -41,10 +41,11 @@ DEV f32x4 mma(const f32x8& w, const f32x8& a, f32x4 c) {
   return c;
 }
 
-// A 32-bit activation as the exact sum of three bf16 numbers: its top 8 significant bits, the next 8, the last 8 (cut off, not rounded, so
-// that each rest is exact; b2 alone can fall under the smallest bf16, below 2^-110).  A product with a bf16 weight is then three bf16
+// A finite 32-bit activation as the exact sum of three bf16 numbers: its top 8 significant bits, the next 8, the last 8 (cut off, not rounded, so
+// that each rest is exact; b2 alone can fall under the smallest bf16, below 2^-110).  A product with a finite bf16 weight is then three bf16
 // products, each exact in 32 bits and summed in 32 bits: the precision of v_mfma_f32_16x16x4_f32 at a fifth of its cycles (three
-// 16x16x32 of 16 cycles for eight of 32).
+// 16x16x32 of 16 cycles for eight of 32).  Where an activation or a weight is not finite the sum of the three is no finite number either,
+// but not always the right one: such sums are added up again by that instruction (lin_body).
 struct Split {
   bf16x8 b0, b1, b2;
 };
@@ -56,8 +57,7 @@ DEV Split split3(const f32x8& x) {
   for (int i = 0; i < 8; ++i) {
     const float v = x[i];  // (a bit cast of an element of a vector reads element 0)
     const unsigned bits = __builtin_bit_cast(unsigned, v);
-    // (of an infinity: inf - inf, NaN, for which fmaxf takes a number that is small beside it; no other rest is below -2^121)
-    const float r = fmaxf(v - __builtin_bit_cast(float, bits & 0xffff0000u), -0x1p121f);
+    const float r = v - __builtin_bit_cast(float, bits & 0xffff0000u);  // (of an infinity or no number: no number)
     const unsigned rest = __builtin_bit_cast(unsigned, r);
     p0[i] = bits;
     p1[i] = rest;

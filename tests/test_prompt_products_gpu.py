@@ -80,6 +80,44 @@ def test_steps_of_many_tiles_per_workgroup(ctx, tmp_path, width, ff, vocab):
     assert U.err(few[:1], K.want(toks[0])[-1:]) < K.tol
 
 
+# Infinite weights and activations that overflow, in 32 bits: an infinite sum comes out, as it does of one 32-bit instruction, wherever its terms
+# agree in sign (of an activation's three pieces the last is zero once in 256, and zero times infinity is no number)
+@pytest.mark.parametrize("where", ["expert", "head", "hidden"])
+def test_infinite_values_in_32_bit_products(ctx, tmp_path, where):
+    width, ff, n = 120, 40, 60
+
+    def edit(W):
+        no_mixers(W)
+        if where == "head":
+            for v in range(203):
+                W["head"][v, v % width] = np.inf * (-1) ** v
+        elif where == "expert":
+            for f in range(0, width, 2):
+                W["l0.mlp.e0.down"][f, f % ff] = np.inf
+        else:  # a hidden value of 1e25 x 1e25, times weights on both sides of 128
+            W["l0.mlp.e0.gate"][3] *= 1e25
+            W["l0.mlp.e0.up"][3] *= 1e25
+            W["l0.mlp.e0.down"][:, 3] = np.resize([0.5, 300, -128, 2.0 ** 20, -1, 127], width)
+    layer = U.parallel(mlp=U.moe(1, 1, ff, 3e38 if where == "hidden" else 0.8, 0))
+    K = U.Case(ctx, tmp_path, U.config([layer], width=width), edit=edit)
+    t, trace = K.tokens(n), []
+    with np.errstate(all="ignore"):
+        logits = K.ref.run(U.O.Sequence(K.ref), t, trace)
+    K.lm.set_trace(True)
+    s = K.lm.seq_open()
+    got = K.lm.step([(s, t, range(n))])
+    want = logits
+    if where != "head":
+        got = K.lm.trace_rows(0, n)
+        with np.errstate(over="ignore"):
+            want = trace[0].astype(np.float32)
+        assert np.isinf(want).any()
+    assert not np.isnan(want).any()
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf]) and np.isfinite(got[~inf]).all()
+    assert np.abs(got[~inf] - want[~inf]).max() < U.F32 * 20
+
+
 # The decay of time mixing multiplies 32-bit activations in bfloat16 runs too, by the 32-bit matrix instruction: a pass of 20 single tokens (a
 # prompt's kernels) and steps of 10 (a step's) give the same bits where every sum runs over one k tile.  Its terms nearly cancel in pairs, so that
 # sums added up otherwise show behind the rounding to bfloat16.
