@@ -671,11 +671,11 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
     const int nr = f.down ? NT : GT;
     if (tile * nr >= a.rt) return;
     // a lane whose row did not choose the expert reads the first row that did: a load of the operand then touches as many lines as the expert has
-    // rows, not 16
+    // rows, not 16.  (A scalar read of that lane: a lane exchange in a branch reads nothing of lanes that are not in it.)
     const int slot = c < f.m.rows ? f.m.active_slot[i * 16 + c] : -1;
     const int own = min(c, f.m.rows - 1) * (f.m.top + f.m.shared) + max(slot, 0);
-    const int one = max(__ffsll(__ballot(slot >= 0)) - 1, 0);
-    const int row = slot >= 0 ? c : one, pos = slot >= 0 ? own : __shfl(own, one);
+    const int one = max(__ffsll(__ballot(slot >= 0)) - 1, 0), first = __builtin_amdgcn_readlane(own, one);
+    const int row = slot >= 0 ? c : one, pos = slot >= 0 ? own : first;
     const int out = slot >= 0 ? own : -1;
     if (f.down) few_body<T, NT, false>(a, tile * NT, 0, a.kt, pos, out, lds);
     else few_body<T, GT, true>(a, tile * GT, 0, a.kt, row, out, lds);
