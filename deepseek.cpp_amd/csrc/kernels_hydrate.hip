@@ -1223,11 +1223,11 @@ __global__ __launch_bounds__(256, 2) void hyd_attn_tile_kernel(const AttnMhaArgs
 #pragma unroll
   for (int r = 0; r < 4; ++r) o[r][0] = o[r][1] = 0.f;
   const int whole = least / 32, steps = (most + 31) / 32;  // steps that every token has all positions of; all steps
-  // Behind them a token without a position has weight 0 for it: nothing is added, unless the value (of a later token) is no number.  Then, and
-  // only then, sums are chosen one by one.
+  // Behind them a token without a position has weight 0 for it: nothing is added, unless the value is infinite or no number.  Then, and only then,
+  // sums are chosen one by one.  (Values of later tokens, and those of the last step, which the steps past the end read again.)
   const int len_n = sps[token(n)].kv_len;
   bool odd = false;
-  for (int t = 32 * whole + (lane >> 4) * 2; t < most; t += 8)  // (this wave's 32 columns)
+  for (int t = 32 * min(whole, steps - 1) + (lane >> 4) * 2; t < most; t += 8)  // (this wave's 32 columns)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const u32 two = __builtin_amdgcn_raw_buffer_load_b32(RV, ((min(t + u, most - 1) * H + h) * HYD_AT_V + 32 * wave + 2 * n) * 2, 0, 0);

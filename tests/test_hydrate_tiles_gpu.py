@@ -79,3 +79,36 @@ def test_attention_before_an_infinite_value(ctx):
     for i in range(first):
         assert np.isfinite(want[i]).all() and np.array_equal(want[i], got[i]), i
         assert np.array_equal(rows[0][i], same[0][i]) and np.array_equal(rows[1][i], same[1][i]), i
+
+
+# An infinite value inside every token's context: attention gives what the kernel for few tokens gives (chunks of up to 7), a tile of a single token whose
+# context is whole steps of 32 included (the 17th: 32, 96 or 128 positions)
+@pytest.mark.parametrize("pos0", [15, 79, 111])
+def test_attention_over_an_infinite_value(ctx, pos0):
+    import dsk
+    c = synth.preset("tiny_v3", "q2_k", False, n_layers=1, first_k_dense_replace=1, v_head_dim=128, qk_nope_head_dim=128, qk_rope_head_dim=64, max_seq_len=160)
+    T = synth.synth_model(c, seed=5)
+    tokens = [int(t) for t in np.random.default_rng(3).integers(0, c.vocab_size, pos0 + 17)]
+    width = c.n_heads * 128
+
+    def run(sizes):
+        m = dsk.Model(ctx, c, T, options={"q2k_tiles": 2, "hydrate_tap_layer": 0})
+        try:
+            assert m.hydrate_why_not() == ""
+            m.hydrate(tokens[:pos0], 0)
+            rows = m.get_cache_rows(0, "v_cache", 0, pos0, width)
+            for i in (0, pos0 - 1):  # (columns of two waves)
+                rows[i, 5 + i % 2 * 64::128] = 0x7C00
+            m.set_cache_rows(0, "v_cache", 0, rows)
+            out, at = [], pos0
+            for n in sizes:
+                m.hydrate(tokens[at:at + n], at)
+                out.append(m.hydrate_buffer("att_out", 0, n, width))
+                at += n
+            return np.concatenate(out)
+        finally:
+            m.close()
+
+    want, got = run([7, 7, 3]), run([17])
+    assert np.isposinf(want).any(axis=1).all() and not np.isnan(want).any()
+    assert np.array_equal(want, got, equal_nan=True)
