@@ -1854,10 +1854,12 @@ int launch_hyd_router(hipStream_t st, const RouterArgs& a, int P, float* Y) {
   const size_t lds = (size_t)P * 16 * 4;
   if (Y && a.norm_w && a.dim % 256 == 0 && chunk <= 2048 && lds <= 60 * 1024 && a.n_routed <= 1024) {
     hipLaunchKernelGGL(hyd_router_norm_kernel, dim3(P), dim3(1024), 0, st, a, Y);
-    // 32 rows a wave where that gives every CU a workgroup, 16 below; a few tokens alone: rows in registers
+    // Up to 44 tokens with a row's weights in registers and the tokens one by one, half a microsecond each; 16 tokens at a time take what their chains
+    // take, however many: 256 rows of 7168, 16 / 44 / 48 tokens 11.8 / 27.1 / 29.3 us against 27.5 / 27.7 / 27.6.  32 rows a wave where that gives
+    // every CU a workgroup, 16 below.
     const int wide = (P + 15) / 16 * ((a.n_routed + 31) / 32) >= 256 ? 2 : 1;
     const dim3 tiles((P + 15) / 16, (a.n_routed + 16 * wide - 1) / (16 * wide));
-    if (P >= 16) {
+    if (P > 44) {
       auto k = RW == 2 ? (wide == 2 ? hyd_router_tile_kernel<8, 2> : hyd_router_tile_kernel<8, 1>) : (wide == 2 ? hyd_router_tile_kernel<4, 2> : hyd_router_tile_kernel<4, 1>);
       hipLaunchKernelGGL(k, tiles, dim3(64 * SL), 0, st, a.w, Y, a.dim, a.n_routed, P, a.partial);
     } else if (RW == 2) hipLaunchKernelGGL(hyd_router_rows_kernel<2>, dim3((a.n_routed + 1) / 2), dim3(1024), lds, st, a.w, Y, a.dim, a.n_routed, P, a.partial);
