@@ -383,9 +383,7 @@ static int hyd_layer(dsk_model* m, int l, int P, int max_kv, int n_short) {
     DSK_TRY(hyd_gemm(m, L.t[DSK_ROLE_SHARED_W2], nullptr, h.a_hsh, P, P, h.eout_sh, dim, EPI_STORE));
   }
   const DTensor &w1 = L.t[DSK_ROLE_W1], &w2 = L.t[DSK_ROLE_W2], &w3 = L.t[DSK_ROLE_W3];
-  // 4 tokens per wave and pass unless the experts are crowded: 8 tokens cost the GLU pair half of its waves (260 registers), while a
-  // second pass over a strip re-reads 75 KB that the first pass just pulled through L2
-  const int nq_e = 1;  // (tasks of 5 rows and more go through the 16-token form: what is left for the quads fits one pass)
+  // (4 tokens per wave and pass: tasks of 5 rows and more go through the 16-token form, one pass takes what is left for the quads)
   {
     HydGemmArgs A;
     memset(&A, 0, sizeof A);
@@ -395,7 +393,7 @@ static int hyd_layer(dsk_model* m, int l, int P, int max_kv, int n_short) {
     A.a_dig = h.a_x.dig;
     A.list = h.list; A.count = h.count; A.list_stride = h.cap;
     A.out = h.hb; A.out_stride = mi; A.act = c.act;
-    DSK_TRY(launch_hyd_gemm(st, A, nq_e));
+    DSK_TRY(launch_hyd_gemm(st, A, 1));
   }
   DSK_TRY(launch_quantize_q8k(st, h.hb, P * K * mi, h.a_hb.qs, h.a_hb.d, h.a_hb.bsums));
   DSK_TRY(launch_hyd_digits(st, h.a_hb.bsums, h.a_hb.dig, (size_t)P * K * (mi / 16)));
@@ -407,7 +405,7 @@ static int hyd_layer(dsk_model* m, int l, int P, int max_kv, int n_short) {
     A.a_dig = h.a_hb.dig;
     A.list = h.list; A.count = h.count; A.list_stride = h.cap;
     A.out = h.eout; A.out_stride = dim; A.epilogue = EPI_STORE; A.act = c.act;
-    DSK_TRY(launch_hyd_gemm(st, A, nq_e));
+    DSK_TRY(launch_hyd_gemm(st, A, 1));
   }
   DSK_TRY(launch_hyd_combine(st, h.X, h.eout, h.route_w, shn > 0 ? h.eout_sh : nullptr, P, K, dim));
   if (l == m->hydrate_tap_layer) {

@@ -290,15 +290,17 @@ __global__ __launch_bounds__(SPREAD && !GLU ? 512 : 256) void hyd_gemm_kernel(co
 }
 
 // ------------------------------------------------------------------------------------
-// Plain matrices times MANY tokens: 16 tokens per wave and pass, the matrix instruction's whole N side.
+// Matrices times MANY tokens: 16 tokens per matrix instruction, its whole N side (hyd_gemm16_kernel: one or two such groups a pass;
+// hyd_gemm16k_kernel: one).
 // The K side of one instruction is one sub-block GROUP g (sub-blocks 4 g .. 4 g + 3: what the float stage keeps apart), so
 // D_g[token][row] is the exact group sum with no zero padding: K-group kg' of lane (row n, kg') carries sub-block 4 g + kg' =
 // field 2 (g & 1) + (kg' >> 1) of the qs bytes of K-group 2 (g >> 1) + (kg' & 1) - the lane's own 16 bytes or those of the lane
 // 32 away (one v_permlane32_swap per dword gives both) - scaled as in hyd_expand; the activation operand of lane (token t, kg') is
 // the token's 16 codes of that sub-block in natural order: four plain 16-byte loads per block, no selector rows.
-// The min term rides the matrix pipe too: a sub-block sum b (|b| <= 2032) is split b = 8 (v1 + v2) + v0 with all three in int8 range,
-// and K slot (sub-block j, {v0, v1, v2, 0}) meets the weight side's {m_j, 8 m_j, 8 m_j, 0} (8 m_j <= 120): the instruction returns
-// sum_j m_j b_j exactly; one instruction per group (the activation side masked to the group's lanes).
+// The min term rides the matrix pipe too.  hyd_gemm16_kernel: in f16, all four groups in one instruction (there).  hyd_gemm16k_kernel, in
+// integers: a sub-block sum b (|b| <= 2048) is split b = 8 (v1 + v2) + v0 with all three in int8 range, and K slot (sub-block j,
+// {v0, v1, v2, 0}) meets the weight side's {m_j, 8 m_j, 8 m_j, 0} (8 m_j <= 120): the instruction returns sum_j m_j b_j exactly; one
+// instruction per group (the activation side masked to the group's lanes).
 // In the C/D layout lane (n, q) holds tokens 4 q .. 4 q + 3 of its row: the float stage (hyd_block's, per token) is lane-local.
 // Same integers, same float chains as hyd_gemm_kernel: same bits.
 // ------------------------------------------------------------------------------------
@@ -818,7 +820,7 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
       return;
     }
     // 32 tokens a pass where that leaves most CUs a workgroup, else 16; then as many strips per workgroup as still do (the staging is paid once
-    // per workgroup, and every choice puts the same number of waves on the chip); at least 2 waves (the staging indices assume >= 128 threads)
+    // per workgroup, and every choice puts the same number of waves on the chip); at least 2 waves, a GLU pair's
     const int per = GLU ? 2 : 1, chunks2 = (A.m + 31) / 32;
     auto groups = [&](int nw) { return (unsigned)((units * per + nw - 1) / nw); };
     if (A.m > 16 && (long long)groups(8) * chunks2 >= 192) {
@@ -1316,7 +1318,9 @@ int launch_hyd_attn(hipStream_t st, const AttnMhaArgs& a, const StepParams* sps,
   if (lds > 96 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_attn: kv_len %d does not fit LDS", max_kv);
   if (a.head_dim > 256 || a.v_dim > 256) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_attn: head_dim %d / v_head_dim %d", a.head_dim, a.v_dim);
   if (n_split > MHA_SPLIT_MAX) n_split = MHA_SPLIT_MAX;  // (launch_head_attn's clamp)
-  // 16 tokens at a time while a context is one softmax and one position a thread (the chunk's contexts are max_kv - P + 1 ... max_kv)
+  // 16 tokens at a time while a context is one softmax and one position a thread (the chunk's contexts are max_kv - P + 1 ... max_kv).  From 8 on:
+  // a tile takes nearly the same for 8 and 16, the kernel behind it half of that for 8.  DeepSeek-V3's heads, contexts that end at 8, 128, 258, 508
+  // and 908, 8 tokens: 12.4, 16.2, 25.9, 32.6, 55 us against 11.8, 18.9, 24.7, 36.8, 64; 16 tokens: 14, 22, 27, 39, 57 against 23, 33, 42, 68, 116.
   const int limit = std::min((int)HYD_AT_MAX_KV, n_split > 1 ? split_min - 1 : max_kv);
   const int n_tile = std::max(0, std::min(P, P - (max_kv - limit)));
   if (n_tile >= 8 && a.v_dim == HYD_AT_V && a.head_dim % 16 == 0 && a.head_dim <= 64 * HYD_AT_NJ && a.rope <= 128) {
@@ -1661,7 +1665,9 @@ int launch_hyd_mla_attn(hipStream_t st, const AttnMlaArgs& a, const StepParams* 
   if (a.lora > 512 || a.lora % 64 || a.rope > 64 || a.rope % 4) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_mla_attn: kv_lora_rank %d / rope %d", a.lora, a.rope);
   const size_t lds = (size_t)max_kv * 4;
   if (lds > 96 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_mla_attn: kv_len %d does not fit LDS", max_kv);
-  // 16 heads of a token at a time; below 8 tokens a workgroup per head fills more of the card (8 workgroups a token against 128)
+  // 16 heads of a token at a time; below 8 tokens a workgroup per head fills more of the card (8 workgroups a token against 128).  DeepSeek-V3's
+  // heads, contexts that end at 8, 68, 138 and 308, 8 tokens: 12.8, 22.2, 32.4, 53 us against 15.3, 23.6, 35.8, 57; 16 tokens: 13, 23, 33, 55
+  // against 32, 49, 72, 112.
   if (P >= 8 && a.lora == HYD_ML_L && a.rope % 16 == 0 && a.n_heads % 16 == 0 && max_kv <= HYD_AT_MAX_KV) {
     const int bytes = 16 * hyd_at_row(max_kv) * 4;
     hipFuncSetAttribute((const void*)hyd_mla_attn_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
@@ -1683,7 +1689,7 @@ int launch_hyd_head_list(hipStream_t st, int* list, int* count, int H, int P, in
 // norm and re-reads the 7.3 MB of router weights per token; here
 //   1. hyd_router_norm_kernel  per token: the router's own rmsnorm scale (router_norm_scale: the 1024-thread tree), the normed
 //      vector y = x * scale * w as f32, and its Q8_K copy - what the experts AND the shared expert's rider consume in decode;
-//   2. hyd_router_rows_kernel  per workgroup RW rows x 16 / RW column slices like router_body, the weights of a (row, slice)
+//   2. hyd_router_rows_kernel (to 44 tokens; then hyd_router_tile_kernel)  per workgroup RW rows x 16 / RW column slices like router_body, the weights of a (row, slice)
 //      held in REGISTERS across all P tokens: per token the same fma chain over the same values, the same wave tree, the
 //      same slice-order sum;
 //   3. hyd_gate_kernel         per token: gate_body on the scores.

@@ -338,9 +338,10 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
 
 // bf16, 256 features x up to 16 NJ rows: 4 waves of 64 features each, all of them on every row.  A weight tile is one wave's own, so weights go
 // straight into its registers a step (two k tiles) ahead - 1 KiB of consecutive bytes a load -, and LDS holds the rows alone: 8 + NJ operand
-// reads out of it feed 4 NJ matrix instructions where lin_body needs 16 for 16.  What bounds it is what a compute unit takes out of L2 (about
-// 48 GB/s) and, with the last tiles of experts seldom full, work on rows that are not there: hence NJ = 8, 4 and 2.  64 experts of 1408 over
-// 2048 rows, top 6, width 2048: gate / up 337 -> 254 us, down 201 -> 164 us (lin_body with a grid of row tiles x feature tiles before).
+// reads out of it feed 4 NJ matrix instructions where lin_body needs 16 for 16.  What bounds it is what compute units take out of L2 (the gate /
+// up launch below about 2.5 GB: 10 TB/s over the card) and, with the last tiles of experts seldom full, work on rows that are not there: hence
+// NJ = 8, 4 and 2.  64 experts of 1408 over 2048 rows, top 6, width 2048: gate / up 337 -> 254 us, down 201 -> 164 us (lin_body with a grid of
+// row tiles x feature tiles before).
 // For plain products, whose row tiles are full, it is within 3 % of lin_kernel either way, and lin_big_kernel has more work per byte.
 template <int NJ>
 __host__ DEV constexpr int wide_stage() { return 2 * NJ * 1024; }

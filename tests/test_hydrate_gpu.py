@@ -101,7 +101,7 @@ def _assert_identical(res, P, pos0):
 def test_hydrate_equals_the_loop_tiny(ctx, P, pos0, chunk, mla):
     """tiny DeepSeek-V3 Q2_K model, MHA and MLA (1 dense + 2 MoE blocks, 16 experts top-4, rows of <= 8 blocks: single-block items):
     token quads that are full, ragged and single; 13 - 48 tokens: the 16-token GEMM forms (plain matrices from 12 tokens on, expert
-    tasks from 6 rows on) with ragged last chunks; chunks that split the prompt (attention over rows an earlier chunk wrote)"""
+    tasks from 5 rows on) with ragged last chunks; chunks that split the prompt (attention over rows an earlier chunk wrote)"""
     c = synth.preset("tiny_v3", "q2_k", mla)
     T = synth.synth_model(c, seed=41)
     rng = np.random.default_rng(P * 31 + pos0)

@@ -89,7 +89,9 @@ def main():
     c.max_seq_len = 1100
     ctx = dsk.Ctx(0)
     opts = {kv.split("=")[0]: int(kv.split("=")[1]) for kv in a.opt}
-    print(json.dumps(measure(ctx, c, [int(p) for p in a.P.split(",")], a.reps, chunk=a.chunk, opts=opts, loop=not a.no_loop, pos0=a.pos0)))
+    from bench import csrc_sha
+    out = measure(ctx, c, [int(p) for p in a.P.split(",")], a.reps, chunk=a.chunk, opts=opts, loop=not a.no_loop, pos0=a.pos0)
+    print(json.dumps(dict(out, attn=a.attn, csrc_sha=csrc_sha())))
 
 
 if __name__ == "__main__":

@@ -135,9 +135,10 @@ def deepseek(ctx, size, prompts, steps=32, ctx_len=512, reps=2, graph=True):
 
 def measure(size="lite", prompts=(512, 2048), batches=(1, 4, 16), compare=True, steps=32, graph=True, ours=True, design="timerax"):
     import dsk
+    from bench import csrc_sha
     ctx = dsk.Ctx(0)
     out = {"metric": f"layered design ({design.capitalize()}) prefill and decode throughput, {size}", "unit": "tok/s", "data": "synthetic (random weights)",
-           "dtype": "bf16"}
+           "dtype": "bf16", "csrc_sha": csrc_sha()}
     if ours:
         out[design] = layered(ctx, size, list(prompts), list(batches), steps, graph=graph, design=design)
         out["value"] = out[design]["decode"][str(batches[0])]["tok_s"]
