@@ -155,3 +155,22 @@ def test_decay_at_the_edges_of_its_tiles(ctx, tmp_path, heads, dim, rank):
         K.lm.step([(s, t[:n], [n - 1])])
         assert U.err(K.lm.trace_rows(0, n), want[0][:n]) < U.F32, n
         K.lm.seq_close(s)
+
+
+# Logits of up to 16 rows are stored into host memory by the product where the vocabulary is whole tiles of 16 (208), else copied behind it (203);
+# more rows are copied.  Rows of prompts and of single tokens (eager, captured, replayed)
+@pytest.mark.parametrize("vocab", [208, 203])
+def test_logits_of_few_and_many_rows(ctx, tmp_path, vocab):
+    K = U.Case(ctx, tmp_path, U.config([U.parallel(mlp=U.moe())], vocab=vocab), dtype="float32")
+    t = K.tokens(26)
+    want = K.want(t)
+    for n in (1, 2, 15, 16, 17, 19):
+        s = K.lm.seq_open()
+        got = K.lm.step([(s, t[:20], range(20 - n, 20))])
+        assert got.shape == (n, vocab) and U.err(got, want[20 - n:20]) < U.F32, n
+        for i in range(20, 26):
+            assert U.err(K.lm.step([(s, t[i:i + 1], [0])]), want[i:i + 1]) < U.F32, (n, i)
+        K.lm.seq_close(s)
+    seqs = [K.lm.seq_open() for _ in range(17)]
+    for i in range(6):
+        assert U.err(K.lm.step([(s, t[i:i + 1], [0]) for s in seqs]), np.repeat(want[i:i + 1], 17, 0)) < U.F32, i
