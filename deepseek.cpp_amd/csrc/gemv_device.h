@@ -17,6 +17,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 #define DEV __device__ __forceinline__
+#include "glob_device.h"
+DEV GemvTask glob(GemvTask t) {  // a task of a launch's descriptor
+  t.qs = glob(t.qs); t.sc = glob(t.sc); t.hm = glob(t.hm); t.dm = glob(t.dm); t.scale = glob(t.scale);
+  t.qs2 = glob(t.qs2); t.sc2 = glob(t.sc2); t.hm2 = glob(t.hm2); t.dm2 = glob(t.dm2); t.scale2 = glob(t.scale2);
+  t.expert_ids = glob(t.expert_ids);
+  t.a_qs = glob(t.a_qs); t.a_d = glob(t.a_d); t.a_bsums = glob(t.a_bsums); t.a_f32 = glob(t.a_f32); t.norm_w = glob(t.norm_w);
+  t.out = glob(t.out); t.accum_w = glob(t.accum_w);
+  return t;
+}
 
 // hipcc would select the two-operand v_dot4c for this builtin and zero the accumulator of every chain with a v_mov: 4 of
 // ~75 instructions per Q2_K item in VALU-bound kernels.  The Makefile therefore builds the kernels without the dot6-insts

@@ -15,7 +15,7 @@ static int cdiv(int a, int b) { return (a + b - 1) / b; }
 template <typename T>
 __global__ __launch_bounds__(256) void chunk_prep_kernel(const ChunkAttnArgs a) {
   const int row = blockIdx.x, lane = threadIdx.x & 63;
-  const SeqDesc sq = a.p.seqs[a.p.row_seq[row]];
+  const SeqDesc sq = seq_at(a.p.seqs + a.p.row_seq[row]);
   const float pos = (float)(sq.pos0 + row - sq.row0);
   const T* P = reinterpret_cast<const T*>(a.proj_t) + (size_t)row * a.ld;
   const int n_heads = a.heads + 2 * a.kv_heads;
@@ -85,7 +85,7 @@ struct ChunkKeys {
 template <typename T, int KT, int VTL>
 ATTN_KERNEL(T) void chunk_attn_kernel(const ChunkAttnArgs a) {
   const int h = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;  // (a sequence's last tiles have the most keys: they start first)
-  const SeqDesc s = a.p.seqs[a.p.qtile[2 * tile]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.qtile[2 * tile]);
   attn_tile<T, KT, VTL>(ChunkKeys<T>{a, s, h, h / (a.heads / a.kv_heads)}, s, a.p.qtile[2 * tile + 1], a.dim_p >> 5, a.vdim_p >> 4, a.vdim, a.scale,
                         reinterpret_cast<T*>(a.out_t) + h * a.vdim, a.out_ld);
 }
@@ -94,7 +94,7 @@ ATTN_KERNEL(T) void chunk_attn_kernel(const ChunkAttnArgs a) {
 template <typename T>
 __global__ __launch_bounds__(256) void chunk_store_kernel(const ChunkAttnArgs a) {
   const int row = blockIdx.x;
-  const SeqDesc sq = a.p.seqs[a.p.row_seq[row]];
+  const SeqDesc sq = seq_at(a.p.seqs + a.p.row_seq[row]);
   const int pos = sq.pos0 + row - sq.row0, end = sq.pos0 + sq.len - 1;
   if (pos / a.chunk != end / a.chunk) return;
   const int nk = a.kv_heads * a.dim_p, nv = a.kv_heads * a.vdim_p;

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const DeltaArgs a, f
   extern __shared__ float lds[];
   const int tid = threadIdx.x, h = blockIdx.y, dim = a.dim, dp = (dim + 15) / 16 * 16;
   float *sk = lds, *sq = sk + 16 * dp, *sg = sq + 16 * dp, *sA = sg + 16 * dp, *sb = sA + 16 * 17;
-  const SeqDesc s = a.p.seqs[a.p.chunk[2 * blockIdx.x]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.chunk[2 * blockIdx.x]);
   const int t0 = a.p.chunk[2 * blockIdx.x + 1], n = min((int)CH, s.len - t0);
   const int kv = h / (a.heads / a.kv_heads), nq = a.kv_heads * dim;
   const size_t row0 = (size_t)s.row0 + t0;
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const DeltaArgs a, f
 // m_t = max(f_t + m_(t-1), i_t) composes: (F, I) then (f, i) = (F + f, max(I + f, i)); one wave per (head, sequence), 64 tokens a turn
 __global__ __launch_bounds__(64) void mlstm_gates_kernel(const MlstmArgs a, const ChunkScan c) {
   const int lane = threadIdx.x, h = blockIdx.x;
-  const SeqDesc s = a.p.seqs[blockIdx.y];
+  const SeqDesc s = seq_at(a.p.seqs + blockIdx.y);
   float* M = reinterpret_cast<float*>(s.state + a.off_m) + h;
   float m = s.pos0 > 0 ? M[s.flip * a.heads] : 0.f;
   for (int t0 = 0; t0 < s.len; t0 += 64) {
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void mlstm_prepare_kernel(const MlstmArgs a, c
   extern __shared__ float lds[];
   const int tid = threadIdx.x, h = blockIdx.y, dim = a.dim, dp = (dim + 15) / 16 * 16;
   float *sk = lds, *sq = sk + 16 * dp, *keep = sq + 16 * dp, *add = keep + 16;
-  const SeqDesc s = a.p.seqs[a.p.chunk[2 * blockIdx.x]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.chunk[2 * blockIdx.x]);
   const int t0 = a.p.chunk[2 * blockIdx.x + 1], n = min((int)CH, s.len - t0);
   const size_t row0 = (size_t)s.row0 + t0;
   for (int i = tid; i < 16 * dp; i += 256) {
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void wkv_prepare_kernel(const WkvArgs a, float
   extern __shared__ float lds[];
   const int tid = threadIdx.x, h = blockIdx.y, dim = a.dim, dp = (dim + 15) / 16 * 16;
   float *sk = lds, *sq = sk + 16 * dp, *sg = sq + 16 * dp, *su = sg + 16 * dp;
-  const SeqDesc s = a.p.seqs[a.p.chunk[2 * blockIdx.x]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.chunk[2 * blockIdx.x]);
   const int t0 = a.p.chunk[2 * blockIdx.x + 1], n = min((int)CH, s.len - t0);
   const size_t row0 = (size_t)s.row0 + t0;
   for (int i = tid; i < 16 * dp; i += 256) {  // rows past the end: no key, no query, no decay
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ScanArgs a) {
   const int cols = NORM ? a.vdim + 1 : a.vdim;
   const int col = blockIdx.x * 16 + c16;
   const bool live = col < cols, norm = NORM && col == a.vdim;
-  const SeqDesc s = a.p.seqs[blockIdx.z];
+  const SeqDesc s = seq_at(a.p.seqs + blockIdx.z);
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * a.dim * a.vdim;
   float* N0 = !NORM ? nullptr : reinterpret_cast<float*>(s.state + a.off_n) + (size_t)h * a.dim;
   const size_t nn = (size_t)a.heads * a.dim;

@@ -89,7 +89,7 @@ DEV void gemv_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, const vo
     grp_idx = g;
   }
   auto task_of = [&](int ti) {
-    GemvTask T = L.t[ti];
+    GemvTask T = glob(L.t[ti]);
     if (bd) {  // re-base the one task to this workgroup's head
       const size_t per = (size_t)T.rows * T.n;
       if (QT == DSK_QUANT_Q2_K) {
@@ -140,7 +140,7 @@ DEV void gemv_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, const vo
       const GemvTask& Tk = L.t[t0 + lane];
       bool here = true;
       if (Tk.e_qs != 0) {
-        const int le = (Tk.expert_ids ? Tk.expert_ids[Tk.slot] : Tk.slot) - Tk.expert_base;
+        const int le = (Tk.expert_ids ? glob(Tk.expert_ids)[Tk.slot] : Tk.slot) - Tk.expert_base;
         here = le >= 0 && le < Tk.local_experts;
       }
       c_rows = here ? Tk.vrow_end - Tk.vrow_begin : 0;
@@ -238,23 +238,23 @@ DEV void gemv_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, const vo
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tid == 0) {
-          const unsigned old = __hip_atomic_fetch_add(L.comb_counter + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const unsigned old = __hip_atomic_fetch_add(glob(L.comb_counter) + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           comb_last = old == (unsigned)L.n_tasks - 1;
           if (comb_last) {
             FINISHER_ACQUIRE();
-            __hip_atomic_store(L.comb_counter + g, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+            __hip_atomic_store(glob(L.comb_counter) + g, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
           }
         }
         __syncthreads();
         if (comb_last) {  // all slots of these rows have landed: x += w_k * out_k (k order), then + shared
           for (int rr = base + tid; rr < min(T.rows, base + RG); rr += NW * 64) {
-            float xv = L.comb_x[rr];
+            float xv = glob(L.comb_x)[rr];
             for (int tj = 0; tj < L.n_tasks; ++tj) {
-              const float v = __hip_atomic_load(L.t[tj].out + rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              if (L.t[tj].accum_w) xv = fmaf(v, *L.t[tj].accum_w, xv);  // src/infer.cpp:874-877
+              const float v = __hip_atomic_load(glob(L.t[tj].out) + rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              if (L.t[tj].accum_w) xv = fmaf(v, *glob(L.t[tj].accum_w), xv);  // src/infer.cpp:874-877
               else xv += v;                                             // src/infer.cpp:900-903
             }
-            L.comb_x[rr] = xv;
+            glob(L.comb_x)[rr] = xv;
           }
         }
         continue;
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
     const bool has = j < n_tasks && row0 < hi;  // wave-uniform
     p_valid[j] = has && rr < hi;
     p_row[j] = p_valid[j] ? rr : (hi > 0 ? hi - 1 : 0);
-    p_out[j] = T.out;
+    p_out[j] = glob(T.out);
     p_epi[j] = T.epilogue;
     KQRsrc B;
     B.qs = make_rsrc_n(T.qs, has);
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_q8_kernel(const GemvLaunch* _
   if (tl) t_bar = wall_clock64();
   // ---- 4. the first row group: steps 2 and 3 requested now, then the four steps multiplied in order ----
   const uint8_t* lds_lane = smem + sub * ITEM_LDS;
-  float* const out = T.out;
+  float* const out = glob(T.out);
   const int epi = T.epilogue;
   {
     const bool has = lo + wave * RPW < hi;
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(1024) void gemv_kvwrite_ahead_kernel(const GemvLaun
     compute_chunk_kq<QT, 1, 4, false>(c0, ITS, ITEMS, sub, LL, q, 0, lds_lane, acc, acc2);
     const float r = lanes_sum(acc[0], LL);
     if (valid_a && sub == 0) {
-      float* o = L.t[ti0].out + row_a;
+      float* o = glob(L.t[ti0].out) + row_a;
       if (L.t[ti0].epilogue == EPI_ADD) *o += r;
       else *o = r;
     }
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(1024) void gemv_kvwrite_ahead_kernel(const GemvLaun
       float acc[1], acc2[1];
       rows_dot_kq<QT, 1, 4, false>(B, ITEMS, sub, LL, q, rb, lds_lane, acc, acc2);
       if (v2 && sub == 0) {
-        float* o = T.out + rw;
+        float* o = glob(T.out) + rw;
         if (T.epilogue == EPI_ADD) *o += acc[0];
         else *o = acc[0];
       }

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(NT) void join_kernel(const JoinArgs a) {
   ConvOne<V, (CONV > 1 ? CONV : 1)> cv;
   SeqDesc sq{};
   float nw[V], pw[V];
-  if constexpr (CONV > 0) sq = a.p.seqs[row];
+  if constexpr (CONV > 0) sq = seq_at(a.p.seqs + row);
   if (a.y_t && tid < a.n_slots) {
     s_w[tid] = a.weight[(size_t)row * a.n_slots + tid];
     s_pos[tid] = a.slot_pos[(size_t)row * a.n_slots + tid];
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(256) void conv_kernel(const PassDesc p, int D, cons
   constexpr int R = RECUR_CHUNK, K = TAPS ? TAPS : 1;
   const int c = V * (blockIdx.y * 256 + threadIdx.x), taps = TAPS ? TAPS : a.taps;
   if (c >= D) return;
-  const SeqDesc s = p.seqs[p.chunk[2 * blockIdx.x]];
+  const SeqDesc s = seq_at(p.seqs + p.chunk[2 * blockIdx.x]);
   const int t0 = p.chunk[2 * blockIdx.x + 1], n_rows = min(R, s.len - t0);
   const float* H = h_f + (size_t)s.row0 * D + c;
   const float* hist = reinterpret_cast<const float*>(s.state + a.off_in) + (size_t)s.flip * (taps - 1) * D + c;

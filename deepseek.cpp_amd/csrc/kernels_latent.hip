@@ -42,7 +42,7 @@ __global__ __launch_bounds__(PREP_NT) void latent_prep_kernel(const LatentArgs a
   constexpr int NT = PREP_NT, U = 4;  // U elements of either latent per thread wait in registers; larger ones are read again
   __shared__ float red[2 * NT / 64];
   const int row = blockIdx.x, tid = threadIdx.x, half = a.rot_dims >> 1, ld = a.rank_p + a.rot_p, cq_k = (a.q_rank + 63) & ~63;
-  const SeqDesc s = a.p.seqs[a.p.row_seq[row]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.row_seq[row]);
   const int pos = s.pos0 + row - s.row0;
   const float *q = a.proj_f + (size_t)row * a.ld + a.col_q, *kv = a.proj_f + (size_t)row * a.ld + a.col_kv;
   float xq[U], xk[U], wq[U], wk[U], sq = 0.f, sk = 0.f;
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(PREP_NT) void latent_prep_kernel(const LatentArgs a
 template <typename T>
 __global__ __launch_bounds__(256) void latent_gather_kernel(const LatentArgs a) {
   typedef typename Frag<T>::type frag;
-  const SeqDesc s = a.p.seqs[blockIdx.y];
+  const SeqDesc s = seq_at(a.p.seqs + blockIdx.y);
   const int ld = a.rank_p + a.rot_p, wave = threadIdx.x >> 6;
   if (s.len == 1) return;
   for (int u = 0; u < 4; ++u) {
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(256) void latent_store_kernel(const LatentArgs a) {
   typedef typename Frag<T>::type frag;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), ld = a.rank_p + a.rot_p;
   if (row >= a.p.rows) return;
-  const SeqDesc s = a.p.seqs[a.p.row_seq[row]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.row_seq[row]);
   const int t = row - s.row0;
   if (s.len == 1 || t < s.len - a.window) return;
   const T* src = reinterpret_cast<const T*>(a.lat_t) + (size_t)(s.key0 + s.hist + t) * ld;
@@ -166,7 +166,7 @@ struct LatentKeys {
 template <typename T, int KT, int VTL>
 ATTN_KERNEL(T) void latent_attn_kernel(const LatentArgs a) {
   const int h = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;  // (a sequence's last tiles have the most keys: they start first)
-  const SeqDesc s = a.p.seqs[a.p.qtile[2 * tile]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.qtile[2 * tile]);
   if (s.len == 1) return;
   attn_tile<T, KT, VTL>(LatentKeys<T>{a, s, h}, s, a.p.qtile[2 * tile + 1], (a.dim_p + a.rot_p) >> 5, a.vdim_p >> 4, a.vdim, a.scale,
                         reinterpret_cast<T*>(a.out_t) + h * a.vdim, a.out_ld);
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(FEW_NT) void latent_few_kernel(const LatentArgs a) 
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
   const int i = blockIdx.y, split = blockIdx.x;
-  const SeqDesc s = a.p.seqs[a.p.single[a.first + i]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.single[a.first + i]);
   const int pos = s.pos0, seen = min(pos + 1, a.window), k0 = split * N, n = min(N, seen - k0);
   if (n <= 0) return;
   const int ld = a.rank_p + a.rot_p, LD = ld + 16 / (int)sizeof(T), LQ = a.rot_p + 8;
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void latent_values_kernel(const LatentArgs a) 
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = blockIdx.x, v0 = blockIdx.y * 64, i = blockIdx.z;
-  const SeqDesc s = a.p.seqs[a.p.single[a.first + i]];
+  const SeqDesc s = seq_at(a.p.seqs + a.p.single[a.first + i]);
   const int n = (min(s.pos0 + 1, a.window) + FewKeys<T>::N - 1) / FewKeys<T>::N;
   float* c = reinterpret_cast<float*>(lds);  // [rank_p] merged latent
   float* w = c + a.rank_p;                   // [splits] weights of the parts

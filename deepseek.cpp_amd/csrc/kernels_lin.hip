@@ -106,12 +106,6 @@ DEV void store_glu(const LinArgs& a, int row, int feature, const f32x4& g, const
   *reinterpret_cast<four*>(reinterpret_cast<T*>(a.out_t) + (size_t)row * a.ld_t + feature) = to_four<T>(v);
 }
 
-// Workgroups go round robin over the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the tiles, in order, so that the
-// tiles of one weight tile (and then its neighbours) meet in one L2.
-DEV int xcd_range(int b, int n) {
-  const int x = b & 7, base = n >> 3, extra = n & 7;
-  return x * base + min(x, extra) + (b >> 3);
-}
 // k tiles per part: even, so that a part is whole steps of the prompt kernels
 __host__ DEV int part_tiles(int kt, int parts) { return parts > 1 ? ((kt / 2 + parts - 1) / parts) * 2 : kt; }
 __host__ DEV int part_tiles(const LinArgs& a) { return part_tiles(a.kt, a.parts); }

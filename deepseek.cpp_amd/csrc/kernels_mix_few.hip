@@ -76,7 +76,7 @@ DEV void attn_few(const MixFewArgs& f, int b, float* lds) {
   const ChunkAttnArgs& a = f.attn;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int split = b % f.splits, g = b / f.splits % a.kv_heads, row = b / f.splits / a.kv_heads;
-  const SeqDesc sq = a.p.seqs[row];
+  const SeqDesc sq = seq_at(a.p.seqs + row);
   const int pos = sq.pos0, first = pos / a.chunk * a.chunk;
   const int n_splits = (pos - first) / ATTN_SPLIT_KEYS + 1;
   if (split >= n_splits) return;
@@ -320,7 +320,7 @@ template <typename T, int RK>
 DEV void mlstm_few(const MlstmArgs& a, int b, float* lds) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int h = b % a.heads, row = b / a.heads;
-  const SeqDesc s = a.p.seqs[row];
+  const SeqDesc s = seq_at(a.p.seqs + row);
   const bool fresh = s.pos0 == 0;
   float *q = lds, *k = q + HD, *v = k + HD, *o = v + HD, *red = o + HD;  // red [16][HD]
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * a.dim * a.vdim;
@@ -402,7 +402,7 @@ DEV void wkv_few(const MixFewArgs& f, int b, float* lds) {
   const WkvArgs& a = f.wkv;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, dim = a.dim;
   const int h = b % a.heads, row = b / a.heads;
-  const SeqDesc s = a.p.seqs[row];
+  const SeqDesc s = seq_at(a.p.seqs + row);
   float *r = lds, *k = r + HD, *v = k + HD, *w = v + HD, *o = w + HD, *bonus = o + HD, *low = bonus + 4;
   float* red = low + f.low_kt * 32;  // [16][HD], before that [4][2 HD]
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * dim * dim;
@@ -456,7 +456,7 @@ DEV void delta_few(const MixFewArgs& f, int b, float* lds) {
   const DeltaArgs& a = f.delta;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = b % a.heads, row = b / a.heads, rep = a.heads / a.kv_heads, kv = h / rep;
-  const SeqDesc s = a.p.seqs[row];
+  const SeqDesc s = seq_at(a.p.seqs + row);
   const bool fresh = s.pos0 == 0;
   const int dim = a.dim, vdim = a.vdim, nq = a.kv_heads * dim, nv = a.heads * vdim, C = 2 * nq + nv, taps = a.taps;
   float *ch = lds, *g = ch + 3 * HD, *gate = g + HD, *o = gate + HD, *sc = o + HD, *low = sc + 4;

@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaArgs a) {
   const int lane = threadIdx.x & 63, unit = blockIdx.y * 4 + (threadIdx.x >> 6);
   const int nq = a.kv_heads * a.dim, nv = a.heads * a.vdim, C = 2 * nq + nv, taps = TAPS ? TAPS : a.taps;
   if (unit >= 2 * a.kv_heads + 2 * a.heads) return;
-  const SeqDesc sq = a.p.seqs[a.p.chunk[2 * blockIdx.x]];
+  const SeqDesc sq = seq_at(a.p.seqs + a.p.chunk[2 * blockIdx.x]);
   const int t0 = a.p.chunk[2 * blockIdx.x + 1], n_rows = min(R, sq.len - t0);
   const size_t row0 = (size_t)sq.row0 + t0;
   if (unit >= 2 * a.kv_heads + a.heads) {
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaArgs a) {
   const int h = blockIdx.y, kv = h / (a.heads / a.kv_heads);
   const int col = blockIdx.x * 16 + vl;
   const bool live = col < a.vdim;
-  const SeqDesc s = a.p.seqs[blockIdx.z];
+  const SeqDesc s = seq_at(a.p.seqs + blockIdx.z);
   const int dim = a.dim, nq = a.kv_heads * dim, nv = a.heads * a.vdim;
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * dim * a.vdim;
   float S[KPL];
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const MlstmArgs a) {
   const int h = blockIdx.y;
   const int col = blockIdx.x * 16 + vl;
   const bool live = col < a.vdim;
-  const SeqDesc s = a.p.seqs[blockIdx.z];
+  const SeqDesc s = seq_at(a.p.seqs + blockIdx.z);
   const int dim = a.dim, nv = a.heads * a.vdim;
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * dim * a.vdim;
   float* N0 = reinterpret_cast<float*>(s.state + a.off_n) + (size_t)h * dim;  // copy `flip` is read, the other written
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(const WkvArgs a) {
   const int h = blockIdx.y, dim = a.dim, n_all = a.heads * dim;
   const int col = blockIdx.x * 16 + vl;
   const bool live = col < dim;
-  const SeqDesc s = a.p.seqs[blockIdx.z];
+  const SeqDesc s = seq_at(a.p.seqs + blockIdx.z);
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * dim * dim;
   float S[KPL];
 #pragma unroll

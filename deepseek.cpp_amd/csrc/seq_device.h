@@ -8,6 +8,8 @@
 // into three bf16 numbers instead (Split).
 #pragma once
 #include "dsk_internal.h"
+#include "glob_device.h"
+#include "layered_kernels.h"
 
 typedef __bf16 bf16;
 typedef bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -15,6 +17,11 @@ typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 #define DEV __device__ __forceinline__
+DEV SeqDesc seq_at(const SeqDesc* p) {
+  SeqDesc s = *p;
+  s.state = glob(s.state);
+  return s;
+}
 
 template <typename T>
 struct Frag;
@@ -121,4 +128,11 @@ DEV float block_sum(float v, float* scratch) {
 #pragma unroll
   for (int i = 0; i < NT / 64; ++i) s += scratch[i];
   return s;
+}
+
+// Workgroups go round robin over the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the work, in order, so that neighbours, which
+// read the same weights or operands, meet in one L2.
+DEV int xcd_range(int b, int n) {
+  const int x = b & 7, base = n >> 3, extra = n & 7;
+  return x * base + min(x, extra) + (b >> 3);
 }

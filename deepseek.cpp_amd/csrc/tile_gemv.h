@@ -52,7 +52,7 @@ DEV void gemv_tile_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, con
     grp_idx = g;
   }
   auto task_of = [&](int ti) {
-    GemvTask T = L.t[ti];
+    GemvTask T = glob(L.t[ti]);
     if (bd) {  // re-base the one task to this workgroup's head (rows per head: a multiple of 16, gemv_plan)
       T.qs += (size_t)head * (size_t)(T.rows >> 4) * (T.n >> 8) * TILE_B;
       T.a_f32 += (size_t)head * T.n;
@@ -87,7 +87,7 @@ DEV void gemv_tile_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, con
       const GemvTask& Tk = L.t[t0 + lane];
       bool here = true;
       if (Tk.e_qs != 0) {
-        const int le = (Tk.expert_ids ? Tk.expert_ids[Tk.slot] : Tk.slot) - Tk.expert_base;
+        const int le = (Tk.expert_ids ? glob(Tk.expert_ids)[Tk.slot] : Tk.slot) - Tk.expert_base;
         here = le >= 0 && le < Tk.local_experts;
       }
       c_rows = here ? Tk.vrow_end - Tk.vrow_begin : 0;
@@ -187,24 +187,24 @@ DEV void gemv_tile_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, con
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-      const unsigned old = __hip_atomic_fetch_add(L.comb_counter + wi, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned old = __hip_atomic_fetch_add(glob(L.comb_counter) + wi, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       comb_last = old == (unsigned)L.n_tasks - 1;
       if (comb_last) {
         FINISHER_ACQUIRE();
-        __hip_atomic_store(L.comb_counter + wi, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
+        __hip_atomic_store(glob(L.comb_counter) + wi, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm
       }
     }
     __syncthreads();
     if (comb_last && comb_out) {
       const int row0 = (int)(comb_out - L.t[t0].out);
       for (int rr = row0 + tid; rr < row0 + comb_rows; rr += NW * 64) {
-        float xv = L.comb_x[rr];
+        float xv = glob(L.comb_x)[rr];
         for (int tj = 0; tj < L.n_tasks; ++tj) {
-          const float v = __hip_atomic_load(L.t[tj].out + rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (L.t[tj].accum_w) xv = fmaf(v, *L.t[tj].accum_w, xv);  // src/infer.cpp:874-877
+          const float v = __hip_atomic_load(glob(L.t[tj].out) + rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (L.t[tj].accum_w) xv = fmaf(v, *glob(L.t[tj].accum_w), xv);  // src/infer.cpp:874-877
           else xv += v;                                             // src/infer.cpp:900-903
         }
-        L.comb_x[rr] = xv;
+        glob(L.comb_x)[rr] = xv;
       }
     }
   }
