@@ -11,7 +11,7 @@
 //                G_(t-1) / G_s below the diagonal, and the bonus on it: B_tt = sum_d q_t u k_t
 // *_prepare: everything that does not depend on S0, for all chunks at once - the operands with decays multiplied in, B, and
 // T = (I + diag(beta) A)^-1 diag(beta), so that U = T (V - Kg S0).  chunk_scan: one workgroup per (16 columns, head, sequence)
-// goes through the chunks; its 4 waves share the key channels.  S stays in MFMA accumulators: their layout (column = lane % 16, rows
+// goes through the chunks; 4 waves share the key channels, a fifth forms the outputs.  S stays in MFMA accumulators: their layout (column = lane % 16, rows
 // 4 (lane / 16) + i) is an operand layout of v_mfma_f32_16x16x4_f32 when step i stands for the k values {4 g + i}.
 #include "layered_kernels.h"
 #include "seq_device.h"
@@ -271,104 +271,165 @@ struct ScanArgs {
   size_t off_s, off_n;
 };
 enum { SCAN_DELTA, SCAN_MLSTM, SCAN_WKV };
-template <typename T, int KIND, int NTL>
-__global__ __launch_bounds__(256) void chunk_scan_kernel(const ScanArgs a) {
+enum { SCAN_WAVES = 5 };  // four that share the key channels, one for the outputs
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+DEV const char* uniform_ptr(const void* p) {
+  const unsigned long long v = (unsigned long long)p;
+  return (const char*)(((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((unsigned)v));
+}
+DEV rsrc_t buffer_of(const char* p, int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p), 0, bytes, 0x00020000); }
+DEV f32x4 load4(rsrc_t r, int off, int base) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, base, 0)); }
+template <typename T>
+DEV float load1(rsrc_t r, int off) {
+  if constexpr (sizeof(T) == 2) return __builtin_bit_cast(float, (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0) << 16);
+  else return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+// One chunk after the other: what bounds it is a chunk's chain - W over a wave's key channels, the exchange of its four parts through LDS, U, the update
+// of S - so everything else is taken off it.  The outputs are a fifth wave's work, a chunk behind and out of LDS alone: a wave that stores and
+// loads waits for its stores (mLSTM: 77 us with its loads in that wave, 47 without).  Their half of S0's products is issued in the shadow of the
+// exchange.  Operands come as buffer loads whose offsets stay in registers (a chunk costs scalar additions), a chunk or two ahead
+// (NB; more gained nothing), and the waits count: no step of the loop may be skipped behind another, and a wave's tiles are all there
+// (FULL) or tested.  All columns of a head read the same operands: an XCD takes a range of (sequence, head, columns) in this order, so
+// that its L2 gets them once.  Three waves a SIMD: two workgroups share a compute unit.
+// 2048 tokens, 16 heads: delta rule of 128 x 128 177 -> 119 us, mLSTM of 64 x 129 100 -> 47; four sequences of up to 901 tokens: delta rule
+// 114 -> 107, wkv of 32 heads of 64 x 64 57 -> 37.
+template <typename T, int KIND, int NTL, bool FULL>
+__global__ __launch_bounds__(64 * SCAN_WAVES) __attribute__((amdgpu_waves_per_eu(NTL > 2 ? 2 : 3))) void chunk_scan_kernel(const ScanArgs a) {
   constexpr bool DELTA = KIND == SCAN_DELTA, NORM = KIND == SCAN_MLSTM;
-  __shared__ __attribute__((aligned(16))) f32x4 ex[2][4][2][64];
+  constexpr int NB = NTL > 1 ? 2 : 3;
+  __shared__ __attribute__((aligned(16))) f32x4 ex_w[DELTA ? 2 : 1][4][64], ex_x[2][4][64], ex_u[2][64], ex_b[2][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
-  const int h = blockIdx.y, dp = (a.dim + 15) / 16 * 16, tiles = dp >> 4;
-  const int cols = NORM ? a.vdim + 1 : a.vdim;
-  const int col = blockIdx.x * 16 + c16;
+  const int dp = (a.dim + 15) / 16 * 16, tiles = dp >> 4;
+  const int cols = NORM ? a.vdim + 1 : a.vdim, col_tiles = (cols + 15) >> 4;
+  const int place = xcd_range(blockIdx.x, gridDim.x), head = place / col_tiles, h = head % a.heads;
+  const int col = (place - head * col_tiles) * 16 + c16;
   const bool live = col < cols, norm = NORM && col == a.vdim;
-  const SeqDesc s = seq_at(a.p.seqs + blockIdx.z);
+  const SeqDesc s = seq_at(a.p.seqs + head / a.heads);
+  const int nc = (s.len + CH - 1) / CH;
+  // this sequence's and head's operands and values, chunk by chunk (chunks behind the last: the last again)
+  const int ops_bytes = (49 * dp + 512) * 4, ld = a.ld_v * (int)sizeof(T);
+  const char* ops0 = uniform_ptr(a.ops) + ((size_t)__builtin_amdgcn_readfirstlane(s.chunk0) * a.heads + h) * ops_bytes;
+  const char* v0 = uniform_ptr(a.v) + (size_t)__builtin_amdgcn_readfirstlane(s.row0) * ld + (size_t)h * a.vdim * sizeof(T);
+  auto ops_of = [&](int c) { return buffer_of(ops0 + (size_t)min(c, nc - 1) * a.heads * ops_bytes, ops_bytes); };
+  auto v_of = [&](int c) {  // (rows past the sequence's end read zero, and columns behind the last one's values compute something nobody stores)
+    c = min(c, nc - 1);
+    return buffer_of(v0 + (size_t)c * CH * ld, (min((int)CH, s.len - c * CH) - 1) * ld + a.vdim * (int)sizeof(T));
+  };
+  const int vcol = min(col, a.vdim - 1), v_off = g * 4 * ld + vcol * (int)sizeof(T), small_off = (c16 * 16 + g * 4) * 4;
+  const int at_q = 64 * dp, at_ke = 128 * dp, at_g = 192 * dp, at_t = 196 * dp, at_b = 196 * dp + 1024;
+
+  if (wave == 4) {  // the outputs of a chunk: O = the parts of (q G)^T S0 + B U, everything out of LDS: behind its stores this wave waits for no load
+    const int row_bytes = a.heads * cols * 4;
+    const char* o0 = uniform_ptr(a.o) + (size_t)__builtin_amdgcn_readfirstlane(s.row0) * row_bytes + (size_t)h * cols * 4;
+    const int o_off = live ? g * 4 * row_bytes + col * 4 : 0x7ff00000;  // (out of every range: not stored, like the rows past the end)
+    lds_barrier();
+    for (int c = 0; c < nc; ++c) {
+      lds_barrier();  // that of chunk c + 1: what chunk c's waves wrote behind theirs is here
+      const f32x4 U = ex_u[c & 1][lane], B = ex_b[c & 1][lane];
+      f32x4 O = (ex_x[c & 1][0][lane] + ex_x[c & 1][1][lane]) + (ex_x[c & 1][2][lane] + ex_x[c & 1][3][lane]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) O = __builtin_amdgcn_mfma_f32_16x16x4f32(B[e], U[e], O, 0, 0, 0);
+      const rsrc_t r = buffer_of(o0 + (size_t)c * CH * row_bytes, (min((int)CH, s.len - c * CH) - 1) * row_bytes + cols * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = O[e];  // (a bit cast of an element of a vector in place takes the first one)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, o_off + e * row_bytes, 0, 0);
+      }
+    }
+    return;
+  }
+
   float* S0 = reinterpret_cast<float*>(s.state + a.off_s) + (size_t)h * a.dim * a.vdim;
   float* N0 = !NORM ? nullptr : reinterpret_cast<float*>(s.state + a.off_n) + (size_t)h * a.dim;
   const size_t nn = (size_t)a.heads * a.dim;
   f32x4 S[NTL];
+  int k_off[NTL], ke_off[NTL], g_off[NTL];
 #pragma unroll
-  for (int i = 0; i < NTL; ++i)
+  for (int i = 0; i < NTL; ++i) {
+    const int tile = FULL ? wave + 4 * i : min(wave + 4 * i, tiles - 1);
+    k_off[i] = (c16 * dp + tile * 16 + g * 4) * 4;
+    ke_off[i] = ((tile * 16 + c16) * 16 + g * 4) * 4;
+    g_off[i] = (tile * 16 + g * 4) * 4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int k = (wave + 4 * i) * 16 + g * 4 + e;
       S[i][e] = s.pos0 > 0 && live && k < a.dim ? (norm ? N0[s.flip * nn + k] : S0[(size_t)k * a.vdim + col]) : 0.f;
     }
-  // Requested without a branch and untouched until they are used, so that the waits count exactly: rows past the end repeat the last
-  // one (their columns of T, B and Ke are zero), columns past the last one compute something nobody stores.
+  }
   struct Operands {
     f32x4 kg[NTL], qg[NTL], ke[NTL], ge[NTL], t, b;
-    T v[4];
+    float v[4];
   };
-  const int vcol = min(col, a.vdim - 1);
-  const int nc = (s.len + CH - 1) / CH;
   auto load = [&](int c, Operands& x) {
-    c = min(c, nc - 1);
-    const Ops o = ops_at(a.ops, (size_t)s.chunk0 + c, a.heads, h, a.dim);
-#pragma unroll
-    for (int i = 0; i < NTL; ++i) {
-      const int tile = min(wave + 4 * i, tiles - 1);
-      if (DELTA) x.kg[i] = *reinterpret_cast<const f32x4*>(o.kg + c16 * dp + tile * 16 + g * 4);
-      x.qg[i] = *reinterpret_cast<const f32x4*>(o.qg + c16 * dp + tile * 16 + g * 4);
-      x.ke[i] = *reinterpret_cast<const f32x4*>(o.ke + (size_t)(tile * 16 + c16) * 16 + g * 4);
-      x.ge[i] = *reinterpret_cast<const f32x4*>(o.gend + tile * 16 + g * 4);
-    }
-    if (DELTA) x.t = *reinterpret_cast<const f32x4*>(o.t + c16 * 16 + g * 4);
-    x.b = *reinterpret_cast<const f32x4*>(o.b + c16 * 16 + g * 4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const size_t row = (size_t)s.row0 + min(c * CH + g * 4 + e, s.len - 1);
-      x.v[e] = reinterpret_cast<const T*>(a.v)[row * a.ld_v + (size_t)h * a.vdim + vcol];
-    }
-  };
-  auto step = [&](int c, const Operands& x, Operands& fill) {  // fill: the operands of chunk c + 2
-    load(c + 2, fill);
-    f32x4 W = {0.f, 0.f, 0.f, 0.f}, X = {0.f, 0.f, 0.f, 0.f};
+    const rsrc_t o = ops_of(c), r = v_of(c);
 #pragma unroll
     for (int i = 0; i < NTL; ++i)
-      if (wave + 4 * i < tiles)
+      if (DELTA) x.kg[i] = load4(o, k_off[i], 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (DELTA) W = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kg[i][e], S[i][e], W, 0, 0, 0);
-          X = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qg[i][e], S[i][e], X, 0, 0, 0);
-        }
-    if (DELTA) ex[c & 1][wave][0][lane] = W;
-    ex[c & 1][wave][1][lane] = X;
+    for (int i = 0; i < NTL; ++i) x.qg[i] = load4(o, k_off[i], at_q);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.v[e] = load1<T>(r, v_off + e * ld);
+    if (DELTA) x.t = load4(o, small_off, at_t);
+    x.b = load4(o, small_off, at_b);
+#pragma unroll
+    for (int i = 0; i < NTL; ++i) {
+      x.ke[i] = load4(o, ke_off[i], at_ke);
+      x.ge[i] = load4(o, g_off[i], at_g);
+    }
+  };
+  auto step = [&](int c, Operands& x) {  // ... and requests the operands of chunk c + NB into x
+    f32x4 W = {0.f, 0.f, 0.f, 0.f}, X = {0.f, 0.f, 0.f, 0.f};
+    if (DELTA) {
+#pragma unroll
+      for (int i = 0; i < NTL; ++i)
+        if (FULL || wave + 4 * i < tiles)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) W = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kg[i][e], S[i][e], W, 0, 0, 0);
+      ex_w[c & 1][wave][lane] = W;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < NTL; ++i)
+      if (FULL || wave + 4 * i < tiles)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) X = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qg[i][e], S[i][e], X, 0, 0, 0);
     lds_barrier();  // (the operands of the next chunks stay in flight)
     f32x4 U;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) U[e] = norm ? 1.f : (float)x.v[e];
+    for (int e = 0; e < 4; ++e) U[e] = norm ? 1.f : x.v[e];
     if (DELTA) {
-      W = (ex[c & 1][0][0][lane] + ex[c & 1][1][0][lane]) + (ex[c & 1][2][0][lane] + ex[c & 1][3][0][lane]);
+      W = (ex_w[c & 1][0][lane] + ex_w[c & 1][1][lane]) + (ex_w[c & 1][2][lane] + ex_w[c & 1][3][lane]);
       const f32x4 r = U - W;
       U = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < 4; ++e) U = __builtin_amdgcn_mfma_f32_16x16x4f32(x.t[e], r[e], U, 0, 0, 0);
     }
+    ex_x[c & 1][wave][lane] = X;
 #pragma unroll
     for (int i = 0; i < NTL; ++i)
-      if (wave + 4 * i < tiles) {
-        S[i] *= x.ge[i];
+      if (FULL || wave + 4 * i < tiles) S[i] *= x.ge[i];
+#pragma unroll
+    for (int i = 0; i < NTL; ++i)
+      if (FULL || wave + 4 * i < tiles)
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.ke[i][e], U[e], S[i], 0, 0, 0);
-      }
-    if (wave == (c & 3)) {  // the waves take turns with the outputs
-      f32x4 O = (ex[c & 1][0][1][lane] + ex[c & 1][1][1][lane]) + (ex[c & 1][2][1][lane] + ex[c & 1][3][1][lane]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) O = __builtin_amdgcn_mfma_f32_16x16x4f32(x.b[e], U[e], O, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = c * CH + g * 4 + e;
-        if (t < s.len && live) a.o[((size_t)(s.row0 + t) * a.heads + h) * cols + col] = O[e];
-      }
+    if (wave == (c & 3)) {
+      ex_u[c & 1][lane] = U;
+      ex_b[c & 1][lane] = x.b;
     }
+    load(c + NB, x);
   };
-  Operands x, y, z;
-  load(0, x);
-  load(1, y);
-  for (int c = 0; c < nc; c += 3) {
-    step(c, x, z);
-    if (c + 1 < nc) step(c + 1, y, x);
-    if (c + 2 < nc) step(c + 2, z, y);
-  }
+  Operands x[NB];
+#pragma unroll
+  for (int u = 0; u < NB; ++u) load(u, x[u]);
+  int c = 0;
+  for (; c + NB <= nc; c += NB)
+#pragma unroll
+    for (int u = 0; u < NB; ++u) step(c + u, x[u]);
+#pragma unroll
+  for (int u = 0; u + 1 < NB; ++u)
+    if (c + u < nc) step(c + u, x[u]);
+  lds_barrier();  // (the last chunk's outputs)
 #pragma unroll
   for (int i = 0; i < NTL; ++i)
 #pragma unroll
@@ -384,10 +445,13 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ScanArgs a) {
 template <typename T, int KIND>
 static int scan_t(hipStream_t st, const ScanArgs& a) {
   if (a.dim < 1 || a.dim > RECUR_MAX_DIM) DSK_FAIL(DSK_ERR_UNSUPPORTED, "recurrence: key size %d (max %d)", a.dim, (int)RECUR_MAX_DIM);
-  const dim3 grid(cdiv(KIND == SCAN_MLSTM ? a.vdim + 1 : a.vdim, 16), a.heads, a.p.n_seqs);
-  if (a.dim <= 64) hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 1>), grid, dim3(256), 0, st, a);
-  else if (a.dim <= 128) hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 2>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 4>), grid, dim3(256), 0, st, a);
+  const dim3 grid((unsigned)cdiv(KIND == SCAN_MLSTM ? a.vdim + 1 : a.vdim, 16) * a.heads * a.p.n_seqs);
+  const int tiles = cdiv(a.dim, 16);
+  if (tiles == 4) hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 1, true>), grid, dim3(64 * SCAN_WAVES), 0, st, a);
+  else if (tiles < 4) hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 1, false>), grid, dim3(64 * SCAN_WAVES), 0, st, a);
+  else if (tiles == 8) hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 2, true>), grid, dim3(64 * SCAN_WAVES), 0, st, a);
+  else if (tiles < 8) hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 2, false>), grid, dim3(64 * SCAN_WAVES), 0, st, a);
+  else hipLaunchKernelGGL((chunk_scan_kernel<T, KIND, 4, false>), grid, dim3(64 * SCAN_WAVES), 0, st, a);
   return DSK_OK;
 }
 int launch_delta_chunks(hipStream_t st, const DeltaArgs& a, const ChunkScan& c) {
