@@ -438,22 +438,27 @@ DEV void stage_q8(const SRC& T, uint8_t* lds, int tid, float* scratch, unsigned 
   }
 }
 
-// Stage an f32 activation vector (F8 / F16 / F32 weights)
-template <int NW, typename SRC>
+// Stage an f32 activation vector (F8 / F16 / F32 weights).
+// (rows_dot_f reads 4 EPI of a vector's elements per lane, neighbouring lanes neighbouring items: element quad q of item i lies at quad
+// q * items + i, so that such a read is consecutive addresses.  As the vector lies in memory, lanes 16 EPI bytes apart, the quads met in a
+// quarter of the LDS banks.)
+template <int EPI>
+DEV int quad_place(int quad, int items) {
+  constexpr int Q = EPI / 4;
+  return (quad & (Q - 1)) * items + quad / Q;
+}
+template <int NW, int EPI, typename SRC>
 DEV void stage_f32(const SRC& T, float* l_x, int tid, float* scratch) {
-  const int n = T.n;
+  const int n = T.n, items = n / EPI;  // (n is a multiple of EPI: gemv_plan)
+  const f32x4* src = reinterpret_cast<const f32x4*>(T.a_f32);
+  f32x4* dst = reinterpret_cast<f32x4*>(l_x);
   if (T.act_mode == ACT_F32_NORM) {
     const float total = wg_sumsq<NW>(T.a_f32, n, tid, scratch);
     const float scale = 1.0f / sqrtf(total / (float)n + T.eps);
-    for (int i = tid; i < n; i += NW * 64) {
-      const float y = T.a_f32[i] * scale * T.norm_w[i];
-      l_x[i] = y;
-    }
+    const f32x4* nw = reinterpret_cast<const f32x4*>(T.norm_w);
+    for (int i = tid; i < (n >> 2); i += NW * 64) dst[quad_place<EPI>(i, items)] = src[i] * scale * nw[i];
   } else {
-    const f32x4* src = reinterpret_cast<const f32x4*>(T.a_f32);
-    f32x4* dst = reinterpret_cast<f32x4*>(l_x);
-    for (int i = tid; i < (n >> 2); i += NW * 64) dst[i] = src[i];
-    for (int i = (n & ~3) + tid; i < n; i += NW * 64) l_x[i] = T.a_f32[i];
+    for (int i = tid; i < (n >> 2); i += NW * 64) dst[quad_place<EPI>(i, items)] = src[i];
   }
 }
 
@@ -680,7 +685,12 @@ DEV void load_chunk_f(ChunkF<QT, R, U, GLU>& c, const WPtr& P, int n, int b0, in
   const int items = n / EPI;
   const int its = (items + LPR - 1) >> lpr_log2;
   const size_t row_bytes = (size_t)n * ESZ;
-  const int sc_cols = (n + b1 - 1) / b1;
+  // (block sides are powers of two in every checkpoint: shifts, not the ~30 instructions of a division)
+  const bool p2 = ((b0 & (b0 - 1)) | (b1 & (b1 - 1))) == 0;
+  const int s0 = __builtin_ctz(b0), s1 = __builtin_ctz(b1), sc_cols = p2 ? (n + b1 - 1) >> s1 : (n + b1 - 1) / b1;
+  size_t sc_row[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) sc_row[r] = (size_t)(p2 ? row[r] >> s0 : row[r] / b0) * sc_cols;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int it = it0 + u;
@@ -689,14 +699,15 @@ DEV void load_chunk_f(ChunkF<QT, R, U, GLU>& c, const WPtr& P, int n, int b0, in
     const bool live = item < items;
     if (!live) item = items - 1;
     c.itemv[u] = item;
+    const int sc_col = p2 ? (item * EPI) >> s1 : (item * EPI) / b1;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       c.w[u][r] = ldg_nt(reinterpret_cast<const u32x4*>(P.qs + (size_t)row[r] * row_bytes + (size_t)item * 16));
-      c.sv[u][r] = P.scale ? P.scale[(size_t)(row[r] / b0) * sc_cols + (item * EPI) / b1] : 1.0f;
+      c.sv[u][r] = P.scale ? P.scale[sc_row[r] + sc_col] : 1.0f;
       c.sv2[u][r] = 0.f;
       if (GLU) {
         c.w2[u][r] = ldg_nt(reinterpret_cast<const u32x4*>(P.qs2 + (size_t)row[r] * row_bytes + (size_t)item * 16));
-        c.sv2[u][r] = P.scale2 ? P.scale2[(size_t)(row[r] / b0) * sc_cols + (item * EPI) / b1] : 1.0f;
+        c.sv2[u][r] = P.scale2 ? P.scale2[sc_row[r] + sc_col] : 1.0f;
       }
       if (!live) c.sv[u][r] = c.sv2[u][r] = 0.f;
     }
@@ -706,7 +717,7 @@ DEV void load_chunk_f(ChunkF<QT, R, U, GLU>& c, const WPtr& P, int n, int b0, in
 template <int QT, int R, int U, bool GLU>
 DEV void compute_chunk_f(const ChunkF<QT, R, U, GLU>& c, int n, int lpr_log2, int it0, const float* l_x, float (&acc)[R], float (&acc2)[R]) {
   constexpr int EPI = FTraits<QT>::EPI;
-  const int its = (n / EPI + (1 << lpr_log2) - 1) >> lpr_log2;
+  const int items = n / EPI, its = (items + (1 << lpr_log2) - 1) >> lpr_log2;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (it0 + u >= its) break;
@@ -714,7 +725,7 @@ DEV void compute_chunk_f(const ChunkF<QT, R, U, GLU>& c, int n, int lpr_log2, in
     float xa[EPI];
 #pragma unroll
     for (int k = 0; k < EPI / 4; ++k) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(l_x + item * EPI + 4 * k);
+      const f32x4 v = reinterpret_cast<const f32x4*>(l_x)[k * items + item];  // (quad_place)
       xa[4 * k] = v.x;
       xa[4 * k + 1] = v.y;
       xa[4 * k + 2] = v.z;

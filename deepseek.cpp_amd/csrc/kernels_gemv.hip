@@ -63,7 +63,7 @@ DEV void gemv_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, const vo
     S.a_f32 = static_cast<const float*>(h_a0); S.norm_w = static_cast<const float*>(h_a1);
     if (h_gwgs > 0) S.a_f32 += (size_t)(bid / h_gwgs) * h_gstride;  // equal groups, equally spaced f32 vectors
     if (KQ) stage_q8<QT == DSK_QUANT_Q2_K, NW>(S, smem, tid, scratch);
-    else stage_f32<NW>(S, reinterpret_cast<float*>(smem), tid, scratch);
+    else stage_f32<NW, FTraits<QT>::EPI>(S, reinterpret_cast<float*>(smem), tid, scratch);
   }
   const int RPW = 64 >> lpr_log2;
   const int rloc = lane >> lpr_log2, sub = lane & ((1 << lpr_log2) - 1);
@@ -112,7 +112,7 @@ DEV void gemv_body(const GemvLaunch* __restrict__ Lp, const void* h_a0, const vo
     const GemvTask Ta = task_of(t0);
     if (tl && tid == 0) tl[6] = wall_clock64();
     if (KQ) stage_q8<QT == DSK_QUANT_Q2_K, NW>(Ta, smem, tid, scratch, tl);
-    else stage_f32<NW>(Ta, reinterpret_cast<float*>(smem), tid, scratch);
+    else stage_f32<NW, FTraits<QT>::EPI>(Ta, reinterpret_cast<float*>(smem), tid, scratch);
   } else if (tl && tid == 0) {
     tl[6] = wall_clock64();
   }
@@ -801,6 +801,22 @@ __global__ __launch_bounds__(1024) void head_attn_kernel(const HeadAttnArgs A, c
     const WPtr P = resolve(T);
     const KQRsrc B = kq_rsrc<QT, false>(P);
     const int nb = T.n >> 8;
+    if constexpr (!KQ) {
+      // Float weights are 3 - 50 times a K-quant head's bytes and cheap to multiply: a wave requests 8 of its row sets at once instead of waiting for
+      // each: V2-Lite's 256 rows of 512 in F8 took 8.3 us, now 5.6
+      constexpr int RS = 8;
+      for (int base = wave * RPW; base < nrows; base += NW * RPW * RS) {
+        int row[RS];
+        float acc[RS], acc2[RS];
+#pragma unroll
+        for (int r = 0; r < RS; ++r) row[r] = h * nrows + min(base + r * NW * RPW + rloc, nrows - 1);
+        rows_dot_f<QT, RS, 1, false>(P, T.n, A.b0, A.b1, lpr_log2, lane, row, act, acc, acc2);
+#pragma unroll
+        for (int r = 0; r < RS; ++r)
+          if (sub == 0 && base + r * NW * RPW + rloc < nrows) out_lds[base + r * NW * RPW + rloc] = acc[r];
+      }
+      return;
+    }
     for (int base = wave * RPW; base < nrows; base += NW * RPW) {  // wave-uniform bounds, no barrier inside
       const int lr = base + rloc;
       const bool valid = lr < nrows;
@@ -809,8 +825,6 @@ __global__ __launch_bounds__(1024) void head_attn_kernel(const HeadAttnArgs A, c
       if constexpr (KQ) {
         int rowblk[1] = {row[0] * nb + (sub >> 2)};
         rows_dot_kq<QT, 1, 4, false>(B, nb * 4, sub, lpr_log2, sub & 3, rowblk, act + sub * ITEM_LDS, acc, acc2);
-      } else {
-        rows_dot_f<QT, 1, 4, false>(P, T.n, A.b0, A.b1, lpr_log2, lane, row, act, acc, acc2);
       }
       if (sub == 0 && valid) out_lds[lr] = acc[0];
     }
@@ -943,11 +957,11 @@ __global__ __launch_bounds__(1024) void head_attn_kernel(const HeadAttnArgs A, c
     } else {
       if (A.has_q) {
         if (KQ) stage_q8<QT == DSK_QUANT_Q2_K, NW>(A.tq, act_q, tid, scratch);
-        else stage_f32<NW>(A.tq, reinterpret_cast<float*>(act_q), tid, scratch);
+        else stage_f32<NW, FTraits<QT>::EPI>(A.tq, reinterpret_cast<float*>(act_q), tid, scratch);
         __syncthreads();  // scratch is reused by the second staging
       }
       if (KQ) stage_q8<QT == DSK_QUANT_Q2_K, NW>(A.tkv, act_kv, tid, scratch);
-      else stage_f32<NW>(A.tkv, reinterpret_cast<float*>(act_kv), tid, scratch);
+      else stage_f32<NW, FTraits<QT>::EPI>(A.tkv, reinterpret_cast<float*>(act_kv), tid, scratch);
       __syncthreads();
     }
     tap_staged();
@@ -1260,7 +1274,7 @@ __global__ __launch_bounds__(1024) void mla_head_kernel(const MlaHeadArgs A, con
       else q8k_block_lds<QT == DSK_QUANT_Q2_K>(v, lane, act + (size_t)wave * 4 * ITEM_LDS);
     }
   } else {
-    for (int i = tid; i < lora; i += NT) reinterpret_cast<float*>(act)[i] = o_s[i];
+    for (int i = tid; i < lora; i += NT) reinterpret_cast<float*>(act)[quad_place<FTraits<QT>::EPI>(i >> 2, lora / FTraits<QT>::EPI) * 4 + (i & 3)] = o_s[i];
   }
   __syncthreads();
 #ifndef DSK_NO_TAPS

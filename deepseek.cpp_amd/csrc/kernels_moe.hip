@@ -381,7 +381,7 @@ __global__ __launch_bounds__(1024) void moe_ffn_f_kernel(const MoeFfnArgs a) {
     ActSrc S;
     S.act_mode = ACT_F32_NORM; S.n = a.dim; S.a_f32 = a.x; S.norm_w = a.norm_w; S.eps = a.eps; S.pre_scale = 0.f;
     S.a_qs = nullptr; S.a_d = nullptr; S.a_bsums = nullptr;
-    stage_f32<NW>(S, actA, tid, scratch);
+    stage_f32<NW, FTraits<QT>::EPI>(S, actA, tid, scratch);
   }
   __syncthreads();
   if (tl && tid == 0) tl[1] = wall_clock64();
@@ -498,9 +498,10 @@ __global__ __launch_bounds__(1024) void moe_ffn_f_kernel(const MoeFfnArgs a) {
       for (int i = tid; i < slots * per; i += NW * 64) {
         const int s = i / per, j = i - s * per;
         const int n = s < K ? a.mi : a.shared_n;
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (j * 4 < n) v = __builtin_amdgcn_raw_buffer_load_b128(hr, (s * a.hb_stride + j * 4) * 4, 0, 16);
-        *reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(actB) + (size_t)s * a.lds_b + (size_t)j * 16) = v;
+        if (j * 4 >= n) continue;
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(hr, (s * a.hb_stride + j * 4) * 4, 0, 16);
+        constexpr int EPI = FTraits<QT>::EPI;
+        *reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(actB) + (size_t)s * a.lds_b + (size_t)quad_place<EPI>(j, n / EPI) * 16) = v;
       }
     }
     __syncthreads();
