@@ -600,14 +600,26 @@ DEV void few_body(const LinArgs& a, int rt0, int k_first, int k_end, int a_row, 
     x[u] = *reinterpret_cast<const frag*>(x0 + (size_t)k * 32);
   };
   int k0 = k_first + wave;
-  for (; k0 + 4 * (U - 1) < k_end; k0 += 4 * U) {  // no condition inside: a load is moved behind it, and then waited for alone
+  if (k0 + 4 * (U - 1) < k_end) {  // a whole round of U k tiles
 #pragma unroll
     for (int u = 0; u < U; ++u) load(u, k0 + 4 * u);
     __builtin_amdgcn_sched_barrier(0);  // (all on their way first)
+    // While another whole round follows, a tile is requested as soon as its registers are free: the stream does not stop between rounds.  (No
+    // condition inside: a load is moved behind it, and then waited for alone)
+    for (; k0 + 4 * (2 * U - 1) < k_end; k0 += 4 * U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) acc[i] = mma(w[u][i], x[u], acc[i]);
+        load(u, k0 + 4 * (U + u));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < NR; ++i) acc[i] = mma(w[u][i], x[u], acc[i]);
+    k0 += 4 * U;
   }
   if (k0 < k_end) {  // the last, short one: zeros behind the end
 #pragma unroll
@@ -652,7 +664,7 @@ struct FewArgs {
 // A load of the operand is `rows` segments of 64 bytes in as many lines, at 16 rows twice the lines of a weight tile's load: where enough
 // workgroups are left (launch_few) one takes NT tiles (of gate and up: two pairs) per load of the operand.
 template <typename T, int NT>
-__global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
+__global__ __launch_bounds__(256, NT > 1 ? 4 : 5) void few_kernel(const FewArgs f) {
   constexpr int GT = NT > 1 ? 4 : 2;  // tiles of a gate / up group
   __shared__ __attribute__((aligned(16))) float lds[4 * (NT > GT ? NT : GT) * 64 * 4];
   const int c = threadIdx.x & 15;
