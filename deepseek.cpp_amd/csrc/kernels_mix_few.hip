@@ -273,19 +273,22 @@ DEV void attn_few(const MixFewArgs& f, int b, float* lds) {
 }
 
 // ---- recurrent heads: how a workgroup holds a head's state [dim][vdim] ----------------------------------------
-// Waves are dealt to groups of 64 columns and to ranges of key channels; a lane keeps RK channels of one column.
+// Waves are dealt to groups of 64 columns and to ranges of key channels; a lane keeps RK channels of one column.  A wave's range is a
+// buffer of its own: a row past its end, a column past the head and everything of a sequence's first token read as 0 and are not
+// stored, with no branch per row (behind a mask each, 64 rows kept 64
+// addresses, most of them in scratch memory; a step of one token of a small layered model 2094 -> 2070 us).
 struct HeadTile {
-  int col, k0, kn, parts;  // this lane's column, its channels [k0, k0 + kn), ranges a column is cut into
+  int col, k0, kn, parts;  // this lane's column, its wave's channels [k0, k0 + kn), ranges a column is cut into
   bool on;
 };
 DEV HeadTile head_tile(int dim, int vdim) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int groups = (vdim + 63) >> 6, parts = NW / groups, per = (dim + parts - 1) / parts;
   HeadTile t;
   const int part = wave / groups;
   t.col = wave % groups * 64 + lane;
   t.k0 = part * per;
-  t.kn = max(0, min(per, dim - t.k0));
+  t.kn = part < parts ? max(0, min(per, dim - t.k0)) : 0;
   t.parts = parts;
   t.on = part < parts && t.col < vdim;
   return t;
@@ -294,16 +297,27 @@ static int head_rk(int dim, int vdim) {  // channels a lane holds
   const int parts = NW / cdiv(vdim, 64);
   return cdiv(dim, parts);
 }
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+DEV rsrc_t tile_buffer(const float* S0, const HeadTile& t, int vdim, bool fresh) {
+  const unsigned long long p = (unsigned long long)(S0 + (size_t)t.k0 * vdim);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)p), hi = __builtin_amdgcn_readfirstlane((unsigned)(p >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((unsigned long long)hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(fresh ? 0 : t.kn * vdim * 4), 0x00020000);
+}
+DEV int tile_lane(const HeadTile& t) { return t.on ? t.col * 4 : (int)0x80000000; }  // (past any buffer's end)
 template <int RK>
 DEV void load_state(const float* S0, const HeadTile& t, int vdim, bool fresh, float (&S)[RK]) {
+  const rsrc_t r = tile_buffer(S0, t, vdim, fresh);
+  int at = tile_lane(t);
 #pragma unroll
-  for (int i = 0; i < RK; ++i) S[i] = !fresh && t.on && i < t.kn ? S0[(size_t)(t.k0 + i) * vdim + t.col] : 0.f;
+  for (int i = 0; i < RK; ++i, at += vdim * 4) S[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0));
 }
 template <int RK>
 DEV void store_state(float* S0, const HeadTile& t, int vdim, const float (&S)[RK]) {
+  const rsrc_t r = tile_buffer(S0, t, vdim, false);
+  int at = tile_lane(t);
+  asm("" : "+v"(at));  // (its own additions: the loads' offsets are not kept)
 #pragma unroll
-  for (int i = 0; i < RK; ++i)
-    if (t.on && i < t.kn) S0[(size_t)(t.k0 + i) * vdim + t.col] = S[i];
+  for (int i = 0; i < RK; ++i, at += vdim * 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, S[i]), r, at, 0, 0);
 }
 // behind the recurrence: o[vdim] in LDS -> RMS norm, weight, gate
 template <typename T, typename G>
