@@ -2,6 +2,7 @@
 // "second-stage projections + attention" kernel (kernels_gemv.hip).  Same arithmetic as the stand-alone
 // kernels of kernels_misc.hip (rope_kv_mha_kernel / attn_mha_kernel, which the op-level entry points use).
 #pragma once
+#include "lane_device.h"
 #include "dsk_internal.h"
 #include <math.h>
 
@@ -79,8 +80,8 @@ ADEV void q8k_block(const float (&v)[4], int lane, int8_t* qs_blk, float* d_out,
   if (amax == 0.f) imax = lane * 4;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
-    const float oa = __shfl_xor(amax, off), ov = __shfl_xor(vmax, off);
-    const int oi = __shfl_xor(imax, off);
+    const float oa = lane_xor(amax, off), ov = lane_xor(vmax, off);
+    const int oi = lane_xor(imax, off);
     if (oa > amax || (oa == amax && oi < imax)) { amax = oa; vmax = ov; imax = oi; }
   }
   int q[4] = {0, 0, 0, 0};
@@ -97,8 +98,8 @@ ADEV void q8k_block(const float (&v)[4], int lane, int8_t* qs_blk, float* d_out,
   const u32 packed = (u32)(q[0] & 0xff) | ((u32)(q[1] & 0xff) << 8) | ((u32)(q[2] & 0xff) << 16) | ((u32)(q[3] & 0xff) << 24);
   reinterpret_cast<u32*>(qs_blk)[lane] = packed;
   int s = q[0] + q[1] + q[2] + q[3];
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
+  s += lane_xor(s, 1);
+  s += lane_xor(s, 2);
   if ((lane & 3) == 0) bsums_blk[lane >> 2] = (int16_t)s;
   if (lane == 0) *d_out = d;
 }
@@ -117,8 +118,8 @@ ADEV void q8k_block_wt(const float (&v)[4], int lane, int8_t* qs_blk, float* d_o
   if (amax == 0.f) imax = lane * 4;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
-    const float oa = __shfl_xor(amax, off), ov = __shfl_xor(vmax, off);
-    const int oi = __shfl_xor(imax, off);
+    const float oa = lane_xor(amax, off), ov = lane_xor(vmax, off);
+    const int oi = lane_xor(imax, off);
     if (oa > amax || (oa == amax && oi < imax)) { amax = oa; vmax = ov; imax = oi; }
   }
   int q[4] = {0, 0, 0, 0};
@@ -135,8 +136,8 @@ ADEV void q8k_block_wt(const float (&v)[4], int lane, int8_t* qs_blk, float* d_o
   const u32 packed = (u32)(q[0] & 0xff) | ((u32)(q[1] & 0xff) << 8) | ((u32)(q[2] & 0xff) << 16) | ((u32)(q[3] & 0xff) << 24);
   __hip_atomic_store(reinterpret_cast<u32*>(qs_blk) + lane, packed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int s = q[0] + q[1] + q[2] + q[3];
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
+  s += lane_xor(s, 1);
+  s += lane_xor(s, 2);
   const int s2 = __shfl_down(s, 4);  // the next sub-block's sum: two int16 go out as one dword
   if ((lane & 7) == 0) __hip_atomic_store(reinterpret_cast<u32*>(bsums_blk) + (lane >> 3), (u32)(s & 0xffff) | ((u32)s2 << 16), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (lane == 0) __hip_atomic_store(d_out, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -4,6 +4,7 @@
 // and four keys in the registers, which is the operand order of the second product when v's key order is permuted alike: the weights
 // never leave their registers.  The next tile's keys and values travel to registers while the current one is worked off.
 #pragma once
+#include "lane_device.h"
 #include "layered_kernels.h"
 #include "seq_device.h"
 
@@ -108,8 +109,8 @@ DEV void attn_tile(const Keys& src, const SeqDesc& sq, int q0, int kts, int vts,
         s[t][i] = pos <= my_pos && pos >= my_first ? s[t][i] * scale2 : -INFINITY;
         mx = fmaxf(mx, s[t][i]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = fmaxf(mx, lane_xor(mx, 16));
+    mx = fmaxf(mx, lane_xor(mx, 32));
     const float ref = mx == -INFINITY ? 0.f : mx;  // nothing visible yet: every weight below is 2^-inf = 0
     const float old = __builtin_amdgcn_exp2f(m - ref);
     float sum = 0.f;
@@ -120,8 +121,8 @@ DEV void attn_tile(const Keys& src, const SeqDesc& sq, int q0, int kts, int vts,
         s[t][i] = __builtin_amdgcn_exp2f(s[t][i] - ref);
         sum += s[t][i];
       }
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
+    sum += lane_xor(sum, 16);
+    sum += lane_xor(sum, 32);
     l = l * old + sum;
     m = mx;
 #pragma unroll

@@ -18,6 +18,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 #define DEV __device__ __forceinline__
 #include "glob_device.h"
+#include "lane_device.h"
 DEV GemvTask glob(GemvTask t) {  // a task of a launch's descriptor
   t.qs = glob(t.qs); t.sc = glob(t.sc); t.hm = glob(t.hm); t.dm = glob(t.dm); t.scale = glob(t.scale);
   t.qs2 = glob(t.qs2); t.sc2 = glob(t.sc2); t.hm2 = glob(t.hm2); t.dm2 = glob(t.dm2); t.scale2 = glob(t.scale2);
@@ -256,14 +257,14 @@ DEV float wave_sum(float v) {  // fixed order: quads, rows of 16, then the four 
 }
 
 // sum over the 2^lpr_log2 lanes that share a row (every lane of the group gets the total);
-// fixed order, DPP inside a 16-lane row, ds_bpermute only across rows
+// fixed order, DPP inside a 16-lane row, lane swaps across rows
 DEV float lanes_sum(float v, int lpr_log2) {
   if (lpr_log2 >= 1) v += dpp_f32<DPP_XOR1>(v);
   if (lpr_log2 >= 2) v += dpp_f32<DPP_XOR2>(v);
   if (lpr_log2 >= 3) v += dpp_f32<DPP_HALF_MIRROR>(v);
   if (lpr_log2 >= 4) v += dpp_f32<DPP_MIRROR>(v);
-  if (lpr_log2 >= 5) v += __shfl_xor(v, 16);
-  if (lpr_log2 >= 6) v += __shfl_xor(v, 32);
+  if (lpr_log2 >= 5) v += lane_xor(v, 16);
+  if (lpr_log2 >= 6) v += lane_xor(v, 32);
   return v;
 }
 

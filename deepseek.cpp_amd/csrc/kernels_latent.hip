@@ -254,7 +254,7 @@ __global__ __launch_bounds__(FEW_NT) void latent_few_kernel(const LatentArgs a) 
       }
       float m = sc;
 #pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+      for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, lane_xor(m, off));
       const float w = expf(sc - m), l = wave_sum(w);
       if (lane < N) pw[hh * LP + lane] = (T)w;
       if (lane == 0 && h0 + hh < a.heads) {
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void latent_values_kernel(const LatentArgs a) 
   float m = -INFINITY, l = 0.f;              // (every wave for itself)
   for (int k = lane; k < n; k += 64) m = fmaxf(m, ml[2 * k]);
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, lane_xor(m, off));
   for (int k = lane; k < n; k += 64) {
     const float e = expf(ml[2 * k] - m);
     l += e * ml[2 * k + 1];

@@ -19,12 +19,12 @@ DEV unsigned short f2h(float f) { return __builtin_bit_cast(unsigned short, (_Fl
 
 DEV float wave_sum(float v) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+  for (int off = 32; off >= 1; off >>= 1) v += lane_xor(v, off);
   return v;
 }
 DEV float wave_max(float v) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, lane_xor(v, off));
   return v;
 }
 // block-wide reductions through a small LDS scratch (deterministic order); all threads get the result
@@ -67,8 +67,8 @@ DEV void q8k_block(const float (&v)[4], int lane, int8_t* qs_blk, float* d_out, 
   if (amax == 0.f) imax = lane * 4;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
-    const float oa = __shfl_xor(amax, off), ov = __shfl_xor(vmax, off);
-    const int oi = __shfl_xor(imax, off);
+    const float oa = lane_xor(amax, off), ov = lane_xor(vmax, off);
+    const int oi = lane_xor(imax, off);
     if (oa > amax || (oa == amax && oi < imax)) { amax = oa; vmax = ov; imax = oi; }
   }
   int q[4] = {0, 0, 0, 0};
@@ -85,8 +85,8 @@ DEV void q8k_block(const float (&v)[4], int lane, int8_t* qs_blk, float* d_out, 
   const u32 packed = (u32)(q[0] & 0xff) | ((u32)(q[1] & 0xff) << 8) | ((u32)(q[2] & 0xff) << 16) | ((u32)(q[3] & 0xff) << 24);
   reinterpret_cast<u32*>(qs_blk)[lane] = packed;
   int s = q[0] + q[1] + q[2] + q[3];
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
+  s += lane_xor(s, 1);
+  s += lane_xor(s, 2);
   if ((lane & 3) == 0) bsums_blk[lane >> 2] = (int16_t)s;
   if (lane == 0) *d_out = d;
 }

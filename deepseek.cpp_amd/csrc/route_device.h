@@ -1,5 +1,6 @@
 // route_device.h -- the router's choice of experts on the device: per row, and for up to 16 rows as one workgroup's work.
 #pragma once
+#include "lane_device.h"
 #include "layered_kernels.h"
 #include "seq_device.h"
 
@@ -31,8 +32,8 @@ DEV void choose(const float* z, int experts, int top, int lane, int* e_out, floa
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
-      const float ob = __shfl_xor(best, off);
-      const int oe = __shfl_xor(be, off);
+      const float ob = lane_xor(best, off);
+      const int oe = lane_xor(be, off);
       if (oe != 0x7fffffff && (be == 0x7fffffff || ob > best || (ob == best && oe < be))) {
         best = ob;
         be = oe;

@@ -2,6 +2,7 @@
 // gate_kernel) and kernels_gemv.hip (router_shared_kernel: the router launch that also carries the shared expert's
 // w1/w3 GLU on the CUs the router leaves idle).
 #pragma once
+#include "lane_device.h"
 #include "attn_device.h"
 
 namespace rd {
@@ -14,7 +15,7 @@ typedef ad::u32x4 u32x4;
 // block-wide reductions through a small LDS scratch (xor-shuffle wave trees: the order the gate has always used)
 RDEV float block_sum(float v, float* scratch, int tid, int nthreads) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+  for (int off = 32; off >= 1; off >>= 1) v += lane_xor(v, off);
   const int nw = nthreads >> 6;
   __syncthreads();
   if ((tid & 63) == 0) scratch[tid >> 6] = v;
@@ -25,7 +26,7 @@ RDEV float block_sum(float v, float* scratch, int tid, int nthreads) {
 }
 RDEV float block_max(float v, float* scratch, int tid, int nthreads) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, lane_xor(v, off));
   const int nw = nthreads >> 6;
   __syncthreads();
   if ((tid & 63) == 0) scratch[tid >> 6] = v;

@@ -9,6 +9,7 @@
 #pragma once
 #include "dsk_internal.h"
 #include "glob_device.h"
+#include "lane_device.h"
 #include "layered_kernels.h"
 
 typedef __bf16 bf16;
@@ -102,7 +103,7 @@ DEV float logsigmoid_f(float x) { return -softplus_f(-x); }
 
 DEV float wave_sum(float v) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+  for (int off = 32; off >= 1; off >>= 1) v += lane_xor(v, off);
   return v;
 }
 // sum over a row of 16 lanes, result in all of them: four DPP adds

@@ -31,6 +31,7 @@
 // Any split of a strip's items over waves / workgroups / launches gives the same bits: the fused expert launch equals the
 // two-launch form, a shard equals the unsharded model, whatever the grids.
 #pragma once
+#include "lane_device.h"
 #include "gemv_device.h"
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -185,7 +186,7 @@ DEV float tile_strip_value(const float* red_strip, int ips, int lane) {
     for (int k = 0; k < 8; ++k)
       if (k0 + k < ips) sg += p[k];
   }
-  const float a = sg + __shfl_xor(sg, 16);
-  return a + __shfl_xor(a, 32);
+  const float a = sg + lane_xor(sg, 16);
+  return a + lane_xor(a, 32);
 }
 
