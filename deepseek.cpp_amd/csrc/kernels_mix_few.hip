@@ -274,9 +274,9 @@ DEV void attn_few(const MixFewArgs& f, int b, float* lds) {
 
 // ---- recurrent heads: how a workgroup holds a head's state [dim][vdim] ----------------------------------------
 // Waves are dealt to groups of 64 columns and to ranges of key channels; a lane keeps RK channels of one column.  A wave's range is a
-// buffer of its own: a row past its end, a column past the head and everything of a sequence's first token read as 0 and are not
-// stored, with no branch per row (behind a mask each, 64 rows kept 64
-// addresses, most of them in scratch memory; a step of one token of a small layered model 2094 -> 2070 us).
+// buffer of its own: a row past its end and a column past the head read as 0 and are not stored, a sequence's first token reads nothing
+// but zeros, with no branch per row (behind a mask each, 64 rows kept 64 addresses, most of them in scratch memory; a step of one
+// token of a small layered model 2094 -> 2070 us).
 struct HeadTile {
   int col, k0, kn, parts;  // this lane's column, its wave's channels [k0, k0 + kn), ranges a column is cut into
   bool on;

@@ -33,6 +33,18 @@ def test_q8k_edge_cases_vs_reference(ctx, ops_gold):
     assert np.array_equal(d, ops_gold["q8_d"])
 
 
+@pytest.mark.parametrize("step", [1, 4, 8, 16, 32, 64, 128])
+def test_q8k_largest_value_at_every_place(ctx, oracle, step):
+    """The largest value and its place go through exchanges at every distance between lanes: a block for each place of the
+    largest, with an equal value of the other sign `step` elements behind it (the first one's sign counts)."""
+    x = np.random.default_rng(step).uniform(-0.9, 0.9, (256, 256)).astype(np.float32)
+    for i in range(256):
+        x[i, i] = 1.0
+        x[i, (i + step) % 256] = -1.0
+    a, b = ctx.q8k_quantize(x.reshape(-1)), oracle.q8k_quantize(x.reshape(-1))
+    assert all(np.array_equal(u, v) for u, v in zip(a, b))
+
+
 def test_q8k_rejects_ragged(ctx):
     import dsk
     with pytest.raises(dsk.DskError):
