@@ -23,7 +23,12 @@ def test_chunks_of_time_mixing(case, dim):
     check(case(U.sandwich([U.no_ff(U.wkv(2, dim))], width=72)))
 
 
-def check(K):
+def test_gates_of_long_sequences(case):
+    """the running maximum goes from wave to wave every 64 tokens, from round to round every 1024"""
+    check(case(U.config([U.parallel(right=U.mlstm(1, 16, 16, 9.0))], width=72, eps=0.05)), [63, 64, 65, 128, 1023, 1024, 1025, 1090])
+
+
+def check(K, LENGTHS=LENGTHS):
     toks = [K.tokens(n + 5, seed=n) for n in LENGTHS]
     want = [K.want(t) for t in toks]
     seqs = [K.lm.seq_open() for _ in toks]
