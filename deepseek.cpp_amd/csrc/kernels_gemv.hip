@@ -23,6 +23,7 @@
 //     (src/infer.cpp:859-872) and the MoE accumulate x += w_k * (W2_k . h_k) over the routed
 //     slots in k order, then the shared expert (src/infer.cpp:873-878, 899-903);
 //   * all reductions are fixed-order shuffles: no atomics, bit-reproducible run to run.
+#include <type_traits>
 #include "dsk_internal.h"
 #include "gemv_device.h"
 #include "tile_gemv.h"
@@ -802,19 +803,31 @@ __global__ __launch_bounds__(1024) void head_attn_kernel(const HeadAttnArgs A, c
     const KQRsrc B = kq_rsrc<QT, false>(P);
     const int nb = T.n >> 8;
     if constexpr (!KQ) {
-      // Float weights are 3 - 50 times a K-quant head's bytes and cheap to multiply: a wave requests 8 of its row sets at once instead of waiting for
-      // each: V2-Lite's 256 rows of 512 in F8 took 8.3 us, now 5.6
-      constexpr int RS = 8;
-      for (int base = wave * RPW; base < nrows; base += NW * RPW * RS) {
-        int row[RS];
-        float acc[RS], acc2[RS];
+      // Float weights are 3 - 50 times a K-quant head's bytes and cheap to multiply: a wave requests several of its row sets at once instead of
+      // waiting for each, but a set past the head's end costs what a real one does (its last row again): as few rounds of at most 8 sets as cover the
+      // head (beyond 16 sets all 8), and no more sets in a round than that takes.  The launch in us with one set after the other / always 8 / by this rule: F8, 256 rows
+      // of 512 (V2-Lite) 14.9 / 11.6 / 11.8, 64 rows of 512 8.9 / 11.0 / 8.9, 64 of 256 8.1 / 10.5 / 8.3; 192 rows of 1536 and 256 of 512 for each
+      // of 128 heads, F8 26.7 / 23.7 / 22.4, F16 39.4 / 37.2 / 32.2; F32, 64 rows of 512 11.0 / 12.9 / 10.4.
+      auto rows_of = [&](auto at_once) {
+        constexpr int RS = decltype(at_once)::value;
+        for (int base = wave * RPW; base < nrows; base += NW * RPW * RS) {
+          int row[RS];
+          float acc[RS], acc2[RS];
 #pragma unroll
-        for (int r = 0; r < RS; ++r) row[r] = h * nrows + min(base + r * NW * RPW + rloc, nrows - 1);
-        rows_dot_f<QT, RS, 1, false>(P, T.n, A.b0, A.b1, lpr_log2, lane, row, act, acc, acc2);
+          for (int r = 0; r < RS; ++r) row[r] = h * nrows + min(base + r * NW * RPW + rloc, nrows - 1);
+          rows_dot_f<QT, RS, 1, false>(P, T.n, A.b0, A.b1, lpr_log2, lane, row, act, acc, acc2);
 #pragma unroll
-        for (int r = 0; r < RS; ++r)
-          if (sub == 0 && base + r * NW * RPW + rloc < nrows) out_lds[base + r * NW * RPW + rloc] = acc[r];
-      }
+          for (int r = 0; r < RS; ++r)
+            if (sub == 0 && base + r * NW * RPW + rloc < nrows) out_lds[base + r * NW * RPW + rloc] = acc[r];
+        }
+      };
+      const int sets = (nrows + NW * RPW - 1) >> (10 - lpr_log2);  // (16 waves of 64 >> lpr_log2 rows)
+      const int need = sets <= 8 ? sets : sets <= 16 ? (sets + 1) >> 1 : 8;
+      if (need > 6) rows_of(std::integral_constant<int, 8>{});
+      else if (need > 4) rows_of(std::integral_constant<int, 6>{});
+      else if (need > 2) rows_of(std::integral_constant<int, 4>{});
+      else if (need > 1) rows_of(std::integral_constant<int, 2>{});
+      else rows_of(std::integral_constant<int, 1>{});
       return;
     }
     for (int base = wave * RPW; base < nrows; base += NW * RPW) {  // wave-uniform bounds, no barrier inside

@@ -19,9 +19,20 @@ def test_scale_blocks_of_any_size(ctx, oracle, block, rows, n):
     assert np.abs(ctx.gemv(2, w8, rows, n, x, s8, block) - want).max() < 2e-5 * np.abs(want).max()
 
 
-# 16 waves of 2 (F8), 1 (F16, F32) rows take 8 row sets at once: heads of fewer rows, of just as many and of more
+# 16 waves of 2 (F8), 1 (F16, F32) rows are a row set, up to 8 sets are taken at once: heads of fewer rows, of just as many and of more
 @pytest.mark.parametrize("quant,nope,vd", [("f8e5m2", 128, 128), ("f8e5m2", 128, 256), ("fp16", 64, 64), ("fp16", 96, 64), ("fp32", 64, 64), ("fp32", 32, 160)])
 def test_head_rows_over_row_sets(ctx, oracle, quant, nope, vd):
+    check_head(ctx, oracle, quant, nope, vd)
+
+
+# every number of sets at once (1, 2, 4, 6, 8), in one round and in more, the last set whole, ragged and past the head's end
+@pytest.mark.parametrize("quant,nope,vd", [("f8e5m2", 16, 12), ("f8e5m2", 16, 16), ("f8e5m2", 20, 24), ("f8e5m2", 48, 48), ("f8e5m2", 64, 72), ("f8e5m2", 96, 96), ("f8e5m2", 112, 100),
+                                           ("fp16", 8, 8), ("fp16", 64, 72), ("fp16", 96, 92), ("fp16", 128, 148), ("fp32", 8, 20), ("fp32", 40, 36), ("fp32", 96, 96)])
+def test_head_rows_of_any_number_of_sets(ctx, oracle, quant, nope, vd):
+    check_head(ctx, oracle, quant, nope, vd)
+
+
+def check_head(ctx, oracle, quant, nope, vd):
     c = synth.preset("tiny_v2lite", quant, False, qk_nope_head_dim=nope, v_head_dim=vd, kv_lora_rank=512)
     T = synth.synth_model(c, seed=5)
     import dsk
