@@ -304,10 +304,13 @@ DEV float load1(rsrc_t r, int off) {
 // loads waits for its stores (mLSTM: 77 us with its loads in that wave, 47 without).  Their half of S0's products is issued in the shadow of the
 // exchange.  Operands come as buffer loads whose offsets stay in registers (a chunk costs scalar additions), a chunk or two ahead
 // (NB; more gained nothing), and the waits count: no step of the loop may be skipped behind another, and a wave's tiles are all there
-// (FULL) or tested.  All columns of a head read the same operands: an XCD takes a range of (sequence, head, columns) in this order, so
-// that its L2 gets them once.  Three waves a SIMD: two workgroups share a compute unit.
-// 2048 tokens, 16 heads: delta rule of 128 x 128 177 -> 119 us, mLSTM of 64 x 129 100 -> 47; four sequences of up to 901 tokens: delta rule
-// 114 -> 107, wkv of 32 heads of 64 x 64 57 -> 37.
+// (FULL) or tested.  All columns of a head read the same operands: an XCD takes a range of (head, sequence, columns) in this order, so
+// that its L2 gets them once and every XCD has a share of each sequence.  (With the sequence in front a long one had two XCDs to itself, two
+// workgroups to a compute unit, and the others waited: 900, 300 and 100 tokens, delta rule of 16 heads 115 us, 63 in this order; 331, 700, 64 and 901
+// tokens 129, now 102.)  Three waves a SIMD: two workgroups share a compute unit.
+// In prompts' passes, with the outputs in turn by the four waves -> now: 2048 tokens, 16 heads: delta rule of 128 x 128 190 -> 133 us, mLSTM of
+// 64 x 129 110 -> 52; those four sequences: delta rule 126 -> 102, wkv of 32 heads of 64 x 64 63 -> 42; 64 heads, 400, 333, 400 and 350 tokens: delta
+// rule 283 -> 290 (the card is full either way), wkv of 112 heads 84 -> 72.
 template <typename T, int KIND, int NTL, bool FULL>
 __global__ __launch_bounds__(64 * SCAN_WAVES) __attribute__((amdgpu_waves_per_eu(NTL > 2 ? 2 : 3))) void chunk_scan_kernel(const ScanArgs a) {
   constexpr bool DELTA = KIND == SCAN_DELTA, NORM = KIND == SCAN_MLSTM;
@@ -316,10 +319,10 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) __attribute__((amdgpu_waves_per_eu
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
   const int dp = (a.dim + 15) / 16 * 16, tiles = dp >> 4;
   const int cols = NORM ? a.vdim + 1 : a.vdim, col_tiles = (cols + 15) >> 4;
-  const int place = xcd_range(blockIdx.x, gridDim.x), head = place / col_tiles, h = head % a.heads;
-  const int col = (place - head * col_tiles) * 16 + c16;
+  const int place = xcd_range(blockIdx.x, gridDim.x), hs = place / col_tiles, h = hs / a.p.n_seqs;
+  const int col = (place - hs * col_tiles) * 16 + c16;
   const bool live = col < cols, norm = NORM && col == a.vdim;
-  const SeqDesc s = seq_at(a.p.seqs + head / a.heads);
+  const SeqDesc s = seq_at(a.p.seqs + (hs - h * a.p.n_seqs));
   const int nc = (s.len + CH - 1) / CH;
   // this sequence's and head's operands and values, chunk by chunk (chunks behind the last: the last again)
   const int ops_bytes = (49 * dp + 512) * 4, ld = a.ld_v * (int)sizeof(T);

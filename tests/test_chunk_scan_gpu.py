@@ -23,6 +23,14 @@ def test_chunks_of_time_mixing(case, dim):
     check(case(U.sandwich([U.no_ff(U.wkv(2, dim))], width=72)))
 
 
+# key sizes past 128 (four tiles a wave, all of them there and not), several heads and column tiles, sequences of all lengths side by side
+@pytest.mark.parametrize("layer", [U.channel_delta(U.delta(2, 1, 130, 40, 3)), U.channel_delta(U.delta(3, 3, 256, 33, 2)),
+                                   U.parallel(right=U.mlstm(3, 130, 33, 9.0)), U.parallel(right=U.mlstm(2, 256, 16, 9.0))],
+                         ids=["delta-130", "delta-256", "mlstm-130", "mlstm-256"])
+def test_chunks_of_large_keys(case, layer):
+    check(case(U.config([layer], width=72, eps=0.05)))
+
+
 def test_gates_of_long_sequences(case):
     """the running maximum goes from wave to wave every 64 tokens, from round to round every 1024"""
     check(case(U.config([U.parallel(right=U.mlstm(1, 16, 16, 9.0))], width=72, eps=0.05)), [63, 64, 65, 128, 1023, 1024, 1025, 1090])
