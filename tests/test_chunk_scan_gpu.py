@@ -31,8 +31,38 @@ def test_chunks_of_large_keys(case, layer):
     check(case(U.config([layer], width=72, eps=0.05)))
 
 
+# 16-bit values are loads of two bytes out of buffers that start at any two bytes (odd numbers of columns) and end with the sequence: against the
+# recurrence token by token on the same 16-bit inputs.  Both sum in 32 bits, so that a value may be rounded to the other of two neighbours behind
+# the mixer and once more behind the last norm, 2^-8 of it each; a wrong row or column is far more.
+@pytest.mark.parametrize("c", [U.config([U.parallel(right=U.mlstm(3, 64, 31, 9.0))], width=72, eps=0.05), U.config([U.parallel(right=U.mlstm(2, 130, 17, 9.0))], width=72, eps=0.05),
+                               U.sandwich([U.no_ff(U.wkv(3, 21))], width=72), U.sandwich([U.no_ff(U.wkv(2, 64))], width=72)],
+                         ids=["mlstm-64", "mlstm-130", "wkv-21", "wkv-64"])
+def test_chunks_in_16_bits(case, c):
+    K, L = case(c, dtype="bfloat16"), case(c, dtype="bfloat16", options="chunk_scan=0")
+    toks = [K.tokens(n + 5, seed=n) for n in LENGTHS]
+    a, b = [K.lm.seq_open() for _ in toks], [L.lm.seq_open() for _ in toks]
+    for cut in ([(t[:n], range(n)) for t, n in zip(toks, LENGTHS)], [(t[n:], range(5)) for t, n in zip(toks, LENGTHS)]):
+        got, want = K.lm.step([(s, *e) for s, e in zip(a, cut)]), L.lm.step([(s, *e) for s, e in zip(b, cut)])
+        assert U.err(got, want) < 2 ** -7
+
+
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 1090, 2047, 2048, 2049, 2100, 3200])
+def test_gates_of_a_long_sequence(case, n):
+    """the running maximum goes from wave to wave every 64 tokens and from round to round every 1024, the third round into the first one's buffer:
+    one sequence in one pass (whose rows the trace holds)"""
+    K = case(U.config([U.parallel(right=U.mlstm(2, 16, 16, 9.0))], width=72, eps=0.05), options="piece_tokens=4096")
+    t = K.tokens(n + 5, seed=n)
+    want = K.want(t)
+    K.lm.set_trace(True)
+    s = K.lm.seq_open()
+    got = K.lm.step([(s, t[:n], range(n))])
+    K.lm.trace_rows(0, n)  # (an error if the last pass held fewer)
+    assert U.err(got, want[:n]) < 3e-5
+    assert U.err(K.lm.step([(s, t[n:], range(5))]), want[n:]) < 3e-5
+
+
 def test_gates_of_long_sequences(case):
-    """the running maximum goes from wave to wave every 64 tokens, from round to round every 1024"""
+    """... and sequences of such lengths side by side, as passes of 2048 rows cut them"""
     check(case(U.config([U.parallel(right=U.mlstm(1, 16, 16, 9.0))], width=72, eps=0.05)), [63, 64, 65, 128, 1023, 1024, 1025, 1090])
 
 
