@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const DeltaArgs a, f
 // m_t = max(f_t + m_(t-1), i_t) composes: (F, I) then (f, i) = (F + f, max(I + f, i)); one workgroup per (head, sequence), a wave per 64 tokens.
 // What bounds it is the chain of a wave's turn (gates, six exchanges that depend on each other, exponentials), not bytes, and only its last sum and
 // maximum depend on the tokens before: the waves make their turns side by side and hand the two numbers on through LDS.  2048 tokens, 16 heads, a
-// wave taking all turns one after the other: 44 us (37 with its loads requested two turns ahead), so below 21; the sums are formed in the same order.
+// wave taking all turns one after the other: 43 us (37 with its loads requested two turns ahead), so 13; the sums are formed in the same order.
 enum { GATE_WAVES = 16 };
 __global__ __launch_bounds__(64 * GATE_WAVES) void mlstm_gates_kernel(const MlstmArgs a, const ChunkScan c) {
   __shared__ float tot[2][GATE_WAVES][2];

@@ -2,7 +2,9 @@
 //
 // __shfl_xor is an LDS instruction (ds_bpermute: an address, a round trip of some 100 cycles, six of them in a row for a wave's sum, eighteen for
 // a block's largest value and its place).  Inside a row of 16 lanes the exchange is a modifier of a vector instruction, across rows one of
-// gfx950's two lane swaps (a DeepSeek token of Q2_K weights 1489 -> 1466 us).  `off` is a constant behind unrolling.
+// gfx950's two lane swaps.  Both in turn on one card, us a token: DeepSeek-V2-Lite's shapes, Q2_K 1459 -> 1431, F8E5M2 1608 -> 1589; 27 small layers with
+// recurrences 2098 -> 2064; V3's shapes and wide layers the same.  `off` is a constant behind unrolling.  Still by LDS: attention in
+// kernels_mix_few.hip, mla_flash_kernel, sampling, and shifts (__shfl_up: the mLSTM's gates).
 #pragma once
 #include <hip/hip_runtime.h>
 template <typename T>

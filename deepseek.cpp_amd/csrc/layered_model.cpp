@@ -1139,8 +1139,9 @@ int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
 }
 
 // Logits of up to FEW rows that only the caller reads are stored into pinned host memory by the product itself: the bytes travel while the weights
-// are still streaming, and no copy follows the last kernel.  (Whole tiles of 16 features: a row of host memory has no padding.)  With make_pages
-// below: steps of 4 rows of 129280 1534 -> 1310 us, of 16 rows 6048 -> 5772, of one row of 102400 2251 -> 2146; the product takes as long as before.
+// are still streaming, and no copy follows the last kernel.  (Whole tiles of 16 features: a row of host memory has no padding.)  Into fresh buffers
+// of the caller's, us a step copied / stored / stored and make_pages below: 4 rows of 129280 1840 / 1645 / 1280, 16 rows 6490 / 6180 / 5510, one row
+// 1358 / 1246 / 1186, 8 rows of 102400 5050 / 4800 / 4250, one row 2230 / 2140 / 2093.  The product takes as long as before.
 bool straight_to_host(const LayeredModel* m, int n, int mode) { return mode == OUT_LOGITS && n <= FEW && m->s.vocab % 16 == 0; }
 // logits of hw rows [r0, r0 + n) into m->logits, or straight_to_host
 int run_head(LayeredModel* m, int r0, int n, int mode) {
