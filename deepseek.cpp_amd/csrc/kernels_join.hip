@@ -1,278 +1,33 @@
 // kernels_join.hip -- between the matrix products of layered models: the 32-bit residual sum with the norm behind it, the causal
 // convolution and the blends with the previous token that may follow the norm, and the router's choice of experts.
+#include "join_device.h"
 #include "layered_kernels.h"
 #include "route_device.h"
-#include "seq_device.h"
 
 #include <math.h>
 
 // ---- residual + norm -----------------------------------------------------------------------------
-// One workgroup per row; a thread keeps VPT groups of V consecutive elements in registers (V = 4, or 1 for widths that 4 does not divide).
-template <typename S, int V>
-DEV void load_v(const S* p, bool in, float (&v)[V]) {
-  if constexpr (V == 4) {
-    typedef S s4 __attribute__((ext_vector_type(4)));
-    const s4 q = in ? *reinterpret_cast<const s4*>(p) : s4{};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (float)q[e];
-  } else {
-    v[0] = in ? (float)p[0] : 0.f;
-  }
-}
-template <typename S, int V>
-DEV void store_v(S* p, const float (&v)[V]) {
-  if constexpr (V == 4) {
-    typedef S s4 __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<s4*>(p) = s4{(S)v[0], (S)v[1], (S)v[2], (S)v[3]};
-  } else {
-    p[0] = (S)v[0];
-  }
-}
-// A sequence's only token of the pass: V channels of h through the convolution.  TAPS = 4: what that needs from memory is requested at
-// once, early enough to be there when h is (the blends' weights: up to MAX_MIX); TAPS = 1: any number of taps, one after the other.
-template <int V, int TAPS>
-struct ConvOne {
-  enum { MAX_MIX = 5, KEPT = TAPS > 1 ? TAPS - 1 : 1, MIX = TAPS > 1 ? (int)MAX_MIX : 1 };
-  float old[KEPT][V], w[V * TAPS], mu[MIX][V], prev[V];
-  const float* hist;
-  float *next, *p_next;
-  DEV void load(const JoinArgs& j, const SeqDesc& s, int c) {
-    const ConvArgs& a = j.conv;
-    const int D = j.width, taps = TAPS > 1 ? TAPS : a.taps;
-    hist = reinterpret_cast<const float*>(s.state + a.off_in) + (size_t)s.flip * (taps - 1) * D + c;
-    next = reinterpret_cast<float*>(s.state + a.off_in) + (size_t)(s.flip ^ 1) * (taps - 1) * D + c;
-    p_next = reinterpret_cast<float*>(s.state + a.off_prev) + c + (size_t)(s.flip ^ 1) * D;
-    if (c >= D) return;
-    if constexpr (TAPS > 1) {
-#pragma unroll
-      for (int t = 0; t < KEPT; ++t) load_v<float, V>(hist + (size_t)t * D, s.pos0 - (taps - 1) + t >= 0, old[t]);
-#pragma unroll
-      for (int e = 0; e < TAPS; ++e) load_v<float, V>(a.w + (size_t)c * taps + e * V, true, *reinterpret_cast<float(*)[V]>(w + e * V));
-    }
-    if (a.mu) {
-      load_v<float, V>(reinterpret_cast<const float*>(s.state + a.off_prev) + c + (size_t)s.flip * D, s.pos0 > 0, prev);
-      if constexpr (TAPS > 1) {
-#pragma unroll
-        for (int i = 0; i < MIX; ++i) load_v<float, V>(a.mu + (size_t)min(i, a.n_mix - 1) * D + c, true, mu[i]);
-      }
-    }
-  }
-  template <typename T>
-  DEV void run(const JoinArgs& j, int row, int pos0, int c, const float (&h)[V]) {
-    const ConvArgs& a = j.conv;
-    const int D = j.width, taps = TAPS > 1 ? TAPS : a.taps;
-    T* out = reinterpret_cast<T*>(a.out_t) + (size_t)row * a.ld + c;
-    float y[V];
-#pragma unroll
-    for (int e = 0; e < V; ++e) y[e] = 0.f;
-    if constexpr (TAPS > 1) {
-#pragma unroll
-      for (int t = 0; t < TAPS; ++t)
-#pragma unroll
-        for (int e = 0; e < V; ++e) y[e] += (t == TAPS - 1 ? h[e] : old[t < KEPT ? t : 0][e]) * w[e * TAPS + t];
-#pragma unroll
-      for (int t = 1; t < KEPT; ++t) store_v<float, V>(next + (size_t)(t - 1) * D, old[t]);
-    } else {
-      for (int t = 0; t < taps - 1; ++t) {
-        float o[V];
-        load_v<float, V>(hist + (size_t)t * D, pos0 - (taps - 1) + t >= 0, o);
-#pragma unroll
-        for (int e = 0; e < V; ++e) y[e] += o[e] * a.w[(size_t)(c + e) * taps + t];
-        if (t > 0) store_v<float, V>(next + (size_t)(t - 1) * D, o);
-      }
-#pragma unroll
-      for (int e = 0; e < V; ++e) y[e] += h[e] * a.w[(size_t)(c + e) * taps + taps - 1];
-    }
-    if (taps > 1) store_v<float, V>(next + (size_t)(taps - 2) * D, h);
-#pragma unroll
-    for (int e = 0; e < V; ++e) y[e] += h[e];
-    if (!a.mu) {
-      store_v<T, V>(out, y);
-      return;
-    }
-    store_v<float, V>(p_next, y);
-    auto blend = [&](int i, const float (&m)[V]) {
-      float v[V];
-#pragma unroll
-      for (int e = 0; e < V; ++e) v[e] = y[e] + (prev[e] - y[e]) * m[e];
-      store_v<T, V>(out + i * a.mix_stride, v);
-    };
-    if constexpr (TAPS > 1) {
-#pragma unroll
-      for (int i = 0; i < MIX; ++i)
-        if (i < a.n_mix) blend(i, mu[i]);
-    } else {
-      for (int i = 0; i < a.n_mix; ++i) {
-        float m[V];
-        load_v<float, V>(a.mu + (size_t)i * D + c, true, m);
-        blend(i, m);
-      }
-    }
-  }
-};
-// the sum of up to 8 rows, all requested at once (threads with many groups of elements: one row after the other)
-template <int V, bool MANY>
-struct LoadSum {
-  float q[MANY ? 1 : 8][V];
-  DEV void load(const float* p, bool in, int parts, size_t stride) {
-    if constexpr (MANY) {
-      load_v<float, V>(p, in, q[0]);
-#pragma unroll 1
-      for (int u = 1; u < parts; ++u) {
-        float w[V];
-        load_v<float, V>(p + u * stride, in, w);
-#pragma unroll
-        for (int e = 0; e < V; ++e) q[0][e] += w[e];
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < 8; ++u) load_v<float, V>(p + u * stride, in && u < max(parts, 1), q[u]);
-    }
-  }
-  DEV void sum(float (&v)[V]) const {
-#pragma unroll
-    for (int e = 0; e < V; ++e) v[e] = MANY ? q[0][e] : ((q[0][e] + q[1][e]) + (q[2][e] + q[3][e])) + ((q[4][e] + q[5][e]) + (q[6][e] + q[7][e]));
-  }
-};
-// CONV: taps of the convolution behind the norm (single tokens; ConvOne), 0: none
 template <typename T, int NT, int VPT, int V, int CONV>
 __global__ __launch_bounds__(NT) void join_kernel(const JoinArgs a) {
-  __shared__ float red[NT / 64], s_w[64];
-  __shared__ int s_pos[64];
-  const int tid = threadIdx.x, D = a.width;
-  const int row = a.only_want ? a.p.want[blockIdx.x] : (int)blockIdx.x;
-  const int hrow = blockIdx.x;
-  float x[VPT][V], add[VPT][V];
-  auto at = [&](int i) { return V * (tid + i * NT); };
-  // with a convolution behind the norm (single tokens: row = sequence): everything it reads and the norms' weights, requested behind the
-  // sum's operands (one group per thread) or together with its use (more)
-  ConvOne<V, (CONV > 1 ? CONV : 1)> cv;
-  SeqDesc sq{};
-  float nw[V], pw[V];
-  if constexpr (CONV > 0) sq = seq_at(a.p.seqs + row);
-  if (a.y_t && tid < a.n_slots) {
-    s_w[tid] = a.weight[(size_t)row * a.n_slots + tid];
-    s_pos[tid] = a.slot_pos[(size_t)row * a.n_slots + tid];
-  }
-#pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    if (a.embed) load_v<bf16, V>(reinterpret_cast<const bf16*>(a.embed) + (size_t)a.p.tokens[row] * D + at(i), at(i) < D, x[i]);
-    else load_v<float, V>(a.x + (size_t)row * D + at(i), at(i) < D, x[i]);
-#pragma unroll
-    for (int e = 0; e < V; ++e) add[i][e] = 0.f;
-  }
-  if constexpr (CONV > 0 && VPT == 1) {
-    if (!a.mix_a) {
-      load_v<float, V>(a.norm_w + at(0), at(0) < D, nw);
-      cv.load(a, sq, at(0));
-    }
-  }
-  if (a.mix_a) {
-    const float* ma = a.mix_a + (size_t)row * a.mix_ld;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      LoadSum<V, (VPT > 2)> q;
-      q.load(ma + at(i), at(i) < D, a.parts_a, a.mix_stride);
-      if constexpr (CONV > 0 && VPT == 1) {
-        if (a.post_w) load_v<float, V>(a.post_w + at(0), at(0) < D, pw);
-        load_v<float, V>(a.norm_w + at(0), at(0) < D, nw);
-        cv.load(a, sq, at(0));
-      }
-      q.sum(add[i]);
-    }
-    if (a.mix_b) {
-      const float* mb = a.mix_b + (size_t)row * a.mix_ld;
-      float vb[VPT][V], sa = 0.f, sb = 0.f;
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        LoadSum<V, (VPT > 2)> q;
-        q.load(mb + at(i), at(i) < D, a.parts_b, a.mix_stride);
-        q.sum(vb[i]);
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-          sa += add[i][e] * add[i][e];
-          sb += vb[i][e] * vb[i][e];
-        }
-      }
-      sa = block_sum<NT>(sa, red);
-      sb = block_sum<NT>(sb, red);
-      const float ra = 1.f / sqrtf(sa / D + a.eps), rb = 1.f / sqrtf(sb / D + a.eps);
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        float wa[V], wb[V];
-        load_v<float, V>(a.pair_wa + at(i), at(i) < D, wa);
-        load_v<float, V>(a.pair_wb + at(i), at(i) < D, wb);
-#pragma unroll
-        for (int e = 0; e < V; ++e) add[i][e] = 0.5f * (add[i][e] * ra * wa[e] + vb[i][e] * rb * wb[e]);
-      }
-    } else if (a.post_w) {
-      float sa = 0.f;
-#pragma unroll
-      for (int i = 0; i < VPT; ++i)
-#pragma unroll
-        for (int e = 0; e < V; ++e) sa += add[i][e] * add[i][e];
-      sa = block_sum<NT>(sa, red);
-      const float ra = 1.f / sqrtf(sa / D + a.eps);
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        float w[V];
-        if constexpr (CONV > 0 && VPT == 1) {
-#pragma unroll
-          for (int e = 0; e < V; ++e) w[e] = pw[e];
-        } else {
-          load_v<float, V>(a.post_w + at(i), at(i) < D, w);
-        }
-#pragma unroll
-        for (int e = 0; e < V; ++e) add[i][e] *= ra * (w[e] + a.norm_offset);
-      }
-    }
-  }
-  if (a.y_t) {
-    __syncthreads();
-#pragma unroll 4
-    for (int k = 0; k < a.n_slots; ++k) {
-      const float w = s_w[k];
-      const T* y = reinterpret_cast<const T*>(a.y_t) + (size_t)s_pos[k] * a.y_ld;
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        float v[V];
-        load_v<T, V>(y + at(i), at(i) < D, v);
-#pragma unroll
-        for (int e = 0; e < V; ++e) add[i][e] += w * v[e];
-      }
-    }
-  }
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      x[i][e] += add[i][e];
-      ss += x[i][e] * x[i][e];
-    }
-    if (!a.only_want && at(i) < D) store_v<float, V>(a.x + (size_t)row * D + at(i), x[i]);
-  }
-  if (!a.norm_w) return;
-  ss = block_sum<NT>(ss, red);
-  const float r = 1.f / sqrtf(ss / D + a.eps);
-  T* h = reinterpret_cast<T*>(a.h_t) + (size_t)hrow * a.h_ld;
-#pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    if (at(i) >= D) continue;
-    float w[V];
-    if constexpr (CONV > 0 && VPT == 1) {
-#pragma unroll
-      for (int e = 0; e < V; ++e) w[e] = nw[e];
-    } else {
-      if constexpr (CONV > 0) cv.load(a, sq, at(i));
-      load_v<float, V>(a.norm_w + at(i), true, w);
-    }
-#pragma unroll
-    for (int e = 0; e < V; ++e) w[e] = x[i][e] * r * (w[e] + a.norm_offset);
-    if constexpr (CONV > 0) cv.template run<T>(a, row, sq.pos0, at(i), w);
-    else if (a.h_f) store_v<float, V>(a.h_f + (size_t)row * D + at(i), w);
-    else store_v<T, V>(h + at(i), w);
-  }
+  __shared__ JoinLds<NT> lds;
+  join_row<T, NT, VPT, V, CONV, false>(a, blockIdx.x, lds);
+}
+template <typename T, int NT, int VPT, int PARTS, int SPLIT, bool MIX>
+__global__ __launch_bounds__(NT) void sandwich_kernel(const SeqDesc* __restrict__ seqs, const JoinArgs a) {
+  __shared__ float red[NT / 64];
+  sandwich_row<T, NT, VPT, PARTS, SPLIT, MIX, false>(a, seqs, blockIdx.x, red);
+}
+template <typename T>
+static int sandwich_t(hipStream_t st, const JoinArgs& a, int n) {
+  const int D = a.width;
+#define ROW(NT, VPT, PARTS, SPLIT) \
+  hipLaunchKernelGGL((a.conv.mu ? sandwich_kernel<T, NT, VPT, PARTS, SPLIT, true> : sandwich_kernel<T, NT, VPT, PARTS, SPLIT, false>), dim3(n * SPLIT), dim3(NT), 0, st, a.p.seqs, a)
+  if (D <= 1024) ROW(256, 1, 8, 1);
+  else if (D <= 2048) ROW(512, 1, 8, 2);
+  else if (D <= 4096) ROW(1024, 1, 8, 4);
+  else ROW(1024, 2, 4, 4);
+#undef ROW
+  return DSK_OK;
 }
 template <typename T, int CONV>
 static int join_t(hipStream_t st, const JoinArgs& a, int n) {
@@ -291,9 +46,11 @@ static int join_t(hipStream_t st, const JoinArgs& a, int n) {
 #undef JOIN
   return DSK_OK;
 }
+bool join_moves(const JoinArgs& a) { return sandwich_fits(a); }
 int launch_join(hipStream_t st, const JoinArgs& a, bool f32) {
   const int n = a.only_want ? a.p.n_want : a.p.rows;
   if (n < 1) DSK_FAIL(DSK_ERR_INVALID, "join: no rows");
+  if (sandwich_fits(a)) return f32 ? sandwich_t<float>(st, a, n) : sandwich_t<bf16>(st, a, n);
   if (!a.conv.w) return f32 ? join_t<float, 0>(st, a, n) : join_t<bf16, 0>(st, a, n);
   if (a.conv.taps == 4 && a.conv.n_mix <= ConvOne<1, 4>::MAX_MIX) return f32 ? join_t<float, 4>(st, a, n) : join_t<bf16, 4>(st, a, n);
   return f32 ? join_t<float, 1>(st, a, n) : join_t<bf16, 1>(st, a, n);

@@ -129,6 +129,7 @@ struct JoinArgs {           // x += (what the previous layer left); h = norm(x)
   int width, h_ld;
   float eps, norm_offset;   // the norm's weight counts as w + norm_offset
   float* x;                 // [rows][width]
+  float* x_next;            // launches that join_moves() names leave the sum here, and x as it is
   const uint16_t* embed;    // first layer: x = embed[token] (nothing to add)
   const float* mix_a;       // mixer output [rows][mix_ld] (nullptr: none)
   int parts_a, parts_b;     // mix_a (mix_b) is the sum of this many, mix_stride elements behind each other
@@ -148,8 +149,8 @@ struct JoinArgs {           // x += (what the previous layer left); h = norm(x)
   ConvArgs conv;            // conv.w: single tokens, convolution and blends in the same launch (h_t and h_f are not used)
 };
 int launch_join(hipStream_t st, const JoinArgs& a, bool f32);
+bool join_moves(const JoinArgs& a);  // the sum goes to x_next (single tokens in front of a sandwich layer's sublayer)
 int launch_conv(hipStream_t st, const PassDesc& p, int width, const float* h_f, const ConvArgs& a, bool f32);
-
 // ---- chunked softmax attention ----
 struct ChunkAttnArgs {
   PassDesc p;

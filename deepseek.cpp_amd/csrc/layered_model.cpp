@@ -106,7 +106,8 @@ struct LayeredModel : ModelHead {
   int32_t own_seq = -1;             // dsk_forward / dsk_hydrate: the model's own sequence
   // workspaces
   int ldw = 0, ldf = 0, h_ld = 0, mix_ld = 0, out_ld = 0, low_ld = 0, hid_ld = 0, y_ld = 0, ld_logits = 0, max_tiles = 0, slots = 0;
-  float* x = nullptr;
+  float *x = nullptr, *x_other = nullptr;  // the residual, and where a launch that moves it leaves the new one: x_all and x_few at the start of a pass
+  float *x_all = nullptr, *x_few = nullptr;
   char *h = nullptr, *hw = nullptr, *wide = nullptr, *out_a = nullptr, *out_b = nullptr, *qb = nullptr, *kb = nullptr, *vb = nullptr, *hidden = nullptr, *y = nullptr;
   float *narrow = nullptr, *mix_a = nullptr, *mix_b = nullptr, *low = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr, *dg = nullptr, *db = nullptr, *o = nullptr;
   int mix_parts[2] = {1, 1};        // of the products that wrote mix_a and mix_b last
@@ -587,7 +588,8 @@ int alloc_work(LayeredModel* m) {
   m->low_ld = low;
   m->slots = tmax;
   m->ld_logits = m->head.rt * 16;
-  DSK_TRY(dev_alloc_n(m, &m->x, n * D));
+  DSK_TRY(dev_alloc_n(m, &m->x_all, n * D));
+  DSK_TRY(dev_alloc_n(m, &m->x_few, (size_t)FEW * D));
   DSK_TRY(dev_alloc(m, (void**)&m->h, n * m->h_ld * e * m->mixes));
   if (sandwich) DSK_TRY(dev_alloc_n(m, &m->h_f, n * D));
   if (m->max_window) {
@@ -1027,6 +1029,8 @@ int enter(LayeredModel* m, JoinArgs j, const float* norm_w, const LayerSpec& s, 
   const ConvArgs conv = conv_args(m, j.p, s, c);
   if (few && m->fused_decode) {
     j.conv = conv;
+    j.x_next = m->x_other;
+    if (join_moves(j)) std::swap(m->x, m->x_other);
     return launch_join(m->ctx->stream, j, m->f32);
   }
   j.h_f = m->h_f;
@@ -1201,6 +1205,8 @@ PassDesc pass_desc(const DescBuf& d, int rows, int n_seqs, int n_want, int n_til
 int run_body(LayeredModel* m, const DescBuf& d, const PassDesc& p, bool few) {
   hipStream_t st = m->ctx->stream;
   const int n = (int)m->L.size();
+  m->x = m->x_all;
+  m->x_other = m->x_few;
   HIP_TRY(hipMemcpyAsync(d.dev, d.host, d.bytes, hipMemcpyHostToDevice, st));
   for (int l = 0; l < n; ++l) DSK_TRY(run_layer(m, p, l, few));
   JoinArgs j = join_args(m, p, n);

@@ -23,6 +23,12 @@ DEV SeqDesc seq_at(const SeqDesc* p) {
   s.state = glob(s.state);
   return s;
 }
+// the same by vector loads: scalar loads come back in any order, so that the first use of any value out of the kernel's arguments waits for all of them
+DEV SeqDesc seq_late(const SeqDesc* p) {
+  int zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+  return seq_at(glob(p) + zero);
+}
 
 template <typename T>
 struct Frag;
