@@ -291,7 +291,7 @@ DEV void join_row(const JoinArgs& a, int block, JoinLds<NT>& lds) {
 // empty where there is nothing to read, so that all of them are on their way at once (behind a branch the compiler waits for each).  What one compute
 // unit takes in bounds it then (a row of 2048: 144 - 184 KiB, of 7168: 350), so SPLIT workgroups share a row: each adds up all of it, for the
 // norms, and makes a part of what follows.  (The new residual goes to x_next: the others still read the old one.)  A launch for one row of 2048 without /
-// with blends 5.8 / 8.0 us as before -> 4.8 / 6.3 without branches -> 4.6 / 5.4 by two workgroups (by four 4.6 / 5.3); four rows of 7168 11.0 / 12.0 ->
+// with blends 5.8 / about 8 us as before -> 4.8 / 6.3 without branches -> 4.6 / 5.4 by two workgroups (by four 4.6 / 5.3); four rows of 7168 11.0 / 12.0 ->
 // 10.4 / 15 -> 9.0 / 12 by two, 8.3 / 11.0 by four, 8.1 / 10.8 by eight.  PARTS: the most parts of the sum; MIX: blends.
 static inline bool sandwich_fits(const JoinArgs& a) {
   return a.conv.w && a.conv.taps == 4 && (!a.conv.mu || a.conv.n_mix <= 5) && !(a.width & 3) && a.width <= 8192 && a.parts_a <= (a.width > 4096 ? 4 : 8) && !a.mix_b && !a.y_t &&

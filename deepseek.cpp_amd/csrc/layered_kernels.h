@@ -151,6 +151,18 @@ struct JoinArgs {           // x += (what the previous layer left); h = norm(x)
 int launch_join(hipStream_t st, const JoinArgs& a, bool f32);
 bool join_moves(const JoinArgs& a);  // the sum goes to x_next (single tokens in front of a sandwich layer's sublayer)
 int launch_conv(hipStream_t st, const PassDesc& p, int width, const float* h_f, const ConvArgs& a, bool f32);
+// The sum and the product that reads its rows in one launch (kernels_enter.hip), bf16, up to ENTER_ROWS rows
+struct EnterSync {
+  unsigned* ready;      // [64]: the tag of the last launch that made the (part of a) row
+  const unsigned* tag;  // *tag + launch: this launch's, a number that `ready` does not hold
+  unsigned launch;
+  unsigned* gave_up;    // set by a workgroup that has looked for a row `spins` times
+  unsigned spins;
+};
+enum { ENTER_SPLIT = 2, ENTER_ROWS = 8 };
+bool enter_fits(const JoinArgs& j, const LinArgs& a);
+int launch_enter(hipStream_t st, const JoinArgs& j, const LinArgs& a, const EnterSync& s);
+
 // ---- chunked softmax attention ----
 struct ChunkAttnArgs {
   PassDesc p;

@@ -77,7 +77,7 @@ struct Seq {
 struct DescBuf {
   char *host = nullptr, *dev = nullptr;
   int cap = 0;
-  size_t o_tok = 0, o_row = 0, o_want = 0, o_tile = 0, o_chunk = 0, o_single = 0, bytes = 0;
+  size_t o_tok = 0, o_row = 0, o_want = 0, o_tile = 0, o_chunk = 0, o_single = 0, o_tag = 0, bytes = 0;
 };
 
 struct Graph {
@@ -91,7 +91,7 @@ struct LayeredModel : ModelHead {
   LayeredSpec s;
   bool f32 = false;
   int piece = 2048;
-  bool use_graph = true, fused_decode = true, trace = false;
+  bool use_graph = true, fused_decode = true, enter_ahead = true, trace = false;
   std::vector<void*> dev;           // device allocations of the model
   double weight_bytes = 0, scratch_bytes = 0;
   uint16_t* embed = nullptr;
@@ -130,8 +130,15 @@ struct LayeredModel : ModelHead {
   int max_chunks = 0;
   float* attn_part = nullptr;       // parts of attention outputs (kernels_mix_few.hip)
   unsigned* attn_arrived = nullptr;
+  // launches that make their rows themselves (kernels_enter.hip): how many this pass has, the tags they leave, the tag of the next pass's first
+  int entered = 0;
+  unsigned* enter_ready = nullptr;
+  unsigned enter_tag = 0;
+  unsigned enter_spins = 1u << 22;  // polls for a row before one of them gives up
+  unsigned* gave_up = nullptr;      // pinned, set then
   int splits = 1;                   // attention workgroups per (sequence, key head) of the current decode step: a power of two
   long long fused_layers = 0;       // layers enqueued with the fused decode launches
+  long long enter_launches = 0;     // ... and launches that make their rows
   std::map<int, Graph> graphs;
   int graph_steps = 0;
   size_t elem() const { return f32 ? 4 : 2; }
@@ -498,6 +505,7 @@ int alloc_desc(LayeredModel* m, DescBuf* d, int cap) {
   d->o_tile = take(2 * (size_t)cap);
   d->o_chunk = take(2 * (size_t)cap);
   d->o_single = take(cap);
+  d->o_tag = take(1);
   d->bytes = off;
   HIP_TRY(hipHostMalloc((void**)&d->host, off, hipHostMallocDefault));
   memset(d->host, 0, off);
@@ -655,6 +663,9 @@ int alloc_work(LayeredModel* m) {
   memset(m->sp_host, 0, sizeof(StepParams) * FEW);
   HIP_TRY(hipHostMalloc((void**)&m->logits_host, (size_t)LOGIT_ROWS * s.vocab * 4, hipHostMallocDefault));
   HIP_TRY(hipHostMalloc((void**)&m->next_host, LOGIT_ROWS * 4, hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc((void**)&m->gave_up, 4, hipHostMallocDefault));
+  *m->gave_up = 0;
+  DSK_TRY(dev_alloc_n(m, &m->enter_ready, 64));  // (zeros: no launch's tag)
   DSK_TRY(alloc_desc(m, &m->big, m->piece));
   DSK_TRY(alloc_desc(m, &m->small, FEW));
   return DSK_OK;
@@ -1022,27 +1033,39 @@ ConvArgs conv_args(LayeredModel* m, const PassDesc& p, const LayerSpec& l, const
   a.mix_stride = (size_t)p.rows * m->h_ld;
   return a;
 }
-// the residual sum and norm in front of a sublayer, and the convolution a sandwich layer has there
-int enter(LayeredModel* m, JoinArgs j, const float* norm_w, const LayerSpec& s, const ConvW& c, bool few) {
+// the residual sum of `j` and the product `a` of its rows: one launch in steps of a few tokens, else `sum` and the product behind it
+template <typename F>
+int sum_and_lin(LayeredModel* m, const JoinArgs& j, const LinArgs& a, bool few, F sum) {
+  if (few && m->fused_decode && m->enter_ahead && !m->f32 && !m->trace && a.rows <= ENTER_ROWS && enter_fits(j, a)) {
+    m->enter_launches++;
+    return launch_enter(m->ctx->stream, j, a, {m->enter_ready, reinterpret_cast<unsigned*>(m->small.dev + m->small.o_tag), (unsigned)m->entered++, m->gave_up, m->enter_spins});
+  }
+  DSK_TRY(sum());
+  return run_lin(m, &a, 1, few);
+}
+// the residual sum and norm in front of a sublayer, the convolution a sandwich layer has there, and the sublayer's first product
+int enter(LayeredModel* m, JoinArgs j, const float* norm_w, const LayerSpec& s, const ConvW& c, const LinArgs& first, bool few) {
+  hipStream_t st = m->ctx->stream;
   j.norm_w = norm_w;
-  if (!s.sandwich) return launch_join(m->ctx->stream, j, m->f32);
-  const ConvArgs conv = conv_args(m, j.p, s, c);
-  if (few && m->fused_decode) {
+  const bool one = few && m->fused_decode;
+  const ConvArgs conv = s.sandwich ? conv_args(m, j.p, s, c) : ConvArgs{};
+  if (s.sandwich && one) {
     j.conv = conv;
     j.x_next = m->x_other;
     if (join_moves(j)) std::swap(m->x, m->x_other);
-    return launch_join(m->ctx->stream, j, m->f32);
   }
-  j.h_f = m->h_f;
-  DSK_TRY(launch_join(m->ctx->stream, j, m->f32));
-  return launch_conv(m->ctx->stream, j.p, m->s.width, m->h_f, conv, m->f32);
+  return sum_and_lin(m, j, first, few, [&]() -> int {
+    if (!s.sandwich || one) return launch_join(st, j, m->f32);
+    JoinArgs k = j;
+    k.h_f = m->h_f;
+    DSK_TRY(launch_join(st, k, m->f32));
+    return launch_conv(st, j.p, m->s.width, m->h_f, conv, m->f32);
+  });
 }
 int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
   const LayerSpec& s = m->s.layers[l];
   const LayerW& w = m->L[l];
   hipStream_t st = m->ctx->stream;
-  DSK_TRY(enter(m, join_args(m, p, l), w.norm, s, w.conv, few));
-  if (m->trace && l > 0) HIP_TRY(hipMemcpyAsync(m->trace_x + (size_t)(l - 1) * m->piece * m->s.width, m->x, (size_t)p.rows * m->s.width * 4, hipMemcpyDeviceToDevice, st));
   LinArgs pr = lin(w.proj, m->h, m->h_ld, p.rows);
   pr.n_wide = w.n_wide;
   pr.out_t = m->wide;
@@ -1055,7 +1078,8 @@ int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
     pr.a_ops = w.conv.n_mix;
     pr.a_stride = (size_t)p.rows * m->h_ld;
   }
-  DSK_TRY(run_lin(m, &pr, 1, few));
+  DSK_TRY(enter(m, join_args(m, p, l), w.norm, s, w.conv, pr, few));
+  if (m->trace && l > 0) HIP_TRY(hipMemcpyAsync(m->trace_x + (size_t)(l - 1) * m->piece * m->s.width, m->x, (size_t)p.rows * m->s.width * 4, hipMemcpyDeviceToDevice, st));
   // the mixers' outputs and their products: attention or the only mixer in `a`, the second of a pair in `b`
   LinArgs outs[2];
   int n_out = 0;
@@ -1118,7 +1142,6 @@ int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
     j.mix_stride = m->mix_stride;
     j.mix_b = nullptr;
     j.post_w = w.post;
-    DSK_TRY(enter(m, j, w.ff_norm, s, w.ff_conv, few));
     LinArgs u = lin(w.ff_up, m->h, m->h_ld, p.rows);
     u.epi = LIN_XIELU;
     u.p0 = w.ff_pos;
@@ -1126,7 +1149,7 @@ int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
     u.n_wide = w.ff_up.rt * 16;
     u.out_t = m->hidden;
     u.ld_t = m->hid_ld;
-    DSK_TRY(run_lin(m, &u, 1, few));
+    DSK_TRY(enter(m, j, w.ff_norm, s, w.ff_conv, u, few));
     const LinArgs d = mix_lin(m, w.ff_down, m->hidden, m->hid_ld, p.rows, few);
     return run_lin(m, &d, 1, few);
   }
@@ -1147,8 +1170,8 @@ int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
 // of the caller's, us a step copied / stored / stored and make_pages below: 4 rows of 129280 1840 / 1645 / 1280, 16 rows 6490 / 6180 / 5510, one row
 // 1358 / 1246 / 1186, 8 rows of 102400 5050 / 4800 / 4250, one row 2230 / 2140 / 2093.  The product takes as long as before.
 bool straight_to_host(const LayeredModel* m, int n, int mode) { return mode == OUT_LOGITS && n <= FEW && m->s.vocab % 16 == 0; }
-// logits of hw rows [r0, r0 + n) into m->logits, or straight_to_host
-int run_head(LayeredModel* m, int r0, int n, int mode) {
+// the product for the logits of hw rows [r0, r0 + n), into m->logits or straight_to_host
+LinArgs head_lin(LayeredModel* m, int r0, int n, int mode) {
   const bool host = straight_to_host(m, n, mode);
   LinArgs a = lin_f(m->head, m->hw + (size_t)r0 * m->h_ld * m->elem(), m->h_ld, n, host ? m->logits_host : m->logits, host ? m->s.vocab : m->ld_logits);
   if (m->s.softcap > 0) {
@@ -1158,6 +1181,10 @@ int run_head(LayeredModel* m, int r0, int n, int mode) {
     a.epi = LIN_SCALE;
     a.p0 = (float)m->s.logit_scale;
   }
+  return a;
+}
+int run_head(LayeredModel* m, int r0, int n, int mode) {
+  const LinArgs a = head_lin(m, r0, n, mode);
   return run_lin(m, &a, 1, n <= FEW);
 }
 int fetch_logits(LayeredModel* m, int n, int mode) {  // behind run_head: n rows into m->logits_host
@@ -1201,10 +1228,11 @@ PassDesc pass_desc(const DescBuf& d, int rows, int n_seqs, int n_want, int n_til
   return p;
 }
 
-// every launch of a pass up to the final norm of the wanted rows (in m->hw)
-int run_body(LayeredModel* m, const DescBuf& d, const PassDesc& p, bool few) {
+// every launch of a pass up to the final norm of the wanted rows (in m->hw); few: their logits too
+int run_body(LayeredModel* m, const DescBuf& d, const PassDesc& p, bool few, int mode) {
   hipStream_t st = m->ctx->stream;
   const int n = (int)m->L.size();
+  m->entered = 0;
   m->x = m->x_all;
   m->x_other = m->x_few;
   HIP_TRY(hipMemcpyAsync(d.dev, d.host, d.bytes, hipMemcpyHostToDevice, st));
@@ -1220,12 +1248,12 @@ int run_body(LayeredModel* m, const DescBuf& d, const PassDesc& p, bool few) {
   j.norm_w = m->final_norm;
   j.h_t = m->hw;
   j.only_want = 1;
-  return launch_join(st, j, m->f32);
+  if (!few) return launch_join(st, j, m->f32);
+  return sum_and_lin(m, j, head_lin(m, 0, p.n_want, mode), true, [&]() { return launch_join(st, j, m->f32); });
 }
 int run_few(LayeredModel* m, const PassDesc& p, int mode) {
-  DSK_TRY(run_body(m, m->small, p, true));
+  DSK_TRY(run_body(m, m->small, p, true, mode));
   if (p.n_want == 0) return DSK_OK;
-  DSK_TRY(run_head(m, 0, p.n_want, mode));
   if (mode == OUT_ARGMAX || mode == OUT_SAMPLE) return run_choice(m, p.n_want, mode);
   return fetch_logits(m, p.n_want, mode);
 }
@@ -1285,6 +1313,14 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
   p.max_hist = max_hist;
   m->last_rows = rows;
   if (few) {
+    // the pass's tags: numbers that no launch has left; when they are through, the words are cleared and the numbers start over
+    const unsigned launches = 2 * (unsigned)m->L.size() + 1;
+    if (m->enter_tag == 0 || m->enter_tag > 0u - 2 * launches) {
+      if (m->enter_tag) HIP_TRY(hipMemsetAsync(m->enter_ready, 0, 64 * sizeof(unsigned), st));
+      m->enter_tag = 1;
+    }
+    *reinterpret_cast<unsigned*>(d.host + d.o_tag) = m->enter_tag;
+    m->enter_tag += launches;
     if (mode == OUT_SAMPLE) {  // (sp_host's temperature and top_p were set by the caller)
       for (int i = 0; i < nw; ++i) m->sp_host[i].coin = coins[i];
     }
@@ -1320,6 +1356,10 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
     }
     if (mode == OUT_LOGITS && out != m->logits_host) make_pages(out, (size_t)nw * m->s.vocab);
     HIP_TRY(hipStreamSynchronize(st));
+    if (*m->gave_up) {
+      *m->gave_up = 0;
+      DSK_FAIL(DSK_ERR_STATE, "step: a launch gave up waiting for its rows; the step's sequences have no valid state (option enter_ahead=0 does without the wait)");
+    }
     if (nw && mode == OUT_LOGITS) {
       if (out != m->logits_host) memcpy(out, m->logits_host, (size_t)nw * m->s.vocab * 4);
     } else if (nw) {
@@ -1327,7 +1367,7 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
     }
   } else {
     m->splits = 1 << 30;  // (a mixer takes as many as its largest window has)
-    DSK_TRY(run_body(m, d, p, false));
+    DSK_TRY(run_body(m, d, p, false, mode));
     const int block = mode == OUT_LOGITS ? LOGIT_ROWS : FEW;
     for (int i = 0; i < nw; i += block) {
       const int n = std::min(block, nw - i);
@@ -1420,7 +1460,7 @@ int l_destroy(dsk_model* h) {
     if (g.second.exec) hipGraphExecDestroy(g.second.exec);
   for (void* p : m->dev) hipFree(p);
   for (void* p : m->slabs) hipFree(p);
-  for (void* p : {(void*)m->sp_host, (void*)m->logits_host, (void*)m->next_host, (void*)m->big.host, (void*)m->small.host})
+  for (void* p : {(void*)m->sp_host, (void*)m->logits_host, (void*)m->next_host, (void*)m->gave_up, (void*)m->big.host, (void*)m->small.host})
     if (p) hipHostFree(p);
   dsk_ctx* ctx = m->ctx;
   delete m;
@@ -1558,6 +1598,7 @@ int l_get_info(dsk_model* h, const char* key, int* value) {
     *value = 0;
     for (auto& g : m->graphs) *value += g.second.exec != nullptr;
   } else if (k == "graph_steps") *value = m->graph_steps;
+  else if (k == "enter_launches") *value = (int)std::min<long long>(m->enter_launches, 0x7fffffff);
   else if (k == "fused_decode_layers") *value = (int)std::min<long long>(m->fused_layers, 0x7fffffff);
   else if (k == "layers") *value = (int)m->L.size();
   else if (k == "width") *value = m->s.width;
@@ -1613,6 +1654,11 @@ int set_options(LayeredModel* m, const char* options) {
       m->piece = v;
     } else if (k == "decode_graph") m->use_graph = v != 0;
     else if (k == "fused_decode") m->fused_decode = v != 0;
+    else if (k == "enter_ahead") m->enter_ahead = v != 0;
+    else if (k == "enter_spins") {
+      if (v < 0) DSK_FAIL(DSK_ERR_INVALID, "open: enter_spins %d", v);
+      m->enter_spins = (unsigned)v;
+    }
     else if (k == "chunk_scan") m->chunk_scan = v != 0;
     else if (k == "prompt_tile") {
       if (v != 0 && v != 128 && v != 256) DSK_FAIL(DSK_ERR_INVALID, "open: prompt_tile %d (0, 128, 256)", v);

@@ -1,4 +1,6 @@
-"""Rows of decoding steps: the residual sum of a sandwich layer shared by several workgroups (join_device.h)."""
+"""Rows of decoding steps: the residual sum of a sandwich layer shared by several workgroups (join_device.h), and the launch that makes its rows
+beside the product that reads them (kernels_enter.hip)."""
+import numpy as np
 import pytest
 
 from tests import layered_util as U
@@ -19,3 +21,37 @@ def test_rows_in_32_bits(ctx, tmp_path, width, ff, taps):
     K = U.Case(ctx, tmp_path, stack(width, ff, taps))
     t = K.tokens(9)
     assert U.err(K.got(t, range(1, 9)), K.want(t)) < U.F32
+
+
+def steps(K, rows, n=7):
+    """logits of n steps of single tokens (the second is captured, the others replay it), other work between them"""
+    seqs, out = [K.lm.seq_open() for _ in range(rows)], []
+    toks = [K.tokens(n, seed=r) for r in range(rows)]
+    for i in range(n):
+        out.append(K.lm.step([(s, t[i:i + 1], [0]) for s, t in zip(seqs, toks)]))
+        if i % 2:
+            K.got(toks[0][:5])
+    for s in seqs:
+        K.lm.seq_close(s)
+    return np.array(out)
+
+
+# the same sums in the same order as two launches: the same bits.  Rounds of 16 k tiles a wave: less than one, one, more; odd numbers of feature tiles
+@pytest.mark.parametrize("rows", [1, 3, 8])
+@pytest.mark.parametrize("width", [36, 1100, 2048])
+@pytest.mark.parametrize("design", ["ranutar", "timerax"])
+def test_rows_beside_their_product(ctx, tmp_path, design, width, rows):
+    c = stack(width, 136) if design == "ranutar" else U.mixed(width)
+    a, b = (U.Case(ctx, tmp_path / str(i), c, dtype="bfloat16", options=f"enter_ahead={i}") for i in (1, 0))
+    x, y = steps(a, rows), steps(b, rows)
+    assert a.lm.info("enter_launches") > 0 and b.lm.info("enter_launches") == 0
+    assert np.isfinite(x).all() and np.array_equal(x, y)
+
+
+def test_a_wait_without_end_is_an_error(ctx, tmp_path):
+    import dsk
+    K = U.Case(ctx, tmp_path, stack(2048, 136), dtype="bfloat16", options="enter_spins=0")
+    s = K.lm.seq_open()
+    with pytest.raises(dsk.DskError, match="gave up"):
+        for t in K.tokens(4):
+            K.lm.step([(s, [t], [0])])
