@@ -4,6 +4,8 @@
 
 #include <rccl/rccl.h>
 
+#include <atomic>
+
 // Where a tensor's bytes come from: host memory (dsk_model_bind) or a byte range of an open file (the .dseek
 // loader, loader.cpp).  Either way they travel through the context's pinned staging ring (context.cpp stage_copy).
 struct HostSrc {
@@ -36,6 +38,30 @@ struct dsk_ctx {
 void ctx_model_released(dsk_ctx* c);
 int stage_copy(dsk_ctx* ctx, const HostSrc& src, uint64_t src_off, void* dev_dst, size_t bytes);
 
+// ---- pinned rows that callers borrow (dsk_rows_lend) ----------------------------------------------
+// Slots at the end of an allocation that a model makes and uses; it is freed when the model and every borrower have let go of it.
+struct RowPool;
+struct dsk_rows {
+  RowPool* pool;
+  unsigned slot;
+};
+struct RowPool {
+  enum { SLOTS = 4 };
+  char* mem;          // hipHostMalloc
+  float* lent;        // slot i: lent + i * slot_floats
+  size_t slot_floats;
+  std::atomic<unsigned> taken{0};
+  std::atomic<int> owners{1};
+  dsk_rows slots[SLOTS];
+  RowPool(void* m, float* first, size_t floats) : mem((char*)m), lent(first), slot_floats(floats) {
+    for (unsigned i = 0; i < SLOTS; ++i) slots[i] = {this, i};
+  }
+  dsk_rows* lend();   // nullptr: none left
+  void let_go();      // one owner less
+  float* rows(const dsk_rows* r) const { return lent + r->slot * slot_floats; }
+  bool holds(const float* p, size_t n) const { return p >= lent && p + n <= lent + SLOTS * slot_floats; }
+};
+
 // ---- model families -------------------------------------------------------------------------------
 // A dsk_model handle is one of several concrete types; all of them start with a ModelHead, whose table carries the calls
 // every family answers (registry.cpp dispatches them).  Calls that exist for one family only check the table (family_is).
@@ -61,6 +87,7 @@ struct Family {
   int (*seq_pos)(dsk_model*, int32_t seq, int32_t* pos);
   int (*step)(dsk_model*, const dsk_step_entry* entries, int n, float* logits);
   int (*step_sample)(dsk_model*, const dsk_step_entry* entries, int n, float temperature, float top_p, const float* coins, int32_t* next);
+  int (*rows_lend)(dsk_model*, int n_rows, float** rows, dsk_rows** hold);  // nullptr: lends none
 };
 struct ModelHead {
   const Family* family = nullptr;

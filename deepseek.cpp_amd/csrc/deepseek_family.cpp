@@ -64,7 +64,7 @@ static int ds_step_sample(dsk_model* m, const dsk_step_entry* e, int n, float te
 
 Family deepseek_family = {  // (not const: a const table of host functions would be emitted for the device too)
     "deepseek",       ds_destroy,  ds_vocab_size, ds_forward,     ds_hydrate,  ds_forward_argmax, ds_forward_sample, ds_forward_prob, ds_host_logits, ds_set_graph,
-    ds_set_trace,     ds_get_trace_x, ds_trace_row, ds_get_info, ds_active_bytes, ds_device_bytes, ds_seq_open, ds_seq_close,     ds_seq_pos,      ds_step,        ds_step_sample};
+    ds_set_trace,     ds_get_trace_x, ds_trace_row, ds_get_info, ds_active_bytes, ds_device_bytes, ds_seq_open, ds_seq_close,     ds_seq_pos,      ds_step,        ds_step_sample, nullptr};
 
 static bool ds_claims(const char* arch) { return !strncmp(arch, "Deepseek", 8); }
 static int ds_open(dsk_ctx* ctx, const char* dir, int dtype, const char* options, dsk_model** out) {

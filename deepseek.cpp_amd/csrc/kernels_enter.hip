@@ -42,7 +42,7 @@ __global__ __launch_bounds__(ENTER_NT) void enter_kernel(const uint16_t* __restr
     JoinLds<NT> join;
     float sums[NT * 4];
   } lds;
-  const LinArgs& a = e.a;
+  LinArgs a = e.a;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int makers = KIND ? rows * ENTER_SPLIT : rows;
   if ((int)blockIdx.x < makers) {
@@ -62,6 +62,7 @@ __global__ __launch_bounds__(ENTER_NT) void enter_kernel(const uint16_t* __restr
 #pragma unroll
   for (int u = 0; u < U; ++u) w[u] = load(u);
   __builtin_amdgcn_sched_barrier(0);
+  if (a.out_at) a.out_f = glob(*glob(a.out_at));
   if (wave == 0) {
     const unsigned tag = *tag_at + e.s.launch;
     unsigned spins = 0;

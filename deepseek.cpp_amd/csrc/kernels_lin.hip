@@ -651,6 +651,7 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
   LinArgs a = f.t[i];
   if (i > 0) b -= f.wg_end[i - 1];
   const int row = min(c, a.rows - 1), part = b / f.groups[i], per = part_tiles(a);
+  if (a.out_at) a.out_f = glob(*glob(a.out_at));
   a.out_f += part * a.part_stride;
   few_body<T, NT, false>(a, b % f.groups[i] * NT, part * per, min(a.kt, part * per + per), a.row_seq ? a.seqs[a.row_seq[row]].row0 : row, c < a.rows ? c : -1, lds);
 }
@@ -660,6 +661,7 @@ static int lin_lds(bool f32) { return lin_stages(f32 ? 4 : 2) * lin_stage(f32 ? 
 static int check_lin(const LinArgs& a, const char* what) {
   if (!a.w || !a.a_t || a.rows < 1 || a.kt < 2 || (a.kt & 1) || a.rt < 1 || a.lda < a.kt * 32) DSK_FAIL(DSK_ERR_INVALID, "%s: rows %d kt %d rt %d lda %d", what, a.rows, a.kt, a.rt, a.lda);
   if (a.parts > 1 && (a.n_wide || a.epi != LIN_STORE || part_tiles(a) * (a.parts - 1) >= a.kt)) DSK_FAIL(DSK_ERR_INVALID, "%s: %d parts of %d", what, a.parts, a.kt);
+  if (a.out_at && a.parts > 1) DSK_FAIL(DSK_ERR_INVALID, "%s: %d parts of an output that moves", what, a.parts);
   if (a.a_seg < 0 || (a.a_seg & 15) || (a.a_seg && a.a_ops < 1)) DSK_FAIL(DSK_ERR_INVALID, "%s: %d features per operand", what, a.a_seg);
   return DSK_OK;
 }
@@ -699,7 +701,7 @@ int lin_parts_few(int rt, int kt, int most) {
 }
 int launch_lin(hipStream_t st, const LinArgs& a, bool f32) {
   DSK_TRY(check_lin(a, "lin"));
-  if ((a.a_seg & 127) || a.row_seq) DSK_FAIL(DSK_ERR_INVALID, "lin: %d features per operand", a.a_seg);
+  if ((a.a_seg & 127) || a.row_seq || a.out_at) DSK_FAIL(DSK_ERR_INVALID, "lin: %d features per operand", a.a_seg);
   if (lin_big(a, std::max(a.parts, 1), f32)) {
     const int row_tiles = cdiv(a.rows, 256), tiles = row_tiles * cdiv(a.rt, 16);
     DSK_TRY(allow_lds(lin_big_kernel, RING * 32 * 1024));

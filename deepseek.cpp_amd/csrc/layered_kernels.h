@@ -63,6 +63,7 @@ struct LinArgs {
   int direct;             // launch_lin in 32 bits: activations whole on the 32-bit matrix instruction (few k tiles; one part)
   const int* row_seq;     // launch_lin_few: output row i reads the first row of sequence row_seq[i] of seqs (nullptr: row i)
   const SeqDesc* seqs;
+  float* const* out_at;   // launch_lin_few, launch_enter: the 32-bit output is where this says (device memory; one part), nullptr: at out_f
 };
 // parts worth splitting k into, at most `most`: launch_lin, launch_lin_few
 int lin_parts(int rows, int rt, int kt, bool f32, int most);

@@ -77,7 +77,7 @@ struct Seq {
 struct DescBuf {
   char *host = nullptr, *dev = nullptr;
   int cap = 0;
-  size_t o_tok = 0, o_row = 0, o_want = 0, o_tile = 0, o_chunk = 0, o_single = 0, o_tag = 0, bytes = 0;
+  size_t o_tok = 0, o_row = 0, o_want = 0, o_tile = 0, o_chunk = 0, o_single = 0, o_tag = 0, o_to = 0, bytes = 0;
 };
 
 struct Graph {
@@ -119,7 +119,9 @@ struct LayeredModel : ModelHead {
   float *weight = nullptr, *logits = nullptr, *trace_x = nullptr, *sample_scratch = nullptr;
   int *slot_pos = nullptr, *chosen = nullptr, *count = nullptr, *cursor = nullptr, *slot_row = nullptr, *tiles = nullptr, *n_tiles = nullptr, *active = nullptr,
       *active_slot = nullptr, *n_active = nullptr, *next_dev = nullptr;
-  float* logits_host = nullptr;     // pinned, LOGIT_ROWS rows
+  float* logits_host = nullptr;     // pinned, LOGIT_ROWS rows, the upper half of them for borrowers
+  RowPool* pool = nullptr;          // owns them
+  float* logits_to = nullptr;       // where this pass's logits go if the product stores them: logits_host or borrowed rows
   int* next_host = nullptr;         // pinned
   StepParams *sp_host = nullptr, *sp_dev = nullptr;
   DescBuf big, small;
@@ -506,6 +508,7 @@ int alloc_desc(LayeredModel* m, DescBuf* d, int cap) {
   d->o_chunk = take(2 * (size_t)cap);
   d->o_single = take(cap);
   d->o_tag = take(1);
+  d->o_to = take(2);
   d->bytes = off;
   HIP_TRY(hipHostMalloc((void**)&d->host, off, hipHostMallocDefault));
   memset(d->host, 0, off);
@@ -662,6 +665,9 @@ int alloc_work(LayeredModel* m) {
   HIP_TRY(hipHostMalloc((void**)&m->sp_host, sizeof(StepParams) * FEW, hipHostMallocDefault));
   memset(m->sp_host, 0, sizeof(StepParams) * FEW);
   HIP_TRY(hipHostMalloc((void**)&m->logits_host, (size_t)LOGIT_ROWS * s.vocab * 4, hipHostMallocDefault));
+  static_assert(LOGIT_ROWS >= 2 * RowPool::SLOTS * FEW, "half of the rows stay the model's");
+  m->pool = new RowPool(m->logits_host, m->logits_host + (size_t)(LOGIT_ROWS - RowPool::SLOTS * FEW) * s.vocab, (size_t)FEW * s.vocab);
+  m->logits_to = m->logits_host;
   HIP_TRY(hipHostMalloc((void**)&m->next_host, LOGIT_ROWS * 4, hipHostMallocDefault));
   HIP_TRY(hipHostMalloc((void**)&m->gave_up, 4, hipHostMallocDefault));
   *m->gave_up = 0;
@@ -1166,14 +1172,16 @@ int run_layer(LayeredModel* m, const PassDesc& p, int l, bool few) {
 }
 
 // Logits of up to FEW rows that only the caller reads are stored into pinned host memory by the product itself: the bytes travel while the weights
-// are still streaming, and no copy follows the last kernel.  (Whole tiles of 16 features: a row of host memory has no padding.)  Into fresh buffers
-// of the caller's, us a step copied / stored / stored and make_pages below: 4 rows of 129280 1840 / 1645 / 1280, 16 rows 6490 / 6180 / 5510, one row
-// 1358 / 1246 / 1186, 8 rows of 102400 5050 / 4800 / 4250, one row 2230 / 2140 / 2093.  The product takes as long as before.
+// are still streaming, and no copy by the device follows the last kernel.  (Whole tiles of 16 features: a row of host memory has no padding.)  Into rows that the
+// caller has borrowed (dsk_rows_lend) that is all; other buffers get a copy.  us a step, a fresh buffer / borrowed rows, one row of 102400 1812 / 1785, four of
+// 129280 1286 / 1178, sixteen 5735 / 5150.  (Copying groups of features while the product runs: its waves have to wait until their stores have arrived, and the head
+// took 342 us instead of 306 with four rows, 110 instead of 70 with one.)
 bool straight_to_host(const LayeredModel* m, int n, int mode) { return mode == OUT_LOGITS && n <= FEW && m->s.vocab % 16 == 0; }
 // the product for the logits of hw rows [r0, r0 + n), into m->logits or straight_to_host
-LinArgs head_lin(LayeredModel* m, int r0, int n, int mode) {
+LinArgs head_lin(LayeredModel* m, int r0, int n, int mode, bool few) {
   const bool host = straight_to_host(m, n, mode);
-  LinArgs a = lin_f(m->head, m->hw + (size_t)r0 * m->h_ld * m->elem(), m->h_ld, n, host ? m->logits_host : m->logits, host ? m->s.vocab : m->ld_logits);
+  LinArgs a = lin_f(m->head, m->hw + (size_t)r0 * m->h_ld * m->elem(), m->h_ld, n, host ? m->logits_to : m->logits, host ? m->s.vocab : m->ld_logits);
+  if (host && few) a.out_at = reinterpret_cast<float* const*>(m->small.dev + m->small.o_to);  // (a captured launch: the place is the pass's)
   if (m->s.softcap > 0) {
     a.epi = LIN_SOFTCAP;
     a.p0 = (float)m->s.softcap;
@@ -1184,7 +1192,7 @@ LinArgs head_lin(LayeredModel* m, int r0, int n, int mode) {
   return a;
 }
 int run_head(LayeredModel* m, int r0, int n, int mode) {
-  const LinArgs a = head_lin(m, r0, n, mode);
+  const LinArgs a = head_lin(m, r0, n, mode, false);
   return run_lin(m, &a, 1, n <= FEW);
 }
 int fetch_logits(LayeredModel* m, int n, int mode) {  // behind run_head: n rows into m->logits_host
@@ -1198,6 +1206,14 @@ void make_pages(float* out, size_t n) {
   volatile float* p = out;
   for (size_t i = 0; i < n; i += 1024) p[i] = p[i];
   if (n) p[n - 1] = p[n - 1];
+}
+// n rows of logits to the caller, and the end of what makes them
+int take_logits(LayeredModel* m, float* out, int n, int mode) {
+  const bool there = straight_to_host(m, n, mode) ? out == m->logits_to : out == m->logits_host;
+  if (!there) make_pages(out, (size_t)n * m->s.vocab);
+  HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+  if (!there) memcpy(out, m->logits_host, (size_t)n * m->s.vocab * 4);
+  return DSK_OK;
 }
 int run_choice(LayeredModel* m, int n, int mode) {  // the next token of every row of m->logits
   hipStream_t st = m->ctx->stream;
@@ -1249,7 +1265,7 @@ int run_body(LayeredModel* m, const DescBuf& d, const PassDesc& p, bool few, int
   j.h_t = m->hw;
   j.only_want = 1;
   if (!few) return launch_join(st, j, m->f32);
-  return sum_and_lin(m, j, head_lin(m, 0, p.n_want, mode), true, [&]() { return launch_join(st, j, m->f32); });
+  return sum_and_lin(m, j, head_lin(m, 0, p.n_want, mode, true), true, [&]() { return launch_join(st, j, m->f32); });
 }
 int run_few(LayeredModel* m, const PassDesc& p, int mode) {
   DSK_TRY(run_body(m, m->small, p, true, mode));
@@ -1320,6 +1336,8 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
       m->enter_tag = 1;
     }
     *reinterpret_cast<unsigned*>(d.host + d.o_tag) = m->enter_tag;
+    m->logits_to = nw && mode == OUT_LOGITS && m->pool->holds(out, (size_t)nw * m->s.vocab) ? out : m->logits_host;
+    *reinterpret_cast<float**>(d.host + d.o_to) = m->logits_to;
     m->enter_tag += launches;
     if (mode == OUT_SAMPLE) {  // (sp_host's temperature and top_p were set by the caller)
       for (int i = 0; i < nw; ++i) m->sp_host[i].coin = coins[i];
@@ -1354,30 +1372,25 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
       HIP_TRY(hipGraphLaunch(g.exec, st));
       m->graph_steps++;
     }
-    if (mode == OUT_LOGITS && out != m->logits_host) make_pages(out, (size_t)nw * m->s.vocab);
-    HIP_TRY(hipStreamSynchronize(st));
+    if (nw && mode == OUT_LOGITS) DSK_TRY(take_logits(m, out, nw, mode));
+    else HIP_TRY(hipStreamSynchronize(st));
     if (*m->gave_up) {
       *m->gave_up = 0;
       DSK_FAIL(DSK_ERR_STATE, "step: a launch gave up waiting for its rows; the step's sequences have no valid state (option enter_ahead=0 does without the wait)");
     }
-    if (nw && mode == OUT_LOGITS) {
-      if (out != m->logits_host) memcpy(out, m->logits_host, (size_t)nw * m->s.vocab * 4);
-    } else if (nw) {
-      memcpy(next, m->next_host, (size_t)nw * 4);
-    }
+    if (nw && mode != OUT_LOGITS) memcpy(next, m->next_host, (size_t)nw * 4);
   } else {
     m->splits = 1 << 30;  // (a mixer takes as many as its largest window has)
     DSK_TRY(run_body(m, d, p, false, mode));
-    const int block = mode == OUT_LOGITS ? LOGIT_ROWS : FEW;
+    const int block = mode != OUT_LOGITS ? FEW : m->pool->taken.load() ? LOGIT_ROWS - RowPool::SLOTS * FEW : LOGIT_ROWS;
     for (int i = 0; i < nw; i += block) {
       const int n = std::min(block, nw - i);
+      float* to = mode == OUT_LOGITS ? out + (size_t)i * m->s.vocab : nullptr;
+      m->logits_to = to && m->pool->holds(to, (size_t)n * m->s.vocab) ? to : m->logits_host;
       DSK_TRY(run_head(m, i, n, mode));
       if (mode == OUT_LOGITS) {
         DSK_TRY(fetch_logits(m, n, mode));
-        float* to = out + (size_t)i * m->s.vocab;
-        if (to != m->logits_host) make_pages(to, (size_t)n * m->s.vocab);
-        HIP_TRY(hipStreamSynchronize(st));
-        if (to != m->logits_host) memcpy(to, m->logits_host, (size_t)n * m->s.vocab * 4);
+        DSK_TRY(take_logits(m, to, n, mode));
       } else {
         if (mode == OUT_SAMPLE)
           for (int k = 0; k < n; ++k) m->sp_host[k].coin = coins[i + k];
@@ -1460,8 +1473,10 @@ int l_destroy(dsk_model* h) {
     if (g.second.exec) hipGraphExecDestroy(g.second.exec);
   for (void* p : m->dev) hipFree(p);
   for (void* p : m->slabs) hipFree(p);
-  for (void* p : {(void*)m->sp_host, (void*)m->logits_host, (void*)m->next_host, (void*)m->gave_up, (void*)m->big.host, (void*)m->small.host})
+  for (void* p : {(void*)m->sp_host, (void*)m->next_host, (void*)m->gave_up, (void*)m->big.host, (void*)m->small.host})
     if (p) hipHostFree(p);
+  if (m->pool) m->pool->let_go();
+  else if (m->logits_host) hipHostFree(m->logits_host);
   dsk_ctx* ctx = m->ctx;
   delete m;
   ctx_model_released(ctx);
@@ -1508,6 +1523,13 @@ int l_seq_pos(dsk_model* h, int32_t s, int32_t* pos) {
   return DSK_OK;
 }
 int l_step(dsk_model* h, const dsk_step_entry* e, int n, float* logits) { return run_step(lm(h), e, n, OUT_LOGITS, logits, nullptr, nullptr); }
+int l_rows_lend(dsk_model* h, int n_rows, float** rows, dsk_rows** hold) {
+  LayeredModel* m = lm(h);
+  if (!straight_to_host(m, n_rows, OUT_LOGITS)) return DSK_OK;
+  if (!(*hold = m->pool->lend())) return DSK_OK;
+  *rows = m->pool->rows(*hold);
+  return DSK_OK;
+}
 int l_step_sample(dsk_model* h, const dsk_step_entry* e, int n, float temperature, float top_p, const float* coins, int32_t* next) {
   LayeredModel* m = lm(h);
   for (int i = 0; i < FEW; ++i) {
@@ -1638,7 +1660,7 @@ double l_active_bytes(const dsk_model* h, int pos) {
 double l_device_bytes(const dsk_model* h) { return lm(h)->weight_bytes + lm(h)->scratch_bytes + lm(h)->cache_bytes; }
 
 const Family layered_family = {"layered",     l_destroy,    l_vocab,       l_forward,      l_hydrate,      l_forward_argmax, l_forward_sample, l_forward_prob, l_host_logits, l_set_graph, l_set_trace,
-                               l_get_trace_x, l_trace_row,  l_get_info,    l_active_bytes, l_device_bytes, l_seq_open,       l_seq_close,      l_seq_pos,      l_step,        l_step_sample};
+                               l_get_trace_x, l_trace_row,  l_get_info,    l_active_bytes, l_device_bytes, l_seq_open,       l_seq_close,      l_seq_pos,      l_step,        l_step_sample,    l_rows_lend};
 
 // ---- opening -------------------------------------------------------------------------------------------------
 int set_options(LayeredModel* m, const char* options) {

@@ -154,6 +154,36 @@ extern "C" int dsk_step(dsk_model* m, const dsk_step_entry* entries, int n, floa
     if (entries[i].n_want > 0 && !logits) DSK_FAIL(DSK_ERR_INVALID, "step: logits are asked for and there is no buffer");
   return F.step(m, entries, n, logits);
 }
+extern "C" int dsk_rows_lend(dsk_model* m, int n_rows, float** rows, dsk_rows** hold) {
+  FAMILY(m, "rows_lend");
+  if (!rows || !hold || n_rows < 1) DSK_FAIL(DSK_ERR_INVALID, "rows_lend: bad argument");
+  *rows = nullptr;
+  *hold = nullptr;
+  return F.rows_lend ? F.rows_lend(m, n_rows, rows, hold) : DSK_OK;
+}
+extern "C" void dsk_rows_return(dsk_rows* hold) {
+  if (!hold) return;
+  RowPool* p = hold->pool;
+  p->taken.fetch_and(~(1u << hold->slot), std::memory_order_release);
+  p->let_go();
+}
+dsk_rows* RowPool::lend() {
+  unsigned t = taken.load(std::memory_order_relaxed);
+  for (;;) {
+    unsigned i = 0;
+    while (i < SLOTS && (t >> i & 1)) ++i;
+    if (i == SLOTS) return nullptr;
+    if (taken.compare_exchange_weak(t, t | 1u << i, std::memory_order_acquire)) {
+      owners.fetch_add(1, std::memory_order_relaxed);
+      return &slots[i];
+    }
+  }
+}
+void RowPool::let_go() {
+  if (owners.fetch_sub(1, std::memory_order_acq_rel) > 1) return;
+  hipHostFree(mem);
+  delete this;
+}
 extern "C" int dsk_step_sample(dsk_model* m, const dsk_step_entry* entries, int n, float temperature, float top_p, const float* coins, int32_t* next) {
   FAMILY(m, "step_sample");
   if (!next || (temperature != 0.0f && !coins)) DSK_FAIL(DSK_ERR_INVALID, "step_sample: null argument");

@@ -180,6 +180,9 @@ def lib():
         L.dsk_seq_close.argtypes = [C.c_void_p, C.c_int32]
         L.dsk_seq_pos.argtypes = [C.c_void_p, C.c_int32, c_i32]
         L.dsk_step.argtypes = [C.c_void_p, c_step, C.c_int, c_f]
+        L.dsk_rows_lend.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p)]
+        L.dsk_rows_return.argtypes = [C.c_void_p]
+        L.dsk_rows_return.restype = None
         L.dsk_step_sample.argtypes = [C.c_void_p, c_step, C.c_int, C.c_float, C.c_float, c_f, c_i32]
         L.dsk_generate.argtypes = [C.c_void_p, C.POINTER(GenRequest), C.c_int, C.c_int, C.c_float, C.c_float]
         L.dsk_hydrate_get_trace_x.argtypes = [C.c_void_p, C.c_int, C.c_int, c_f]
@@ -588,6 +591,17 @@ def build_for(dirname: str) -> None:
     subprocess.check_call(["make", "-s", "-j8", "-C", os.path.join(HERE, "csrc"), "layered" if layered else "all"], stdout=2)
 
 
+class Rows:
+    """borrowed rows of logits: given back when the last array over them is gone"""
+
+    def __init__(self, at, hold, shape):
+        self.__array_interface__ = {"shape": shape, "typestr": "<f4", "data": (at, False), "version": 3}
+        self._hold, self._give_back = hold, lib().dsk_rows_return
+
+    def __del__(self):
+        self._give_back(self._hold)
+
+
 class LM:
     """A model opened by what its directory says it is (dsk_model_open): sequences, batched steps, generation."""
 
@@ -626,10 +640,17 @@ class LM:
             arr[i] = StepEntry(e[0], toks.size, toks.ctypes.data_as(c_i32), want.size, want.ctypes.data_as(c_i32))
         return arr, keep
 
+    def _rows(self, n):
+        """[n, vocab] float32 for logits: rows that the device writes (dsk_rows_lend) as long as the model has some left, else an ordinary array"""
+        rows, hold = C.c_void_p(), C.c_void_p()
+        if n:
+            check(lib().dsk_rows_lend(self.h, n, C.byref(rows), C.byref(hold)))
+        return np.asarray(Rows(rows.value, hold.value, (n, self.vocab))) if hold.value else np.empty((n, self.vocab), np.float32)
+
     def step(self, entries):
         """entries: (sequence, tokens, wanted places); returns [wanted, vocab] float32, in the order of the entries"""
         arr, keep = self._entries(entries)
-        out = np.zeros((sum(arr[i].n_want for i in range(len(entries))), self.vocab), np.float32)
+        out = self._rows(sum(arr[i].n_want for i in range(len(entries))))
         check(lib().dsk_step(self.h, arr, len(entries), _f(out)))
         return out
 

@@ -479,6 +479,12 @@ typedef struct dsk_step_entry {
   const int32_t* want;
 } dsk_step_entry;
 int dsk_step(dsk_model* m, const dsk_step_entry* entries, int n, float* logits);
+/* Room for the logits of n_rows tokens that the device writes itself: passed to dsk_step (or any call that takes host_logits), no copy follows.  A model
+ * lends a few of them; *rows is NULL when none is left (or it has none that large, or does not lend) and an ordinary buffer is to be used.  The rows
+ * stay the borrower's until dsk_rows_return, which any thread may call, also behind dsk_model_destroy. */
+typedef struct dsk_rows dsk_rows;
+int dsk_rows_lend(dsk_model* m, int n_rows, float** rows, dsk_rows** hold);
+void dsk_rows_return(dsk_rows* hold);
 /* ... the next token of every entry instead, chosen on the device from its last token's logits the way dsk_forward_sample
  * does (temperature 0: the first largest logit); coins[i] in [0, 1] is entry i's random draw; want[] is ignored. */
 int dsk_step_sample(dsk_model* m, const dsk_step_entry* entries, int n, float temperature, float top_p, const float* coins, int32_t* next);
