@@ -303,7 +303,7 @@ int launch_repack_q2k_tiles(hipStream_t st, const uint8_t* aos, size_t gb0, size
 int launch_planes_to_tiles_q2k(hipStream_t st, const uint8_t* qs, const uint8_t* sc, const uint8_t* dm, size_t gb0, size_t n_blocks, int rows, int nb,
                                size_t e_bytes, uint8_t* tiles);
 int launch_repack_q3k(hipStream_t st, const uint8_t* aos, size_t n_blocks, uint8_t* qs, uint8_t* hm, uint8_t* sc, uint8_t* dm);
-int launch_embed(hipStream_t st, const DTensor& t, const StepParams* sp, int token_override, int b0, int b1, float* x);
+int launch_embed(hipStream_t st, const DTensor& t, const StepParams* sp, StepParams* sp_dev, int token_override, int b0, int b1, float* x);  // sp_dev: takes a copy of *sp
 int launch_embed_rows(hipStream_t st, const DTensor& t, const StepParams* sps, int P, int b0, int b1, float* x);  // P rows, tokens from the step rows
 struct RouterArgs {       // F32 router GEMV (+ optional rmsnorm prologue) + moe_gate in the last workgroup
   const float* w;         // (E, dim)

@@ -106,7 +106,7 @@ struct dsk_model : ModelHead {
   unsigned long long* moe_timeline = nullptr;  // base of [8 kinds][1024 workgroups][8]
   unsigned long long* timeline_of(int kind) const { return moe_timeline ? moe_timeline + (size_t)kind * DSK_TL_WGS * 8 : nullptr; }
   unsigned* err_host = nullptr;    // pinned, device-visible: bounded spins report here
-  int lp_head = -1;
+  int lp_head = -1, lp_head_host = -1;
   // batched prompt ingestion (hydrate.cpp): buffers allocated by the first dsk_hydrate call that takes the batched path
   struct HydState* hyd = nullptr;
   int hydrate_chunk = 512;          // option "hydrate_chunk": tokens per batched chunk (every weight matrix is read once per chunk: a 512-token prompt

@@ -157,7 +157,7 @@ extern "C" int dsk_embed_row(dsk_ctx* ctx, int quant, const void* w, size_t w_by
     HIP_TRY(hipMemcpyAsync(tg.t.scale, scale, (size_t)cdiv(vocab, b0) * cdiv(dim, b1) * 4, hipMemcpyHostToDevice, st));
   DevBuf dout;
   DSK_TRY(dout.alloc((size_t)dim * 4));
-  DSK_TRY(launch_embed(st, tg.t, nullptr, token, b0, b1, dout.as<float>()));
+  DSK_TRY(launch_embed(st, tg.t, nullptr, nullptr, token, b0, b1, dout.as<float>()));
   HIP_TRY(hipMemcpyAsync(out, dout.p, (size_t)dim * 4, hipMemcpyDeviceToHost, st));
   return finish(ctx);
 }
