@@ -80,6 +80,7 @@ __host__ DEV constexpr int lin_step(int size) { return size == 2 ? 2 : 1; }
 __host__ DEV constexpr int lin_stage(int size) { return lin_step(size) * 8 * 1024 * (1 + size / 2); }
 // 32 features (tiles rt, rt + 1) x 32 rows (from `first` on) of a wave by itself on v_mfma_f32_16x16x4_f32, operands straight from memory: one chain of
 // the instruction per sum.  f0: a feature whose operand it is.
+template <int EPI>
 DEV void direct_tile(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int rt, int first, int k0, int k1) {
   const int lane = threadIdx.x & 63;
   const bf16x8* w[2];
@@ -119,17 +120,17 @@ DEV void direct_tile(const LinArgs& a, const int* gather, int row0, int n_rows, 
   for (int j = 0; j < 2; ++j) {
     const int r = first + j * 16 + (lane & 15);
     if (r >= n_rows || rt >= a.rt) continue;
-    if (a.epi == LIN_GLU) {
+    if constexpr (EPI == LIN_GLU) {
       store_glu<float>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[0][j], acc[1][j]);
     } else {
-      store_plain<float>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[0][j]);
-      if (rt + 1 < a.rt) store_plain<float>(a, row0 + r, rt * 16 + 16 + (lane >> 4) * 4, acc[1][j]);
+      store_plain<float, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[0][j]);
+      if (rt + 1 < a.rt) store_plain<float, EPI>(a, row0 + r, rt * 16 + 16 + (lane >> 4) * 4, acc[1][j]);
     }
   }
 }
 // 128 features from f0 on x n_rows <= 128 rows, k tiles [k0, k1): 4 waves of 64 x 64.  gather: a table (slot -> row) or nullptr; out rows are
 // row0 + local row.
-template <typename T>
+template <typename T, int EPI>
 DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
   typedef typename Frag<T>::type frag;
   constexpr int AB = 64 * (int)sizeof(frag);  // bytes of an A fragment
@@ -265,7 +266,7 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
         for (int e = 0; e < 4; ++e) bad = fmaf(acc[i][j][e], 0.f, bad);
     if (__any(bad != bad)) {
 #pragma unroll 1
-      for (int i = 0; i < 4; ++i) direct_tile(a, gather, row0, n_rows, f0, rt0 + wm * 4 + (i & 1) * 2, wn * 64 + (i >> 1) * 32, k0, k1);
+      for (int i = 0; i < 4; ++i) direct_tile<EPI>(a, gather, row0, n_rows, f0, rt0 + wm * 4 + (i & 1) * 2, wn * 64 + (i >> 1) * 32, k0, k1);
       return;
     }
   }
@@ -277,10 +278,10 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
     for (int i = 0; i < 4; ++i) {
       const int rt = rt0 + wm * 4 + i;
       if (rt >= a.rt) continue;
-      if (a.epi == LIN_GLU) {
+      if constexpr (EPI == LIN_GLU) {
         if (!(i & 1)) store_glu<T>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[i][j], acc[i | 1][j]);
       } else {
-        store_plain<T>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+        store_plain<T, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
       }
     }
   }
@@ -295,7 +296,7 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
 // For plain products, whose row tiles are full, it is within 3 % of lin_kernel either way, and lin_big_kernel has more work per byte.
 template <int NJ>
 __host__ DEV constexpr int wide_stage() { return 2 * NJ * 1024; }
-template <int NJ>
+template <int NJ, int EPI>
 DEV void wide_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
   constexpr int STAGE = wide_stage<NJ>(), AL = NJ / 2;  // AL: this wave's loads of rows in a step
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = k1 - k0;
@@ -367,20 +368,20 @@ DEV void wide_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
     for (int i = 0; i < 4; ++i) {
       const int rt = rt0 + i;
       if (rt >= a.rt) continue;
-      if (a.epi == LIN_GLU) {
+      if constexpr (EPI == LIN_GLU) {
         if (!(i & 1)) store_glu<bf16>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[i][j], acc[i | 1][j]);
       } else {
-        store_plain<bf16>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+        store_plain<bf16, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
       }
     }
   }
 }
-template <typename T>
+template <typename T, int EPI>
 __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 128, per = part_tiles(a), k0 = blockIdx.y * per;
   a.out_f += blockIdx.y * a.part_stride;
-  lin_body<T>(a, nullptr, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
+  lin_body<T, EPI>(a, nullptr, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
 }
 
 // LinArgs.direct: products of a few k tiles (the decay of time mixing: two), 64 features x 64 rows per workgroup.  Three pieces have nothing to save
@@ -389,12 +390,13 @@ __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_ti
 // few_body: in bfloat16 runs another rounding of the decay turns roundings behind it.
 __global__ __launch_bounds__(256) void lin_direct_kernel(const LinArgs a, const int row_tiles, const int tiles) {
   const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 64, f0 = b / row_tiles * 64, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  direct_tile(a, nullptr, row0, min(64, a.rows - row0), f0, (f0 >> 4) + (wave & 1) * 2, (wave >> 1) * 32, 0, a.kt);
+  direct_tile<LIN_STORE>(a, nullptr, row0, min(64, a.rows - row0), f0, (f0 >> 4) + (wave & 1) * 2, (wave >> 1) * 32, 0, a.kt);
 }
 
 // 256 features x 256 rows per workgroup: 8 waves of 128 x 64; twice the matrix work per byte staged.  A ring of RING stages of one k tile
 // (32 KiB): while a tile is multiplied the next one's operands are read into the other set of registers, and RING - 1 more are on their way.
 enum { RING = 4 };
+template <int EPI>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lin_big_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int STAGE = 32 * 1024;
@@ -464,14 +466,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     step(kt + 1, q, p);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int st0 = rt0 + wm * 8;
+  const bool pairs = wide_pairs(a) && (st0 + 8) * 16 <= a.n_wide && st0 + 8 <= a.rt;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r = wn * 64 + j * 16 + (lane & 15);
-    if (r >= n_rows) continue;
+    if (pairs) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int rt = rt0 + wm * 8 + i;
-      if (rt < a.rt) store_plain<bf16>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+      for (int i = 0; i < 8; i += 2) store_wide_pair<EPI == LIN_TANH_F ? LIN_STORE : EPI>(a, r < n_rows, row0 + r, st0 + i, acc[i][j], acc[i + 1][j]);
+    } else if (r < n_rows) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (st0 + i < a.rt) store_plain<bf16, EPI>(a, row0 + r, (st0 + i) * 16 + (lane >> 4) * 4, acc[i][j]);
     }
   }
 }
@@ -498,10 +504,10 @@ DEV void set_expert(LinArgs& a, const MoeArgs& m, const ExpertMat& e, int expert
 // grid.x: an upper bound of the tiles.  The routed experts' come first, in groups of four row tiles (mostly one expert's, they are sorted) and in a
 // group feature tile by feature tile, and an XCD takes a contiguous range: the workgroups that read one weight tile meet in one L2, and
 // the rows of a group stay in it.  The shared expert's tiles, the longest, start first.
-template <typename T>
-__global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs m, const int down, const int shared_tiles) {
+template <typename T, bool down>
+__global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs m, const int shared_tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  constexpr int FT = sizeof(T) == 2 ? 16 : 8;
+  constexpr int FT = sizeof(T) == 2 ? 16 : 8, EPI = down ? LIN_STORE : LIN_GLU;
   const ExpertMat& e = down ? m.down : m.up;
   const int row_tiles = *m.n_tiles - shared_tiles, ft = (e.rt + FT - 1) / FT, sft = (e.shared_rt + FT - 1) / FT;
   int b = blockIdx.x, tile, f;
@@ -524,11 +530,11 @@ __global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs
   const int* gather = down ? nullptr : m.slot_row;
   const int row0 = m.tiles[4 * tile + 1], rows = m.tiles[4 * tile + 2];
   if constexpr (sizeof(T) == 2) {
-    if (rows > 64) wide_body<8>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
-    else if (rows > 32) wide_body<4>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
-    else wide_body<2>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    if (rows > 64) wide_body<8, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    else if (rows > 32) wide_body<4, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    else wide_body<2, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
   } else {
-    lin_body<T>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
+    lin_body<T, EPI>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
   }
 }
 
@@ -699,24 +705,28 @@ int lin_parts_few(int rt, int kt, int most) {
   const int n = std::max(std::min({1024 / rt, kt / 16, most}), 1);
   return cdiv(kt, part_tiles(kt, n));
 }
+#define LIN_EPI(K, T) (a.epi == LIN_STORE ? K<T LIN_STORE> : a.epi == LIN_XIELU ? K<T LIN_XIELU> : a.epi == LIN_TANH_F ? K<T LIN_TANH_F> : K<T - 1>)
 int launch_lin(hipStream_t st, const LinArgs& a, bool f32) {
   DSK_TRY(check_lin(a, "lin"));
   if ((a.a_seg & 127) || a.row_seq || a.out_at) DSK_FAIL(DSK_ERR_INVALID, "lin: %d features per operand", a.a_seg);
   if (lin_big(a, std::max(a.parts, 1), f32)) {
     const int row_tiles = cdiv(a.rows, 256), tiles = row_tiles * cdiv(a.rt, 16);
-    DSK_TRY(allow_lds(lin_big_kernel, RING * 32 * 1024));
-    hipLaunchKernelGGL(lin_big_kernel, dim3(tiles, std::max(a.parts, 1)), dim3(512), RING * 32 * 1024, st, a, row_tiles, tiles);
+    auto k = LIN_EPI(lin_big_kernel, );
+    DSK_TRY(allow_lds(k, RING * 32 * 1024));
+    hipLaunchKernelGGL(k, dim3(tiles, std::max(a.parts, 1)), dim3(512), RING * 32 * 1024, st, a, row_tiles, tiles);
     return DSK_OK;
   }
   if (a.direct) {
-    if (!f32 || a.parts > 1) DSK_FAIL(DSK_ERR_INVALID, "lin: direct products are 32-bit ones in one part");
+    if (!f32 || a.parts > 1 || a.epi != LIN_STORE) DSK_FAIL(DSK_ERR_INVALID, "lin: direct products are 32-bit ones in one part, stored as they are");
     const int row_tiles = cdiv(a.rows, 64), tiles = row_tiles * cdiv(a.rt, 4);
     hipLaunchKernelGGL(lin_direct_kernel, dim3(tiles), dim3(256), 0, st, a, row_tiles, tiles);
     return DSK_OK;
   }
   const int row_tiles = cdiv(a.rows, 128), tiles = row_tiles * cdiv(a.rt, 8), lds = lin_lds(f32);
   const dim3 grid(tiles, std::max(a.parts, 1));
-  auto k = f32 ? lin_kernel<float> : lin_kernel<bf16>;
+#define LIN_F32 float,
+#define LIN_BF16 bf16,
+  auto k = f32 ? LIN_EPI(lin_kernel, LIN_F32) : LIN_EPI(lin_kernel, LIN_BF16);
   DSK_TRY(allow_lds(k, lds));
   hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, row_tiles, tiles);
   return DSK_OK;
@@ -726,13 +736,10 @@ int launch_experts(hipStream_t st, const MoeArgs& m, bool down, bool f32) {
   const ExpertMat& e = down ? m.down : m.up;
   const int shared_tiles = m.shared ? cdiv(m.rows, MOE_TILE) : 0, ft = f32 ? 8 : 16;
   const dim3 grid((m.max_tiles - shared_tiles) * cdiv(e.rt, ft) + ((shared_tiles * cdiv(e.shared_rt, ft) + 7) & ~7));
-  if (f32) {
-    const int lds = lin_lds(f32);
-    DSK_TRY(allow_lds(expert_kernel<float>, lds));
-    hipLaunchKernelGGL(expert_kernel<float>, grid, dim3(256), lds, st, a, m, (int)down, shared_tiles);
-  } else {
-    hipLaunchKernelGGL(expert_kernel<bf16>, grid, dim3(256), 2 * wide_stage<8>(), st, a, m, (int)down, shared_tiles);
-  }
+  const int lds = f32 ? lin_lds(f32) : 2 * wide_stage<8>();
+  auto k = f32 ? (down ? expert_kernel<float, true> : expert_kernel<float, false>) : (down ? expert_kernel<bf16, true> : expert_kernel<bf16, false>);
+  DSK_TRY(allow_lds(k, lds));
+  hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, m, shared_tiles);
   return DSK_OK;
 }
 // Four tiles per workgroup from 9 rows and 1536 tiles on, in bf16: a step of 16 sequences, us with one tile -> four, 8080 tiles 450 -> 320, 2328
