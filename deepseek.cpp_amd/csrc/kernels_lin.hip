@@ -395,37 +395,63 @@ __global__ __launch_bounds__(256) void lin_direct_kernel(const LinArgs a, const 
 
 // 256 features x 256 rows per workgroup: 8 waves of 128 x 64; twice the matrix work per byte staged.  A ring of RING stages of one k tile
 // (32 KiB): while a tile is multiplied the next one's operands are read into the other set of registers, and RING - 1 more are on their way.
+//
+// streams = 0: a workgroup per tile (and part of k).  Else the tiles of a row of them, k step by k step behind each other, are dealt out evenly to that
+// many workgroups, each of which works off one stretch without a stop between tiles: a product whose tiles do not fill the last round of compute units loses
+// none of them.  A tile that a stretch's end cuts (never in more than two pieces: streams <= feature tiles) is added up by whichever of the two workgroups
+// comes second; nobody waits.  The row tiles of one stretch are neighbours on one XCD and run in step, so that weights and rows meet in its L2.
 enum { RING = 4 };
+struct LinStream {
+  int streams;
+  float* sums;        // [streams][row tiles][2][256 x 256]: pieces in front of and behind the start of a stretch
+  unsigned* pieces;   // [streams][row tiles]: how many of them are there, zero between launches
+};
 template <int EPI>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lin_big_kernel(LinArgs a, const int row_tiles, const int tiles) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lin_big_kernel(LinArgs a, const int row_tiles, const int tiles, const LinStream ls) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
+  __shared__ unsigned s_there;
   constexpr int STAGE = 32 * 1024;
-  const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 256, f0 = b / row_tiles * 256, per = part_tiles(a), k0 = blockIdx.y * per, n = min(a.kt - k0, per);
-  a.out_f += blockIdx.y * a.part_stride;
+  const int b = xcd_range(blockIdx.x, ls.streams ? ls.streams * row_tiles : tiles), row_tile = b % row_tiles, row0 = row_tile * 256, stream = b / row_tiles;
+  // this workgroup's k tiles, counted through the feature tiles
+  int first, last;
+  if (ls.streams) {
+    const long long pairs = (long long)(tiles / row_tiles) * (a.kt >> 1);
+    first = (int)(pairs * stream / ls.streams) * 2;
+    last = (int)(pairs * (stream + 1) / ls.streams) * 2;
+  } else {
+    const int per = part_tiles(a);
+    first = stream * a.kt + blockIdx.y * per;
+    last = min(first + per, (stream + 1) * a.kt);
+    a.out_f += blockIdx.y * a.part_stride;
+  }
   const int n_rows = min(256, a.rows - row0);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1, rt0 = f0 >> 4;
-  const char *src_w[2], *src_a[2];  // this wave's share of a stage: weight tiles and row groups 2 * wave + {0, 1}
+  const int wm = wave & 1, wn = wave >> 1;
+  int at_a[2];  // this wave's share of a stage: weight tiles and row groups 2 * wave + {0, 1}
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int t = 2 * wave + i;
-    src_w[i] = reinterpret_cast<const char*>(a.w) + ((size_t)min(rt0 + t, a.rt - 1) * a.kt + k0) * 1024 + lane * 16;
-    src_a[i] = reinterpret_cast<const char*>(operand<bf16>(a, f0) + (size_t)(row0 + min(t * 16 + block_row(lane), n_rows - 1)) * a.lda + (size_t)k0 * 32 + block_group(lane) * 8);
-  }
-  auto stage = [&](int kt, char* buf) {  // (past the end: the last tile again, never read)
-    kt = min(kt, n - 1);
+  for (int i = 0; i < 2; ++i) at_a[i] = (row0 + min((2 * wave + i) * 16 + block_row(lane), n_rows - 1)) * a.lda + block_group(lane) * 8;
+  int f_in = first / a.kt, k_in = first - f_in * a.kt, left = last - first;  // what is requested next
+  auto stage = [&](char* buf) {  // (past the end: the last tile again, never read)
+    const bf16* x = operand<bf16>(a, f_in * 256) + (size_t)k_in * 32;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int slot = 2 * wave + i;
-      __builtin_amdgcn_global_load_lds((gptr)(src_w[i] + (size_t)kt * 1024), (lptr)(buf + slot * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gptr)(src_a[i] + (size_t)kt * 64), (lptr)(buf + 16 * 1024 + slot * 1024), 16, 0, 0);
+      const uint16_t* w = a.w + ((size_t)min(f_in * 16 + slot, a.rt - 1) * a.kt + k_in) * 512;
+      __builtin_amdgcn_global_load_lds((gptr)(w + lane * 8), (lptr)(buf + slot * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr)(x + at_a[i]), (lptr)(buf + 16 * 1024 + slot * 1024), 16, 0, 0);
     }
+    const int go = left > 1, wrap = go && k_in + 1 == a.kt;
+    left -= go;
+    f_in += wrap;
+    k_in = wrap ? 0 : k_in + go;
   };
   f32x4 acc[8][4];
+  auto clear = [&]() {
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
   struct Operands {
     bf16x8 w[8], x[4];
   };
@@ -436,12 +462,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < 8; ++i) o.w[i] = *reinterpret_cast<const bf16x8*>(buf + (wm * 8 + i) * 1024 + lane * 16);
   };
   int cur = 0;
-  auto step = [&](int kt, const Operands& now, Operands& next) {
-    // tile kt + 1 is here when at most the loads of RING - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
-    // tile kt in registers, so that its buffer takes tile kt + RING
+  auto step = [&](const Operands& now, Operands& next) {
+    // the next k tile is here when at most the loads of RING - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
+    // this one in registers, so that its buffer takes the one RING tiles on
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (RING - 2)) : "memory");
     lds_barrier();
-    stage(kt + RING, lds + cur * STAGE);
+    stage(lds + cur * STAGE);
     cur = cur + 1 == RING ? 0 : cur + 1;
     read(lds + cur * STAGE, next);
 #pragma unroll
@@ -455,30 +481,78 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
   };
+  // the piece of a cut tile: true if the other one is there and is in the sums now, else ours is left for whoever works off the other one
+  auto joined = [&](int cut, bool behind) {
+    const int at = cut * row_tiles + row_tile;
+    unsigned* there = ls.pieces + at;
+    float* ours = ls.sums + ((size_t)at * 2 + behind) * 65536;
+    float* theirs = ls.sums + ((size_t)at * 2 + !behind) * 65536;
+    auto look = [&](unsigned v) {  // (a value of thread 0, to everybody)
+      __syncthreads();
+      if (tid == 0) s_there = v;
+      __syncthreads();
+      return s_there != 0;
+    };
+    bool second = look(tid == 0 ? __hip_atomic_load(there, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0);
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    if (!second) {
+      const auto r = __builtin_amdgcn_make_buffer_rsrc(ours, 0, 65536 * 4, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), r, tid * 16, (i * 4 + j) * 8192, 16 /* sc1 */);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      second = look(tid == 0 ? __hip_atomic_fetch_add(there, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0);
+      if (!second) return false;
+    }
+    if (tid == 0) __hip_atomic_store(there, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(theirs, 0, 65536 * 4, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f32x4 o[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, tid * 16, (i * 4 + j) * 8192, 16));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] += o[j];
+    }
+    return true;
+  };
   Operands p, q;
 #pragma unroll
-  for (int i = 0; i < RING; ++i) stage(i, lds + i * STAGE);
+  for (int i = 0; i < RING; ++i) stage(lds + i * STAGE);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (RING - 1)) : "memory");
   lds_barrier();
   read(lds, p);
-  for (int kt = 0; kt < n; kt += 2) {  // (n is even)
-    step(kt, p, q);
-    step(kt + 1, q, p);
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const int st0 = rt0 + wm * 8;
-  const bool pairs = wide_pairs(a) && (st0 + 8) * 16 <= a.n_wide && st0 + 8 <= a.rt;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = wn * 64 + j * 16 + (lane & 15);
-    if (pairs) {
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) store_wide_pair<EPI == LIN_TANH_F ? LIN_STORE : EPI>(a, r < n_rows, row0 + r, st0 + i, acc[i][j], acc[i + 1][j]);
-    } else if (r < n_rows) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (st0 + i < a.rt) store_plain<bf16, EPI>(a, row0 + r, (st0 + i) * 16 + (lane >> 4) * 4, acc[i][j]);
+  for (int at = first; at < last;) {
+    const int f = at / a.kt, end = min(last, (f + 1) * a.kt);
+    const bool cut_front = ls.streams && at > f * a.kt, cut_end = ls.streams && end < (f + 1) * a.kt;
+    clear();
+    for (; at < end; at += 2) {  // (stretches and parts are even)
+      step(p, q);
+      step(q, p);
     }
+    if (cut_front || cut_end) {
+      if (!joined(cut_front ? stream : stream + 1, cut_front)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        continue;
+      }
+    }
+    const int rt0 = f * 16 + wm * 8;
+    const bool pairs = wide_pairs(a) && (rt0 + 8) * 16 <= a.n_wide && rt0 + 8 <= a.rt;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = wn * 64 + j * 16 + (lane & 15);
+      if (pairs) {
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) store_wide_pair<EPI == LIN_TANH_F ? LIN_STORE : EPI>(a, r < n_rows, row0 + r, rt0 + i, acc[i][j], acc[i + 1][j]);
+      } else if (r < n_rows) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (rt0 + i < a.rt) store_plain<bf16, EPI>(a, row0 + r, (rt0 + i) * 16 + (lane >> 4) * 4, acc[i][j]);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (a step counts loads alone)
   }
 }
 
@@ -676,24 +750,49 @@ static int allow_lds(K k, int bytes) {
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   return DSK_OK;
 }
-// Microseconds a prompt product takes on 256 compute units, by measurement: two workgroups of 128 x 128 on one work 1.3 us on a step of 64
-// columns (one alone 1.05), one of 256 x 256 takes 1.84 us and starts and ends slower; a part more writes and reads its sums.
-// In 32 bits a step of 64 columns takes 1.75 us alone and 3.2 us of two.
-static double lin_cost(int rows, int rt, int kt, int parts, bool big, bool f32) {
-  const double k = part_tiles(kt, parts) / 2, sums = (parts - 1) * 3.2e-5 * rows * rt;
-  if (big) return f32 ? 1e9 : cdiv(cdiv(rows, 256) * cdiv(rt, 16) * parts, 256) * (15 + 1.84 * k) + sums;
-  const int n = cdiv(rows, 128) * cdiv(rt, 8) * parts;
-  return (n <= 256 ? (f32 ? 1.75 : 1.05) * k : cdiv(n, 512) * (f32 ? 3.2 : 1.3) * k) + 5 + sums;
+// Microseconds a prompt product takes on 256 compute units, by measurement of 20 shapes of 100 - 2000 rows and k of 2048 - 27648 (within a tenth of most): a
+// step of 64 columns takes a workgroup of 128 x 128 alone on its compute unit 0.6 us (0.85 with weights out of HBM), two of them 1.0 - 1.08; one of 256 x 256
+// takes 1.17 us, and 1.55 when all of them run (the card's clock).  Both start and end in 3 and 8 us; a part more writes and reads its sums.
+// Stretches (LinStream) leave no compute unit empty, but their rows and weights meet in L2 less often (1.72 us), and tiles that they cut are stored and read:
+// 2000 rows and 2048 x 16896 145 us, by 128 x 128 163, by 256 x 256 168; 7168 x 32896 803, 1066, 895; but 1500 rows and 7168 x 27648 550, 658, 541.
+// In 32 bits a step of 64 columns takes 1.48 us alone, 2.6 - 3 us of two.
+enum { LIN_SMALL, LIN_BIG, LIN_STREAM };
+static int lin_streams(int rows, int rt) {  // stretches of a row of 256 x 256 tiles; 0: they would cut a tile more than once
+  const int n = 256 / cdiv(rows, 256);
+  return n >= 2 && n <= cdiv(rt, 16) ? n : 0;
 }
-static bool lin_big(const LinArgs& a, int parts, bool f32) {
-  if (f32 || (a.a_seg & 255)) return false;
-  return a.tile ? a.tile == 256 : lin_cost(a.rows, a.rt, a.kt, parts, true, f32) < lin_cost(a.rows, a.rt, a.kt, parts, false, f32);
+static double lin_cost(int rows, int rt, int kt, int parts, int kind, bool f32) {
+  const double k = part_tiles(kt, parts) / 2, sums = (parts - 1) * 3.2e-5 * rows * rt;
+  if (kind != LIN_SMALL && f32) return 1e9;
+  if (kind == LIN_STREAM) {
+    const int n = lin_streams(rows, rt);
+    return n && parts == 1 ? 32 + 1.72 * k * cdiv(rt, 16) / n : 1e9;
+  }
+  if (kind == LIN_BIG) {
+    const int n = cdiv(rows, 256) * cdiv(rt, 16) * parts, rest = n % 256;
+    return n / 256 * (8 + 1.55 * k) + (rest ? 8 + (1.17 + 0.38 / 256 * rest) * k : 0) + sums;
+  }
+  const int n = cdiv(rows, 128) * cdiv(rt, 8) * parts, rest = n % 512;
+  if (f32) return 3 + (n <= 256 ? 1.48 : 1.6 + 1.9 / 512 * n) * k + sums;
+  return 3 + (n / 512 * 1.08 + (rest == 0 ? 0 : rest <= 256 ? 0.85 : 1.0)) * k + sums;
+}
+static int lin_kind(int rows, int rt, int kt, int parts, bool f32) {
+  int best = LIN_SMALL;
+  for (int kind : {LIN_BIG, LIN_STREAM})
+    if (lin_cost(rows, rt, kt, parts, kind, f32) < lin_cost(rows, rt, kt, parts, best, f32)) best = kind;
+  return best;
+}
+static int lin_kind(const LinArgs& a, int parts, bool f32, const LinSpace& space) {
+  if (f32 || (a.a_seg & 255)) return LIN_SMALL;
+  int kind = lin_kind(a.rows, a.rt, a.kt, parts, f32);
+  if (a.tile) kind = a.tile == 128 ? LIN_SMALL : parts == 1 && lin_streams(a.rows, a.rt) ? LIN_STREAM : LIN_BIG;
+  return kind == LIN_STREAM && space.slots < LIN_SLOTS ? LIN_BIG : kind;
 }
 int lin_parts(int rows, int rt, int kt, bool f32, int most) {
   int best = 1;
   double least = 0;
   for (int n = 1; n <= most && (n == 1 || kt / n >= 16); ++n) {
-    const double c = std::min(lin_cost(rows, rt, kt, n, false, f32), lin_cost(rows, rt, kt, n, true, f32));
+    const double c = lin_cost(rows, rt, kt, n, lin_kind(rows, rt, kt, n, f32), f32);
     if (n == 1 || c < least) {
       least = c;
       best = n;
@@ -701,19 +800,27 @@ int lin_parts(int rows, int rt, int kt, bool f32, int most) {
   }
   return cdiv(kt, part_tiles(kt, best));  // (no part may be empty)
 }
+bool lin_streams_some(int rows, int rt, int kt, int tile) {
+  bool some = false;
+  for (int r = rows; r > 0; r -= 256)  // (row tiles decide)
+    some = some || (tile ? tile == 256 && lin_streams(r, rt) : lin_kind(r, rt, kt, 1, false) == LIN_STREAM);
+  return some;
+}
 int lin_parts_few(int rt, int kt, int most) {
   const int n = std::max(std::min({1024 / rt, kt / 16, most}), 1);
   return cdiv(kt, part_tiles(kt, n));
 }
 #define LIN_EPI(K, T) (a.epi == LIN_STORE ? K<T LIN_STORE> : a.epi == LIN_XIELU ? K<T LIN_XIELU> : a.epi == LIN_TANH_F ? K<T LIN_TANH_F> : K<T - 1>)
-int launch_lin(hipStream_t st, const LinArgs& a, bool f32) {
+int launch_lin(hipStream_t st, const LinArgs& a, bool f32, const LinSpace& space) {
   DSK_TRY(check_lin(a, "lin"));
   if ((a.a_seg & 127) || a.row_seq || a.out_at) DSK_FAIL(DSK_ERR_INVALID, "lin: %d features per operand", a.a_seg);
-  if (lin_big(a, std::max(a.parts, 1), f32)) {
+  const int kind = lin_kind(a, std::max(a.parts, 1), f32, space);
+  if (kind != LIN_SMALL) {
     const int row_tiles = cdiv(a.rows, 256), tiles = row_tiles * cdiv(a.rt, 16);
+    const LinStream ls{kind == LIN_STREAM ? lin_streams(a.rows, a.rt) : 0, space.sums, space.pieces};
     auto k = LIN_EPI(lin_big_kernel, );
     DSK_TRY(allow_lds(k, RING * 32 * 1024));
-    hipLaunchKernelGGL(k, dim3(tiles, std::max(a.parts, 1)), dim3(512), RING * 32 * 1024, st, a, row_tiles, tiles);
+    hipLaunchKernelGGL(k, dim3(ls.streams ? ls.streams * row_tiles : tiles, std::max(a.parts, 1)), dim3(512), RING * 32 * 1024, st, a, row_tiles, tiles, ls);
     return DSK_OK;
   }
   if (a.direct) {

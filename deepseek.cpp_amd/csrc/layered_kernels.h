@@ -59,7 +59,7 @@ struct LinArgs {
   size_t a_stride;        // ... a_stride elements behind each other (launch_lin: a_seg is a multiple of 128, else of 16)
   int parts;              // > 1: k in `parts` ranges, each with a 32-bit output of its own (part_stride elements behind each other; n_wide = 0,
   size_t part_stride;     // LIN_STORE); the reader adds them up
-  int tile;               // launch_lin: 0 chooses, 128 or 256 (bf16)
+  int tile;               // launch_lin: 0 chooses, 128 or 256 (bf16; in stretches where they can be)
   int direct;             // launch_lin in 32 bits: activations whole on the 32-bit matrix instruction (few k tiles; one part)
   const int* row_seq;     // launch_lin_few: output row i reads the first row of sequence row_seq[i] of seqs (nullptr: row i)
   const SeqDesc* seqs;
@@ -68,7 +68,15 @@ struct LinArgs {
 // parts worth splitting k into, at most `most`: launch_lin, launch_lin_few
 int lin_parts(int rows, int rt, int kt, bool f32, int most);
 int lin_parts_few(int rt, int kt, int most);
-int launch_lin(hipStream_t st, const LinArgs& a, bool f32);          // any number of rows (tiles of 128)
+// room for the pieces of tiles that two workgroups share: 256 slots of two tiles of 256 x 256 sums, and their words (zero between launches)
+enum { LIN_SLOTS = 256, LIN_SLOT_FLOATS = 2 * 256 * 256 };
+struct LinSpace {
+  float* sums;
+  unsigned* pieces;
+  int slots;  // LIN_SLOTS, or 0: no such room
+};
+int launch_lin(hipStream_t st, const LinArgs& a, bool f32, const LinSpace& space = LinSpace{});  // any number of rows
+bool lin_streams_some(int rows, int rt, int kt, int tile);             // does a product of up to that many rows take such room (bf16; tile: LinArgs)?
 int launch_lin_few(hipStream_t st, const LinArgs* a, int n, bool f32);  // up to 16 rows; n <= 4 products in one launch
 
 // ---- experts ----

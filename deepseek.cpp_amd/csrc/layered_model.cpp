@@ -15,7 +15,7 @@
 
 namespace {
 
-enum { FEW = 16, LOGIT_ROWS = 128, MIX_PARTS = 4, MIX_PARTS_FEW = 8 };
+enum { FEW = 16, LOGIT_ROWS = 128, MIX_ROWS = 4, MIX_PARTS = 8, MIX_PARTS_FEW = 8 };
 
 size_t up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -128,6 +128,7 @@ struct LayeredModel : ModelHead {
   int last_rows = 0;
   bool chunk_scan = true;
   int tile = 0;                     // of prompt products (LinArgs::tile)
+  LinSpace space{};                 // of prompt products
   ChunkScan scan{};                 // operands of the recurrences over chunks (kernels_chunk_scan.hip)
   int max_chunks = 0;
   float* attn_part = nullptr;       // parts of attention outputs (kernels_mix_few.hip)
@@ -599,6 +600,15 @@ int alloc_work(LayeredModel* m) {
   m->low_ld = low;
   m->slots = tmax;
   m->ld_logits = m->head.rt * 16;
+  bool streams = false;
+  for (const LayerW& w : m->L)
+    for (const PackedMat* p : {&w.proj, &w.a_o, &w.m_o, &w.d_o, &w.w_o, &w.l_o, &w.l_uq, &w.l_ukv, &w.ff_up, &w.ff_down})
+      streams |= !m->f32 && p->w && lin_streams_some((int)n, p->rt, p->kt, m->tile);
+  if (streams) {
+    DSK_TRY(dev_alloc_n(m, &m->space.sums, (size_t)LIN_SLOTS * LIN_SLOT_FLOATS));
+    DSK_TRY(dev_alloc_n(m, &m->space.pieces, LIN_SLOTS));
+    m->space.slots = LIN_SLOTS;
+  }
   DSK_TRY(dev_alloc_n(m, &m->x_all, n * D));
   DSK_TRY(dev_alloc_n(m, &m->x_few, (size_t)FEW * D));
   DSK_TRY(dev_alloc(m, (void**)&m->h, n * m->h_ld * e * m->mixes));
@@ -619,7 +629,7 @@ int alloc_work(LayeredModel* m) {
   DSK_TRY(dev_alloc_n(m, &m->narrow, n * m->ldf));
   DSK_TRY(dev_alloc(m, (void**)&m->out_a, n * m->out_ld * e));
   DSK_TRY(dev_alloc(m, (void**)&m->out_b, n * m->out_ld * e));
-  const size_t mix_rows = std::max<size_t>(n * MIX_PARTS, FEW * MIX_PARTS_FEW);
+  const size_t mix_rows = std::max<size_t>(n * MIX_ROWS, FEW * MIX_PARTS_FEW);
   DSK_TRY(dev_alloc_n(m, &m->mix_a, mix_rows * m->mix_ld));
   DSK_TRY(dev_alloc_n(m, &m->mix_b, mix_rows * m->mix_ld));
   DSK_TRY(dev_alloc(m, (void**)&m->qb, n * aq * e));
@@ -697,7 +707,7 @@ LinArgs lin_f(const PackedMat& w, const void* a, int lda, int rows, float* out, 
 // A product whose output the next residual sum reads (mix_a; second: mix_b), split over k where its tiles alone leave compute units idle
 LinArgs mix_lin(LayeredModel* m, const PackedMat& w, const void* a, int lda, int rows, bool few, bool second = false) {
   LinArgs l = lin_f(w, a, lda, rows, second ? m->mix_b : m->mix_a, m->mix_ld);
-  l.parts = m->mix_parts[second] = few ? lin_parts_few(w.rt, w.kt, MIX_PARTS_FEW) : lin_parts(rows, w.rt, w.kt, m->f32, MIX_PARTS);
+  l.parts = m->mix_parts[second] = few ? lin_parts_few(w.rt, w.kt, MIX_PARTS_FEW) : lin_parts(rows, w.rt, w.kt, m->f32, std::min<int>(MIX_PARTS, MIX_ROWS * m->piece / rows));
   l.part_stride = m->mix_stride = (size_t)rows * m->mix_ld;
   return l;
 }
@@ -706,7 +716,7 @@ int run_lin(LayeredModel* m, const LinArgs* a, int n, bool few) {
   for (int i = 0; i < n; ++i) {
     LinArgs l = a[i];
     l.tile = m->tile;
-    DSK_TRY(launch_lin(m->ctx->stream, l, m->f32));
+    DSK_TRY(launch_lin(m->ctx->stream, l, m->f32, m->space));
   }
   return DSK_OK;
 }

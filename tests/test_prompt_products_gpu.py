@@ -174,3 +174,23 @@ def test_logits_of_few_and_many_rows(ctx, tmp_path, vocab):
     seqs = [K.lm.seq_open() for _ in range(17)]
     for i in range(6):
         assert U.err(K.lm.step([(s, t[i:i + 1], [0]) for s in seqs]), np.repeat(want[i:i + 1], 17, 0)) < U.F32, i
+
+
+# Stretches over several 256 x 256 tiles (LinStream): four to eight row tiles in 64 to 32 stretches of 67 feature tiles, a last tile of features that is not full, rows that end
+# inside a tile, cuts at the first and last steps of a tile; blends (an operand per feature range) and xIELU.  The same rows by tiles of 128: sums in
+# another order alone, 32 bits of a sum of up to 2048 products, bfloat16 behind it
+@pytest.mark.parametrize("rows", [769, 1280, 1500, 1537, 2048])
+def test_products_in_stretches(ctx, tmp_path, rows):
+    c = U.sandwich([dict(U.wkv(32, 64), mlp=U.dense(16900))], width=2048, vocab=64)
+    runs = [U.Case(ctx, tmp_path / str(tile), c, dtype="bfloat16", options=f"prompt_tile={tile}") for tile in (256, 128)]
+    t = runs[0].tokens(rows)
+    got = []
+    for K in runs:
+        K.lm.set_trace(True)
+        for _ in range(2):  # (the words between the workgroups are zero again behind the first)
+            s = K.lm.seq_open()
+            K.lm.step([(s, t, [rows - 1])])
+            got.append(K.lm.trace_rows(0, rows))
+            K.lm.seq_close(s)
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]) and np.array_equal(got[2], got[3])
+    assert U.err(got[0], got[2]) < 0.02
