@@ -2,12 +2,13 @@
 //
 //   lin_kernel      prompts: 128 features x 128 rows per workgroup, 4 waves of 64 x 64, both operands through LDS in fragment
 //                   order (global_load_lds, 16 bytes per lane: LDS reads are lane-linear, no bank conflicts), two buffers
-//   lin_big_kernel  the same with 256 x 256 and a ring of four stages, where there are enough of such tiles (bf16)
+//   rows_kernel     the same in 32 bits, 128 features x 128 or 64 rows, each wave with rows of its own
+//   lin_big_kernel  lin_kernel's with 256 x 256 and a ring of four stages, where there are enough of such tiles (bf16)
 //   lin_direct_kernel  32-bit activations times a few k tiles, operands straight from memory
 //   few_kernel      up to 16 rows (decoding): 4 waves share 16 or 64 features and split k; weights stream from HBM straight into the
 //                   MFMA operand registers, 1 KiB contiguous per wave and load
 //   expert_kernel   the experts' products of prompts, rows gathered per expert: 256 features x 128 (64, 32) rows, weights straight
-//                   into registers (32 bits: lin_kernel's tiles)
+//                   into registers (32 bits: rows_kernel's tiles)
 // few_kernel takes plain products and the experts', several of them in one launch.
 #include "layered_kernels.h"
 #include "lin_device.h"
@@ -74,10 +75,12 @@ int launch_fill_random_f32(hipStream_t st, float* dst, size_t n, float scale, ui
 
 // ---- prompts -------------------------------------------------------------------------------------
 // What a workgroup keeps in LDS.  bf16: two stages of two k tiles (8 weight tiles and 8 row groups each), 64 KiB; deeper rings with a barrier
-// per k tile were no faster (two workgroups on a compute unit hide each other's waits).  32 bits: a ring of three stages of one k tile, 72 KiB.
-__host__ DEV constexpr int lin_stages(int size) { return size == 2 ? 2 : 3; }
-__host__ DEV constexpr int lin_step(int size) { return size == 2 ? 2 : 1; }
-__host__ DEV constexpr int lin_stage(int size) { return lin_step(size) * 8 * 1024 * (1 + size / 2); }
+// per k tile were no faster (two workgroups on a compute unit hide each other's waits).
+enum { LIN_STEP = 2, LIN_STAGE = LIN_STEP * 16 * 1024, LIN_LDS = 2 * LIN_STAGE };
+// 32 bits, 64 J rows: a ring of three stages of one k tile (8 weight tiles, 4 J row groups of two KiB), 72 or 48 KiB.
+enum { ROWS_RING = 3 };
+template <int J>
+__host__ DEV constexpr int rows_stage() { return 8 * 1024 * (1 + J); }
 // 32 features (tiles rt, rt + 1) x 32 rows (from `first` on) of a wave by itself on v_mfma_f32_16x16x4_f32, operands straight from memory: one chain of
 // the instruction per sum.  f0: a feature whose operand it is.
 template <int EPI>
@@ -128,30 +131,22 @@ DEV void direct_tile(const LinArgs& a, const int* gather, int row0, int n_rows, 
     }
   }
 }
-// 128 features from f0 on x n_rows <= 128 rows, k tiles [k0, k1): 4 waves of 64 x 64.  gather: a table (slot -> row) or nullptr; out rows are
-// row0 + local row.
-template <typename T, int EPI>
-DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
-  typedef typename Frag<T>::type frag;
-  constexpr int AB = 64 * (int)sizeof(frag);  // bytes of an A fragment
-  constexpr int KS = lin_step(sizeof(T)), STAGE = lin_stage(sizeof(T)), R = lin_stages(sizeof(T)), H = sizeof(T) / 2, WB = 8 * KS * 1024;
+// 128 features from f0 on x n_rows <= 128 rows, k tiles [k0, k1), bf16: 4 waves of 64 x 64.
+template <int EPI>
+DEV void lin_body(const LinArgs& a, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
+  constexpr int KS = LIN_STEP, WB = 8 * KS * 1024;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1, n = k1 - k0;
   const int rt0 = f0 >> 4;
   // this wave's share of the staging: two weight tiles and two row groups, the k tiles of a stage
-  const char *src_w[2], *src_a[2][H];
+  const char *src_w[2], *src_a[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)  // (tiles past the end: any valid one, never stored)
     src_w[i] = reinterpret_cast<const char*>(a.w) + ((size_t)min(rt0 + 2 * wave + i, a.rt - 1) * a.kt + k0) * 1024 + lane * 16;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int t = 2 * wave + i;
-#pragma unroll
-    for (int h = 0; h < H; ++h) {  // (a block of 16 x 32 floats is two loads of 8 rows)
-      int r = min(t * 16 + (H == 1 ? block_row(lane) : h * 8 + (lane >> 3)), n_rows - 1);
-      r = gather ? gather[row0 + r] : row0 + r;
-      src_a[i][h] = reinterpret_cast<const char*>(operand<T>(a, f0) + (size_t)r * a.lda + (size_t)k0 * 32) + (H == 1 ? block_group(lane) : (lane & 7) ^ (lane >> 3)) * 16;
-    }
+    const int r = row0 + min((2 * wave + i) * 16 + block_row(lane), n_rows - 1);
+    src_a[i] = reinterpret_cast<const char*>(operand<bf16>(a, f0) + (size_t)r * a.lda + (size_t)k0 * 32) + block_group(lane) * 16;
   }
   auto stage = [&](int kt, char* buf) {
 #pragma unroll
@@ -162,112 +157,31 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) {
-        const int slot = (2 * wave + i) * KS + kk;
-#pragma unroll
-        for (int h = 0; h < H; ++h)
-          __builtin_amdgcn_global_load_lds((gptr)(src_a[i][h] + (size_t)(kt + kk) * 32 * sizeof(T)), (lptr)(buf + WB + slot * AB + h * 1024), 16, 0, 0);
-      }
+      for (int kk = 0; kk < KS; ++kk)
+        __builtin_amdgcn_global_load_lds((gptr)(src_a[i] + (size_t)(kt + kk) * 64), (lptr)(buf + WB + ((2 * wave + i) * KS + kk) * 1024), 16, 0, 0);
   };
   f32x4 acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (sizeof(T) == 2) {
-    stage(0, lds);
-    for (int kt = 0; kt < n; kt += KS) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads into LDS; the barrier makes it everybody's
-      __syncthreads();
-      char* cur = lds + ((kt / KS) & 1) * STAGE;
-      if (kt + KS < n) stage(kt + KS, lds + (((kt / KS) & 1) ^ 1) * STAGE);
+  stage(0, lds);
+  for (int kt = 0; kt < n; kt += KS) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads into LDS; the barrier makes it everybody's
+    __syncthreads();
+    char* cur = lds + ((kt / KS) & 1) * LIN_STAGE;
+    if (kt + KS < n) stage(kt + KS, lds + (((kt / KS) & 1) ^ 1) * LIN_STAGE);
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) {
-        bf16x8 w[4], x[4];
+    for (int kk = 0; kk < KS; ++kk) {
+      bf16x8 w[4], x[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const bf16x8*>(cur + ((wm * 4 + i) * KS + kk) * 1024 + lane * 16);
+      for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const bf16x8*>(cur + ((wm * 4 + i) * KS + kk) * 1024 + lane * 16);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const bf16x8*>(cur + WB + ((wn * 4 + j) * KS + kk) * AB + block_place(lane) * 16);
+      for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const bf16x8*>(cur + WB + ((wn * 4 + j) * KS + kk) * 1024 + block_place(lane) * 16);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = mma(w[i], x[j], acc[i][j]);
-      }
-    }
-  } else {
-    // While a k tile is multiplied the next one's operands are read into the other set of registers and the loads of R - 1 more are on
-    // their way.  What bounds it: per wave and k tile 48 matrix instructions (768 cycles) and the 176 vector instructions (704 cycles)
-    // that take 32 activations apart; they are issued in turns, a row group's matrix work beside the splitting of the next.
-    // 301 x 2048 x 16896: 303 us with v_mfma_f32_16x16x4_f32, 97 us so; 301 x 16896 x 2048 in 4 parts: 304 -> 108 us.
-    struct Operands {
-      bf16x8 w[4];
-      f32x8 x[4];
-    };
-    // eight lanes to the 128 bytes of a row, its pieces of 16 bytes exchanged by the row's place as in block_place
-    const int at = (lane & 15) * 128 + (((lane >> 4) * 2) ^ (lane & 7)) * 16;
-    auto read = [&](const char* buf, Operands& o) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const char* s = buf + WB + (wn * 4 + j) * AB;
-        o.x[j] = __builtin_shufflevector(*reinterpret_cast<const f32x4*>(s + at), *reinterpret_cast<const f32x4*>(s + (at ^ 16)), 0, 1, 2, 3, 4, 5, 6, 7);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o.w[i] = *reinterpret_cast<const bf16x8*>(buf + (wm * 4 + i) * 1024 + lane * 16);
-    };
-    int cur = 0;
-    auto step = [&](int kt, const Operands& now, Operands& next) {
-      // tile kt + 1 is here when at most the loads of R - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
-      // tile kt in registers, so that its buffer takes tile kt + R (past the end: the last one again, never read)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 + 2 * H) * (R - 2)) : "memory");
-      lds_barrier();
-      stage(min(kt + R, n - 1), lds + cur * STAGE);
-      cur = cur + 1 == R ? 0 : cur + 1;
-      read(lds + cur * STAGE, next);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const Split x = split3(now.x[j]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[i], x.b2, acc[i][j]);  // (one piece after the other: no instruction waits for the last)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[i], x.b1, acc[i][j]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i][j] = mma(now.w[i], x.b0, acc[i][j]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (j == 0) __builtin_amdgcn_sched_group_barrier(0x002, 48, 0);
-#pragma unroll
-        for (int i = 0; i < 12; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (j == 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          if (j < 3) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-        }
-      }
-    };
-    Operands p, q;
-#pragma unroll
-    for (int i = 0; i < R; ++i) stage(min(i, n - 1), lds + i * STAGE);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 + 2 * H) * (R - 1)) : "memory");
-    lds_barrier();
-    read(lds, p);
-    for (int kt = 0; kt < n; kt += 2) {  // (n is even)
-      step(kt, p, q);
-      step(kt + 1, q, p);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // Three pieces stand for the activation while everything is finite: an infinity's rest is no number, and neither is a zero rest times an
-    // infinite weight.  A wave with a sum that is not finite adds its tiles up again.
-    float bad = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bad = fmaf(acc[i][j][e], 0.f, bad);
-    if (__any(bad != bad)) {
-#pragma unroll 1
-      for (int i = 0; i < 4; ++i) direct_tile<EPI>(a, gather, row0, n_rows, f0, rt0 + wm * 4 + (i & 1) * 2, wn * 64 + (i >> 1) * 32, k0, k1);
-      return;
+        for (int j = 0; j < 4; ++j) acc[i][j] = mma(w[i], x[j], acc[i][j]);
     }
   }
 #pragma unroll
@@ -277,11 +191,138 @@ DEV void lin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int rt = rt0 + wm * 4 + i;
+      if (rt < a.rt) store_plain<bf16, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+    }
+  }
+}
+// 128 features from f0 on x n_rows <= 64 J rows, k tiles [k0, k1), 32 bits: 4 waves of 128 features x 16 J rows.  gather: a table (slot -> row) or
+// nullptr; out rows are row0 + local row.
+// Activations are taken apart into three bf16 numbers (split3, 44 vector instructions for 16 rows of a k tile, 176 cycles); a wave has rows of its own, so
+// that no two of them take the same ones apart: per wave and k tile 24 J matrix instructions (384 J cycles) and 44 J vector instructions beside them.
+// While a k tile is multiplied the next one's operands are read and taken apart, and the loads of ROWS_RING - 1 more are on their way (rings of four and
+// five were not faster, and leave room for a workgroup less).  The matrix instructions bound it where compute units are full (128 rows: 1.23 us for two
+// workgroups' steps of 64 columns, of 1.28), what a wave does alone where they are not.  4 waves of 64 x 64, each row taken apart by two of them and that
+// work behind the matrix work, took 99 us for 301 x 2048 x 16896, 100 for 301 x 16896 x 2048 and 42 - 65 for 301 x 2048 x 2176 - 8320; this 62, 62 and
+// 25 - 39, with v_mfma_f32_16x16x4_f32 the first was 303.
+template <int J, int EPI>
+DEV void rows_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
+  constexpr int R = ROWS_RING, STAGE = rows_stage<J>(), WB = 8 * 1024, LOADS = 2 + 2 * J;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = k1 - k0;
+  const int rt0 = f0 >> 4, own = wave * 16 * J;
+  // this wave's share of the staging: two weight tiles and its own rows (a block of 16 x 32 floats is two loads of 8 rows)
+  const char *src_w[2], *src_a[2 * J];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)  // (tiles past the end: any valid one, never stored)
+    src_w[i] = reinterpret_cast<const char*>(a.w) + ((size_t)min(rt0 + 2 * wave + i, a.rt - 1) * a.kt + k0) * 1024 + lane * 16;
+#pragma unroll
+  for (int h = 0; h < 2 * J; ++h) {
+    int r = min(own + h * 8 + (lane >> 3), n_rows - 1);
+    r = gather ? gather[row0 + r] : row0 + r;
+    src_a[h] = reinterpret_cast<const char*>(operand<float>(a, f0) + (size_t)r * a.lda + (size_t)k0 * 32) + ((lane & 7) ^ (lane >> 3)) * 16;
+  }
+  auto stage = [&](int kt, char* buf) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((gptr)(src_w[i] + (size_t)kt * 1024), (lptr)(buf + (2 * wave + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int h = 0; h < 2 * J; ++h) __builtin_amdgcn_global_load_lds((gptr)(src_a[h] + (size_t)kt * 128), (lptr)(buf + WB + (wave * 2 * J + h) * 1024), 16, 0, 0);
+  };
+  f32x4 acc[8][J];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  struct Operands {
+    bf16x8 w[8];
+    Split x[J];
+  };
+  // eight lanes to the 128 bytes of a row, its pieces of 16 bytes exchanged by the row's place as in block_place
+  const int at = (lane & 15) * 128 + (((lane >> 4) * 2) ^ (lane & 7)) * 16;
+  auto read_x = [&](const char* buf, f32x8 (&x)[J]) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const char* s = buf + WB + (wave * J + j) * 2048;
+      x[j] = __builtin_shufflevector(*reinterpret_cast<const f32x4*>(s + at), *reinterpret_cast<const f32x4*>(s + (at ^ 16)), 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  };
+  auto read_w = [&](const char* buf, int i, Operands& o) { o.w[i] = *reinterpret_cast<const bf16x8*>(buf + i * 1024 + lane * 16); };
+  int cur = 0;
+  auto step = [&](int kt, const Operands& now, Operands& next) {
+    // tile kt + 1 is here when at most the loads of R - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
+    // tile kt in registers, so that its buffer takes tile kt + R (past the end: the last one again, never read)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * (R - 2)) : "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), which the barrier waits for: so that the compiler knows and the first products wait for no reads
+    lds_barrier();
+    stage(min(kt + R, n - 1), lds + cur * STAGE);
+    cur = cur + 1 == R ? 0 : cur + 1;
+    const char* buf = lds + cur * STAGE;
+    f32x8 x[J];
+    read_x(buf, x);
+    __builtin_amdgcn_sched_barrier(0);
+    // Four matrix instructions at a time: beside the first eight the weights are read, beside the last 16 J the next rows are taken apart, a pair of
+    // columns (11 vector instructions) by four of them.  (One piece after the other: no instruction waits for the last.)
+#pragma unroll
+    for (int g = 0; g < 6 * J; ++g) {
+      const int j = g / 6, piece = 2 - g % 6 / 2, half = g % 2 * 4, pair = g - 2 * J;
+#pragma unroll
+      for (int i = half; i < half + 4; ++i) acc[i][j] = mma(now.w[i], __builtin_bit_cast(bf16x8, now.x[j].b[piece]), acc[i][j]);
+      if (g < 2)
+#pragma unroll
+        for (int i = half; i < half + 4; ++i) read_w(buf, i, next);
+      if (pair >= 0) split_pair(x[pair / 4], pair % 4, next.x[pair / 4]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (g < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (pair >= 0) __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  Operands p, q;
+#pragma unroll
+  for (int i = 0; i < R; ++i) stage(min(i, n - 1), lds + i * STAGE);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * (R - 1)) : "memory");
+  lds_barrier();
+  {
+    f32x8 x[J];
+    read_x(lds, x);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) read_w(lds, i, p);
+#pragma unroll
+    for (int i = 0; i < 4 * J; ++i) split_pair(x[i / 4], i % 4, p.x[i / 4]);
+  }
+  for (int kt = 0; kt < n; kt += 2) {  // (n is even)
+    step(kt, p, q);
+    step(kt + 1, q, p);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (own >= n_rows) return;
+  // Three pieces stand for the activation while everything is finite: an infinity's rest is no number, and neither is a zero rest times an
+  // infinite weight.  A wave with a sum that is not finite adds its tiles up again.
+  float bad = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad = fmaf(acc[i][j][e], 0.f, bad);
+  if (__any(bad != bad)) {
+#pragma unroll 1
+    for (int i = 0; i < 8; i += 2) direct_tile<EPI>(a, gather, row0, min(n_rows, own + 16 * J), f0, rt0 + i, own, k0, k1);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int r = own + j * 16 + (lane & 15);
+    if (r >= n_rows) continue;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int rt = rt0 + i;
       if (rt >= a.rt) continue;
       if constexpr (EPI == LIN_GLU) {
-        if (!(i & 1)) store_glu<T>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[i][j], acc[i | 1][j]);
+        if (!(i & 1)) store_glu<float>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[i][j], acc[i | 1][j]);
       } else {
-        store_plain<T, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+        store_plain<float, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
       }
     }
   }
@@ -376,16 +417,23 @@ DEV void wide_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
     }
   }
 }
-template <typename T, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 128, per = part_tiles(a), k0 = blockIdx.y * per;
   a.out_f += blockIdx.y * a.part_stride;
-  lin_body<T, EPI>(a, nullptr, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
+  lin_body<EPI>(a, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
+}
+template <int J, int EPI>
+__global__ __launch_bounds__(256, 4 - J) void rows_kernel(LinArgs a, const int row_tiles, const int tiles) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 64 * J, per = part_tiles(a), k0 = blockIdx.y * per;
+  a.out_f += blockIdx.y * a.part_stride;
+  rows_body<J, EPI>(a, nullptr, row0, min(64 * J, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
 }
 
 // LinArgs.direct: products of a few k tiles (the decay of time mixing: two), 64 features x 64 rows per workgroup.  Three pieces have nothing to save
-// there, latency and the output bound it: 2048 features of 1996 rows 12.4 us, of 301 rows 8.0 (in three pieces by lin_kernel's tiles 21.6 and 9.6, by
+// there, latency and the output bound it: 2048 features of 1996 rows 12.4 us, of 301 rows 8.0 (in three pieces by tiles of 128 x 128 21.6 and 9.6, by
 // its tiles with this instruction 24.8 and 11.6; waves of 64 x 64 with the whole k in one straight line 24.5 and 21.7).  And a sum is one chain, as in
 // few_body: in bfloat16 runs another rounding of the decay turns roundings behind it.
 __global__ __launch_bounds__(256) void lin_direct_kernel(const LinArgs a, const int row_tiles, const int tiles) {
@@ -608,7 +656,8 @@ __global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs
     else if (rows > 32) wide_body<4, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
     else wide_body<2, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
   } else {
-    lin_body<T, EPI>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
+    if (rows > 64) rows_body<2, EPI>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
+    else rows_body<1, EPI>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
   }
 }
 
@@ -737,7 +786,6 @@ __global__ __launch_bounds__(256) void few_kernel(const FewArgs f) {
 }
 
 // ---- launches ------------------------------------------------------------------------------------
-static int lin_lds(bool f32) { return lin_stages(f32 ? 4 : 2) * lin_stage(f32 ? 4 : 2); }
 static int check_lin(const LinArgs& a, const char* what) {
   if (!a.w || !a.a_t || a.rows < 1 || a.kt < 2 || (a.kt & 1) || a.rt < 1 || a.lda < a.kt * 32) DSK_FAIL(DSK_ERR_INVALID, "%s: rows %d kt %d rt %d lda %d", what, a.rows, a.kt, a.rt, a.lda);
   if (a.parts > 1 && (a.n_wide || a.epi != LIN_STORE || part_tiles(a) * (a.parts - 1) >= a.kt)) DSK_FAIL(DSK_ERR_INVALID, "%s: %d parts of %d", what, a.parts, a.kt);
@@ -755,36 +803,44 @@ static int allow_lds(K k, int bytes) {
 // takes 1.17 us, and 1.55 when all of them run (the card's clock).  Both start and end in 3 and 8 us; a part more writes and reads its sums.
 // Stretches (LinStream) leave no compute unit empty, but their rows and weights meet in L2 less often (1.72 us), and tiles that they cut are stored and read:
 // 2000 rows and 2048 x 16896 145 us, by 128 x 128 163, by 256 x 256 168; 7168 x 32896 803, 1066, 895; but 1500 rows and 7168 x 27648 550, 658, 541.
-// In 32 bits a step of 64 columns takes 1.48 us alone, 2.6 - 3 us of two.
-enum { LIN_SMALL, LIN_BIG, LIN_STREAM };
+// In 32 bits a step of 64 columns takes a workgroup of 128 rows alone 1.08 us, two of them 2.45, and one of 64 rows 0.64, three of them 1.96 (us by 128 and
+// by 64 rows: 301 rows and 2048 x 16896 78 and 62, 2000 rows 347 and 365; 301 rows and 2048 x 2176 40 and 25).
+enum { LIN_SMALL, LIN_HALF, LIN_BIG, LIN_STREAM };  // (the second: 64 rows instead of 128, 32 bits)
 static int lin_streams(int rows, int rt) {  // stretches of a row of 256 x 256 tiles; 0: they would cut a tile more than once
   const int n = 256 / cdiv(rows, 256);
   return n >= 2 && n <= cdiv(rt, 16) ? n : 0;
 }
 static double lin_cost(int rows, int rt, int kt, int parts, int kind, bool f32) {
   const double k = part_tiles(kt, parts) / 2, sums = (parts - 1) * 3.2e-5 * rows * rt;
-  if (kind != LIN_SMALL && f32) return 1e9;
+  if (f32 ? kind > LIN_HALF : kind == LIN_HALF) return 1e9;
   if (kind == LIN_STREAM) {
     const int n = lin_streams(rows, rt);
     return n && parts == 1 ? 32 + 1.72 * k * cdiv(rt, 16) / n : 1e9;
+  }
+  if (f32) {  // rounds of as many workgroups as compute units have room for, and what the last one leaves empty
+    const bool half = kind == LIN_HALF;
+    const int n = cdiv(rows, half ? 64 : 128) * cdiv(rt, 8) * parts, at_once = half ? 768 : 512;
+    const double r = n % at_once / 256.;
+    const double rest = r == 0 ? 0 : half ? (r <= 1 ? 0.64 : (r <= 2 ? 0.72 : 1.) + 0.32 * r) : r <= 1 ? 1.08 : 1.75 + 0.35 * r;
+    return 3 + (n / at_once * (half ? 1.96 : 2.45) + rest) * k + sums;
   }
   if (kind == LIN_BIG) {
     const int n = cdiv(rows, 256) * cdiv(rt, 16) * parts, rest = n % 256;
     return n / 256 * (8 + 1.55 * k) + (rest ? 8 + (1.17 + 0.38 / 256 * rest) * k : 0) + sums;
   }
   const int n = cdiv(rows, 128) * cdiv(rt, 8) * parts, rest = n % 512;
-  if (f32) return 3 + (n <= 256 ? 1.48 : 1.6 + 1.9 / 512 * n) * k + sums;
   return 3 + (n / 512 * 1.08 + (rest == 0 ? 0 : rest <= 256 ? 0.85 : 1.0)) * k + sums;
 }
 static int lin_kind(int rows, int rt, int kt, int parts, bool f32) {
   int best = LIN_SMALL;
-  for (int kind : {LIN_BIG, LIN_STREAM})
+  for (int kind : {LIN_HALF, LIN_BIG, LIN_STREAM})
     if (lin_cost(rows, rt, kt, parts, kind, f32) < lin_cost(rows, rt, kt, parts, best, f32)) best = kind;
   return best;
 }
 static int lin_kind(const LinArgs& a, int parts, bool f32, const LinSpace& space) {
-  if (f32 || (a.a_seg & 255)) return LIN_SMALL;
+  if (!f32 && (a.a_seg & 255)) return LIN_SMALL;
   int kind = lin_kind(a.rows, a.rt, a.kt, parts, f32);
+  if (f32) return kind;
   if (a.tile) kind = a.tile == 128 ? LIN_SMALL : parts == 1 && lin_streams(a.rows, a.rt) ? LIN_STREAM : LIN_BIG;
   return kind == LIN_STREAM && space.slots < LIN_SLOTS ? LIN_BIG : kind;
 }
@@ -815,7 +871,7 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32, const LinSpace& space
   DSK_TRY(check_lin(a, "lin"));
   if ((a.a_seg & 127) || a.row_seq || a.out_at) DSK_FAIL(DSK_ERR_INVALID, "lin: %d features per operand", a.a_seg);
   const int kind = lin_kind(a, std::max(a.parts, 1), f32, space);
-  if (kind != LIN_SMALL) {
+  if (kind > LIN_HALF) {
     const int row_tiles = cdiv(a.rows, 256), tiles = row_tiles * cdiv(a.rt, 16);
     const LinStream ls{kind == LIN_STREAM ? lin_streams(a.rows, a.rt) : 0, space.sums, space.pieces};
     auto k = LIN_EPI(lin_big_kernel, );
@@ -829,11 +885,12 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32, const LinSpace& space
     hipLaunchKernelGGL(lin_direct_kernel, dim3(tiles), dim3(256), 0, st, a, row_tiles, tiles);
     return DSK_OK;
   }
-  const int row_tiles = cdiv(a.rows, 128), tiles = row_tiles * cdiv(a.rt, 8), lds = lin_lds(f32);
+  const int high = kind == LIN_HALF ? 64 : 128, row_tiles = cdiv(a.rows, high), tiles = row_tiles * cdiv(a.rt, 8);
+  const int lds = !f32 ? (int)LIN_LDS : ROWS_RING * (kind == LIN_HALF ? rows_stage<1>() : rows_stage<2>());
   const dim3 grid(tiles, std::max(a.parts, 1));
-#define LIN_F32 float,
-#define LIN_BF16 bf16,
-  auto k = f32 ? LIN_EPI(lin_kernel, LIN_F32) : LIN_EPI(lin_kernel, LIN_BF16);
+#define LIN_J1 1,
+#define LIN_J2 2,
+  auto k = !f32 ? LIN_EPI(lin_kernel, ) : kind == LIN_HALF ? LIN_EPI(rows_kernel, LIN_J1) : LIN_EPI(rows_kernel, LIN_J2);
   DSK_TRY(allow_lds(k, lds));
   hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, row_tiles, tiles);
   return DSK_OK;
@@ -843,7 +900,7 @@ int launch_experts(hipStream_t st, const MoeArgs& m, bool down, bool f32) {
   const ExpertMat& e = down ? m.down : m.up;
   const int shared_tiles = m.shared ? cdiv(m.rows, MOE_TILE) : 0, ft = f32 ? 8 : 16;
   const dim3 grid((m.max_tiles - shared_tiles) * cdiv(e.rt, ft) + ((shared_tiles * cdiv(e.shared_rt, ft) + 7) & ~7));
-  const int lds = f32 ? lin_lds(f32) : 2 * wide_stage<8>();
+  const int lds = f32 ? ROWS_RING * rows_stage<2>() : 2 * wide_stage<8>();
   auto k = f32 ? (down ? expert_kernel<float, true> : expert_kernel<float, false>) : (down ? expert_kernel<bf16, true> : expert_kernel<bf16, false>);
   DSK_TRY(allow_lds(k, lds));
   hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, m, shared_tiles);

@@ -59,32 +59,25 @@ DEV f32x4 mma(const f32x8& w, const f32x8& a, f32x4 c) {
 // that each rest is exact; b2 alone can fall under the smallest bf16, below 2^-110).  A product with a finite bf16 weight is then three bf16
 // products, each exact in 32 bits and summed in 32 bits: the precision of v_mfma_f32_16x16x4_f32 at a fifth of its cycles (three
 // 16x16x32 of 16 cycles for eight of 32).  Where an activation or a weight is not finite the sum of the three is no finite number either,
-// but not always the right one: such sums are added up again by that instruction (lin_body).
+// but not always the right one: such sums are added up again by that instruction (rows_body).
+typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
 struct Split {
-  bf16x8 b0, b1, b2;
+  u32x4v b[3];  // eight bf16 each
 };
-DEV Split split3(const f32x8& x) {
-  typedef unsigned u32x8 __attribute__((ext_vector_type(8)));
-  typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
-  u32x8 p0, p1, p2;
+DEV void split_pair(const f32x8& x, int i, Split& o) {  // elements 2 i and 2 i + 1
+  unsigned p[3][2];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float v = x[i];  // (a bit cast of an element of a vector reads element 0)
+  for (int e = 0; e < 2; ++e) {
+    const float v = x[2 * i + e];  // (a bit cast of an element of a vector reads element 0)
     const unsigned bits = __builtin_bit_cast(unsigned, v);
     const float r = v - __builtin_bit_cast(float, bits & 0xffff0000u);  // (of an infinity or no number: no number)
     const unsigned rest = __builtin_bit_cast(unsigned, r);
-    p0[i] = bits;
-    p1[i] = rest;
-    p2[i] = __builtin_bit_cast(unsigned, r - __builtin_bit_cast(float, rest & 0xffff0000u));
+    p[0][e] = bits;
+    p[1][e] = rest;
+    p[2][e] = __builtin_bit_cast(unsigned, r - __builtin_bit_cast(float, rest & 0xffff0000u));
   }
-  u32x4v o0, o1, o2;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {  // the high halves of two words
-    o0[i] = __builtin_amdgcn_perm(p0[2 * i + 1], p0[2 * i], 0x07060302);
-    o1[i] = __builtin_amdgcn_perm(p1[2 * i + 1], p1[2 * i], 0x07060302);
-    o2[i] = __builtin_amdgcn_perm(p2[2 * i + 1], p2[2 * i], 0x07060302);
-  }
-  return {__builtin_bit_cast(bf16x8, o0), __builtin_bit_cast(bf16x8, o1), __builtin_bit_cast(bf16x8, o2)};
+  for (int k = 0; k < 3; ++k) o.b[k][i] = __builtin_amdgcn_perm(p[k][1], p[k][0], 0x07060302);  // the high halves of two words
 }
 
 // A block of 16 rows x 32 columns on its way from row-major memory to operands: loaded row by row, four lanes to a row, lane l's 8 columns
