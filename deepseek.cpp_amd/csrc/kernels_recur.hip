@@ -11,32 +11,44 @@
 
 #include <math.h>
 
+#include <algorithm>
+#include <type_traits>
+
 static int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // ---- delta rule: what enters the recurrence -----------------------------------------------------------
 // A wave takes one unit for the (up to 16) rows of a chunk: a q or k head (short causal convolution, silu, unit norm), a v head
-// (convolution, silu) or a head's decays and step sizes.  Lanes are channels; TAPS = 0: any number of taps, else that many in registers.
-template <typename T, int TAPS>
+// (convolution, silu) or 64 of a head's decays, and its step sizes.  Lanes are channels; TAPS = 0: any number of taps, else that many in registers.
+// 64 NI channels hold the larger head.  Everything is requested at once, from places that are always there, and what doesn't belong is dropped behind:
+// behind a branch the compiler waits for each load.  2048 rows of 16 heads of 128 (107 MB) 64 us before, 42 so.
+template <typename T, int TAPS, int NI>
 __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaArgs a) {
-  constexpr int NI = RECUR_MAX_DIM / 64, R = RECUR_CHUNK;
-  const int lane = threadIdx.x & 63, unit = blockIdx.y * 4 + (threadIdx.x >> 6);
+  constexpr int R = RECUR_CHUNK;
+  const int lane = threadIdx.x & 63, unit = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int nq = a.kv_heads * a.dim, nv = a.heads * a.vdim, C = 2 * nq + nv, taps = TAPS ? TAPS : a.taps;
-  if (unit >= 2 * a.kv_heads + 2 * a.heads) return;
+  if (unit >= 2 * a.kv_heads + (1 + NI) * a.heads) return;
   const SeqDesc sq = seq_at(a.p.seqs + a.p.chunk[2 * blockIdx.x]);
   const int t0 = a.p.chunk[2 * blockIdx.x + 1], n_rows = min(R, sq.len - t0);
   const size_t row0 = (size_t)sq.row0 + t0;
   if (unit >= 2 * a.kv_heads + a.heads) {
-    const int h = unit - 2 * a.kv_heads - a.heads;
+    const int h = (unit - 2 * a.kv_heads - a.heads) / NI, part = (unit - 2 * a.kv_heads - a.heads) % NI;
     const float rate = a.a_rate[h];
     if (a.head_decay) {
-      if (lane < n_rows) a.g[(row0 + lane) * a.heads + h] = expf(-rate * softplus_f(a.gate_f[(row0 + lane) * a.ld_gate + a.col_a + h] + a.dt_bias[h]));
-    } else for (int i = lane; i < a.dim; i += 64) {
-      const float bias = a.dt_bias[h * a.dim + i];
-#pragma unroll 4
-      for (int t = 0; t < n_rows; ++t)
-        a.g[((row0 + t) * a.heads + h) * a.dim + i] = expf(-rate * softplus_f(a.low_f[(row0 + t) * a.ld_low + h * a.dim + i] + bias));
+      if (part == 0 && lane < n_rows) a.g[(row0 + lane) * a.heads + h] = expf(-rate * softplus_f(a.gate_f[(row0 + lane) * a.ld_gate + a.col_a + h] + a.dt_bias[h]));
+    } else {
+      const int d = lane + 64 * part, c = h * a.dim + min(d, a.dim - 1);
+      const float bias = a.dt_bias[c];
+      float low[R];
+#pragma unroll
+      for (int t = 0; t < R; ++t) low[t] = a.low_f[(row0 + min(t, n_rows - 1)) * a.ld_low + c];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        const float g = expf(-rate * softplus_f(low[t] + bias));
+        if (t < n_rows && d < a.dim) a.g[(row0 + t) * a.heads * a.dim + c] = g;
+      }
     }
-    if (lane < n_rows) a.beta[(row0 + lane) * a.heads + h] = sigmoid_f(a.gate_f[(row0 + lane) * a.ld_gate + a.col_b + h]);
+    if (part == 0 && lane < n_rows) a.beta[(row0 + lane) * a.heads + h] = sigmoid_f(a.gate_f[(row0 + lane) * a.ld_gate + a.col_b + h]);
     return;
   }
   const bool is_v = unit >= 2 * a.kv_heads, is_q = unit < a.kv_heads;
@@ -52,33 +64,53 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaArgs a) {
   float y[NI][R], ss[R];
 #pragma unroll
   for (int t = 0; t < R; ++t) ss[t] = 0.f;
+  if constexpr (TAPS > 0) {
+    constexpr int K = TAPS - 1;  // rows in front of the chunk
+    T x[NI][R + K];
+    float old[NI][K], w[NI][TAPS];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int c = lane + 64 * i;
+    for (int i = 0; i < NI; ++i) {
+      const int c = min(lane + 64 * i, n - 1);
 #pragma unroll
-    for (int t = 0; t < R; ++t) y[i][t] = 0.f;
-    if (c >= n) continue;
-    const float* w = a.conv_w + (size_t)(c0 + c) * taps;
-    if constexpr (TAPS > 0) {
-      float x[R + TAPS - 1];
+      for (int r = 0; r < R + K; ++r) x[i][r] = P[(size_t)min(max(t0 - K + r, 0), sq.len - 1) * a.ld + c];
 #pragma unroll
-      for (int r = 0; r < R + TAPS - 1; ++r) x[r] = input(min(t0 - (TAPS - 1) + r, sq.len - 1), c);
+      for (int r = 0; r < K; ++r) old[i][r] = hist[(size_t)r * C + c];
 #pragma unroll
-      for (int t = 0; t < R; ++t)
-#pragma unroll
-        for (int j = 0; j < TAPS; ++j) y[i][t] += x[t + j] * w[j];
-    } else {
-#pragma unroll
-      for (int t = 0; t < R; ++t)
-        if (t < n_rows)
-          for (int j = 0; j < taps; ++j) y[i][t] += input(t0 + t - (taps - 1) + j, c) * w[j];
+      for (int j = 0; j < TAPS; ++j) w[i][j] = a.conv_w[(size_t)(c0 + c) * TAPS + j];
     }
+    __builtin_amdgcn_sched_barrier(0);  // (all on their way first)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      float in[R + K];
+#pragma unroll
+      for (int r = 0; r < R + K; ++r) in[r] = r >= K || t0 - K + r >= 0 ? (float)x[i][r] : t0 == 0 && sq.pos0 - K + r >= 0 ? old[i][r] : 0.f;
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        y[i][t] = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) y[i][t] += in[t + j] * w[i][j];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int c = lane + 64 * i;
+      const float* w = a.conv_w + (size_t)(c0 + c) * taps;
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        y[i][t] = 0.f;
+        if (t < n_rows && c < n)
+          for (int j = 0; j < taps; ++j) y[i][t] += input(t0 + t - (taps - 1) + j, c) * w[j];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int t = 0; t < R; ++t) {
       y[i][t] = silu_f(y[i][t]);
-      ss[t] += y[i][t] * y[i][t];
+      ss[t] += lane + 64 * i < n ? y[i][t] * y[i][t] : 0.f;
     }
-  }
   float* dst = is_v ? a.v + row0 * nv + c0 - 2 * nq : is_q ? a.q + row0 * nq + c0 : a.k + row0 * nq + c0 - nq;
   const int ld = is_v ? nv : nq;
 #pragma unroll
@@ -88,21 +120,48 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaArgs a) {
     for (int i = 0; i < NI; ++i)
       if (t < n_rows && lane + 64 * i < n) dst[(size_t)t * ld + lane + 64 * i] = y[i][t] * r;
   }
-  if (t0 + n_rows == sq.len) {  // the portion's end: keep the inputs of its last taps - 1 tokens, in the other copy
-    float* next = reinterpret_cast<float*>(sq.state + a.off_conv) + (size_t)(sq.flip ^ 1) * (taps - 1) * C + c0;
+  if (t0 + n_rows < sq.len) return;
+  // the portion's end: keep the inputs of its last taps - 1 tokens, in the other copy
+  float* next = reinterpret_cast<float*>(sq.state + a.off_conv) + (size_t)(sq.flip ^ 1) * (taps - 1) * C + c0;
+  if constexpr (TAPS > 0) {
+    constexpr int K = TAPS - 1;
+    float in[NI][K], old[NI][K];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+        const int c = min(lane + 64 * i, n - 1), u = sq.len - K + j;
+        in[i][j] = (float)P[(size_t)max(u, 0) * a.ld + c];
+        old[i][j] = hist[(size_t)min(max(u + K, 0), K - 1) * C + c];
+      }
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+        const int u = sq.len - K + j;
+        if (lane + 64 * i < n) next[(size_t)j * C + lane + 64 * i] = u >= 0 ? in[i][j] : sq.pos0 + u >= 0 ? old[i][j] : 0.f;
+      }
+  } else {
     for (int j = 0; j < taps - 1; ++j)
       for (int c = lane; c < n; c += 64) next[(size_t)j * C + c] = input(sq.len - (taps - 1) + j, c);
   }
 }
+template <typename T, int NI>
+static void delta_prep_n(hipStream_t st, const DeltaArgs& a) {
+  const dim3 grid(a.p.n_chunks, cdiv(2 * a.kv_heads + (1 + NI) * a.heads, 4));
+  switch (a.taps) {
+    case 2: hipLaunchKernelGGL((delta_prep_kernel<T, 2, NI>), grid, dim3(256), 0, st, a); break;
+    case 3: hipLaunchKernelGGL((delta_prep_kernel<T, 3, NI>), grid, dim3(256), 0, st, a); break;
+    case 4: hipLaunchKernelGGL((delta_prep_kernel<T, 4, NI>), grid, dim3(256), 0, st, a); break;
+    default: hipLaunchKernelGGL((delta_prep_kernel<T, 0, NI>), grid, dim3(256), 0, st, a);
+  }
+}
 template <typename T>
 static void delta_prep_t(hipStream_t st, const DeltaArgs& a) {
-  const dim3 grid(a.p.n_chunks, cdiv(2 * a.kv_heads + 2 * a.heads, 4));
-  switch (a.taps) {
-    case 2: hipLaunchKernelGGL((delta_prep_kernel<T, 2>), grid, dim3(256), 0, st, a); break;
-    case 3: hipLaunchKernelGGL((delta_prep_kernel<T, 3>), grid, dim3(256), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((delta_prep_kernel<T, 4>), grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((delta_prep_kernel<T, 0>), grid, dim3(256), 0, st, a);
-  }
+  const int n = std::max(a.dim, a.vdim);
+  if (n <= 64) delta_prep_n<T, 1>(st, a);
+  else if (n <= 128) delta_prep_n<T, 2>(st, a);
+  else delta_prep_n<T, 4>(st, a);
 }
 int launch_delta_prep(hipStream_t st, const DeltaArgs& a, bool f32) {
   if (a.dim > RECUR_MAX_DIM || a.vdim > RECUR_MAX_DIM) DSK_FAIL(DSK_ERR_UNSUPPORTED, "delta: key size %d, value size %d (max %d)", a.dim, a.vdim, (int)RECUR_MAX_DIM);
@@ -239,58 +298,88 @@ int launch_delta_scan(hipStream_t st, const DeltaArgs& a) {
 }
 
 // ---- behind a recurrence: per-head RMS norm, weight, gate ---------------------------------------------
-// value(h, i): element i of head h; gate(c): the factor; w[c or i]: by place among all heads or inside one
-template <typename T, typename V, typename G>
-DEV void head_norm_gate(V value, int heads, int vdim, float eps, const float* w, bool shared_w, G gate, T* out) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int h = wave; h < heads; h += 4) {
-    float v[RECUR_MAX_DIM / 64], ss = 0.f;
+// value(h, i): element i of head h, gate(c) a factor's input and act() the factor; w[c or i]: by place among all heads or inside one.  64 NI elements hold a
+// head.  A wave requests all of HU heads at once, from places that are always there: 1996 rows of 32 heads of 64 (wkv) 18.5 us with a head at a time and
+// the gate behind the norm, 15.9 so; 16 heads of 128 (delta rule) 16.2 and 13.1;
+// 301 rows in 32 bits 9.9 and 6.0, 8.5 and 5.6.
+template <typename T, int NI, typename V, typename G, typename A>
+DEV void head_norm_gate(V value, int heads, int vdim, float eps, const float* w, bool shared_w, G gate, A act, T* out) {
+  constexpr int HU = NI < 4 ? 4 / NI : 1;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  for (int h0 = wave; h0 < heads; h0 += 4 * HU) {
+    float v[HU][NI], g[HU][NI], weight[HU][NI];
 #pragma unroll
-    for (int i = 0; i < RECUR_MAX_DIM / 64; ++i) {
-      v[i] = lane + 64 * i < vdim ? value(h, lane + 64 * i) : 0.f;
-      ss += v[i] * v[i];
-    }
-    const float r = 1.f / sqrtf(wave_sum(ss) / vdim + eps);
+    for (int u = 0; u < HU; ++u)
 #pragma unroll
-    for (int i = 0; i < RECUR_MAX_DIM / 64; ++i) {
-      const int e = lane + 64 * i, c = h * vdim + e;
-      if (e < vdim) out[c] = (T)(v[i] * r * w[shared_w ? e : c] * gate(c));
+      for (int i = 0; i < NI; ++i) {
+        const int h = min(h0 + 4 * u, heads - 1), e = min(lane + 64 * i, vdim - 1);
+        v[u][i] = value(h, e);
+        g[u][i] = gate(h * vdim + e);
+        weight[u][i] = w[shared_w ? e : h * vdim + e];
+      }
+    __builtin_amdgcn_sched_barrier(0);  // (all on their way first)
+#pragma unroll
+    for (int u = 0; u < HU; ++u) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if (lane + 64 * i >= vdim) v[u][i] = 0.f;
+        ss += v[u][i] * v[u][i];
+      }
+      const float r = 1.f / sqrtf(wave_sum(ss) / vdim + eps);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        if (h0 + 4 * u < heads && lane + 64 * i < vdim) out[(h0 + 4 * u) * vdim + lane + 64 * i] = (T)(v[u][i] * r * weight[u][i] * act(g[u][i]));
     }
   }
 }
-template <typename T>
+template <typename K>
+static int head_sizes(int vdim, K launch) {
+  if (vdim <= 64) return launch(std::integral_constant<int, 1>());
+  if (vdim <= 128) return launch(std::integral_constant<int, 2>());
+  return launch(std::integral_constant<int, 4>());
+}
+template <typename T, int NI>
 __global__ __launch_bounds__(256) void delta_out_kernel(const DeltaArgs a) {
   const size_t row = blockIdx.x;
   const float *gl = a.low_f + row * a.ld_low + (size_t)a.heads * a.dim, *o = a.o + row * a.heads * a.vdim;
   const T* gp = reinterpret_cast<const T*>(a.proj_t) + row * a.ld + a.col_g;
-  head_norm_gate<T>([&](int h, int i) { return o[h * a.vdim + i]; }, a.heads, a.vdim, a.eps, a.out_norm, true,
-                    [&](int c) { return a.silu_gate ? silu_f((float)gp[c]) : sigmoid_f(gl[c]); }, reinterpret_cast<T*>(a.out_t) + row * a.out_ld);
+  T* out = reinterpret_cast<T*>(a.out_t) + row * a.out_ld;
+  auto value = [&](int h, int i) { return o[h * a.vdim + i]; };
+  if (a.silu_gate) head_norm_gate<T, NI>(value, a.heads, a.vdim, a.eps, a.out_norm, true, [&](int c) { return (float)gp[c]; }, [](float g) { return silu_f(g); }, out);
+  else head_norm_gate<T, NI>(value, a.heads, a.vdim, a.eps, a.out_norm, true, [&](int c) { return gl[c]; }, [](float g) { return sigmoid_f(g); }, out);
 }
 int launch_delta_out(hipStream_t st, const DeltaArgs& a, bool f32) {
-  if (f32) hipLaunchKernelGGL(delta_out_kernel<float>, dim3(a.p.rows), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(delta_out_kernel<bf16>, dim3(a.p.rows), dim3(256), 0, st, a);
-  return DSK_OK;
+  return head_sizes(a.vdim, [&](auto ni) -> int {
+    constexpr int NI = decltype(ni)::value;
+    if (f32) hipLaunchKernelGGL((delta_out_kernel<float, NI>), dim3(a.p.rows), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((delta_out_kernel<bf16, NI>), dim3(a.p.rows), dim3(256), 0, st, a);
+    return DSK_OK;
+  });
 }
-template <typename T, bool RAW>
+template <typename T, bool RAW, int NI>
 __global__ __launch_bounds__(256) void mlstm_out_kernel(const MlstmArgs a, const float* __restrict__ floor_) {
   const size_t row = blockIdx.x;
   const int ld = RAW ? a.vdim + 1 : a.vdim;
   const float* o = a.o + row * a.heads * ld;
   const T* gl = reinterpret_cast<const T*>(a.proj_t) + row * a.ld + a.col_g;
-  head_norm_gate<T>([&](int h, int i) {
+  head_norm_gate<T, NI>([&](int h, int i) {
     const float v = o[h * ld + i];
     return RAW ? v / (fmaxf(fabsf(o[h * ld + a.vdim]), floor_[row * a.heads + h]) + a.floor_eps) : v;
-  }, a.heads, a.vdim, a.eps, a.out_norm, false, [&](int c) { return sigmoid_f((float)gl[c]); }, reinterpret_cast<T*>(a.out_t) + row * a.out_ld);
+  }, a.heads, a.vdim, a.eps, a.out_norm, false, [&](int c) { return (float)gl[c]; }, [](float g) { return sigmoid_f(g); }, reinterpret_cast<T*>(a.out_t) + row * a.out_ld);
 }
 int launch_mlstm_out(hipStream_t st, const MlstmArgs& a, const ChunkScan* c, bool f32) {
   if (a.vdim > RECUR_MAX_DIM) DSK_FAIL(DSK_ERR_UNSUPPORTED, "mlstm: value size %d (max %d)", a.vdim, (int)RECUR_MAX_DIM);
   const float* fl = c ? c->floor : nullptr;
-  const dim3 g(a.p.rows), b(256);
-  if (f32 && c) hipLaunchKernelGGL((mlstm_out_kernel<float, true>), g, b, 0, st, a, fl);
-  else if (f32) hipLaunchKernelGGL((mlstm_out_kernel<float, false>), g, b, 0, st, a, fl);
-  else if (c) hipLaunchKernelGGL((mlstm_out_kernel<bf16, true>), g, b, 0, st, a, fl);
-  else hipLaunchKernelGGL((mlstm_out_kernel<bf16, false>), g, b, 0, st, a, fl);
-  return DSK_OK;
+  return head_sizes(a.vdim, [&](auto ni) -> int {
+    constexpr int NI = decltype(ni)::value;
+    const dim3 g(a.p.rows), b(256);
+    if (f32 && c) hipLaunchKernelGGL((mlstm_out_kernel<float, true, NI>), g, b, 0, st, a, fl);
+    else if (f32) hipLaunchKernelGGL((mlstm_out_kernel<float, false, NI>), g, b, 0, st, a, fl);
+    else if (c) hipLaunchKernelGGL((mlstm_out_kernel<bf16, true, NI>), g, b, 0, st, a, fl);
+    else hipLaunchKernelGGL((mlstm_out_kernel<bf16, false, NI>), g, b, 0, st, a, fl);
+    return DSK_OK;
+  });
 }
 
 // ---- mLSTM: the scan ---------------------------------------------------------------------------------
@@ -517,16 +606,19 @@ static int wkv_t(hipStream_t st, const WkvArgs& a) {
   }, "wkv");
 }
 int launch_wkv_scan(hipStream_t st, const WkvArgs& a, bool f32) { return f32 ? wkv_t<float>(st, a) : wkv_t<bf16>(st, a); }
-template <typename T>
+template <typename T, int NI>
 __global__ __launch_bounds__(256) void wkv_out_kernel(const WkvArgs a) {
   const size_t row = blockIdx.x;
   const float* o = a.o + row * a.heads * a.dim;
   const T* gp = reinterpret_cast<const T*>(a.proj_t) + row * a.ld + a.col_g;
-  head_norm_gate<T>([&](int h, int i) { return o[h * a.dim + i]; }, a.heads, a.dim, a.eps, a.out_norm, false, [&](int c) { return silu_f((float)gp[c]); },
-                    reinterpret_cast<T*>(a.out_t) + row * a.out_ld);
+  head_norm_gate<T, NI>([&](int h, int i) { return o[h * a.dim + i]; }, a.heads, a.dim, a.eps, a.out_norm, false, [&](int c) { return (float)gp[c]; },
+                        [](float g) { return silu_f(g); }, reinterpret_cast<T*>(a.out_t) + row * a.out_ld);
 }
 int launch_wkv_out(hipStream_t st, const WkvArgs& a, bool f32) {
-  if (f32) hipLaunchKernelGGL(wkv_out_kernel<float>, dim3(a.p.rows), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(wkv_out_kernel<bf16>, dim3(a.p.rows), dim3(256), 0, st, a);
-  return DSK_OK;
+  return head_sizes(a.dim, [&](auto ni) -> int {
+    constexpr int NI = decltype(ni)::value;
+    if (f32) hipLaunchKernelGGL((wkv_out_kernel<float, NI>), dim3(a.p.rows), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((wkv_out_kernel<bf16, NI>), dim3(a.p.rows), dim3(256), 0, st, a);
+    return DSK_OK;
+  });
 }
