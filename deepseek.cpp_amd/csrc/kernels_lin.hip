@@ -250,7 +250,6 @@ DEV void rows_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
     // tile kt + 1 is here when at most the loads of R - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
     // tile kt in registers, so that its buffer takes tile kt + R (past the end: the last one again, never read)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * (R - 2)) : "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), which the barrier waits for: so that the compiler knows and the first products wait for no reads
     lds_barrier();
     stage(min(kt + R, n - 1), lds + cur * STAGE);
     cur = cur + 1 == R ? 0 : cur + 1;
@@ -803,7 +802,7 @@ static int allow_lds(K k, int bytes) {
 // takes 1.17 us, and 1.55 when all of them run (the card's clock).  Both start and end in 3 and 8 us; a part more writes and reads its sums.
 // Stretches (LinStream) leave no compute unit empty, but their rows and weights meet in L2 less often (1.72 us), and tiles that they cut are stored and read:
 // 2000 rows and 2048 x 16896 145 us, by 128 x 128 163, by 256 x 256 168; 7168 x 32896 803, 1066, 895; but 1500 rows and 7168 x 27648 550, 658, 541.
-// In 32 bits a step of 64 columns takes a workgroup of 128 rows alone 1.08 us, two of them 2.45, and one of 64 rows 0.64, three of them 1.96 (us by 128 and
+// In 32 bits a step of 64 columns takes a workgroup of 128 rows alone 1.08 us (1.5 with weights out of HBM), two of them 2.45, and one of 64 rows 0.64, three of them 1.96 (us by 128 and
 // by 64 rows: 301 rows and 2048 x 16896 78 and 62, 2000 rows 347 and 365; 301 rows and 2048 x 2176 40 and 25).
 enum { LIN_SMALL, LIN_HALF, LIN_BIG, LIN_STREAM };  // (the second: 64 rows instead of 128, 32 bits)
 static int lin_streams(int rows, int rt) {  // stretches of a row of 256 x 256 tiles; 0: they would cut a tile more than once
@@ -821,7 +820,7 @@ static double lin_cost(int rows, int rt, int kt, int parts, int kind, bool f32) 
     const bool half = kind == LIN_HALF;
     const int n = cdiv(rows, half ? 64 : 128) * cdiv(rt, 8) * parts, at_once = half ? 768 : 512;
     const double r = n % at_once / 256.;
-    const double rest = r == 0 ? 0 : half ? (r <= 1 ? 0.64 : (r <= 2 ? 0.72 : 1.) + 0.32 * r) : r <= 1 ? 1.08 : 1.75 + 0.35 * r;
+    const double rest = r == 0 ? 0 : half ? (r <= 1 ? 0.64 : (r <= 2 ? 0.72 : 1.) + 0.32 * r) : r <= 1 ? 1.3 : 1.75 + 0.35 * r;
     return 3 + (n / at_once * (half ? 1.96 : 2.45) + rest) * k + sums;
   }
   if (kind == LIN_BIG) {

@@ -93,7 +93,12 @@ DEV typename Frag<T>::four to_four(const f32x4& v) {
 }
 
 // a barrier for LDS traffic only: global loads and stores stay in flight across it (__syncthreads drains them)
-DEV void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// The wait is stated twice: the compiler does not know of the one inside the assembly, and without the first it makes the first instruction that uses
+// what was read in front of the barrier wait for everything that is read behind it.
+DEV void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
 
 DEV float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
 DEV float silu_f(float x) { return x * sigmoid_f(x); }
