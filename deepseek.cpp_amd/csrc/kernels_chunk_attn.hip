@@ -61,32 +61,34 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(const ChunkAttnArgs a) 
 }
 
 // ---- attention -----------------------------------------------------------------------------------------
-// keys and values of one head: the portion's from the workspace, older ones of the same chunk from the sequence's cache
+// Keys and values of one head: the portion's from the workspace, older ones of the same chunk from the sequence's cache.  Both are rows of one length, so
+// that a position's address is one of two starts and a multiple of it (found by a division behind a branch, each of a tile's loads was waited for by itself).
 template <typename T>
 struct ChunkKeys {
   typedef typename Frag<T>::type frag;
   typedef typename Frag<T>::four four;
   const ChunkAttnArgs& a;
   const SeqDesc& s;
-  int h, g;
+  int h;
+  const T *k_new, *k_old, *v_new, *v_old;  // of position 0, were it there
+  DEV ChunkKeys(const ChunkAttnArgs& a, const SeqDesc& s, int h) : a(a), s(s), h(h) {
+    const int g = h / (a.heads / a.kv_heads);
+    const ptrdiff_t fresh = (ptrdiff_t)s.row0 - s.pos0, kept = -(ptrdiff_t)first(s.pos0);
+    k_new = reinterpret_cast<const T*>(a.k_t) + (fresh * a.kv_heads + g) * a.dim_p;
+    v_new = reinterpret_cast<const T*>(a.v_t) + (fresh * a.kv_heads + g) * a.vdim_p;
+    k_old = reinterpret_cast<const T*>(s.state + a.off_k) + (kept * a.kv_heads + g) * a.dim_p;
+    v_old = reinterpret_cast<const T*>(s.state + a.off_v) + (kept * a.kv_heads + g) * a.vdim_p;
+  }
   DEV int first(int pos) const { return pos / a.chunk * a.chunk; }
   DEV frag q(int row, int gr) const { return *reinterpret_cast<const frag*>(reinterpret_cast<const T*>(a.q_t) + ((size_t)(s.row0 + row) * a.heads + h) * a.dim_p + gr * 8); }
-  DEV frag k(int pos, int gr) const {
-    const T* p = pos >= s.pos0 ? reinterpret_cast<const T*>(a.k_t) + ((size_t)(s.row0 + pos - s.pos0) * a.kv_heads + g) * a.dim_p
-                               : reinterpret_cast<const T*>(s.state + a.off_k) + ((size_t)(pos % a.chunk) * a.kv_heads + g) * a.dim_p;
-    return *reinterpret_cast<const frag*>(p + gr * 8);
-  }
-  DEV four v(int pos, int c) const {
-    const T* p = pos >= s.pos0 ? reinterpret_cast<const T*>(a.v_t) + ((size_t)(s.row0 + pos - s.pos0) * a.kv_heads + g) * a.vdim_p
-                               : reinterpret_cast<const T*>(s.state + a.off_v) + ((size_t)(pos % a.chunk) * a.kv_heads + g) * a.vdim_p;
-    return *reinterpret_cast<const four*>(p + c);
-  }
+  DEV frag k(int pos, int gr) const { return *reinterpret_cast<const frag*>((pos >= s.pos0 ? k_new : k_old) + (size_t)pos * (a.kv_heads * a.dim_p) + gr * 8); }
+  DEV four v(int pos, int c) const { return *reinterpret_cast<const four*>((pos >= s.pos0 ? v_new : v_old) + (size_t)pos * (a.kv_heads * a.vdim_p) + c); }
 };
 template <typename T, int KT, int VTL>
 ATTN_KERNEL(T) void chunk_attn_kernel(const ChunkAttnArgs a) {
-  const int h = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;  // (a sequence's last tiles have the most keys: they start first)
+  const auto [tile, h] = attn_place(a.p.n_qtiles, a.heads);
   const SeqDesc s = seq_at(a.p.seqs + a.p.qtile[2 * tile]);
-  attn_tile<T, KT, VTL>(ChunkKeys<T>{a, s, h, h / (a.heads / a.kv_heads)}, s, a.p.qtile[2 * tile + 1], a.dim_p >> 5, a.vdim_p >> 4, a.vdim, a.scale,
+  attn_tile<T, KT, VTL>(ChunkKeys<T>(a, s, h), s, a.p.qtile[2 * tile + 1], a.dim_p >> 5, a.vdim_p >> 4, a.vdim, a.scale,
                         reinterpret_cast<T*>(a.out_t) + h * a.vdim, a.out_ld);
 }
 
@@ -120,7 +122,7 @@ static int attn_t(hipStream_t st, const ChunkAttnArgs& a) {
     constexpr int KT = decltype(kt)::value, VTL = decltype(vt)::value, lds = attn_tile_lds<T, KT, VTL>();
     auto k = chunk_attn_kernel<T, KT, VTL>;
     HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    hipLaunchKernelGGL(k, dim3(a.p.n_qtiles, a.heads), dim3(256), lds, st, a);
+    hipLaunchKernelGGL(k, dim3(a.p.n_qtiles * a.heads), dim3(256), lds, st, a);
     return (int)DSK_OK;
   }, "chunk attention");
 }

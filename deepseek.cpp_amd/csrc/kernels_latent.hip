@@ -148,27 +148,29 @@ struct LatentKeys {
   const LatentArgs& a;
   const SeqDesc& s;
   int h;
+  const T *key, *rot, *value;  // of position 0, were it there
+  DEV LatentKeys(const LatentArgs& a, const SeqDesc& s, int h) : a(a), s(s), h(h) {
+    const ptrdiff_t row = (ptrdiff_t)s.key0 + s.hist - s.pos0;
+    key = reinterpret_cast<const T*>(a.kv_t) + row * a.kv_ld + h * a.dim_p;
+    value = reinterpret_cast<const T*>(a.kv_t) + row * a.kv_ld + a.heads * a.dim_p + h * a.vdim_p;
+    rot = reinterpret_cast<const T*>(a.lat_t) + row * (a.rank_p + a.rot_p) + a.rank_p - a.dim_p;
+  }
   DEV int first(int pos) const { return max(0, pos - a.window + 1); }
-  DEV size_t key_row(int pos) const { return (size_t)(s.key0 + s.hist + pos - s.pos0); }
   DEV frag q(int row, int gr) const {
     return *reinterpret_cast<const frag*>(reinterpret_cast<const T*>(a.q_t) + (size_t)(s.row0 + row) * a.q_ld + (size_t)h * (a.dim_p + a.rot_p) + gr * 8);
   }
   DEV frag k(int pos, int gr) const {
-    const size_t r = key_row(pos);
-    const T* p = gr * 8 < a.dim_p ? reinterpret_cast<const T*>(a.kv_t) + r * a.kv_ld + (size_t)h * a.dim_p
-                                  : reinterpret_cast<const T*>(a.lat_t) + r * (a.rank_p + a.rot_p) + a.rank_p - a.dim_p;
-    return *reinterpret_cast<const frag*>(p + gr * 8);
+    const bool own = gr * 8 < a.dim_p;
+    return *reinterpret_cast<const frag*>((own ? key : rot) + (size_t)pos * (own ? a.kv_ld : a.rank_p + a.rot_p) + gr * 8);
   }
-  DEV four v(int pos, int c) const {
-    return *reinterpret_cast<const four*>(reinterpret_cast<const T*>(a.kv_t) + key_row(pos) * a.kv_ld + (size_t)a.heads * a.dim_p + (size_t)h * a.vdim_p + c);
-  }
+  DEV four v(int pos, int c) const { return *reinterpret_cast<const four*>(value + (size_t)pos * a.kv_ld + c); }
 };
 template <typename T, int KT, int VTL>
 ATTN_KERNEL(T) void latent_attn_kernel(const LatentArgs a) {
-  const int h = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;  // (a sequence's last tiles have the most keys: they start first)
+  const auto [tile, h] = attn_place(a.p.n_qtiles, a.heads);
   const SeqDesc s = seq_at(a.p.seqs + a.p.qtile[2 * tile]);
   if (s.len == 1) return;
-  attn_tile<T, KT, VTL>(LatentKeys<T>{a, s, h}, s, a.p.qtile[2 * tile + 1], (a.dim_p + a.rot_p) >> 5, a.vdim_p >> 4, a.vdim, a.scale,
+  attn_tile<T, KT, VTL>(LatentKeys<T>(a, s, h), s, a.p.qtile[2 * tile + 1], (a.dim_p + a.rot_p) >> 5, a.vdim_p >> 4, a.vdim, a.scale,
                         reinterpret_cast<T*>(a.out_t) + h * a.vdim, a.out_ld);
 }
 
@@ -384,7 +386,7 @@ static int attn_t(hipStream_t st, const LatentArgs& a) {
     constexpr int KT = decltype(kt)::value, VTL = decltype(vt)::value, lds = attn_tile_lds<T, KT, VTL>();
     auto k = latent_attn_kernel<T, KT, VTL>;
     HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    hipLaunchKernelGGL(k, dim3(a.p.n_qtiles, a.heads), dim3(256), lds, st, a);
+    hipLaunchKernelGGL(k, dim3(a.p.n_qtiles * a.heads), dim3(256), lds, st, a);
     return (int)DSK_OK;
   }, "latent attention");
 }
