@@ -77,6 +77,8 @@ int launch_fill_random_f32(hipStream_t st, float* dst, size_t n, float scale, ui
 // What a workgroup keeps in LDS.  bf16: two stages of two k tiles (8 weight tiles and 8 row groups each), 64 KiB; deeper rings with a barrier
 // per k tile were no faster (two workgroups on a compute unit hide each other's waits).
 enum { LIN_STEP = 2, LIN_STAGE = LIN_STEP * 16 * 1024, LIN_LDS = 2 * LIN_STAGE };
+enum { LONE_RING = 4 };  // stages of one k tile, 64 KiB as well
+static_assert(LONE_RING * 16 * 1024 == LIN_LDS, "one size for both");
 // 32 bits, 64 J rows: a ring of three stages of one k tile (8 weight tiles, 4 J row groups of two KiB), 72 or 48 KiB.
 enum { ROWS_RING = 3 };
 template <int J>
@@ -184,6 +186,90 @@ DEV void lin_body(const LinArgs& a, int row0, int n_rows, int f0, int k0, int k1
         for (int j = 0; j < 4; ++j) acc[i][j] = mma(w[i], x[j], acc[i][j]);
     }
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = wn * 64 + j * 16 + (lane & 15);
+    if (r >= n_rows) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rt = rt0 + wm * 4 + i;
+      if (rt < a.rt) store_plain<bf16, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+    }
+  }
+}
+// The same where workgroups have a compute unit each: nobody else hides their waits.  While a k tile is multiplied the next one's operands are read into the
+// other set of registers and the loads of LONE_RING - 1 more are on their way.  k = 2048, up to 256 workgroups: 20.4 - 24 us -> 15.5 - 18, with weights
+// out of HBM (2048 x 27648, 216 workgroups of 40 rows, k = 7168) 107 -> 77; but of two on a compute unit each (300 rows x 16896, k = 2048) 33.6 -> 34.4, and
+// 1100 rows x 27648, k = 7168 462 -> 550.  A ring of three: as fast, 93 us out of HBM.
+template <int EPI>
+DEV void lone_body(const LinArgs& a, int row0, int n_rows, int f0, int k0, int k1, char* lds) {
+  constexpr int R = LONE_RING, STAGE = 16 * 1024, WB = 8 * 1024;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1, n = k1 - k0;
+  const int rt0 = f0 >> 4;
+  // this wave's share of the staging: two weight tiles and two row groups
+  const char *src_w[2], *src_a[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)  // (tiles past the end: any valid one, never stored)
+    src_w[i] = reinterpret_cast<const char*>(a.w) + ((size_t)min(rt0 + 2 * wave + i, a.rt - 1) * a.kt + k0) * 1024 + lane * 16;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = row0 + min((2 * wave + i) * 16 + block_row(lane), n_rows - 1);
+    src_a[i] = reinterpret_cast<const char*>(operand<bf16>(a, f0) + (size_t)r * a.lda + (size_t)k0 * 32) + block_group(lane) * 16;
+  }
+  auto stage = [&](int kt, char* buf) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((gptr)(src_w[i] + (size_t)kt * 1024), (lptr)(buf + (2 * wave + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds((gptr)(src_a[i] + (size_t)kt * 64), (lptr)(buf + WB + (2 * wave + i) * 1024), 16, 0, 0);
+  };
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  struct Operands {
+    bf16x8 w[4], x[4];
+  };
+  auto read = [&](const char* buf, int i, Operands& o) {
+    o.w[i] = *reinterpret_cast<const bf16x8*>(buf + (wm * 4 + i) * 1024 + lane * 16);
+    o.x[i] = *reinterpret_cast<const bf16x8*>(buf + WB + (wn * 4 + i) * 1024 + block_place(lane) * 16);
+  };
+  int cur = 0;
+  auto step = [&](int kt, const Operands& now, Operands& next) {
+    // tile kt + 1 is here when at most the loads of R - 2 tiles are outstanding; behind the barrier everybody's are, and everybody holds
+    // tile kt in registers, so that its buffer takes tile kt + R (past the end: the last one again, never read)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (R - 2)) : "memory");
+    lds_barrier();
+    stage(min(kt + R, n - 1), lds + cur * STAGE);
+    cur = cur + 1 == R ? 0 : cur + 1;
+    const char* buf = lds + cur * STAGE;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // two reads beside four matrix instructions
+      read(buf, i, next);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = mma(now.w[i], now.x[j], acc[i][j]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  Operands p, q;
+#pragma unroll
+  for (int i = 0; i < R; ++i) stage(min(i, n - 1), lds + i * STAGE);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (R - 1)) : "memory");
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) read(lds, i, p);
+  for (int kt = 0; kt < n; kt += 2) {  // (n is even)
+    step(kt, p, q);
+    step(kt + 1, q, p);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r = wn * 64 + j * 16 + (lane & 15);
@@ -416,12 +502,13 @@ DEV void wide_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
     }
   }
 }
-template <int EPI>
+template <bool LONE, int EPI>
 __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int b = xcd_range(blockIdx.x, tiles), row0 = b % row_tiles * 128, per = part_tiles(a), k0 = blockIdx.y * per;
   a.out_f += blockIdx.y * a.part_stride;
-  lin_body<EPI>(a, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
+  if constexpr (LONE) lone_body<EPI>(a, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
+  else lin_body<EPI>(a, row0, min(128, a.rows - row0), b / row_tiles * 128, k0, min(a.kt, k0 + per), lds);
 }
 template <int J, int EPI>
 __global__ __launch_bounds__(256, 4 - J) void rows_kernel(LinArgs a, const int row_tiles, const int tiles) {
@@ -798,7 +885,7 @@ static int allow_lds(K k, int bytes) {
   return DSK_OK;
 }
 // Microseconds a prompt product takes on 256 compute units, by measurement of 20 shapes of 100 - 2000 rows and k of 2048 - 27648 (within a tenth of most): a
-// step of 64 columns takes a workgroup of 128 x 128 alone on its compute unit 0.6 us (0.85 with weights out of HBM), two of them 1.0 - 1.08; one of 256 x 256
+// step of 64 columns takes a workgroup of 128 x 128 alone on its compute unit 0.4 us (0.6 with weights out of HBM), two of them 1.0 - 1.08; one of 256 x 256
 // takes 1.17 us, and 1.55 when all of them run (the card's clock).  Both start and end in 3 and 8 us; a part more writes and reads its sums.
 // Stretches (LinStream) leave no compute unit empty, but their rows and weights meet in L2 less often (1.72 us), and tiles that they cut are stored and read:
 // 2000 rows and 2048 x 16896 145 us, by 128 x 128 163, by 256 x 256 168; 7168 x 32896 803, 1066, 895; but 1500 rows and 7168 x 27648 550, 658, 541.
@@ -828,7 +915,7 @@ static double lin_cost(int rows, int rt, int kt, int parts, int kind, bool f32) 
     return n / 256 * (8 + 1.55 * k) + (rest ? 8 + (1.17 + 0.38 / 256 * rest) * k : 0) + sums;
   }
   const int n = cdiv(rows, 128) * cdiv(rt, 8) * parts, rest = n % 512;
-  return 3 + (n / 512 * 1.08 + (rest == 0 ? 0 : rest <= 256 ? 0.85 : 1.0)) * k + sums;
+  return 3 + (n / 512 * 1.08 + (rest == 0 ? 0 : n <= 256 ? 0.6 : rest <= 256 ? 0.85 : 1.0)) * k + sums;
 }
 static int lin_kind(int rows, int rt, int kt, int parts, bool f32) {
   int best = LIN_SMALL;
@@ -889,7 +976,10 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32, const LinSpace& space
   const dim3 grid(tiles, std::max(a.parts, 1));
 #define LIN_J1 1,
 #define LIN_J2 2,
-  auto k = !f32 ? LIN_EPI(lin_kernel, ) : kind == LIN_HALF ? LIN_EPI(rows_kernel, LIN_J1) : LIN_EPI(rows_kernel, LIN_J2);
+#define LIN_LONE true,
+#define LIN_SHARED false,
+  const bool lone = tiles * std::max(a.parts, 1) <= 256;  // (lin_cost)
+  auto k = !f32 ? (lone ? LIN_EPI(lin_kernel, LIN_LONE) : LIN_EPI(lin_kernel, LIN_SHARED)) : kind == LIN_HALF ? LIN_EPI(rows_kernel, LIN_J1) : LIN_EPI(rows_kernel, LIN_J2);
   DSK_TRY(allow_lds(k, lds));
   hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, row_tiles, tiles);
   return DSK_OK;

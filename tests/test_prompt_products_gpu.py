@@ -196,18 +196,20 @@ def test_products_in_stretches(ctx, tmp_path, rows):
     assert U.err(got[0], got[2]) < 0.02
 
 
-# 32-bit products by workgroups of 64 and of 128 rows (whichever lin_cost finds the cheaper): rows short of, at and behind a wave's 16 and a workgroup's
+# 32-bit products by workgroups of 64 and of 128 rows (whichever lin_cost finds the cheaper), bfloat16 products of workgroups with a compute unit each (one k
+# step is less than their ring, a width of 64) and not: rows short of, at and behind a wave's 16 and a workgroup's
 # 64 against the oracle, and, where 16 row tiles of 128 by 32 tiles of 128 features fill whole rounds of workgroups, the whole prompt at once against the
 # same prompt in pieces of 64 rows.  Sums of up to 4096 products in another order of parts: the tolerance of 32 bits.
+@pytest.mark.parametrize("dtype,tol", [("float32", U.F32), ("bfloat16", U.B16)])
 @pytest.mark.parametrize("n", [17, 31, 33, 63, 64, 65, 129, 193, 1921, 2048])
-def test_32_bit_products_of_64_and_128_rows(ctx, tmp_path, n):
-    K = U.Case(ctx, tmp_path, U.sandwich([dict(U.wkv(4, 16), mlp=U.dense(4096))], width=64, vocab=72), dtype="float32")
+def test_products_of_64_and_128_rows(ctx, tmp_path, n, dtype, tol):
+    K = U.Case(ctx, tmp_path, U.sandwich([dict(U.wkv(4, 16), mlp=U.dense(4096))], width=64, vocab=72), dtype=dtype)
     t = K.tokens(n)
     s = K.lm.seq_open()
     got = K.lm.step([(s, t, range(n))])
     if n < 200:
-        assert U.err(got, K.want(t)) < U.F32
+        assert U.err(got, K.want(t)) < tol
         return
     p = K.lm.seq_open()
     cut = [K.lm.step([(p, t[i:i + 64], range(min(64, n - i)))]) for i in range(0, n, 64)]
-    assert U.err(got, np.concatenate(cut)) < U.F32
+    assert U.err(got, np.concatenate(cut)) < tol
