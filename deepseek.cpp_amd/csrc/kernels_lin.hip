@@ -502,6 +502,71 @@ DEV void wide_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
     }
   }
 }
+// The same for few rows, which are bound by the weights' way out of HBM: a ring of four k tiles, the weights' in registers, the rows' in LDS (NJ KiB each),
+// where wide_body has two steps of two.  64 experts of 1408, 60 prompt rows: gate / up 136 -> 125 us (5.9 TB/s), down 92.7 -> 89; 300 rows: down 101 -> 92, but gate / up
+// of 33 to 64 rows are left to wide_body (151, 155 so).  Rings of six and eight are no faster; 128 rows by a ring of three 268 -> 271 us.
+template <int NJ, int EPI>
+DEV void thin_body(const LinArgs& a, const int* gather, int row0, int n_rows, int f0, char* lds) {
+  constexpr int RING = 4, STAGE = NJ * 1024;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = a.kt;
+  const int rt0 = (f0 >> 4) + 4 * wave, own = min(wave, NJ - 1);  // (with fewer row groups than waves some load the same one)
+  const char* src_w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) src_w[i] = reinterpret_cast<const char*>(a.w) + (size_t)min(rt0 + i, a.rt - 1) * a.kt * 1024 + lane * 16;  // (past the end: never stored)
+  int r = min(own * 16 + block_row(lane), n_rows - 1);
+  r = gather ? gather[row0 + r] : row0 + r;
+  const char* src_a = reinterpret_cast<const char*>(operand<bf16>(a, f0) + (size_t)r * a.lda + block_group(lane) * 8);
+  bf16x8 w[RING][4];
+  auto load = [&](int kt, int slot) {  // (past the end: the last one again, not used)
+    kt = min(kt, n - 1);
+    __builtin_amdgcn_global_load_lds((gptr)(src_a + (size_t)kt * 64), (lptr)(lds + slot * STAGE + own * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[slot][i] = *reinterpret_cast<const bf16x8*>(src_w[i] + (size_t)kt * 1024);
+  };
+  f32x4 acc[4][NJ];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int kt, int slot) {
+    // this k tile is here when at most the loads of the RING - 2 behind it are outstanding; the barrier makes it everybody's, and everybody has read
+    // the one before it, whose place the one RING - 1 tiles on takes
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (RING - 2) * 5);  // vmcnt (the builtin: the compiler counts the weights' loads itself)
+    lds_barrier();
+    load(kt + RING - 1, (slot + RING - 1) % RING);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(lds + slot * STAGE + j * 1024 + block_place(lane) * 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i][j] = mma(w[slot][i], x, acc[i][j]);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < RING - 1; ++i) load(i, i);
+  int kt = 0;
+  for (; kt + RING <= n; kt += RING)
+#pragma unroll
+    for (int i = 0; i < RING; ++i) step(kt + i, i);
+#pragma unroll
+  for (int i = 0; i < RING - 1; ++i)
+    if (kt + i < n) step(kt + i, i);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int r = j * 16 + (lane & 15);
+    if (r >= n_rows) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rt = rt0 + i;
+      if (rt >= a.rt) continue;
+      if constexpr (EPI == LIN_GLU) {
+        if (!(i & 1)) store_glu<bf16>(a, row0 + r, (rt >> 1) * 16 + (lane >> 4) * 4, acc[i][j], acc[i | 1][j]);
+      } else {
+        store_plain<bf16, EPI>(a, row0 + r, rt * 16 + (lane >> 4) * 4, acc[i][j]);
+      }
+    }
+  }
+}
 template <bool LONE, int EPI>
 __global__ __launch_bounds__(256, 2) void lin_kernel(LinArgs a, const int row_tiles, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -739,8 +804,9 @@ __global__ __launch_bounds__(256, 2) void expert_kernel(LinArgs a, const MoeArgs
   const int row0 = m.tiles[4 * tile + 1], rows = m.tiles[4 * tile + 2];
   if constexpr (sizeof(T) == 2) {
     if (rows > 64) wide_body<8, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    else if (rows > 32 && down) thin_body<4, EPI>(a, gather, row0, rows, f * 256, lds);
     else if (rows > 32) wide_body<4, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
-    else wide_body<2, EPI>(a, gather, row0, rows, f * 256, 0, a.kt, lds);
+    else thin_body<2, EPI>(a, gather, row0, rows, f * 256, lds);
   } else {
     if (rows > 64) rows_body<2, EPI>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
     else rows_body<1, EPI>(a, gather, row0, rows, f * 128, 0, a.kt, lds);
