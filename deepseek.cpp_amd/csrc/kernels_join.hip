@@ -61,7 +61,7 @@ int launch_join(hipStream_t st, const JoinArgs& a, bool f32) {
 // Its rows are requested at once, from places that are always there, and what doesn't belong is dropped behind (behind a branch the compiler waits for
 // each row); the kept inputs of the next portion come out of the registers.  What bounds it is that chain of loads, sums and stores, so a thread has one
 // channel, not four, and a compute unit four times the waves: 2048 channels of 1996 rows 11.2 -> 10.5 us, of 301 rows in 32 bits 7.8 -> 6.2 (two channels: 11.7
-// and 7.0), 7168 channels of 700 rows 12.4 -> 12.0.
+// and 7.0), 7168 channels of 700 rows 12.4 -> 12.0; but of 2000 rows, where waves are enough either way and the width of a load counts, 19.8 -> 25.1.
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_kernel(const PassDesc p, int D, const float* __restrict__ h_f, const ConvArgs a) {
   constexpr int R = RECUR_CHUNK, K = TAPS ? TAPS : 1;
