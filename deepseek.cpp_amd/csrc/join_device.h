@@ -194,20 +194,14 @@ DEV void join_row(const JoinArgs& a, int block, JoinLds<NT>& lds) {
     }
     if (a.mix_b) {
       const float* mb = a.mix_b + (size_t)row * a.mix_ld;
-      float vb[VPT][V], sa = 0.f, sb = 0.f;
+      float vb[VPT][V];
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
         LoadSum<V, (VPT > 2)> q;
         q.load(mb + at(i), at(i) < D, a.parts_b, a.mix_stride);
         q.sum(vb[i]);
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-          sa += add[i][e] * add[i][e];
-          sb += vb[i][e] * vb[i][e];
-        }
       }
-      sa = block_sum<NT>(sa, red);
-      sb = block_sum<NT>(sb, red);
+      const float sa = block_sum<NT>(squares<VPT, V, V == 1 ? 0 : 1>(add), red), sb = block_sum<NT>(squares<VPT, V, V == 1 ? 0 : 1>(vb), red);
       const float ra = 1.f / sqrtf(sa / D + a.eps), rb = 1.f / sqrtf(sb / D + a.eps);
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
@@ -218,12 +212,7 @@ DEV void join_row(const JoinArgs& a, int block, JoinLds<NT>& lds) {
         for (int e = 0; e < V; ++e) add[i][e] = 0.5f * (add[i][e] * ra * wa[e] + vb[i][e] * rb * wb[e]);
       }
     } else if (a.post_w) {
-      float sa = 0.f;
-#pragma unroll
-      for (int i = 0; i < VPT; ++i)
-#pragma unroll
-        for (int e = 0; e < V; ++e) sa += add[i][e] * add[i][e];
-      sa = block_sum<NT>(sa, red);
+      const float sa = block_sum<NT>(squares<VPT, V, V == 1 ? 0 : 1>(add), red);
       const float ra = 1.f / sqrtf(sa / D + a.eps);
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
@@ -254,18 +243,14 @@ DEV void join_row(const JoinArgs& a, int block, JoinLds<NT>& lds) {
       }
     }
   }
-  float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) {
-      x[i][e] += add[i][e];
-      ss += x[i][e] * x[i][e];
-    }
+    for (int e = 0; e < V; ++e) x[i][e] += add[i][e];
     if (!a.only_want && at(i) < D) store_v<float, V>(a.x + (size_t)row * D + at(i), x[i]);
   }
   if (!a.norm_w) return;
-  ss = block_sum<NT>(ss, red);
+  const float ss = block_sum<NT>(squares<VPT, V>(x), red);
   const float r = 1.f / sqrtf(ss / D + a.eps);
   T* h = reinterpret_cast<T*>(a.h_t) + (size_t)hrow * a.h_ld;
 #pragma unroll
@@ -316,10 +301,6 @@ template <bool PUB>
 DEV void store_out(const __amdgpu_buffer_rsrc_t& r, int at, const f32x4& v, float) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, at * 4, 0, PUB ? 16 : 0);
-}
-DEV void add_squares(float& ss, const f32x4& v) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) ss += v[e] * v[e];
 }
 template <typename T, int NT, int VPT, int PARTS, int SPLIT, bool MIX, bool PUB>
 DEV void sandwich_row(const JoinArgs& a, const SeqDesc* seqs, int block, float (&red)[NT / 64]) {
@@ -374,29 +355,27 @@ DEV void sandwich_row(const JoinArgs& a, const SeqDesc* seqs, int block, float (
     for (int t = 0; t < KEPT; ++t) old[i][t] = load4(range(in + flip * half + (size_t)t * bytes, pos0 - KEPT + t >= 0, bytes), own(i) * 4);
     if constexpr (MIX) prev[i] = load4(range(state + cv.off_prev + (size_t)flip * bytes, pos0 > 0, bytes), own(i) * 4);
   }
-  float ss = 0.f;
+  f32x4 sum[VPT];
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
 #pragma unroll
     for (int n = 1; n < PARTS; n *= 2)
 #pragma unroll
       for (int u = 0; u + n < PARTS; u += 2 * n) q[i][u] += q[i][u + n];
-    add_squares(ss, q[i][0]);
+    sum[i] = q[i][0];
   }
-  ss = block_sum<NT>(ss, red);
-  const float ra = 1.f / sqrtf(ss / D + a.eps);
-  ss = 0.f;
+  const float sa = block_sum<NT>(squares<VPT, 4>(sum), red);
+  const float ra = 1.f / sqrtf(sa / D + a.eps);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float add = a.post_w ? q[i][0][e] * (ra * (pw[i][e] + a.norm_offset)) : q[i][0][e];
+      const float add = a.post_w ? sum[i][e] * (ra * (pw[i][e] + a.norm_offset)) : sum[i][e];
       x[i][e] = (a.embed ? x[i][e] : xs[i][e]) + add;
     }
-    add_squares(ss, x[i]);
     store4(rx, own(i) * 4, x[i]);
   }
-  ss = block_sum<NT>(ss, red);
+  const float ss = block_sum<NT>(squares<VPT, 4>(x), red);
   if constexpr (VPT > 1) load_mu();  // (for the registers)
   const float r = 1.f / sqrtf(ss / D + a.eps);
 #pragma unroll

@@ -322,7 +322,8 @@ __global__ __launch_bounds__(256) void wkv_prepare_kernel(const WkvArgs a, float
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-      acc[t] += q[t] * (t == sx ? bonus : w);
+      const float p = t == sx ? bonus : w;
+      acc[t] = t < 15 ? fmaf(q[t], p, acc[t]) : acc[t] + product(q[t], p);  // (the last row's have always been rounded: results stay what they are)
       w *= g[t];
       w = t == sx ? ks : w;
     }

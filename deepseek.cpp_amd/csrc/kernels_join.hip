@@ -24,7 +24,7 @@ static int sandwich_t(hipStream_t st, const JoinArgs& a, int n) {
   hipLaunchKernelGGL((a.conv.mu ? sandwich_kernel<T, NT, VPT, PARTS, SPLIT, true> : sandwich_kernel<T, NT, VPT, PARTS, SPLIT, false>), dim3(n * SPLIT), dim3(NT), 0, st, a.p.seqs, a)
   if (D <= 1024) ROW(256, 1, 8, 1);
   else if (D <= 2048) ROW(512, 1, 8, 2);
-  else if (D <= 4096) ROW(1024, 1, 8, 4);
+  else if (D <= 4096) ROW(512, 2, 8, 4);
   else ROW(1024, 2, 4, 4);
 #undef ROW
   return DSK_OK;

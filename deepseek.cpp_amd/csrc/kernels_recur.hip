@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaArgs a) {
 #pragma unroll
     for (int t = 0; t < R; ++t) {
       y[i][t] = silu_f(y[i][t]);
-      ss[t] += lane + 64 * i < n ? y[i][t] * y[i][t] : 0.f;
+      ss[t] = fmaf(y[i][t], lane + 64 * i < n ? y[i][t] : 0.f, ss[t]);
     }
   float* dst = is_v ? a.v + row0 * nv + c0 - 2 * nq : is_q ? a.q + row0 * nq + c0 : a.k + row0 * nq + c0 - nq;
   const int ld = is_v ? nv : nq;
@@ -320,13 +320,10 @@ DEV void head_norm_gate(V value, int heads, int vdim, float eps, const float* w,
     __builtin_amdgcn_sched_barrier(0);  // (all on their way first)
 #pragma unroll
     for (int u = 0; u < HU; ++u) {
-      float ss = 0.f;
+      float x[NI][1];
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        if (lane + 64 * i >= vdim) v[u][i] = 0.f;
-        ss += v[u][i] * v[u][i];
-      }
-      const float r = 1.f / sqrtf(wave_sum(ss) / vdim + eps);
+      for (int i = 0; i < NI; ++i) x[i][0] = v[u][i] = lane + 64 * i < vdim ? v[u][i] : 0.f;
+      const float r = 1.f / sqrtf(wave_sum(squares<NI, 1>(x)) / vdim + eps);
 #pragma unroll
       for (int i = 0; i < NI; ++i)
         if (h0 + 4 * u < heads && lane + 64 * i < vdim) out[(h0 + 4 * u) * vdim + lane + 64 * i] = (T)(v[u][i] * r * weight[u][i] * act(g[u][i]));

@@ -122,6 +122,23 @@ DEV float row_sum(float v) {
   v += dpp_f<0x140>(v);  // row_mirror
   return v;
 }
+// a product that is rounded: not to be fused with a sum
+DEV float product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+// The sum of a thread's N x V squares in one order of roundings: the square at `rounded` is, all others go into the sum as they are, in order.  (Left to
+// itself the compiler rounds the first or the second, by what stands around it.  A norm's last bit moves the bfloat16 roundings behind it, and a router's
+// close calls follow those: results would change with the neighbourhood of this sum.)
+template <int N, int V, int ROUNDED = 1, typename R>
+DEV float squares(const R (&x)[N]) {
+  constexpr int F = ROUNDED < N * V ? ROUNDED : 0;
+  float s = product(x[F / V][F % V], x[F / V][F % V]);
+#pragma unroll
+  for (int i = 0; i < N * V; ++i)
+    if (i != F) s = fmaf(x[i / V][i % V], x[i / V][i % V], s);
+  return s;
+}
 // sum over a workgroup of NT threads, result in every thread; scratch: NT / 64 floats of LDS
 template <int NT>
 DEV float block_sum(float v, float* scratch) {
