@@ -597,14 +597,17 @@ __global__ __launch_bounds__(256) void lin_direct_kernel(const LinArgs a, const 
 //
 // streams = 0: a workgroup per tile (and part of k).  Else the tiles of a row of them, k step by k step behind each other, are dealt out evenly to that
 // many workgroups, each of which works off one stretch without a stop between tiles: a product whose tiles do not fill the last round of compute units loses
-// none of them.  A tile that a stretch's end cuts (never in more than two pieces: streams <= feature tiles) is added up by whichever of the two workgroups
-// comes second; nobody waits.  The row tiles of one stretch are neighbours on one XCD and run in step, so that weights and rows meet in its L2.
-enum { RING = 4 };
+// none of them.  A tile that a stretch's end cuts (never in more than two pieces: streams <= feature tiles) is still added up in one order, as everywhere
+// else: a workgroup takes the tiles of its stretch from the last one down, so that the front of the tile at its end, whose sums it leaves for the next
+// stretch, is its first work, and going on from the sums of the tile at its start its last.  Should those not be there after CUT_LOOKS looks, it works off
+// the front itself.  The row tiles of one stretch are neighbours on one XCD and run in step, so that weights and rows meet in its L2.
+enum { RING = 4, CUT_LOOKS = 64 };
 struct LinStream {
   int streams;
-  float* sums;        // [streams][row tiles][2][256 x 256]: pieces in front of and behind the start of a stretch
-  unsigned* pieces;   // [streams][row tiles]: how many of them are there, zero between launches
+  float* sums;        // [streams][row tiles][256 x 256]: of the front of the tile that the stretch's start cuts
+  unsigned* pieces;   // [streams][row tiles]: CUT_STORED and CUT_TAKEN as they come, zero between launches
 };
+enum { CUT_STORED = 1, CUT_TAKEN = 2 };
 template <int EPI>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lin_big_kernel(LinArgs a, const int row_tiles, const int tiles, const LinStream ls) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -623,13 +626,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     last = min(first + per, (stream + 1) * a.kt);
     a.out_f += blockIdx.y * a.part_stride;
   }
+  const int f_first = first / a.kt, f_last = (last - 1) / a.kt;
+  const int k_first = first - f_first * a.kt, k_last = last - f_last * a.kt;  // of the first tile from, of the last one up to
   const int n_rows = min(256, a.rows - row0);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   int at_a[2];  // this wave's share of a stage: weight tiles and row groups 2 * wave + {0, 1}
 #pragma unroll
   for (int i = 0; i < 2; ++i) at_a[i] = (row0 + min((2 * wave + i) * 16 + block_row(lane), n_rows - 1)) * a.lda + block_group(lane) * 8;
-  int f_in = first / a.kt, k_in = first - f_in * a.kt, left = last - first;  // what is requested next
+  int f_in = f_last, k_in = f_last == f_first ? k_first : 0, to_in = k_last;  // what is requested next
   auto stage = [&](char* buf) {  // (past the end: the last tile again, never read)
     const bf16* x = operand<bf16>(a, f_in * 256) + (size_t)k_in * 32;
 #pragma unroll
@@ -639,10 +644,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       __builtin_amdgcn_global_load_lds((gptr)(w + lane * 8), (lptr)(buf + slot * 1024), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((gptr)(x + at_a[i]), (lptr)(buf + 16 * 1024 + slot * 1024), 16, 0, 0);
     }
-    const int go = left > 1, wrap = go && k_in + 1 == a.kt;
-    left -= go;
-    f_in += wrap;
-    k_in = wrap ? 0 : k_in + go;
+    const bool end = k_in + 1 == to_in, down = end && f_in > f_first;
+    f_in -= down;
+    k_in = down ? (f_in == f_first ? k_first : 0) : k_in + !end;
+    to_in = down ? a.kt : to_in;
   };
   f32x4 acc[8][4];
   auto clear = [&]() {
@@ -680,62 +685,70 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
   };
-  // the piece of a cut tile: true if the other one is there and is in the sums now, else ours is left for whoever works off the other one
-  auto joined = [&](int cut, bool behind) {
-    const int at = cut * row_tiles + row_tile;
-    unsigned* there = ls.pieces + at;
-    float* ours = ls.sums + ((size_t)at * 2 + behind) * 65536;
-    float* theirs = ls.sums + ((size_t)at * 2 + !behind) * 65536;
-    auto look = [&](unsigned v) {  // (a value of thread 0, to everybody)
-      __syncthreads();
-      if (tid == 0) s_there = v;
-      __syncthreads();
-      return s_there != 0;
-    };
-    bool second = look(tid == 0 ? __hip_atomic_load(there, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0);
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    if (!second) {
-      const auto r = __builtin_amdgcn_make_buffer_rsrc(ours, 0, 65536 * 4, 0x00020000);
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  // the front of the tile at the stretch's end: its sums for the next stretch
+  auto leave = [&]() {
+    const int at = (stream + 1) * row_tiles + row_tile;
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(ls.sums + (size_t)at * 65536, 0, 65536 * 4, 0x00020000);
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), r, tid * 16, (i * 4 + j) * 8192, 16 /* sc1 */);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      second = look(tid == 0 ? __hip_atomic_fetch_add(there, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0);
-      if (!second) return false;
+      for (int j = 0; j < 4; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), r, tid * 16, (i * 4 + j) * 8192, 16 /* sc1 */);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0 && __hip_atomic_fetch_add(ls.pieces + at, (unsigned)CUT_STORED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      __hip_atomic_store(ls.pieces + at, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (not waited for)
+  };
+  // the sums of the tile that the stretch's start cuts: true if they are there
+  auto take = [&]() {
+    const int at = stream * row_tiles + row_tile;
+    __syncthreads();
+    if (tid == 0) {
+      unsigned* word = ls.pieces + at;
+      for (int i = 0; i < CUT_LOOKS && !__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); ++i) __builtin_amdgcn_s_sleep(8);
+      s_there = __hip_atomic_fetch_add(word, (unsigned)CUT_TAKEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (s_there) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (tid == 0) __hip_atomic_store(there, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const auto r = __builtin_amdgcn_make_buffer_rsrc(theirs, 0, 65536 * 4, 0x00020000);
+    __syncthreads();
+    if (!s_there) return false;
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(ls.sums + (size_t)at * 65536, 0, 65536 * 4, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      f32x4 o[4];
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, tid * 16, (i * 4 + j) * 8192, 16));
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] += o[j];
-    }
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, tid * 16, (i * 4 + j) * 8192, 16));
     return true;
   };
   Operands p, q;
+  auto start = [&]() {
 #pragma unroll
-  for (int i = 0; i < RING; ++i) stage(lds + i * STAGE);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (RING - 1)) : "memory");
-  lds_barrier();
-  read(lds, p);
-  for (int at = first; at < last;) {
-    const int f = at / a.kt, end = min(last, (f + 1) * a.kt);
-    const bool cut_front = ls.streams && at > f * a.kt, cut_end = ls.streams && end < (f + 1) * a.kt;
+    for (int i = 0; i < RING; ++i) stage(lds + i * STAGE);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (RING - 1)) : "memory");
+    lds_barrier();
+    cur = 0;
+    read(lds, p);
+  };
+  start();
+  for (int f = f_last; f >= f_first; --f) {
+    int at = f == f_first ? k_first : 0;
+    const int end = f == f_last ? k_last : a.kt;
     clear();
+    if (ls.streams && at > 0) {
+      const bool there = take();
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): a step counts loads into LDS alone (the builtin: the compiler knows that the sums are here)
+      if (!there) {
+        lds_barrier();
+        at = k_in = 0;
+        to_in = end;
+        start();
+      }
+    }
     for (; at < end; at += 2) {  // (stretches and parts are even)
       step(p, q);
       step(q, p);
     }
-    if (cut_front || cut_end) {
-      if (!joined(cut_front ? stream : stream + 1, cut_front)) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        continue;
-      }
+    if (ls.streams && end < a.kt) {
+      leave();
+      continue;
     }
     const int rt0 = f * 16 + wm * 8;
     const bool pairs = wide_pairs(a) && (rt0 + 8) * 16 <= a.n_wide && rt0 + 8 <= a.rt;
@@ -954,7 +967,7 @@ static int allow_lds(K k, int bytes) {
 // step of 64 columns takes a workgroup of 128 x 128 alone on its compute unit 0.4 us (0.6 with weights out of HBM), two of them 1.0 - 1.08; one of 256 x 256
 // takes 1.17 us, and 1.55 when all of them run (the card's clock).  Both start and end in 3 and 8 us; a part more writes and reads its sums.
 // Stretches (LinStream) leave no compute unit empty, but their rows and weights meet in L2 less often (1.72 us), and tiles that they cut are stored and read:
-// 2000 rows and 2048 x 16896 145 us, by 128 x 128 163, by 256 x 256 168; 7168 x 32896 803, 1066, 895; but 1500 rows and 7168 x 27648 550, 658, 541.
+// 2000 rows and 2048 x 16896 132 us, by 128 x 128 163, by 256 x 256 159; 7168 x 32896 779, 1066, 878; but 1500 rows and 7168 x 27648 522, 658, 520.
 // In 32 bits a step of 64 columns takes a workgroup of 128 rows alone 1.08 us (1.5 with weights out of HBM), two of them 2.45, and one of 64 rows 0.64, three of them 1.96 (us by 128 and
 // by 64 rows: 301 rows and 2048 x 16896 78 and 62, 2000 rows 347 and 365; 301 rows and 2048 x 2176 40 and 25).
 enum { LIN_SMALL, LIN_HALF, LIN_BIG, LIN_STREAM };  // (the second: 64 rows instead of 128, 32 bits)

@@ -68,8 +68,8 @@ struct LinArgs {
 // parts worth splitting k into, at most `most`: launch_lin, launch_lin_few
 int lin_parts(int rows, int rt, int kt, bool f32, int most);
 int lin_parts_few(int rt, int kt, int most);
-// room for the pieces of tiles that two workgroups share: 256 slots of two tiles of 256 x 256 sums, and their words (zero between launches)
-enum { LIN_SLOTS = 256, LIN_SLOT_FLOATS = 2 * 256 * 256 };
+// room for the fronts of tiles that two workgroups share: 256 slots of 256 x 256 sums (64 MiB), and their words (zero between launches)
+enum { LIN_SLOTS = 256, LIN_SLOT_FLOATS = 256 * 256 };
 struct LinSpace {
   float* sums;
   unsigned* pieces;

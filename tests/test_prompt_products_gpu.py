@@ -213,3 +213,19 @@ def test_products_of_64_and_128_rows(ctx, tmp_path, n, dtype, tol):
     p = K.lm.seq_open()
     cut = [K.lm.step([(p, t[i:i + 64], range(min(64, n - i)))]) for i in range(0, n, 64)]
     assert U.err(got, np.concatenate(cut)) < tol
+
+
+# A sum has one order, that of k, whichever tiles make it: stretches (whose workgroups go on from each other's sums where they cut a tile), 256 x 256 and 128 x 128 tiles give
+# the same bits.  256 feature tiles of 256 and more in stretches of several sizes; a cut tile's front of one step up to all but one
+@pytest.mark.parametrize("rows,ff", [(257, 66000), (513, 40000), (769, 16900), (1280, 16900), (1500, 12300), (2048, 9000)])
+def test_tiles_and_stretches_give_the_same_bits(ctx, tmp_path, rows, ff):
+    c = U.sandwich([dict(U.wkv(2, 16), mlp=U.dense(ff))], width=256, vocab=64)
+    got = []
+    for tile in (256, 128):
+        K = U.Case(ctx, tmp_path / str(tile), c, dtype="bfloat16", options=f"prompt_tile={tile}")
+        K.lm.set_trace(True)
+        s, t = K.lm.seq_open(), K.tokens(rows)
+        K.lm.step([(s, t, [rows - 1])])
+        got.append(K.lm.trace_rows(0, rows))
+        K.lm.close()
+    assert np.isfinite(got[0]).all() and np.array_equal(*got)
