@@ -1009,17 +1009,33 @@ static int lin_kind(const LinArgs& a, int parts, bool f32, const LinSpace& space
   if (a.tile) kind = a.tile == 128 ? LIN_SMALL : parts == 1 && lin_streams(a.rows, a.rt) ? LIN_STREAM : LIN_BIG;
   return kind == LIN_STREAM && space.slots < LIN_SLOTS ? LIN_BIG : kind;
 }
-int lin_parts(int rows, int rt, int kt, bool f32, int most) {
+template <typename C>
+static int cheapest_parts(int kt, int most, C cost) {
   int best = 1;
   double least = 0;
   for (int n = 1; n <= most && (n == 1 || kt / n >= 16); ++n) {
-    const double c = lin_cost(rows, rt, kt, n, lin_kind(rows, rt, kt, n, f32), f32);
+    const double c = cost(n);
     if (n == 1 || c < least) {
       least = c;
       best = n;
     }
   }
   return cdiv(kt, part_tiles(kt, best));  // (no part may be empty)
+}
+int lin_parts(int rows, int rt, int kt, bool f32, int most) {
+  return cheapest_parts(kt, most, [&](int n) { return lin_cost(rows, rt, kt, n, lin_kind(rows, rt, kt, n, f32), f32); });
+}
+// Where a router reads what comes of a product the number of parts is no matter of tuning: it decides the order in which a sum is added up, with that the
+// roundings behind it, and a router decides close calls by those.  A step of 27 such layers behind a prompt of 300 tokens came out 0.13 apart, relative,
+// from a change of a sum's last bit in one row.  So these costs stay as they are, whatever the kernels take (tiles and stretches alike add a part up in the order of k):
+// the mixers' products of a width of 2048 take 15.0 us for 700 rows (lin_cost's parts: 13.2), 17.7 for 1200 (18.3), 22.4 for 2048 (20.9).
+int lin_parts_fixed(int rows, int rt, int kt, bool f32, int most) {
+  return cheapest_parts(kt, most, [&](int parts) {
+    const double k = part_tiles(kt, parts) / 2, sums = (parts - 1) * 3.2e-5 * rows * rt;
+    const int n = cdiv(rows, 128) * cdiv(rt, 8) * parts;
+    const double small = (n <= 256 ? (f32 ? 1.75 : 1.05) * k : cdiv(n, 512) * (f32 ? 3.2 : 1.3) * k) + 5 + sums;
+    return f32 ? small : std::min(small, cdiv(cdiv(rows, 256) * cdiv(rt, 16) * parts, 256) * (15 + 1.84 * k) + sums);
+  });
 }
 bool lin_streams_some(int rows, int rt, int kt, int tile) {
   bool some = false;

@@ -67,6 +67,7 @@ struct LinArgs {
 };
 // parts worth splitting k into, at most `most`: launch_lin, launch_lin_few
 int lin_parts(int rows, int rt, int kt, bool f32, int most);
+int lin_parts_fixed(int rows, int rt, int kt, bool f32, int most);     // launch_lin, where a router reads what comes of the sums
 int lin_parts_few(int rt, int kt, int most);
 // room for the fronts of tiles that two workgroups share: 256 slots of 256 x 256 sums (64 MiB), and their words (zero between launches)
 enum { LIN_SLOTS = 256, LIN_SLOT_FLOATS = 256 * 256 };

@@ -111,6 +111,7 @@ struct LayeredModel : ModelHead {
   char *h = nullptr, *hw = nullptr, *wide = nullptr, *out_a = nullptr, *out_b = nullptr, *qb = nullptr, *kb = nullptr, *vb = nullptr, *hidden = nullptr, *y = nullptr;
   float *narrow = nullptr, *mix_a = nullptr, *mix_b = nullptr, *low = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr, *dg = nullptr, *db = nullptr, *o = nullptr;
   int mix_parts[2] = {1, 1};        // of the products that wrote mix_a and mix_b last
+  bool routed = false;              // some layer has a router
   size_t mix_stride = 0;
   // sandwich layers, latent attention
   float *h_f = nullptr, *turn = nullptr, *lat_part = nullptr, *lat_ml = nullptr;
@@ -652,6 +653,7 @@ int alloc_work(LayeredModel* m) {
   DSK_TRY(dev_alloc_n(m, &m->attn_part, part));
   DSK_TRY(dev_alloc_n(m, &m->attn_arrived, arrived));
   if (hidden) DSK_TRY(dev_alloc(m, (void**)&m->hidden, n * hidden * m->hid_ld * e));
+  m->routed = experts > 0;
   if (experts) {
     const size_t ns = n * tmax;
     m->max_tiles = (int)(ns / MOE_TILE) + experts + 2;
@@ -707,7 +709,9 @@ LinArgs lin_f(const PackedMat& w, const void* a, int lda, int rows, float* out, 
 // A product whose output the next residual sum reads (mix_a; second: mix_b), split over k where its tiles alone leave compute units idle
 LinArgs mix_lin(LayeredModel* m, const PackedMat& w, const void* a, int lda, int rows, bool few, bool second = false) {
   LinArgs l = lin_f(w, a, lda, rows, second ? m->mix_b : m->mix_a, m->mix_ld);
-  l.parts = m->mix_parts[second] = few ? lin_parts_few(w.rt, w.kt, MIX_PARTS_FEW) : lin_parts(rows, w.rt, w.kt, m->f32, std::min<int>(MIX_PARTS, MIX_ROWS * m->piece / rows));
+  l.parts = m->mix_parts[second] = few         ? lin_parts_few(w.rt, w.kt, MIX_PARTS_FEW)
+                                   : m->routed ? lin_parts_fixed(rows, w.rt, w.kt, m->f32, MIX_ROWS)
+                                               : lin_parts(rows, w.rt, w.kt, m->f32, std::min<int>(MIX_PARTS, MIX_ROWS * m->piece / rows));
   l.part_stride = m->mix_stride = (size_t)rows * m->mix_ld;
   return l;
 }
