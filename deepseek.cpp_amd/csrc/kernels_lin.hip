@@ -517,8 +517,7 @@ DEV void thin_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
   r = gather ? gather[row0 + r] : row0 + r;
   const char* src_a = reinterpret_cast<const char*>(operand<bf16>(a, f0) + (size_t)r * a.lda + block_group(lane) * 8);
   bf16x8 w[RING][4];
-  auto load = [&](int kt, int slot) {  // (past the end: the last one again, not used)
-    kt = min(kt, n - 1);
+  auto load = [&](int kt, int slot) {
     __builtin_amdgcn_global_load_lds((gptr)(src_a + (size_t)kt * 64), (lptr)(lds + slot * STAGE + own * 1024), 16, 0, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[slot][i] = *reinterpret_cast<const bf16x8*>(src_w[i] + (size_t)kt * 1024);
@@ -528,12 +527,7 @@ DEV void thin_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](int kt, int slot) {
-    // this k tile is here when at most the loads of the RING - 2 behind it are outstanding; the barrier makes it everybody's, and everybody has read
-    // the one before it, whose place the one RING - 1 tiles on takes
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (RING - 2) * 5);  // vmcnt (the builtin: the compiler counts the weights' loads itself)
-    lds_barrier();
-    load(kt + RING - 1, (slot + RING - 1) % RING);
+  auto use = [&](int slot) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const bf16x8 x = *reinterpret_cast<const bf16x8*>(lds + slot * STAGE + j * 1024 + block_place(lane) * 16);
@@ -541,16 +535,46 @@ DEV void thin_body(const LinArgs& a, const int* gather, int row0, int n_rows, in
       for (int i = 0; i < 4; ++i) acc[i][j] = mma(w[slot][i], x, acc[i][j]);
     }
   };
+  // Loads are counted: every one of a k tile's five is used, so that none can go, and groups do not mix.
+  auto step = [&](int kt, int slot) {
+    // this k tile is here when at most the loads of the RING - 2 behind it are outstanding; the barrier makes it everybody's, and everybody has read
+    // the one before it, whose place the one RING - 1 tiles on takes
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (RING - 2) * 5);  // vmcnt (the builtin: the compiler counts the weights' loads itself)
+    lds_barrier();
+    load(kt + RING - 1, (slot + RING - 1) % RING);
+    use(slot);
+  };
 #pragma unroll
-  for (int i = 0; i < RING - 1; ++i) load(i, i);
+  for (int i = 0; i < RING - 1; ++i) {
+    load(min(i, n - 1), i);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  }
+  static_assert(RING == 4, "what is left below");
   int kt = 0;
-  for (; kt + RING <= n; kt += RING)
+  for (; kt + 2 * RING - 2 < n; kt += RING)
 #pragma unroll
     for (int i = 0; i < RING; ++i) step(kt + i, i);
-#pragma unroll
-  for (int i = 0; i < RING - 1; ++i)
-    if (kt + i < n) step(kt + i, i);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int left = n - kt;  // 4 or 6, or n = 2; steps while there is a k tile to request, and then all that is on its way at once
+  if (left > 2) step(kt, 0);
+  if (left > 4) {
+    step(kt + 1, 1);
+    step(kt + 2, 2);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  lds_barrier();
+  if (left == 6) {
+    use(3);
+    use(0);
+    use(1);
+  } else if (left == 4) {
+    use(1);
+    use(2);
+    use(3);
+  } else {
+    use(0);
+    use(1);
+  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int r = j * 16 + (lane & 15);

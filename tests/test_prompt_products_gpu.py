@@ -40,6 +40,20 @@ def test_expert_products_at_the_edges_of_row_tiles(ctx, tmp_path, ff, shared, dt
         K.lm.seq_close(s)
 
 
+# k tiles of 32 in a ring of four: 2, 4, 6, 8, 10 and 14 of them (gate and up: the width; down: ff), so that 2, 4 or 6 are left behind whole rounds
+@pytest.mark.parametrize("width,ff", [(64, 448), (128, 320), (192, 256), (256, 192), (320, 128), (448, 64)])
+def test_expert_products_of_few_rows_and_k_tiles(ctx, tmp_path, width, ff):
+    K = U.Case(ctx, tmp_path, U.config([U.parallel(mlp=U.moe(1, 1, ff, 0.8, 0))], width=width), edit=no_mixers, dtype="bfloat16")
+    t, want = K.tokens(64), []
+    K.ref.run(U.O.Sequence(K.ref), t, want)
+    K.lm.set_trace(True)
+    for n in (17, 32, 33, 48, 64):
+        s = K.lm.seq_open()
+        K.lm.step([(s, t[:n], [n - 1])])
+        assert U.err(K.lm.trace_rows(0, n), want[0][:n]) < 0.02, n
+        K.lm.seq_close(s)
+
+
 # several experts, rows spread unevenly: groups of four row tiles with and without neighbours of the same expert, a last group that is short
 @pytest.mark.parametrize("experts,top", [(3, 1), (6, 2), (40, 7)])
 def test_expert_products_over_many_experts(ctx, tmp_path, experts, top):
