@@ -69,7 +69,7 @@ struct LayerW {
 
 struct Seq {
   char* base = nullptr;
-  bool live = false;
+  bool live = false, lost = false;  // lost: a step failed half way through its state
   int pos = 0, flip = 0;
 };
 
@@ -1388,9 +1388,15 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
     }
     if (nw && mode == OUT_LOGITS) DSK_TRY(take_logits(m, out, nw, mode));
     else HIP_TRY(hipStreamSynchronize(st));
-    if (*m->gave_up) {
+    if (*m->gave_up) {  // recurrent states are updated in place: the step cannot be taken again.  Later steps do without the wait.
       *m->gave_up = 0;
-      DSK_FAIL(DSK_ERR_STATE, "step: a launch gave up waiting for its rows; the step's sequences have no valid state (option enter_ahead=0 does without the wait)");
+      for (const Part& q : parts) m->seqs[e[q.entry].seq].lost = true;
+      m->enter_ahead = false;
+      for (auto& it : m->graphs) {
+        if (it.second.exec) hipGraphExecDestroy(it.second.exec);
+        it.second.exec = nullptr;
+      }
+      DSK_FAIL(DSK_ERR_STATE, "step: a launch gave up waiting for its rows; the step's sequences have no valid state and can only be closed (later steps do without the wait)");
     }
     if (nw && mode != OUT_LOGITS) memcpy(next, m->next_host, (size_t)nw * 4);
   } else {
@@ -1428,11 +1434,16 @@ int check_seq(LayeredModel* m, int32_t s) {
   if (s < 0 || s >= (int)m->seqs.size() || !m->seqs[s].live) DSK_FAIL(DSK_ERR_INVALID, "sequence %d is not open", s);
   return DSK_OK;
 }
+int check_state(LayeredModel* m, int32_t s) {
+  DSK_TRY(check_seq(m, s));
+  if (m->seqs[s].lost) DSK_FAIL(DSK_ERR_STATE, "sequence %d has no valid state since a step of it failed", s);
+  return DSK_OK;
+}
 
 // A step in passes of at most `piece` rows.  Only an entry's last part may want its last row (modes ARGMAX / SAMPLE).
 int run_step(LayeredModel* m, const dsk_step_entry* e, int n, int mode, float* out, int32_t* next, const float* coins) {
   HIP_TRY(hipSetDevice(m->ctx->device));
-  for (int i = 0; i < n; ++i) DSK_TRY(check_seq(m, e[i].seq));
+  for (int i = 0; i < n; ++i) DSK_TRY(check_state(m, e[i].seq));
   std::vector<Part> parts;
   std::vector<int> want, want_entry;
   int rows = 0, keys = 0;  // keys: rows of the key workspace (latent attention)
@@ -1505,6 +1516,7 @@ int l_seq_open(dsk_model* h, int32_t* seq) {
     for (size_t i = 0; i < m->seqs.size(); ++i)
       if (!m->seqs[i].live) {
         m->seqs[i].live = true;
+        m->seqs[i].lost = false;
         m->seqs[i].pos = m->seqs[i].flip = 0;  // position 0: kernels start from zero state and read nothing of the arena
         *seq = (int32_t)i;
         return DSK_OK;
@@ -1561,7 +1573,10 @@ int own_seq(LayeredModel* m, const int32_t* tokens, int n, int pos) {
   dsk_model* h = reinterpret_cast<dsk_model*>(m);
   if (m->own_seq < 0) DSK_TRY(l_seq_open(h, &m->own_seq));
   Seq& s = m->seqs[m->own_seq];
-  if (pos == 0) s.pos = s.flip = 0;
+  if (pos == 0) {
+    s.lost = false;
+    s.pos = s.flip = 0;
+  }
   if (pos != s.pos) DSK_FAIL(DSK_ERR_STATE, "forward: position %d, but the sequence stands at %d (a recurrent state cannot go back)", pos, s.pos);
   return DSK_OK;
 }

@@ -453,7 +453,8 @@ int dsk_bench_router(dsk_ctx* ctx, int n_routed, int dim, int ksplit, int flags,
  * "chunk_scan" (1: prompts run their recurrences over chunks of tokens as matrix products; 0: token by token), "prompt_tile"
  * (tiles of prompt products in bfloat16: 128 or 256 rows and features; 0, the default: whichever is faster), "enter_ahead" (1: steps of up
  * to 8 single tokens make a layer's rows in the launch of the product that reads them; 0: in one of their own), "enter_spins" (how often a
- * workgroup of such a launch looks for its rows before the step fails). */
+ * workgroup of such a launch looks for its rows before the step fails).  Behind a step that failed so its sequences have no valid state: they take
+ * no further step and can only be closed (dsk_forward's own starts anew at position 0), and the model's later steps go as with enter_ahead=0. */
 enum { DSK_DTYPE_BF16 = 0, DSK_DTYPE_F32 = 1 };
 int dsk_dir_architecture(const char* dir, char* out, int cap); /* needs no GPU */
 int dsk_config_check(const char* config_json);                  /* is this the configuration of a layered design? needs no GPU */

@@ -55,3 +55,32 @@ def test_a_wait_without_end_is_an_error(ctx, tmp_path):
     with pytest.raises(dsk.DskError, match="gave up"):
         for t in K.tokens(4):
             K.lm.step([(s, [t], [0])])
+
+
+# Behind it: the step's sequences are closed to steps (their recurrent states were updated in place), others and new ones go on, in two launches; the model's
+# own sequence starts anew at position 0
+def test_a_step_that_gave_up_is_not_taken_again(ctx, tmp_path):
+    import dsk
+    K = U.Case(ctx, tmp_path / "0", stack(2048, 136), dtype="bfloat16", options="enter_spins=0")
+    same = U.Case(ctx, tmp_path / "1", stack(2048, 136), dtype="bfloat16", options="enter_ahead=0")
+    t, lone = K.tokens(6), K.lm.seq_open()
+    a, b = K.lm.seq_open(), same.lm.seq_open()
+    K.lm.step([(lone, t[:3], [])])
+    n = 0
+    with pytest.raises(dsk.DskError, match="gave up"):
+        for n in range(6):
+            K.lm.step([(a, t[n:n + 1], [0])])
+    for _ in range(2):
+        with pytest.raises(dsk.DskError, match="no valid state"):
+            K.lm.step([(a, t[n:n + 1], [0])])
+    with pytest.raises(dsk.DskError, match="no valid state"):
+        K.lm.step([(lone, t[3:4], [0]), (a, t[n:n + 1], [0])])
+    before = K.lm.info("enter_launches")
+    K.lm.seq_close(a)
+    a = K.lm.seq_open()
+    for i in range(6):  # (eager, captured, replayed)
+        assert np.array_equal(K.lm.step([(a, t[i:i + 1], [0])]), same.lm.step([(b, t[i:i + 1], [0])])), i
+    assert K.lm.info("enter_launches") == before
+    c = same.lm.seq_open()
+    same.lm.step([(c, t[:3], [])])
+    assert np.array_equal(K.lm.step([(lone, t[3:4], [0])]), same.lm.step([(c, t[3:4], [0])]))
