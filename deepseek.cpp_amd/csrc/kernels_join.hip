@@ -61,7 +61,7 @@ int launch_join(hipStream_t st, const JoinArgs& a, bool f32) {
 // Its rows are requested at once, from places that are always there, and what doesn't belong is dropped behind (behind a branch the compiler waits for
 // each row); the kept inputs of the next portion come out of the registers.  What bounds it is that chain of loads, sums and stores, so a thread has one
 // channel, not four, and a compute unit four times the waves: 2048 channels of 1996 rows 11.2 -> 10.5 us, of 301 rows in 32 bits 7.8 -> 6.2 (two channels: 11.7
-// and 7.0), 7168 channels of 700 rows 12.4 -> 12.0; but of 2000 rows, where waves are enough either way and the width of a load counts, 19.8 -> 25.1.
+// and 7.0).  With work for all of them either way the width of a load counts (conv_wide).
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_kernel(const PassDesc p, int D, const float* __restrict__ h_f, const ConvArgs a) {
   constexpr int R = RECUR_CHUNK, K = TAPS ? TAPS : 1;
@@ -134,8 +134,80 @@ __global__ __launch_bounds__(256) void conv_kernel(const PassDesc p, int D, cons
     if (has_prev) P[(size_t)(s.flip ^ 1) * D] = y;
   }
 }
+// The same with four channels a thread, by loads and stores of 16 bytes a lane: rows are requested as their places come, and the sums of a row are the same, in
+// the same order.  From 4 M elements on (us with one channel / with four, without blends and with): 2048 channels of 700 rows 5.8 / 7.3 and 15.2 / 16.9, of 2000 8.6 / 8.7
+// and 19.3 / 19.9, of 4000 15.1 / 13.1 and 32.9 / 25.3; 7168 channels of 300 rows 6.4 / 7.1 and 16.0 / 17.1, of 500 7.5 / 7.5 and 20.0 / 19.2, of 2000 20.3 / 17.8 and
+// 40.9 / 31.1; in 32 bits, 2000 rows, 22.1 / 18.8.  (Slower in a few places where rows are a power of two apart: 4096 channels of 1600 rows 10.8 / 14.8.)
+static bool conv_wide(const PassDesc& p, int D, const ConvArgs& a) {
+  return a.taps >= 2 && a.taps <= 4 && !(D & 3) && !(a.ld & 3) && (size_t)p.n_chunks * D >= 1 << 18;
+}
+template <typename T, int TAPS>
+__global__ __launch_bounds__(256) void conv_wide_kernel(const PassDesc p, int D, const float* __restrict__ h_f, const ConvArgs a) {
+  constexpr int R = RECUR_CHUNK, K = TAPS;
+  const int c = 4 * (blockIdx.y * 256 + threadIdx.x);
+  if (c >= D) return;
+  const SeqDesc s = seq_at(p.seqs + p.chunk[2 * blockIdx.x]);
+  const int t0 = p.chunk[2 * blockIdx.x + 1], n_rows = min(R, s.len - t0);
+  const float* H = h_f + (size_t)s.row0 * D + c;
+  const float* hist = reinterpret_cast<const float*>(s.state + a.off_in) + (size_t)s.flip * (K - 1) * D + c;
+  float* next = reinterpret_cast<float*>(s.state + a.off_in) + (size_t)(s.flip ^ 1) * (K - 1) * D + c;
+  float* P = a.mu ? reinterpret_cast<float*>(s.state + a.off_prev) + c : nullptr;
+  T* out = reinterpret_cast<T*>(a.out_t) + (size_t)(s.row0 + t0) * a.ld + c;
+  const bool has_prev = a.mu != nullptr;
+  auto input = [&](int u, float (&v)[4]) {  // row u of the portion; before it: the kept inputs, zero before the sequence's start
+    if (u >= 0) load_v<float, 4>(H + (size_t)u * D, true, v);
+    else load_v<float, 4>(hist + (size_t)(max(u, 1 - K) + K - 1) * D, u >= 1 - K && s.pos0 + u >= 0, v);
+  };
+  float w[4][K], x[R + K][4], y[R + 1][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int j = 0; j < K; ++j) w[e][j] = a.w[(size_t)(c + e) * K + j];
+#pragma unroll
+  for (int r = 0; r < R + K; ++r) input(min(t0 - K + r, s.len - 1), x[r]);
+#pragma unroll
+  for (int t = 0; t <= R; ++t)  // of input x[t + K - 1]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float z = 0.f;
+#pragma unroll
+      for (int j = 0; j < K; ++j) z += x[t + j][e] * w[e][j];
+      y[t][e] = x[t + K - 1][e] + z;
+    }
+  if (has_prev && t0 == 0) load_v<float, 4>(P + (size_t)s.flip * D, s.pos0 > 0, y[0]);
+  for (int i = 0; i < (has_prev ? a.n_mix : 1); ++i) {
+    float mu[4];
+    load_v<float, 4>(has_prev ? a.mu + (size_t)i * D + c : a.w, has_prev, mu);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = y[t + 1][e] + (y[t][e] - y[t + 1][e]) * mu[e];
+      if (t < n_rows) store_v<T, 4>(out + i * a.mix_stride + (size_t)t * a.ld, v);
+    }
+  }
+  if (t0 + n_rows < s.len) return;
+  for (int j = 0; j < K - 1; ++j) {  // the portion's end: what the next one needs, in the other copy
+    float v[4];
+    input(s.len - (K - 1) + j, v);
+    store_v<float, 4>(next + (size_t)j * D, v);
+  }
+  if (!has_prev) return;
+#pragma unroll
+  for (int t = 1; t < R; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[t + 1][e] = t < n_rows ? y[t + 1][e] : y[t][e];
+  store_v<float, 4>(P + (size_t)(s.flip ^ 1) * D, y[R]);
+}
 template <typename T>
 static void conv_t(hipStream_t st, const PassDesc& p, int D, const float* h_f, const ConvArgs& a) {
+  if (conv_wide(p, D, a)) {
+    const dim3 grid(p.n_chunks, (D / 4 + 255) / 256);
+    if (a.taps == 2) hipLaunchKernelGGL((conv_wide_kernel<T, 2>), grid, dim3(256), 0, st, p, D, h_f, a);
+    else if (a.taps == 3) hipLaunchKernelGGL((conv_wide_kernel<T, 3>), grid, dim3(256), 0, st, p, D, h_f, a);
+    else hipLaunchKernelGGL((conv_wide_kernel<T, 4>), grid, dim3(256), 0, st, p, D, h_f, a);
+    return;
+  }
   const dim3 grid(p.n_chunks, (D + 255) / 256);
   switch (a.taps) {
     case 2: hipLaunchKernelGGL((conv_kernel<T, 2>), grid, dim3(256), 0, st, p, D, h_f, a); break;

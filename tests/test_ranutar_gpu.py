@@ -218,3 +218,26 @@ def test_bad_weights_are_errors(case, ctx, tmp_path):
         del W[name]
         with pytest.raises(dsk.DskError, match=name + " is missing"):
             dsk.LM(ctx, U.save(tmp_path / "gone", K.c, W))
+
+
+# The convolution of prompts takes four channels a thread from 37 chunks of 7168 channels on (rows 577), one below: the rows that both prompts have are the same
+# bits, in both types.  Then a second portion, which starts from the inputs that the first has kept, in 32 bits against the oracle (bfloat16 rounds alike in
+# either form).  With blends (time mixing) and without.
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("layer", [U.wkv(2, 16), U.latent(2, 16, 8, 16, 12, 20, 6)], ids=["blends", "plain"])
+def test_convolution_by_one_and_by_four_channels(ctx, tmp_path, layer, taps, dtype):
+    K = U.Case(ctx, tmp_path, alone(U.no_ff(layer), width=7168, taps=taps), dtype=dtype)
+    t, got, want = K.tokens(1170), [], []
+    K.lm.set_trace(True)
+    for n in (576, 577):
+        s = K.lm.seq_open()
+        K.lm.step([(s, t[:n], [n - 1])])
+        first = K.lm.trace_rows(0, n)
+        K.lm.step([(s, t[n:n + 593], [592])])  # (four channels)
+        got.append(np.concatenate([first, K.lm.trace_rows(0, 593)]))
+        K.lm.seq_close(s)
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0][:576], got[1][:576])
+    if dtype == "float32":
+        K.ref.run(U.O.Sequence(K.ref), t, want)
+        assert U.err(got[0], want[0][:1169]) < TOL and U.err(got[1], want[0]) < TOL
