@@ -57,6 +57,8 @@ struct RowPool {
     for (unsigned i = 0; i < SLOTS; ++i) slots[i] = {this, i};
   }
   dsk_rows* lend();   // nullptr: none left
+  bool take_all();    // nobody has borrowed any, and nobody can until give_all()
+  void give_all() { taken.store(0, std::memory_order_release); }
   void let_go();      // one owner less
   float* rows(const dsk_rows* r) const { return lent + r->slot * slot_floats; }
   bool holds(const float* p, size_t n) const { return p >= lent && p + n <= lent + SLOTS * slot_floats; }

@@ -1402,7 +1402,15 @@ int run_pass(LayeredModel* m, const dsk_step_entry* e, const std::vector<Part>& 
   } else {
     m->splits = 1 << 30;  // (a mixer takes as many as its largest window has)
     DSK_TRY(run_body(m, d, p, false, mode));
-    const int block = mode != OUT_LOGITS ? FEW : m->pool->taken.load() ? LOGIT_ROWS - RowPool::SLOTS * FEW : LOGIT_ROWS;
+    // the borrowers' rows too, where more are wanted than there are others and nobody has borrowed any: not meanwhile either
+    constexpr int own = LOGIT_ROWS - RowPool::SLOTS * FEW;
+    struct All {
+      RowPool* pool;
+      ~All() {
+        if (pool) pool->give_all();
+      }
+    } all{mode == OUT_LOGITS && nw > own && m->pool->take_all() ? m->pool : nullptr};
+    const int block = mode != OUT_LOGITS ? FEW : all.pool ? LOGIT_ROWS : own;
     for (int i = 0; i < nw; i += block) {
       const int n = std::min(block, nw - i);
       float* to = mode == OUT_LOGITS ? out + (size_t)i * m->s.vocab : nullptr;

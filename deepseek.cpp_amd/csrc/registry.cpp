@@ -179,6 +179,10 @@ dsk_rows* RowPool::lend() {
     }
   }
 }
+bool RowPool::take_all() {
+  unsigned none = 0;
+  return taken.compare_exchange_strong(none, (1u << SLOTS) - 1, std::memory_order_acquire);
+}
 void RowPool::let_go() {
   if (owners.fetch_sub(1, std::memory_order_acq_rel) > 1) return;
   hipHostFree(mem);

@@ -66,3 +66,40 @@ def test_rows_of_prompts(ctx, tmp_path, vocab, n):
     import dsk
     with pytest.raises(dsk.DskError):
         dsk.check(dsk.lib().dsk_rows_lend(K.lm.h, 0, C.byref(rows), C.byref(hold)))
+
+
+# Rows that are borrowed while a prompt's logits are on their way stay the borrower's: a prompt that wants many rows uses the borrowers' own room for
+# them only if nobody has borrowed any, and lends none meanwhile
+def test_rows_borrowed_beside_a_prompt(ctx, tmp_path):
+    import threading
+
+    import dsk
+    K = model(ctx, tmp_path, vocab=4096)
+    t, stop, seen = K.tokens(150), threading.Event(), []
+
+    def borrow():
+        n = 0
+        while not stop.is_set():
+            rows, hold = C.c_void_p(), C.c_void_p()
+            dsk.check(dsk.lib().dsk_rows_lend(K.lm.h, 16, C.byref(rows), C.byref(hold)))
+            if not hold.value:
+                continue
+            a = np.ctypeslib.as_array(C.cast(rows, C.POINTER(C.c_float)), (16, 4096))
+            n += 1
+            a[:] = n
+            ok = True
+            for _ in range(20):
+                ok &= bool((a == n).all())
+            seen.append(ok)
+            dsk.lib().dsk_rows_return(hold)
+
+    b = threading.Thread(target=borrow)
+    want = K.got(t)
+    b.start()
+    try:
+        for _ in range(40):
+            assert np.array_equal(K.got(t), want)
+    finally:
+        stop.set()
+        b.join()
+    assert seen and all(seen)
