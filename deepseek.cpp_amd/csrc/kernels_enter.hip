@@ -11,8 +11,9 @@
 // What bounds it is that chain, slower among the weights' requests: a sum ready 4.3 us after the start of a launch of 8.7 MB is ready after 9 us in one
 // of 69 MB, whose weights take 10.5.  Both launches / this one, us, one row of 2048: 33 MB behind blends 14.4 / 12.6, 33 MB 14.2 / 11.0, 8.7 MB 9.4 / 7.1, 69 MB
 // 19.2 / 16.0, the logits' 419 MB 76.7 / 70.  16 tiles a wave ahead: with 12 the 69 MB take 18.0, with 8 18.6 (a second round waits for the rows), and 80 registers let
-// three workgroups share a compute unit, all of a launch at once (84: 18.5).  Readers that poll the rows themselves, a tag in every 8 bytes, took 19.2:
-// their loads are in the sum's way.
+// three workgroups share a compute unit, all of a launch at once (84: 18.5).  (That is the sum alone and with the convolution; with blends behind it, 92 registers,
+// two share one, and launches of more than 512 workgroups - more than 16 K features - come in two rounds.)  Readers that poll the rows themselves, a tag in every 8 bytes, took
+// 19.2: their loads are in the sum's way.
 //
 // Up to 8 rows and a width of 2048 (launch_enter): a step of 27 lite layers, us of kernels, apart / together, one row 1914 / 1766, two 1926 / 1798, four 1997 / 1898, eight
 // 2194 / 2144, but sixteen 2667 / 2740, as each reader takes all rows past its caches; four rows of 7168 by 1024 threads: 69 MB 21 / 26 us, 396 MB 80 / 80.

@@ -283,7 +283,7 @@ DEV void lone_body(const LinArgs& a, int row0, int n_rows, int f0, int k0, int k
 }
 // 128 features from f0 on x n_rows <= 64 J rows, k tiles [k0, k1), 32 bits: 4 waves of 128 features x 16 J rows.  gather: a table (slot -> row) or
 // nullptr; out rows are row0 + local row.
-// Activations are taken apart into three bf16 numbers (split3, 44 vector instructions for 16 rows of a k tile, 176 cycles); a wave has rows of its own, so
+// Activations are taken apart into three bf16 numbers (split_pair, 44 vector instructions for 16 rows of a k tile, 176 cycles); a wave has rows of its own, so
 // that no two of them take the same ones apart: per wave and k tile 24 J matrix instructions (384 J cycles) and 44 J vector instructions beside them.
 // While a k tile is multiplied the next one's operands are read and taken apart, and the loads of ROWS_RING - 1 more are on their way (rings of four and
 // five were not faster, and leave room for a workgroup less).  The matrix instructions bound it where compute units are full (128 rows: 1.23 us for two
@@ -996,7 +996,7 @@ static int allow_lds(K k, int bytes) {
 // by 64 rows: 301 rows and 2048 x 16896 78 and 62, 2000 rows 347 and 365; 301 rows and 2048 x 2176 40 and 25).
 enum { LIN_SMALL, LIN_HALF, LIN_BIG, LIN_STREAM };  // (the second: 64 rows instead of 128, 32 bits)
 static int lin_streams(int rows, int rt) {  // stretches of a row of 256 x 256 tiles; 0: they would cut a tile more than once
-  const int n = 256 / cdiv(rows, 256);
+  const int n = LIN_SLOTS / cdiv(rows, 256);  // (a workgroup for each compute unit)
   return n >= 2 && n <= cdiv(rt, 16) ? n : 0;
 }
 static double lin_cost(int rows, int rt, int kt, int parts, int kind, bool f32) {
@@ -1097,7 +1097,7 @@ int launch_lin(hipStream_t st, const LinArgs& a, bool f32, const LinSpace& space
 #define LIN_J2 2,
 #define LIN_LONE true,
 #define LIN_SHARED false,
-  const bool lone = tiles * std::max(a.parts, 1) <= 256;  // (lin_cost)
+  const bool lone = tiles * std::max(a.parts, 1) <= LIN_SLOTS;  // (lin_cost: compute units)
   auto k = !f32 ? (lone ? LIN_EPI(lin_kernel, LIN_LONE) : LIN_EPI(lin_kernel, LIN_SHARED)) : kind == LIN_HALF ? LIN_EPI(rows_kernel, LIN_J1) : LIN_EPI(rows_kernel, LIN_J2);
   DSK_TRY(allow_lds(k, lds));
   hipLaunchKernelGGL(k, grid, dim3(256), lds, st, a, row_tiles, tiles);

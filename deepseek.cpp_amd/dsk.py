@@ -648,7 +648,9 @@ class LM:
         return np.asarray(Rows(rows.value, hold.value, (n, self.vocab))) if hold.value else np.empty((n, self.vocab), np.float32)
 
     def step(self, entries):
-        """entries: (sequence, tokens, wanted places); returns [wanted, vocab] float32, in the order of the entries"""
+        """entries: (sequence, tokens, wanted places); returns [wanted, vocab] float32, in the order of the entries.  The first four results of up to 16
+        rows that are held at once are the model's own pinned rows (dsk_rows_lend): copy what is to be kept for long, since any view of one keeps the
+        room of 128 rows alive, also behind close()."""
         arr, keep = self._entries(entries)
         out = self._rows(sum(arr[i].n_want for i in range(len(entries))))
         check(lib().dsk_step(self.h, arr, len(entries), _f(out)))

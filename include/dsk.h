@@ -451,7 +451,8 @@ int dsk_bench_router(dsk_ctx* ctx, int n_routed, int dim, int ksplit, int flags,
  * options: "key=value[,key=value]" or NULL.  Layered models: "piece_tokens" (tokens one pass of a step runs, default 2048),
  * "decode_graph" (1: steps of single tokens replay a captured graph), "fused_decode" (1: the fused launches for such steps),
  * "chunk_scan" (1: prompts run their recurrences over chunks of tokens as matrix products; 0: token by token), "prompt_tile"
- * (tiles of prompt products in bfloat16: 128 or 256 rows and features; 0, the default: whichever is faster), "enter_ahead" (1: steps of up
+ * (tiles of prompt products in bfloat16: 128 or 256 rows and features, the latter in stretches over several tiles where they can be; 0, the default:
+ * whichever is faster; all give the same bits), "enter_ahead" (1: steps of up
  * to 8 single tokens make a layer's rows in the launch of the product that reads them; 0: in one of their own), "enter_spins" (how often a
  * workgroup of such a launch looks for its rows before the step fails).  Behind a step that failed so its sequences have no valid state: they take
  * no further step and can only be closed (dsk_forward's own starts anew at position 0), and the model's later steps go as with enter_ahead=0. */
@@ -482,7 +483,8 @@ typedef struct dsk_step_entry {
 int dsk_step(dsk_model* m, const dsk_step_entry* entries, int n, float* logits);
 /* Room for the logits of n_rows tokens that the device writes itself: passed to dsk_step (or any call that takes host_logits), no copy follows.  A model
  * lends a few of them; *rows is NULL when none is left (or it has none that large, or does not lend) and an ordinary buffer is to be used.  The rows
- * stay the borrower's until dsk_rows_return, which any thread may call, also behind dsk_model_destroy. */
+ * stay the borrower's until dsk_rows_return, which any thread may call, also behind dsk_model_destroy.  Layered models lend four times up to 16 rows,
+ * where the vocabulary is a multiple of 16; borrowed rows keep the model's whole room for logits (128 rows of pinned memory) alive behind its end. */
 typedef struct dsk_rows dsk_rows;
 int dsk_rows_lend(dsk_model* m, int n_rows, float** rows, dsk_rows** hold);
 void dsk_rows_return(dsk_rows* hold);

@@ -230,7 +230,7 @@ def test_products_of_64_and_128_rows(ctx, tmp_path, n, dtype, tol):
 
 
 # A sum has one order, that of k, whichever tiles make it: stretches (whose workgroups go on from each other's sums where they cut a tile), 256 x 256 and 128 x 128 tiles give
-# the same bits.  256 feature tiles of 256 and more in stretches of several sizes; a cut tile's front of one step up to all but one
+# the same bits, and those are near the oracle's values.  Stretches of one to two and a half tiles; a cut tile's front of one step up to all but one
 @pytest.mark.parametrize("rows,ff", [(257, 66000), (513, 40000), (769, 16900), (1280, 16900), (1500, 12300), (2048, 9000)])
 def test_tiles_and_stretches_give_the_same_bits(ctx, tmp_path, rows, ff):
     c = U.sandwich([dict(U.wkv(2, 16), mlp=U.dense(ff))], width=256, vocab=64)
@@ -242,4 +242,6 @@ def test_tiles_and_stretches_give_the_same_bits(ctx, tmp_path, rows, ff):
         K.lm.step([(s, t, [rows - 1])])
         got.append(K.lm.trace_rows(0, rows))
         K.lm.close()
-    assert np.isfinite(got[0]).all() and np.array_equal(*got)
+    want = []
+    K.ref.run(U.O.Sequence(K.ref), t, want)
+    assert np.isfinite(got[0]).all() and np.array_equal(*got) and U.err(got[0], want[0]) < U.B16

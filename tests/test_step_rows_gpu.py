@@ -48,6 +48,27 @@ def test_rows_beside_their_product(ctx, tmp_path, design, width, rows):
     assert np.isfinite(x).all() and np.array_equal(x, y)
 
 
+# logits of some of a step's rows, in any place: the last launch makes those rows alone.  The norm by itself (the final one) in front of the output product
+@pytest.mark.parametrize("want", [[0], [2], [1, 3], [0, 1, 2, 4]])
+@pytest.mark.parametrize("design", ["ranutar", "timerax"])
+def test_some_rows_beside_the_output_product(ctx, tmp_path, design, want):
+    c = stack(1100, 136) if design == "ranutar" else U.mixed(1100)
+    got = []
+    for i in (1, 0):
+        K = U.Case(ctx, tmp_path / str(i), c, dtype="bfloat16", options=f"enter_ahead={i}")
+        toks, seqs = [K.tokens(5, seed=r) for r in range(5)], [K.lm.seq_open() for _ in range(5)]
+        some = [K.lm.step([(s, t[n:n + 1], [0] if r in want else []) for r, (s, t) in enumerate(zip(seqs, toks))]).copy() for n in range(4)]  # (eager, captured, replayed)
+        every = K.lm.step([(s, t[4:5], [0]) for s, t in zip(seqs, toks)]).copy()
+        got.append((np.array(some), every))
+        assert (K.lm.info("enter_launches") > 0) == bool(i)
+    assert got[0][0].shape[1] == len(want) and np.isfinite(got[0][0]).all()
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    K = U.Case(ctx, tmp_path / "2", c, dtype="bfloat16")  # ... which are those of steps that want all
+    seqs = [K.lm.seq_open() for _ in range(5)]
+    for n in range(4):
+        assert np.array_equal(K.lm.step([(s, t[n:n + 1], [0]) for s, t in zip(seqs, toks)])[want], got[0][0][n])
+
+
 def test_a_wait_without_end_is_an_error(ctx, tmp_path):
     import dsk
     K = U.Case(ctx, tmp_path, stack(2048, 136), dtype="bfloat16", options="enter_spins=0")
