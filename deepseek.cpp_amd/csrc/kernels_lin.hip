@@ -623,13 +623,13 @@ __global__ __launch_bounds__(256) void lin_direct_kernel(const LinArgs a, const 
 // many workgroups, each of which works off one stretch without a stop between tiles: a product whose tiles do not fill the last round of compute units loses
 // none of them.  A tile that a stretch's end cuts (never in more than two pieces: streams <= feature tiles) is still added up in one order, as everywhere
 // else: a workgroup takes the tiles of its stretch from the last one down, so that the front of the tile at its end, whose sums it leaves for the next
-// stretch, is its first work, and going on from the sums of the tile at its start its last.  Should those not be there after CUT_LOOKS looks, it works off
+// stretch, is its first work, and going on from the sums of the tile at its start its last.  Should those not be there after `looks` looks, it works off
 // the front itself.  The row tiles of one stretch are neighbours on one XCD and run in step, so that weights and rows meet in its L2.
-enum { RING = 4, CUT_LOOKS = 64 };
+enum { RING = 4 };
 struct LinStream {
   int streams;
   float* sums;        // [streams][row tiles][256 x 256]: of the front of the tile that the stretch's start cuts
-  unsigned* pieces;   // [streams][row tiles]: CUT_STORED and CUT_TAKEN as they come, zero between launches
+  unsigned* pieces;   // [streams][row tiles]: CUT_STORED and CUT_TAKEN as they come, zero between launches; behind them (LIN_SLOTS) `looks`
 };
 enum { CUT_STORED = 1, CUT_TAKEN = 2 };
 template <int EPI>
@@ -729,9 +729,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     if (tid == 0) {
       unsigned* word = ls.pieces + at;
-      for (int i = 0; i < CUT_LOOKS && !__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); ++i) __builtin_amdgcn_s_sleep(8);
-      s_there = __hip_atomic_fetch_add(word, (unsigned)CUT_TAKEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (s_there) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int looks = (int)ls.pieces[LIN_SLOTS];
+      for (int i = 0; i < looks && !__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); ++i) __builtin_amdgcn_s_sleep(8);
+      const unsigned there = __hip_atomic_fetch_add(word, (unsigned)CUT_TAKEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (there) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      s_there = looks < 0 ? 0 : there;
     }
     __syncthreads();
     if (!s_there) return false;
@@ -743,28 +745,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     return true;
   };
   Operands p, q;
-  auto start = [&]() {
-#pragma unroll
-    for (int i = 0; i < RING; ++i) stage(lds + i * STAGE);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (RING - 1)) : "memory");
-    lds_barrier();
-    cur = 0;
-    read(lds, p);
-  };
-  start();
+  bool empty = true;  // the ring
   for (int f = f_last; f >= f_first; --f) {
     int at = f == f_first ? k_first : 0;
     const int end = f == f_last ? k_last : a.kt;
     clear();
     if (ls.streams && at > 0) {
-      const bool there = take();
+      empty = !take();
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): a step counts loads into LDS alone (the builtin: the compiler knows that the sums are here)
-      if (!there) {
+      if (empty) {
         lds_barrier();
-        at = k_in = 0;
+        at = k_in = cur = 0;
         to_in = end;
-        start();
       }
+    }
+    if (empty) {
+#pragma unroll
+      for (int i = 0; i < RING; ++i) stage(lds + i * STAGE);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (RING - 1)) : "memory");
+      lds_barrier();
+      read(lds, p);
+      empty = false;
     }
     for (; at < end; at += 2) {  // (stretches and parts are even)
       step(p, q);
@@ -991,7 +992,7 @@ static int allow_lds(K k, int bytes) {
 // step of 64 columns takes a workgroup of 128 x 128 alone on its compute unit 0.4 us (0.6 with weights out of HBM), two of them 1.0 - 1.08; one of 256 x 256
 // takes 1.17 us, and 1.55 when all of them run (the card's clock).  Both start and end in 3 and 8 us; a part more writes and reads its sums.
 // Stretches (LinStream) leave no compute unit empty, but their rows and weights meet in L2 less often (1.72 us), and tiles that they cut are stored and read:
-// 2000 rows and 2048 x 16896 132 us, by 128 x 128 163, by 256 x 256 159; 7168 x 32896 779, 1066, 878; but 1500 rows and 7168 x 27648 522, 658, 520.
+// 2000 rows and 2048 x 16896 132 us, by 128 x 128 163, by 256 x 256 163; 7168 x 32896 762, 1066, 868; 1500 rows and 7168 x 27648 518, 658, 526.
 // In 32 bits a step of 64 columns takes a workgroup of 128 rows alone 1.08 us (1.5 with weights out of HBM), two of them 2.45, and one of 64 rows 0.64, three of them 1.96 (us by 128 and
 // by 64 rows: 301 rows and 2048 x 16896 78 and 62, 2000 rows 347 and 365; 301 rows and 2048 x 2176 40 and 25).
 enum { LIN_SMALL, LIN_HALF, LIN_BIG, LIN_STREAM };  // (the second: 64 rows instead of 128, 32 bits)

@@ -70,7 +70,8 @@ int lin_parts(int rows, int rt, int kt, bool f32, int most);
 int lin_parts_fixed(int rows, int rt, int kt, bool f32, int most);     // launch_lin, where a router reads what comes of the sums
 int lin_parts_few(int rt, int kt, int most);
 // room for the fronts of tiles that two workgroups share: a slot of 256 x 256 sums for each of 256 compute units (64 MiB, allocated
-// with a model one of whose products takes it at some number of rows), and their words (zero between launches)
+// with a model one of whose products takes it at some number of rows), and their words (zero between launches), with one more behind them: how often a
+// workgroup looks for such a front before it adds that up itself (negative: it always does)
 enum { LIN_SLOTS = 256, LIN_SLOT_FLOATS = 256 * 256 };
 struct LinSpace {
   float* sums;

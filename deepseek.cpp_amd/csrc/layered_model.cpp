@@ -130,6 +130,7 @@ struct LayeredModel : ModelHead {
   bool chunk_scan = true;
   int tile = 0;                     // of prompt products (LinArgs::tile)
   LinSpace space{};                 // of prompt products
+  int cut_looks = 64;               // of its workgroups for each other's sums
   ChunkScan scan{};                 // operands of the recurrences over chunks (kernels_chunk_scan.hip)
   int max_chunks = 0;
   float* attn_part = nullptr;       // parts of attention outputs (kernels_mix_few.hip)
@@ -607,7 +608,8 @@ int alloc_work(LayeredModel* m) {
       streams |= !m->f32 && p->w && lin_streams_some((int)n, p->rt, p->kt, m->tile);
   if (streams) {
     DSK_TRY(dev_alloc_n(m, &m->space.sums, (size_t)LIN_SLOTS * LIN_SLOT_FLOATS));
-    DSK_TRY(dev_alloc_n(m, &m->space.pieces, LIN_SLOTS));
+    DSK_TRY(dev_alloc_n(m, &m->space.pieces, LIN_SLOTS + 1));
+    HIP_TRY(hipMemcpyAsync(m->space.pieces + LIN_SLOTS, &m->cut_looks, sizeof(int), hipMemcpyHostToDevice, m->ctx->stream));
     m->space.slots = LIN_SLOTS;
   }
   DSK_TRY(dev_alloc_n(m, &m->x_all, n * D));
@@ -1719,6 +1721,7 @@ int set_options(LayeredModel* m, const char* options) {
       m->enter_spins = (unsigned)v;
     }
     else if (k == "chunk_scan") m->chunk_scan = v != 0;
+    else if (k == "cut_looks") m->cut_looks = v;
     else if (k == "prompt_tile") {
       if (v != 0 && v != 128 && v != 256) DSK_FAIL(DSK_ERR_INVALID, "open: prompt_tile %d (0, 128, 256)", v);
       m->tile = v;

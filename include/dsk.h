@@ -452,7 +452,8 @@ int dsk_bench_router(dsk_ctx* ctx, int n_routed, int dim, int ksplit, int flags,
  * "decode_graph" (1: steps of single tokens replay a captured graph), "fused_decode" (1: the fused launches for such steps),
  * "chunk_scan" (1: prompts run their recurrences over chunks of tokens as matrix products; 0: token by token), "prompt_tile"
  * (tiles of prompt products in bfloat16: 128 or 256 rows and features, the latter in stretches over several tiles where they can be; 0, the default:
- * whichever is faster; all give the same bits), "enter_ahead" (1: steps of up
+ * whichever is faster; all give the same bits), "cut_looks" (how often a workgroup looks for what its neighbour leaves it of such a tile before it adds up
+ * the whole itself, negative: it always does; the same bits either way), "enter_ahead" (1: steps of up
  * to 8 single tokens make a layer's rows in the launch of the product that reads them; 0: in one of their own), "enter_spins" (how often a
  * workgroup of such a launch looks for its rows before the step fails).  Behind a step that failed so its sequences have no valid state: they take
  * no further step and can only be closed (dsk_forward's own starts anew at position 0), and the model's later steps go as with enter_ahead=0. */
