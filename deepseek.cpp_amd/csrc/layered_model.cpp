@@ -1721,7 +1721,10 @@ int set_options(LayeredModel* m, const char* options) {
       m->enter_spins = (unsigned)v;
     }
     else if (k == "chunk_scan") m->chunk_scan = v != 0;
-    else if (k == "cut_looks") m->cut_looks = v;
+    else if (k == "cut_looks") {
+      if (v > 1 << 16) DSK_FAIL(DSK_ERR_INVALID, "open: cut_looks %d (up to 65536)", v);
+      m->cut_looks = v;
+    }
     else if (k == "prompt_tile") {
       if (v != 0 && v != 128 && v != 256) DSK_FAIL(DSK_ERR_INVALID, "open: prompt_tile %d (0, 128, 256)", v);
       m->tile = v;
