@@ -135,11 +135,11 @@ __global__ __launch_bounds__(256) void conv_kernel(const PassDesc p, int D, cons
   }
 }
 // The same with four channels a thread, by loads and stores of 16 bytes a lane: rows are requested as their places come, and the sums of a row are the same, in
-// the same order.  From 4 M elements on (us with one channel / with four, without blends and with): 2048 channels of 700 rows 5.8 / 7.3 and 15.2 / 16.9, of 2000 8.6 / 8.7
+// the same order.  Beyond 4 M elements (us with one channel / with four, without blends and with): 2048 channels of 700 rows 5.8 / 7.3 and 15.2 / 16.9, of 2000 8.6 / 8.7
 // and 19.3 / 19.9, of 4000 15.1 / 13.1 and 32.9 / 25.3; 7168 channels of 300 rows 6.4 / 7.1 and 16.0 / 17.1, of 500 7.5 / 7.5 and 20.0 / 19.2, of 2000 20.3 / 17.8 and
 // 40.9 / 31.1; in 32 bits, 2000 rows, 22.1 / 18.8.  (Slower in a few places where rows are a power of two apart: 4096 channels of 1600 rows 10.8 / 14.8.)
 static bool conv_wide(const PassDesc& p, int D, const ConvArgs& a) {
-  return a.taps >= 2 && a.taps <= 4 && !(D & 3) && !(a.ld & 3) && (size_t)p.n_chunks * D >= 1 << 18;
+  return a.taps >= 2 && a.taps <= 4 && !(D & 3) && !(a.ld & 3) && (size_t)p.n_chunks * D > 1 << 18;
 }
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_wide_kernel(const PassDesc p, int D, const float* __restrict__ h_f, const ConvArgs a) {
