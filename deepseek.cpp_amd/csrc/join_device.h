@@ -209,7 +209,10 @@ DEV void join_row(const JoinArgs& a, int block, JoinLds<NT>& lds) {
         load_v<float, V>(a.pair_wa + at(i), at(i) < D, wa);
         load_v<float, V>(a.pair_wb + at(i), at(i) < D, wb);
 #pragma unroll
-        for (int e = 0; e < V; ++e) add[i][e] = 0.5f * (add[i][e] * ra * wa[e] + vb[i][e] * rb * wb[e]);
+        for (int e = 0; e < V; ++e) {  // (of the two products one is rounded, in rows of up to 1024 that four does not divide the first: see squares)
+          const float u = add[i][e] * ra, v = vb[i][e] * rb;
+          add[i][e] = 0.5f * (NT == 256 && V == 1 ? fmaf(v, wb[e], product(u, wa[e])) : fmaf(u, wa[e], product(v, wb[e])));
+        }
       }
     } else if (a.post_w) {
       const float sa = block_sum<NT>(squares<VPT, V, V == 1 ? 0 : 1>(add), red);

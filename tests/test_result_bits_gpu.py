@@ -27,15 +27,19 @@ def sandwich():
     return U.sandwich([U.no_ff(U.wkv(7, 72)), U.no_ff(U.head_delta(3, 3, 128, 64)), U.no_ff(U.latent(3, 64, 16, 64, 36, 28, 50))], width=2048, vocab=208)
 
 
+def odd():
+    return U.mixed(250, vocab=208)  # (routers, pairs of mixers, a width that four does not divide)
+
+
 # last tokens of prompts of one, three and more row tiles, of several at once, and of two steps behind them
-LENGTHS = {"routed": ((40,), (301,), (1300, 77), (2048,)), "sandwich": ((45,), (17, 3, 130))}
+LENGTHS = {"routed": ((40,), (301,), (1300, 77), (2048,)), "sandwich": ((45,), (17, 3, 130)), "odd": ((45,), (17, 3, 130))}
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
-@pytest.mark.parametrize("design", ["routed", "sandwich"])
+@pytest.mark.parametrize("design", ["routed", "sandwich", "odd"])
 def test_logits_keep_their_bits(ctx, design, dtype):
     import dsk
-    c = {"routed": routed, "sandwich": sandwich}[design]()
+    c = {"routed": routed, "sandwich": sandwich, "odd": odd}[design]()
     lm, rng, got = dsk.LM(ctx, dtype=dtype, config=c, seed=3), np.random.default_rng(11), {}
     for lengths in LENGTHS[design]:
         seqs = [lm.seq_open() for _ in lengths]
