@@ -255,6 +255,23 @@ struct MoeFfnArgs {
   int tap_stride;
   double algo_bytes;
 };
+// The routed experts' W2 + the shared expert's + the combine, rows of x owned by workgroups (kernels_experts.hip); K-quant planes, one GPU.
+struct MoeDownArgs {
+  const float* hb;       // hidden vectors [slot][hb_stride] (slot K: the shared expert's)
+  const int* route_e;
+  const float* route_w;
+  float* x;              // residual stream
+  float* eout;           // slot outputs [slot][dim]
+  const uint8_t *w2_qs, *w2_sc, *w2_hm, *w2_dm, *sw2_qs, *sw2_sc, *sw2_hm, *sw2_dm;
+  int quant, K, hb_stride, mi, shared_n, dim, n_experts;
+  int lpr_log2;          // lanes per row: the generic plan's
+  int rows_wg, grid, cw, lds_b, lds, div_nb, div_rows;  // filled by moe_down_plan; cw: waves that multiply, the others stage
+  int8_t* tap_qs;        // parity taps (dsk_model_run_block): slot s's staged hidden vector at s * tap_stride
+  float* tap_d;
+  int tap_stride;
+};
+int moe_down_plan(MoeDownArgs& a, int n_cus);
+int launch_moe_down(hipStream_t st, const MoeDownArgs& a);
 int moe_ffn_plan(MoeFfnArgs& a, int n_cus);
 int launch_moe_ffn(hipStream_t st, const MoeFfnArgs& a, hipEvent_t ev_start, hipEvent_t ev_stop);
 int moe_ffn_plan_tile(MoeFfnArgs& a, int n_cus);

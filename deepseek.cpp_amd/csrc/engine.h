@@ -94,6 +94,7 @@ struct dsk_model : ModelHead {
   std::vector<int> lp_sh13;  // shared expert's w1/w3 GLU riding in the router launch (-1: it is a task of lp_w13)
   // routed experts in one launch (kernels_moe.hip); grid == 0: the layer keeps the two-launch form (lp_w13, lp_w2)
   std::vector<MoeFfnArgs> moe_ffn;
+  std::vector<MoeDownArgs> moe_down;  // grid == 0: the layer's second half is the generic launch lp_w2
   bool att_q8_in_wo = false;       // DSK_ATT_Q8_IN_WO=1: wo quantises the attention output in its own prologue (no finisher hand-off in the attention launch)
   bool fuse_moe = true;            // DSK_NO_FUSE_MOE at model creation switches it off (A/B, bit-identity tests)
   unsigned* moe_ctr = nullptr;     // slot_ctr[16] | slot_pass[16]
@@ -115,6 +116,7 @@ struct dsk_model : ModelHead {
                                     // uniformly drawn experts - a measurement of balanced routing; the shipped library has no way to set it
   int hydrate_tap_layer = -1;       // option "hydrate_tap_layer" (parity harness): the block whose intermediates a batched chunk copies aside for
                                     // dsk_hydrate_get_buffer; the chunk itself runs unchanged
+  bool expert_launches = true;      // option "expert_launches": the experts' launches of latency-bound models (kernels_experts.hip)
   int gemv_ahead = 3;               // option "gemv_ahead" (bits): 1 the first-stage projection launch, 2 wo request weights ahead of the staging of their vector (round 6, kernels_gemv.hip)
   bool hydrate_batched = true;      // option "hydrate_batched": 0 = dsk_hydrate always runs the per-token loop
   bool hydrate_tile_copies = true;  // option "hydrate_tile_copies": the batched path may keep tile-record copies of the plane-layout Q2_K matrices (hydrate.cpp)

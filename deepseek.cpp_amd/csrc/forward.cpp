@@ -151,6 +151,9 @@ int build_plans(dsk_model* m) {
     MoeFfnArgs z;
     memset(&z, 0, sizeof z);
     m->moe_ffn.assign(nl, z);
+    MoeDownArgs d;
+    memset(&d, 0, sizeof d);
+    m->moe_down.assign(nl, d);
   }
   for (int l = 0; l < nl; ++l) {
     Layer& L = m->L[l];
@@ -380,6 +383,21 @@ int build_plans(dsk_model* m) {
       else { h.comb_geometry = 1; h.zero_absent = 1; }
       h.algo_bytes = bytes;
       DSK_TRY(add_plan(m, h, &m->lp_w2[l]));
+      if (kq && !w2.tiled && !m->sharded() && m->expert_launches) {
+        MoeDownArgs a;
+        memset(&a, 0, sizeof a);
+        a.hb = m->hb; a.route_e = ae; a.route_w = aw; a.x = m->x; a.eout = m->eout;
+        a.w2_qs = w2.qs; a.w2_sc = w2.sc; a.w2_hm = w2.hm; a.w2_dm = w2.dm;
+        if (c.n_shared_experts > 0) {
+          const DTensor& s2 = L.t[DSK_ROLE_SHARED_W2];
+          a.sw2_qs = s2.qs; a.sw2_sc = s2.sc; a.sw2_hm = s2.hm; a.sw2_dm = s2.dm;
+          a.shared_n = shared_n;
+        }
+        a.quant = wq; a.K = K; a.hb_stride = hb_stride; a.mi = mi; a.dim = c.dim; a.n_experts = c.n_routed_experts;
+        a.lpr_log2 = m->plans[m->lp_w2[l]].lpr_log2;
+        if (moe_down_plan(a, m->ctx->n_cus) == DSK_OK) m->moe_down[l] = a;
+        else dsk_clear_error();  // the generic launch then
+      }
     }
     // 8+9 in ONE launch (kernels_moe.hip): K-quants, one GPU, the shared expert's w1/w3 riding in the router launch
     // (or no shared expert).  Same lanes per row as the two plans above => bit-identical results.
@@ -498,21 +516,25 @@ void free_plans(dsk_model* m) {
   m->plans_dev = nullptr;
 }
 
-static int run_plan(dsk_model* m, const char* name, int idx) {
-  if (idx < 0) DSK_FAIL(DSK_ERR_STATE, "missing launch plan for %s", name);
+template <typename F>
+static int run_timed(dsk_model* m, const char* name, double bytes, F launch) {
   if (m->profiling && !m->class_filter) {
     // the kernel's own dispatch timestamps (hipExtLaunchKernel): in-situ duration, as rocprofv3 reports it
     Prof p;
-    DSK_TRY(prof_begin(m, name, m->plans[idx].algo_bytes, &p, false));
+    DSK_TRY(prof_begin(m, name, bytes, &p, false));
     g_prof_start = p.e0; g_prof_stop = p.e1;
-    int r = gemv_launch(m->ctx->stream, m->plans_dev + idx, m->plans[idx]);
+    int r = launch();
     g_prof_start = g_prof_stop = nullptr;
     DSK_TRY(r);
     m->ktimes[p.idx].ev.push_back({p.e0, p.e1});
     return DSK_OK;
   }
-  PROFILED(name, m->plans[idx].algo_bytes, gemv_launch(m->ctx->stream, m->plans_dev + idx, m->plans[idx]));
+  PROFILED(name, bytes, launch());
   return DSK_OK;
+}
+static int run_plan(dsk_model* m, const char* name, int idx) {
+  if (idx < 0) DSK_FAIL(DSK_ERR_STATE, "missing launch plan for %s", name);
+  return run_timed(m, name, m->plans[idx].algo_bytes, [&] { return gemv_launch(m->ctx->stream, m->plans_dev + idx, m->plans[idx]); });
 }
 
 // ---------------------------------------------------------------------------------
@@ -658,6 +680,15 @@ static int ffn(dsk_model* m, int l) {
     return DSK_OK;
   }
   DSK_TRY(run_plan(m, "gemv_experts_w13", m->lp_w13[l]));
+  if (m->moe_down[l].grid > 0) {
+    MoeDownArgs a = m->moe_down[l];
+    if (m->stage_layer == l && m->tap_qs) {
+      a.tap_qs = m->tap_qs + m->tap_off_hb;
+      a.tap_d = m->tap_d + m->tap_off_hb / 256;
+      a.tap_stride = a.hb_stride;
+    }
+    return run_timed(m, "gemv_experts_w2", m->plans[m->lp_w2[l]].algo_bytes, [&] { return launch_moe_down(st, a); });
+  }
   DSK_TRY(run_plan(m, "gemv_experts_w2", m->lp_w2[l]));
   if (exchange || (m->sharded() && m->class_filter)) {
     // every routed slot is non-zero on exactly one rank: a sum all-reduce is exact and order-independent

@@ -465,7 +465,7 @@ DEV void stage_f32(const SRC& T, float* l_x, int tid, float* scratch) {
 
 // parity tap: the staged item records of an n-vector back to the linear Q8_K form (int8 codes, block scales)
 template <int LAY>
-__device__ __attribute__((noinline)) void dump_staged_q8(const uint8_t* lds, int n, int8_t* qs, float* d, int tid, int nthreads) {
+DEV void dump_staged_q8_inline(const uint8_t* lds, int n, int8_t* qs, float* d, int tid, int nthreads) {
   constexpr bool Q2META = LAY == LAY_Q2;
   if (LAY == LAY_TILE) {
     for (int i = tid; i < (n >> 4); i += nthreads)
@@ -482,6 +482,10 @@ __device__ __attribute__((noinline)) void dump_staged_q8(const uint8_t* lds, int
     const float* m = reinterpret_cast<const float*>(lds + (size_t)b * 4 * ITEM_LDS + 72);
     d[b] = Q2META ? m[1] : m[0];
   }
+}
+template <int LAY>
+__device__ __attribute__((noinline)) void dump_staged_q8(const uint8_t* lds, int n, int8_t* qs, float* d, int tid, int nthreads) {
+  dump_staged_q8_inline<LAY>(lds, n, qs, d, tid, nthreads);
 }
 
 template <int QT>

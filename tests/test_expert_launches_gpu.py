@@ -1,0 +1,67 @@
+"""The experts' launches of latency-bound models (kernels_experts.hip, option "expert_launches") against the generic launches: the same arithmetic per
+row in the same order, so logits, routing, slot outputs and the residual stream have to be the same bits."""
+import numpy as np
+import pytest
+
+from tools import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def same(ctx, c, T=None, seed=None, tokens=(5, 9, 700, 3, 44), options=None):
+    import dsk
+    o = dict({"fuse_moe": 0, "q2k_tiles": 0}, **(options or {}))
+    A, B = (dsk.Model(ctx, c, T, synth_seed=seed, options=dict(o, expert_launches=on)) for on in (1, 0))
+    for graph in (True, False):
+        for m in (A, B):
+            m.set_graph(graph)
+        for pos, tok in enumerate(tokens):
+            la, lb = A.forward(tok, pos), B.forward(tok, pos)
+            assert np.all(np.isfinite(lb)) and np.array_equal(la, lb), (graph, pos)
+            for a, b in zip(A.routing(), B.routing()):
+                assert np.array_equal(a, b), (graph, pos)
+            assert np.array_equal(A.slot_outputs(), B.slot_outputs()), (graph, pos)
+    x = np.random.default_rng(1).standard_normal(c.dim).astype(np.float32)
+    layer = c.first_k_dense_replace
+    assert np.array_equal(A.run_block(layer, x, 2), B.run_block(layer, x, 2))
+    n = (c.n_active_routed + (c.n_shared_experts > 0)) * max(1, c.n_shared_experts) * c.moe_intermediate_size
+    for name, count, dt in (("q8.hb.qs", n, np.int8), ("q8.hb.d", n // 256, np.float32)):  # what the slots staged
+        assert np.array_equal(A.stage(name, count, dt).view(np.uint8), B.stage(name, count, dt).view(np.uint8)), name
+    A.close()
+    B.close()
+
+
+# rows of x per workgroup 1 (a part of the workgroups' rows missing) and 2; hidden vectors of 1 - 3 blocks; K = 1; without a shared expert
+SMALL = [dict(), dict(dim=768, moe_intermediate_size=512), dict(n_shared_experts=0, moe_intermediate_size=768), dict(n_active_routed=1, n_shared_experts=1),
+         dict(n_active_routed=8, dim=256)]
+
+
+@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+@pytest.mark.parametrize("over", SMALL, ids=[",".join(f"{k[:8]}{v}" for k, v in o.items()) or "tiny" for o in SMALL])
+def test_small_shapes_same_bits(ctx, quant, over):
+    c = synth.preset("tiny_v2lite", quant, False, **over)
+    same(ctx, c, synth.synth_model(c, seed=7))
+
+
+@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+def test_v2lite_shapes_same_bits(ctx, quant):
+    c = synth.preset("v2lite", quant, False, n_layers=3, max_seq_len=64)
+    same(ctx, c, seed=5, tokens=(5, 90000, 3))
+
+
+@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+def test_largest_values_of_both_signs_in_a_block(ctx, quant):
+    """hidden values in pairs v, -v: a block's largest magnitude occurs with both signs, and the first one's sign decides the codes"""
+    c = synth.preset("tiny_v2lite", quant, False)
+    T = synth.synth_model(c, seed=11)
+    at = (81, 83) if quant == "q2_k" else (109,)  # the high bytes of the block's float16 factors
+    per = 84 if quant == "q2_k" else 110
+    for name, t in T.items():
+        if ".mlp.w1." in name or "shared_mlp.w1." in name:
+            t.data[..., 1::2, :] = t.data[..., 0::2, :]
+        if ".mlp.w3." in name or "shared_mlp.w3." in name:
+            d = t.data[..., 0::2, :].copy().reshape(-1, per)
+            for b in at:
+                d[:, b] ^= 0x80
+            t.data[..., 1::2, :] = d.reshape(t.data[..., 0::2, :].shape)
+    same(ctx, c, T)
