@@ -270,6 +270,31 @@ struct MoeDownArgs {
   float* tap_d;
   int tap_stride;
 };
+// ... their w1 / w3, the gate in front and the shared expert's: behind launch_router_scores
+struct MoeUpArgs {
+  const float* scores;   // router rows' scores (E)
+  const int8_t* a_qs;    // Q8_K of rmsnorm(x)
+  const float* a_d;
+  const int16_t* a_bsums;
+  const float* bias;     // the gate's (null: none)
+  int *route_e;          // K experts and weights, E scores: written by workgroup 0
+  float *route_w, *scores_out;
+  float* hb;             // hidden vectors [slot][hb_stride]
+  const uint8_t *w1_qs, *w1_sc, *w1_hm, *w1_dm, *w3_qs, *w3_sc, *w3_hm, *w3_dm;
+  const uint8_t *sw1_qs, *sw1_sc, *sw1_hm, *sw1_dm, *sw3_qs, *sw3_sc, *sw3_hm, *sw3_dm;
+  int quant, E, K, hb_stride, mi, shared_n, dim, act;
+  int norm_topk_prob, scoring;
+  float scaling;
+  int lpr_log2;          // lanes per row: the generic plan's
+  int grid, lds;         // filled by moe_up_plan
+  unsigned div_mi;
+  int8_t* tap_qs;        // parity tap: the staged vector
+  float* tap_d;
+};
+struct RouterArgs;
+int moe_up_plan(MoeUpArgs& a, int n_cus);
+int launch_router_scores(hipStream_t st, const RouterArgs& r, float* xn);  // r.q_qs or xn: rmsnorm(x) left behind as Q8_K or in 32 bits
+int launch_moe_up(hipStream_t st, const MoeUpArgs& a);
 int moe_down_plan(MoeDownArgs& a, int n_cus);
 int launch_moe_down(hipStream_t st, const MoeDownArgs& a);
 int moe_ffn_plan(MoeFfnArgs& a, int n_cus);

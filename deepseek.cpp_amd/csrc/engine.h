@@ -94,6 +94,7 @@ struct dsk_model : ModelHead {
   std::vector<int> lp_sh13;  // shared expert's w1/w3 GLU riding in the router launch (-1: it is a task of lp_w13)
   // routed experts in one launch (kernels_moe.hip); grid == 0: the layer keeps the two-launch form (lp_w13, lp_w2)
   std::vector<MoeFfnArgs> moe_ffn;
+  std::vector<MoeUpArgs> moe_up;      // grid == 0: the router launch with the gate, the generic launch lp_w13
   std::vector<MoeDownArgs> moe_down;  // grid == 0: the layer's second half is the generic launch lp_w2
   bool att_q8_in_wo = false;       // DSK_ATT_Q8_IN_WO=1: wo quantises the attention output in its own prologue (no finisher hand-off in the attention launch)
   bool fuse_moe = true;            // DSK_NO_FUSE_MOE at model creation switches it off (A/B, bit-identity tests)

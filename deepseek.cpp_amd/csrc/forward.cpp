@@ -154,6 +154,9 @@ int build_plans(dsk_model* m) {
     MoeDownArgs d;
     memset(&d, 0, sizeof d);
     m->moe_down.assign(nl, d);
+    MoeUpArgs u;
+    memset(&u, 0, sizeof u);
+    m->moe_up.assign(nl, u);
   }
   for (int l = 0; l < nl; ++l) {
     Layer& L = m->L[l];
@@ -397,6 +400,27 @@ int build_plans(dsk_model* m) {
         a.lpr_log2 = m->plans[m->lp_w2[l]].lpr_log2;
         if (moe_down_plan(a, m->ctx->n_cus) == DSK_OK) m->moe_down[l] = a;
         else dsk_clear_error();  // the generic launch then
+        MoeUpArgs u;
+        memset(&u, 0, sizeof u);
+        u.scores = m->router_partial; u.a_qs = m->a_xb.qs; u.a_d = m->a_xb.d; u.a_bsums = m->a_xb.bsums;
+        u.bias = L.t[DSK_ROLE_MOEGATE_BIAS].bound() ? reinterpret_cast<const float*>(L.t[DSK_ROLE_MOEGATE_BIAS].qs) : nullptr;
+        u.route_e = m->route_e + (size_t)l * K; u.route_w = m->route_w + (size_t)l * K; u.scores_out = m->gate_scores + (size_t)l * c.n_routed_experts;
+        u.hb = m->hb;
+        u.w1_qs = w1.qs; u.w1_sc = w1.sc; u.w1_hm = w1.hm; u.w1_dm = w1.dm;
+        u.w3_qs = w3.qs; u.w3_sc = w3.sc; u.w3_hm = w3.hm; u.w3_dm = w3.dm;
+        if (c.n_shared_experts > 0) {
+          const DTensor &s1 = L.t[DSK_ROLE_SHARED_W1], &s3 = L.t[DSK_ROLE_SHARED_W3];
+          u.sw1_qs = s1.qs; u.sw1_sc = s1.sc; u.sw1_hm = s1.hm; u.sw1_dm = s1.dm;
+          u.sw3_qs = s3.qs; u.sw3_sc = s3.sc; u.sw3_hm = s3.hm; u.sw3_dm = s3.dm;
+          u.shared_n = shared_n;
+        }
+        u.quant = wq; u.E = c.n_routed_experts; u.K = K; u.hb_stride = hb_stride; u.mi = mi; u.dim = c.dim; u.act = c.act;
+        u.norm_topk_prob = c.norm_topk_prob; u.scoring = c.scoring_func; u.scaling = c.routed_scaling_factor;
+        u.lpr_log2 = m->plans[m->lp_w13[l]].lpr_log2;
+        // (one wave decides: no groups; the router's slices as in router_gate_kernel<2>; the shared expert's rows are this launch's)
+        const bool own = c.topk_method != DSK_TOPK_GROUP_LIMITED_GREEDY && m->router_ksplit >= 8 && m->lp_sh13[l] < 0 && m->moe_down[l].grid > 0;
+        if (own && moe_up_plan(u, m->ctx->n_cus) == DSK_OK) m->moe_up[l] = u;
+        else dsk_clear_error();
       }
     }
     // 8+9 in ONE launch (kernels_moe.hip): K-quants, one GPU, the shared expert's w1/w3 riding in the router launch
@@ -648,7 +672,9 @@ static int ffn(dsk_model* m, int l) {
   r.scores_out = m->gate_scores + (size_t)l * E;
   if (is_kq(c.weight_quant) && c.dim % 256 == 0) { r.q_qs = m->a_xb.qs; r.q_d = m->a_xb.d; r.q_bsums = m->a_xb.bsums; }
   if (m->moe_ffn[l].grid > 0) { r.zero_ctr = m->moe_ffn[l].slot_ctr; r.zero_n = std::min(16, std::max(K, m->n_slots)); }  // re-arm the expert launch's slot counters
-  if (m->lp_sh13[l] >= 0) {
+  if (m->moe_up[l].grid > 0 && m->moe_ffn[l].grid <= 0) {
+    DSK_TRY(run_timed(m, "router_gate", (double)E * c.dim * 4 + c.dim * 8.0, [&] { return launch_router_scores(st, r, nullptr); }));
+  } else if (m->lp_sh13[l] >= 0) {
     const GemvLaunch& hs = m->plans[m->lp_sh13[l]];
     PROFILED("router_gate", (double)E * c.dim * 4 + c.dim * 8.0 + hs.algo_bytes, launch_router_shared(st, r, m->plans_dev + m->lp_sh13[l], hs));
   } else {
@@ -679,7 +705,13 @@ static int ffn(dsk_model* m, int l) {
     }
     return DSK_OK;
   }
-  DSK_TRY(run_plan(m, "gemv_experts_w13", m->lp_w13[l]));
+  if (m->moe_up[l].grid > 0) {
+    MoeUpArgs u = m->moe_up[l];
+    if (m->stage_layer == l && m->tap_qs) { u.tap_qs = m->tap_qs + m->tap_off_xffn; u.tap_d = m->tap_d + m->tap_off_xffn / 256; }
+    DSK_TRY(run_timed(m, "gemv_experts_w13", m->plans[m->lp_w13[l]].algo_bytes, [&] { return launch_moe_up(st, u); }));
+  } else {
+    DSK_TRY(run_plan(m, "gemv_experts_w13", m->lp_w13[l]));
+  }
   if (m->moe_down[l].grid > 0) {
     MoeDownArgs a = m->moe_down[l];
     if (m->stage_layer == l && m->tap_qs) {

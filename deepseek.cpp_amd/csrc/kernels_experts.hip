@@ -2,8 +2,10 @@
 // bytes (one GPU, K-quant planes; V2-Lite's shapes): rows of x owned by workgroups in the second half.
 //
 // Replaces, for the selected experts e_0..e_{K-1} of a token (src/infer.cpp:853-878, 899-903), the launches of the generic multi-task GEMV:
+//     router rows' scores, rmsnorm(x) left behind                             router_scores_kernel
+//     moe_gate, h_k = act(W1[e_k] xb) * (W3[e_k] xb), the shared expert's too  experts_up_kernel
 //     o_k  = W2[e_k] h_k,  x += w_k * o_k  (k order),  x += shared_out        experts_down_kernel
-// Lanes per row, column steps, trees of lanes and the order of the combine are the generic launches': the same bits.
+// Nothing is handed over inside a launch.  Lanes per row, column steps, trees of lanes and the order of the combine are the generic launches': the same bits.
 #include "dsk_internal.h"
 #include "gemv_device.h"
 
@@ -74,10 +76,209 @@ DEV void q8k_four_blocks_lds(const f32x4 (&t)[4], int lane, uint8_t* blk) {
   }
 }
 
+// moe_gate for up to 64 experts without groups (src/infer.cpp:493-599) by ONE wave, lane e = expert e: the softmax's trees and the order of the sum of the
+// weights are gate_body's (router_device.h), whose other 15 waves only add zeros here; the k rounds of "largest unmasked, first among equals" are k
+// rounds of a wave maximum.  Returns in lane k < K the k-th expert, w its weight; sc: the lane's expert's score.
+DEV int gate_wave(float v, float bias, bool has_bias, int lane, int E, int K, int scoring, int norm_topk_prob, float scaling, float& sc, float& w) {
+  if (scoring == DSK_SCORE_SOFTMAX) {  // src/infer.cpp:472-487
+    float mx = v;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, lane_xor(mx, off));
+    const float ex = lane < E ? expf(v - mx) : 0.f;
+    float sum = ex;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) sum += lane_xor(sum, off);
+    v = ex / sum;
+  } else {
+    v = 1.0f / (1.0f + expf(-v));  // sigmoid, src/infer.cpp:489-491
+  }
+  if (has_bias) v += bias;
+  if (lane >= E) v = -INFINITY;
+  sc = v;
+  float left = v;
+  unsigned long long taken = 0;
+  int sel = 0;
+  float sk = 0.f, wsum = 0.f;
+  for (int k = 0; k < K; ++k) {
+    const float m = ad::wave_max_dpp(left);
+    unsigned long long at = __ballot(left == m && lane < E) & ~taken;
+    if (at == 0) at = ~taken;  // (scores that are no numbers: the first ones left; K <= E)
+    const int e = __builtin_ctzll(at);
+    taken |= 1ull << e;
+    const float s = u2f(__builtin_amdgcn_readlane(__builtin_bit_cast(u32, v), e));
+    wsum += s;
+    if (lane == k) { sel = e; sk = s; }
+    if (lane == e) left = -INFINITY;
+  }
+  if (!norm_topk_prob) wsum = 1.0f;
+  w = sk / wsum * scaling;
+  return sel;
+}
+
+// An argument read at entry, with the others, in one trip.  The compiler reads a kernel's arguments where they are used, a trip each, and turns
+// `cond ? a.p : a.q` into a choice between their two places and a read behind it.
+template <typename T>
+DEV T arg(T v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
 // v / d for 0 <= v < 2^16 / d (moe_down_plan looks at the range): m = ceil(2^16 / d)
 DEV int div_small(int v, int m) { return (v * m) >> 16; }
 
 }  // namespace
+
+// ------------------------------------------------------------------------------------------------------------
+// The router's rows (src/infer.cpp:839, 847): workgroup = 2 rows x 8 column slices, slices added in order like router_gate_kernel's.  The gate is the next
+// launch's, so nothing is published, counted or waited for here; and a wave's weights do not wait for the norm's scale: everything is requested at
+// entry.  Workgroup b leaves block b of rmsnorm(x) behind, as Q8_K or in 32 bits.  64 experts of 2048 columns: 7.5 us with the gate in the last workgroup to
+// arrive, 4.9 here.
+// ------------------------------------------------------------------------------------------------------------
+template <int NL>  // 256-column pieces of a slice
+__global__ __launch_bounds__(1024) void router_scores_kernel(const float* __restrict__ x, const float* __restrict__ norm_w, const float* __restrict__ w, float* __restrict__ scores,
+                                                            int dim, int E, float eps, int8_t* q_qs, float* q_d, int16_t* q_bsums, float* xn) {
+  constexpr int SL = 8;
+  __shared__ float scratch[16], part[16];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x;
+  const int r = wave & 1, sl = wave >> 1, row = min(bid * 2 + r, E - 1);
+  const int k0 = sl * NL * 256;
+  f32x4 xs, xv[NL], nw[NL], wv[NL];
+  xs = *reinterpret_cast<const f32x4*>(x + min(tid * 4, dim - 4));
+#pragma unroll
+  for (int k = 0; k < NL; ++k) {
+    const int i = min(k0 + k * 256, dim - 256) + lane * 4;
+    xv[k] = *reinterpret_cast<const f32x4*>(x + i);
+    nw[k] = *reinterpret_cast<const f32x4*>(norm_w + i);
+    wv[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w + (size_t)row * dim + i));
+  }
+  // the sum of squares and its trees as in router_norm_scale (dim <= 4096: a thread has one piece)
+  float ss = 0.f;
+  if (tid * 4 < dim) {
+    ss = fmaf(xs.x, xs.x, ss);
+    ss = fmaf(xs.y, xs.y, ss);
+    ss = fmaf(xs.z, xs.z, ss);
+    ss = fmaf(xs.w, xs.w, ss);
+  }
+  ss = wave_sum(ss);
+  if (lane == 0) scratch[wave] = ss;
+  lds_barrier();
+  const float scale = 1.0f / sqrtf(scratch_total<16>(scratch) / (float)dim + eps);
+  float acc = 0.f;
+#pragma unroll
+  for (int k = 0; k < NL; ++k) {
+    if (k0 + k * 256 >= dim) continue;  // wave-uniform
+    const float y[4] = {xv[k].x * scale * nw[k].x, xv[k].y * scale * nw[k].y, xv[k].z * scale * nw[k].z, xv[k].w * scale * nw[k].w};
+    acc = fmaf(wv[k].x, y[0], acc);
+    acc = fmaf(wv[k].y, y[1], acc);
+    acc = fmaf(wv[k].z, y[2], acc);
+    acc = fmaf(wv[k].w, y[3], acc);
+    const int b = (k0 >> 8) + k;
+    if (r == 0 && b % (int)gridDim.x == bid) {
+      if (q_qs) ad::q8k_block(y, lane, q_qs + (size_t)b * 256, q_d + b, q_bsums + (size_t)b * 16);
+      else *reinterpret_cast<f32x4*>(xn + b * 256 + lane * 4) = f32x4{y[0], y[1], y[2], y[3]};
+    }
+  }
+  acc = wave_sum(acc);
+  if (lane == 0) part[wave] = acc;
+  lds_barrier();
+  if (tid < 2 && bid * 2 + tid < E) {
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < SL; ++k) v += part[k * 2 + tid];
+    scores[bid * 2 + tid] = v;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// First half: every workgroup decides the gate for itself out of the scores (one wave, ~0.5 us: less than handing a decision over), while other waves stage the
+// normed vector; then its share of the shared expert's and of the chosen experts' rows, all of a wave's requested at once.  Bound by latency (16.5 MB: 2.5
+// us): V2-Lite's shapes in Q2_K 9.4 us by the generic launch, whose waves took two rounds, 7.3 here; with the router's launch a token 1303 -> 1130 us.
+// ------------------------------------------------------------------------------------------------------------
+template <int QT>
+__global__ __launch_bounds__(1024) void experts_up_kernel(const float* __restrict__ scores, const int8_t* __restrict__ a_qs, const float* __restrict__ a_d,
+                                                         const int16_t* __restrict__ a_bsums, int E, int K, const MoeUpArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ int sel_s[64];
+  constexpr int CW = 12;  // waves that multiply; three stage, one decides
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x, G = gridDim.x;
+  const int lpr_log2 = arg(a.lpr_log2), RPW = 64 >> lpr_log2;
+  const uint8_t *w1_qs = arg(a.w1_qs), *w1_sc = arg(a.w1_sc), *w1_dm = arg(a.w1_dm), *w3_qs = arg(a.w3_qs), *w3_sc = arg(a.w3_sc), *w3_dm = arg(a.w3_dm);
+  const uint8_t *sw1_qs = arg(a.sw1_qs), *sw1_sc = arg(a.sw1_sc), *sw1_dm = arg(a.sw1_dm), *sw3_qs = arg(a.sw3_qs), *sw3_sc = arg(a.sw3_sc), *sw3_dm = arg(a.sw3_dm);
+  const uint8_t *w1_hm = nullptr, *w3_hm = nullptr, *sw1_hm = nullptr, *sw3_hm = nullptr;
+  if (QT == DSK_QUANT_Q3_K) { w1_hm = arg(a.w1_hm); w3_hm = arg(a.w3_hm); sw1_hm = arg(a.sw1_hm); sw3_hm = arg(a.sw3_hm); }
+  float* const hb = glob(arg(a.hb));
+  const float* const bias_p = glob(arg(a.bias));
+  const int mi = arg(a.mi), shared_n = arg(a.shared_n), dim = arg(a.dim), act = arg(a.act), hb_stride = arg(a.hb_stride), scoring = arg(a.scoring), norm_topk = arg(a.norm_topk_prob);
+  const float scaling = arg(a.scaling);
+  const u32 div_mi = arg(a.div_mi);
+  int8_t* const tap_qs = glob(arg(a.tap_qs));
+  if (wave == 15) {
+    const int e = lane < E ? lane : E - 1;
+    const float v = scores[e], bias = bias_p ? bias_p[e] : 0.f;
+    float sc, w;
+    const int sel = gate_wave(lane < E ? v : -INFINITY, bias, bias_p != nullptr, lane, E, K, scoring, norm_topk, scaling, sc, w);
+    sel_s[lane] = sel;
+    if (bid == 0) {
+      if (lane < E) a.scores_out[lane] = sc;
+      if (lane < K) { a.route_e[lane] = sel; a.route_w[lane] = w; }
+    }
+  } else if (wave >= CW) {
+    for (int i = tid - CW * 64; i < dim >> 4; i += 192) {  // runs of 16 codes, their sums and their block's scale into item records (stage_q8)
+      const u32x4 run = reinterpret_cast<const u32x4*>(a_qs)[i];
+      const int bs = a_bsums[i];
+      const float d = a_d[i >> 4];
+      const int b = i >> 4, j = i & 15, h = j >> 3, sidx = (j >> 1) & 3, lh = j & 1;
+      uint8_t* rec = smem + (size_t)(b * 4 + 2 * h + lh) * ITEM_LDS;
+      *reinterpret_cast<u32x4*>(rec + sidx * 16) = run;
+      float* m = reinterpret_cast<float*>(rec + 72);
+      if (QT == DSK_QUANT_Q2_K) {
+        rec[64 + sidx] = (uint8_t)(bs >> 8);
+        rec[68 + sidx] = (uint8_t)(bs & 0xff);
+        m[0] = d * 0.0625f;
+        m[1] = d;
+      } else {
+        reinterpret_cast<short*>(rec + 64)[sidx] = (short)bs;
+        m[0] = d;
+      }
+    }
+  }
+  lds_barrier();
+  if (tap_qs && bid == 0) dump_staged_q8_inline<QT == DSK_QUANT_Q2_K>(smem, dim, tap_qs, a.tap_d, tid, 1024);
+  if (wave >= CW) return;
+  const int rloc = lane >> lpr_log2, sub = lane & ((1 << lpr_log2) - 1), q = sub & 3, nb = dim >> 8, items = 1 << lpr_log2;
+  // this workgroup's rows of the shared expert and of the chosen ones (slot-major), each an even share, in steps of RPW rows
+  const int s_lo = (int)((unsigned)(shared_n * bid) / (unsigned)G), s_hi = (int)((unsigned)(shared_n * (bid + 1)) / (unsigned)G);
+  const int v_lo = (int)((unsigned)(K * mi * bid) / (unsigned)G), v_hi = (int)((unsigned)(K * mi * (bid + 1)) / (unsigned)G);
+  const int JS = (s_hi - s_lo + RPW - 1) >> (6 - lpr_log2), J = JS + ((v_hi - v_lo + RPW - 1) >> (6 - lpr_log2));
+  const uint8_t* lds_lane = smem + sub * ITEM_LDS;
+  struct Step { ChunkKQ<QT, 1, 1, true> c; int out; };
+  auto request = [&](int j, Step& S) {
+    const bool sh = j < JS;  // wave-uniform
+    const int v = (sh ? s_lo + j * RPW : v_lo + (j - JS) * RPW) + rloc, end = sh ? s_hi : v_hi;
+    const bool valid = j < J && v < end;
+    const int vv = min(v, max(end - 1, 0)), slot = sh ? K : min((int)__umulhi((u32)vv, div_mi), K - 1), rr = sh ? vv : vv - slot * mi;
+    S.out = valid ? slot * hb_stride + rr : -1;
+    const int rowblk[1] = {((sh ? 0 : sel_s[slot] * mi) + rr) * nb + (sub >> 2)};
+    KQRsrc B;
+    B.qs = make_rsrc_n(sh ? sw1_qs : w1_qs, j < J); B.sc = make_rsrc_n(sh ? sw1_sc : w1_sc, j < J);
+    B.dm = make_rsrc_n(sh ? sw1_dm : w1_dm, j < J); B.hm = make_rsrc_n(sh ? sw1_hm : w1_hm, j < J);
+    B.qs2 = make_rsrc_n(sh ? sw3_qs : w3_qs, j < J); B.sc2 = make_rsrc_n(sh ? sw3_sc : w3_sc, j < J);
+    B.dm2 = make_rsrc_n(sh ? sw3_dm : w3_dm, j < J); B.hm2 = make_rsrc_n(sh ? sw3_hm : w3_hm, j < J);
+    load_chunk_kq<QT, 1, 1, true>(S.c, B, 1, items, sub, lpr_log2, q, rowblk, 0);
+  };
+  auto finish = [&](const Step& S) {
+    float acc[1] = {0.f}, acc2[1] = {0.f};
+    compute_chunk_kq<QT, 1, 1, true>(S.c, 1, items, sub, lpr_log2, q, 0, lds_lane, acc, acc2);
+    const float g = lanes_sum(acc[0], lpr_log2), u = lanes_sum(acc2[0], lpr_log2);
+    if (sub == 0 && S.out >= 0) hb[S.out] = act_fn(g, act) * u;  // src/infer.cpp:859-872
+  };
+  for (int j = wave; j < J; j += 2 * CW) {
+    Step S0, S1;
+    request(j, S0);
+    request(j + CW, S1);  // (a step that is not there reads through an empty descriptor: no branch around its loads)
+    finish(S0);
+    finish(S1);
+  }
+}
 
 // ------------------------------------------------------------------------------------------------------------
 // Second half: workgroup b owns rows [b * rows_wg, +rows_wg) of x for ALL slots, so that nothing has to be handed over between workgroups (the
@@ -94,35 +295,39 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int NW = 16, U = QT == DSK_QUANT_Q2_K ? 6 : 4;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x;
+  const uint8_t *w2_qs = arg(a.w2_qs), *w2_sc = arg(a.w2_sc), *w2_dm = arg(a.w2_dm), *sw2_qs = arg(a.sw2_qs), *sw2_sc = arg(a.sw2_sc), *sw2_dm = arg(a.sw2_dm);
+  const uint8_t *w2_hm = nullptr, *sw2_hm = nullptr;
+  if (QT == DSK_QUANT_Q3_K) { w2_hm = arg(a.w2_hm); sw2_hm = arg(a.sw2_hm); }
+  float* const eout = glob(arg(a.eout));
+  const int mi = arg(a.mi), shared_n = arg(a.shared_n), dim = arg(a.dim), rows_wg = arg(a.rows_wg), lpr_log2 = arg(a.lpr_log2), lds_b = arg(a.lds_b), div_nb = arg(a.div_nb),
+            div_rows = arg(a.div_rows);
+  int8_t* const tap_qs = glob(arg(a.tap_qs));
   uint8_t* act = smem;                                                   // [slot][lds_b] item records
-  float* o_s = reinterpret_cast<float*>(smem + (size_t)a.lds_b * (K + 1));  // [slot][rows_wg]
-  const int nbR = a.mi >> 8, nbS = a.shared_n >> 8, slots = K + (nbS > 0 ? 1 : 0);
-  const int r_lo = bid * a.rows_wg, nrows = min(a.rows_wg, a.dim - r_lo);
-  // (everything of the arguments that is needed later is read now, in one trip: where it is used it would be one of its own)
-  asm volatile("" ::"s"(a.w2_qs), "s"(a.w2_sc), "s"(a.w2_dm), "s"(a.sw2_qs), "s"(a.sw2_sc), "s"(a.sw2_dm), "s"(a.eout), "s"(a.dim), "s"(a.rows_wg), "s"(a.lpr_log2),
-               "s"(a.lds_b), "s"(a.tap_qs));
+  float* o_s = reinterpret_cast<float*>(smem + (size_t)lds_b * (K + 1));  // [slot][rows_wg]
+  const int nbR = mi >> 8, nbS = shared_n >> 8, slots = K + (nbS > 0 ? 1 : 0);
+  const int r_lo = bid * rows_wg, nrows = min(rows_wg, dim - r_lo);
   float xv = 0.f, rw = 0.f;  // the rows' old values, the slots' weights (the last wave adds up)
   if (wave < cw) {
     const int e_all = route_e[lane < K ? lane : K - 1];
-    const int lpr_log2 = a.lpr_log2, RPW = 64 >> lpr_log2;
+    const int RPW = 64 >> lpr_log2;
     const int rloc = lane >> lpr_log2, sub = lane & ((1 << lpr_log2) - 1), q = sub & 3;
     // steps of RPW rows: the shared expert's first (its rows are the longest), then the routed slots' (slot, row) slot-major
-    const int WS = nbS > 0 ? (a.rows_wg + RPW - 1) >> (6 - lpr_log2) : 0, WR = (a.rows_wg * K + RPW - 1) >> (6 - lpr_log2);
+    const int WS = nbS > 0 ? (rows_wg + RPW - 1) >> (6 - lpr_log2) : 0, WR = (rows_wg * K + RPW - 1) >> (6 - lpr_log2);
     ChunkKQ<QT, 1, U, false> c;
     bool wait = true;
     for (int st = wave; st < WS + WR; st += cw) {
       const bool sh = st < WS;  // wave-uniform
       const int v = (sh ? st : st - WS) * RPW + rloc;
-      const int slot = sh ? K : min(div_small(v, a.div_rows), K - 1), rr0 = sh ? v : v - slot * a.rows_wg;
+      const int slot = sh ? K : min(div_small(v, div_rows), K - 1), rr0 = sh ? v : v - slot * rows_wg;
       const bool valid = rr0 < nrows;
       const int rr = valid ? rr0 : nrows - 1, nb = sh ? nbS : nbR, items = nb * 4, its = (items + (1 << lpr_log2) - 1) >> lpr_log2;
       const int e = sh ? 0 : __shfl(e_all, slot);
-      const int rowblk[1] = {(e * a.dim + r_lo + rr) * nb + (sub >> 2)};
+      const int rowblk[1] = {(e * dim + r_lo + rr) * nb + (sub >> 2)};
       WPtr P;
       P.present = true; P.qs2 = P.sc2 = P.hm2 = P.dm2 = nullptr; P.scale = P.scale2 = nullptr;
-      P.qs = sh ? a.sw2_qs : a.w2_qs; P.sc = sh ? a.sw2_sc : a.w2_sc; P.hm = sh ? a.sw2_hm : a.w2_hm; P.dm = sh ? a.sw2_dm : a.w2_dm;
+      P.qs = sh ? sw2_qs : w2_qs; P.sc = sh ? sw2_sc : w2_sc; P.hm = sh ? sw2_hm : w2_hm; P.dm = sh ? sw2_dm : w2_dm;
       const KQRsrc B = kq_rsrc<QT, false>(P);
-      const uint8_t* lds_lane = act + (size_t)slot * a.lds_b + sub * ITEM_LDS;
+      const uint8_t* lds_lane = act + (size_t)slot * lds_b + sub * ITEM_LDS;
       float acc[1] = {0.f}, dummy[1] = {0.f};
       for (int it0 = 0; it0 < its; it0 += U) {
         load_chunk_kq<QT, 1, U, false>(c, B, its, items, sub, lpr_log2, q, rowblk, it0);
@@ -131,7 +336,7 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
         compute_chunk_kq<QT, 1, U, false>(c, its, items, sub, lpr_log2, q, it0, lds_lane, acc, dummy);
       }
       const float o = lanes_sum(acc[0], lpr_log2);
-      if (sub == 0 && valid) o_s[slot * a.rows_wg + rr] = o;
+      if (sub == 0 && valid) o_s[slot * rows_wg + rr] = o;
     }
     if (wait) lds_barrier();
   } else {
@@ -140,11 +345,11 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
       f32x4 t0[4], t1[4];
       auto request = [&](int bb0, f32x4 (&t)[4]) {
         const int b = min(bb0 + r16, nblk - 1);  // (lanes past the end: the last block again, the same values to the same place)
-        const int s = b < K * nbR ? div_small(b, a.div_nb) : K, bb = b - s * nbR;
+        const int s = b < K * nbR ? div_small(b, div_nb) : K, bb = b - s * nbR;
         const float* src = hb + (size_t)s * hb_stride + bb * 256 + j * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) t[i] = *reinterpret_cast<const f32x4*>(src + 64 * i);
-        return act + (size_t)s * a.lds_b + (size_t)bb * 4 * ITEM_LDS;
+        return act + (size_t)s * lds_b + (size_t)bb * 4 * ITEM_LDS;
       };
       uint8_t* dst = request(b0, t0);
       uint8_t* const dst1 = request(b0 + sw * 4, t1);
@@ -162,15 +367,15 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
     rw = route_w[lane < K ? lane : K - 1];
     lds_barrier();
   }
-  if (a.tap_qs && bid == 0)  // parity tap: what the slots staged
+  if (tap_qs && bid == 0)  // parity tap: what the slots staged
     for (int s = 0; s < slots; ++s)
-      dump_staged_q8_inline<QT == DSK_QUANT_Q2_K>(act + (size_t)s * a.lds_b, s < K ? a.mi : a.shared_n, a.tap_qs + (size_t)s * a.tap_stride,
+      dump_staged_q8_inline<QT == DSK_QUANT_Q2_K>(act + (size_t)s * lds_b, s < K ? mi : shared_n, tap_qs + (size_t)s * a.tap_stride,
                                                  a.tap_d + (size_t)s * (a.tap_stride >> 8), tid, 1024);
   lds_barrier();
   if (wave == NW - 1 && lane < nrows) {  // x += w_k * o_k in k order (src/infer.cpp:874-877), then the shared expert (:900-903)
     for (int k = 0; k < slots; ++k) {
-      const float o = o_s[k * a.rows_wg + lane];
-      a.eout[(size_t)k * a.dim + r_lo + lane] = o;
+      const float o = o_s[k * rows_wg + lane];
+      eout[(size_t)k * dim + r_lo + lane] = o;
       if (k < K) xv = fmaf(o, u2f(__builtin_amdgcn_readlane(__builtin_bit_cast(u32, rw), k)), xv);
       else xv += o;
     }
@@ -179,6 +384,45 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
 }
 
 // ---- host side ------------------------------------------------------------------------------------------
+int moe_up_plan(MoeUpArgs& a, int n_cus) {
+  if (a.quant != DSK_QUANT_Q2_K && a.quant != DSK_QUANT_Q3_K) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: K-quant planes only");
+  if (a.E < 1 || a.E > 64 || a.K < 1 || a.K > a.E || a.K > 15 || a.mi < 1 || a.shared_n < 0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: shapes");
+  // rows of one column step; router slices of one or two pieces, the norm of one piece a thread
+  if (a.dim % 256 || a.dim > 4096 || a.dim / 64 != 1 << a.lpr_log2) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: rows of %d", a.dim);
+  if ((double)a.E * a.mi * (a.dim / 256) * 64.0 >= 2147483648.0 || (double)a.shared_n * (a.dim / 256) * 64.0 >= 2147483648.0)
+    DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: a stack exceeds the 31-bit offset of a buffer load");
+  // (v * ceil(2^32 / d) >> 32 == v / d while v * (d - 1) < 2^32)
+  if (a.mi < 2 || (double)a.K * a.mi * a.mi >= 4294967296.0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: too many rows");
+  a.div_mi = (unsigned)((4294967296ull + a.mi - 1) / a.mi);
+  const int rows = a.K * a.mi + a.shared_n, RPW = 64 >> a.lpr_log2;
+  a.grid = n_cus < (rows + RPW - 1) / RPW ? n_cus : (rows + RPW - 1) / RPW;
+  a.lds = a.dim / 64 * ITEM_LDS;
+  return DSK_OK;
+}
+
+int launch_router_scores(hipStream_t st, const RouterArgs& r, float* xn) {
+  auto go = [&](auto k) {
+    const dim3 grid((r.n_routed + 1) / 2), block(1024);
+    if (g_prof_start && g_prof_stop)
+      hipExtLaunchKernelGGL(k, grid, block, 0u, st, g_prof_start, g_prof_stop, 0u, r.x, r.norm_w, r.w, r.partial, r.dim, r.n_routed, r.eps, r.q_qs, r.q_d, r.q_bsums, xn);
+    else hipLaunchKernelGGL(k, grid, block, 0u, st, r.x, r.norm_w, r.w, r.partial, r.dim, r.n_routed, r.eps, r.q_qs, r.q_d, r.q_bsums, xn);
+  };
+  if (r.dim > 2048) go(router_scores_kernel<2>);  // (pieces of a slice as in router_body: ceil(dim / 2048))
+  else go(router_scores_kernel<1>);
+  return DSK_OK;
+}
+
+int launch_moe_up(hipStream_t st, const MoeUpArgs& a) {
+  auto go = [&](auto k) {
+    if (g_prof_start && g_prof_stop)
+      hipExtLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, g_prof_start, g_prof_stop, 0u, a.scores, a.a_qs, a.a_d, a.a_bsums, a.E, a.K, a);
+    else hipLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, a.scores, a.a_qs, a.a_d, a.a_bsums, a.E, a.K, a);
+  };
+  if (a.quant == DSK_QUANT_Q2_K) go(experts_up_kernel<DSK_QUANT_Q2_K>);
+  else go(experts_up_kernel<DSK_QUANT_Q3_K>);
+  return DSK_OK;
+}
+
 int moe_down_plan(MoeDownArgs& a, int n_cus) {
   const bool q2 = a.quant == DSK_QUANT_Q2_K, q3 = a.quant == DSK_QUANT_Q3_K;
   if (!q2 && !q3) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: K-quant planes only");

@@ -195,8 +195,8 @@ int dsk_model_destroy(dsk_model* m);
  *                        bias row) into the XCDs' L2 (0: off; results unaffected)
  *   "moe_q8_handoff"  1  fused expert launch: hidden vectors handed over as Q8_K, quantised once by their producers
  *   "fuse_moe_float"  1  fused expert launch for F8E5M2 / F16 / F32 weights too (0: two launches; bit-identical)
- *   "expert_launches" 1  K-quant experts that do not run as one launch: the second half by workgroups that own rows of x for every slot
- *                        (0: the generic launches; bit-identical)
+ *   "expert_launches" 1  K-quant experts that do not run as one launch: the gate inside the first half, the second half by workgroups that own rows of x
+ *                        for every slot (0: the router with the gate and the generic launches; bit-identical)
  *   "timeline"        0  in-kernel wall-clock stamps for dsk_model_get_timeline
  *   "moe_spin_limit"  0  polls before the fused expert launch's hand-off wait gives up (0: 2^20); < 0: fault
  *                        injection (a give-up is reported although the hand-off succeeded: exercises the fallback)
@@ -226,7 +226,7 @@ int dsk_model_set_option(dsk_model* m, const char* key, int value);
  * that hit it was re-run transparently), "fused_moe_layers", "graph_captured", "exchange_calls" (RCCL collectives this
  * model has enqueued eagerly), "tiled_tensors" (weight tensors held as tile records, option "q2k_tiles"),
  * "hydrate_batched_tokens" / "hydrate_looped_tokens", "hydrate_tile_copy_mb" (MiB of tile copies the batched prompt path holds),
- * "gemv_ahead_plans". */
+ * "gemv_ahead_plans", "expert_up_layers" / "expert_down_layers" (MoE blocks that run those launches, option "expert_launches"). */
 int dsk_model_get_info(dsk_model* m, const char* key, int* value);
 /* models created on the context and not yet destroyed (a context destroyed while models are alive is freed by the last
  * dsk_model_destroy) */

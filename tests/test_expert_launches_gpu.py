@@ -8,10 +8,13 @@ from tools import synth
 pytestmark = pytest.mark.gpu
 
 
-def same(ctx, c, T=None, seed=None, tokens=(5, 9, 700, 3, 44), options=None):
+def same(ctx, c, T=None, seed=None, tokens=(5, 9, 700, 3, 44), options=None, up=False):
     import dsk
     o = dict({"fuse_moe": 0, "q2k_tiles": 0}, **(options or {}))
     A, B = (dsk.Model(ctx, c, T, synth_seed=seed, options=dict(o, expert_launches=on)) for on in (1, 0))
+    blocks = c.n_layers - c.first_k_dense_replace
+    assert [m.info("expert_down_layers") for m in (A, B)] == [blocks, 0]
+    assert [m.info("expert_up_layers") for m in (A, B)] == [blocks if up else 0, 0]
     for graph in (True, False):
         for m in (A, B):
             m.set_graph(graph)
@@ -46,7 +49,24 @@ def test_small_shapes_same_bits(ctx, quant, over):
 @pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
 def test_v2lite_shapes_same_bits(ctx, quant):
     c = synth.preset("v2lite", quant, False, n_layers=3, max_seq_len=64)
-    same(ctx, c, seed=5, tokens=(5, 90000, 3))
+    same(ctx, c, seed=5, tokens=(5, 90000, 3), up=True)
+
+
+# the gate by one wave: an odd number of experts, all 64, as many as are chosen; sigmoid with a bias and normed weights; 32 and 64 lanes a row, two router
+# pieces a slice; rows that no workgroup count divides; no shared expert
+GATE = [dict(n_routed_experts=33, n_active_routed=5), dict(n_routed_experts=64, n_active_routed=8, n_shared_experts=0, moe_intermediate_size=768),
+        dict(n_routed_experts=3, n_active_routed=3), dict(dim=4096, n_routed_experts=16, scoring_func="sigmoid", has_moegate_bias=True, norm_topk_prob=True,
+                                                          routed_scaling_factor=2.5)]
+
+
+@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+@pytest.mark.parametrize("over", GATE, ids=["33 of 5", "64 of 8", "3 of 3", "sigmoid 4096"])
+def test_gate_inside_the_first_half_same_bits(ctx, quant, over):
+    over = dict(over)
+    if over.pop("has_moegate_bias", False):
+        over["arch"] = "DeepseekV3ForCausalLM"
+    c = synth.preset("v2lite", quant, False, **dict(dict(n_layers=2, hidden_dim=512, vocab_size=512, moe_intermediate_size=256, max_seq_len=64), **over))
+    same(ctx, c, seed=9, tokens=(5, 400, 3), up=True)
 
 
 @pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
