@@ -430,6 +430,26 @@ struct HeadAttnArgs {
 int head_attn_plan(HeadAttnArgs& A);
 int launch_head_attn(hipStream_t st, const HeadAttnArgs& A, const StepParams* sp, int max_kv, int n_split);
 int launch_attn_mha(hipStream_t st, const AttnMhaArgs& a, const StepParams* sp, int kv_len_override, int max_kv);
+// The same for models without a query latent, everything requested at once (kernels_head.hip); the output in 32 bits
+struct HeadShortArgs {
+  const uint8_t *qs, *sc, *hm, *dm;  // wkv_b
+  const float* scale;
+  float* out;            // (H, v)
+  int quant, nope, rope, lora, is_v3, lkv_log2, lds_kv, b0, b1, sh0, sh1, sc_cols;  // (sh: the shift of a power of two, else -1)
+  float eps;
+  unsigned long long* timeline;
+  int8_t* tap_qs;        // parity tap: the staged Q8_K vector of norm(kv_a[:lora])
+  float* tap_d;
+  int pf_wgs;            // HeadAttnArgs::pf_wgs
+  const void* pf_p[6];
+  int pf_n[6];
+  // the leading arguments of the launch
+  const float *kv_a, *norm_w, *q;
+  uint16_t *key_cache, *value_cache;
+  int H, hd, vd, sets, grid;  // grid == 0: head_attn_kernel
+};
+int head_short_plan(HeadShortArgs& S, const HeadAttnArgs& A, int max_kv);
+int launch_head_short(hipStream_t st, const HeadShortArgs& S, const StepParams* sp, int max_kv);
 struct AttnMlaArgs {
   float* q_rope;         // (H, rope)
   const float* q_c;      // (H, lora)

@@ -126,6 +126,8 @@ struct dsk_model : ModelHead {
   const char* hydrate_why = nullptr;  // why the last dsk_hydrate call looped (nullptr: it did not)
   std::vector<MlaHeadArgs> mla_head;   // per layer (MLA path)
   std::vector<double> head_attn_bytes;
+  bool head_short_opt = true;             // option "head_short"
+  std::vector<HeadShortArgs> head_short;  // per layer (MHA without a query latent); grid == 0: head_attn
   std::vector<HeadAttnArgs> head_attn;  // per layer (MHA path): second-stage projections + attention, one launch
   bool graph_primed[8] = {false, false, false, false, false, false, false, false};
   const char* class_filter = nullptr;  // dsk_time_kernel_class

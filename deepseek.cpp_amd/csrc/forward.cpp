@@ -140,6 +140,15 @@ int build_plans(dsk_model* m) {
   m->lp_w13.assign(nl, -1); m->lp_w2.assign(nl, -1); m->lp_sh13.assign(nl, -1);
   m->plans.clear();
   m->head_attn.assign(nl, HeadAttnArgs());
+  {
+    HeadShortArgs z;
+    memset(&z, 0, sizeof z);
+    m->head_short.assign(nl, z);
+  }
+  // Heads that go through launch_head_short leave their output in 32 bits, and wo's workgroups quantise it (K-quants): up to 16 blocks, one per wave.  V2-Lite
+  // (8 blocks): wo 4.8 -> 5.1 us.  (V3's 64: 9.5 -> 13.2, dearer than the hand-over between heads.)
+  const bool short_heads = m->head_short_opt && !c.use_mla && c.q_lora_rank == 0 && (!kq || (H * c.v_head_dim <= 4096 && H * c.v_head_dim % 256 == 0));
+  if (short_heads && kq) m->att_q8_in_wo = true;
   m->mla_head.assign(nl, MlaHeadArgs());
   {
     MlaFlashArgs z;
@@ -221,6 +230,7 @@ int build_plans(dsk_model* m) {
         DSK_TRY(head_attn_plan(A));
         A.a.out = m->att_out;
         m->head_attn[l] = A;
+        if (short_heads) DSK_TRY(head_short_plan(m->head_short[l], A, std::min(c.max_seq_len, std::max(1, c.rs_original_max_position_embeddings))));
         m->head_attn_bytes[l] = bytes;
       }
     }
@@ -273,7 +283,7 @@ int build_plans(dsk_model* m) {
       T.out = m->x; T.epilogue = EPI_ADD;
       h.algo_bytes = weight_bytes_2d(m, wq, T.rows, T.n) + io_bytes(wq, T.n, T.rows) + 4.0 * T.rows;
       h.timeline = m->timeline_of(2);
-      h.ahead = m->gemv_ahead & 2;  // (gemv_ahead_q8_kernel: the first row group's first half requested ahead of the vector's copy into LDS)
+      h.ahead = m->gemv_ahead & 2;  // (gemv_ahead_q8_kernel, gemv_ahead_kernel: the first weights requested ahead of the vector's staging)
       DSK_TRY(add_plan(m, h, &m->lp_wo[l]));
     }
     if (!L.is_moe) {
@@ -511,6 +521,12 @@ int build_plans(dsk_model* m) {
         if (m->L[l].is_moe) f32v(m->L[l].t[DSK_ROLE_MOEGATE_BIAS], c.n_routed_experts, &A.pf_p[3], &A.pf_n[3]);  // the gate workgroup's
         else if (m->lp_w2[l] >= 0) { A.pf_p[3] = m->plans_dev + m->lp_w2[l]; A.pf_n[3] = (int)sizeof(GemvLaunch); }  // dense block: w2's descriptor
         // (the step parameters - rope table - as a further range: no gain)
+        if (m->head_short[l].grid > 0) {
+          HeadShortArgs& S = m->head_short[l];
+          S.pf_wgs = A.pf_wgs;
+          memcpy(S.pf_p, A.pf_p, sizeof S.pf_p);
+          memcpy(S.pf_n, A.pf_n, sizeof S.pf_n);
+        }
       }
       if (c.use_mla && m->lp_wo[l] >= 0 && m->mla_head[l].a.n_heads > 0) {
         MlaHeadArgs& A = m->mla_head[l];
@@ -601,9 +617,15 @@ static int attention_mha(dsk_model* m, int l, int max_kv) {
     HA.tap_d = m->tap_d + m->tap_off_qa / 256;
     HA.tap_stride = (int)(m->tap_off_kva - m->tap_off_qa);
   }
-  PROFILED("attn_mha", m->head_attn_bytes[l] + (double)m->sp_host->kv_len * H * (hd + c.v_head_dim) * 2 + (double)H * (hd * 2 + c.v_head_dim * 11),
-           launch_head_attn(st, HA, m->sp_dev, max_kv,
-                            m->mha_split > 1 && m->sp_host->kv_len >= m->mha_split_min ? m->mha_split : 1));
+  const double attn_bytes = m->head_attn_bytes[l] + (double)m->sp_host->kv_len * H * (hd + c.v_head_dim) * 2 + (double)H * (hd * 2 + c.v_head_dim * 11);
+  const int n_split = m->mha_split > 1 && m->sp_host->kv_len >= m->mha_split_min ? m->mha_split : 1;
+  if (n_split == 1 && m->head_short[l].grid > 0) {
+    HeadShortArgs S = m->head_short[l];
+    if (HA.tap_qs) { S.tap_qs = HA.tap_qs + HA.tap_stride; S.tap_d = HA.tap_d + (HA.tap_stride >> 8); }
+    PROFILED("attn_mha", attn_bytes, launch_head_short(st, S, m->sp_dev, max_kv));
+  } else {
+    PROFILED("attn_mha", attn_bytes, launch_head_attn(st, HA, m->sp_dev, max_kv, n_split));
+  }
   DSK_TRY(run_plan(m, "gemv_wo", m->lp_wo[l]));  // residual: src/infer.cpp:832-834
   return DSK_OK;
 }

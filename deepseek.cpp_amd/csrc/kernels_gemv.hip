@@ -296,7 +296,8 @@ __global__ __launch_bounds__(NW * 64) void gemv_kernel(const GemvLaunch* __restr
 // (Straight-line on purpose: row length and lanes per row are template constants and a (task, row group) pair that does not exist
 // for a wave reads through a NULL buffer descriptor - zeros, no memory traffic - instead of being branched around.  With a load
 // inside a branch hipcc's waitcnt pass must assume either path at the join and waits for EVERYTHING before x is touched.)
-template <int ITEMS, int LL>
+// (NORM: false: the vector as it is, src/quant.cpp:616-653 alone - wo behind heads that leave 32-bit outputs, kernels_head.hip)
+template <int ITEMS, int LL, bool NORM = true>
 __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __restrict__ Lp, const float* __restrict__ x, const float* __restrict__ norm_w,
                                                          float eps) {
   constexpr int QT = DSK_QUANT_Q2_K, NW = 16, KB1 = 32 / NW, nb = ITEMS / 4, n = nb * 256, ITS = (ITEMS + (1 << LL) - 1) >> LL;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
   for (int k = 0; k < KB1; ++k) {
     const int b = wave + NW * k < nb ? wave + NW * k : nb - 1;  // (a wave without a k-th block re-reads the last one and drops it)
     t[k] = *reinterpret_cast<const f32x4*>(x + b * 256 + lane * 4);
-    wv[k] = *reinterpret_cast<const f32x4*>(norm_w + b * 256 + lane * 4);
+    if (NORM) wv[k] = *reinterpret_cast<const f32x4*>(norm_w + b * 256 + lane * 4);
   }
   // ---- 2. the descriptor, this workgroup's share, and the weights of (at most) two (task, row group) pairs ----
   const int rloc = lane >> LL, sub = lane & ((1 << LL) - 1), q = sub & 3;
@@ -354,26 +355,30 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
     load_chunk_kq<QT, 1, 2, false>(ch[j], B, ITS, ITEMS, sub, LL, q, rowblk, 0);
   }
   // ---- 3. rmsnorm (src/infer.cpp:601-611) + Q8_K of x into LDS: stage_q8's single-pass path, second half, LDS-only barriers ----
-  float ss = 0.f;
+  float scale = 1.f;
+  if constexpr (NORM) {
+    float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < KB1; ++k) {
-    if (wave + NW * k < nb) {
-      ss = fmaf(t[k].x, t[k].x, ss);
-      ss = fmaf(t[k].y, t[k].y, ss);
-      ss = fmaf(t[k].z, t[k].z, ss);
-      ss = fmaf(t[k].w, t[k].w, ss);
+    for (int k = 0; k < KB1; ++k) {
+      if (wave + NW * k < nb) {
+        ss = fmaf(t[k].x, t[k].x, ss);
+        ss = fmaf(t[k].y, t[k].y, ss);
+        ss = fmaf(t[k].z, t[k].z, ss);
+        ss = fmaf(t[k].w, t[k].w, ss);
+      }
     }
+    ss = wave_sum(ss);
+    if (lane == 0) scratch[wave] = ss;
+    lds_barrier();
+    const float total = scratch_total<NW>(scratch);
+    scale = 1.0f / sqrtf(total / (float)n + eps);
   }
-  ss = wave_sum(ss);
-  if (lane == 0) scratch[wave] = ss;
-  lds_barrier();
-  const float total = scratch_total<NW>(scratch);
-  const float scale = 1.0f / sqrtf(total / (float)n + eps);
 #pragma unroll
   for (int k = 0; k < KB1; ++k) {
     const int b = wave + NW * k;
     if (b < nb) {
-      float v[4] = {t[k].x * scale * wv[k].x, t[k].y * scale * wv[k].y, t[k].z * scale * wv[k].z, t[k].w * scale * wv[k].w};
+      float v[4] = {t[k].x, t[k].y, t[k].z, t[k].w};
+      if (NORM) { v[0] = v[0] * scale * wv[k].x; v[1] = v[1] * scale * wv[k].y; v[2] = v[2] * scale * wv[k].z; v[3] = v[3] * scale * wv[k].w; }
       q8k_block_lds<LAY_Q2>(v, lane, smem + (size_t)b * 4 * ITEM_LDS);
     }
   }
@@ -636,7 +641,7 @@ static bool gemv_kvwrite_ahead_ok(const GemvLaunch& h) {
   if (T0.act_mode != ACT_F32_NORM || T0.n != 1536 || h.lpr_log2 != 3) return false;  // (the one instantiation: 24 items at 8 lanes per row)
   for (int i = 0; i < h.n_tasks; ++i) {
     const GemvTask& T = h.t[i];
-    if (T.n != T0.n || T.a_f32 != T0.a_f32 || T.norm_w != T0.norm_w || T.act_mode != ACT_F32_NORM || T.e_qs != 0 || T.accum_w) return false;
+    if (T.n != T0.n || T.a_f32 != T0.a_f32 || T.norm_w != T0.norm_w || T.act_mode != T0.act_mode || T.e_qs != 0 || T.accum_w) return false;
   }
   return h.grid == h.grp_wg_end[0];
 }
@@ -648,10 +653,10 @@ static bool gemv_ahead_ok(const GemvLaunch& h) {
   // the instantiations: DeepSeek-V3 (rows of 7168: 112 items at 64 lanes per row, two column steps) and V2-Lite (rows of 2048: 32 items
   // at 32 lanes per row, one step)
   const bool v3 = T0.n == 7168 && h.lpr_log2 == 6 && h.U == 2, v2l = T0.n == 2048 && h.lpr_log2 == 5 && h.U == 1;
-  if (T0.act_mode != ACT_F32_NORM || !(v3 || v2l)) return false;
+  if (!(T0.act_mode == ACT_F32_NORM && (v3 || v2l)) && !(T0.act_mode == ACT_F32 && v2l && h.n_tasks == 1)) return false;
   for (int i = 0; i < h.n_tasks; ++i) {
     const GemvTask& T = h.t[i];
-    if (T.n != T0.n || T.a_f32 != T0.a_f32 || T.norm_w != T0.norm_w || T.act_mode != ACT_F32_NORM || T.e_qs != 0 || T.accum_w) return false;
+    if (T.n != T0.n || T.a_f32 != T0.a_f32 || T.norm_w != T0.norm_w || T.act_mode != T0.act_mode || T.e_qs != 0 || T.accum_w) return false;
   }
   const int RG = 16 * (64 >> h.lpr_log2);
   const long vtotal = h.t[h.n_tasks - 1].vrow_end, units = (vtotal + h.part_unit - 1) / h.part_unit;
@@ -1424,8 +1429,8 @@ static void launch_one(hipStream_t st, const GemvLaunch* dev, const GemvLaunch& 
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
     if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, a0, a1, a2, hn, hm, he, gw, gs);
     else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, a0, a1, a2, hn, hm, he, gw, gs);
-  } else if (QT == DSK_QUANT_Q2_K && R == 1 && (U == 2 || U == 1) && NW == 16 && (h.ahead & 1) && hn > 0 && hm == ACT_F32_NORM && gemv_ahead_ok(h)) {
-    auto k = U == 2 ? gemv_ahead_kernel<112, 6> : gemv_ahead_kernel<32, 5>;
+  } else if (QT == DSK_QUANT_Q2_K && R == 1 && (U == 2 || U == 1) && NW == 16 && hn > 0 && (hm == ACT_F32_NORM ? h.ahead & 1 : hm == ACT_F32 ? h.ahead & 2 : 0) && gemv_ahead_ok(h)) {
+    auto k = hm == ACT_F32 ? gemv_ahead_kernel<32, 5, false> : U == 2 ? gemv_ahead_kernel<112, 6> : gemv_ahead_kernel<32, 5>;
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
     if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, (const float*)a0, (const float*)a1, he);
     else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, (const float*)a0, (const float*)a1, he);
@@ -1509,6 +1514,7 @@ int gemv_ahead_kind(const GemvLaunch& h, bool kvwrite) {
   if (h.NW != 16 || h.R != 1 || h.bd_heads != 0 || h.n_groups != 1) return 0;
   const GemvTask& T = h.t[h.grp_t0[0]];
   if ((h.ahead & 1) && T.act_mode == ACT_F32_NORM && gemv_ahead_ok(h)) return 1;
+  if ((h.ahead & 2) && T.act_mode == ACT_F32 && gemv_ahead_ok(h)) return 1;
   if ((h.ahead & 2) && T.act_mode == ACT_Q8 && gemv_ahead_q8_ok(h)) return 2;
   return 0;
 }

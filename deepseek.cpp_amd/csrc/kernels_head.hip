@@ -1,0 +1,378 @@
+// kernels_head.hip -- MHA of one token for models without a query latent (src/infer.cpp:943-1049, 728-762): per head, the rows of wkv_b, RoPE, the cache
+// entries and attention in one launch, with everything that does not depend on anything requested at once.
+//
+// head_attn_kernel (kernels_gemv.hip) does the same as a chain: latents, rows, query, rope's inputs, cache write, keys, each a trip of 0.7 - 1 us behind a
+// barrier that waits for stores.  Of those only the latents -> rows -> current key and value depend on each other.  So: the latents, the query, the
+// rope's inputs and the head's rows are requested at entry, keys and values (of up to 256 positions) behind the first barrier; the current position's
+// key and value go from LDS into the scores and the mix, rounded as the cache rounds them, and to the cache at the very end; barriers are for LDS
+// only.  Values, sums and their orders are head_attn_kernel's: the same bits.  The output leaves in 32 bits; wo quantises it (8 blocks for V2-Lite: cheaper in each of
+// its workgroups than a hand-over between heads here).
+// Bound by latency: 16 workgroups.  V2-Lite at 62 positions, us: Q2_K 13.2 -> 6.9, F8E5M2 12.8 -> 9.1 (its 131 KB of rows are 2.7 us for the one compute unit); a token 1130 -> 985, 1602 -> 1505.
+#include "dsk_internal.h"
+#include "gemv_device.h"
+
+// RS x ROUNDS row sets of a wave, two rounds on their way
+template <int QT, int RS, int ROUNDS>
+__global__ __launch_bounds__(1024) void head_attn_short_kernel(const StepParams* __restrict__ sp, const float* __restrict__ kv_a, const float* __restrict__ norm_w,
+                                                              const float* __restrict__ q, uint16_t* kcache, uint16_t* vcache, int H, int hv, const HeadShortArgs A) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float q_s[256];
+  __shared__ __attribute__((aligned(16))) float kvb_s[512];
+  __shared__ __attribute__((aligned(16))) uint16_t kr_s[128];  // this position's rotated key part, as the cache holds it
+  __shared__ __attribute__((aligned(16))) float part[4096];
+  constexpr bool KQ = QT == DSK_QUANT_Q2_K || QT == DSK_QUANT_Q3_K;
+  constexpr int NW = 16, NT = 1024, VN = RS == 4 ? 2 : QT == DSK_QUANT_Q3_K ? 4 : 8;  // (VN: values of a thread requested early; as many as the registers hold)
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, h = blockIdx.x;
+  if (h >= H) {  // prefetch workgroups (HeadAttnArgs::pf_wgs)
+    tail_prefetch(A.pf_p, A.pf_n, tid, NT);
+    return;
+  }
+  const unsigned long long t_entry = A.timeline ? wall_clock64() : 0ull;
+  unsigned long long t_staged = 0, t_rows = 0, t_scores = 0, t_mix = 0;
+  const int hd = hv & 0xffff, vd = hv >> 16, nope = A.nope, rope = A.rope, n = A.lora, nrows = nope + vd, half = rope >> 1;
+  uint8_t* act = smem;
+  float* att = reinterpret_cast<float*>(smem + A.lds_kv);
+  // ---- requests.  What few waves need comes first: an older load in a branch does not blur what the compiler knows of the ones behind it ----
+  f32x4 lt, lw;
+  float2 qp, kp, cs;
+  float qn;
+  const bool latent_wave = wave < (n + 255) >> 8, rope_wave = wave == NW - 1, q_wave = wave >= 8 && wave < 8 + ((nope + 63) >> 6);
+  const bool latent = tid * 4 < n;  // (n is a multiple of 256 for K-quants; float rows may end inside a wave)
+  if (rope_wave) {
+    const int i = min(lane, half - 1);
+    qp = *reinterpret_cast<const float2*>(q + (size_t)h * hd + nope + 2 * i);
+    kp = *reinterpret_cast<const float2*>(kv_a + n + 2 * i);
+    cs = *reinterpret_cast<const float2*>(sp->rope_cs + 2 * i);
+  }
+  if (q_wave) qn = q[(size_t)h * hd + min(tid - 512, nope - 1)];
+  if (latent_wave) {
+    const int i = latent ? tid * 4 : n - 4;
+    lt = *reinterpret_cast<const f32x4*>(kv_a + i);
+    lw = *reinterpret_cast<const f32x4*>(norm_w + i);
+  }
+  const int lpr_log2 = A.lkv_log2, RPW = 64 >> lpr_log2, rloc = lane >> lpr_log2, sub = lane & ((1 << lpr_log2) - 1);
+  const int base = wave * RPW + rloc, sets_stride = NW * RPW;
+  WPtr P;
+  P.present = true; P.qs = A.qs; P.sc = A.sc; P.hm = A.hm; P.dm = A.dm; P.scale = A.scale; P.qs2 = P.sc2 = P.hm2 = P.dm2 = nullptr; P.scale2 = nullptr;
+  struct Rows {
+    ChunkKQ<KQ ? QT : DSK_QUANT_Q2_K, RS, 1, false> k;
+    u32x4 w[RS];
+    float sv[RS];
+  };
+  auto request_rows = [&](Rows& R, int set0) {
+    int row[RS];
+#pragma unroll
+    for (int r = 0; r < RS; ++r) row[r] = h * nrows + min(base + (set0 + r) * sets_stride, nrows - 1);
+    if constexpr (KQ) {
+      int rowblk[RS];
+#pragma unroll
+      for (int r = 0; r < RS; ++r) rowblk[r] = row[r] * (n >> 8) + (sub >> 2);
+      load_chunk_kq<QT, RS, 1, false>(R.k, kq_rsrc<QT, false>(P), 1, 1 << lpr_log2, sub, lpr_log2, sub & 3, rowblk, 0);
+    } else {  // (one exact column step: the item of a lane is its place in the row)
+      constexpr int EPI = FTraits<KQ ? DSK_QUANT_F16 : QT>::EPI, ESZ = 16 / EPI;
+      const int sc_col = A.sh1 >= 0 ? sub * EPI >> A.sh1 : sub * EPI / A.b1;
+#pragma unroll
+      for (int r = 0; r < RS; ++r) {
+        R.w[r] = ldg_nt(reinterpret_cast<const u32x4*>(P.qs + (size_t)row[r] * n * ESZ + sub * 16));
+        R.sv[r] = QT == DSK_QUANT_F8E5M2 && P.scale ? P.scale[(A.sh0 >= 0 ? row[r] >> A.sh0 : row[r] / A.b0) * A.sc_cols + sc_col] : 1.0f;
+      }
+    }
+  };
+  Rows ra, rb;
+  request_rows(ra, 0);
+  request_rows(rb, RS);
+  const int kv_pos = sp->kv_pos, kv_len = sp->kv_len, kv_sink = sp->kv_sink;
+  // ---- rmsnorm of the latent (src/infer.cpp:950, 601-611): the sum of squares in the order of the two forms of head_attn_kernel ----
+  if (latent_wave) {
+    float ss = 0.f;
+    if constexpr (KQ) ss = fmaf(lt.x, lt.x, fmaf(lt.y, lt.y, fmaf(lt.z, lt.z, lt.w * lt.w)));
+    else if (latent) {
+      ss = fmaf(lt.x, lt.x, ss);
+      ss = fmaf(lt.y, lt.y, ss);
+      ss = fmaf(lt.z, lt.z, ss);
+      ss = fmaf(lt.w, lt.w, ss);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) scratch[wave] = ss;
+  } else if (lane == 0) {
+    scratch[wave] = 0.f;
+  }
+  lds_barrier();
+  // ---- keys and values: 16 lanes a position, positions 4 wave .. + 3 of every 64; thread (g, i4) positions g, g + TG, ... ----
+  const int grp = lane >> 4, sl = lane & 15;
+  const int tpp = vd >> 2, TG = NT / tpp, g = tid / tpp, i4 = tid - g * tpp;
+  if (kv_sink > 0) {  // rotation of the sink keys by one position, in f16 (src/infer.cpp:1008-1020)
+    for (int r = 0; r < kv_sink; ++r) {
+      uint16_t* kh = kcache + ((size_t)r * H + h) * hd + nope;
+      float re = 0.f, im = 0.f;
+      if (tid < half) ad::rope_rot(ad::h2f(kh[2 * tid]), ad::h2f(kh[2 * tid + 1]), sp->rope_cs1[2 * tid], sp->rope_cs1[2 * tid + 1], re, im);
+      __syncthreads();
+      if (tid < half) {
+        kh[A.is_v3 ? 2 * tid : tid] = ad::f2h(re);
+        kh[A.is_v3 ? 2 * tid + 1 : tid + half] = ad::f2h(im);
+      }
+      __syncthreads();
+    }
+  }
+  // (buffer loads: one lane offset each for keys and values, the steps in scalar registers, and zeros without traffic behind the context's end)
+  const u32 krow = (u32)H * hd * 2, vrow = (u32)H * vd * 2;
+  const rsrc_t KB = __builtin_amdgcn_make_buffer_rsrc(kcache, 0, (int)(kv_len * krow), 0x00020000), VB = __builtin_amdgcn_make_buffer_rsrc(vcache, 0, (int)(kv_len * vrow), 0x00020000);
+  const u32 koff = ((u32)(wave * 4 + grp) * H + h) * hd * 2 + sl * 8;
+  const u32 voff = g < TG ? ((u32)g * H + h) * vd * 2 + i4 * 8 : 0xfffffff0u;
+  const bool in2 = 128 + sl * 4 < hd, in1 = 64 + sl * 4 < hd, in0 = sl * 4 < hd;
+  ad::f16x4 k[4][3], v[VN];
+  auto request_keys = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (t0 + u * 64 >= kv_len) break;
+      const int step = (t0 + u * 64) * (int)krow;
+      k[u][0] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(KB, (int)koff, step, 0));
+      k[u][1] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(KB, (int)koff + 128, step, 0));
+      k[u][2] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(KB, (int)koff + 256, step, 0));
+    }
+  };
+  request_keys(0);
+#pragma unroll
+  for (int j = 0; j < VN; ++j)
+    if (j * TG < kv_len) v[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(VB, (int)voff, j * TG * (int)vrow, 0));
+  // ---- the latent staged; the query and this position's key part rotated ----
+  if (latent_wave) {
+    if constexpr (KQ) {
+      float total = 0.f;
+      for (int i = 0; i < n >> 8; ++i) total += scratch[i];
+      const float scale = 1.0f / sqrtf(total / (float)n + A.eps);
+      const float y[4] = {lt.x * scale * lw.x, lt.y * scale * lw.y, lt.z * scale * lw.z, lt.w * scale * lw.w};
+      q8k_block_lds<QT == DSK_QUANT_Q2_K>(y, lane, act + (size_t)wave * 4 * ITEM_LDS);
+    } else {
+      const float scale = 1.0f / sqrtf(scratch_total<NW>(scratch) / (float)n + A.eps);
+      constexpr int EPI = FTraits<KQ ? DSK_QUANT_F16 : QT>::EPI;
+      if (latent) reinterpret_cast<f32x4*>(act)[quad_place<EPI>(tid, n / EPI)] = lt * scale * lw;
+    }
+  }
+  if (rope_wave) {
+    if (lane < half) {
+      float re, im;
+      const int a = A.is_v3 ? 2 * lane : lane, b = A.is_v3 ? 2 * lane + 1 : lane + half;
+      ad::rope_rot(qp.x, qp.y, cs.x, cs.y, re, im);
+      q_s[nope + a] = re;
+      q_s[nope + b] = im;
+      ad::rope_rot(kp.x, kp.y, cs.x, cs.y, re, im);
+      kr_s[a] = ad::f2h(re);
+      kr_s[b] = ad::f2h(im);
+    }
+  }
+  if (q_wave && tid - 512 < nope) q_s[tid - 512] = qn;
+  lds_barrier();
+  if (A.timeline) t_staged = wall_clock64();
+  if constexpr (KQ) {
+    if (A.tap_qs && h == 0) dump_staged_q8_inline<QT == DSK_QUANT_Q2_K>(act, n, A.tap_qs, A.tap_d, tid, NT);
+  }
+  // ---- the head's rows of wkv_b ----
+  f32x4 xa4[KQ ? 1 : FTraits<KQ ? DSK_QUANT_F16 : QT>::EPI / 4];
+  if constexpr (!KQ) {
+    constexpr int EPI = FTraits<KQ ? DSK_QUANT_F16 : QT>::EPI;
+#pragma unroll
+    for (int i = 0; i < EPI / 4; ++i) xa4[i] = reinterpret_cast<const f32x4*>(act)[i * (n / EPI) + sub];  // (quad_place)
+  }
+  auto finish_rows = [&](const Rows& R, int set0) {
+    float acc[RS], dummy[RS];
+#pragma unroll
+    for (int r = 0; r < RS; ++r) acc[r] = 0.f;
+    if constexpr (KQ) compute_chunk_kq<QT, RS, 1, false>(R.k, 1, 1 << lpr_log2, sub, lpr_log2, sub & 3, 0, act + sub * ITEM_LDS, acc, dummy);
+    else {
+#pragma unroll
+      for (int r = 0; r < RS; ++r) acc[r] = fmaf(fitem<QT>(R.w[r], reinterpret_cast<const float*>(xa4), 0.f), R.sv[r], 0.f);
+    }
+#pragma unroll
+    for (int r = 0; r < RS; ++r) {
+      const float o = lanes_sum(acc[r], lpr_log2);
+      if (sub == 0 && base + (set0 + r) * sets_stride < nrows) kvb_s[base + (set0 + r) * sets_stride] = o;
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r += 2) {
+    finish_rows(ra, r * RS);
+    if (r + 2 < ROUNDS) request_rows(ra, (r + 2) * RS);
+    finish_rows(rb, (r + 1) * RS);
+    if (r + 2 < ROUNDS) request_rows(rb, (r + 3) * RS);
+  }
+  lds_barrier();
+  if (A.timeline) t_rows = wall_clock64();
+  // ---- scores ----
+  {
+    float qv[3][4];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const f32x4 t = *reinterpret_cast<const f32x4*>(q_s + min(64 * j + sl * 4, hd - 4));
+      const bool in = 64 * j + sl * 4 < hd;
+      qv[j][0] = in ? t.x : 0.f; qv[j][1] = in ? t.y : 0.f; qv[j][2] = in ? t.z : 0.f; qv[j][3] = in ? t.w : 0.f;
+    }
+    const float inv = sqrtf((float)hd);
+    const int pw = wave * 4 + grp;
+    for (int t0 = 0; t0 < kv_len; t0 += 256) {
+      if ((kv_pos & 63) == pw && kv_pos >= t0 && kv_pos < t0 + 256) {  // this position's key is not in the cache yet
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const int d0 = min(64 * j + sl * 4, hd - 4);
+          const f32x4 x = *reinterpret_cast<const f32x4*>(kvb_s + min(d0, nope - 4));
+          const ad::f16x4 y = *reinterpret_cast<const ad::f16x4*>(kr_s + max(d0 - nope, 0));
+          const ad::f16x4 c = d0 < nope ? ad::f16x4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w} : y;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (u == (kv_pos - t0) >> 6) k[u][j] = c;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + u * 64 + pw;
+        if (t0 + u * 64 >= kv_len) break;
+        float p = 0.f;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (j == 0 ? in0 : j == 1 ? in1 : in2) {
+            p = fmaf(qv[j][0], (float)k[u][j].x, p);
+            p = fmaf(qv[j][1], (float)k[u][j].y, p);
+            p = fmaf(qv[j][2], (float)k[u][j].z, p);
+            p = fmaf(qv[j][3], (float)k[u][j].w, p);
+          }
+        p = ad::row16_sum(p);
+        if (sl == 0 && t < kv_len) att[t] = p / inv;
+      }
+      if (t0 + 256 < kv_len) request_keys(t0 + 256);
+    }
+  }
+  lds_barrier();
+  if (A.timeline) t_scores = wall_clock64();
+  // ---- softmax (src/infer.cpp:472-487): a wave's trees over 64 positions, the waves' sums in order ----
+  if (kv_len <= 64) {
+    if (wave == 0) {
+      const float a0 = lane < kv_len ? att[lane] : -INFINITY;
+      const float mx = ad::wave_max_dpp(a0);
+      const float e = lane < kv_len ? expf(a0 - mx) : 0.f;
+      const float sum = ad::wave_sum_dpp(e);
+      if (lane < kv_len) att[lane] = e / sum;
+    }
+  } else {
+    float mx = -INFINITY;
+    for (int t = tid; t < kv_len; t += NT) mx = fmaxf(mx, att[t]);
+    mx = ad::wave_max_dpp(mx);
+    if (lane == 0) part[wave] = mx;
+    lds_barrier();
+    mx = part[0];
+    for (int i = 1; i < NW; ++i) mx = fmaxf(mx, part[i]);
+    float sum = 0.f;
+    for (int t = tid; t < kv_len; t += NT) {
+      const float e = expf(att[t] - mx);
+      att[t] = e;
+      sum += e;
+    }
+    sum = ad::wave_sum_dpp(sum);
+    if (lane == 0) part[NW + wave] = sum;
+    lds_barrier();
+    float total = 0.f;
+    for (int i = 0; i < NW; ++i) total += part[NW + i];
+    for (int t = tid; t < kv_len; t += NT) att[t] = att[t] / total;
+  }
+  lds_barrier();
+  // ---- values: every thread its positions in order, then the groups in order ----
+  auto value_here = [&]() {  // this position's, as the cache will hold it
+    const f32x4 x = *reinterpret_cast<const f32x4*>(kvb_s + nope + i4 * 4);
+    return ad::f16x4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w};
+  };
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  auto mix = [&](int t, ad::f16x4 y) {
+    if (t == kv_pos) y = value_here();
+    const float w = att[t];
+    acc[0] = fmaf(w, (float)y.x, acc[0]);
+    acc[1] = fmaf(w, (float)y.y, acc[1]);
+    acc[2] = fmaf(w, (float)y.z, acc[2]);
+    acc[3] = fmaf(w, (float)y.w, acc[3]);
+  };
+  if (g < TG) {
+#pragma unroll
+    for (int j = 0; j < VN; ++j)
+      if (g + j * TG < kv_len) mix(g + j * TG, v[j]);
+    for (int t0 = g + VN * TG; t0 - g < kv_len; t0 += 4 * TG) {
+      ad::f16x4 y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(VB, (int)voff, (t0 - g + j * TG) * (int)vrow, 0));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (t0 + j * TG < kv_len) mix(t0 + j * TG, y[j]);
+    }
+    *reinterpret_cast<f32x4*>(part + (size_t)g * vd + i4 * 4) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+  }
+  lds_barrier();
+  if (A.timeline) t_mix = wall_clock64();
+  if (tid < vd) {
+    float o = 0.f;
+    const int ng = min(TG, kv_len);  // (the others' sums are zeros)
+    for (int g0 = 0; g0 < ng; g0 += 8) {
+      float y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = part[min(g0 + i, ng - 1) * vd + tid];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o += g0 + i < ng ? y[i] : 0.f;
+    }
+    A.out[(size_t)h * vd + tid] = o;
+  }
+  // ---- the cache entries (src/infer.cpp:985-1005) ----
+  uint16_t* kc = kcache + ((size_t)kv_pos * H + h) * hd;
+  uint16_t* vc = vcache + ((size_t)kv_pos * H + h) * vd;
+  if (tid >= 512) {
+    const int i = tid - 512;
+    if (i < nope) kc[i] = ad::f2h(kvb_s[i]);
+    if (i < rope) kc[nope + i] = kr_s[i];
+    if (i < vd) vc[i] = ad::f2h(kvb_s[nope + i]);
+  }
+  if (A.timeline && tid == 0 && blockIdx.x < DSK_TL_WGS) {
+    unsigned long long* tl = A.timeline + (size_t)blockIdx.x * 8;
+    tl[0] = t_entry; tl[1] = t_staged; tl[2] = t_rows; tl[3] = t_scores; tl[4] = t_mix; tl[5] = wall_clock64();
+  }
+}
+
+// ---- host side ------------------------------------------------------------------------------------------
+int head_short_plan(HeadShortArgs& S, const HeadAttnArgs& A, int max_kv) {
+  const bool kq = A.quant == DSK_QUANT_Q2_K || A.quant == DSK_QUANT_Q3_K;
+  const int epi = kq ? 64 : A.quant == DSK_QUANT_F16 ? 8 : 16, n = A.tkv.n, nope = A.a.nope, vd = A.a.v_dim, rope = A.a.rope, hd = A.a.head_dim;
+  S.grid = 0;
+  if ((double)max_kv * A.a.n_heads * (hd > vd ? hd : vd) * 2 >= 2147483648.0) return DSK_OK;  // (32-bit offsets into a cache)
+  if (A.has_q || A.tiled || A.quant == DSK_QUANT_F32 || A.tkv.act_mode != ACT_F32_NORM) return DSK_OK;
+  // rows of one column step, at most 16 row sets of the workgroup (floats: two rounds of 8; K-quants: one of 2); the norm one piece a thread, in the first 8 waves
+  const int lpr = 1 << A.lkv_log2, sets = (nope + vd + 16 * (64 / lpr) - 1) / (16 * (64 / lpr));
+  if (n % (kq ? 256 : epi) || n % 4 || n / epi != lpr || n > 2048 || sets > (kq ? 2 : 16)) return DSK_OK;
+  if (hd != nope + rope || hd > 192 || hd % 4 || nope % 4 || nope < 4 || nope > 448 || rope < 2 || rope > 128 || rope % 2 || vd % 4 || vd < 4 || vd > 256 || nope + vd > 512 ||
+      1024 / (vd / 4) * vd > 4096 || A.a.n_heads < 1) return DSK_OK;
+  S.qs = A.tkv.qs; S.sc = A.tkv.sc; S.hm = A.tkv.hm; S.dm = A.tkv.dm; S.scale = A.tkv.scale;
+  S.quant = A.quant; S.nope = nope; S.rope = rope; S.lora = n; S.is_v3 = A.a.is_v3; S.eps = A.tkv.eps; S.out = A.a.out; S.lkv_log2 = A.lkv_log2; S.lds_kv = A.lds_kv;
+  S.b0 = A.b0 < 1 ? 1 : A.b0; S.b1 = A.b1 < 1 ? 1 : A.b1; S.H = A.a.n_heads; S.hd = hd; S.vd = vd; S.kv_a = A.a.kv_a; S.norm_w = A.tkv.norm_w; S.q = A.a.q;
+  S.key_cache = A.a.key_cache; S.value_cache = A.a.value_cache; S.timeline = A.timeline;
+  S.sets = sets;
+  S.sh0 = (S.b0 & (S.b0 - 1)) ? -1 : __builtin_ctz(S.b0); S.sh1 = (S.b1 & (S.b1 - 1)) ? -1 : __builtin_ctz(S.b1); S.sc_cols = (n + S.b1 - 1) / S.b1;
+  S.grid = A.a.n_heads;
+  return DSK_OK;
+}
+int launch_head_short(hipStream_t st, const HeadShortArgs& S, const StepParams* sp, int max_kv) {
+  const size_t lds = (size_t)S.lds_kv + (size_t)max_kv * 4;
+  if (lds > 120 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "attn: kv_len %d does not fit LDS", max_kv);
+  auto go = [&](auto k) {
+    if (lds > 40 * 1024) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(k, dim3(S.grid + (S.pf_wgs > 0 ? S.pf_wgs : 0)), dim3(1024), lds, st, sp, S.kv_a, S.norm_w, S.q, S.key_cache, S.value_cache, S.H, S.hd | S.vd << 16, S);
+  };
+  // (a set past the head's end costs what a real one does)
+  auto floats = [&](auto qt) {
+    constexpr int QT = decltype(qt)::value;
+    if (S.sets > 8) go(head_attn_short_kernel<QT, 4, 4>);
+    else if (S.sets > 4) go(head_attn_short_kernel<QT, 4, 2>);
+    else if (S.sets > 2) go(head_attn_short_kernel<QT, 2, 2>);
+    else go(head_attn_short_kernel<QT, 1, 2>);
+  };
+  switch (S.quant) {
+    case DSK_QUANT_F16: floats(std::integral_constant<int, DSK_QUANT_F16>{}); break;
+    case DSK_QUANT_F8E5M2: floats(std::integral_constant<int, DSK_QUANT_F8E5M2>{}); break;
+    case DSK_QUANT_Q2_K: go(head_attn_short_kernel<DSK_QUANT_Q2_K, 1, 2>); break;
+    default: go(head_attn_short_kernel<DSK_QUANT_Q3_K, 1, 2>); break;
+  }
+  return DSK_OK;
+}
