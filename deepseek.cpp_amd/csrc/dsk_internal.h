@@ -255,7 +255,7 @@ struct MoeFfnArgs {
   int tap_stride;
   double algo_bytes;
 };
-// The routed experts' W2 + the shared expert's + the combine, rows of x owned by workgroups (kernels_experts.hip); K-quant planes, one GPU.
+// The routed experts' W2 + the shared expert's + the combine, rows of x owned by workgroups (kernels_experts.hip); K-quant planes, F8E5M2, F16; one GPU.
 struct MoeDownArgs {
   const float* hb;       // hidden vectors [slot][hb_stride] (slot K: the shared expert's)
   const int* route_e;
@@ -265,7 +265,10 @@ struct MoeDownArgs {
   const uint8_t *w2_qs, *w2_sc, *w2_hm, *w2_dm, *sw2_qs, *sw2_sc, *sw2_hm, *sw2_dm;
   int quant, K, hb_stride, mi, shared_n, dim, n_experts;
   int lpr_log2;          // lanes per row: the generic plan's
-  int rows_wg, grid, cw, lds_b, lds, div_nb, div_rows;  // filled by moe_down_plan; cw: waves that multiply, the others stage
+  const float *w2_scale, *sw2_scale;  // floats: block scales (F8E5M2), bytes and scales per expert
+  size_t e2_qs, e2_scale;
+  int b0, b1;
+  int rows_wg, grid, cw, lds_b, lds, div_nb, div_rows, sh0, sh1;  // filled by moe_down_plan; cw (K-quants): waves that multiply, the others stage
   int8_t* tap_qs;        // parity taps (dsk_model_run_block): slot s's staged hidden vector at s * tap_stride
   float* tap_d;
   int tap_stride;
@@ -286,7 +289,11 @@ struct MoeUpArgs {
   int norm_topk_prob, scoring;
   float scaling;
   int lpr_log2;          // lanes per row: the generic plan's
-  int grid, lds;         // filled by moe_up_plan
+  const float* xn;       // floats: rmsnorm(x) in 32 bits; block scales (F8E5M2), bytes and scales per expert
+  const float *w1_scale, *w3_scale, *sw1_scale, *sw3_scale;
+  size_t e13_qs, e13_scale;
+  int b0, b1;
+  int grid, lds, its, sh0, sh1, sc_cols;  // filled by moe_up_plan
   unsigned div_mi;
   int8_t* tap_qs;        // parity tap: the staged vector
   float* tap_d;

@@ -396,17 +396,18 @@ int build_plans(dsk_model* m) {
       else { h.comb_geometry = 1; h.zero_absent = 1; }
       h.algo_bytes = bytes;
       DSK_TRY(add_plan(m, h, &m->lp_w2[l]));
-      if (kq && !w2.tiled && !m->sharded() && m->expert_launches) {
+      if (wq != DSK_QUANT_F32 && !w2.tiled && !m->sharded() && m->expert_launches) {
         MoeDownArgs a;
         memset(&a, 0, sizeof a);
         a.hb = m->hb; a.route_e = ae; a.route_w = aw; a.x = m->x; a.eout = m->eout;
         a.w2_qs = w2.qs; a.w2_sc = w2.sc; a.w2_hm = w2.hm; a.w2_dm = w2.dm;
         if (c.n_shared_experts > 0) {
           const DTensor& s2 = L.t[DSK_ROLE_SHARED_W2];
-          a.sw2_qs = s2.qs; a.sw2_sc = s2.sc; a.sw2_hm = s2.hm; a.sw2_dm = s2.dm;
+          a.sw2_qs = s2.qs; a.sw2_sc = s2.sc; a.sw2_hm = s2.hm; a.sw2_dm = s2.dm; a.sw2_scale = s2.scale;
           a.shared_n = shared_n;
         }
         a.quant = wq; a.K = K; a.hb_stride = hb_stride; a.mi = mi; a.dim = c.dim; a.n_experts = c.n_routed_experts;
+        a.w2_scale = w2.scale; a.e2_qs = w2.e_qs; a.e2_scale = w2.e_scale; a.b0 = c.block_size[0]; a.b1 = c.block_size[1];
         a.lpr_log2 = m->plans[m->lp_w2[l]].lpr_log2;
         if (moe_down_plan(a, m->ctx->n_cus) == DSK_OK) m->moe_down[l] = a;
         else dsk_clear_error();  // the generic launch then
@@ -421,10 +422,11 @@ int build_plans(dsk_model* m) {
         if (c.n_shared_experts > 0) {
           const DTensor &s1 = L.t[DSK_ROLE_SHARED_W1], &s3 = L.t[DSK_ROLE_SHARED_W3];
           u.sw1_qs = s1.qs; u.sw1_sc = s1.sc; u.sw1_hm = s1.hm; u.sw1_dm = s1.dm;
-          u.sw3_qs = s3.qs; u.sw3_sc = s3.sc; u.sw3_hm = s3.hm; u.sw3_dm = s3.dm;
+          u.sw3_qs = s3.qs; u.sw3_sc = s3.sc; u.sw3_hm = s3.hm; u.sw3_dm = s3.dm; u.sw1_scale = s1.scale; u.sw3_scale = s3.scale;
           u.shared_n = shared_n;
         }
         u.quant = wq; u.E = c.n_routed_experts; u.K = K; u.hb_stride = hb_stride; u.mi = mi; u.dim = c.dim; u.act = c.act;
+        u.xn = m->xb; u.w1_scale = w1.scale; u.w3_scale = w3.scale; u.e13_qs = w1.e_qs; u.e13_scale = w1.e_scale; u.b0 = c.block_size[0]; u.b1 = c.block_size[1];
         u.norm_topk_prob = c.norm_topk_prob; u.scoring = c.scoring_func; u.scaling = c.routed_scaling_factor;
         u.lpr_log2 = m->plans[m->lp_w13[l]].lpr_log2;
         // (one wave decides: no groups; the router's slices as in router_gate_kernel<2>; the shared expert's rows are this launch's)
@@ -437,7 +439,7 @@ int build_plans(dsk_model* m) {
     // (or no shared expert).  Same lanes per row as the two plans above => bit-identical results.
     // Float weights (F8E5M2 / F16 / F32): moe_ffn_f_kernel, the shared expert's w1 / w3 computed in the same launch.
     const bool fuse_kq = kq && c.dim % 256 == 0 && (c.n_shared_experts == 0 || m->lp_sh13[l] >= 0);
-    const bool fuse_f = !kq && m->fuse_moe_float;
+    const bool fuse_f = !kq && m->fuse_moe_float && m->moe_up[l].grid <= 0;  // (three launches without a hand-over are faster: kernels_experts.hip)
     if ((fuse_kq || fuse_f) && !m->sharded() && m->fuse_moe && K + 1 <= 16) {
       MoeFfnArgs a;
       memset(&a, 0, sizeof a);
@@ -695,7 +697,7 @@ static int ffn(dsk_model* m, int l) {
   if (is_kq(c.weight_quant) && c.dim % 256 == 0) { r.q_qs = m->a_xb.qs; r.q_d = m->a_xb.d; r.q_bsums = m->a_xb.bsums; }
   if (m->moe_ffn[l].grid > 0) { r.zero_ctr = m->moe_ffn[l].slot_ctr; r.zero_n = std::min(16, std::max(K, m->n_slots)); }  // re-arm the expert launch's slot counters
   if (m->moe_up[l].grid > 0 && m->moe_ffn[l].grid <= 0) {
-    DSK_TRY(run_timed(m, "router_gate", (double)E * c.dim * 4 + c.dim * 8.0, [&] { return launch_router_scores(st, r, nullptr); }));
+    DSK_TRY(run_timed(m, "router_gate", (double)E * c.dim * 4 + c.dim * 8.0, [&] { return launch_router_scores(st, r, m->moe_up[l].quant == DSK_QUANT_F8E5M2 || m->moe_up[l].quant == DSK_QUANT_F16 ? m->xb : nullptr); }));
   } else if (m->lp_sh13[l] >= 0) {
     const GemvLaunch& hs = m->plans[m->lp_sh13[l]];
     PROFILED("router_gate", (double)E * c.dim * 4 + c.dim * 8.0 + hs.algo_bytes, launch_router_shared(st, r, m->plans_dev + m->lp_sh13[l], hs));

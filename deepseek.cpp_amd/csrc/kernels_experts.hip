@@ -188,6 +188,19 @@ __global__ __launch_bounds__(1024) void router_scores_kernel(const float* __rest
   }
 }
 
+// one wave's gate over the router's scores: the chosen experts to the workgroup's LDS, and by workgroup 0 to memory
+DEV void decide(const float* scores, const float* bias_p, int lane, int bid, int E, int K, int scoring, int norm_topk, float scaling, int* sel_s, const MoeUpArgs& a) {
+  const int e = lane < E ? lane : E - 1;
+  const float v = scores[e], bias = bias_p ? bias_p[e] : 0.f;
+  float sc, w;
+  const int sel = gate_wave(lane < E ? v : -INFINITY, bias, bias_p != nullptr, lane, E, K, scoring, norm_topk, scaling, sc, w);
+  sel_s[lane] = sel;
+  if (bid == 0) {
+    if (lane < E) a.scores_out[lane] = sc;
+    if (lane < K) { a.route_e[lane] = sel; a.route_w[lane] = w; }
+  }
+}
+
 // ------------------------------------------------------------------------------------------------------------
 // First half: every workgroup decides the gate for itself out of the scores (one wave, ~0.5 us: less than handing a decision over), while other waves stage the
 // normed vector; then its share of the shared expert's and of the chosen experts' rows, all of a wave's requested at once.  Bound by latency (16.5 MB: 2.5
@@ -212,15 +225,7 @@ __global__ __launch_bounds__(1024) void experts_up_kernel(const float* __restric
   const u32 div_mi = arg(a.div_mi);
   int8_t* const tap_qs = glob(arg(a.tap_qs));
   if (wave == 15) {
-    const int e = lane < E ? lane : E - 1;
-    const float v = scores[e], bias = bias_p ? bias_p[e] : 0.f;
-    float sc, w;
-    const int sel = gate_wave(lane < E ? v : -INFINITY, bias, bias_p != nullptr, lane, E, K, scoring, norm_topk, scaling, sc, w);
-    sel_s[lane] = sel;
-    if (bid == 0) {
-      if (lane < E) a.scores_out[lane] = sc;
-      if (lane < K) { a.route_e[lane] = sel; a.route_w[lane] = w; }
-    }
+    decide(scores, bias_p, lane, bid, E, K, scoring, norm_topk, scaling, sel_s, a);
   } else if (wave >= CW) {
     for (int i = tid - CW * 64; i < dim >> 4; i += 192) {  // runs of 16 codes, their sums and their block's scale into item records (stage_q8)
       const u32x4 run = reinterpret_cast<const u32x4*>(a_qs)[i];
@@ -277,6 +282,95 @@ __global__ __launch_bounds__(1024) void experts_up_kernel(const float* __restric
     request(j + CW, S1);  // (a step that is not there reads through an empty descriptor: no branch around its loads)
     finish(S0);
     finish(S1);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// The same for F8E5M2 and F16 weights: a row is ITS steps of a whole wave (moe_ffn_f_kernel's lanes and order), its values' factors stay in registers for all rows of
+// a wave, and the next two rows are on their way while one is multiplied.  V2-Lite's shapes in F8E5M2: 46 MB in 12.4 us, a pure stream of that size taking 9.6 (16
+// waves that multiply instead of 12, or the shared expert's rows requested before the gate: the same).
+// ------------------------------------------------------------------------------------------------------------
+template <int QT, int ITS>
+__global__ __launch_bounds__(1024) void experts_up_f_kernel(const float* __restrict__ scores, const float* __restrict__ xn, int E, int K, const MoeUpArgs a) {
+  constexpr int EPI = FTraits<QT>::EPI, CW = 12, ITEMS = ITS * 64, DIM = ITEMS * EPI;
+  constexpr bool F8 = QT == DSK_QUANT_F8E5M2;
+  __shared__ __attribute__((aligned(16))) float x_s[DIM];
+  __shared__ int sel_s[64];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x, G = gridDim.x;
+  const uint8_t *w1 = arg(a.w1_qs), *w3 = arg(a.w3_qs), *sw1 = arg(a.sw1_qs), *sw3 = arg(a.sw3_qs);
+  const float *w1_scale = nullptr, *w3_scale = nullptr, *sw1_scale = nullptr, *sw3_scale = nullptr;
+  if (F8) { w1_scale = arg(a.w1_scale); w3_scale = arg(a.w3_scale); sw1_scale = arg(a.sw1_scale); sw3_scale = arg(a.sw3_scale); }
+  const size_t e_qs = arg(a.e13_qs), e_scale = arg(a.e13_scale);
+  float* const hb = glob(arg(a.hb));
+  const float* const bias_p = glob(arg(a.bias));
+  const int mi = arg(a.mi), shared_n = arg(a.shared_n), act = arg(a.act), hb_stride = arg(a.hb_stride), scoring = arg(a.scoring), norm_topk = arg(a.norm_topk_prob);
+  const int b0 = arg(a.b0), sh0 = arg(a.sh0), sc_cols = arg(a.sc_cols);
+  const float scaling = arg(a.scaling);
+  const u32 div_mi = arg(a.div_mi);
+  int sc_off[ITS];  // (the scale's column of an item)
+#pragma unroll
+  for (int u = 0; u < ITS; ++u) sc_off[u] = (a.sh1 >= 0 ? (u * 64 + lane) * EPI >> a.sh1 : (u * 64 + lane) * EPI / a.b1) * 4;
+  const int s_lo = (int)((unsigned)(shared_n * bid) / (unsigned)G), s_hi = (int)((unsigned)(shared_n * (bid + 1)) / (unsigned)G);
+  const int v_lo = (int)((unsigned)(K * mi * bid) / (unsigned)G), v_hi = (int)((unsigned)(K * mi * (bid + 1)) / (unsigned)G);
+  const int JS = s_hi - s_lo, J = JS + v_hi - v_lo;
+  struct Row { u32x4 w[ITS], u[ITS]; float sw[ITS], su[ITS]; int out; };
+  auto request = [&](int j, Row& R) {  // (a row that is not there reads through an empty descriptor)
+    const bool live = j < J, sh = j < JS;
+    const int v = sh ? s_lo + j : min(v_lo + j - JS, v_hi - 1), slot = sh ? K : (int)__umulhi((u32)max(v, 0), div_mi), rr = sh ? v : v - slot * mi;
+    const int e = sh ? 0 : __builtin_amdgcn_readfirstlane(sel_s[min(slot, K - 1)]);
+    R.out = live ? slot * hb_stride + rr : -1;
+    const size_t at = (sh ? 0 : e * e_qs) + (size_t)rr * (DIM * FTraits<QT>::ESZ);
+    const rsrc_t B1 = make_rsrc_n((sh ? sw1 : w1) + at, live), B3 = make_rsrc_n((sh ? sw3 : w3) + at, live);
+#pragma unroll
+    for (int u = 0; u < ITS; ++u) {
+      R.w[u] = __builtin_amdgcn_raw_buffer_load_b128(B1, lane * 16, u * 1024, BUF_NT);
+      R.u[u] = __builtin_amdgcn_raw_buffer_load_b128(B3, lane * 16, u * 1024, BUF_NT);
+    }
+    if constexpr (F8) {
+      const size_t sat = (sh ? 0 : e * e_scale) + (size_t)(sh0 >= 0 ? rr >> sh0 : rr / b0) * sc_cols;
+      const rsrc_t S1 = make_rsrc_n((sh ? sw1_scale : w1_scale) + sat, live), S3 = make_rsrc_n((sh ? sw3_scale : w3_scale) + sat, live);
+#pragma unroll
+      for (int u = 0; u < ITS; ++u) {
+        R.sw[u] = u2f(__builtin_amdgcn_raw_buffer_load_b32(S1, sc_off[u], 0, 0));
+        R.su[u] = u2f(__builtin_amdgcn_raw_buffer_load_b32(S3, sc_off[u], 0, 0));
+      }
+    }
+  };
+  float xa[ITS][EPI];
+  auto finish = [&](const Row& R) {
+    float g = 0.f, up = 0.f;
+#pragma unroll
+    for (int u = 0; u < ITS; ++u) {
+      g = fmaf(fitem<QT>(R.w[u], xa[u], 0.f), F8 ? R.sw[u] : 1.0f, g);
+      up = fmaf(fitem<QT>(R.u[u], xa[u], 0.f), F8 ? R.su[u] : 1.0f, up);
+    }
+    g = lanes_sum(g, 6);
+    up = lanes_sum(up, 6);
+    if (lane == 0 && R.out >= 0) hb[R.out] = act_fn(g, act) * up;  // src/infer.cpp:859-872
+  };
+  if (wave == 15) {
+    decide(scores, bias_p, lane, bid, E, K, scoring, norm_topk, scaling, sel_s, a);
+  } else if (wave >= CW) {
+    for (int i = tid - CW * 64; i < DIM / 4; i += 192)
+      reinterpret_cast<f32x4*>(x_s)[quad_place<EPI>(i, ITEMS)] = reinterpret_cast<const f32x4*>(xn)[i];
+  }
+  lds_barrier();
+  if (wave >= CW) return;
+#pragma unroll
+  for (int u = 0; u < ITS; ++u)
+#pragma unroll
+    for (int k = 0; k < EPI / 4; ++k) {
+      const f32x4 t = reinterpret_cast<const f32x4*>(x_s)[k * ITEMS + u * 64 + lane];
+      xa[u][4 * k] = t.x; xa[u][4 * k + 1] = t.y; xa[u][4 * k + 2] = t.z; xa[u][4 * k + 3] = t.w;
+    }
+  Row A, B;
+  request(wave, A);
+  request(wave + CW, B);
+  for (int j = wave; j < J; j += 2 * CW) {
+    finish(A);
+    request(j + 2 * CW, A);
+    finish(B);
+    request(j + 3 * CW, B);
   }
 }
 
@@ -383,17 +477,159 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
   }
 }
 
+// ------------------------------------------------------------------------------------------------------------
+// The same for F8E5M2 and F16 weights (lanes, order and combine of moe_ffn_f_kernel): nothing to quantise, so all waves copy the hidden vectors, between the
+// request of their first weights and their use.  V2-Lite's shapes in F8E5M2: 23 MB in 8.4 us.  Router, first and second half were 7.0 + 23.3 us with both halves in one
+// launch, 4.7 + 12.4 + 8.4 here: the hand-over inside it cost more than a launch; a token 1505 -> 1351 us.
+// ------------------------------------------------------------------------------------------------------------
+template <int QT>
+__global__ __launch_bounds__(1024) void experts_down_f_kernel(const float* __restrict__ hb, const int* __restrict__ route_e, const float* __restrict__ route_w, float* x,
+                                                             int hb_stride, int K, const MoeDownArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr int NW = 16, EPI = FTraits<QT>::EPI, ESZ = FTraits<QT>::ESZ, U = 6, HQ = 4;
+  constexpr bool F8 = QT == DSK_QUANT_F8E5M2;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x;
+  const uint8_t *w2 = arg(a.w2_qs), *sw2 = arg(a.sw2_qs);
+  const float *w2_scale = nullptr, *sw2_scale = nullptr;
+  if (F8) { w2_scale = arg(a.w2_scale); sw2_scale = arg(a.sw2_scale); }
+  const size_t e_qs = arg(a.e2_qs), e_scale = arg(a.e2_scale);
+  float* const eout = glob(arg(a.eout));
+  const int mi = arg(a.mi), shared_n = arg(a.shared_n), dim = arg(a.dim), rows_wg = arg(a.rows_wg), lpr_log2 = arg(a.lpr_log2), lds_b = arg(a.lds_b), div_q = arg(a.div_nb),
+            div_rows = arg(a.div_rows), b0 = arg(a.b0), b1 = arg(a.b1), sh0 = arg(a.sh0), sh1 = arg(a.sh1);
+  float* o_s = reinterpret_cast<float*>(smem + (size_t)lds_b * (K + 1));  // [slot][rows_wg]
+  const int slots = K + (shared_n > 0 ? 1 : 0), r_lo = bid * rows_wg, nrows = min(rows_wg, dim - r_lo);
+  float xv = 0.f, rw = 0.f;
+  if (wave == NW - 1) {
+    xv = x[r_lo + (lane < nrows ? lane : nrows - 1)];
+    rw = route_w[lane < K ? lane : K - 1];
+  }
+  const int e_all = route_e[lane < K ? lane : K - 1];
+  // 1. the hidden vectors' pieces of 16 bytes, the first HQ of a thread: piece i of the slots behind each other
+  const int pR = mi >> 2, pieces = K * pR + (shared_n >> 2);
+  auto piece = [&](int i, const float*& src, uint8_t*& dst) {
+    const int ii = min(i, pieces - 1), s = ii < K * pR ? (int)__umulhi((u32)ii, (u32)div_q) : K, j = ii - s * pR, n = s < K ? mi : shared_n;
+    src = hb + (size_t)s * hb_stride + j * 4;
+    dst = smem + (size_t)s * lds_b + (size_t)quad_place<EPI>(j, n / EPI) * 16;
+  };
+  f32x4 hv[HQ];
+  uint8_t* hd[HQ];
+#pragma unroll
+  for (int k = 0; k < HQ; ++k) {
+    const float* src;
+    piece(tid + k * 1024, src, hd[k]);
+    hv[k] = *reinterpret_cast<const f32x4*>(src);
+  }
+  // 2. this wave's steps of RPW rows: the shared expert's first (the longest), then the routed slots'; the first two chunks of U column steps
+  const int RPW = 64 >> lpr_log2, rloc = lane >> lpr_log2, sub = lane & ((1 << lpr_log2) - 1);
+  const int WS = shared_n > 0 ? (rows_wg + RPW - 1) >> (6 - lpr_log2) : 0, WR = (rows_wg * K + RPW - 1) >> (6 - lpr_log2);
+  struct Chunk { u32x4 w[U]; float sv[U]; };
+  struct Step { const uint8_t* row; const float* sc; int items, its, slot, rr; bool valid; };
+  auto step_of = [&](int st) {
+    Step S;
+    const bool sh = st < WS;
+    const int v = (sh ? st : st - WS) * RPW + rloc, n = sh ? shared_n : mi;
+    S.slot = sh ? K : min(div_small(v, div_rows), K - 1);
+    const int rr0 = sh ? v : v - S.slot * rows_wg;
+    S.valid = st < WS + WR && rr0 < nrows;
+    S.rr = min(rr0, nrows - 1);
+    S.items = n / EPI;
+    S.its = (S.items + (1 << lpr_log2) - 1) >> lpr_log2;
+    const int e = sh ? 0 : __shfl(e_all, S.slot), r = r_lo + S.rr;
+    S.row = (sh ? sw2 : w2 + e * e_qs) + (size_t)r * n * ESZ;
+    if (F8) S.sc = (sh ? sw2_scale : w2_scale + e * e_scale) + (size_t)(sh0 >= 0 ? r >> sh0 : r / b0) * (sh1 >= 0 ? (n + b1 - 1) >> sh1 : (n + b1 - 1) / b1);
+    return S;
+  };
+  auto request = [&](const Step& S, int it0, Chunk& C) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int item = min(sub + ((it0 + u) << lpr_log2), S.items - 1);
+      C.w[u] = ldg_nt(reinterpret_cast<const u32x4*>(S.row + (size_t)item * 16));
+      if (F8) C.sv[u] = S.sc[sh1 >= 0 ? item * EPI >> sh1 : item * EPI / b1];
+    }
+  };
+  auto multiply = [&](const Step& S, int it0, const Chunk& C, float acc) {
+    const f32x4* l = reinterpret_cast<const f32x4*>(smem + (size_t)S.slot * lds_b);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (it0 + u >= S.its) break;
+      const int it = sub + ((it0 + u) << lpr_log2), item = min(it, S.items - 1);
+      float xa[EPI];
+#pragma unroll
+      for (int k = 0; k < EPI / 4; ++k) {
+        const f32x4 t = l[k * S.items + item];  // (quad_place)
+        xa[4 * k] = t.x; xa[4 * k + 1] = t.y; xa[4 * k + 2] = t.z; xa[4 * k + 3] = t.w;
+      }
+      const float sv = it < S.items ? (F8 ? C.sv[u] : 1.0f) : 0.f;
+      acc = fmaf(fitem<QT>(C.w[u], xa, 0.f), sv, acc);
+    }
+    return acc;
+  };
+  Chunk A, B;
+  Step S = step_of(wave);
+  if (wave < WS + WR) {
+    request(S, 0, A);
+    if (U < S.its) request(S, U, B);
+  }
+  // 3. the hidden vectors into LDS
+#pragma unroll
+  for (int k = 0; k < HQ; ++k) *reinterpret_cast<f32x4*>(hd[k]) = hv[k];  // (pieces past the end: the last one again)
+  for (int i = tid + HQ * 1024; i < pieces; i += 1024) {
+    const float* src;
+    uint8_t* dst;
+    piece(i, src, dst);
+    *reinterpret_cast<f32x4*>(dst) = *reinterpret_cast<const f32x4*>(src);
+  }
+  lds_barrier();
+  // 4. column steps in order
+  for (int st = wave; st < WS + WR; st += NW) {
+    if (st != wave) {
+      S = step_of(st);
+      request(S, 0, A);
+      if (U < S.its) request(S, U, B);
+    }
+    float acc = 0.f;
+    for (int it0 = 0; it0 < S.its; it0 += 2 * U) {
+      acc = multiply(S, it0, A, acc);
+      if (it0 + 2 * U < S.its) request(S, it0 + 2 * U, A);
+      if (it0 + U < S.its) acc = multiply(S, it0 + U, B, acc);
+      if (it0 + 3 * U < S.its) request(S, it0 + 3 * U, B);
+    }
+    const float o = lanes_sum(acc, lpr_log2);
+    if (sub == 0 && S.valid) o_s[S.slot * rows_wg + S.rr] = o;
+  }
+  lds_barrier();
+  if (wave == NW - 1 && lane < nrows) {  // x += w_k * o_k in k order (src/infer.cpp:874-877), then the shared expert (:900-903)
+    for (int k = 0; k < slots; ++k) {
+      const float o = o_s[k * rows_wg + lane];
+      eout[(size_t)k * dim + r_lo + lane] = o;
+      if (k < K) xv = fmaf(o, u2f(__builtin_amdgcn_readlane(__builtin_bit_cast(u32, rw), k)), xv);
+      else xv += o;
+    }
+    x[r_lo + lane] = xv;
+  }
+}
+
 // ---- host side ------------------------------------------------------------------------------------------
 int moe_up_plan(MoeUpArgs& a, int n_cus) {
-  if (a.quant != DSK_QUANT_Q2_K && a.quant != DSK_QUANT_Q3_K) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: K-quant planes only");
+  const bool kq = a.quant == DSK_QUANT_Q2_K || a.quant == DSK_QUANT_Q3_K, f8 = a.quant == DSK_QUANT_F8E5M2;
+  if (!kq && !f8 && a.quant != DSK_QUANT_F16) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: weights");
   if (a.E < 1 || a.E > 64 || a.K < 1 || a.K > a.E || a.K > 15 || a.mi < 1 || a.shared_n < 0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: shapes");
-  // rows of one column step; router slices of one or two pieces, the norm of one piece a thread
-  if (a.dim % 256 || a.dim > 4096 || a.dim / 64 != 1 << a.lpr_log2) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: rows of %d", a.dim);
-  if ((double)a.E * a.mi * (a.dim / 256) * 64.0 >= 2147483648.0 || (double)a.shared_n * (a.dim / 256) * 64.0 >= 2147483648.0)
+  // router slices of one or two pieces, the norm of one piece a thread; K-quants: rows of one column step; floats: of 1, 2 or (F16) 4 steps of a whole wave
+  if (a.dim % 256 || a.dim > 4096) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: rows of %d", a.dim);
+  if (kq && a.dim / 64 != 1 << a.lpr_log2) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: rows of %d", a.dim);
+  if (!kq) {
+    a.its = a.dim / (f8 ? 16 : 8) / 64;
+    if (a.lpr_log2 != 6 || a.its * 64 * (f8 ? 16 : 8) != a.dim || !(a.its == 1 || a.its == 2 || (a.its == 4 && !f8))) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: rows of %d", a.dim);
+    if (a.b0 < 1) a.b0 = 1;
+    if (a.b1 < 1) a.b1 = 1;
+    a.sh0 = (a.b0 & (a.b0 - 1)) ? -1 : __builtin_ctz(a.b0); a.sh1 = (a.b1 & (a.b1 - 1)) ? -1 : __builtin_ctz(a.b1); a.sc_cols = (a.dim + a.b1 - 1) / a.b1;
+  }
+  if (kq && ((double)a.E * a.mi * (a.dim / 256) * 64.0 >= 2147483648.0 || (double)a.shared_n * (a.dim / 256) * 64.0 >= 2147483648.0))
     DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: a stack exceeds the 31-bit offset of a buffer load");
   // (v * ceil(2^32 / d) >> 32 == v / d while v * (d - 1) < 2^32)
   if (a.mi < 2 || (double)a.K * a.mi * a.mi >= 4294967296.0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: too many rows");
   a.div_mi = (unsigned)((4294967296ull + a.mi - 1) / a.mi);
+  if ((double)(a.K * a.mi > a.shared_n ? a.K * a.mi : a.shared_n) * n_cus >= 4294967296.0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_up: too many rows");
   const int rows = a.K * a.mi + a.shared_n, RPW = 64 >> a.lpr_log2;
   a.grid = n_cus < (rows + RPW - 1) / RPW ? n_cus : (rows + RPW - 1) / RPW;
   a.lds = a.dim / 64 * ITEM_LDS;
@@ -418,30 +654,48 @@ int launch_moe_up(hipStream_t st, const MoeUpArgs& a) {
       hipExtLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, g_prof_start, g_prof_stop, 0u, a.scores, a.a_qs, a.a_d, a.a_bsums, a.E, a.K, a);
     else hipLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, a.scores, a.a_qs, a.a_d, a.a_bsums, a.E, a.K, a);
   };
-  if (a.quant == DSK_QUANT_Q2_K) go(experts_up_kernel<DSK_QUANT_Q2_K>);
-  else go(experts_up_kernel<DSK_QUANT_Q3_K>);
+  auto floats = [&](auto k) {
+    if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, dim3(a.grid), dim3(1024), 0u, st, g_prof_start, g_prof_stop, 0u, a.scores, a.xn, a.E, a.K, a);
+    else hipLaunchKernelGGL(k, dim3(a.grid), dim3(1024), 0u, st, a.scores, a.xn, a.E, a.K, a);
+  };
+  switch (a.quant) {
+    case DSK_QUANT_Q2_K: go(experts_up_kernel<DSK_QUANT_Q2_K>); break;
+    case DSK_QUANT_Q3_K: go(experts_up_kernel<DSK_QUANT_Q3_K>); break;
+    case DSK_QUANT_F8E5M2: a.its == 1 ? floats(experts_up_f_kernel<DSK_QUANT_F8E5M2, 1>) : floats(experts_up_f_kernel<DSK_QUANT_F8E5M2, 2>); break;
+    default: a.its == 1 ? floats(experts_up_f_kernel<DSK_QUANT_F16, 1>) : a.its == 2 ? floats(experts_up_f_kernel<DSK_QUANT_F16, 2>) : floats(experts_up_f_kernel<DSK_QUANT_F16, 4>);
+  }
   return DSK_OK;
 }
 
 int moe_down_plan(MoeDownArgs& a, int n_cus) {
-  const bool q2 = a.quant == DSK_QUANT_Q2_K, q3 = a.quant == DSK_QUANT_Q3_K;
-  if (!q2 && !q3) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: K-quant planes only");
-  if (a.K < 1 || a.K > 15 || a.dim < 1 || a.mi < 256 || a.mi % 256 || a.shared_n % 256 || a.shared_n < 0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: shapes");
+  const bool kq = a.quant == DSK_QUANT_Q2_K || a.quant == DSK_QUANT_Q3_K, f8 = a.quant == DSK_QUANT_F8E5M2;
+  const int unit = kq ? 256 : f8 ? 16 : 8;
+  if (!kq && !f8 && a.quant != DSK_QUANT_F16) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: weights");
+  if (a.K < 1 || a.K > 15 || a.dim < 1 || a.mi < unit || a.mi % unit || a.shared_n % unit || a.shared_n < 0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: shapes");
   const int lpr = 1 << a.lpr_log2, RPW = 64 / lpr, nbR = a.mi >> 8, nbS = a.shared_n >> 8;
-  if (lpr < 4 || lpr > 64 || (nbR * 4) % lpr || (nbS * 4) % lpr) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: %d lanes do not divide the rows", lpr);
+  if (lpr > 64 || (kq && (lpr < 4 || (nbR * 4) % lpr || (nbS * 4) % lpr))) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: %d lanes do not divide the rows", lpr);
   a.rows_wg = (a.dim + n_cus - 1) / n_cus;
   a.grid = (a.dim + a.rows_wg - 1) / a.rows_wg;
   if (a.rows_wg > 64) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: %d rows per workgroup", a.rows_wg);
-  // one descriptor spans the stack: a lane's byte offset (expert, row, block) must fit its 32-bit offset field
-  if ((double)a.n_experts * a.dim * nbR * 64.0 >= 2147483648.0 || (double)a.dim * nbS * 64.0 >= 2147483648.0)
+  // K-quants: one descriptor spans the stack: a lane's byte offset (expert, row, block) must fit its 32-bit offset field
+  if (kq && ((double)a.n_experts * a.dim * nbR * 64.0 >= 2147483648.0 || (double)a.dim * nbS * 64.0 >= 2147483648.0))
     DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: a stack exceeds the 31-bit offset of a buffer load");
-  a.div_nb = (65536 + nbR - 1) / nbR;
-  a.div_rows = (65536 + a.rows_wg - 1) / a.rows_wg;
-  // (v * ceil(2^16 / d) >> 16 == v / d while v * (d - 1) < 2^16)
+  // (v * ceil(2^16 / d) >> 16 == v / d while v * (d - 1) < 2^16; with 2^32 likewise)
   const long nblk = (long)a.K * nbR + nbS, nv = (long)a.K * a.rows_wg + RPW;
-  if (nblk * (nbR - 1) >= 65536 || nv * (a.rows_wg - 1) >= 65536 || nblk >= 32768) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: too many blocks");
-  const int nB = nbR > nbS ? nbR : nbS;
-  a.lds_b = nB * 4 * ITEM_LDS;
+  a.div_rows = (65536 + a.rows_wg - 1) / a.rows_wg;
+  if (nv * (a.rows_wg - 1) >= 65536) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: too many rows");
+  if (kq) {
+    a.div_nb = (65536 + nbR - 1) / nbR;
+    if (nblk * (nbR - 1) >= 65536 || nblk >= 32768) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: too many blocks");
+  } else {
+    if (a.mi < 8 || (double)(a.K * (a.mi / 4) + a.shared_n / 4) * (a.mi / 4) >= 4294967296.0) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: too many values");
+    a.div_nb = (unsigned)((4294967296ull + a.mi / 4 - 1) / (a.mi / 4));
+    if (a.b0 < 1) a.b0 = 1;
+    if (a.b1 < 1) a.b1 = 1;
+    a.sh0 = (a.b0 & (a.b0 - 1)) ? -1 : __builtin_ctz(a.b0); a.sh1 = (a.b1 & (a.b1 - 1)) ? -1 : __builtin_ctz(a.b1);
+  }
+  const int nB = a.mi > a.shared_n ? a.mi : a.shared_n;
+  a.lds_b = kq ? nB / 64 * ITEM_LDS : nB * 4;
   const size_t lds = (size_t)a.lds_b * (a.K + 1) + (size_t)(a.K + 1) * a.rows_wg * 4;
   if (lds > 150 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "moe_down: activations do not fit LDS");
   a.lds = (int)lds;
@@ -457,7 +711,17 @@ int launch_moe_down(hipStream_t st, const MoeDownArgs& a) {
       hipExtLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, g_prof_start, g_prof_stop, 0u, a.hb, a.route_e, a.route_w, a.x, a.hb_stride, a.K, a.cw, a);
     else hipLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, a.hb, a.route_e, a.route_w, a.x, a.hb_stride, a.K, a.cw, a);
   };
-  if (a.quant == DSK_QUANT_Q2_K) go(experts_down_kernel<DSK_QUANT_Q2_K>);
-  else go(experts_down_kernel<DSK_QUANT_Q3_K>);
+  auto floats = [&](auto k) {
+    if (a.lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, a.lds);
+    if (g_prof_start && g_prof_stop)
+      hipExtLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, g_prof_start, g_prof_stop, 0u, a.hb, a.route_e, a.route_w, a.x, a.hb_stride, a.K, a);
+    else hipLaunchKernelGGL(k, dim3(a.grid), dim3(1024), (uint32_t)a.lds, st, a.hb, a.route_e, a.route_w, a.x, a.hb_stride, a.K, a);
+  };
+  switch (a.quant) {
+    case DSK_QUANT_Q2_K: go(experts_down_kernel<DSK_QUANT_Q2_K>); break;
+    case DSK_QUANT_Q3_K: go(experts_down_kernel<DSK_QUANT_Q3_K>); break;
+    case DSK_QUANT_F8E5M2: floats(experts_down_f_kernel<DSK_QUANT_F8E5M2>); break;
+    default: floats(experts_down_f_kernel<DSK_QUANT_F16>);
+  }
   return DSK_OK;
 }

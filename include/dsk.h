@@ -198,8 +198,8 @@ int dsk_model_destroy(dsk_model* m);
  *                        bias row) into the XCDs' L2 (0: off; results unaffected)
  *   "moe_q8_handoff"  1  fused expert launch: hidden vectors handed over as Q8_K, quantised once by their producers
  *   "fuse_moe_float"  1  fused expert launch for F8E5M2 / F16 / F32 weights too (0: two launches; bit-identical)
- *   "expert_launches" 1  K-quant experts that do not run as one launch: the gate inside the first half, the second half by workgroups that own rows of x
- *                        for every slot (0: the router with the gate and the generic launches; bit-identical)
+ *   "expert_launches" 1  experts (K-quant planes that do not run as one launch, F8E5M2, F16): the gate inside the first half, the second half by workgroups that own
+ *                        rows of x for every slot (0: the router with the gate and one launch or the generic ones; bit-identical)
  *   "timeline"        0  in-kernel wall-clock stamps for dsk_model_get_timeline
  *   "moe_spin_limit"  0  polls before the fused expert launch's hand-off wait gives up (0: 2^20); < 0: fault
  *                        injection (a give-up is reported although the hand-off succeeded: exercises the fallback)

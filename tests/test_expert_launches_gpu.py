@@ -10,11 +10,15 @@ pytestmark = pytest.mark.gpu
 
 def same(ctx, c, T=None, seed=None, tokens=(5, 9, 700, 3, 44), options=None, up=False):
     import dsk
-    o = dict({"fuse_moe": 0, "q2k_tiles": 0}, **(options or {}))
+    # floats: the other side is the one launch (the generic launches stage x with as many waves as their rows ask for, and with four the sum of squares
+    # can differ in its last bit)
+    floats = c.quant in ("f8e5m2", "fp16") and up
+    o = dict({"fuse_moe": int(floats), "q2k_tiles": 0}, **(options or {}))
     A, B = (dsk.Model(ctx, c, T, synth_seed=seed, options=dict(o, expert_launches=on)) for on in (1, 0))
     blocks = c.n_layers - c.first_k_dense_replace
     assert [m.info("expert_down_layers") for m in (A, B)] == [blocks, 0]
     assert [m.info("expert_up_layers") for m in (A, B)] == [blocks if up else 0, 0]
+    assert [m.info("fused_moe_layers") for m in (A, B)] == [0, blocks if floats else 0]
     for graph in (True, False):
         for m in (A, B):
             m.set_graph(graph)
@@ -27,8 +31,8 @@ def same(ctx, c, T=None, seed=None, tokens=(5, 9, 700, 3, 44), options=None, up=
     x = np.random.default_rng(1).standard_normal(c.dim).astype(np.float32)
     layer = c.first_k_dense_replace
     assert np.array_equal(A.run_block(layer, x, 2), B.run_block(layer, x, 2))
-    n = (c.n_active_routed + (c.n_shared_experts > 0)) * max(1, c.n_shared_experts) * c.moe_intermediate_size
-    for name, count, dt in (("q8.hb.qs", n, np.int8), ("q8.hb.d", n // 256, np.float32)):  # what the slots staged
+    n = (c.n_active_routed + (c.n_shared_experts > 0)) * max(1, c.n_shared_experts) * c.moe_intermediate_size if c.quant in ("q2_k", "q3_k") else 0
+    for name, count, dt in (("q8.hb.qs", n, np.int8), ("q8.hb.d", n // 256, np.float32)) if n else ():  # what the slots staged
         assert np.array_equal(A.stage(name, count, dt).view(np.uint8), B.stage(name, count, dt).view(np.uint8)), name
     A.close()
     B.close()
@@ -39,14 +43,17 @@ SMALL = [dict(), dict(dim=768, moe_intermediate_size=512), dict(n_shared_experts
          dict(n_active_routed=8, dim=256)]
 
 
-@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+QUANTS = ["q2_k", "q3_k", "f8e5m2", "fp16"]
+
+
+@pytest.mark.parametrize("quant", QUANTS)
 @pytest.mark.parametrize("over", SMALL, ids=[",".join(f"{k[:8]}{v}" for k, v in o.items()) or "tiny" for o in SMALL])
 def test_small_shapes_same_bits(ctx, quant, over):
     c = synth.preset("tiny_v2lite", quant, False, **over)
     same(ctx, c, synth.synth_model(c, seed=7))
 
 
-@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+@pytest.mark.parametrize("quant", QUANTS)
 def test_v2lite_shapes_same_bits(ctx, quant):
     c = synth.preset("v2lite", quant, False, n_layers=3, max_seq_len=64)
     same(ctx, c, seed=5, tokens=(5, 90000, 3), up=True)
@@ -59,14 +66,23 @@ GATE = [dict(n_routed_experts=33, n_active_routed=5), dict(n_routed_experts=64, 
                                                           routed_scaling_factor=2.5)]
 
 
-@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+@pytest.mark.parametrize("quant", QUANTS)
 @pytest.mark.parametrize("over", GATE, ids=["33 of 5", "64 of 8", "3 of 3", "sigmoid 4096"])
 def test_gate_inside_the_first_half_same_bits(ctx, quant, over):
     over = dict(over)
+    if quant in ("f8e5m2", "fp16") and over.get("dim") == 4096:
+        over["dim"] = 2048  # (floats: rows of up to 32 values a lane)
     if over.pop("has_moegate_bias", False):
         over["arch"] = "DeepseekV3ForCausalLM"
     c = synth.preset("v2lite", quant, False, **dict(dict(n_layers=2, hidden_dim=512, vocab_size=512, moe_intermediate_size=256, max_seq_len=64), **over))
     same(ctx, c, seed=9, tokens=(5, 400, 3), up=True)
+
+
+def test_float_rows_of_fewer_steps_same_bits(ctx):
+    """F8E5M2 and F16 over two MoE blocks whose hidden rows end inside a group of lanes and whose block scales change within a row"""
+    for quant, over in (("f8e5m2", dict(moe_intermediate_size=176, n_shared_experts=2)), ("fp16", dict(moe_intermediate_size=104, n_shared_experts=1))):
+        c = synth.preset("v2lite", quant, False, n_layers=3, hidden_dim=512, vocab_size=512, max_seq_len=64, n_routed_experts=9, n_active_routed=4, **over)
+        same(ctx, c, seed=13, tokens=(5, 400, 3), up=True)
 
 
 @pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
