@@ -457,6 +457,8 @@ struct HeadShortArgs {
 };
 int head_short_plan(HeadShortArgs& S, const HeadAttnArgs& A, int max_kv);
 int launch_head_short(hipStream_t st, const HeadShortArgs& S, const StepParams* sp, int max_kv);
+bool head_latent_supported(const HeadAttnArgs& A, int max_kv);  // ... behind a query latent: DeepSeek-V3's heads in Q2_K
+int launch_head_latent(hipStream_t st, const HeadAttnArgs& A, const StepParams* sp, int max_kv);
 struct AttnMlaArgs {
   float* q_rope;         // (H, rope)
   const float* q_c;      // (H, lora)

@@ -148,7 +148,7 @@ int ds_get_info(dsk_model* m, const char* key, int* value) {
   else if (k == "fused_moe_layers") { int n = 0; for (auto& a : m->moe_ffn) n += a.grid > 0; *value = n; }
   else if (k == "expert_up_layers") { int n = 0; for (size_t l = 0; l < m->moe_up.size(); ++l) n += m->moe_up[l].grid > 0 && m->moe_ffn[l].grid <= 0; *value = n; }
   else if (k == "expert_down_layers") { int n = 0; for (size_t l = 0; l < m->moe_down.size(); ++l) n += m->moe_down[l].grid > 0 && m->moe_ffn[l].grid <= 0; *value = n; }
-  else if (k == "head_short_layers") { int n = 0; for (auto& a : m->head_short) n += a.grid > 0; *value = n; }
+  else if (k == "head_short_layers") { int n = 0; for (auto& a : m->head_short) n += a.grid > 0; for (char b : m->head_latent) n += b; *value = n; }
   else if (k == "graph_captured") { int n = 0; for (auto g : m->graph) n += g != nullptr; *value = n; }
   else if (k == "exchange_calls") *value = m->exchange_calls;
   else if (k == "tiled_tensors") {  // weight tensors stored as tile records (option "q2k_tiles")

@@ -128,6 +128,7 @@ struct dsk_model : ModelHead {
   std::vector<double> head_attn_bytes;
   bool head_short_opt = true;             // option "head_short"
   std::vector<HeadShortArgs> head_short;  // per layer (MHA without a query latent); grid == 0: head_attn
+  std::vector<char> head_latent;          // per layer (MHA behind a query latent): launch_head_latent below the split regime
   std::vector<HeadAttnArgs> head_attn;  // per layer (MHA path): second-stage projections + attention, one launch
   bool graph_primed[8] = {false, false, false, false, false, false, false, false};
   const char* class_filter = nullptr;  // dsk_time_kernel_class

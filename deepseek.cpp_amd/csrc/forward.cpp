@@ -144,6 +144,7 @@ int build_plans(dsk_model* m) {
     HeadShortArgs z;
     memset(&z, 0, sizeof z);
     m->head_short.assign(nl, z);
+    m->head_latent.assign(nl, 0);
   }
   // Heads that go through launch_head_short leave their output in 32 bits, and wo's workgroups quantise it (K-quants): up to 16 blocks, one per wave.  V2-Lite
   // (8 blocks): wo 4.8 -> 5.1 us.  (V3's 64: 9.5 -> 13.2, dearer than the hand-over between heads.)
@@ -230,7 +231,9 @@ int build_plans(dsk_model* m) {
         DSK_TRY(head_attn_plan(A));
         A.a.out = m->att_out;
         m->head_attn[l] = A;
-        if (short_heads) DSK_TRY(head_short_plan(m->head_short[l], A, std::min(c.max_seq_len, std::max(1, c.rs_original_max_position_embeddings))));
+        const int kv_cap = std::min(c.max_seq_len, std::max(1, c.rs_original_max_position_embeddings));
+        if (short_heads) DSK_TRY(head_short_plan(m->head_short[l], A, kv_cap));
+        m->head_latent[l] = m->head_short_opt && head_latent_supported(A, kv_cap);
         m->head_attn_bytes[l] = bytes;
       }
     }
@@ -625,6 +628,8 @@ static int attention_mha(dsk_model* m, int l, int max_kv) {
     HeadShortArgs S = m->head_short[l];
     if (HA.tap_qs) { S.tap_qs = HA.tap_qs + HA.tap_stride; S.tap_d = HA.tap_d + (HA.tap_stride >> 8); }
     PROFILED("attn_mha", attn_bytes, launch_head_short(st, S, m->sp_dev, max_kv));
+  } else if (n_split == 1 && m->head_latent[l]) {
+    PROFILED("attn_mha", attn_bytes, launch_head_latent(st, HA, m->sp_dev, max_kv));
   } else {
     PROFILED("attn_mha", attn_bytes, launch_head_attn(st, HA, m->sp_dev, max_kv, n_split));
   }

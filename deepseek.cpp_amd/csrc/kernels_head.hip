@@ -1,15 +1,205 @@
-// kernels_head.hip -- MHA of one token for models without a query latent (src/infer.cpp:943-1049, 728-762): per head, the rows of wkv_b, RoPE, the cache
+// kernels_head.hip -- MHA of one token (src/infer.cpp:943-1049, 728-762): per head, the rows of wkv_b (and of wq_b: head_attn_latent_kernel), RoPE, the cache
 // entries and attention in one launch, with everything that does not depend on anything requested at once.
 //
 // head_attn_kernel (kernels_gemv.hip) does the same as a chain: latents, rows, query, rope's inputs, cache write, keys, each a trip of 0.7 - 1 us behind a
 // barrier that waits for stores.  Of those only the latents -> rows -> current key and value depend on each other.  So: the latents, the query, the
 // rope's inputs and the head's rows are requested at entry, keys and values (of up to 256 positions) behind the first barrier; the current position's
 // key and value go from LDS into the scores and the mix, rounded as the cache rounds them, and to the cache at the very end; barriers are for LDS
-// only.  Values, sums and their orders are head_attn_kernel's: the same bits.  The output leaves in 32 bits; wo quantises it (8 blocks for V2-Lite: cheaper in each of
-// its workgroups than a hand-over between heads here).
+// only.  Values, sums and their orders are head_attn_kernel's: the same bits.  Without a query latent the output leaves in 32 bits and wo quantises it (8 blocks for
+// V2-Lite: cheaper in each of its workgroups than a hand-over between heads here).
 // Bound by latency: 16 workgroups.  V2-Lite at 62 positions, us: Q2_K 13.2 -> 6.9, F8E5M2 12.8 -> 9.1 (its 131 KB of rows are 2.7 us for the one compute unit); a token 1130 -> 985, 1602 -> 1505.
 #include "dsk_internal.h"
 #include "gemv_device.h"
+
+namespace {
+
+// what attention needs of a head's shape, and where
+struct HeadShape { int H, h, hd, vd, nope, rope, is_v3; uint16_t *kcache, *vcache; int kv_pos, kv_len; };
+
+// Keys and values on their way: 16 lanes a position, positions 4 wave .. + 3 of every 64; thread (g, i4) the values of positions g, g + TG, ...  Buffer loads: one
+// lane offset each for keys and values, the steps in scalar registers, and zeros without traffic behind the context's end (the range check of a
+// raw buffer counts the scalar offset).
+template <int VN>
+struct HeadKV {
+  rsrc_t KB, VB;
+  u32 krow, vrow, koff, voff;
+  int grp, sl, TG, g, i4;
+  ad::f16x4 k[4][3], v[VN];
+};
+template <int VN>
+DEV void head_keys(const HeadShape& S, HeadKV<VN>& R, int t0) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    if (t0 + u * 64 >= S.kv_len) break;
+    const int step = (t0 + u * 64) * (int)R.krow;
+    R.k[u][0] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)R.koff, step, 0));
+    R.k[u][1] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)R.koff + 128, step, 0));
+    R.k[u][2] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)R.koff + 256, step, 0));
+  }
+}
+template <int VN>
+DEV void head_places(const HeadShape& S, HeadKV<VN>& R, int tid, int wave, int lane) {
+  const int tpp = S.vd >> 2;
+  R.grp = lane >> 4; R.sl = lane & 15;
+  R.TG = 1024 / tpp; R.g = tid / tpp; R.i4 = tid - R.g * tpp;
+  R.krow = (u32)S.H * S.hd * 2; R.vrow = (u32)S.H * S.vd * 2;
+  R.KB = __builtin_amdgcn_make_buffer_rsrc(S.kcache, 0, (int)(S.kv_len * R.krow), 0x00020000);
+  R.VB = __builtin_amdgcn_make_buffer_rsrc(S.vcache, 0, (int)(S.kv_len * R.vrow), 0x00020000);
+  R.koff = ((u32)(wave * 4 + R.grp) * S.H + S.h) * S.hd * 2 + R.sl * 8;
+  R.voff = R.g < R.TG ? ((u32)R.g * S.H + S.h) * S.vd * 2 + R.i4 * 8 : 0xfffffff0u;
+}
+template <int VN>
+DEV void head_values(const HeadShape& S, HeadKV<VN>& R) {
+#pragma unroll
+  for (int j = 0; j < VN; ++j)
+    if (j * R.TG < S.kv_len) R.v[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.VB, (int)R.voff, j * R.TG * (int)R.vrow, 0));
+}
+// rotation of the sink keys by one position, in f16 (src/infer.cpp:1008-1020), in front of the keys' requests
+DEV void head_sinks(const HeadShape& S, const StepParams* sp, int kv_sink, int tid) {
+  const int half = S.rope >> 1;
+  for (int r = 0; r < kv_sink; ++r) {
+    uint16_t* kh = S.kcache + ((size_t)r * S.H + S.h) * S.hd + S.nope;
+    float re = 0.f, im = 0.f;
+    if (tid < half) ad::rope_rot(ad::h2f(kh[2 * tid]), ad::h2f(kh[2 * tid + 1]), sp->rope_cs1[2 * tid], sp->rope_cs1[2 * tid + 1], re, im);
+    __syncthreads();
+    if (tid < half) {
+      kh[S.is_v3 ? 2 * tid : tid] = ad::f2h(re);
+      kh[S.is_v3 ? 2 * tid + 1 : tid + half] = ad::f2h(im);
+    }
+    __syncthreads();
+  }
+}
+// Scores, softmax and mix (src/infer.cpp:1022-1045) in attn_mha_body's order; returns output tid of the head (tid < vd).  qv: the lane's 12 values of the rotated query;
+// kvb_s: the head's rows of wkv_b; kr_s: this position's rotated key part, as the cache will hold it.  part: 4096 floats, att: kv_len.
+template <int VN>
+DEV float head_attend(const HeadShape& S, HeadKV<VN>& R, const float (&qv)[3][4], const float* kvb_s, const uint16_t* kr_s, float* att, float* part, int tid, int wave, int lane,
+                      bool timed, unsigned long long (&stamps)[2]) {
+  constexpr int NW = 16, NT = 1024;
+  const int hd = S.hd, vd = S.vd, nope = S.nope, kv_len = S.kv_len, kv_pos = S.kv_pos, grp = R.grp, sl = R.sl, TG = R.TG, g = R.g, i4 = R.i4;
+  {
+    const bool in2 = 128 + sl * 4 < hd, in1 = 64 + sl * 4 < hd, in0 = sl * 4 < hd;
+    const float inv = sqrtf((float)hd);
+    const int pw = wave * 4 + grp;
+    for (int t0 = 0; t0 < kv_len; t0 += 256) {
+      if ((kv_pos & 63) == pw && kv_pos >= t0 && kv_pos < t0 + 256) {  // this position's key is not in the cache yet
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const int d0 = min(64 * j + sl * 4, hd - 4);
+          const f32x4 x = *reinterpret_cast<const f32x4*>(kvb_s + min(d0, nope - 4));
+          const ad::f16x4 y = *reinterpret_cast<const ad::f16x4*>(kr_s + max(d0 - nope, 0));
+          const ad::f16x4 c = d0 < nope ? ad::f16x4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w} : y;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (u == (kv_pos - t0) >> 6) R.k[u][j] = c;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + u * 64 + pw;
+        if (t0 + u * 64 >= kv_len) break;
+        float p = 0.f;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (j == 0 ? in0 : j == 1 ? in1 : in2) {
+            p = fmaf(qv[j][0], (float)R.k[u][j].x, p);
+            p = fmaf(qv[j][1], (float)R.k[u][j].y, p);
+            p = fmaf(qv[j][2], (float)R.k[u][j].z, p);
+            p = fmaf(qv[j][3], (float)R.k[u][j].w, p);
+          }
+        p = ad::row16_sum(p);
+        if (sl == 0 && t < kv_len) att[t] = p / inv;
+      }
+      if (t0 + 256 < kv_len) head_keys(S, R, t0 + 256);
+    }
+  }
+  lds_barrier();
+  if (timed) stamps[0] = wall_clock64();
+  // ---- softmax (src/infer.cpp:472-487): a wave's trees over 64 positions, the waves' sums in order ----
+  if (kv_len <= 64) {
+    if (wave == 0) {
+      const float a0 = lane < kv_len ? att[lane] : -INFINITY;
+      const float mx = ad::wave_max_dpp(a0);
+      const float e = lane < kv_len ? expf(a0 - mx) : 0.f;
+      const float sum = ad::wave_sum_dpp(e);
+      if (lane < kv_len) att[lane] = e / sum;
+    }
+  } else {
+    float mx = -INFINITY;
+    for (int t = tid; t < kv_len; t += NT) mx = fmaxf(mx, att[t]);
+    mx = ad::wave_max_dpp(mx);
+    if (lane == 0) part[wave] = mx;
+    lds_barrier();
+    mx = part[0];
+    for (int i = 1; i < NW; ++i) mx = fmaxf(mx, part[i]);
+    float sum = 0.f;
+    for (int t = tid; t < kv_len; t += NT) {
+      const float e = expf(att[t] - mx);
+      att[t] = e;
+      sum += e;
+    }
+    sum = ad::wave_sum_dpp(sum);
+    if (lane == 0) part[NW + wave] = sum;
+    lds_barrier();
+    float total = 0.f;
+    for (int i = 0; i < NW; ++i) total += part[NW + i];
+    for (int t = tid; t < kv_len; t += NT) att[t] = att[t] / total;
+  }
+  lds_barrier();
+  // ---- values: every thread its positions in order, then the groups in order ----
+  auto value_here = [&]() {  // this position's, as the cache will hold it
+    const f32x4 x = *reinterpret_cast<const f32x4*>(kvb_s + nope + i4 * 4);
+    return ad::f16x4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w};
+  };
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  auto mix = [&](int t, ad::f16x4 y) {
+    if (t == kv_pos) y = value_here();
+    const float w = att[t];
+    acc[0] = fmaf(w, (float)y.x, acc[0]);
+    acc[1] = fmaf(w, (float)y.y, acc[1]);
+    acc[2] = fmaf(w, (float)y.z, acc[2]);
+    acc[3] = fmaf(w, (float)y.w, acc[3]);
+  };
+  if (g < TG) {
+#pragma unroll
+    for (int j = 0; j < VN; ++j)
+      if (g + j * TG < kv_len) mix(g + j * TG, R.v[j]);
+    for (int t0 = g + VN * TG; t0 - g < kv_len; t0 += 4 * TG) {
+      ad::f16x4 y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.VB, (int)R.voff, (t0 - g + j * TG) * (int)R.vrow, 0));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (t0 + j * TG < kv_len) mix(t0 + j * TG, y[j]);
+    }
+    *reinterpret_cast<f32x4*>(part + (size_t)g * vd + i4 * 4) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+  }
+  lds_barrier();
+  if (timed) stamps[1] = wall_clock64();
+  float o = 0.f;
+  if (tid < vd) {
+    const int ng = min(TG, kv_len);  // (the others' sums are zeros)
+    for (int g0 = 0; g0 < ng; g0 += 8) {
+      float y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = part[min(g0 + i, ng - 1) * vd + tid];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o += g0 + i < ng ? y[i] : 0.f;
+    }
+  }
+  return o;
+}
+// the cache entries (src/infer.cpp:985-1005), by the upper half of the workgroup
+DEV void head_cache(const HeadShape& S, const float* kvb_s, const uint16_t* kr_s, int tid) {
+  uint16_t* kc = S.kcache + ((size_t)S.kv_pos * S.H + S.h) * S.hd;
+  uint16_t* vc = S.vcache + ((size_t)S.kv_pos * S.H + S.h) * S.vd;
+  const int i = tid - 512;
+  if (i < 0) return;
+  if (i < S.nope) kc[i] = ad::f2h(kvb_s[i]);
+  if (i < S.rope) kc[S.nope + i] = kr_s[i];
+  if (i < S.vd) vc[i] = ad::f2h(kvb_s[S.nope + i]);
+}
+
+}  // namespace
 
 // RS x ROUNDS row sets of a wave, two rounds on their way
 template <int QT, int RS, int ROUNDS>
@@ -29,7 +219,7 @@ __global__ __launch_bounds__(1024) void head_attn_short_kernel(const StepParams*
     return;
   }
   const unsigned long long t_entry = A.timeline ? wall_clock64() : 0ull;
-  unsigned long long t_staged = 0, t_rows = 0, t_scores = 0, t_mix = 0;
+  unsigned long long t_staged = 0, t_rows = 0, stamps[2] = {0, 0};
   const int hd = hv & 0xffff, vd = hv >> 16, nope = A.nope, rope = A.rope, n = A.lora, nrows = nope + vd, half = rope >> 1;
   uint8_t* act = smem;
   float* att = reinterpret_cast<float*>(smem + A.lds_kv);
@@ -99,43 +289,12 @@ __global__ __launch_bounds__(1024) void head_attn_short_kernel(const StepParams*
     scratch[wave] = 0.f;
   }
   lds_barrier();
-  // ---- keys and values: 16 lanes a position, positions 4 wave .. + 3 of every 64; thread (g, i4) positions g, g + TG, ... ----
-  const int grp = lane >> 4, sl = lane & 15;
-  const int tpp = vd >> 2, TG = NT / tpp, g = tid / tpp, i4 = tid - g * tpp;
-  if (kv_sink > 0) {  // rotation of the sink keys by one position, in f16 (src/infer.cpp:1008-1020)
-    for (int r = 0; r < kv_sink; ++r) {
-      uint16_t* kh = kcache + ((size_t)r * H + h) * hd + nope;
-      float re = 0.f, im = 0.f;
-      if (tid < half) ad::rope_rot(ad::h2f(kh[2 * tid]), ad::h2f(kh[2 * tid + 1]), sp->rope_cs1[2 * tid], sp->rope_cs1[2 * tid + 1], re, im);
-      __syncthreads();
-      if (tid < half) {
-        kh[A.is_v3 ? 2 * tid : tid] = ad::f2h(re);
-        kh[A.is_v3 ? 2 * tid + 1 : tid + half] = ad::f2h(im);
-      }
-      __syncthreads();
-    }
-  }
-  // (buffer loads: one lane offset each for keys and values, the steps in scalar registers, and zeros without traffic behind the context's end)
-  const u32 krow = (u32)H * hd * 2, vrow = (u32)H * vd * 2;
-  const rsrc_t KB = __builtin_amdgcn_make_buffer_rsrc(kcache, 0, (int)(kv_len * krow), 0x00020000), VB = __builtin_amdgcn_make_buffer_rsrc(vcache, 0, (int)(kv_len * vrow), 0x00020000);
-  const u32 koff = ((u32)(wave * 4 + grp) * H + h) * hd * 2 + sl * 8;
-  const u32 voff = g < TG ? ((u32)g * H + h) * vd * 2 + i4 * 8 : 0xfffffff0u;
-  const bool in2 = 128 + sl * 4 < hd, in1 = 64 + sl * 4 < hd, in0 = sl * 4 < hd;
-  ad::f16x4 k[4][3], v[VN];
-  auto request_keys = [&](int t0) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (t0 + u * 64 >= kv_len) break;
-      const int step = (t0 + u * 64) * (int)krow;
-      k[u][0] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(KB, (int)koff, step, 0));
-      k[u][1] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(KB, (int)koff + 128, step, 0));
-      k[u][2] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(KB, (int)koff + 256, step, 0));
-    }
-  };
-  request_keys(0);
-#pragma unroll
-  for (int j = 0; j < VN; ++j)
-    if (j * TG < kv_len) v[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(VB, (int)voff, j * TG * (int)vrow, 0));
+  const HeadShape S{H, h, hd, vd, nope, rope, A.is_v3, kcache, vcache, kv_pos, kv_len};
+  HeadKV<VN> R;
+  if (kv_sink > 0) head_sinks(S, sp, kv_sink, tid);
+  head_places(S, R, tid, wave, lane);
+  head_keys(S, R, 0);
+  head_values(S, R);
   // ---- the latent staged; the query and this position's key part rotated ----
   if (latent_wave) {
     if constexpr (KQ) {
@@ -199,137 +358,176 @@ __global__ __launch_bounds__(1024) void head_attn_short_kernel(const StepParams*
   }
   lds_barrier();
   if (A.timeline) t_rows = wall_clock64();
-  // ---- scores ----
-  {
-    float qv[3][4];
+  float qv[3][4];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const f32x4 t = *reinterpret_cast<const f32x4*>(q_s + min(64 * j + sl * 4, hd - 4));
-      const bool in = 64 * j + sl * 4 < hd;
-      qv[j][0] = in ? t.x : 0.f; qv[j][1] = in ? t.y : 0.f; qv[j][2] = in ? t.z : 0.f; qv[j][3] = in ? t.w : 0.f;
-    }
-    const float inv = sqrtf((float)hd);
-    const int pw = wave * 4 + grp;
-    for (int t0 = 0; t0 < kv_len; t0 += 256) {
-      if ((kv_pos & 63) == pw && kv_pos >= t0 && kv_pos < t0 + 256) {  // this position's key is not in the cache yet
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const int d0 = min(64 * j + sl * 4, hd - 4);
-          const f32x4 x = *reinterpret_cast<const f32x4*>(kvb_s + min(d0, nope - 4));
-          const ad::f16x4 y = *reinterpret_cast<const ad::f16x4*>(kr_s + max(d0 - nope, 0));
-          const ad::f16x4 c = d0 < nope ? ad::f16x4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w} : y;
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (u == (kv_pos - t0) >> 6) k[u][j] = c;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = t0 + u * 64 + pw;
-        if (t0 + u * 64 >= kv_len) break;
-        float p = 0.f;
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          if (j == 0 ? in0 : j == 1 ? in1 : in2) {
-            p = fmaf(qv[j][0], (float)k[u][j].x, p);
-            p = fmaf(qv[j][1], (float)k[u][j].y, p);
-            p = fmaf(qv[j][2], (float)k[u][j].z, p);
-            p = fmaf(qv[j][3], (float)k[u][j].w, p);
-          }
-        p = ad::row16_sum(p);
-        if (sl == 0 && t < kv_len) att[t] = p / inv;
-      }
-      if (t0 + 256 < kv_len) request_keys(t0 + 256);
-    }
+  for (int j = 0; j < 3; ++j) {
+    const f32x4 t = *reinterpret_cast<const f32x4*>(q_s + min(64 * j + R.sl * 4, hd - 4));
+    const bool in = 64 * j + R.sl * 4 < hd;
+    qv[j][0] = in ? t.x : 0.f; qv[j][1] = in ? t.y : 0.f; qv[j][2] = in ? t.z : 0.f; qv[j][3] = in ? t.w : 0.f;
   }
-  lds_barrier();
-  if (A.timeline) t_scores = wall_clock64();
-  // ---- softmax (src/infer.cpp:472-487): a wave's trees over 64 positions, the waves' sums in order ----
-  if (kv_len <= 64) {
-    if (wave == 0) {
-      const float a0 = lane < kv_len ? att[lane] : -INFINITY;
-      const float mx = ad::wave_max_dpp(a0);
-      const float e = lane < kv_len ? expf(a0 - mx) : 0.f;
-      const float sum = ad::wave_sum_dpp(e);
-      if (lane < kv_len) att[lane] = e / sum;
-    }
-  } else {
-    float mx = -INFINITY;
-    for (int t = tid; t < kv_len; t += NT) mx = fmaxf(mx, att[t]);
-    mx = ad::wave_max_dpp(mx);
-    if (lane == 0) part[wave] = mx;
-    lds_barrier();
-    mx = part[0];
-    for (int i = 1; i < NW; ++i) mx = fmaxf(mx, part[i]);
-    float sum = 0.f;
-    for (int t = tid; t < kv_len; t += NT) {
-      const float e = expf(att[t] - mx);
-      att[t] = e;
-      sum += e;
-    }
-    sum = ad::wave_sum_dpp(sum);
-    if (lane == 0) part[NW + wave] = sum;
-    lds_barrier();
-    float total = 0.f;
-    for (int i = 0; i < NW; ++i) total += part[NW + i];
-    for (int t = tid; t < kv_len; t += NT) att[t] = att[t] / total;
-  }
-  lds_barrier();
-  // ---- values: every thread its positions in order, then the groups in order ----
-  auto value_here = [&]() {  // this position's, as the cache will hold it
-    const f32x4 x = *reinterpret_cast<const f32x4*>(kvb_s + nope + i4 * 4);
-    return ad::f16x4{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w};
-  };
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  auto mix = [&](int t, ad::f16x4 y) {
-    if (t == kv_pos) y = value_here();
-    const float w = att[t];
-    acc[0] = fmaf(w, (float)y.x, acc[0]);
-    acc[1] = fmaf(w, (float)y.y, acc[1]);
-    acc[2] = fmaf(w, (float)y.z, acc[2]);
-    acc[3] = fmaf(w, (float)y.w, acc[3]);
-  };
-  if (g < TG) {
-#pragma unroll
-    for (int j = 0; j < VN; ++j)
-      if (g + j * TG < kv_len) mix(g + j * TG, v[j]);
-    for (int t0 = g + VN * TG; t0 - g < kv_len; t0 += 4 * TG) {
-      ad::f16x4 y[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(VB, (int)voff, (t0 - g + j * TG) * (int)vrow, 0));
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (t0 + j * TG < kv_len) mix(t0 + j * TG, y[j]);
-    }
-    *reinterpret_cast<f32x4*>(part + (size_t)g * vd + i4 * 4) = f32x4{acc[0], acc[1], acc[2], acc[3]};
-  }
-  lds_barrier();
-  if (A.timeline) t_mix = wall_clock64();
-  if (tid < vd) {
-    float o = 0.f;
-    const int ng = min(TG, kv_len);  // (the others' sums are zeros)
-    for (int g0 = 0; g0 < ng; g0 += 8) {
-      float y[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) y[i] = part[min(g0 + i, ng - 1) * vd + tid];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) o += g0 + i < ng ? y[i] : 0.f;
-    }
-    A.out[(size_t)h * vd + tid] = o;
-  }
-  // ---- the cache entries (src/infer.cpp:985-1005) ----
-  uint16_t* kc = kcache + ((size_t)kv_pos * H + h) * hd;
-  uint16_t* vc = vcache + ((size_t)kv_pos * H + h) * vd;
-  if (tid >= 512) {
-    const int i = tid - 512;
-    if (i < nope) kc[i] = ad::f2h(kvb_s[i]);
-    if (i < rope) kc[nope + i] = kr_s[i];
-    if (i < vd) vc[i] = ad::f2h(kvb_s[nope + i]);
-  }
+  const float o = head_attend(S, R, qv, kvb_s, kr_s, att, part, tid, wave, lane, A.timeline != nullptr, stamps);
+  if (tid < vd) A.out[(size_t)h * vd + tid] = o;
+  head_cache(S, kvb_s, kr_s, tid);
   if (A.timeline && tid == 0 && blockIdx.x < DSK_TL_WGS) {
     unsigned long long* tl = A.timeline + (size_t)blockIdx.x * 8;
-    tl[0] = t_entry; tl[1] = t_staged; tl[2] = t_rows; tl[3] = t_scores; tl[4] = t_mix; tl[5] = wall_clock64();
+    tl[0] = t_entry; tl[1] = t_staged; tl[2] = t_rows; tl[3] = stamps[0]; tl[4] = stamps[1]; tl[5] = wall_clock64();
   }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// The same behind a query latent, for DeepSeek-V3's heads in Q2_K (192 rows of 1536, 256 of 512, 8 lanes a row): the two latents normed and quantised in one pass, then
+// wkv_b's and wq_b's rows as in head_attn_kernel, whose order and bits these are.  A compute unit returns loads in order and holds ~50 KB of them: the first rows
+// are requested at entry, the next behind the latents, keys and values behind those and under the multiplies.  The output is quantised here, by the last of
+// a block's heads (64 blocks: dearer in each of wo's workgroups).  128 heads, us a launch: at 20 positions 16.5 -> 12.3, at 200 19.8 -> 14.9; five of V3's blocks 487 -> 465 a
+// token.
+// ------------------------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(1024) void head_attn_latent_kernel(const StepParams* __restrict__ sp, const float* __restrict__ q_a, const float* __restrict__ kv_a,
+                                                               const float* __restrict__ q_norm, const float* __restrict__ kv_norm, uint16_t* kcache, uint16_t* vcache,
+                                                               const HeadAttnArgs A) {
+  constexpr int QT = DSK_QUANT_Q2_K, NQ = 1536, NKV = 512, NBQ = NQ / 256, NBKV = NKV / 256, HD = 192, NOPE = 128, VN = 8;
+  __shared__ __attribute__((aligned(16))) uint8_t act[(NQ + NKV) / 64 * ITEM_LDS];
+  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float q_s[HD];
+  __shared__ __attribute__((aligned(16))) float kvb_s[256];
+  __shared__ __attribute__((aligned(16))) float cs_s[64];
+  __shared__ __attribute__((aligned(16))) uint16_t kr_s[64];
+  __shared__ __attribute__((aligned(16))) float part[4096];
+  __shared__ int last_flag;
+  extern __shared__ __attribute__((aligned(16))) float att[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, h = blockIdx.x;
+  const int H = A.a.n_heads;
+  if (h >= H) {  // prefetch workgroups (HeadAttnArgs::pf_wgs)
+    tail_prefetch(A.pf_p, A.pf_n, tid, 1024);
+    return;
+  }
+  unsigned long long* const tl = A.timeline && h < DSK_TL_WGS ? A.timeline + (size_t)h * 8 : nullptr;
+  const unsigned long long t_entry = tl ? wall_clock64() : 0ull;
+  unsigned long long t_staged = 0, t_rows = 0, stamps[2] = {0, 0};
+  uint8_t *act_q = act, *act_kv = act + NQ / 64 * ITEM_LDS;
+  // ---- requests at entry: the rope's inputs (one wave), the latents (a block each of eight waves), the head's rows of wkv_b ----
+  float2 kp, cs;
+  f32x4 lt, lw;
+  if (wave == 15) {
+    kp = *reinterpret_cast<const float2*>(kv_a + NKV + 2 * (lane & 31));
+    cs = *reinterpret_cast<const float2*>(sp->rope_cs + 2 * (lane & 31));
+  }
+  const bool is_q = wave < NBQ, mine = wave < NBQ + NBKV;
+  if (mine) {
+    lt = *reinterpret_cast<const f32x4*>((is_q ? q_a + wave * 256 : kv_a + (wave - NBQ) * 256) + lane * 4);
+    lw = *reinterpret_cast<const f32x4*>((is_q ? q_norm + wave * 256 : kv_norm + (wave - NBQ) * 256) + lane * 4);
+  }
+  const int rloc = lane >> 3, sub = lane & 7, q = sub & 3, lr0 = wave * 8 + rloc, lr1 = 128 + lr0;
+  WPtr P;
+  P.present = true; P.hm = nullptr; P.scale = P.scale2 = nullptr; P.qs2 = P.sc2 = P.hm2 = P.dm2 = nullptr;
+  P.qs = A.tkv.qs; P.sc = A.tkv.sc; P.dm = A.tkv.dm;
+  const KQRsrc Bk = kq_rsrc<QT, false>(P);
+  P.qs = A.tq.qs; P.sc = A.tq.sc; P.dm = A.tq.dm;
+  const KQRsrc Bq = kq_rsrc<QT, false>(P);
+  const int rbq0[1] = {(h * HD + lr0) * NBQ + (sub >> 2)}, rbq1[1] = {(h * HD + (lr1 < HD ? lr1 : HD - 1)) * NBQ + (sub >> 2)};
+  const int rbk0[1] = {(h * 256 + lr0) * NBKV + (sub >> 2)}, rbk1[1] = {(h * 256 + lr1) * NBKV + (sub >> 2)};
+  ChunkKQ<QT, 1, 3, false> cq0, cq1;
+  ChunkKQ<QT, 1, 1, false> ck0, ck1;
+  load_chunk_kq<QT, 1, 1, false>(ck0, Bk, 1, 8, sub, 3, q, rbk0, 0);
+  load_chunk_kq<QT, 1, 1, false>(ck1, Bk, 1, 8, sub, 3, q, rbk1, 0);
+  const int kv_pos = sp->kv_pos, kv_len = sp->kv_len, kv_sink = sp->kv_sink;
+  // ---- both latents normed and quantised (src/infer.cpp:946-974, quant.cpp:616-653); this position's key part rotated ----
+  if (mine) {
+    float ss = fmaf(lt.x, lt.x, fmaf(lt.y, lt.y, fmaf(lt.z, lt.z, lt.w * lt.w)));
+    ss = wave_sum(ss);
+    if (lane == 0) scratch[wave] = ss;
+  }
+  lds_barrier();
+  if (mine) {
+    float total = 0.f;
+    if (is_q) for (int i = 0; i < NBQ; ++i) total += scratch[i];
+    else for (int i = NBQ; i < NBQ + NBKV; ++i) total += scratch[i];
+    const float scale = 1.0f / sqrtf(total / (float)(is_q ? NQ : NKV) + (is_q ? A.tq.eps : A.tkv.eps));
+    const float y[4] = {lt.x * scale * lw.x, lt.y * scale * lw.y, lt.z * scale * lw.z, lt.w * scale * lw.w};
+    q8k_block_lds<LAY_Q2>(y, lane, act + (size_t)wave * 4 * ITEM_LDS);
+  }
+  const int is_v3 = A.a.is_v3;
+  if (wave == 15 && lane < 32) {
+    float re, im;
+    ad::rope_rot(kp.x, kp.y, cs.x, cs.y, re, im);
+    kr_s[is_v3 ? 2 * lane : lane] = ad::f2h(re);
+    kr_s[is_v3 ? 2 * lane + 1 : lane + 32] = ad::f2h(im);
+    cs_s[2 * lane] = cs.x;
+    cs_s[2 * lane + 1] = cs.y;
+  }
+  lds_barrier();
+  if (tl) t_staged = wall_clock64();
+  if (A.tap_qs && h == 0) {  // parity tap
+    dump_staged_q8_inline<LAY_Q2>(act_q, NQ, A.tap_qs, A.tap_d, tid, 1024);
+    dump_staged_q8_inline<LAY_Q2>(act_kv, NKV, A.tap_qs + A.tap_stride, A.tap_d + (A.tap_stride >> 8), tid, 1024);
+  }
+  // ---- the rows, in the order of their arrival ----
+  const HeadShape S{H, h, HD, 128, NOPE, 64, is_v3, kcache, vcache, kv_pos, kv_len};
+  HeadKV<VN> R;
+  load_chunk_kq<QT, 1, 3, false>(cq0, Bq, 3, 24, sub, 3, q, rbq0, 0);
+  if (wave < 8) load_chunk_kq<QT, 1, 3, false>(cq1, Bq, 3, 24, sub, 3, q, rbq1, 0);
+  if (kv_sink > 0) head_sinks(S, sp, kv_sink, tid);
+  float acc[1] = {0.f}, dummy[1] = {0.f};
+  compute_chunk_kq<QT, 1, 1, false>(ck0, 1, 8, sub, 3, q, 0, act_kv + sub * ITEM_LDS, acc, dummy);
+  float v = lanes_sum(acc[0], 3);
+  if (sub == 0) kvb_s[lr0] = v;
+  acc[0] = 0.f;
+  compute_chunk_kq<QT, 1, 1, false>(ck1, 1, 8, sub, 3, q, 0, act_kv + sub * ITEM_LDS, acc, dummy);
+  v = lanes_sum(acc[0], 3);
+  if (sub == 0) kvb_s[lr1] = v;
+  acc[0] = 0.f;
+  compute_chunk_kq<QT, 1, 3, false>(cq0, 3, 24, sub, 3, q, 0, act_q + sub * ITEM_LDS, acc, dummy);
+  v = lanes_sum(acc[0], 3);
+  if (sub == 0) q_s[lr0] = v;
+  head_places(S, R, tid, wave, lane);  // (in the registers of the rows that are done)
+  head_keys(S, R, 0);
+  if (wave < 8) {
+    acc[0] = 0.f;
+    compute_chunk_kq<QT, 1, 3, false>(cq1, 3, 24, sub, 3, q, 0, act_q + sub * ITEM_LDS, acc, dummy);
+    v = lanes_sum(acc[0], 3);
+    if (sub == 0) q_s[lr1] = v;
+  }
+  head_values(S, R);
+  lds_barrier();
+  if (tl) t_rows = wall_clock64();
+  // ---- the query's part of this lane, rotated where it is read (src/infer.cpp:648-685) ----
+  float qv[3][4];
+  const int sl = lane & 15;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const f32x4 t = *reinterpret_cast<const f32x4*>(q_s + 64 * j + sl * 4);
+    qv[j][0] = t.x; qv[j][1] = t.y; qv[j][2] = t.z; qv[j][3] = t.w;
+  }
+  if (is_v3) {  // pairs (2 p, 2 p + 1) stay where they are
+    const f32x4 t = *reinterpret_cast<const f32x4*>(q_s + NOPE + sl * 4), c = *reinterpret_cast<const f32x4*>(cs_s + sl * 4);
+    ad::rope_rot(t.x, t.y, c.x, c.y, qv[2][0], qv[2][1]);
+    ad::rope_rot(t.z, t.w, c.z, c.w, qv[2][2], qv[2][3]);
+  } else {  // real parts in front of imaginary ones
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int o = sl * 4 + i, p = o & 31;
+      float re, im;
+      ad::rope_rot(q_s[NOPE + 2 * p], q_s[NOPE + 2 * p + 1], cs_s[2 * p], cs_s[2 * p + 1], re, im);
+      qv[2][i] = o < 32 ? re : im;
+    }
+  }
+  const float o = head_attend(S, R, qv, kvb_s, kr_s, att, part, tid, wave, lane, tl != nullptr, stamps);
+  ad::attn_out_q8(A.a, h, tid, o, &last_flag);
+  head_cache(S, kvb_s, kr_s, tid);
+  if (tl && tid == 0) { tl[0] = t_entry; tl[1] = t_staged; tl[2] = t_rows; tl[3] = stamps[0]; tl[4] = stamps[1]; tl[5] = wall_clock64(); }
+}
+// (the launches head_attn_latent_kernel is for: everything about the heads is compiled in)
+bool head_latent_supported(const HeadAttnArgs& A, int max_kv) {
+  return A.quant == DSK_QUANT_Q2_K && A.has_q && !A.tiled && A.lq_log2 == 3 && A.lkv_log2 == 3 && A.tq.n == 1536 && A.tkv.n == 512 && A.a.head_dim == 192 && A.a.nope == 128 &&
+         A.a.rope == 64 && A.a.v_dim == 128 && A.a.lora == 512 && A.tq.act_mode == ACT_F32_NORM && A.tkv.act_mode == ACT_F32_NORM &&
+         (double)max_kv * A.a.n_heads * 192 * 2 < 2147483648.0;
+}
+int launch_head_latent(hipStream_t st, const HeadAttnArgs& A, const StepParams* sp, int max_kv) {
+  const size_t lds = (size_t)max_kv * 4;
+  if (lds > 120 * 1024) DSK_FAIL(DSK_ERR_UNSUPPORTED, "attn: kv_len %d does not fit LDS", max_kv);
+  auto k = head_attn_latent_kernel;
+  if (lds > 40 * 1024) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(k, dim3(A.a.n_heads + (A.pf_wgs > 0 ? A.pf_wgs : 0)), dim3(1024), lds, st, sp, A.tq.a_f32, A.tkv.a_f32, A.tq.norm_w, A.tkv.norm_w, A.a.key_cache, A.a.value_cache, A);
+  return DSK_OK;
 }
 
 // ---- host side ------------------------------------------------------------------------------------------

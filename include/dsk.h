@@ -187,8 +187,8 @@ int dsk_model_destroy(dsk_model* m);
  *   "ride_kvwrite"    1  MLA: the latent cache write rides in the second-stage projection launch
  *   "att_q8_in_wo"    0  wo quantises the attention output in its own prologue (no finisher in the attention launch); always so where
  *                        "head_short" applies to K-quants
- *   "head_short"      1  MHA without a query latent: everything of a head that does not depend on anything requested at once (0: the
- *                        general per-head launch; bit-identical)
+ *   "head_short"      1  MHA without a query latent, and DeepSeek-V3's heads in Q2_K: everything of a head that does not depend on anything
+ *                        requested at once (0: the general per-head launch; bit-identical)
  *   "compact_absent"  1  expert-sharded w1/w3 launch compacts its row space over the experts present on the rank
  *   "rider_fill"      4  workgroup fill divisor of the shared expert's rider (1..16)
  *   "mla_flash_min" 320  context length from which MLA attention runs on the matrix cores

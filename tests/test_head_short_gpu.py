@@ -37,7 +37,7 @@ def same(ctx, c, positions, T=None, seed=3, short=True, **options):
     assert np.array_equal(A.run_block(0, x, pos), B.run_block(0, x, pos))
     assert np.array_equal(A.stage("att_out", c.n_heads * c.v_head_dim), B.stage("att_out", c.n_heads * c.v_head_dim))
     if c.quant in ("q2_k", "q3_k"):
-        for point, count in (("kv_a", c.kv_lora_rank), ("att", c.n_heads * c.v_head_dim)):
+        for point, count in (("kv_a", c.kv_lora_rank), ("att", c.n_heads * c.v_head_dim)) + ((("q_a", c.q_lora_rank),) if c.q_lora_rank else ()):
             for a, b in zip(A.stage_q8(point, count), B.stage_q8(point, count)):
                 assert np.array_equal(a, b), point
     A.close()
@@ -69,6 +69,18 @@ def test_small_heads(ctx, quant, over):
 def test_ring_and_sinks(ctx, quant):
     """past the ring: the current position is in the middle of the rows, and the sink keys turn by one position each token"""
     c = synth.preset("v2lite", quant, False, n_layers=2, hidden_dim=512, vocab_size=512, n_routed_experts=0, max_seq_len=96, rs_original_max_position_embeddings=80)
+    same(ctx, c, [79, 80, 81, 130, 200])
+
+
+@pytest.mark.parametrize("arch", ["DeepseekV3ForCausalLM", "DeepseekV2ForCausalLM"])  # (rope's pairs in place, or apart)
+def test_heads_behind_a_query_latent(ctx, arch):
+    c = synth.preset("v3", "q2_k", False, arch=arch, dim=512, hidden_dim=512, vocab_size=512, n_layers=2, n_routed_experts=0, n_shared_experts=0, max_seq_len=1100)
+    same(ctx, c, [0, 1, 15, 16, 62, 63, 64, 127, 128, 200, 255, 256, 300, 511, 700, 1022, 1023, 1024])
+
+
+def test_heads_behind_a_query_latent_past_the_ring(ctx):
+    c = synth.preset("v3", "q2_k", False, dim=512, hidden_dim=512, vocab_size=512, n_layers=2, n_routed_experts=0, n_shared_experts=0, max_seq_len=96,
+                     rs_original_max_position_embeddings=80)
     same(ctx, c, [79, 80, 81, 130, 200])
 
 
