@@ -666,8 +666,14 @@ __global__ __launch_bounds__(64 * NW, 2) void hyd_gemm16_kernel(const HydGemmArg
   constexpr int SG = GLU ? NW / 2 : NW;  // strips per workgroup
   const int strips = (A.rows + 15) >> 4;
   const int groups = (strips + SG - 1) / SG;
-  const int task = A.n_experts > 0 ? (int)blockIdx.x / groups : 0;
-  const int group = (int)blockIdx.x - task * groups;
+  int task = 0, group = (int)blockIdx.x, base = (int)blockIdx.y * 16 * MT, part = -1;
+  if (A.n_experts > 0) { task = group / groups; group -= task * groups; }
+  if (MT == 2 && A.halve_from > 0) {  // plain matrices: (chunk, strip group) pairs in one sequence, those from halve_from - 1 on as two workgroups each
+    const int b = (int)blockIdx.x, full = A.halve_from - 1, pair = b < full ? b : full + ((b - full) >> 1);
+    base = pair / groups * 32;
+    group = pair - pair / groups * groups;
+    if (b >= full) { part = (b - full) & 1; base += part * 16; }
+  }
   const int cnt = A.count ? __builtin_amdgcn_readfirstlane(A.count[task]) : A.m;
   if (cnt <= 0 || cnt < A.cnt_min || (A.cnt_max > 0 && cnt > A.cnt_max)) return;
   const int* list = A.list ? A.list + (size_t)task * A.list_stride : nullptr;
@@ -679,9 +685,10 @@ __global__ __launch_bounds__(64 * NW, 2) void hyd_gemm16_kernel(const HydGemmArg
   const rsrc_t RA = make_rsrc_n(A.a_qs, (u32)((size_t)A.a_rows * n));
   const rsrc_t RB = make_rsrc_n(A.a_bsums, (u32)((size_t)A.a_rows * (n >> 4) * 2));
   const rsrc_t RD = make_rsrc_n(A.a_d, (u32)((size_t)A.a_rows * nb * 4));
-  for (int base = (int)blockIdx.y * 16 * MT; base < cnt; base += (int)gridDim.y * 16 * MT) {
-    if (MT > 1 && cnt - base > 16) hyd16_pass<GLU, SEG4, NW, MT>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
+  for (; base < cnt; base += (int)gridDim.y * 16 * MT) {
+    if (MT > 1 && part < 0 && cnt - base > 16) hyd16_pass<GLU, SEG4, NW, MT>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
     else hyd16_pass<GLU, SEG4, NW, 1>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
+    if (MT == 2 && A.halve_from > 0) break;
   }
 }
 
@@ -791,6 +798,7 @@ static void hyd_gemm16_launch(hipStream_t st, dim3 grid, const HydGemmArgs& A) {
   if (A.n > 8 * 256) hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, true, NW, MT>), grid, dim3(64 * NW), 2 * hyd16_stage_b<MT>(), st, A);
   else hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, false, NW, MT>), grid, dim3(64 * NW), 2 * hyd16_stage_b<MT>(), st, A);
 }
+enum { HYD_CUS = 256 };
 template <bool GLU, int NQ>
 static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
   const long long units = (long long)(A.n_experts > 0 ? A.n_experts : 1) * ((A.rows + 15) >> 4);
@@ -819,12 +827,21 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
       hipLaunchKernelGGL((hyd_gemm16k_kernel<GLU>), dim3((unsigned)units, (unsigned)chunks), dim3(64 * ips_), lds_k, st, A);
       return;
     }
-    // 32 tokens a pass where that leaves most CUs a workgroup, else 16; then as many strips per workgroup as still do (the staging is paid once
-    // per workgroup, and every choice puts the same number of waves on the chip); at least 2 waves, a GLU pair's
+    // 16 tokens a pass as long as that is one workgroup of 8 waves a compute unit (more do not fit beside each other), with as many strips per
+    // workgroup as still leaves most CUs one; at least 2 waves, a GLU pair's.  Past that, 32 tokens: a workgroup then takes 1.5 times as long, but
+    // two rounds of 16 tokens take 2 (DeepSeek-V3's wo at 77 tokens, 280 workgroups or 168: 95.5 us -> 66.7).  What is left for a last round of at most
+    // half the CUs goes out as workgroups of 16 tokens, all CUs for 3 / 4 of a round (the same at 512 tokens, 896 workgroups: 268 -> 254).
     const int per = GLU ? 2 : 1, chunks2 = (A.m + 31) / 32;
     auto groups = [&](int nw) { return (unsigned)((units * per + nw - 1) / nw); };
-    if (A.m > 16 && (long long)groups(8) * chunks2 >= 192) {
-      hyd_gemm16_launch<GLU, 8, 2>(st, dim3(groups(8), (unsigned)chunks2), A);
+    if (A.m > 16 && (long long)groups(8) * chunks > HYD_CUS) {
+      const long long pairs = (long long)groups(8) * chunks2, left = pairs % HYD_CUS;
+      if (left > 0 && left <= HYD_CUS / 2 && pairs + left < (1ll << 30)) {
+        HydGemmArgs B = A;
+        B.halve_from = (int)(pairs - left) + 1;
+        hyd_gemm16_launch<GLU, 8, 2>(st, dim3((unsigned)(pairs + left)), B);
+      } else {
+        hyd_gemm16_launch<GLU, 8, 2>(st, dim3(groups(8), (unsigned)chunks2), A);
+      }
       return;
     }
     int nw = 8;
