@@ -292,15 +292,16 @@ __global__ __launch_bounds__(NW * 64) void gemv_kernel(const GemvLaunch* __restr
 // with LDS-only barriers (gemv_device.h lds_barrier), then the multiplies on registers that have been travelling since entry.
 // Same device functions, same column-step order, same lane trees as gemv_body: same bits.  The planner selects it (GemvLaunch::
 // ahead) for one activation group of <= 2 plain tasks, rows of <= 2 column steps, a share of <= one row group per workgroup.
+// What wo adds its rows to is requested at entry as well: V3's token of five blocks 464 -> 458 us (gemv_ahead_q8_kernel).
 // ------------------------------------------------------------------------------------
 // (Straight-line on purpose: row length and lanes per row are template constants and a (task, row group) pair that does not exist
 // for a wave reads through a NULL buffer descriptor - zeros, no memory traffic - instead of being branched around.  With a load
 // inside a branch hipcc's waitcnt pass must assume either path at the join and waits for EVERYTHING before x is touched.)
 // (NORM: false: the vector as it is, src/quant.cpp:616-653 alone - wo behind heads that leave 32-bit outputs, kernels_head.hip)
-template <int ITEMS, int LL, bool NORM = true>
+template <int QT, int ITEMS, int LL, bool NORM = true>
 __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __restrict__ Lp, const float* __restrict__ x, const float* __restrict__ norm_w,
                                                          float eps) {
-  constexpr int QT = DSK_QUANT_Q2_K, NW = 16, KB1 = 32 / NW, nb = ITEMS / 4, n = nb * 256, ITS = (ITEMS + (1 << LL) - 1) >> LL;
+  constexpr int LAY = QT == DSK_QUANT_Q2_K ? LAY_Q2 : LAY_Q3, NW = 16, KB1 = 32 / NW, nb = ITEMS / 4, n = nb * 256, ITS = (ITEMS + (1 << LL) - 1) >> LL;
   constexpr int RPW = 64 >> LL;
   static_assert(ITS <= 2 && nb <= 32, "gemv_ahead_kernel: rows of at most two column steps");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -333,6 +334,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
   int p_row[2];
   bool p_valid[2];
   float* p_out[2];
+  float p_old[2];  // (wo: what its row is added to, requested in front of the weights and not behind the multiplies)
   int p_epi[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -346,11 +348,13 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
     p_row[j] = p_valid[j] ? rr : (hi > 0 ? hi - 1 : 0);
     p_out[j] = glob(T.out);
     p_epi[j] = T.epilogue;
+    p_old[j] = NORM ? 0.f : p_out[j][p_row[j]];
     KQRsrc B;
     B.qs = make_rsrc_n(T.qs, has);
     B.sc = make_rsrc_n(T.sc, has);
     B.dm = make_rsrc_n(T.dm, has);
-    B.hm = B.qs2 = B.sc2 = B.dm2 = B.hm2 = B.qs;
+    B.hm = QT == DSK_QUANT_Q3_K ? make_rsrc_n(T.hm, has) : B.qs;
+    B.qs2 = B.sc2 = B.dm2 = B.hm2 = B.qs;
     const int rowblk[1] = {has ? p_row[j] * nb + (sub >> 2) : 0};
     load_chunk_kq<QT, 1, 2, false>(ch[j], B, ITS, ITEMS, sub, LL, q, rowblk, 0);
   }
@@ -379,7 +383,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
     if (b < nb) {
       float v[4] = {t[k].x, t[k].y, t[k].z, t[k].w};
       if (NORM) { v[0] = v[0] * scale * wv[k].x; v[1] = v[1] * scale * wv[k].y; v[2] = v[2] * scale * wv[k].z; v[3] = v[3] * scale * wv[k].w; }
-      q8k_block_lds<LAY_Q2>(v, lane, smem + (size_t)b * 4 * ITEM_LDS);
+      q8k_block_lds<LAY>(v, lane, smem + (size_t)b * 4 * ITEM_LDS);
     }
   }
   if (tl) t_staged = wall_clock64();
@@ -387,7 +391,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
   if (tl) t_bar = wall_clock64();
 #ifndef DSK_NO_TAPS
   if (L.tap_qs && bid == 0) {  // parity tap: what this launch staged (taps are armed for eager block runs only)
-    dump_staged_q8<LAY_Q2>(smem, n, L.tap_qs, L.tap_d, tid, NW * 64);
+    dump_staged_q8<LAY>(smem, n, L.tap_qs, L.tap_d, tid, NW * 64);
   }
 #endif
   // ---- 4. the multiplies (registers requested in 2.), the lane tree, the store ----
@@ -400,13 +404,114 @@ __global__ __launch_bounds__(1024) void gemv_ahead_kernel(const GemvLaunch* __re
     if (tl && j == 0) t_rows = wall_clock64();
     if (p_valid[j] && sub == 0) {
       float* o = p_out[j] + p_row[j];
-      if (p_epi[j] == EPI_ADD) *o += r;  // residual add, src/infer.cpp:832-834
-      else *o = r;
+      if (p_epi[j] != EPI_ADD) *o = r;
+      else if (NORM) *o += r;  // residual add, src/infer.cpp:832-834
+      else *o = p_old[j] + r;
     }
   }
   if (tl && tid == 0) {
     tl[0] = t_entry; tl[6] = t_staged; tl[7] = tl[1] = t_bar; tl[2] = t_rows; tl[3] = wall_clock64();
   }
+}
+// The same for F8E5M2 and F16 weights: rows of ITS whole column steps, a row to a wave (the first-stage projections by 16 waves, wo by NW).  Row sums in
+// rows_dot_f's order, the sum of squares in wg_sumsq's: the same bits.  A chain of round trips bounds them, not their 7.5 and 4.2 MB: V2-Lite in F8E5M2, first
+// stage 6.9 -> 4.9 us, wo 5.4 -> 4.6 by kernel time, a token's 27 of each 1346 -> 1212 us.
+template <int QT, int NW, int ITS, bool NORM>
+__global__ __launch_bounds__(NW * 64) void gemv_ahead_f_kernel(const GemvLaunch* __restrict__ Lp, const float* __restrict__ x, const float* __restrict__ norm_w, float eps) {
+  constexpr int EPI = FTraits<QT>::EPI, n = ITS * 64 * EPI, NQ = n / 4, KQ = (NQ + NW * 64 - 1) / (NW * 64);
+  static_assert(KQ <= 8, "gemv_ahead_f_kernel: wg_sumsq's single pass");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ float scratch[16];
+  const GemvLaunch& L = *Lp;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x;
+  // ---- 1. this thread's quads of x and of the norm weights ----
+  f32x4 t[KQ], wv[KQ];
+#pragma unroll
+  for (int k = 0; k < KQ; ++k) {
+    const int i = min(tid + k * NW * 64, NQ - 1);  // (a thread without a k-th quad re-reads the last one and drops it)
+    t[k] = reinterpret_cast<const f32x4*>(x)[i];
+    if (NORM) wv[k] = reinterpret_cast<const f32x4*>(norm_w)[i];
+  }
+  // ---- 2. the descriptor, this wave's row of the tasks' rows behind each other, its weights and block scales ----
+  const int n_tasks = L.grp_t0[1], nwg = L.grp_wg_end[0], first = L.t[0].vrow_end, vtotal = L.t[n_tasks - 1].vrow_end;
+  const unsigned units = (unsigned)vtotal;  // (part_unit is 1)
+  const int row0 = __builtin_amdgcn_readfirstlane((int)(units * (unsigned)bid / (unsigned)nwg)) + wave;
+  const int r_hi = __builtin_amdgcn_readfirstlane((int)(units * (unsigned)(bid + 1) / (unsigned)nwg));
+  const bool has = row0 < r_hi;
+  const GemvTask& T = L.t[has && row0 >= first ? 1 : 0];
+  const int row = has ? row0 - T.vrow_begin : 0;
+  float* const out = glob(T.out) + row;
+  const int epi = T.epilogue;
+  float old = 0.f;
+  if (!NORM) old = *out;  // (wo: what the row is added to)
+  const int b0 = L.b0, b1 = L.b1;
+  const bool p2 = ((b0 & (b0 - 1)) | (b1 & (b1 - 1))) == 0;
+  const int s0 = __builtin_ctz(b0), s1 = __builtin_ctz(b1), sc_cols = p2 ? (n + b1 - 1) >> s1 : (n + b1 - 1) / b1;
+  const rsrc_t W = make_rsrc_n(T.qs + (size_t)row * (n * FTraits<QT>::ESZ), has);
+  const bool scaled = T.scale != nullptr;
+  const rsrc_t S = make_rsrc_n(scaled ? T.scale + (size_t)(p2 ? row >> s0 : row / b0) * sc_cols : nullptr, scaled && has);
+  u32x4 w[ITS];
+  float sv[ITS];
+#pragma unroll
+  for (int u = 0; u < ITS; ++u) {
+    const int item = u * 64 + lane;
+    w[u] = __builtin_amdgcn_raw_buffer_load_b128(W, lane * 16, u * 1024, BUF_NT);
+    sv[u] = u2f(__builtin_amdgcn_raw_buffer_load_b32(S, (p2 ? item * EPI >> s1 : item * EPI / b1) * 4, 0, 0));
+  }
+  // ---- 3. rmsnorm (src/infer.cpp:601-611) of x into LDS (stage_f32), barriers for LDS alone ----
+  float scale = 1.f;
+  if constexpr (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < KQ; ++k)
+      if (tid + k * NW * 64 < NQ) {
+        ss = fmaf(t[k].x, t[k].x, ss);
+        ss = fmaf(t[k].y, t[k].y, ss);
+        ss = fmaf(t[k].z, t[k].z, ss);
+        ss = fmaf(t[k].w, t[k].w, ss);
+      }
+    ss = wave_sum(ss);
+    if (lane == 0) scratch[wave] = ss;
+    lds_barrier();
+    scale = 1.0f / sqrtf(scratch_total<NW>(scratch) / (float)n + eps);
+  }
+#pragma unroll
+  for (int k = 0; k < KQ; ++k) {
+    const int i = tid + k * NW * 64;
+    if (i < NQ) reinterpret_cast<f32x4*>(smem)[quad_place<EPI>(i, n / EPI)] = NORM ? t[k] * scale * wv[k] : t[k];
+  }
+  lds_barrier();
+  // ---- 4. the multiplies, the lane tree, the store ----
+  float acc = 0.f;
+#pragma unroll
+  for (int u = 0; u < ITS; ++u) {
+    float xa[EPI];
+#pragma unroll
+    for (int k = 0; k < EPI / 4; ++k) {
+      const f32x4 v = reinterpret_cast<const f32x4*>(smem)[k * (n / EPI) + u * 64 + lane];  // (quad_place)
+      xa[4 * k] = v.x; xa[4 * k + 1] = v.y; xa[4 * k + 2] = v.z; xa[4 * k + 3] = v.w;
+    }
+    acc = fmaf(fitem<QT>(w[u], xa, 0.f), scaled ? sv[u] : 1.0f, acc);
+  }
+  acc = lanes_sum(acc, 6);
+  if (has && lane == 0) *out = epi != EPI_ADD ? acc : (NORM ? *out : old) + acc;  // residual add, src/infer.cpp:832-834
+}
+// its number of column steps, 0: another plan
+static int gemv_ahead_f_steps(const GemvLaunch& h) {
+  const int epi = h.quant == DSK_QUANT_F8E5M2 ? 16 : 8;
+  if (h.tiled || (h.quant != DSK_QUANT_F8E5M2 && h.quant != DSK_QUANT_F16) || h.glu || h.R != 1 || h.n_groups != 1 || h.bd_heads != 0 || h.lpr_log2 != 6) return 0;
+  if (h.comb_x || h.comb_geometry || h.compact_absent || h.zero_absent || h.n_tasks > 2 || h.part_unit != 1 || h.grid != h.grp_wg_end[0] || h.timeline) return 0;
+  const GemvTask& T0 = h.t[0];
+  const bool norm = T0.act_mode == ACT_F32_NORM;
+  if (!(norm ? h.ahead & 1 : T0.act_mode == ACT_F32 && h.n_tasks == 1 && h.ahead & 2)) return 0;
+  for (int i = 0; i < h.n_tasks; ++i) {
+    const GemvTask& T = h.t[i];
+    if (T.n != T0.n || T.a_f32 != T0.a_f32 || T.norm_w != T0.norm_w || T.act_mode != T0.act_mode || T.e_qs != 0 || T.accum_w) return 0;
+  }
+  const long vtotal = h.t[h.n_tasks - 1].vrow_end, per = (vtotal + h.grid - 1) / h.grid;
+  const int its = T0.n / (64 * epi);
+  if (its * 64 * epi != T0.n || !(its == 1 || its == 2 || its == 4) || T0.n * 4 > 64 * 1024 || per > h.NW || vtotal * (h.grid + 1) >= 1l << 32) return 0;
+  return norm && h.NW != 16 ? 0 : its;
 }
 // The same for a plain one-task launch on a READY Q8_K vector with rows of four column steps (wo: 7168 rows of 16384 over 256
 // workgroups = two row groups of 16 each): the first row group's first two steps (43 KB per workgroup: what a CU keeps in flight)
@@ -444,12 +549,14 @@ __global__ __launch_bounds__(1024) void gemv_ahead_q8_kernel(const GemvLaunch* _
   ChunkKQ<QT, 1, 2, false> ca, cb;
   int row, rowblk[1];
   bool valid;
+  float old;  // (what the first row group is added to)
   {
     const int rr = lo + wave * RPW + rloc;
     const bool has = lo + wave * RPW < hi;
     valid = rr < hi;
     row = valid ? rr : (hi > 0 ? hi - 1 : 0);
     rowblk[0] = row * nb + (sub >> 2);
+    old = glob(T.out)[row];
     KQRsrc B0 = B;
     B0.qs = make_rsrc_n(T.qs, has); B0.sc = make_rsrc_n(T.sc, has); B0.dm = make_rsrc_n(T.dm, has);
     load_chunk_kq<QT, 1, 2, false>(ca, B0, ITS, ITEMS, sub, LL, q, rowblk, 0);
@@ -483,9 +590,7 @@ __global__ __launch_bounds__(1024) void gemv_ahead_q8_kernel(const GemvLaunch* _
     const float r = lanes_sum(acc[0], LL);
     if (tl) t_rows = wall_clock64();
     if (valid && sub == 0) {
-      float* o = out + row;
-      if (epi == EPI_ADD) *o += r;  // residual add, src/infer.cpp:832-834
-      else *o = r;
+      out[row] = epi == EPI_ADD ? old + r : r;  // residual add, src/infer.cpp:832-834
     }
   }
   // ---- 5. the remaining row groups ----
@@ -647,12 +752,12 @@ static bool gemv_kvwrite_ahead_ok(const GemvLaunch& h) {
 }
 // the plans gemv_ahead_kernel runs (set by gemv_plan: GemvLaunch::ahead)
 static bool gemv_ahead_ok(const GemvLaunch& h) {
-  if (h.tiled || h.quant != DSK_QUANT_Q2_K || h.glu || h.R != 1 || h.NW != 16 || h.n_groups != 1 || h.bd_heads != 0) return false;
+  if (h.tiled || (h.quant != DSK_QUANT_Q2_K && h.quant != DSK_QUANT_Q3_K) || h.glu || h.R != 1 || h.NW != 16 || h.n_groups != 1 || h.bd_heads != 0) return false;
   if (h.comb_x || h.comb_geometry || h.compact_absent || h.zero_absent || h.n_tasks > 2) return false;
   const GemvTask& T0 = h.t[0];
   // the instantiations: DeepSeek-V3 (rows of 7168: 112 items at 64 lanes per row, two column steps) and V2-Lite (rows of 2048: 32 items
   // at 32 lanes per row, one step)
-  const bool v3 = T0.n == 7168 && h.lpr_log2 == 6 && h.U == 2, v2l = T0.n == 2048 && h.lpr_log2 == 5 && h.U == 1;
+  const bool v3 = h.quant == DSK_QUANT_Q2_K && T0.n == 7168 && h.lpr_log2 == 6 && h.U == 2, v2l = T0.n == 2048 && h.lpr_log2 == 5 && h.U == 1;
   if (!(T0.act_mode == ACT_F32_NORM && (v3 || v2l)) && !(T0.act_mode == ACT_F32 && v2l && h.n_tasks == 1)) return false;
   for (int i = 0; i < h.n_tasks; ++i) {
     const GemvTask& T = h.t[i];
@@ -1429,8 +1534,9 @@ static void launch_one(hipStream_t st, const GemvLaunch* dev, const GemvLaunch& 
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
     if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, a0, a1, a2, hn, hm, he, gw, gs);
     else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, a0, a1, a2, hn, hm, he, gw, gs);
-  } else if (QT == DSK_QUANT_Q2_K && R == 1 && (U == 2 || U == 1) && NW == 16 && hn > 0 && (hm == ACT_F32_NORM ? h.ahead & 1 : hm == ACT_F32 ? h.ahead & 2 : 0) && gemv_ahead_ok(h)) {
-    auto k = hm == ACT_F32 ? gemv_ahead_kernel<32, 5, false> : U == 2 ? gemv_ahead_kernel<112, 6> : gemv_ahead_kernel<32, 5>;
+  } else if ((QT == DSK_QUANT_Q2_K || QT == DSK_QUANT_Q3_K) && R == 1 && (U == 2 || U == 1) && NW == 16 && hn > 0 && (hm == ACT_F32_NORM ? h.ahead & 1 : hm == ACT_F32 ? h.ahead & 2 : 0) && gemv_ahead_ok(h)) {
+    constexpr int KT = QT == DSK_QUANT_Q3_K ? QT : DSK_QUANT_Q2_K;
+    auto k = hm == ACT_F32 ? gemv_ahead_kernel<KT, 32, 5, false> : U == 2 ? gemv_ahead_kernel<DSK_QUANT_Q2_K, 112, 6> : gemv_ahead_kernel<KT, 32, 5>;
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
     if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, (const float*)a0, (const float*)a1, he);
     else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, (const float*)a0, (const float*)a1, he);
@@ -1439,6 +1545,15 @@ static void launch_one(hipStream_t st, const GemvLaunch* dev, const GemvLaunch& 
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
     if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, (const int8_t*)a0, (const float*)a1, (const int16_t*)a2);
     else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, (const int8_t*)a0, (const float*)a1, (const int16_t*)a2);
+  } else if ((QT == DSK_QUANT_F8E5M2 || QT == DSK_QUANT_F16) && R == 1 && hn > 0 && gemv_ahead_f_steps(h)) {
+    constexpr int FT = QT == DSK_QUANT_F16 ? QT : DSK_QUANT_F8E5M2;
+    const int its = gemv_ahead_f_steps(h);
+    auto go = [&](auto k) {
+      if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, (const float*)a0, (const float*)a1, he);
+      else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, (const float*)a0, (const float*)a1, he);
+    };
+    if (hm == ACT_F32_NORM) go(its == 1 ? gemv_ahead_f_kernel<FT, 16, 1, true> : its == 2 ? gemv_ahead_f_kernel<FT, 16, 2, true> : gemv_ahead_f_kernel<FT, 16, 4, true>);
+    else go(its == 1 ? gemv_ahead_f_kernel<FT, NW, 1, false> : its == 2 ? gemv_ahead_f_kernel<FT, NW, 2, false> : gemv_ahead_f_kernel<FT, NW, 4, false>);
   } else {
     auto k = gemv_kernel<QT, R, U, false, NW>;
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
@@ -1511,8 +1626,10 @@ bool gemv_kvwrite_supported(const GemvLaunch& h) {
 // projections), 2 gemv_ahead_q8_kernel (wo), 3 gemv_kvwrite_ahead_kernel (the MLA second stage; `kvwrite`: launched with the rider)
 int gemv_ahead_kind(const GemvLaunch& h, bool kvwrite) {
   if (kvwrite) return gemv_kvwrite_supported(h) && gemv_kvwrite_ahead_ok(h) ? 3 : 0;
-  if (h.NW != 16 || h.R != 1 || h.bd_heads != 0 || h.n_groups != 1) return 0;
+  if (h.R != 1 || h.bd_heads != 0 || h.n_groups != 1) return 0;
   const GemvTask& T = h.t[h.grp_t0[0]];
+  if (gemv_ahead_f_steps(h)) return T.act_mode == ACT_F32_NORM ? 1 : 2;
+  if (h.NW != 16) return 0;
   if ((h.ahead & 1) && T.act_mode == ACT_F32_NORM && gemv_ahead_ok(h)) return 1;
   if ((h.ahead & 2) && T.act_mode == ACT_F32 && gemv_ahead_ok(h)) return 1;
   if ((h.ahead & 2) && T.act_mode == ACT_Q8 && gemv_ahead_q8_ok(h)) return 2;
