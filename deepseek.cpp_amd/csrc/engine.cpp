@@ -144,6 +144,7 @@ int ds_get_info(dsk_model* m, const char* key, int* value) {
     }
     *value = n;
   }
+  else if (k == "gemv_stream_plans") *value = (m->lp_head >= 0 && gemv_streams(m->plans[m->lp_head])) + (m->lp_head_host >= 0 && gemv_streams(m->plans[m->lp_head_host]));
   else if (k == "hydrate_tile_copy_mb") *value = (int)(m->hydrate_tile_copy_bytes / 1048576.0);
   else if (k == "fused_moe_layers") { int n = 0; for (auto& a : m->moe_ffn) n += a.grid > 0; *value = n; }
   else if (k == "expert_up_layers") { int n = 0; for (size_t l = 0; l < m->moe_up.size(); ++l) n += m->moe_up[l].grid > 0 && m->moe_ffn[l].grid <= 0; *value = n; }

@@ -496,6 +496,7 @@ int build_plans(dsk_model* m) {
     task_weights(T, cls);
     task_act_norm(T, m->x, m->g[DSK_ROLE_FINAL_NORM], c.norm_eps);
     T.out = m->logits;
+    h.ahead = m->gemv_ahead & 1 ? 4 : 0;  // (gemv_stream_kernel)
     h.algo_bytes = weight_bytes_2d(m, wq, T.rows, T.n) + c.dim * 8.0 + 4.0 * T.rows;
     DSK_TRY(add_plan(m, h, &m->lp_head));
     // a token whose logits only the host reads: stored into its buffer, most of them while the weights still stream (129280 logits: the launch 57 -> 63 us

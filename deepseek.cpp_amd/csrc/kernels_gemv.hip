@@ -612,6 +612,155 @@ __global__ __launch_bounds__(1024) void gemv_ahead_q8_kernel(const GemvLaunch* _
     tl[0] = t_entry; tl[6] = t_staged; tl[7] = tl[1] = t_bar; tl[2] = t_rows; tl[3] = wall_clock64();
   }
 }
+// One plain matrix of many short rows on rmsnorm(x) (the classifier of V2-Lite's widths): the rows of a wave, RG apart, as one stream.  With a row group
+// requested, waited for and multiplied before the next one, 102400 rows of 2048 took 25 us in Q2_K (69 MB), 52 in F8E5M2 (210 MB), 70 in F16 (419 MB); so 22, 40
+// and 68 (17 and 37 with the output in the card's memory).  Q3_K, bound by its unpacking, took 32 either way, and V3's rows of seven steps, whose stream the plain
+// kernel keeps up, 63 -> 70 with their sums through LDS.  Here AHEAD groups (eight of Q2_K: 24.4) are on their way behind x and while it is staged, and a
+// group's registers are requested anew as soon as it is multiplied; rows past the share are out of the descriptors' range: no memory traffic.  The sums of a
+// round leave through LDS, a wave 64 rows: the output may be the host's memory, where a store of a row or two
+// is a bus transaction as well.  ITS column steps of 1 << LL lanes; sums in gemv_body's order, the same bits.
+template <int QT, int LL, int ITS, int AHEAD>
+__global__ __launch_bounds__(1024) void gemv_stream_kernel(const GemvLaunch* __restrict__ Lp, const float* __restrict__ x, const float* __restrict__ norm_w, float eps) {
+  constexpr bool KQ = QT == DSK_QUANT_Q2_K;
+  constexpr int NW = 16, RPW = 64 >> LL, RG = NW * RPW;
+  constexpr int EPI = KQ ? 64 : FTraits<KQ ? DSK_QUANT_F16 : QT>::EPI, n = (ITS << LL) * EPI, nb = n / 256, NQ = n / 4, KX = (NQ + 1023) / 1024;
+  static_assert(KQ ? ITS == 1 : LL == 6, "gemv_stream_kernel: whole column steps");
+  static_assert(KX == 1 && AHEAD * RG <= 1024, "gemv_stream_kernel: x is a quad, a round a row a thread");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ float scratch[16], sums[2][AHEAD * RG];
+  const GemvLaunch& L = *Lp;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, bid = blockIdx.x;
+  const int i = min(tid, NQ - 1);
+  const f32x4 t = reinterpret_cast<const f32x4*>(x)[i], wv = reinterpret_cast<const f32x4*>(norm_w)[i];
+  const GemvTask& T = L.t[0];
+  const int rows = T.rows, nwg = L.grp_wg_end[0], rloc = lane >> LL, sub = lane & ((1 << LL) - 1), q = sub & 3;
+  const int r_lo = (int)((long long)rows * bid / nwg), r_hi = (int)((long long)rows * (bid + 1) / nwg);  // (part_unit is 1)
+  float* const out = glob(T.out);
+  auto whole = [](const void* p, size_t bytes) {  // (readfirstlane returns an int: its sign has no place in an address)
+    const unsigned long long v = (unsigned long long)p;
+    const u32 lo = __builtin_amdgcn_readfirstlane((u32)v), hi = __builtin_amdgcn_readfirstlane((u32)(v >> 32)), records = __builtin_amdgcn_readfirstlane((u32)bytes);
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((unsigned long long)hi << 32) | lo), 0, (int)records, 0x00020000);
+  };
+  struct Group {
+    u32x4 w[ITS];
+    u32 sc, dm;
+    float sv[ITS];
+  };
+  constexpr int NOWHERE = 0x7fff0000;  // (past every descriptor's end: gemv_stream_ok)
+  Group G[AHEAD];
+  int b0 = 1, b1 = 1, s0 = 0, s1 = 0, sc_cols = 0;
+  bool p2 = true, scaled = false;
+  rsrc_t W, SC, DM;
+  if constexpr (KQ) {
+    W = whole(T.qs, (size_t)rows * nb * 64);
+    SC = whole(T.sc, (size_t)rows * nb * 16);
+    DM = whole(T.dm, (size_t)rows * nb * 4);
+  } else {
+    W = whole(T.qs, (size_t)rows * n * FTraits<QT>::ESZ);
+    b0 = L.b0; b1 = L.b1;
+    p2 = ((b0 & (b0 - 1)) | (b1 & (b1 - 1))) == 0;
+    s0 = __builtin_ctz(b0); s1 = __builtin_ctz(b1);
+    sc_cols = p2 ? (n + b1 - 1) >> s1 : (n + b1 - 1) / b1;
+    scaled = T.scale != nullptr;
+    SC = whole(T.scale, scaled ? (size_t)((rows + b0 - 1) / b0) * sc_cols * 4 : 0);
+  }
+  auto row_of = [&](int g) { return r_lo + g * RG + wave * RPW + rloc; };
+  auto request = [&](int g, Group& o) {
+    const int row = row_of(g);
+    const bool in = row < r_hi;
+    if constexpr (KQ) {
+      const int blk = row * nb + (sub >> 2);
+      o.w[0] = __builtin_amdgcn_raw_buffer_load_b128(W, in ? blk * 64 + q * 16 : NOWHERE, 0, BUF_NT);
+      o.sc = __builtin_amdgcn_raw_buffer_load_b32(SC, in ? blk * 16 + q * 4 : NOWHERE, 0, BUF_NT);
+      o.dm = __builtin_amdgcn_raw_buffer_load_b32(DM, in ? blk * 4 : NOWHERE, 0, BUF_NT);
+    } else {
+      const int sc_row = (p2 ? row >> s0 : row / b0) * sc_cols;
+#pragma unroll
+      for (int u = 0; u < ITS; ++u) {
+        const int item = u * 64 + lane;
+        o.w[u] = __builtin_amdgcn_raw_buffer_load_b128(W, in ? (row * (n / EPI) + item) * 16 : NOWHERE, 0, BUF_NT);
+        if (QT == DSK_QUANT_F8E5M2) o.sv[u] = u2f(__builtin_amdgcn_raw_buffer_load_b32(SC, in && scaled ? (sc_row + (p2 ? item * EPI >> s1 : item * EPI / b1)) * 4 : NOWHERE, 0, 0));
+      }
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < AHEAD; ++d) request(d, G[d]);
+  // rmsnorm (src/infer.cpp:601-611), K-quants: + Q8_K, into LDS: stage_q8's and stage_f32's sums, barriers for LDS alone
+  float ss = 0.f;
+  if (tid < NQ) {
+    ss = fmaf(t.x, t.x, ss);
+    ss = fmaf(t.y, t.y, ss);
+    ss = fmaf(t.z, t.z, ss);
+    ss = fmaf(t.w, t.w, ss);
+  }
+  ss = wave_sum(ss);
+  if (lane == 0) scratch[wave] = ss;
+  lds_barrier();
+  const float scale = 1.0f / sqrtf(scratch_total<NW>(scratch) / (float)n + eps);
+  if (tid < NQ) {
+    if constexpr (KQ) {
+      const float v[4] = {t.x * scale * wv.x, t.y * scale * wv.y, t.z * scale * wv.z, t.w * scale * wv.w};
+      q8k_block_lds<LAY_Q2>(v, lane, smem + (size_t)wave * 4 * ITEM_LDS);
+    } else {
+      reinterpret_cast<f32x4*>(smem)[quad_place<EPI>(tid, n / EPI)] = t * scale * wv;
+    }
+  }
+  lds_barrier();
+#ifndef DSK_NO_TAPS
+  if constexpr (KQ) {
+    if (L.tap_qs && bid == 0) dump_staged_q8<LAY_Q2>(smem, n, L.tap_qs, L.tap_d, tid, NW * 64);
+  }
+#endif
+  // the vector's part of a lane stays in registers: every row meets the same one
+  u32x4 a[4], meta;
+  if constexpr (KQ) {
+    const uint8_t* rec = smem + sub * ITEM_LDS;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a[s] = *reinterpret_cast<const u32x4*>(rec + s * 16);
+    meta = *reinterpret_cast<const u32x4*>(rec + 64);
+  }
+  const int groups = (r_hi - r_lo + RG - 1) / RG;
+  int turn = 0;
+  for (int g0 = 0; g0 < groups; g0 += AHEAD, ++turn) {
+    float* const mine = sums[turn & 1];
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) {
+      float acc = 0.f;
+      Group& o = G[d];
+      if constexpr (KQ) acc = q2k_item(o.w[0], o.sc, o.dm, a, meta, acc);
+      else {
+#pragma unroll
+        for (int u = 0; u < ITS; ++u) {
+          float xa[EPI];
+#pragma unroll
+          for (int k = 0; k < EPI / 4; ++k) {
+            const f32x4 v = reinterpret_cast<const f32x4*>(smem)[k * (n / EPI) + u * 64 + lane];  // (quad_place)
+            xa[4 * k] = v.x; xa[4 * k + 1] = v.y; xa[4 * k + 2] = v.z; xa[4 * k + 3] = v.w;
+          }
+          acc = fmaf(fitem<QT>(o.w[u], xa, 0.f), QT == DSK_QUANT_F8E5M2 && scaled ? o.sv[u] : 1.0f, acc);
+        }
+      }
+      request(g0 + d + AHEAD, o);
+      acc = lanes_sum(acc, LL);
+      if (sub == 0) mine[d * RG + wave * RPW + rloc] = acc;
+    }
+    lds_barrier();  // (a wave writes here again behind the next one)
+    const int row = r_lo + g0 * RG + tid;
+    if (tid < AHEAD * RG && row < r_hi) out[row] = mine[tid];
+  }
+}
+// the plans it runs: shares of more than two row groups (a group or less: the kernels above), planes that 31-bit offsets reach
+static bool gemv_stream_ok(const GemvLaunch& h) {
+  if (h.tiled || h.glu || h.R != 1 || h.NW != 16 || h.n_tasks != 1 || h.n_groups != 1 || h.bd_heads != 0 || !(h.ahead & 4) || h.timeline || h.part_unit != 1) return false;
+  if (h.comb_x || h.comb_geometry || h.compact_absent || h.zero_absent || h.grid != h.grp_wg_end[0]) return false;
+  const GemvTask& T = h.t[0];
+  if (T.act_mode != ACT_F32_NORM || T.e_qs != 0 || T.accum_w || T.epilogue != EPI_STORE || T.rows <= 2 * h.grid * (16 * (64 >> h.lpr_log2))) return false;
+  const bool f8 = h.quant == DSK_QUANT_F8E5M2;
+  if (h.quant == DSK_QUANT_Q2_K) return h.lpr_log2 >= 4 && T.n == 64 << h.lpr_log2 && (double)T.rows * T.n / 4 < 0x7fff0000;
+  if (!f8 && h.quant != DSK_QUANT_F16) return false;
+  const int step = f8 ? 1024 : 512;
+  return h.lpr_log2 == 6 && (T.n == step || T.n == 2 * step || (T.n == 4 * step && !f8)) && (double)T.rows * T.n * (f8 ? 1 : 2) < 0x7fff0000;
+}
 static bool gemv_ahead_q8_ok(const GemvLaunch& h) {
   if (h.tiled || h.quant != DSK_QUANT_Q2_K || h.glu || h.R != 1 || h.NW != 16 || h.n_groups != 1 || h.bd_heads != 0 || h.n_tasks != 1) return false;
   if (h.comb_x || h.comb_geometry || h.compact_absent || h.zero_absent || h.tap_qs) return false;
@@ -1534,6 +1683,22 @@ static void launch_one(hipStream_t st, const GemvLaunch* dev, const GemvLaunch& 
     if (h.lds_bytes > 64 * 1024) hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h.lds_bytes);
     if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, a0, a1, a2, hn, hm, he, gw, gs);
     else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, a0, a1, a2, hn, hm, he, gw, gs);
+  } else if (QT != DSK_QUANT_F32 && QT != DSK_QUANT_Q3_K && R == 1 && NW == 16 && hn > 0 && gemv_stream_ok(h)) {
+    constexpr int ST = QT == DSK_QUANT_F32 || QT == DSK_QUANT_Q3_K ? DSK_QUANT_F16 : QT;
+    auto go = [&](auto k) {
+      if (g_prof_start && g_prof_stop) hipExtLaunchKernelGGL(k, grid, block, (uint32_t)h.lds_bytes, st, g_prof_start, g_prof_stop, 0u, dev, (const float*)a0, (const float*)a1, he);
+      else hipLaunchKernelGGL(k, grid, block, h.lds_bytes, st, dev, (const float*)a0, (const float*)a1, he);
+    };
+    if constexpr (ST == DSK_QUANT_Q2_K)
+      go(h.lpr_log2 == 4 ? gemv_stream_kernel<ST, 4, 1, 4> : h.lpr_log2 == 5 ? gemv_stream_kernel<ST, 5, 1, 4> : gemv_stream_kernel<ST, 6, 1, 4>);
+    else {
+      const int its = hn / (64 * FTraits<ST>::EPI);
+      if (its == 4) {
+        if constexpr (ST == DSK_QUANT_F16) go(gemv_stream_kernel<ST, 6, 4, 4>);
+      } else {
+        go(its == 1 ? gemv_stream_kernel<ST, 6, 1, 8> : gemv_stream_kernel<ST, 6, 2, 4>);
+      }
+    }
   } else if ((QT == DSK_QUANT_Q2_K || QT == DSK_QUANT_Q3_K) && R == 1 && (U == 2 || U == 1) && NW == 16 && hn > 0 && (hm == ACT_F32_NORM ? h.ahead & 1 : hm == ACT_F32 ? h.ahead & 2 : 0) && gemv_ahead_ok(h)) {
     constexpr int KT = QT == DSK_QUANT_Q3_K ? QT : DSK_QUANT_Q2_K;
     auto k = hm == ACT_F32 ? gemv_ahead_kernel<KT, 32, 5, false> : U == 2 ? gemv_ahead_kernel<DSK_QUANT_Q2_K, 112, 6> : gemv_ahead_kernel<KT, 32, 5>;
@@ -1635,6 +1800,7 @@ int gemv_ahead_kind(const GemvLaunch& h, bool kvwrite) {
   if ((h.ahead & 2) && T.act_mode == ACT_Q8 && gemv_ahead_q8_ok(h)) return 2;
   return 0;
 }
+bool gemv_streams(const GemvLaunch& h) { return gemv_stream_ok(h); }
 int launch_gemv_kvwrite(hipStream_t st, const GemvLaunch* dev, const GemvLaunch& h, const MlaKvArgs& kv, const StepParams* sp) {
   if (!gemv_kvwrite_supported(h)) DSK_FAIL(DSK_ERR_INVALID, "gemv_kvwrite: unsupported plan");
   if (kv.rope > 128 || (kv.rope & 1)) DSK_FAIL(DSK_ERR_UNSUPPORTED, "rope dim %d (max 128, even)", kv.rope);

@@ -229,7 +229,7 @@ int dsk_model_set_option(dsk_model* m, const char* key, int value);
  * that hit it was re-run transparently), "fused_moe_layers", "graph_captured", "exchange_calls" (RCCL collectives this
  * model has enqueued eagerly), "tiled_tensors" (weight tensors held as tile records, option "q2k_tiles"),
  * "hydrate_batched_tokens" / "hydrate_looped_tokens", "hydrate_tile_copy_mb" (MiB of tile copies the batched prompt path holds),
- * "gemv_ahead_plans", "expert_up_layers" / "expert_down_layers" (MoE blocks that run those launches, option "expert_launches"),
+ * "gemv_ahead_plans", "gemv_stream_plans" (of the classifier's two plans), "expert_up_layers" / "expert_down_layers" (MoE blocks that run those launches, option "expert_launches"),
  * "head_short_layers". */
 int dsk_model_get_info(dsk_model* m, const char* key, int* value);
 /* models created on the context and not yet destroyed (a context destroyed while models are alive is freed by the last

@@ -40,3 +40,26 @@ def test_weights_ahead_same_bits(ctx, quant, over):
             assert np.array_equal(A.get_cache_rows(layer, name, 0, 4, width), B.get_cache_rows(layer, name, 0, 4, width))
     A.close()
     B.close()
+
+
+# classifiers as a stream of row groups: shares that are no whole rounds nor row groups, rows of 16, 32 and 64 lanes (K-quants) and of 1, 2 and 4 steps (floats),
+# scales' blocks of no power of two
+STREAMS = [("q2_k", 2048, 102400), ("q2_k", 1024, 40001), ("q2_k", 4096, 9001), ("f8e5m2", 2048, 102400), ("f8e5m2", 1024, 8193), ("f8e5m2", 2048, 10007),
+           ("fp16", 2048, 10007), ("fp16", 512, 33333), ("fp16", 1024, 8200)]
+
+
+@pytest.mark.parametrize("quant,dim,vocab", STREAMS)
+def test_classifier_stream_same_bits(ctx, quant, dim, vocab):
+    import dsk
+    c = synth.preset("v2lite", quant, False, n_layers=2, max_seq_len=64, hidden_dim=512, vocab_size=vocab, dim=dim, n_heads=8)
+    if vocab == 10007 and quant == "f8e5m2":
+        c.block_size = (48, 80)
+    A, B = (dsk.Model(ctx, c, None, synth_seed=31, options={"gemv_ahead": on}) for on in (0, 3))
+    assert [m.info("gemv_stream_plans") for m in (A, B)] == [0, 2]
+    for pos, t in enumerate((3, 500, 17)):
+        la, lb = A.forward(t, pos), B.forward(t, pos)
+        assert np.all(np.isfinite(la)) and np.array_equal(la, lb), pos
+    x = np.random.default_rng(1).standard_normal(c.dim).astype(np.float32)
+    assert np.array_equal(A.run_head(x), B.run_head(x))
+    A.close()
+    B.close()
