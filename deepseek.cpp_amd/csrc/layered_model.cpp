@@ -118,7 +118,7 @@ struct LayeredModel : ModelHead {
   char *cq = nullptr, *lq = nullptr, *lat = nullptr, *kv = nullptr, *qabs = nullptr;
   int mixes = 1, lq_ld = 0, cq_ld = 0, kv_ld = 0, max_window = 0, key_cap = 0;  // mixes: blends of h; key_cap: rows of the key workspace
   float *weight = nullptr, *logits = nullptr, *trace_x = nullptr, *sample_scratch = nullptr;
-  int *slot_pos = nullptr, *chosen = nullptr, *count = nullptr, *cursor = nullptr, *slot_row = nullptr, *tiles = nullptr, *n_tiles = nullptr, *active = nullptr,
+  int *slot_pos = nullptr, *chosen = nullptr, *count = nullptr, *slot_row = nullptr, *tiles = nullptr, *n_tiles = nullptr, *active = nullptr,
       *active_slot = nullptr, *n_active = nullptr, *next_dev = nullptr;
   float* logits_host = nullptr;     // pinned, LOGIT_ROWS rows, the upper half of them for borrowers
   RowPool* pool = nullptr;          // owns them
@@ -664,8 +664,7 @@ int alloc_work(LayeredModel* m) {
     DSK_TRY(dev_alloc_n(m, &m->slot_pos, ns));
     DSK_TRY(dev_alloc_n(m, &m->chosen, ns));
     DSK_TRY(dev_alloc_n(m, &m->slot_row, ns));
-    DSK_TRY(dev_alloc_n(m, &m->count, experts));
-    DSK_TRY(dev_alloc_n(m, &m->cursor, experts));
+    DSK_TRY(dev_alloc_n(m, &m->count, (n + 15) / 16 * experts));
     DSK_TRY(dev_alloc_n(m, &m->tiles, 4 * (size_t)m->max_tiles));
     DSK_TRY(dev_alloc_n(m, &m->n_tiles, 1));
     DSK_TRY(dev_alloc_n(m, &m->active, experts + 1));
@@ -906,7 +905,6 @@ MoeArgs moe_args(LayeredModel* m, const PassDesc& p, const LayerSpec& l, const L
   a.slot_pos = m->slot_pos;
   a.chosen = m->chosen;
   a.count = m->count;
-  a.cursor = m->cursor;
   a.slot_row = m->slot_row;
   a.tiles = m->tiles;
   a.n_tiles = m->n_tiles;

@@ -7,43 +7,52 @@
 #include <math.h>
 
 enum { ROUTE_EPL = 8, ROUTE_MAX_EXPERTS = 64 * ROUTE_EPL };
-// one wave chooses the `top` largest of a row's logits (lowest index first among equals) and the softmax over them; lane k holds
-// choice k for k < top (top <= 64)
+// floats in an order that whole numbers have (0: none; no number and both zeros as one float each), and back
+DEV unsigned order_of(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v + 0.f);
+  return v != v ? 1u : u >> 31 ? ~u : u | 0x80000000u;
+}
+DEV float of_order(unsigned o) { return __builtin_bit_cast(float, o >> 31 ? o ^ 0x80000000u : ~o); }
+DEV unsigned wave_max(unsigned v) {
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));   // quad_perm [1, 0, 3, 2]
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));   // quad_perm [2, 3, 0, 1]
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));  // row_half_mirror
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));  // row_mirror
+  v = max(v, lane_xor(v, 16));
+  v = max(v, lane_xor(v, 32));
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
+// One wave chooses the `top` largest of a row's logits (lowest index first among equals) and the softmax over them; lane k holds
+// choice k for k < top (top <= 64).  All lanes are on.  A choice is the largest value of the wave and the first lane that has it: with value and index
+// exchanged together, six rounds of a dozen instructions each, the chain was four times as long (route_count_kernel).
 DEV void choose(const float* z, int experts, int top, int lane, int* e_out, float* w_out) {
-  float v[ROUTE_EPL];
+  unsigned v[ROUTE_EPL];
 #pragma unroll
   for (int i = 0; i < ROUTE_EPL; ++i) {
     const int e = lane + 64 * i;
-    v[i] = e < experts ? z[e] : -INFINITY;
+    v[i] = e < experts ? order_of(z[e]) : 0u;
   }
   int mine = 0;
   float zm = -INFINITY, first = 0.f;
-  unsigned taken = 0;
   for (int k = 0; k < top; ++k) {
-    float best = -INFINITY;
-    int be = 0x7fffffff;
+    unsigned best = v[0];
+#pragma unroll
+    for (int i = 1; i < ROUTE_EPL; ++i) best = max(best, v[i]);
+    best = wave_max(best);
+    int be = -1;
 #pragma unroll
     for (int i = 0; i < ROUTE_EPL; ++i) {
-      const int e = lane + 64 * i;
-      if (e < experts && !((taken >> i) & 1) && (v[i] > best || be == 0x7fffffff)) {
-        best = v[i];
-        be = e;
+      const unsigned long long has = __ballot(v[i] == best);
+      if (be < 0 && has) {
+        be = 64 * i + __ffsll(has) - 1;
+        if (be == 64 * i + lane) v[i] = 0u;
       }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      const float ob = lane_xor(best, off);
-      const int oe = lane_xor(be, off);
-      if (oe != 0x7fffffff && (be == 0x7fffffff || ob > best || (ob == best && oe < be))) {
-        best = ob;
-        be = oe;
-      }
-    }
-    if ((be & 63) == lane) taken |= 1u << (be >> 6);
-    if (k == 0) first = best;
+    const float value = of_order(best);
+    if (k == 0) first = value;
     if (lane == k) {
       mine = be;
-      zm = best;
+      zm = value;
     }
   }
   const float ex = lane < top ? expf(zm - first) : 0.f;
