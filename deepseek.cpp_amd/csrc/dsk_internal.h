@@ -568,7 +568,6 @@ struct HydGemmArgs {
   int out_stride;
   int epilogue, act;      // EPI_STORE / EPI_ADD (ignored for GLU pairs); DSK_ACT_*
   const unsigned* a_dig;  // optional: the sub-block sums as digit words (launch_hyd_digits): the quads' min term then rides the matrix pipe
-  int halve_from = 0;     // 0, or (the launcher's) 1 + the first pair of 32 tokens and a strip group that goes out as two workgroups
 };
 int launch_hyd_gemm(hipStream_t st, const HydGemmArgs& A, int nq);
 int launch_hyd_digits(hipStream_t st, const int16_t* bsums, unsigned* dig, size_t count);

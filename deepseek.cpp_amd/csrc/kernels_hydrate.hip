@@ -666,14 +666,8 @@ __global__ __launch_bounds__(64 * NW, 2) void hyd_gemm16_kernel(const HydGemmArg
   constexpr int SG = GLU ? NW / 2 : NW;  // strips per workgroup
   const int strips = (A.rows + 15) >> 4;
   const int groups = (strips + SG - 1) / SG;
-  int task = 0, group = (int)blockIdx.x, base = (int)blockIdx.y * 16 * MT, part = -1;
-  if (A.n_experts > 0) { task = group / groups; group -= task * groups; }
-  if (MT == 2 && A.halve_from > 0) {  // plain matrices: (chunk, strip group) pairs in one sequence, those from halve_from - 1 on as two workgroups each
-    const int b = (int)blockIdx.x, full = A.halve_from - 1, pair = b < full ? b : full + ((b - full) >> 1);
-    base = pair / groups * 32;
-    group = pair - pair / groups * groups;
-    if (b >= full) { part = (b - full) & 1; base += part * 16; }
-  }
+  const int task = A.n_experts > 0 ? (int)blockIdx.x / groups : 0;
+  const int group = (int)blockIdx.x - task * groups;
   const int cnt = A.count ? __builtin_amdgcn_readfirstlane(A.count[task]) : A.m;
   if (cnt <= 0 || cnt < A.cnt_min || (A.cnt_max > 0 && cnt > A.cnt_max)) return;
   const int* list = A.list ? A.list + (size_t)task * A.list_stride : nullptr;
@@ -685,11 +679,31 @@ __global__ __launch_bounds__(64 * NW, 2) void hyd_gemm16_kernel(const HydGemmArg
   const rsrc_t RA = make_rsrc_n(A.a_qs, (u32)((size_t)A.a_rows * n));
   const rsrc_t RB = make_rsrc_n(A.a_bsums, (u32)((size_t)A.a_rows * (n >> 4) * 2));
   const rsrc_t RD = make_rsrc_n(A.a_d, (u32)((size_t)A.a_rows * nb * 4));
-  for (; base < cnt; base += (int)gridDim.y * 16 * MT) {
-    if (MT > 1 && part < 0 && cnt - base > 16) hyd16_pass<GLU, SEG4, NW, MT>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
+  for (int base = (int)blockIdx.y * 16 * MT; base < cnt; base += (int)gridDim.y * 16 * MT) {
+    if (MT > 1 && cnt - base > 16) hyd16_pass<GLU, SEG4, NW, MT>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
     else hyd16_pass<GLU, SEG4, NW, 1>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
-    if (MT == 2 && A.halve_from > 0) break;
   }
+}
+// One plain matrix by 32 tokens and a group of 8 waves' strips a workgroup, (chunk, group) pairs in one sequence, those from `full` on as two workgroups of 16
+// tokens each.  (A kernel of its own: with its cases in the one above the experts' launches, thousands of workgroups most of which find no rows, took 3 - 10 %
+// longer, 13 tokens of five blocks 1985 -> 2025 us.)
+template <bool GLU, bool SEG4>
+__global__ __launch_bounds__(512, 2) void hyd_gemm16_halves_kernel(const HydGemmArgs A, const int full) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // 2 x hyd16_stage_b
+  constexpr int NW = 8, SG = GLU ? NW / 2 : NW;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int strips = (A.rows + 15) >> 4, groups = (strips + SG - 1) / SG, b = (int)blockIdx.x;
+  const int pair = b < full ? b : full + ((b - full) >> 1), base = pair / groups * 32 + (b < full ? 0 : ((b - full) & 1) * 16), group = pair % groups;
+  if (base >= A.m) return;
+  const int strip = group * SG + (GLU ? wave >> 1 : wave);
+  const bool live = strip < strips;
+  const int n = A.n, nb = n >> 8;
+  const rsrc_t W = make_rsrc((GLU && (wave & 1) ? A.W3 : A.W) + (size_t)(live ? strip : 0) * nb * TILE_B);
+  const rsrc_t RA = make_rsrc_n(A.a_qs, (u32)((size_t)A.a_rows * n));
+  const rsrc_t RB = make_rsrc_n(A.a_bsums, (u32)((size_t)A.a_rows * (n >> 4) * 2));
+  const rsrc_t RD = make_rsrc_n(A.a_d, (u32)((size_t)A.a_rows * nb * 4));
+  if (b < full && A.m - base > 16) hyd16_pass<GLU, SEG4, NW, 2>(A, W, RA, RB, RD, nullptr, base, A.m, live, strip, lds);
+  else hyd16_pass<GLU, SEG4, NW, 1>(A, W, RA, RB, RD, nullptr, base, A.m, live, strip, lds);
 }
 
 // Long rows, few strips (the first-stage projections: 96 + 36 strips of 28 blocks; the shared expert's w1 / w3): a strip's row is a
@@ -835,10 +849,9 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
     auto groups = [&](int nw) { return (unsigned)((units * per + nw - 1) / nw); };
     if (A.m > 16 && (long long)groups(8) * chunks > HYD_CUS) {
       const long long pairs = (long long)groups(8) * chunks2, left = pairs % HYD_CUS;
-      if (left > 0 && left <= HYD_CUS / 2 && pairs + left < (1ll << 30)) {
-        HydGemmArgs B = A;
-        B.halve_from = (int)(pairs - left) + 1;
-        hyd_gemm16_launch<GLU, 8, 2>(st, dim3((unsigned)(pairs + left)), B);
+      if (!A.count && left > 0 && left <= HYD_CUS / 2 && pairs + left < (1ll << 30)) {
+        auto k = A.n > 8 * 256 ? hyd_gemm16_halves_kernel<GLU, true> : hyd_gemm16_halves_kernel<GLU, false>;
+        hipLaunchKernelGGL(k, dim3((unsigned)(pairs + left)), dim3(512), 2 * hyd16_stage_b<2>(), st, A, (int)(pairs - left));
       } else {
         hyd_gemm16_launch<GLU, 8, 2>(st, dim3(groups(8), (unsigned)chunks2), A);
       }
