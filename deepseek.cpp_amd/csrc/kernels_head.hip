@@ -10,6 +10,7 @@
 // Bound by latency: 16 workgroups.  V2-Lite at 62 positions, us: Q2_K 13.2 -> 6.9, F8E5M2 12.8 -> 9.1 (its 131 KB of rows are 2.7 us for the one compute unit); a token 1130 -> 985, 1602 -> 1505.
 #include "dsk_internal.h"
 #include "gemv_device.h"
+#include "head_rows.h"
 
 namespace {
 
@@ -17,8 +18,7 @@ namespace {
 struct HeadShape { int H, h, hd, vd, nope, rope, is_v3; uint16_t *kcache, *vcache; int kv_pos, kv_len; };
 
 // Keys and values on their way: 16 lanes a position, positions 4 wave .. + 3 of every 64; thread (g, i4) the values of positions g, g + TG, ...  Buffer loads: one
-// lane offset each for keys and values, the steps in scalar registers, and zeros without traffic behind the context's end (the range check of a
-// raw buffer counts the scalar offset).
+// lane offset each for keys and values, a step's distance added to it, and zeros without traffic behind the context's end (head_rows.h).
 template <int VN>
 struct HeadKV {
   rsrc_t KB, VB;
@@ -30,11 +30,10 @@ template <int VN>
 DEV void head_keys(const HeadShape& S, HeadKV<VN>& R, int t0) {
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    if (t0 + u * 64 >= S.kv_len) break;
-    const int step = (t0 + u * 64) * (int)R.krow;
-    R.k[u][0] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)R.koff, step, 0));
-    R.k[u][1] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)R.koff + 128, step, 0));
-    R.k[u][2] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)R.koff + 256, step, 0));
+    if (!head_step_there(t0 + u * HEAD_KEY_STEP, S.kv_len)) break;
+    const u32 at = R.koff + (u32)(t0 + u * HEAD_KEY_STEP) * R.krow;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) R.k[u][j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.KB, (int)(at + 128 * j), 0, 0));
   }
 }
 template <int VN>
@@ -42,17 +41,21 @@ DEV void head_places(const HeadShape& S, HeadKV<VN>& R, int tid, int wave, int l
   const int tpp = S.vd >> 2;
   R.grp = lane >> 4; R.sl = lane & 15;
   R.TG = 1024 / tpp; R.g = tid / tpp; R.i4 = tid - R.g * tpp;
-  R.krow = (u32)S.H * S.hd * 2; R.vrow = (u32)S.H * S.vd * 2;
+  R.krow = head_row_bytes(S.H, S.hd); R.vrow = head_row_bytes(S.H, S.vd);
   R.KB = __builtin_amdgcn_make_buffer_rsrc(S.kcache, 0, (int)(S.kv_len * R.krow), 0x00020000);
   R.VB = __builtin_amdgcn_make_buffer_rsrc(S.vcache, 0, (int)(S.kv_len * R.vrow), 0x00020000);
-  R.koff = ((u32)(wave * 4 + R.grp) * S.H + S.h) * S.hd * 2 + R.sl * 8;
-  R.voff = R.g < R.TG ? ((u32)R.g * S.H + S.h) * S.vd * 2 + R.i4 * 8 : 0xfffffff0u;
+  R.koff = head_key_at(wave * 4 + R.grp, R.sl, S.H, S.h, S.hd);
+  R.voff = head_value_at(R.g, R.i4, R.TG, S.H, S.h, S.vd);
+}
+// values of the group's position g + first, where any group has one
+template <int VN>
+DEV void head_value(const HeadShape& S, const HeadKV<VN>& R, int first, ad::f16x4& v) {
+  if (head_step_there(first, S.kv_len)) v = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.VB, (int)(R.voff + (u32)first * R.vrow), 0, 0));
 }
 template <int VN>
 DEV void head_values(const HeadShape& S, HeadKV<VN>& R) {
 #pragma unroll
-  for (int j = 0; j < VN; ++j)
-    if (j * R.TG < S.kv_len) R.v[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.VB, (int)R.voff, j * R.TG * (int)R.vrow, 0));
+  for (int j = 0; j < VN; ++j) head_value(S, R, j * R.TG, R.v[j]);
 }
 // rotation of the sink keys by one position, in f16 (src/infer.cpp:1008-1020), in front of the keys' requests
 DEV void head_sinks(const HeadShape& S, const StepParams* sp, int kv_sink, int tid) {
@@ -163,13 +166,13 @@ DEV float head_attend(const HeadShape& S, HeadKV<VN>& R, const float (&qv)[3][4]
 #pragma unroll
     for (int j = 0; j < VN; ++j)
       if (g + j * TG < kv_len) mix(g + j * TG, R.v[j]);
-    for (int t0 = g + VN * TG; t0 - g < kv_len; t0 += 4 * TG) {
+    for (int first = VN * TG; first < kv_len; first += 4 * TG) {  // (uniform)
       ad::f16x4 y[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = __builtin_bit_cast(ad::f16x4, __builtin_amdgcn_raw_buffer_load_b64(R.VB, (int)R.voff, (t0 - g + j * TG) * (int)R.vrow, 0));
+      for (int j = 0; j < 4; ++j) head_value(S, R, first + j * TG, y[j]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (t0 + j * TG < kv_len) mix(t0 + j * TG, y[j]);
+        if (g + first + j * TG < kv_len) mix(g + first + j * TG, y[j]);
     }
     *reinterpret_cast<f32x4*>(part + (size_t)g * vd + i4 * 4) = f32x4{acc[0], acc[1], acc[2], acc[3]};
   }
@@ -519,7 +522,7 @@ __global__ __launch_bounds__(1024) void head_attn_latent_kernel(const StepParams
 bool head_latent_supported(const HeadAttnArgs& A, int max_kv) {
   return A.quant == DSK_QUANT_Q2_K && A.has_q && !A.tiled && A.lq_log2 == 3 && A.lkv_log2 == 3 && A.tq.n == 1536 && A.tkv.n == 512 && A.a.head_dim == 192 && A.a.nope == 128 &&
          A.a.rope == 64 && A.a.v_dim == 128 && A.a.lora == 512 && A.tq.act_mode == ACT_F32_NORM && A.tkv.act_mode == ACT_F32_NORM &&
-         (double)max_kv * A.a.n_heads * 192 * 2 < 2147483648.0;
+         head_rows_fit(max_kv, A.a.n_heads, 192, 128);
 }
 int launch_head_latent(hipStream_t st, const HeadAttnArgs& A, const StepParams* sp, int max_kv) {
   const size_t lds = (size_t)max_kv * 4;
@@ -535,7 +538,7 @@ int head_short_plan(HeadShortArgs& S, const HeadAttnArgs& A, int max_kv) {
   const bool kq = A.quant == DSK_QUANT_Q2_K || A.quant == DSK_QUANT_Q3_K;
   const int epi = kq ? 64 : A.quant == DSK_QUANT_F16 ? 8 : 16, n = A.tkv.n, nope = A.a.nope, vd = A.a.v_dim, rope = A.a.rope, hd = A.a.head_dim;
   S.grid = 0;
-  if ((double)max_kv * A.a.n_heads * (hd > vd ? hd : vd) * 2 >= 2147483648.0) return DSK_OK;  // (32-bit offsets into a cache)
+  if (!head_rows_fit(max_kv, A.a.n_heads, hd, vd)) return DSK_OK;
   if (A.has_q || A.tiled || A.quant == DSK_QUANT_F32 || A.tkv.act_mode != ACT_F32_NORM) return DSK_OK;
   // rows of one column step, at most 16 row sets of the workgroup (floats: two rounds of 8; K-quants: one of 2); the norm one piece a thread, in the first 8 waves
   const int lpr = 1 << A.lkv_log2, sets = (nope + vd + 16 * (64 / lpr) - 1) / (16 * (64 / lpr));
