@@ -228,7 +228,10 @@ int launch_conv(hipStream_t st, const PassDesc& p, int width, const float* h_f, 
 // workgroup adds those up (offsets of the experts' ranges, and where its own rows' slots lie in them) and places its slots, and the tiles' table is made by all
 // of them.  With counters in memory (a workgroup's counts added to them, a launch of one workgroup for the offsets, ranges taken from cursors) it was three
 // launches, 11.0 + 4.7 + 4.8 us for 2048 rows and 64 experts, 8.7 + 4.6 + 4.6 for 40; two: 6.6 + 5.0 and 6.1 + 4.8.
-enum { ROUTE_ROWS = 16 };
+// Every workgroup adding up all the others' counts is work by the square of the rows, so past ROUTE_SQUARE numbers read a launch between the two makes running sums of
+// the counts and the second reads two of them an expert (route_sums_kernel).  Second launch alone, us: 4096 rows and 256 experts, at the line, 8.2; 8192 rows
+// 19.0, with the sums 5.0 + 5.0; 16384 rows 61.7 and 5.5 + 6.3, of 64 experts 20.0 and 5.1 + 6.1.
+enum { ROUTE_ROWS = 16, ROUTE_SQUARE = 1 << 24 };
 __global__ __launch_bounds__(1024) void route_count_kernel(const MoeArgs a) {  // a wave per row, one histogram
   __shared__ int hist[ROUTE_MAX_EXPERTS];
   const int tid = threadIdx.x, lane = tid & 63, ns = a.top + a.shared;
@@ -248,6 +251,37 @@ __global__ __launch_bounds__(1024) void route_count_kernel(const MoeArgs a) {  /
   lds_barrier();
   for (int i = tid; i < a.experts; i += 1024) a.count[(size_t)blockIdx.x * a.experts + i] = hist[i];
 }
+// Running sums over the workgroups' counts, in place, the sums over all in a row behind them: 16 experts to a workgroup, 64 runs of its rows.
+__global__ __launch_bounds__(1024) void route_sums_kernel(int* count, int experts, int groups) {
+  __shared__ int part[16][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = tid & 15, run = tid >> 4, e = blockIdx.x * 16 + col;
+  const int per = (groups + 63) / 64, g0 = min(run * per, groups), g1 = e < experts ? min(g0 + per, groups) : g0;
+  int* const c = count + min(e, experts - 1);
+  int sum = 0;
+#pragma unroll 8
+  for (int g = g0; g < g1; ++g) sum += c[(size_t)g * experts];
+  int before = sum;  // inclusive over the wave's four runs, then over the waves
+  for (int d = 16; d < 64; d <<= 1) {
+    const int o = __shfl_up(before, d);
+    before += lane >= d ? o : 0;
+  }
+  if (lane >= 48) part[wave][col] = before;
+  before -= sum;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) before += part[w][col];
+  if (run == 63 && e < experts) c[(size_t)groups * experts] = before + sum;
+  for (int at = g0; at < g1; at += 8) {
+    int v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = c[(size_t)min(at + i, g1 - 1) * experts];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (at + i < g1) c[(size_t)(at + i) * experts] = before;
+      before += v[i];
+    }
+  }
+}
+template <bool SUMMED>
 __global__ __launch_bounds__(1024) void route_sort_kernel(const MoeArgs a) {
   __shared__ int total[1024], before[1024], base[ROUTE_MAX_EXPERTS], n[ROUTE_MAX_EXPERTS], wave_off[ROUTE_MAX_EXPERTS / 64], wave_til[ROUTE_MAX_EXPERTS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ns = a.top + a.shared, me = blockIdx.x, groups = gridDim.x;
@@ -256,7 +290,7 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const MoeArgs a) {
   const int mine = in && k < a.top ? a.chosen[(size_t)row * a.top + k] : -1;
   const int shift = a.experts <= 64 ? 6 : a.experts <= 128 ? 7 : a.experts <= 256 ? 8 : 9, per = 1024 >> shift, e = tid & ((1 << shift) - 1);
   int sum = 0, sum_before = 0;
-  if (e < a.experts) {
+  if (!SUMMED && e < a.experts) {
     const int* c = a.count + e;
 #pragma unroll 8
     for (int g = tid >> shift; g < groups; g += per) {
@@ -265,19 +299,25 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const MoeArgs a) {
       sum_before += g < me ? v : 0;
     }
   }
-  total[tid] = sum;
-  before[tid] = sum_before;
+  if (!SUMMED) {
+    total[tid] = sum;
+    before[tid] = sum_before;
+  }
   if (tid < ROUTE_MAX_EXPERTS) n[tid] = 0;
   __syncthreads();
   // experts' counts, and inclusive sums of counts and tiles: a thread an expert, within a wave and over the waves
   int count = 0, off = 0, til = 0;
   if (tid < ROUTE_MAX_EXPERTS) {
     int own_before = 0;
-    if (tid < a.experts)
+    if (SUMMED && tid < a.experts) {
+      count = a.count[(size_t)groups * a.experts + tid];
+      own_before = a.count[(size_t)me * a.experts + tid];
+    } else if (tid < a.experts) {
       for (int g = 0; g < per; ++g) {
         count += total[(g << shift) + tid];
         own_before += before[(g << shift) + tid];
       }
+    }
     off = count;
     til = (count + MOE_TILE - 1) / MOE_TILE;
 #pragma unroll
@@ -340,7 +380,12 @@ int launch_route(hipStream_t st, const MoeArgs& a) {
   DSK_TRY(check_route(a));
   const dim3 grid((a.rows + ROUTE_ROWS - 1) / ROUTE_ROWS);
   hipLaunchKernelGGL(route_count_kernel, grid, dim3(1024), 0, st, a);
-  hipLaunchKernelGGL(route_sort_kernel, grid, dim3(1024), 0, st, a);
+  if ((long long)grid.x * grid.x * a.experts > ROUTE_SQUARE) {
+    hipLaunchKernelGGL(route_sums_kernel, dim3((a.experts + 15) / 16), dim3(1024), 0, st, a.count, a.experts, (int)grid.x);
+    hipLaunchKernelGGL(route_sort_kernel<true>, grid, dim3(1024), 0, st, a);
+  } else {
+    hipLaunchKernelGGL(route_sort_kernel<false>, grid, dim3(1024), 0, st, a);
+  }
   return DSK_OK;
 }
 int launch_route_few(hipStream_t st, const MoeArgs& a) {

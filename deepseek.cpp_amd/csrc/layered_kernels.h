@@ -97,7 +97,7 @@ struct MoeArgs {
   int* slot_pos;            // [rows][top + shared]: where the slot's hidden / output row is
   int* chosen;              // [rows][top]
   // many rows: slots sorted by expert
-  int* count;               // [rows / 16, rounded up][experts]: by how many of 16 rows each was chosen
+  int* count;               // [rows / 16, rounded up, + 1][experts]: by how many of 16 rows each was chosen; the last row: by all (launch_route)
   int* slot_row;            // [rows * (top + shared)]: the row a sorted slot belongs to
   int* tiles;               // [max_tiles][4]: expert (experts = the shared one), first slot, slots, -
   int* n_tiles;

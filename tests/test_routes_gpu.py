@@ -25,3 +25,13 @@ def test_equal_logits_go_to_the_lowest_index(case, kind):
                     if kind != "all equal":
                         W[k][::3] = -0.0
     case(U.config([U.channel_delta(mlp=U.moe(70, 5))], width=64), edit=edit).check_trace(37, cuts=([20],))
+
+
+# passes whose counts are summed by a launch of their own (workgroups of 16 rows, squared, times experts > 2^24): around that line, several of 64 runs empty, whole and
+# broken ones, experts that are no whole workgroups of 16
+@pytest.mark.parametrize("experts,top,shared,n", [(512, 2, 0, 2896), (512, 2, 0, 2897), (509, 3, 72, 3001), (130, 5, 0, 5900), (256, 8, 72, 8192)])
+def test_long_passes(case, experts, top, shared, n):
+    mixer = U.delta(heads=1, kv_heads=1, dim=16, vdim=16)
+    m = case(U.config([U.channel_delta(mixer, mlp=U.moe(experts, top, ff=16, shared=shared))], width=64), options="piece_tokens=8192")
+    assert m.lm.info("piece_tokens") == 8192
+    m.check_trace(n)
