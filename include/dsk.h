@@ -222,7 +222,7 @@ int dsk_model_destroy(dsk_model* m);
  *   "hydrate_tap_layer" -1  parity harness: copy block l's stages of every batched chunk aside for dsk_hydrate_get_buffer
  *   "gemv_ahead"      3  bits: 1 the first-stage projection launch (and the MLA second stage), 2 wo request their first weights
  *                        behind the loads of their vector and AHEAD of its staging (kernels_gemv.hip gemv_ahead_kernel & co;
- *                        bit-identical to 0; Q2_K, Q3_K: instantiated for the DeepSeek-V3 (Q2_K) and V2-Lite row lengths;
+ *                        bit-identical to 0; Q2_K, Q3_K: instantiated for the DeepSeek-V3 (Q2_K) and V2-Lite row lengths, Q3_K's wo for none;
  *                        F8E5M2, F16: rows of 1, 2 or 4 steps of a wave; other shapes run the plain kernel); get_info "gemv_ahead_plans" counts the launch plans that run such a kernel */
 int dsk_model_set_option(dsk_model* m, const char* key, int value);
 /* Read-only counters: "handoff_fallbacks" (times a hand-off give-up moved the model to the two-launch form; the token
