@@ -21,6 +21,7 @@
 // integer the decode lane converts to float, and lane (n, t) of the result holds all four groups of ITS (token, row):
 // the float stage - dx * d, the min term, the per-item partials, the final (S0 + S1) + (S2 + S3) - is lane-local.
 #include "dsk_internal.h"
+#include "hyd_rounds.h"
 #include "tile_device.h"
 #include <algorithm>
 #include <type_traits>
@@ -684,25 +685,24 @@ __global__ __launch_bounds__(64 * NW, 2) void hyd_gemm16_kernel(const HydGemmArg
     else hyd16_pass<GLU, SEG4, NW, 1>(A, W, RA, RB, RD, list, base, cnt, live, strip, lds);
   }
 }
-// One plain matrix by 32 tokens and a group of 8 waves' strips a workgroup, (chunk, group) pairs in one sequence, those from `full` on as two workgroups of 16
-// tokens each.  (A kernel of its own: with its cases in the one above the experts' launches, thousands of workgroups most of which find no rows, took 3 - 10 %
+// One plain matrix by 32 tokens and a group of 8 waves' strips a workgroup, (chunk, group) pairs in one sequence, the last ones as two workgroups of 16
+// tokens each (hyd_rounds.h).  (A kernel of its own: with its cases in the one above the experts' launches, thousands of workgroups most of which find no rows, took 3 - 10 %
 // longer, 13 tokens of five blocks 1985 -> 2025 us.)
 template <bool GLU, bool SEG4>
-__global__ __launch_bounds__(512, 2) void hyd_gemm16_halves_kernel(const HydGemmArgs A, const int full) {
+__global__ __launch_bounds__(512, 2) void hyd_gemm16_halves_kernel(const HydGemmArgs A, const HydRounds rounds) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // 2 x hyd16_stage_b
   constexpr int NW = 8, SG = GLU ? NW / 2 : NW;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int strips = (A.rows + 15) >> 4, groups = (strips + SG - 1) / SG, b = (int)blockIdx.x;
-  const int pair = b < full ? b : full + ((b - full) >> 1), base = pair / groups * 32 + (b < full ? 0 : ((b - full) & 1) * 16), group = pair % groups;
-  if (base >= A.m) return;
-  const int strip = group * SG + (GLU ? wave >> 1 : wave);
+  const int strips = (A.rows + 15) >> 4, groups = (strips + SG - 1) / SG;
+  const HydRound r = hyd_round(rounds, groups, (int)blockIdx.x);  // (base < m: hyd_rounds_grid)
+  const int base = r.base, strip = r.group * SG + (GLU ? wave >> 1 : wave);
   const bool live = strip < strips;
   const int n = A.n, nb = n >> 8;
   const rsrc_t W = make_rsrc((GLU && (wave & 1) ? A.W3 : A.W) + (size_t)(live ? strip : 0) * nb * TILE_B);
   const rsrc_t RA = make_rsrc_n(A.a_qs, (u32)((size_t)A.a_rows * n));
   const rsrc_t RB = make_rsrc_n(A.a_bsums, (u32)((size_t)A.a_rows * (n >> 4) * 2));
   const rsrc_t RD = make_rsrc_n(A.a_d, (u32)((size_t)A.a_rows * nb * 4));
-  if (b < full && A.m - base > 16) hyd16_pass<GLU, SEG4, NW, 2>(A, W, RA, RB, RD, nullptr, base, A.m, live, strip, lds);
+  if (!r.half && A.m - base > 16) hyd16_pass<GLU, SEG4, NW, 2>(A, W, RA, RB, RD, nullptr, base, A.m, live, strip, lds);
   else hyd16_pass<GLU, SEG4, NW, 1>(A, W, RA, RB, RD, nullptr, base, A.m, live, strip, lds);
 }
 
@@ -848,10 +848,10 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
     const int per = GLU ? 2 : 1, chunks2 = (A.m + 31) / 32;
     auto groups = [&](int nw) { return (unsigned)((units * per + nw - 1) / nw); };
     if (A.m > 16 && (long long)groups(8) * chunks > HYD_CUS) {
-      const long long pairs = (long long)groups(8) * chunks2, left = pairs % HYD_CUS;
-      if (!A.count && left > 0 && left <= HYD_CUS / 2 && pairs + left < (1ll << 30)) {
+      const HydRounds R = hyd_rounds((long long)groups(8) * chunks2, HYD_CUS);
+      if (!A.count && R.left > 0) {
         auto k = A.n > 8 * 256 ? hyd_gemm16_halves_kernel<GLU, true> : hyd_gemm16_halves_kernel<GLU, false>;
-        hipLaunchKernelGGL(k, dim3((unsigned)(pairs + left)), dim3(512), 2 * hyd16_stage_b<2>(), st, A, (int)(pairs - left));
+        hipLaunchKernelGGL(k, dim3((unsigned)hyd_rounds_grid(R, (int)groups(8), A.m)), dim3(512), 2 * hyd16_stage_b<2>(), st, A, R);
       } else {
         hyd_gemm16_launch<GLU, 8, 2>(st, dim3(groups(8), (unsigned)chunks2), A);
       }
