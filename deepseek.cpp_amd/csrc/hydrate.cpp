@@ -266,7 +266,7 @@ static int hyd_gemm(dsk_model* m, const DTensor& w, const DTensor* w3, const Hyd
   A.m = P; A.out = out; A.out_stride = out_stride; A.epilogue = epilogue; A.act = m->c.act;
   // plain matrices: 8 tokens per wave and pass (168 / 236 VGPRs: 3 / 2 waves per SIMD; 16 tokens need 260 / 366 and leave one),
   // the four waves of a workgroup on consecutive chunks of the same strip
-  return launch_hyd_gemm(m->ctx->stream, A, P <= 4 ? 1 : 2);
+  return launch_hyd_gemm(m->ctx->stream, A, P <= 4 ? 1 : 2, m->ctx->n_cus);
 }
 
 // n_short: the chunk's first tokens whose context is below the MLA matrix-core regime (all of them for MHA)
@@ -314,7 +314,7 @@ static int hyd_layer(dsk_model* m, int l, int P, int max_kv, int n_short) {
       A.a_qs = h.a_lat.qs; A.a_d = h.a_lat.d; A.a_bsums = h.a_lat.bsums; A.a_rows = P * H; A.a_div = 1;
       A.list = h.head_list; A.count = h.head_count; A.list_stride = h.cap;
       A.out = h.att; A.out_stride = vd; A.epilogue = EPI_STORE; A.act = c.act;
-      DSK_TRY(launch_hyd_gemm(st, A, P <= 4 ? 1 : 2));
+      DSK_TRY(launch_hyd_gemm(st, A, P <= 4 ? 1 : 2, m->ctx->n_cus));
     }
     DSK_TRY(hyd_tap_q8(m, l, "q_a", h.a_qa, P, qlr));
     DSK_TRY(hyd_tap(m, l, "q_rope", h.q_rope, P, (size_t)H * rope * 4));
@@ -393,7 +393,7 @@ static int hyd_layer(dsk_model* m, int l, int P, int max_kv, int n_short) {
     A.a_dig = h.a_x.dig;
     A.list = h.list; A.count = h.count; A.list_stride = h.cap;
     A.out = h.hb; A.out_stride = mi; A.act = c.act;
-    DSK_TRY(launch_hyd_gemm(st, A, 1));
+    DSK_TRY(launch_hyd_gemm(st, A, 1, m->ctx->n_cus));
   }
   DSK_TRY(launch_quantize_q8k(st, h.hb, P * K * mi, h.a_hb.qs, h.a_hb.d, h.a_hb.bsums));
   DSK_TRY(launch_hyd_digits(st, h.a_hb.bsums, h.a_hb.dig, (size_t)P * K * (mi / 16)));
@@ -405,7 +405,7 @@ static int hyd_layer(dsk_model* m, int l, int P, int max_kv, int n_short) {
     A.a_dig = h.a_hb.dig;
     A.list = h.list; A.count = h.count; A.list_stride = h.cap;
     A.out = h.eout; A.out_stride = dim; A.epilogue = EPI_STORE; A.act = c.act;
-    DSK_TRY(launch_hyd_gemm(st, A, 1));
+    DSK_TRY(launch_hyd_gemm(st, A, 1, m->ctx->n_cus));
   }
   DSK_TRY(launch_hyd_combine(st, h.X, h.eout, h.route_w, shn > 0 ? h.eout_sh : nullptr, P, K, dim));
   if (l == m->hydrate_tap_layer) {

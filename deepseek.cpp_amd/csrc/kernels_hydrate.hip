@@ -812,9 +812,8 @@ static void hyd_gemm16_launch(hipStream_t st, dim3 grid, const HydGemmArgs& A) {
   if (A.n > 8 * 256) hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, true, NW, MT>), grid, dim3(64 * NW), 2 * hyd16_stage_b<MT>(), st, A);
   else hipLaunchKernelGGL((hyd_gemm16_kernel<GLU, false, NW, MT>), grid, dim3(64 * NW), 2 * hyd16_stage_b<MT>(), st, A);
 }
-enum { HYD_CUS = 256 };
 template <bool GLU, int NQ>
-static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
+static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A, int n_cus) {
   const long long units = (long long)(A.n_experts > 0 ? A.n_experts : 1) * ((A.rows + 15) >> 4);
   // expert stacks: the tasks with HYD16_EXPERT_MIN rows or more go through the 16-token form (their rows share the expanded tile 16 at
   // a time instead of 4), the others stay with the quads below
@@ -847,8 +846,8 @@ static void hyd_gemm_launch(hipStream_t st, const HydGemmArgs& A) {
     // half the CUs goes out as workgroups of 16 tokens, all CUs for 3 / 4 of a round (the same at 512 tokens, 896 workgroups: 268 -> 254).
     const int per = GLU ? 2 : 1, chunks2 = (A.m + 31) / 32;
     auto groups = [&](int nw) { return (unsigned)((units * per + nw - 1) / nw); };
-    if (A.m > 16 && (long long)groups(8) * chunks > HYD_CUS) {
-      const HydRounds R = hyd_rounds((long long)groups(8) * chunks2, HYD_CUS);
+    if (A.m > 16 && (long long)groups(8) * chunks > n_cus) {
+      const HydRounds R = hyd_rounds((long long)groups(8) * chunks2, n_cus);
       if (!A.count && R.left > 0) {
         auto k = A.n > 8 * 256 ? hyd_gemm16_halves_kernel<GLU, true> : hyd_gemm16_halves_kernel<GLU, false>;
         hipLaunchKernelGGL(k, dim3((unsigned)hyd_rounds_grid(R, (int)groups(8), A.m)), dim3(512), 2 * hyd16_stage_b<2>(), st, A, R);
@@ -889,13 +888,13 @@ int launch_hyd_digits(hipStream_t st, const int16_t* bsums, unsigned* dig, size_
   hipLaunchKernelGGL(hyd_digits_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, bsums, dig, count);
   return DSK_OK;
 }
-int launch_hyd_gemm(hipStream_t st, const HydGemmArgs& A, int nq) {
+int launch_hyd_gemm(hipStream_t st, const HydGemmArgs& A, int nq, int n_cus) {
   if (A.n % 256 || A.rows < 1 || A.a_rows < 1 || A.a_div < 1) DSK_FAIL(DSK_ERR_INVALID, "hyd_gemm: bad shape");
   if ((size_t)A.a_rows * A.n >= (size_t)HYD_OOB) DSK_FAIL(DSK_ERR_UNSUPPORTED, "hyd_gemm: activation array too large for 30-bit offsets");
   const bool glu = A.W3 != nullptr;
   // (16 tokens per wave and pass - NQ 4 - needs 260 / 366 registers with the pipeline's double buffers: not built)
-  if (nq >= 2) { if (glu) hyd_gemm_launch<true, 2>(st, A); else hyd_gemm_launch<false, 2>(st, A); }
-  else { if (glu) hyd_gemm_launch<true, 1>(st, A); else hyd_gemm_launch<false, 1>(st, A); }
+  if (nq >= 2) { if (glu) hyd_gemm_launch<true, 2>(st, A, n_cus); else hyd_gemm_launch<false, 2>(st, A, n_cus); }
+  else { if (glu) hyd_gemm_launch<true, 1>(st, A, n_cus); else hyd_gemm_launch<false, 1>(st, A, n_cus); }
   return DSK_OK;
 }
 
