@@ -75,7 +75,7 @@ extern "C" int dsk_model_create(dsk_ctx* ctx, const dsk_config* cfg, dsk_model**
   if (getenv("DSK_NO_FUSE_SHARED")) m->ride_shared = false;
   if (getenv("DSK_NO_KVWRITE_RIDE")) m->ride_kvwrite = false;
   if (getenv("DSK_NO_COMPACT")) m->compact_absent = false;
-  m->att_q8_in_wo = env_i("DSK_ATT_Q8_IN_WO", 0) != 0;
+  m->att_q8_in_wo = env_i("DSK_ATT_Q8_IN_WO", -1);
   m->rider_fill = env_i("DSK_RIDER_FILL", m->rider_fill);
   m->mla_flash_min_kv = std::max(32, env_i("DSK_MLA_FLASH_MIN", m->mla_flash_min_kv));
   m->mha_split_min = env_i("DSK_MHA_SPLIT_MIN", 0);
@@ -99,7 +99,7 @@ extern "C" int dsk_model_set_option(dsk_model* m, const char* key, int value) {
   if (k == "fuse_moe") m->fuse_moe = value != 0;
   else if (k == "fuse_shared") m->ride_shared = value != 0;
   else if (k == "ride_kvwrite") m->ride_kvwrite = value != 0;
-  else if (k == "att_q8_in_wo") m->att_q8_in_wo = value != 0;
+  else if (k == "att_q8_in_wo") m->att_q8_in_wo = value;
   else if (k == "compact_absent") m->compact_absent = value != 0;
   else if (k == "rider_fill") { if (value < 1 || value > 16) DSK_FAIL(DSK_ERR_INVALID, "set_option: rider_fill %d", value); m->rider_fill = value; }
   else if (k == "mla_flash_min") m->mla_flash_min_kv = std::max(32, value);
@@ -149,6 +149,7 @@ int ds_get_info(dsk_model* m, const char* key, int* value) {
   else if (k == "fused_moe_layers") { int n = 0; for (auto& a : m->moe_ffn) n += a.grid > 0; *value = n; }
   else if (k == "expert_up_layers") { int n = 0; for (size_t l = 0; l < m->moe_up.size(); ++l) n += m->moe_up[l].grid > 0 && m->moe_ffn[l].grid <= 0; *value = n; }
   else if (k == "expert_down_layers") { int n = 0; for (size_t l = 0; l < m->moe_down.size(); ++l) n += m->moe_down[l].grid > 0 && m->moe_ffn[l].grid <= 0; *value = n; }
+  else if (k == "att_q8_in_wo") *value = is_kq(m->c.weight_quant) && m->wo_quantises;
   else if (k == "head_short_layers") { int n = 0; for (auto& a : m->head_short) n += a.grid > 0; for (char b : m->head_latent) n += b; *value = n; }
   else if (k == "graph_captured") { int n = 0; for (auto g : m->graph) n += g != nullptr; *value = n; }
   else if (k == "exchange_calls") *value = m->exchange_calls;

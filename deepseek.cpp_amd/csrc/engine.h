@@ -96,7 +96,8 @@ struct dsk_model : ModelHead {
   std::vector<MoeFfnArgs> moe_ffn;
   std::vector<MoeUpArgs> moe_up;      // grid == 0: the router launch with the gate, the generic launch lp_w13
   std::vector<MoeDownArgs> moe_down;  // grid == 0: the layer's second half is the generic launch lp_w2
-  bool att_q8_in_wo = false;       // DSK_ATT_Q8_IN_WO=1: wo quantises the attention output in its own prologue (no finisher hand-off in the attention launch)
+  int att_q8_in_wo = -1;           // DSK_ATT_Q8_IN_WO=1: wo quantises the attention output in its own prologue (no finisher hand-off in the attention launch); -1: by size
+  bool wo_quantises = false;       // what became of it (build_plans)
   bool fuse_moe = true;            // DSK_NO_FUSE_MOE at model creation switches it off (A/B, bit-identity tests)
   unsigned* moe_ctr = nullptr;     // slot_ctr[16] | slot_pass[16]
   unsigned* moe_blk_ctr = nullptr; // per-block arrivals of the fused expert launch (hidden vectors quantised by their producers)

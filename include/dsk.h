@@ -185,8 +185,9 @@ int dsk_model_destroy(dsk_model* m);
  *   "fuse_moe"        1  routed experts of a MoE block in one launch (0: two launches; bit-identical)
  *   "fuse_shared"     1  the shared expert's w1/w3 rides in the router launch (0: ninth task of the experts' launch)
  *   "ride_kvwrite"    1  MLA: the latent cache write rides in the second-stage projection launch
- *   "att_q8_in_wo"    0  wo quantises the attention output in its own prologue (no finisher in the attention launch); always so where
- *                        "head_short" applies to K-quants
+ *   "att_q8_in_wo"   -1  1: wo quantises the attention output in its own prologue (no finisher in the attention launch); 0: it never does, and
+ *                        "head_short" does not apply to K-quants without a query latent; -1: with "head_short", in K-quant MHA models
+ *                        without a query latent and of up to 4096 attention outputs (bit-identical)
  *   "head_short"      1  MHA without a query latent, and DeepSeek-V3's heads in Q2_K: everything of a head that does not depend on anything
  *                        requested at once (0: the general per-head launch; bit-identical)
  *   "compact_absent"  1  expert-sharded w1/w3 launch compacts its row space over the experts present on the rank
@@ -230,7 +231,7 @@ int dsk_model_set_option(dsk_model* m, const char* key, int value);
  * model has enqueued eagerly), "tiled_tensors" (weight tensors held as tile records, option "q2k_tiles"),
  * "hydrate_batched_tokens" / "hydrate_looped_tokens", "hydrate_tile_copy_mb" (MiB of tile copies the batched prompt path holds),
  * "gemv_ahead_plans", "gemv_stream_plans" (of the classifier's two plans), "expert_up_layers" / "expert_down_layers" (MoE blocks that run those launches, option "expert_launches"),
- * "head_short_layers". */
+ * "head_short_layers", "att_q8_in_wo" (1: a K-quant model's wo quantises). */
 int dsk_model_get_info(dsk_model* m, const char* key, int* value);
 /* models created on the context and not yet destroyed (a context destroyed while models are alive is freed by the last
  * dsk_model_destroy) */

@@ -15,10 +15,13 @@ def cache_rows(c, n, seed):
     return {"k_cache": f16(n, H * hd), "v_cache": f16(n, H * c.v_head_dim)}
 
 
-def same(ctx, c, positions, T=None, seed=3, short=True, **options):
+def same(ctx, c, positions, T=None, seed=3, short=True, in_wo=None, **options):
     import dsk
     A, B = (dsk.Model(ctx, c, T, synth_seed=None if T is not None else seed, options=dict(options, head_short=on)) for on in (1, 0))
     assert [m.info("head_short_layers") for m in (A, B)] == [c.n_layers if short else 0, 0]
+    if in_wo is None:  # (without a query latent: all of these have up to 16 blocks of output)
+        in_wo = int(c.quant in ("q2_k", "q3_k") and not c.q_lora_rank)
+    assert [m.info("att_q8_in_wo") for m in (A, B)] == [in_wo, options.get("att_q8_in_wo", 0) if c.quant in ("q2_k", "q3_k") else 0]
     n = min(c.max_seq_len, c.rs_original_max_position_embeddings)
     for l in range(c.n_layers):
         for name, rows in cache_rows(c, n, 10 + l).items():
@@ -84,7 +87,19 @@ def test_heads_behind_a_query_latent_past_the_ring(ctx):
     same(ctx, c, [79, 80, 81, 130, 200])
 
 
+@pytest.mark.parametrize("quant", ["fp16", "q2_k", "q3_k"])
 @pytest.mark.parametrize("over", [dict(qk_nope_head_dim=192, qk_rope_head_dim=64), dict(q_lora_rank=256)], ids=["heads of 256", "query latent"])
-def test_heads_of_other_forms_keep_the_general_kernel(ctx, over):
-    c = synth.preset("tiny_v2lite", "fp16", False, **over)
+def test_heads_of_other_forms_keep_the_general_kernel(ctx, quant, over):
+    c = synth.preset("tiny_v2lite", quant, False, **over)
     same(ctx, c, [0, 3, 40], T=synth.synth_model(c, seed=5), short=False)
+
+
+@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+def test_who_quantises_the_output(ctx, quant):
+    """the caller's word holds: never in wo, which heads that leave 32 bits then do not come in front of; always; by size, which 17 blocks are too large for"""
+    c = synth.preset("tiny_v2lite", quant, False)
+    T = synth.synth_model(c, seed=5)
+    same(ctx, c, [0, 3, 40], T=T, short=False, in_wo=0, att_q8_in_wo=0)
+    same(ctx, c, [0, 3, 40], T=T, in_wo=1, att_q8_in_wo=1)
+    c = synth.preset("tiny_v2lite", quant, False, n_heads=34, v_head_dim=128)
+    same(ctx, c, [0, 3, 40], T=synth.synth_model(c, seed=5), short=False, in_wo=0)
