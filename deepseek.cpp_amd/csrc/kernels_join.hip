@@ -231,7 +231,8 @@ int launch_conv(hipStream_t st, const PassDesc& p, int width, const float* h_f, 
 // Every workgroup adding up all the others' counts is work by the square of the rows, so past ROUTE_SQUARE numbers read a launch between the two makes running sums of
 // the counts and the second reads two of them an expert (route_sums_kernel).  Second launch alone, us: 4096 rows and 256 experts, at the line, 8.2; 8192 rows
 // 19.0, with the sums 5.0 + 5.0; 16384 rows 61.7 and 5.5 + 6.3, of 64 experts 20.0 and 5.1 + 6.1.
-enum { ROUTE_ROWS = 16, ROUTE_SQUARE = 1 << 24 };
+enum { ROUTE_SQUARE = 1 << 24 };
+static_assert(ROUTE_ROWS * 64 == 1024, "a wave a row, and a thread for each of its slots (check_route: at most 64)");
 __global__ __launch_bounds__(1024) void route_count_kernel(const MoeArgs a) {  // a wave per row, one histogram
   __shared__ int hist[ROUTE_MAX_EXPERTS];
   const int tid = threadIdx.x, lane = tid & 63, ns = a.top + a.shared;

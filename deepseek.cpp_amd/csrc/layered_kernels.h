@@ -89,6 +89,7 @@ struct ExpertMat {          // one of the two matrices of a set of experts
   size_t stride;
   int kt, rt, shared_kt, shared_rt;
 };
+enum { ROUTE_ROWS = 16 };  // rows of a workgroup of launch_route
 struct MoeArgs {
   int rows, width_ld, experts, top, shared;  // shared: 0 or 1 extra slot per row
   const float* logits;      // router logits [rows][ld_logits]
@@ -97,7 +98,7 @@ struct MoeArgs {
   int* slot_pos;            // [rows][top + shared]: where the slot's hidden / output row is
   int* chosen;              // [rows][top]
   // many rows: slots sorted by expert
-  int* count;               // [rows / 16, rounded up, + 1][experts]: by how many of 16 rows each was chosen; the last row: by all (launch_route)
+  int* count;               // [rows / ROUTE_ROWS, rounded up, + 1][experts]: by how many of so many rows each was chosen; the last row: by all (launch_route)
   int* slot_row;            // [rows * (top + shared)]: the row a sorted slot belongs to
   int* tiles;               // [max_tiles][4]: expert (experts = the shared one), first slot, slots, -
   int* n_tiles;

@@ -664,7 +664,7 @@ int alloc_work(LayeredModel* m) {
     DSK_TRY(dev_alloc_n(m, &m->slot_pos, ns));
     DSK_TRY(dev_alloc_n(m, &m->chosen, ns));
     DSK_TRY(dev_alloc_n(m, &m->slot_row, ns));
-    DSK_TRY(dev_alloc_n(m, &m->count, ((n + 15) / 16 + 1) * experts));
+    DSK_TRY(dev_alloc_n(m, &m->count, ((n + ROUTE_ROWS - 1) / ROUTE_ROWS + 1) * experts));
     DSK_TRY(dev_alloc_n(m, &m->tiles, 4 * (size_t)m->max_tiles));
     DSK_TRY(dev_alloc_n(m, &m->n_tiles, 1));
     DSK_TRY(dev_alloc_n(m, &m->active, experts + 1));
