@@ -1,11 +1,12 @@
 // kernels_experts.hip -- the routed experts of one token in launches of their own, for models whose launches are bound by latency and not by
-// bytes (one GPU, K-quant planes; V2-Lite's shapes): rows of x owned by workgroups in the second half.
+// bytes (one GPU, K-quant planes, F8E5M2 and F16; V2-Lite's shapes): the gate inside the first half, rows of x owned by workgroups in the second.
 //
 // Replaces, for the selected experts e_0..e_{K-1} of a token (src/infer.cpp:853-878, 899-903), the launches of the generic multi-task GEMV:
 //     router rows' scores, rmsnorm(x) left behind                             router_scores_kernel
 //     moe_gate, h_k = act(W1[e_k] xb) * (W3[e_k] xb), the shared expert's too  experts_up_kernel
 //     o_k  = W2[e_k] h_k,  x += w_k * o_k  (k order),  x += shared_out        experts_down_kernel
-// Nothing is handed over inside a launch.  Lanes per row, column steps, trees of lanes and the order of the combine are the generic launches': the same bits.
+// Nothing is handed over inside a launch.  Lanes per row, column steps, trees of lanes and the order of the combine are the generic launches', with
+// float weights the one launch's (kernels_moe.hip moe_ffn_f_kernel): the same bits.
 #include "dsk_internal.h"
 #include "gemv_device.h"
 

@@ -182,7 +182,8 @@ int dsk_model_destroy(dsk_model* m);
  * shapes or diagnostics is an explicit option of ONE model: the library never reads the environment (a stray variable
  * in the host application's environment must not change kernels or numerics; only -DDSK_AB builds, made by
  * tools/ab_build.sh for measurements, seed these options from DSK_* variables).  Keys (int values):
- *   "fuse_moe"        1  routed experts of a MoE block in one launch (0: two launches; bit-identical)
+ *   "fuse_moe"        1  routed experts of a MoE block in one launch (0: two launches; bit-identical); F8E5M2 / F16 blocks of get_info
+ *                        "expert_up_layers" ("expert_launches") do not ask for it
  *   "fuse_shared"     1  the shared expert's w1/w3 rides in the router launch (0: ninth task of the experts' launch)
  *   "ride_kvwrite"    1  MLA: the latent cache write rides in the second-stage projection launch
  *   "att_q8_in_wo"   -1  1: wo quantises the attention output in its own prologue (no finisher in the attention launch); 0: it never does, and
@@ -198,9 +199,11 @@ int dsk_model_destroy(dsk_model* m);
  *                        expert launch, read what the following launches open with (descriptors, norm weights, the gate's
  *                        bias row) into the XCDs' L2 (0: off; results unaffected)
  *   "moe_q8_handoff"  1  fused expert launch: hidden vectors handed over as Q8_K, quantised once by their producers
- *   "fuse_moe_float"  1  fused expert launch for F8E5M2 / F16 / F32 weights too (0: two launches; bit-identical)
- *   "expert_launches" 1  experts (K-quant planes that do not run as one launch, F8E5M2, F16): the gate inside the first half, the second half by workgroups that own
- *                        rows of x for every slot (0: the router with the gate and one launch or the generic ones; bit-identical)
+ *   "fuse_moe_float"  1  fused expert launch for F8E5M2 / F16 / F32 weights too, likewise (0: two launches; bit-identical where these stage their
+ *                        vector with 16 waves as well, else the norm's sum of squares has another order)
+ *   "expert_launches" 1  experts of one GPU (K-quant planes that do not run as one launch, F8E5M2, F16): the gate inside the first half (up to 64 experts
+ *                        without groups), the second half by workgroups that own rows of x for every slot.  0: the router with the gate and one launch
+ *                        or the generic ones; bit-identical to these for K-quants, to the one launch for F8E5M2 / F16
  *   "timeline"        0  in-kernel wall-clock stamps for dsk_model_get_timeline
  *   "moe_spin_limit"  0  polls before the fused expert launch's hand-off wait gives up (0: 2^20); < 0: fault
  *                        injection (a give-up is reported although the hand-off succeeded: exercises the fallback)
@@ -221,7 +224,8 @@ int dsk_model_destroy(dsk_model* m);
  *   "hydrate_tile_copies" 1  at "q2k_tiles" = 1 the first batched dsk_hydrate call may copy the plane-layout matrices it multiplies
  *                        into tile records (0: no copies - such a model then runs the loop)
  *   "hydrate_tap_layer" -1  parity harness: copy block l's stages of every batched chunk aside for dsk_hydrate_get_buffer
- *   "gemv_ahead"      3  bits: 1 the first-stage projection launch (and the MLA second stage), 2 wo request their first weights
+ *   "gemv_ahead"      3  bits: 1 the first-stage projection launch (and the MLA second stage, and classifiers of up to 4096 columns as a stream of
+ *                        row groups: gemv_stream_kernel), 2 wo request their first weights
  *                        behind the loads of their vector and AHEAD of its staging (kernels_gemv.hip gemv_ahead_kernel & co;
  *                        bit-identical to 0; Q2_K, Q3_K: instantiated for the DeepSeek-V3 (Q2_K) and V2-Lite row lengths, Q3_K's wo for none;
  *                        F8E5M2, F16: rows of 1, 2 or 4 steps of a wave; other shapes run the plain kernel); get_info "gemv_ahead_plans" counts the launch plans that run such a kernel */
