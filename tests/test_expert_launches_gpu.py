@@ -78,6 +78,18 @@ def test_gate_inside_the_first_half_same_bits(ctx, quant, over):
     same(ctx, c, seed=9, tokens=(5, 400, 3), up=True)
 
 
+# more steps of a workgroup than its twelve waves have on their way at once (two each): 30 and 36 of two rows, 55 of one row
+MANY = [dict(n_routed_experts=12, n_active_routed=10, moe_intermediate_size=1280), dict(n_routed_experts=12, n_active_routed=10),
+        dict(dim=4096, n_routed_experts=9, n_active_routed=9, moe_intermediate_size=1280)]
+
+
+@pytest.mark.parametrize("quant", ["q2_k", "q3_k"])
+@pytest.mark.parametrize("over", MANY, ids=["30 steps", "36 steps", "55 steps"])
+def test_more_steps_than_waves_request_same_bits(ctx, quant, over):
+    c = synth.preset("v2lite", quant, False, **dict(dict(n_layers=2, hidden_dim=512, vocab_size=512, max_seq_len=64), **over))
+    same(ctx, c, seed=21, tokens=(5, 400, 3), up=True)
+
+
 def test_float_rows_of_fewer_steps_same_bits(ctx):
     """F8E5M2 and F16 over two MoE blocks whose hidden rows end inside a group of lanes and whose block scales change within a row"""
     for quant, over in (("f8e5m2", dict(moe_intermediate_size=176, n_shared_experts=2)), ("fp16", dict(moe_intermediate_size=104, n_shared_experts=1))):
