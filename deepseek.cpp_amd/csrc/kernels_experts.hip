@@ -132,7 +132,7 @@ DEV int div_small(int v, int m) { return (v * m) >> 16; }
 // The router's rows (src/infer.cpp:839, 847): workgroup = 2 rows x 8 column slices, slices added in order like router_gate_kernel's.  The gate is the next
 // launch's, so nothing is published, counted or waited for here; and a wave's weights do not wait for the norm's scale: everything is requested at
 // entry.  Workgroup b leaves block b of rmsnorm(x) behind, as Q8_K or in 32 bits.  64 experts of 2048 columns: 7.5 us with the gate in the last workgroup to
-// arrive, 4.9 here.
+// arrive, 3.9 here; in F8E5M2 models, whose x is left in 32 bits, 7.2 and 4.8 (medians over a token's launches, here and below).
 // ------------------------------------------------------------------------------------------------------------
 template <int NL>  // 256-column pieces of a slice
 __global__ __launch_bounds__(1024) void router_scores_kernel(const float* __restrict__ x, const float* __restrict__ norm_w, const float* __restrict__ w, float* __restrict__ scores,
@@ -205,7 +205,7 @@ DEV void decide(const float* scores, const float* bias_p, int lane, int bid, int
 // ------------------------------------------------------------------------------------------------------------
 // First half: every workgroup decides the gate for itself out of the scores (one wave, ~0.5 us: less than handing a decision over), while other waves stage the
 // normed vector; then its share of the shared expert's and of the chosen experts' rows, all of a wave's requested at once.  Bound by latency (16.5 MB: 2.5
-// us): V2-Lite's shapes in Q2_K 9.4 us by the generic launch, whose waves took two rounds, 7.3 here; with the router's launch a token 1303 -> 1130 us.
+// us): V2-Lite's shapes in Q2_K 9.4 us by the generic launch, whose waves took two rounds, 8.1 - 8.4 here; with the router's launch a token 1303 -> 1130 us.
 // ------------------------------------------------------------------------------------------------------------
 template <int QT>
 __global__ __launch_bounds__(1024) void experts_up_kernel(const float* __restrict__ scores, const int8_t* __restrict__ a_qs, const float* __restrict__ a_d,
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(1024) void experts_up_kernel(const float* __restric
 
 // ------------------------------------------------------------------------------------------------------------
 // The same for F8E5M2 and F16 weights: a row is ITS steps of a whole wave (moe_ffn_f_kernel's lanes and order), its values' factors stay in registers for all rows of
-// a wave, and the next two rows are on their way while one is multiplied.  V2-Lite's shapes in F8E5M2: 46 MB in 12.4 us, a pure stream of that size taking 9.6 (16
+// a wave, and the next two rows are on their way while one is multiplied.  V2-Lite's shapes in F8E5M2: 46 MB in 12.4 - 13.2 us, a pure stream of that size taking 9.6 (16
 // waves that multiply instead of 12, or the shared expert's rows requested before the gate: the same).
 // ------------------------------------------------------------------------------------------------------------
 template <int QT, int ITS>
@@ -380,8 +380,8 @@ __global__ __launch_bounds__(1024) void experts_up_f_kernel(const float* __restr
 // generic launch deals (slot, rows) to its workgroups and needs a publish, an arrival, an acquire and a read before the last one can add up).  What a
 // workgroup needs of it is a chain: the experts' ids, the weights, the multiplies.  Its first waves do that; the others meanwhile read and
 // quantise the slots' hidden vectors (12288 values for V2-Lite), so that neither waits for the other's loads.  Bound by latency: 8.3 MB of weights
-// are 1.2 us.  V2-Lite (6 of 64 experts of 1536, shared 3072, Q2_K), us a launch: generic 13.2 (224 workgroups of 4 waves, two rows per lane and the
-// hand-over), here 7.4; with the arguments read where they are used, two copies of the quantisation and a stack of descriptors 9.6.  A token
+// are 1.2 us.  V2-Lite (6 of 64 experts of 1536, shared 3072, Q2_K), us a launch: generic 13.0 (224 workgroups of 4 waves, two rows per lane and the
+// hand-over), here 7.5; with the arguments read where they are used, two copies of the quantisation and a stack of descriptors 9.6.  A token
 // 1460 -> 1303 us.
 // ------------------------------------------------------------------------------------------------------------
 template <int QT>
@@ -480,8 +480,8 @@ __global__ __launch_bounds__(1024) void experts_down_kernel(const float* __restr
 
 // ------------------------------------------------------------------------------------------------------------
 // The same for F8E5M2 and F16 weights (lanes, order and combine of moe_ffn_f_kernel): nothing to quantise, so all waves copy the hidden vectors, between the
-// request of their first weights and their use.  V2-Lite's shapes in F8E5M2: 23 MB in 8.4 us.  Router, first and second half were 7.0 + 23.3 us with both halves in one
-// launch, 4.7 + 12.4 + 8.4 here: the hand-over inside it cost more than a launch; a token 1505 -> 1351 us.
+// request of their first weights and their use.  V2-Lite's shapes in F8E5M2: 23 MB in 8.5 us.  Router, first and second half were 7.2 + 23.6 us with both halves in one
+// launch, 4.8 + 12.4 + 8.5 here: the hand-over inside it cost more than a launch; a token 1505 -> 1341 us.
 // ------------------------------------------------------------------------------------------------------------
 template <int QT>
 __global__ __launch_bounds__(1024) void experts_down_f_kernel(const float* __restrict__ hb, const int* __restrict__ route_e, const float* __restrict__ route_w, float* x,

@@ -7,7 +7,7 @@
 // key and value go from LDS into the scores and the mix, rounded as the cache rounds them, and to the cache at the very end; barriers are for LDS
 // only.  Values, sums and their orders are head_attn_kernel's: the same bits.  Without a query latent the output leaves in 32 bits and wo quantises it (8 blocks for
 // V2-Lite: cheaper in each of its workgroups than a hand-over between heads here).
-// Bound by latency: 16 workgroups.  V2-Lite at 62 positions, us: Q2_K 13.2 -> 6.9, F8E5M2 12.8 -> 9.1 (its 131 KB of rows are 2.7 us for the one compute unit); a token 1130 -> 985, 1602 -> 1505.
+// Bound by latency: 16 workgroups.  V2-Lite, medians over a token's launches, us: Q2_K at 62 positions 13.4 -> 7.4, F8E5M2 at 25 12.6 -> 9.3 (its 131 KB of rows are 2.7 us for the one compute unit); a token 1130 -> 985, 1602 -> 1505.
 #include "dsk_internal.h"
 #include "gemv_device.h"
 #include "head_rows.h"
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(1024) void head_attn_short_kernel(const StepParams*
 // The same behind a query latent, for DeepSeek-V3's heads in Q2_K (192 rows of 1536, 256 of 512, 8 lanes a row): the two latents normed and quantised in one pass, then
 // wkv_b's and wq_b's rows as in head_attn_kernel, whose order and bits these are.  A compute unit returns loads in order and holds ~50 KB of them: the first rows
 // are requested at entry, the next behind the latents, keys and values behind those and under the multiplies.  The output is quantised here, by the last of
-// a block's heads (64 blocks: dearer in each of wo's workgroups).  128 heads, us a launch: at 20 positions 16.5 -> 12.3, at 200 19.8 -> 14.9; five of V3's blocks 487 -> 465 a
+// a block's heads (64 blocks: dearer in each of wo's workgroups).  128 heads, us a launch: at 20 positions 16.5 -> 12.3, at 200 20.2 -> 14.8; five of V3's blocks 487 -> 465 a
 // token.
 // ------------------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void head_attn_latent_kernel(const StepParams* __restrict__ sp, const float* __restrict__ q_a, const float* __restrict__ kv_a,
