@@ -1,5 +1,5 @@
-"""The experts' launches of latency-bound models (kernels_experts.hip, option "expert_launches") against the generic launches: the same arithmetic per
-row in the same order, so logits, routing, slot outputs and the residual stream have to be the same bits."""
+"""The experts' launches of latency-bound models (kernels_experts.hip, option "expert_launches") against the generic launches, with both halves of float models
+against the one launch: the same arithmetic per row in the same order, so logits, routing, slot outputs and the residual stream have to be the same bits."""
 import numpy as np
 import pytest
 

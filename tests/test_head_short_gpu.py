@@ -1,4 +1,4 @@
-"""Heads of models without a query latent (kernels_head.hip, option "head_short") against head_attn_kernel: the same values and sums in the same order, so
+"""Heads of models without a query latent, and V3's (kernels_head.hip, option "head_short"), against head_attn_kernel: the same values and sums in the same order, so
 logits, cache rows and the attention output have to be the same bits."""
 import numpy as np
 import pytest
